@@ -9,10 +9,12 @@
 namespace hipserve {
 
 // residual[T, H] (fp32, in place) += ls1 * mix + ls2 * (1/top) * sum_j y[pair_slot[t*top+j]] + extra;
-// out = residual normalised in `groups` consecutive parts, times w (fp32 [H]). Null inputs are skipped.
+// out = residual normalised in `groups` consecutive parts, times w (fp32 [H]). Null inputs are skipped. With a
+// table [table_rows, H] the residual is not read: row t starts as table[ids[t]].
 void launch_scaled_add_group_rmsnorm(void* out, float* residual, const float* w, int T, int H, int groups, float eps,
                                      const void* mix, const float* ls1, const void* y, const int* pair_slot, int top,
-                                     const float* ls2, const void* extra, bool f32, hipStream_t s);
+                                     const float* ls2, const void* extra, const void* table, const long* ids,
+                                     long table_rows, bool f32, hipStream_t s);
 
 // proj[T, ld] rows = [q latent (q_rank) | kv latent (kv_rank) | rotary key (rot_dim) | ...]:
 // cq[T, q_rank] = RMSNorm(q latent) * q_norm; cache row slots[t] (>= 0) = [RMSNorm(kv latent) * kv_norm |

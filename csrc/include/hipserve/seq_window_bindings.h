@@ -133,9 +133,9 @@ inline void window_attention_mfma(at::Tensor& out, const at::Tensor& proj, const
 inline void activation(at::Tensor& out, const at::Tensor& x, int64_t kind, double c0, double c1) {
   CHECK_DEV(x);
   const bool f32 = is_f32(x, "activation");
-  TORCH_CHECK(kind >= 0 && kind <= 4, "activation: 0 = tanh, 1 = xielu, 2 = relu2, 3 = silu_mul, 4 = clamped_glu");
+  TORCH_CHECK(kind >= 0 && kind <= 5, "activation: 0 = tanh, 1 = xielu, 2 = relu2, 3 = silu_mul, 4 = clamped_glu, 5 = softcap");
   TORCH_CHECK(out.scalar_type() == x.scalar_type() && rows2d(x) && rows2d(out) && out.size(0) == x.size(0));
-  TORCH_CHECK(kind >= 3 ? (x.size(1) == 2 * out.size(1) && out.data_ptr() != x.data_ptr()) : out.size(1) == x.size(1));
+  TORCH_CHECK(kind == 3 || kind == 4 ? (x.size(1) == 2 * out.size(1) && out.data_ptr() != x.data_ptr()) : out.size(1) == x.size(1));
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   hipserve::launch_activation(out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), x.size(0), out.size(1), kind,
                               (float)c0, (float)c1, f32, cur_stream());

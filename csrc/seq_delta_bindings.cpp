@@ -21,7 +21,8 @@ void scaled_add_group_rmsnorm(at::Tensor& out, at::Tensor& residual, const at::T
                               const c10::optional<at::Tensor>& mix, const c10::optional<at::Tensor>& ls1,
                               const c10::optional<at::Tensor>& y, const c10::optional<at::Tensor>& pair_slot,
                               int64_t top, const c10::optional<at::Tensor>& ls2,
-                              const c10::optional<at::Tensor>& extra) {
+                              const c10::optional<at::Tensor>& extra, const c10::optional<at::Tensor>& table,
+                              const c10::optional<at::Tensor>& ids) {
   CHECK_DEV(out); CHECK_CONTIG(out); CHECK_F32(residual); CHECK_F32(w);
   const bool f32 = is_f32(out, "scaled_add_group_rmsnorm");
   TORCH_CHECK(residual.dim() == 2 && out.sizes() == residual.sizes());
@@ -39,11 +40,16 @@ void scaled_add_group_rmsnorm(at::Tensor& out, at::Tensor& residual, const at::T
   }
   if (extra.has_value())
     TORCH_CHECK(extra->scalar_type() == out.scalar_type() && extra->is_contiguous() && extra->sizes() == residual.sizes());
+  if (table.has_value()) {
+    TORCH_CHECK(table->scalar_type() == out.scalar_type() && table->is_contiguous() && table->dim() == 2 && table->size(1) == H);
+    TORCH_CHECK(ids.has_value() && ids->scalar_type() == at::kLong && ids->is_contiguous() && ids->numel() == T);
+  }
   c10::hip::HIPGuardMasqueradingAsCUDA g(out.device());
   hipserve::launch_scaled_add_group_rmsnorm(
       out.data_ptr(), residual.data_ptr<float>(), w.data_ptr<float>(), T, H, groups, (float)eps, opt_ptr(mix),
       (const float*)opt_ptr(ls1), opt_ptr(y), (const int*)opt_ptr(pair_slot), y.has_value() ? top : 0,
-      (const float*)opt_ptr(ls2), opt_ptr(extra), f32, cur_stream());
+      (const float*)opt_ptr(ls2), opt_ptr(extra), opt_ptr(table), table.has_value() ? ids->data_ptr<long>() : nullptr,
+      table.has_value() ? table->size(0) : 0, f32, cur_stream());
 }
 
 
@@ -320,7 +326,8 @@ void wkv_step(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const at::
 TORCH_LIBRARY(hipserve_delta, m) {
   def_window_ops(m);
   m.def("scaled_add_group_rmsnorm(Tensor(a!) out, Tensor(b!) residual, Tensor w, int groups, float eps, Tensor? mix, "
-        "Tensor? ls1, Tensor? y, Tensor? pair_slot, int top, Tensor? ls2, Tensor? extra) -> ()");
+        "Tensor? ls1, Tensor? y, Tensor? pair_slot, int top, Tensor? ls2, Tensor? extra, Tensor? table=None, "
+        "Tensor? ids=None) -> ()");
   m.def("gated_delta(Tensor(a!) y, Tensor(b!) S, Tensor(c!) conv_state, Tensor proj, Tensor conv_w, Tensor a_log, "
         "Tensor dt_bias, Tensor norm_w, Tensor? decay, Tensor? gate, Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, "
         "Tensor(d!) scratch, int heads, int kv_heads, int dim, int vdim, int taps, float eps, int off_a, int off_g, int off_b, "

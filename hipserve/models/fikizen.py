@@ -16,7 +16,6 @@ step's block tables, the recurrences their sequences' state slots.
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 
 from .layer_list import LayerListModel
 
@@ -30,10 +29,11 @@ class FikizenModel(LayerListModel):
         if meta.id_src is not None:  # decode lookahead: row i's id is the previous step's sample tok[src[i]]
             src, tok = meta.id_src
             ids = torch.where(src >= 0, tok.index_select(0, src.clamp(min=0)), ids)
-        residual = F.embedding(ids, self.embed).to(torch.float32, copy=True)
-        h = torch.empty(T, H, device=residual.device, dtype=self.dtype)
+        residual = torch.empty(T, H, device=ids.device, dtype=torch.float32)
+        h = torch.empty(T, H, device=ids.device, dtype=self.dtype)
         first = self.layers[self.runs[0][0]].norm1 if self.runs else self.final_norm
-        ops.scaled_add_group_rmsnorm(h, residual, first, 1, cfg.norm_eps)
+        # the first norm reads the embedding table itself
+        ops.scaled_add_group_rmsnorm(h, residual, first, 1, cfg.norm_eps, table=self.embed, ids=ids.long().contiguous())
         for r, (i, _, _) in enumerate(self.runs):
             lw = self.layers[i]
             mix = lw.mixer.forward(h, meta, kv_caches[r], state[r] if state is not None else None)
@@ -55,4 +55,4 @@ class FikizenModel(LayerListModel):
         """32-bit logits = cap * tanh(head . hidden / cap)."""
         lg = super().compute_logits(hidden)
         cap = self.cfg.logit_softcap
-        return torch.tanh(lg / cap) * cap if cap > 0 else lg
+        return self.ops.activation(lg, lg, "softcap", cap) if cap > 0 else lg

@@ -167,11 +167,14 @@ class KesiraxModel:
         if meta.id_src is not None:  # decode lookahead: row i's id is the previous step's sample tok[src[i]]
             src, tok = meta.id_src
             ids = torch.where(src >= 0, tok.index_select(0, src.clamp(min=0)), ids)
-        x0 = F.embedding(ids, self.embed)                 # the embedding output (model dtype)
-        residual = x0.to(torch.float32, copy=True)    # never an alias of x0 (float32 models)
-        h = torch.empty(T, H, device=x0.device, dtype=self.dtype)
+        # the embedding output (model dtype), where a loop pass adds it again
+        x0 = F.embedding(ids, self.embed) if any(again for _, _, again in self.runs) else None
+        residual = torch.empty(T, H, device=ids.device, dtype=torch.float32)
+        h = torch.empty(T, H, device=ids.device, dtype=self.dtype)
         first = self.layers[self.runs[0][0]] if self.runs else None
-        ops.scaled_add_group_rmsnorm(h, residual, first.norm if first else self.final_norm, cfg.norm_groups, cfg.norm_eps)
+        # the first norm reads the embedding table itself
+        ops.scaled_add_group_rmsnorm(h, residual, first.norm if first else self.final_norm, cfg.norm_groups, cfg.norm_eps,
+                                     table=self.embed, ids=ids.long().contiguous())
         for r, (i, _, _) in enumerate(self.runs):
             lw = self.layers[i]
             if isinstance(lw.mixer, LatentAttention):
@@ -208,4 +211,4 @@ class KesiraxModel:
             lg = torch.mm(hidden, self.lm_head.t(), out_dtype=torch.float32)
         else:
             lg = F.linear(hidden.float(), self.lm_head.float())
-        return lg * self.cfg.logit_scale
+        return lg if self.cfg.logit_scale == 1.0 else lg.mul_(self.cfg.logit_scale)

@@ -224,9 +224,10 @@ class KernelOps:
 
     # ---- layer-list decoders (csrc/kernels/seq/*.hip; bf16 or true fp32 activations)
     def scaled_add_group_rmsnorm(self, out, residual, w, groups, eps, mix=None, ls1=None, y=None, pair_slot=None,
-                                 top=0, ls2=None, extra=None):
+                                 top=0, ls2=None, extra=None, table=None, ids=None):
+        """``table`` / ``ids``: the rows start as table[ids] instead of what ``residual`` holds."""
         lib = self._delta if self.norm_library == "delta" else self._seq
-        lib.scaled_add_group_rmsnorm(out, residual, w, groups, eps, mix, ls1, y, pair_slot, top, ls2, extra)
+        lib.scaled_add_group_rmsnorm(out, residual, w, groups, eps, mix, ls1, y, pair_slot, top, ls2, extra, table, ids)
         return out
 
     def latent_prepare(self, cq, cache, proj, positions, slots, q_norm, kv_norm, inv_freq, q_rank, kv_rank,
@@ -370,7 +371,7 @@ class KernelOps:
         self._delta.delta_rule(out, state[0], proj, wl, a_b, w0, norm_w, meta.seq_cu, meta.seq_ctx, meta.seq_state,
                              scratch, sp.heads, sp.dim, eps, out_scale)
 
-    ACTIVATIONS = {"tanh": 0, "xielu": 1, "relu2": 2, "silu_mul": 3, "clamped_glu": 4}
+    ACTIVATIONS = {"tanh": 0, "xielu": 1, "relu2": 2, "silu_mul": 3, "clamped_glu": 4, "softcap": 5}
 
     def activation(self, out, x, kind, c0=0.0, c1=0.0):
         self._window_lib.activation(out, x, self.ACTIVATIONS[kind], c0, c1)
@@ -623,8 +624,8 @@ class ReferenceOps:
 
     # ---- layer-list decoders (models/mixers.py)
     def scaled_add_group_rmsnorm(self, out, residual, w, groups, eps, mix=None, ls1=None, y=None, pair_slot=None,
-                                 top=0, ls2=None, extra=None):
-        ref.scaled_add_group_rmsnorm(out, residual, w, groups, eps, mix, ls1, y, pair_slot, top, ls2, extra)
+                                 top=0, ls2=None, extra=None, table=None, ids=None):
+        ref.scaled_add_group_rmsnorm(out, residual, w, groups, eps, mix, ls1, y, pair_slot, top, ls2, extra, table, ids)
         return out
 
     def latent_prepare(self, cq, cache, proj, positions, slots, q_norm, kv_norm, inv_freq, q_rank, kv_rank,

@@ -400,10 +400,12 @@ def top_logprobs(logits, nreq, out_ids, out_lp):
 # attention on a paged latent cache, minGRU scan over state slots, table-routed experts
 
 def scaled_add_group_rmsnorm(out, residual, w, groups, eps, mix=None, ls1=None, y=None, pair_slot=None, top=0,
-                             ls2=None, extra=None):
-    """residual (fp32, in place) += ls1 * mix + ls2 * mean_j y[pair_slot[t * top + j]] + extra;
-    out = residual normalised in ``groups`` equal consecutive parts, times w."""
+                             ls2=None, extra=None, table=None, ids=None):
+    """residual (fp32, in place; starts as table[ids] with a ``table``) += ls1 * mix + ls2 * mean_j y[pair_slot[t * top + j]]
+    + extra; out = residual normalised in ``groups`` equal consecutive parts, times w."""
     T, H = residual.shape
+    if table is not None:
+        residual.copy_(table.index_select(0, ids))
     if mix is not None:
         residual += mix.float() * ls1.float() if ls1 is not None else mix.float()
     if y is not None:
@@ -751,7 +753,7 @@ def activation(out, x, kind, c0=0.0, c1=0.0):
     """Elementwise: ``tanh``; ``relu2`` = max(z, 0)^2; ``xielu`` with c0 = softplus(p),
     c1 = 1/2 + softplus(q): c0 z^2 + z/2 for z > 0, c1 (exp(z) - 1 - z) + z/2 otherwise;
     ``silu_mul``: x rows = [gate | up], out = silu(gate) * up (half as wide); ``clamped_glu``: the same with
-    g sigmoid(1.702 g) (u + 1), g = min(gate, c0), u = clamp(up, -c0, c0)."""
+    g sigmoid(1.702 g) (u + 1), g = min(gate, c0), u = clamp(up, -c0, c0); ``softcap`` = c0 tanh(z / c0)."""
     z = x.float()
     if kind == "tanh":
         r = torch.tanh(z)
@@ -763,6 +765,8 @@ def activation(out, x, kind, c0=0.0, c1=0.0):
     elif kind == "clamped_glu":
         n = z.shape[-1] // 2
         r = clamped_glu(z[..., :n], z[..., n:], c0)
+    elif kind == "softcap":
+        r = torch.tanh(z / c0) * c0
     elif kind == "xielu":
         zn = z.clamp(max=0.0)
         r = torch.where(z > 0, c0 * z * z + 0.5 * z, c1 * (torch.expm1(zn) - zn) + 0.5 * z)
