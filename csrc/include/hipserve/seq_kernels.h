@@ -16,6 +16,13 @@ void launch_scaled_add_group_rmsnorm(void* out, float* residual, const float* w,
                                      const float* ls2, const void* extra, const void* table, const long* ids,
                                      long table_rows, bool f32, hipStream_t s);
 
+// out[b, m, n] = act(x[b, m] . W[b, n] + bias[n]) of up to 64 rows m (skinny_linear.hip): bf16 operands, K % 8 == 0, x rows at
+// multiples of 16 bytes; W [batch, N, K]; act 0 tanh, 1 xIELU, 2 relu^2, 3 SiLU gate, 4 clamped gate (N / 2 columns),
+// 5 soft cap, -1 none.
+void launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs,
+                          const void* w, const void* bias, int batch, int M, int N, int K, int act, float c0, float c1,
+                          hipStream_t s);
+
 // proj[T, ld] rows = [q latent (q_rank) | kv latent (kv_rank) | rotary key (rot_dim) | ...]:
 // cq[T, q_rank] = RMSNorm(q latent) * q_norm; cache row slots[t] (>= 0) = [RMSNorm(kv latent) * kv_norm |
 // RoPE(rotary key)], rotate-half over the first 2 * nfreq dims with angle pos * inv_freq[i].
@@ -54,9 +61,10 @@ void launch_mingru_scan(void* y, float* state, const void* proj, const float* b_
 // expert is < 0 or >= E (no weights) are skipped. act 0: none, 1: squared ReLU, 2: W[e] = [gate rows; up rows]
 // and out[slot, N / 2] = silu(gate) * up, 3: the same with g sigmoid(1.702 g) (u + 1), g = min(gate, limit),
 // u = clamp(up, -limit, limit). row_scale (may be null): the products of pair p are multiplied by row_scale[p] first.
+// pairs: how many (token, choice) pairs the tiles hold (0: guessed from their capacity).
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,
                         int ntiles_cap, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
-                        float limit, bool f32, hipStream_t s);
+                        float limit, int pairs, bool f32, hipStream_t s);
 
 // Norms before and after a sublayer (sandwich.hip): residual[T, H] (fp32, in place; `table` [vocab, H] in the activation
 // type: it starts as table_scale * table[ids[t]]) += mult * y / rms(y) * w_post; out = residual / rms(residual) * w_next.

@@ -1,5 +1,5 @@
 // Bindings shared by the layer-list decoders' kernel libraries (each library links its own copy of the
-// kernels): the expert alignment and the expert GEMMs of the mixtures of experts.
+// kernels): products of a few rows, the expert alignment and the expert GEMMs of the mixtures of experts.
 #pragma once
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
@@ -48,7 +48,7 @@ inline void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor
 
 inline void expert_gemm(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const at::Tensor& slots,
                         const at::Tensor& tile_expert, int64_t tile, int64_t gather_k, int64_t act,
-                        const c10::optional<at::Tensor>& row_scale, double limit) {
+                        const c10::optional<at::Tensor>& row_scale, double limit, int64_t pairs) {
   auto i32 = [](const at::Tensor& t) { return t.scalar_type() == at::kInt && t.is_contiguous(); };
   TORCH_CHECK(x.is_cuda() && out.is_contiguous() && w.is_contiguous() && i32(slots) && i32(tile_expert));
   TORCH_CHECK(x.scalar_type() == at::kFloat || x.scalar_type() == at::kBFloat16, "expert_gemm: bf16 or fp32 activations");
@@ -65,20 +65,47 @@ inline void expert_gemm(at::Tensor& out, const at::Tensor& x, const at::Tensor& 
   TORCH_CHECK(x.size(1) == K && out.size(1) == (act >= 2 ? N / 2 : N) && out.size(0) >= cap);
   TORCH_CHECK(tile % 32 == 0 && cap % tile == 0 && tile_expert.numel() * tile >= cap, "tiles of a multiple of 32 slots");
   TORCH_CHECK(gather_k > 0 || x.size(0) >= cap, "ungathered x needs one row per slot");
+  TORCH_CHECK(pairs >= 0 && pairs <= cap, "expert_gemm: at most a pair per slot");
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   hipserve::launch_expert_gemm(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), slots.data_ptr<int>(),
                                tile_expert.data_ptr<int>(), cap / tile, tile, gather_k, N, K, act, w.size(0),
-                               (const float*)opt_ptr(row_scale), (float)limit, f32,
+                               (const float*)opt_ptr(row_scale), (float)limit, pairs, f32,
                                c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
 }
 
+// out = act(x . w^T + bias) of at most 64 rows: x [M, K] or [B, M, K], w [N, K] or [B, N, K], out [M, N'] or [B, M, N'].
+inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias,
+                          int64_t act, double c0, double c1) {
+  CHECK_DEV(x); CHECK_CONTIG(w);
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
+              (out.scalar_type() == at::kBFloat16 || out.scalar_type() == at::kFloat), "skinny_linear: bf16 operands");
+  const long d = x.dim();
+  TORCH_CHECK((d == 2 || d == 3) && w.dim() == d && out.dim() == d, "skinny_linear: rows or batches of rows");
+  const long B = d == 3 ? x.size(0) : 1, M = x.size(-2), K = x.size(-1), N = w.size(-2);
+  TORCH_CHECK(w.size(-1) == K && (d == 2 || (w.size(0) == B && out.size(0) == B)) && out.size(-2) == M && M <= 64 && K % 8 == 0 &&
+              N < (1L << 31) && K < (1L << 31) && B < 65536, "skinny_linear: shapes");
+  const bool glu = act == 3 || act == 4;
+  TORCH_CHECK(act >= -1 && act <= 5 && (!glu || N % 2 == 0) && out.size(-1) == (glu ? N / 2 : N), "skinny_linear: activation");
+  auto aligned = [](const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
+  TORCH_CHECK(x.stride(-1) == 1 && out.stride(-1) == 1 && x.stride(-2) % 8 == 0 && (d == 2 || x.stride(0) % 8 == 0) && aligned(x) &&
+              aligned(w), "skinny_linear: rows at multiples of 16 bytes");
+  if (bias.has_value())
+    TORCH_CHECK(d == 2 && bias->scalar_type() == at::kBFloat16 && bias->is_contiguous() && bias->numel() == N, "skinny_linear: bias");
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  hipserve::launch_skinny_linear(out.data_ptr(), out.scalar_type() == at::kFloat, out.stride(-2), d == 3 ? out.stride(0) : 0,
+                                 x.data_ptr(), x.stride(-2), d == 3 ? x.stride(0) : 0, w.data_ptr(), opt_ptr(bias), B, M, N, K,
+                                 act, (float)c0, (float)c1, cur_stream());
+}
+
 inline void def_moe_ops(torch::Library& m) {
+  m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int act, float c0, float c1) -> ()");
   m.def("moe_align(Tensor ids, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, Tensor(c!) pair_slot) -> ()");
   m.def("expert_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor slots, Tensor tile_expert, int tile, int gather_k, "
-        "int act, Tensor? row_scale=None, float limit=0.0) -> ()");
+        "int act, Tensor? row_scale=None, float limit=0.0, int pairs=0) -> ()");
 }
 
 inline void impl_moe_ops(torch::Library& m) {
+  m.impl("skinny_linear", &skinny_linear);
   m.impl("moe_align", &moe_align);
   m.impl("expert_gemm", &expert_gemm);
 }

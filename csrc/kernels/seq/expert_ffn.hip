@@ -8,7 +8,9 @@
 // multiplied by row_scale[pair] first (the pair's weight on its input: the products are linear in it). Any N and K: edges are bounds-checked. A workgroup
 // computes a [32 slots x 64 columns] block, x and W staged through LDS in K-chunks of 32, fp32
 // accumulation; bf16 and fp32 element types.
-#include "seq_common.h"
+#include <algorithm>
+
+#include "skinny.h"
 #include "hipserve/seq_kernels.h"
 
 namespace hipserve {
@@ -189,17 +191,99 @@ __global__ __launch_bounds__(256) void expert_gemm_mfma_kernel(
   }
 }
 
+// bf16, tiles with few live slots (decode steps): 16 columns per workgroup, K split over its waves (skinny.h).
+template <int NT, int KU, bool GLU>
+__global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
+    unsigned short* __restrict__ out, const unsigned short* __restrict__ x, long x_ld,
+    const unsigned short* __restrict__ w, const int* __restrict__ slots, const int* __restrict__ tile_expert,
+    int gather_k, int N, int K, int act, int E, const float* __restrict__ row_scale, float limit) {
+  constexpr int ST = 2;   // a tile is 32 slots
+  __shared__ __attribute__((aligned(16))) float red[kSkWaves * 16 * ST * kSkLd];
+  const int e = tile_expert[blockIdx.y];
+  if (e < 0 || e >= E) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+  const int slot0 = blockIdx.y * 16 * ST, No = GLU ? N / 2 : N, n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
+  const bool low = c < 8;
+  const int g8 = g + 4 * (c >> 3);
+  const unsigned short* wr[NT][2];
+  const unsigned short* xr[ST][2];
+  bool live[ST][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int cc = (c & 7) + 8 * h;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+      wr[nt][h] = w + ((long)e * N + (GLU ? nt * No + min(n0 + cc, No - 1) : min(n0 + 16 * nt + cc, N - 1))) * K + 8 * g8;
+#pragma unroll
+    for (int st = 0; st < ST; ++st) {
+      const int slot = slot0 + 16 * st + cc, p = slots[slot];
+      live[st][h] = p >= 0;
+      xr[st][h] = x + (p < 0 ? 0 : gather_k > 0 ? (long)(p / gather_k) : (long)slot) * x_ld + 8 * g8;
+    }
+  }
+  f32x4 acc[NT][ST];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
+  skinny_accumulate<ST, NT, KU>(acc, wr, xr, live, K, g8, low, wave);
+  float v[NT][1];
+  skinny_reduce<ST, NT>(v, acc, red);
+  const int slot = slot0 + (tid >> 4), p = slots[slot];   // 512 threads: an element of the [32, 16] result each
+  if (p < 0) return;
+  const float f = row_scale != nullptr ? row_scale[p] : 1.f;
+#pragma unroll
+  for (int nt = 0; nt < (GLU ? 1 : NT); ++nt) {
+    const int n = n0 + 16 * nt + (tid & 15);
+    if (n >= No) continue;
+    float r = v[nt][0] * f;
+    if constexpr (GLU) {
+      const float u = v[1][0] * f;
+      r = act == 3 ? clamped_glu_f(r, u, limit) : r * sigmoid_f(r) * u;
+    } else if (act == 1) {
+      r = fmaxf(r, 0.f);
+      r *= r;
+    }
+    out[(long)slot * No + n] = f32_to_bf16(r);
+  }
+}
+
+// Which of the two kernels serves tiles of 32 slots; cold weights, us with the launch: expert_gemm_mfma takes 10 + 0.95 per
+// step of 128 k (its steps wait for their loads) while its workgroups of 128 columns are at most 512; expert_gemm_skinny
+// 5.2 plus the weights at 5 TB/s, or what its workgroups of 16 columns read at 34 KB per us and CU. 2 of 16 experts of
+// 2048 -> 1024 -> 2048: 2 pairs 23 -> 7.2 us (up) and 18 -> 5.5 (down), 96 pairs on all 16 experts 26 -> 21 (up); 1400
+// pairs stay on the tile kernel (26 against 87 expected).
+bool skinny_tiles(int pairs, int N, int K, int E, bool glu) {
+  const double used = std::min(E, pairs), tiles = used + pairs / 32, rows = std::min(32.0, pairs / used);
+  const double wgs = std::max(1.0, tiles * N / 16 / 256);
+  const double ours = 5.2 + std::max(used * N * K * 2 / 5.0e6, wgs * 2 * K * (16 + rows / (glu ? 2 : 1)) / 34e3);
+  return ours < (10 + 0.95 * K / 128) * std::max(1.0, tiles * N / 128 / 512);
+}
+
 }  // namespace
 
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,
                         int ntiles_cap, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
-                        float limit, bool f32, hipStream_t s) {
+                        float limit, int pairs, bool f32, hipStream_t s) {
   if (ntiles_cap <= 0) return;
+  // the capacity covers a partly filled tile per expert
+  pairs = pairs > 0 ? pairs : std::max(1, ntiles_cap * tile - E * (tile - 1));
   const int No = act >= 2 ? N / 2 : N;
   if (!f32 && K % 8 == 0 && No % 8 == 0 && x_ld % 8 == 0 && (tile == 32 || tile == 64)) {
     dim3 mg(act >= 2 ? (No + 63) / 64 : (N + 127) / 128, ntiles_cap);
     auto o = (unsigned short*)out;
     auto xi = (const unsigned short*)x, wi = (const unsigned short*)w;
+    if (tile == 32 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && skinny_tiles(pairs, N, K, E, act >= 2)) {
+      const dim3 sg((No + 15) / 16, ntiles_cap);
+#define HS_ES(NT, KU, GLU)                                                                                          \
+  expert_gemm_skinny_kernel<NT, KU, GLU><<<sg, kSkThreads, 0, s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K, \
+                                                                   act, E, row_scale, limit)
+      if (act >= 2) HS_ES(2, 4, true);
+      else if (K <= 1024) HS_ES(1, 4, false);
+      else HS_ES(1, 8, false);
+#undef HS_ES
+      return;
+    }
     if (tile == 32) expert_gemm_mfma_kernel<2><<<mg, 256, 0, s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K, act, E, row_scale, limit);
     else expert_gemm_mfma_kernel<4><<<mg, 256, 0, s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K, act, E, row_scale, limit);
     return;

@@ -53,6 +53,5 @@ class FikizenModel(LayerListModel):
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """32-bit logits = cap * tanh(head . hidden / cap)."""
-        lg = super().compute_logits(hidden)
         cap = self.cfg.logit_softcap
-        return self.ops.activation(lg, lg, "softcap", cap) if cap > 0 else lg
+        return self.ops.linear(hidden, self.lm_head, out_f32=True, **({"act": "softcap", "c0": cap} if cap > 0 else {}))

@@ -205,10 +205,5 @@ class KesiraxModel:
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """32-bit logits = head . hidden * logit_scale."""
-        if hidden.dtype == torch.float32:
-            lg = F.linear(hidden, self.lm_head)
-        elif hidden.is_cuda:
-            lg = torch.mm(hidden, self.lm_head.t(), out_dtype=torch.float32)
-        else:
-            lg = F.linear(hidden.float(), self.lm_head.float())
+        lg = self.ops.linear(hidden, self.lm_head, out_f32=True)
         return lg if self.cfg.logit_scale == 1.0 else lg.mul_(self.cfg.logit_scale)

@@ -11,7 +11,6 @@ having one).
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 
 from ..parallel.comm import TPGroup
 from .mixers import make_ff, make_mixer
@@ -164,11 +163,7 @@ class LayerListModel:
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """32-bit logits = head . hidden."""
-        if hidden.dtype == torch.float32:
-            return F.linear(hidden, self.lm_head)
-        if hidden.is_cuda:
-            return torch.mm(hidden, self.lm_head.t(), out_dtype=torch.float32)
-        return F.linear(hidden.float(), self.lm_head.float())
+        return self.ops.linear(hidden, self.lm_head, out_f32=True)
 
 
 def _proj_width(mixer) -> int:

@@ -4,8 +4,8 @@ spec (``config.LatentAttentionSpec`` / ``MinGRUSpec`` / ``TableMoESpec``) and ru
 engine's op set (``ops.KernelOps`` on a GPU, ``ops.ReferenceOps`` on the CPU), so another
 design can list them in its own layer order.
 
-Dense projections are vendor GEMMs (``F.linear`` / ``torch.bmm``); everything between
-them is one op of the op set:
+Dense projections are ``ops.linear`` (the vendor's GEMMs, or a weight-streaming kernel for a few rows) and batched GEMMs
+over the heads; everything between them is one op of the op set:
 
 * latent attention: merged [q-latent | kv-latent | rotary key | gate] projection ->
   ``latent_prepare`` (both latent RMSNorms, rotary key part, paged cache write) -> query
@@ -132,6 +132,8 @@ class LatentAttention:
         self.w_uq = None       # [heads * (dim + rot_dim), q_rank]
         self.w_uk = None       # [heads, dim, kv_rank]
         self.w_uk_wide = None  # [heads, dim, kv_rank + rot_dim], zero rotary columns (made at first use)
+        self.w_uk_t = None     # [heads, kv_rank, dim] (made at first use)
+        self.w_uv = None       # [heads, vdim, kv_rank]
         self.w_uv_t = None     # [heads, kv_rank, vdim]
         self.w_o = None        # [hidden, heads * vdim]
         rd = s.rot_dims or s.rot_dim
@@ -155,7 +157,8 @@ class LatentAttention:
         self.kv_norm = get(prefix + "dkv.norm").to(dev, torch.float32)
         self.w_uq = uq.to(dev, dt).contiguous()
         self.w_uk = get(prefix + "uk").to(dev, dt).view(s.heads, s.dim, s.kv_rank).contiguous()
-        self.w_uv_t = get(prefix + "uv").to(dev, dt).view(s.heads, s.vdim, s.kv_rank).transpose(1, 2).contiguous()
+        self.w_uv = get(prefix + "uv").to(dev, dt).view(s.heads, s.vdim, s.kv_rank).contiguous()
+        self.w_uv_t = self.w_uv.transpose(1, 2).contiguous()
         self.w_o = get(prefix + "o").to(dev, dt).contiguous()
 
     def init_random(self, gen, std: float):
@@ -180,32 +183,41 @@ class LatentAttention:
     def forward(self, h: torch.Tensor, meta, cache: torch.Tensor, state=None) -> torch.Tensor:
         s, ops = self.spec, self.ops
         T = h.shape[0]
-        proj = F.linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         _side(self, proj)
         gate_off = s.q_rank + s.key_dim
         cq = torch.empty(T, s.q_rank, device=h.device, dtype=h.dtype)
         ops.latent_prepare(cq, cache, proj, meta.positions, meta.slot_mapping, self.q_norm, self.kv_norm,
                            self.inv_freq, s.q_rank, s.kv_rank, s.rot_dim, self.eps)
-        q = F.linear(cq, self.w_uq)                                    # [T, heads * (dim + rot_dim)]
+        q = self.ops.linear(cq, self.w_uq)                             # [T, heads * (dim + rot_dim)]
         qh = q.view(T, s.heads, s.dim + s.rot_dim)
         if ops.latent_query_in_place(h.dtype, s.kv_rank, s.rot_dim):
             # the absorption GEMM writes the attention kernel's query rows directly: bf16, the cached width,
             # zero weight columns where the attention op puts the rotated part
-            if self.w_uk_wide is None:
-                self.w_uk_wide = F.pad(self.w_uk, (0, s.rot_dim)).contiguous()
-            q_abs = torch.bmm(qh[:, :, : s.dim].transpose(0, 1), self.w_uk_wide)   # [heads, T, kv_rank + rot_dim]
+            q_abs = torch.empty(s.heads, T, s.key_dim, device=h.device, dtype=h.dtype)
+            q_heads = qh[:, :, : s.dim].transpose(0, 1)
+            if self.w_uk_t is None:
+                self.w_uk_t = self.w_uk.transpose(1, 2).contiguous()
+            if not ops.linear_heads(q_abs[:, :, : s.kv_rank], q_heads, self.w_uk_t):
+                if self.w_uk_wide is None:
+                    self.w_uk_wide = F.pad(self.w_uk, (0, s.rot_dim)).contiguous()
+                torch.bmm(q_heads, self.w_uk_wide, out=q_abs)              # [heads, T, kv_rank + rot_dim]
         else:
             q_abs = _mm32(qh[:, :, : s.dim].transpose(0, 1), self.w_uk)            # [heads, T, kv_rank] fp32
         o_lat = torch.empty(s.heads, T, s.kv_rank, device=h.device, dtype=h.dtype)
         ops.latent_attention(o_lat, q_abs, q, proj, cache, meta, self.inv_freq, s.heads, s.dim, s.rot_dim,
                              s.kv_rank, gate_off if s.gate == "head" else -1, s.scale, s.window)
-        o = torch.bmm(o_lat, self.w_uv_t)                              # [heads, T, vdim]
+        cat = torch.empty(T, s.heads * s.vdim, device=h.device, dtype=h.dtype)
+        if s.gate != "channel" and ops.linear_heads(cat.view(T, s.heads, s.vdim).transpose(0, 1), o_lat, self.w_uv):
+            return ops.linear(cat, self.w_o)                           # the heads were written side by side
+        o = torch.empty(s.heads, T, s.vdim, device=h.device, dtype=h.dtype)
+        if not ops.linear_heads(o, o_lat, self.w_uv):
+            torch.bmm(o_lat, self.w_uv_t, out=o)                       # [heads, T, vdim]
         if s.gate == "channel":
             # heads side by side per token, each element times the sigmoid of its gate column: one pass
-            cat = torch.empty(T, s.heads * s.vdim, device=h.device, dtype=h.dtype)
             ops.gate_mul(cat, o, proj[:, gate_off:gate_off + s.heads * s.vdim])
-            return F.linear(cat, self.w_o)
-        return F.linear(o.transpose(0, 1).reshape(T, s.heads * s.vdim), self.w_o)
+            return self.ops.linear(cat, self.w_o)
+        return self.ops.linear(o.transpose(0, 1).reshape(T, s.heads * s.vdim), self.w_o)
 
 
 class MinGRU:
@@ -236,10 +248,10 @@ class MinGRU:
         return (num_slots, self.spec.width)
 
     def forward(self, h: torch.Tensor, meta, state: torch.Tensor) -> torch.Tensor:
-        proj = F.linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         y = torch.empty(h.shape[0], self.spec.width, device=h.device, dtype=h.dtype)
         self.ops.mingru_scan(y, state, proj, self.b_z, self.b_x, meta)
-        return F.linear(y, self.w_o)
+        return self.ops.linear(y, self.w_o)
 
 
 class TableMoE:
@@ -282,9 +294,9 @@ class TableMoE:
         pair_slot = torch.empty(P, dtype=torch.int32, device=dev)
         ops.moe_align(experts, s.experts, tile, slots, tile_expert, pair_slot)
         act = torch.empty(cap, s.ff, device=dev, dtype=h.dtype)
-        ops.expert_gemm(act, h, self.w_up, slots, tile_expert, tile, s.top, True)
+        ops.expert_gemm(act, h, self.w_up, slots, tile_expert, tile, s.top, True, pairs=P)
         y = torch.empty(cap, self.hidden, device=dev, dtype=h.dtype)
-        ops.expert_gemm(y, act, self.w_down, slots, tile_expert, tile, 0, False)
+        ops.expert_gemm(y, act, self.w_down, slots, tile_expert, tile, 0, False, pairs=P)
         return y, pair_slot
 
     def _packed_ok(self, h: torch.Tensor, P: int) -> bool:
@@ -320,15 +332,6 @@ class TableMoE:
         y = torch.empty(cap, H, dtype=h.dtype, device=dev)
         op.prefill_gemm_packed_grouped(y, act, pd, H, 0, tile_expert, ntiles, gemm.PW_WM, gemm.PW_RW)
         return y, pair_slot
-
-
-def _linear32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """x . w^T with a 32-bit result (inputs of the recurrences' decays stay 32-bit)."""
-    if x.dtype == torch.float32:
-        return F.linear(x, w)
-    if x.is_cuda:
-        return torch.mm(x, w.t(), out_dtype=torch.float32)
-    return F.linear(x.float(), w.float())
 
 
 def _rand(gen, *shape, std=1.0):
@@ -430,7 +433,7 @@ class WindowAttention:
         a wider one (a column slice, overwritten)."""
         s, ops = self.spec, self.ops
         if proj is None:
-            proj = F.linear(h, self.w_in, self.b_in)
+            proj = self.ops.linear(h, self.w_in, self.b_in)
             _side(self, proj)
         ops.attn_prepare(proj, cache, meta, self.inv_freq, s, self.q_norm, self.k_norm, self.eps)
         ops.window_attention(out, proj, cache, meta, s, self.gate_off, out_scale, self.lam, self.eps, self.sink_w)
@@ -438,7 +441,7 @@ class WindowAttention:
 
     def forward(self, h, meta, cache, state):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return F.linear(self.mix(h, meta, cache, state, out), self.w_o, self.b_o)
+        return self.ops.linear(self.mix(h, meta, cache, state, out), self.w_o, self.b_o)
 
 
 class Wkv:
@@ -491,16 +494,16 @@ class Wkv:
         mixed = torch.empty(5, T, self.hidden, device=x.device, dtype=self.dtype)
         ops.token_shift(mixed, x, state[1], self.mu, meta)
         proj = torch.bmm(mixed[:4], self.w_in_t)                       # [4, T, heads * dim]: r, k, v, gate
-        low = F.linear(mixed[4], self.w1)
+        low = self.ops.linear(mixed[4], self.w1)
         out = torch.empty(T, s.size, device=x.device, dtype=self.dtype)
         if meta.max_q == 1 and s.dim <= self.STEP_MAX_DIM and low.shape[1] <= self.STEP_MAX_RANK:
             # every sequence brings one row (decode steps): bottleneck, recurrence, norm and gate in one launch
             ops.wkv_step(out, state[0], proj, low, self.w2, self.w0, self.u, self.norm, s, self.eps, meta)
-            return F.linear(out, self.w_o)
+            return self.ops.linear(out, self.w_o)
         ops.activation(low, low, "tanh")
-        wl = _linear32(low, self.w2)
+        wl = self.ops.linear(low, self.w2, out_f32=True)
         ops.wkv(out, state[0], proj, wl, self.w0, self.u, self.norm, s, self.eps, meta)
-        return F.linear(out, self.w_o)
+        return self.ops.linear(out, self.w_o)
 
 
 class GatedDelta:
@@ -582,7 +585,7 @@ class GatedDelta:
         s, ops = self.spec, self.ops
         assert out_scale == 1.0
         if proj is None:
-            proj = F.linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in)
         weights = (self.conv_w, self.a_log, self.dt_bias, self.norm)
         offs = (self.off_a, self.off_g, self.off_b)
         ra, rg = (self.w_a2.shape[1], self.w_g2.shape[1]) if s.channel_decay else (0, 0)
@@ -592,14 +595,14 @@ class GatedDelta:
             return out
         decay = gate = None
         if s.channel_decay:
-            decay = _linear32(proj[:, self.off_a:self.off_a + ra], self.w_a2)
-            gate = F.linear(proj[:, self.off_g:self.off_g + rg], self.w_g2)
+            decay = self.ops.linear(proj[:, self.off_a:self.off_a + ra], self.w_a2, out_f32=True)
+            gate = self.ops.linear(proj[:, self.off_g:self.off_g + rg], self.w_g2)
         ops.gated_delta(out, state, proj, *weights, decay, gate, offs, s, self.eps, meta)
         return out
 
     def forward(self, h, meta, cache, state):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return F.linear(self.mix(h, meta, cache, state, out), self.w_o)
+        return self.ops.linear(self.mix(h, meta, cache, state, out), self.w_o)
 
 
 class DeltaRule:
@@ -639,16 +642,16 @@ class DeltaRule:
 
     def mix(self, h, meta, cache, state, out, out_scale: float = 1.0):
         N, ops = self.spec.size, self.ops
-        proj = F.linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         low = torch.empty(h.shape[0], self.w2.shape[1], device=h.device, dtype=h.dtype)
         ops.activation(low, proj[:, 5 * N:], "tanh")
-        wl = _linear32(low, self.w2)
+        wl = self.ops.linear(low, self.w2, out_f32=True)
         ops.delta_rule(out, state, proj, wl, self.a_b, self.w0, self.norm, self.spec, self.eps, meta, out_scale)
         return out
 
     def forward(self, h, meta, cache, state):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return F.linear(self.mix(h, meta, cache, state, out), self.w_o)
+        return self.ops.linear(self.mix(h, meta, cache, state, out), self.w_o)
 
 
 class MLstm:
@@ -691,12 +694,12 @@ class MLstm:
 
     def forward(self, h, meta, cache, state):
         s = self.spec
-        proj = F.linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in)
         _side(self, proj)
-        gates = _linear32(h, self.w_if)                                # [T, 2 * heads], 32-bit
+        gates = self.ops.linear(h, self.w_if, out_f32=True)               # [T, 2 * heads]
         out = torch.empty(h.shape[0], s.out_size, device=h.device, dtype=h.dtype)
         self.ops.mlstm(out, state, proj, gates, self.b_if, self.norm, s, self.eps, meta)
-        return F.linear(out, self.w_o)
+        return self.ops.linear(out, self.w_o)
 
 
 class Lightning:
@@ -735,13 +738,13 @@ class Lightning:
 
     def mix(self, h, meta, cache, state, out, out_scale: float = 1.0, proj=None):
         if proj is None:
-            proj = F.linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in)
         self.ops.lightning(out, state[0], proj, self.powers, self.norm, self.spec, self.eps, meta, out_scale)
         return out
 
     def forward(self, h, meta, cache, state):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return F.linear(self.mix(h, meta, cache, state, out), self.w_o)
+        return self.ops.linear(self.mix(h, meta, cache, state, out), self.w_o)
 
 
 class NormedPair(NamedTuple):
@@ -803,13 +806,13 @@ class ParallelMixer:
     def _forward_normed(self, h, meta, cache, state):
         pl = pr = None
         if self.w_in is not None:
-            proj = F.linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in)
             pl, pr = proj[:, :self.split], proj[:, self.split:]
         ys = []
         for m, p in ((self.left, pl), (self.right, pr)):
             out = torch.empty(h.shape[0], m.out_size, device=h.device, dtype=h.dtype)
             m.mix(h, meta, cache, state, out, 1.0, **({} if p is None else {"proj": p}))
-            ys.append(F.linear(out, m.w_o, getattr(m, "b_o", None)))
+            ys.append(self.ops.linear(out, m.w_o, getattr(m, "b_o", None)))
         return NormedPair(ys[0], self.left_norm, ys[1], self.right_norm, self.spec.left_scale, self.spec.right_scale)
 
     def forward(self, h, meta, cache, state):
@@ -818,13 +821,13 @@ class ParallelMixer:
         a, b = self.left.out_size, self.right.out_size
         buf = torch.empty(h.shape[0], a + b, device=h.device, dtype=h.dtype)
         if self.w_in is not None:
-            proj = F.linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in)
             self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale, proj[:, :self.split])
             self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale, proj[:, self.split:])
-            return F.linear(buf, self.w_o)
+            return self.ops.linear(buf, self.w_o)
         self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale)
         self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale)
-        return F.linear(buf, self.w_o)
+        return self.ops.linear(buf, self.w_o)
 
 
 class DenseFF:
@@ -860,23 +863,18 @@ class DenseFF:
         return t
 
     def forward(self, h):
-        up = F.linear(h, self.w_up)
+        ff, act = self.spec.ff, self.spec.act
+        c0 = self.spec.limit if act == "clamped_glu" else self.c0
+        if act != "polynorm" and not self.side_rows:
+            return self.ops.linear(self.ops.linear(h, self.w_up, act=act, c0=c0, c1=self.c1), self.w_down)
+        up = self.ops.linear(h, self.w_up)
         _side(self, up)
-        ff = self.spec.ff
-        if self.spec.act == "polynorm":
-            act = torch.empty(h.shape[0], ff, device=h.device, dtype=h.dtype)
-            self.ops.polynorm(act, up[:, :ff], self.coef, self.eps)
-            return F.linear(act, self.w_down)
-        if self.spec.act == "clamped_glu":
-            act = torch.empty(h.shape[0], ff, device=h.device, dtype=h.dtype)
-            self.ops.activation(act, up[:, :2 * ff], "clamped_glu", self.spec.limit)
-            return F.linear(act, self.w_down)
-        if self.side_rows:
-            act = torch.empty(h.shape[0], ff, device=h.device, dtype=h.dtype)
-            self.ops.activation(act, up[:, :ff], self.spec.act, self.c0, self.c1)
-            return F.linear(act, self.w_down)
-        self.ops.activation(up, up, self.spec.act, self.c0, self.c1)
-        return F.linear(up, self.w_down)
+        out = torch.empty(h.shape[0], ff, device=h.device, dtype=h.dtype)
+        if act == "polynorm":
+            self.ops.polynorm(out, up[:, :ff], self.coef, self.eps)
+        else:
+            self.ops.activation(out, up[:, :2 * ff] if act == "clamped_glu" else up[:, :ff], act, c0, self.c1)
+        return self.ops.linear(out, self.w_down)
 
 
 class RoutedMoE:
@@ -939,7 +937,7 @@ class RoutedMoE:
         T, dev = h.shape[0], h.device
         ids = torch.empty(T, s.top, dtype=torch.int32, device=dev)
         wts = torch.empty(T, s.top, dtype=torch.float32, device=dev)
-        logits = _linear32(h, self.w_router)
+        logits = self.ops.linear(h, self.w_router, out_f32=True)
         if s.shared_gate:
             n = s.experts + s.identity
             logits, self.shared_gate = logits[:, :n], logits[:, n:]
@@ -960,9 +958,9 @@ class RoutedMoE:
         ops.route_align(ids, wts, slots, tile_expert, pair_slot, *router, nb, tile, *options)
         act = torch.empty(cap, s.ff, device=dev, dtype=h.dtype)
         # the gate and the pair's input weight in the epilogue
-        ops.expert_gemm(act, h, self.w_gu, slots, tile_expert, tile, s.top, self.epilogue, scale, s.limit)
+        ops.expert_gemm(act, h, self.w_gu, slots, tile_expert, tile, s.top, self.epilogue, scale, s.limit, pairs=P)
         ye = torch.empty(cap, self.hidden, device=dev, dtype=h.dtype)
-        ops.expert_gemm(ye, act, self.w_down, slots, tile_expert, tile, 0, 0)
+        ops.expert_gemm(ye, act, self.w_down, slots, tile_expert, tile, 0, 0, pairs=P)
         return ye, pair_slot, ids, wts, s.experts, h, self._shared(h)
 
     def _shared(self, h: torch.Tensor):
@@ -970,13 +968,16 @@ class RoutedMoE:
         n = self.spec.shared_ff
         if not n and not self.side_rows:
             return None
-        g = F.linear(h, self.ws_gu)
+        act = "silu_mul" if self.spec.act == "silu" else "clamped_glu"
+        if not self.side_rows:
+            return self.ops.linear(self.ops.linear(h, self.ws_gu, act=act, c0=self.spec.shared_limit), self.ws_down)
+        g = self.ops.linear(h, self.ws_gu)
         _side(self, g)
         if not n:
             return None
         a = torch.empty(h.shape[0], n, device=h.device, dtype=h.dtype)
-        self.ops.activation(a, g[:, :2 * n], "silu_mul" if self.spec.act == "silu" else "clamped_glu", self.spec.shared_limit)
-        return F.linear(a, self.ws_down)
+        self.ops.activation(a, g[:, :2 * n], act, self.spec.shared_limit)
+        return self.ops.linear(a, self.ws_down)
 
     def _packed_ok(self, h: torch.Tensor, P: int, nb: int) -> bool:
         from ..ops import core_built

@@ -15,6 +15,7 @@ import os
 import threading
 
 import torch
+import torch.nn.functional as F
 
 from . import reference as ref
 
@@ -371,6 +372,56 @@ class KernelOps:
         self._delta.delta_rule(out, state[0], proj, wl, a_b, w0, norm_w, meta.seq_cu, meta.seq_ctx, meta.seq_state,
                              scratch, sp.heads, sp.dim, eps, out_scale)
 
+    # ---- dense layers
+    SKINNY_ROWS = 64
+    GLU_ACTS = ("silu_mul", "clamped_glu")
+
+    @staticmethod
+    def skinny_pays(rows: int, cols: int, k: int, glu: bool = False) -> bool:
+        """Whether ``skinny_linear`` is expected to be faster than the vendor's GEMM for ``rows`` x ``cols`` results (``cols``
+        over all batches). Both sides in us, fitted to cold weights of 1024 .. 32000 columns and k of 1024 .. 12288: ours is
+        a latency plus the weights at 5 TB/s, or what a workgroup of 16 columns reads (weights and rows) at 34 KB per us and
+        compute unit; the vendor's is hardly ever below 10.5 (7.5 up to k = 1024) and streams large weights at 4.2 TB/s.
+        Examples, ours / vendor: 2048 x 2048 with 1, 16, 32, 48 rows 4.7 / 11.0, 6.2 / 11.1, 8.0 / 11.2, 10.2 / 11.2; 6144 x
+        2048 with 1, 16, 32, 48 rows 7.7 / 12.6, 10.3 / 12.3, 13.7 / 12.3, 17.8 / 12.9; 2048 x 6144 with 1, 16 rows 9.0 / 10.9,
+        13.2 / 11.1; 3072 x 1024 with 1, 48 rows 3.7 / 7.3, 6.7 / 11.1; 32000 x 2048 with 1, 16, 32 rows 26 / 34, 34 / 34, 46 / 34."""
+        weights = 2.0 * cols * k
+        per_cu = max(1.0, cols / (32 if glu else 16) / 256) * 2.0 * k * ((32 if glu else 16) + rows)
+        return 3.2 + max(weights / 5.0e6, per_cu / 34e3) < max(7.5 if k <= 1024 else 10.5, 3.2 + weights / 4.2e6)
+
+    def _skinny_ok(self, x, w) -> bool:
+        """The shapes, types and alignment that ``skinny_linear`` takes."""
+        return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == w.dim() and 0 < x.shape[-2] <= self.SKINNY_ROWS
+                and x.shape[-1] % 8 == 0 and x.stride(-1) == 1 and x.stride(-2) % 8 == 0 and x.stride(0) % 8 == 0
+                and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
+
+    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0):
+        """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands. A few bf16 rows run the
+        weight-streaming kernel with the activation in its epilogue, anything else the vendor's GEMM and a second launch."""
+        if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or bias.dtype == x.dtype):
+            glu = act in self.GLU_ACTS
+            T, N, K = x.shape[0], w.shape[0], w.shape[1]
+            if self.skinny_pays(T, N, K, glu):
+                out = torch.empty(T, N // 2 if glu else N, device=x.device, dtype=torch.float32 if out_f32 else x.dtype)
+                self._moe_lib.skinny_linear(out, x, w, bias, -1 if act is None else self.ACTIVATIONS[act], c0, c1)
+                return out
+        if out_f32 and x.dtype != torch.float32:
+            y = torch.mm(x, w.t(), out_dtype=torch.float32)
+        else:
+            y = F.linear(x, w, bias)
+        if act is None:
+            return y
+        out = torch.empty(*y.shape[:-1], y.shape[-1] // 2, device=y.device, dtype=y.dtype) if act in self.GLU_ACTS else y
+        return self.activation(out, y, act, c0, c1)
+
+    def linear_heads(self, out, x, w) -> bool:
+        """out[h] = x[h] . w[h]^T for a few bf16 rows (x [heads, T, K], w [heads, N, K], out [heads, T, N], strided rows);
+        False, and nothing done, where the vendor's batched GEMM is the one to run."""
+        if not (x.dim() == 3 and self._skinny_ok(x, w) and self.skinny_pays(x.shape[1], w.shape[0] * w.shape[1], w.shape[2])):
+            return False
+        self._moe_lib.skinny_linear(out, x, w, None, -1, 0.0, 0.0)
+        return True
+
     ACTIVATIONS = {"tanh": 0, "xielu": 1, "relu2": 2, "silu_mul": 3, "clamped_glu": 4, "softcap": 5}
 
     def activation(self, out, x, kind, c0=0.0, c1=0.0):
@@ -476,10 +527,11 @@ class KernelOps:
         te = torch.searchsorted(ends, t, right=True)
         tile_expert.copy_(torch.where(te < E, te, torch.full_like(te, -1)).to(torch.int32))
 
-    def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0):
+    def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0, pairs=0):
         """act: False / 0 none, True / 1 squared ReLU, 2: w = [gate rows; up rows], out = silu(gate) * up, 3: the same
-        with the gate clamped at ``limit``; ``row_scale`` fp32 [pairs] multiplies each pair's product before it."""
-        self._moe_lib.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, int(act), row_scale, limit)
+        with the gate clamped at ``limit``; ``row_scale`` fp32 [pairs] multiplies each pair's product before it;
+        ``pairs``: how many (token, choice) pairs the tiles hold, where the caller knows (the choice of kernel)."""
+        self._moe_lib.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, int(act), row_scale, limit, pairs)
 
     # ---- norms before and after every sublayer (csrc/kernels/seq/sandwich.hip)
     def sandwich_update(self, out, residual, w_next, eps, y=None, w_post=None, mult=1.0, table=None):
@@ -646,7 +698,7 @@ class ReferenceOps:
     def moe_align(self, experts, E, tile, slots, tile_expert, pair_slot):
         ref.moe_align(experts, E, tile, slots, tile_expert, pair_slot)
 
-    def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0):
+    def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0, pairs=0):
         ref.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, int(act), row_scale, limit)
 
     def stream_update(self, out, dst, src, coef, w, eps, y1=None, y2=None):
@@ -722,6 +774,18 @@ class ReferenceOps:
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
         ref.delta_rule(out, state[0], proj, wl, a_b, w0, norm_w, sp, eps, meta.seq_cu, meta.seq_ctx,
                        meta.seq_state, out_scale)
+
+    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0):
+        if out_f32 and x.dtype != torch.float32:
+            x, w = x.float(), w.float()
+        y = F.linear(x, w, bias)
+        if act is None:
+            return y
+        out = y.new_empty(*y.shape[:-1], y.shape[-1] // 2) if act in KernelOps.GLU_ACTS else y
+        return self.activation(out, y, act, c0, c1)
+
+    def linear_heads(self, out, x, w) -> bool:
+        return False
 
     def activation(self, out, x, kind, c0=0.0, c1=0.0):
         ref.activation(out, x, kind, c0, c1)

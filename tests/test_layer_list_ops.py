@@ -84,3 +84,113 @@ def test_softcap(shape, dev):
     get_ops(dev).activation(y, y, "softcap", 25.0)
     # division, tanh and product: a few units in the last place of numbers up to 25
     assert (y.cpu().double() - want).abs().max() <= 25 * 4 * 2.0 ** -23
+
+
+# ------------------------------------------------------------------ dense layers of a few rows
+def dense_case(B, M, N, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(B, M, K, generator=g).bfloat16(), (torch.randn(B, N, K, generator=g) / K ** 0.5).bfloat16()
+
+
+def act64(z, act, c0, c1):
+    """The activations in 64 bits."""
+    if act in ("silu_mul", "clamped_glu"):
+        g, u = z.chunk(2, -1)
+        if act == "silu_mul":
+            return g * torch.sigmoid(g) * u
+        g, u = g.clamp(max=c0), u.clamp(-c0, c0)
+        return g * torch.sigmoid(1.702 * g) * (u + 1)
+    return {None: lambda: z, "tanh": z.tanh, "relu2": lambda: z.relu() ** 2, "softcap": lambda: torch.tanh(z / c0) * c0,
+            "xielu": lambda: torch.where(z > 0, c0 * z * z + z / 2, c1 * (torch.expm1(z.clamp(max=0)) - z) + z / 2)}[act]()
+
+
+def close_to(got, want, x, w, scale=1.0):
+    """A bf16 rounding of the result, and 32-bit sums of K products taken in any order (times the activation's slope)."""
+    K = x.shape[-1]
+    err = scale * K * 2.0 ** -24 * torch.matmul(x.double().abs(), w.double().abs().transpose(-1, -2)).max()
+    tol = 2.0 ** -8 if got.dtype == torch.bfloat16 else 2.0 ** -21
+    assert ((got.double().cpu() - want).abs() <= tol * want.abs() + err + 1e-6).all()
+
+
+@gpu
+@pytest.mark.parametrize("M", [1, 3, 5, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(1, 8), (16, 64), (40, 72), (17, 512), (96, 520), (33, 1024), (48, 1032), (130, 2048), (16, 6152)])
+def test_skinny_linear(M, N, K):
+    """Row tiles, columns and k that fill the tiles of 16 rows, 16 columns and 64 k partly; bias, 32-bit results, row strides."""
+    (x,), (w,) = dense_case(1, M, N, K, M + N + K)
+    ops = get_ops("cuda")
+    want = x.double() @ w.double().T
+    wide = torch.zeros(M, K + 24, dtype=torch.bfloat16, device="cuda")
+    wide[:, 8:8 + K] = x.cuda()
+    out = torch.full((M, N + 5), 7.0, device="cuda")
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(N)).bfloat16()
+    ops._moe_lib.skinny_linear(out[:, :N], wide[:, 8:8 + K], w.cuda(), None, -1, 0.0, 0.0)
+    close_to(out[:, :N], want, x, w)
+    assert (out[:, N:] == 7.0).all()
+    half = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    ops._moe_lib.skinny_linear(half, x.cuda(), w.cuda(), bias.cuda(), -1, 0.0, 0.0)
+    close_to(half, want + bias.double(), x, w)
+
+
+@gpu
+@pytest.mark.parametrize("M", [1, 16, 31, 50])
+@pytest.mark.parametrize("act,c0,c1", [("tanh", 0, 0), ("xielu", 0.8, 0.7), ("relu2", 0, 0), ("silu_mul", 0, 0), ("clamped_glu", 1.0, 0),
+                                       ("softcap", 2.0, 0)])
+def test_linear_with_activation(M, act, c0, c1):
+    """``ops.linear`` with an activation in the kernel's epilogue, and beside it (rows past the kernel's)."""
+    ops = get_ops("cuda")
+    ops.norm_library = "delta"
+    for rows in (M, 70):
+        (x,), (w,) = dense_case(1, rows, 96, 520, M)
+        z = x.double() @ w.double().T
+        got = ops.linear(x.cuda(), w.cuda(), act=act, c0=c0, c1=c1)
+        want = act64(z, act, c0, c1)
+        if rows == M:
+            assert ops.skinny_pays(M, 96, 520, act in ops.GLU_ACTS)
+            close_to(got, want, x, w, scale=12.0)
+        else:   # the product is rounded to bf16 before the activation, whose slope is below 12 for numbers up to 5
+            assert ((got.double().cpu() - want).abs() <= 12 * 2.0 ** -8 * z.abs().max()).all()
+
+
+@gpu
+@pytest.mark.parametrize("B,M,N,K", [(3, 1, 40, 16), (16, 17, 512, 128), (5, 64, 24, 520), (2, 33, 128, 512)])
+def test_skinny_heads(B, M, N, K):
+    """Batches with a stride of their own: heads side by side per row, in and out."""
+    x, w = dense_case(B, M, N, K, B + M)
+    rows = x.transpose(0, 1).contiguous().cuda()          # [M, B, K]
+    out = torch.empty(M, B, N, dtype=torch.bfloat16, device="cuda")
+    assert get_ops("cuda").linear_heads(out.transpose(0, 1), rows.transpose(0, 1), w.cuda())
+    close_to(out.transpose(0, 1), x.double() @ w.double().transpose(1, 2), x, w)
+
+
+def test_linear_reference():
+    (x,), (w,) = dense_case(1, 5, 32, 64, 0)
+    ops = get_ops("cpu")
+    z = x.double() @ w.double().T
+    assert ops.linear(x, w, out_f32=True).dtype == torch.float32
+    for act, c0 in ((None, 0), ("silu_mul", 0), ("softcap", 2.0)):
+        assert (ops.linear(x.float(), w.float(), act=act, c0=c0) - act64(z, act, c0, 0)).abs().max() < 1e-5
+
+
+# ------------------------------------------------------------------ experts
+@gpu
+@pytest.mark.parametrize("tokens,E,top", [(1, 16, 2), (2, 3, 1), (48, 16, 2), (40, 2, 2), (300, 4, 2)])
+@pytest.mark.parametrize("N,K", [(64, 40), (1024, 2048), (48, 512)])
+@pytest.mark.parametrize("act", [0, 1, 2, 3])
+def test_expert_gemm_tiles_of_few_rows(tokens, E, top, N, K, act):
+    """The weight-streaming kernel (few live slots per tile, unused tiles) and the tile kernel, gathered and not."""
+    g = torch.Generator().manual_seed(tokens + N)
+    x = torch.randn(tokens, K, generator=g).bfloat16()
+    w = (torch.randn(E, N, K, generator=g) / K ** 0.5).bfloat16()
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(tokens)]).int()
+    scale = torch.rand(tokens * top, generator=g) if act >= 2 else None
+    ops, P, tile = get_ops("cuda"), tokens * top, 32
+    cap = -(-(P + E * (tile - 1)) // tile) * tile
+    slots, tiles, pair = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (cap, cap // tile, P))
+    ops.moe_align(ids.view(-1).cuda(), E, tile, slots, tiles, pair)
+    out = torch.empty(cap, N // 2 if act >= 2 else N, dtype=torch.bfloat16, device="cuda")
+    ops.expert_gemm(out, x.cuda(), w.cuda(), slots, tiles, tile, top, act, scale.cuda() if scale is not None else None, 1.0, P)
+    xp, wp = x.repeat_interleave(top, 0), w[ids.view(-1).long()]
+    z = torch.einsum("pk,pnk->pn", xp.double(), wp.double()) * (scale.double()[:, None] if scale is not None else 1.0)
+    want = act64(z, {0: None, 1: "relu2", 2: "silu_mul", 3: "clamped_glu"}[act], 1.0, 0.0)
+    close_to(out[pair.long()], want, x, w.view(-1, K), scale=12.0)
