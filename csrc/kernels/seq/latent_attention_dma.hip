@@ -1,0 +1,508 @@
+// Latent attention on the matrix cores for cache rows of 128, 256 or 512 latent dims and 64 rotary ones (bf16): the
+// products of latent_attention_mfma.hip with the cache rows copied straight into LDS.
+//
+// That kernel loads a 32-key tile into registers, stores it to LDS and only then multiplies: a tile waits for its page
+// lookup and for its rows (about 3 us) before 0.5 us of products, its operand reads wait one by one (no registers left),
+// and the V operand of P . V is gathered from LDS two bytes at a time. Here
+//   * global_load_lds brings the rows into one of four LDS buffers, two tiles ahead of the products;
+//   * a buffer holds [32][latent dims] and [32][64 rotary dims]; the eight 16-byte chunks of every 128 bytes are
+//     XOR-swizzled by the key, by choosing which chunk a lane copies, so that both the row-wise operand reads of
+//     S = K . Q^T and the transposing reads below spread over the banks without padding;
+//   * the V^T operand comes from ds_read_tr16_b64: within 16 lanes, lane l gets element l % 4 of the 8 bytes that lane
+//     4 j + l / 4 addresses, j = 0 .. 3. Lane (c, g) addresses key 16 h + 4 g + c / 4, dims 4 (c % 4) .. + 3 and so
+//     receives keys 16 h + 4 g + 0 .. 3 of dim c: half of an MFMA operand in the key order of P;
+//   * waves 0 - 3 (one per SIMD) compute the scores and softmax of 16 rows each, waves 4 - 7 the P . V of the previous tile,
+//     DV / 4 latent dims each for all 64 rows: the softmax of one tile runs beside the products of another, neither half
+//     holds the other's registers (queries 72, outputs 128 per lane), and a tile costs one barrier;
+//   * the queries' rotary part is rotated when the operands are loaded (its halves meet in one lane), no pass of its own.
+// What bounds it: LDS reads (every K row goes to four waves: 181 KB per tile of 64 rows against 1088 cycles of products).
+// @NUMBERS@
+// latent_dma_decode_kernel serves decode rows: a workgroup takes 16 heads of one sequence and a run of keys, 64 of them
+// at a time; its waves split the keys for S and the latent dims for P . V. @DECODE@
+#include "seq_common.h"
+#include "hipserve/seq_kernels.h"
+
+namespace hipserve {
+namespace {
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
+
+constexpr int kKeys = 32, kRot = 64, kPLd = 40;   // kPLd: row stride of P in elements (16-byte rows, padded)
+constexpr float kLog2e = 1.44269504088896341f;
+
+// All LDS and vector memory operations issued so far are done, then every wave of the workgroup is here.
+HS_DEVICE void barrier_all() {
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+// All but the wave's last N vector memory operations are done.
+template <int N>
+HS_DEVICE void copied_but() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
+}
+// 1 KB from the lanes' addresses to LDS, 16 bytes per lane side by side, asynchronously. Written out because the compiler
+// would otherwise wait for every copy in flight before the next transposing read; the waits are the callers' copied_but.
+HS_DEVICE void copy_1k(const unsigned short* src, const unsigned char* lds) {
+  const unsigned at = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds;
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(at)), "v"(src) : "memory");   // nothing else in this file uses m0
+}
+// The same for LDS operations alone: copies into LDS may still be in flight.
+HS_DEVICE void barrier_lds() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// K tile rows in LDS: [KEYS][DV] then [KEYS][64]; 16-byte chunk ch of key k sits at chunk ch ^ (k & 7).
+template <int DV, int KEYS> struct Tile {
+  static constexpr int kMain = KEYS * DV * 2, kBytes = kMain + KEYS * kRot * 2;
+  static HS_DEVICE int main_at(int k, int ch) { return k * DV * 2 + ((ch ^ (k & 7)) << 4); }
+  static HS_DEVICE int rot_at(int k, int ch) { return kMain + k * kRot * 2 + ((ch ^ (k & 7)) << 4); }
+  // The wave copies keys 8 w .. 8 w + 7 of the tile; `row` = element offset of key `lane` % KEYS's cache row.
+  static HS_DEVICE void copy(unsigned char* lds, const unsigned short* cache, long row, int w, int lane) {
+    constexpr int kPer = 512 / DV, kChunks = DV / 8;   // keys and 16-byte chunks of a key in one 1 KB copy
+#pragma unroll
+    for (int i = 0; i < 8 / kPer; ++i) {
+      const int k = 8 * w + i * kPer + lane / kChunks, ch = (lane % kChunks) ^ (k & 7);
+      const unsigned short* src = cache + __shfl(row, k, 64) + 8 * ch;
+      copy_1k(src, lds + (8 * w + i * kPer) * DV * 2);
+    }
+    const int k = 8 * w + lane / 8, ch = (lane & 7) ^ (k & 7);
+    const unsigned short* src = cache + __shfl(row, k, 64) + DV + 8 * ch;
+    copy_1k(src, lds + kMain + 8 * w * kRot * 2);
+  }
+  // The lane's places in a tile: the swizzle touches three bits of the chunk, so two (keys) and up to four (values)
+  // offsets serve all operands, with constants added.
+  static constexpr int NPW = DV / 64, JB = NPW < 4 ? NPW : 4;   // 16-dim value tiles per wave
+  struct Places { int key[2], rot[2], val[JB]; };
+  static HS_DEVICE Places places(int wave, int c, int g) {
+    Places p;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) { p.key[i] = main_at(c, 4 * i + g); p.rot[i] = rot_at(c, 4 * i + g); }
+#pragma unroll
+    for (int j = 0; j < JB; ++j)
+      p.val[j] = main_at(4 * g + (c >> 2), 2 * (wave * NPW + j) + ((c & 3) >> 1)) + 8 * (c & 1);
+    return p;
+  }
+  // MFMA operand of 32-dim step ks of key rows k0 + c (k0 a multiple of 16): dims 32 ks + 8 g .. + 7
+  static HS_DEVICE bf16x8 key_operand(const unsigned char* lds, const Places& p, int k0, int ks) {
+    const int at = ks < DV / 32 ? p.key[ks & 1] + (ks >> 1) * 128 + k0 * DV * 2 : p.rot[ks & 1] + k0 * kRot * 2;
+    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(lds + at));
+  }
+  // MFMA operand of the wave's value tile j against keys k0 .. k0 + 31 (k0 a multiple of 32): lane (c, g) holds dim c,
+  // keys k0 + 16 (e / 4) + 4 g + e % 4
+  static HS_DEVICE bf16x8 value_operand(unsigned char* lds, const Places& p, int k0, int j) {
+    s16x4 h[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      h[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+          (lds_s16x4)(lds + p.val[j % JB] + (j / JB) * 128 + (k0 + 16 * i) * DV * 2));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+};
+
+// Query operands of one (token, head) row: the latent part from qc, the last 64 dims from qc too, or rotated here from
+// the projection's rotary part (q_rot: its 64 numbers; entry i pairs with i + 32, angle pos * inv_freq[i]).
+template <int DV>
+HS_DEVICE void load_query(bf16x8 (&qf)[DV / 32 + 2], bool act, const unsigned short* qc, const unsigned short* q_rot, float pos,
+                          const float* __restrict__ inv_freq, int g) {
+  constexpr int KL = DV / 32;
+  const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+  for (int ks = 0; ks < KL; ++ks)
+    qf[ks] = __builtin_bit_cast(bf16x8, act ? *reinterpret_cast<const u16x8*>(qc + 32 * ks + 8 * g) : zero);
+  u16x8 a = zero, b = zero;
+  if (act) {
+    const unsigned short* src = q_rot != nullptr ? q_rot : qc + DV;
+    a = *reinterpret_cast<const u16x8*>(src + 8 * g);
+    b = *reinterpret_cast<const u16x8*>(src + 32 + 8 * g);
+  }
+  if (q_rot != nullptr && act) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      float sn, cs;
+      sincosf(pos * inv_freq[8 * g + e], &sn, &cs);
+      const float u = bf16_to_f32(a[e]), w = bf16_to_f32(b[e]);
+      a[e] = f32_to_bf16(u * cs - w * sn);
+      b[e] = f32_to_bf16(w * cs + u * sn);
+    }
+  }
+  qf[KL] = __builtin_bit_cast(bf16x8, a);
+  qf[KL + 1] = __builtin_bit_cast(bf16x8, b);
+}
+
+// 64 (token, head) rows of consecutive tokens of one sequence. Iteration i: waves 0 - 3 turn tile i into P, waves 4 - 7 add
+// tile i - 1 to the outputs, all copy tile i + 2 into the buffer that tile i - 2 has left.
+template <int DV>
+__global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
+    unsigned short* __restrict__ o_lat, const unsigned short* __restrict__ qc, const unsigned short* __restrict__ q,
+    const long* __restrict__ positions, const float* __restrict__ inv_freq, const unsigned short* __restrict__ proj,
+    long proj_ld, const unsigned short* __restrict__ cache, int block_size, const int* __restrict__ seq_cu,
+    const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0, int seq1, int tq, int hc,
+    int T_rows, int heads, int dim, int gate_off, float scale, int window) {
+  using KT = Tile<DV, kKeys>;
+  constexpr int KS = DV / 32 + 2, NPW = KT::NPW, Dk = DV + kRot;
+  constexpr int kMainCopies = DV / 128;   // a wave's share of a tile: 4 keys of the latent part, 1 KB per copy
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  unsigned short* p_lds = reinterpret_cast<unsigned short*>(smem + 4 * KT::kBytes);   // [2][64][kPLd], MFMA k order
+  float* alpha = reinterpret_cast<float*>(p_lds + 2 * 64 * kPLd);                     // [2][64]
+  float* l_lds = alpha + 2 * 64;                                                      // [64] (epilogue)
+  int s, tok0;
+  if (!find_row_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int r0 = seq_cu[s], n = seq_cu[s + 1] - r0, ctx = seq_ctx[s];
+  const int ntok = min(tq, n - tok0);
+  const int h0 = blockIdx.y * hc, nh = min(hc, heads - h0);
+  const int p_first = ctx - n + tok0, hi = p_first + ntok - 1;
+  // tiles start at multiples of 32: a wave's 4 keys (8 of the rotary part) lie on one page, looked up by the scalar unit
+  const int lo = (window > 0 ? max(0, p_first - window + 1) : 0) & ~(kKeys - 1);
+  const int ntiles = (hi - lo) / kKeys + 1;
+  const int* bt = seq_bt + (long)s * bt_width;
+  // the first of the keys 4 wave .. + 3 of tile t that exists, and its page; keys past the last one are the last one again
+  auto page_of = [&](int t, int k) { return bt[min(lo + t * kKeys + k, hi) / block_size]; };
+  auto copy = [&](int t, int page, int page_rot) {
+    unsigned char* lds = smem + (t & 3) * KT::kBytes;
+    const int j0 = lo + t * kKeys;
+    constexpr int kPer = 512 / DV, kChunks = DV / 8;   // keys and 16-byte chunks of a key per copy
+#pragma unroll
+    for (int i = 0; i < kMainCopies; ++i) {
+      const int k = 4 * wave + i * kPer + lane / kChunks, ch = (lane % kChunks) ^ (k & 7);
+      const unsigned short* src = cache + ((long)page * block_size + min(j0 + k, hi) % block_size) * Dk + 8 * ch;
+      copy_1k(src, lds + (4 * wave + i * kPer) * DV * 2);
+    }
+    if (wave < 4) {
+      const int k = 8 * wave + lane / 8, ch = (lane & 7) ^ (k & 7);
+      const unsigned short* src = cache + ((long)page_rot * block_size + min(j0 + k, hi) % block_size) * Dk + DV + 8 * ch;
+      copy_1k(src, lds + KT::kMain + 8 * wave * kRot * 2);
+    }
+  };
+  const int krot = 8 * (wave & 3);
+  copy(0, page_of(0, 4 * wave), page_of(0, krot));
+  if (ntiles > 1) copy(1, page_of(1, 4 * wave), page_of(1, krot));
+  int page = page_of(2, 4 * wave), page_rot = page_of(2, krot);   // clamped: always an existing page
+  const typename KT::Places at = KT::places(wave & 3, c, g);
+  if (wave < 4) {
+    const int sr = 16 * wave + c, srt = sr / hc, srh = sr % hc;
+    const bool sact = srt < ntok && srh < nh;
+    const long strow = r0 + tok0 + (sact ? srt : 0);
+    const int shead = h0 + (sact ? srh : 0);
+    const int spos = p_first + srt;
+    const int s_lo = window > 0 ? max(0, spos - window + 1) : 0;
+    bf16x8 qf[KS];
+    load_query<DV>(qf, sact, qc + ((long)shead * T_rows + strow) * Dk,
+                   q != nullptr ? q + strow * heads * (dim + kRot) + (long)shead * (dim + kRot) + dim : nullptr,
+                   (float)positions[strow], inv_freq, g);
+    float m_run = -INFINITY, l_run = 0.f;
+    const float scale2 = scale * kLog2e;
+    for (int i = 0; i <= ntiles; ++i) {
+      if (i + 1 < ntiles) copied_but<kMainCopies + 1>();   // tile i + 1 may still be on its way
+      else copied_but<0>();
+      barrier_lds();
+      if (i + 2 < ntiles) {
+        copy(i + 2, page, page_rot);
+        page = page_of(i + 3, 4 * wave);
+        page_rot = page_of(i + 3, krot);
+      }
+      if (i == ntiles) break;
+      const unsigned char* kt = smem + (i & 3) * KT::kBytes;
+      const int j0 = lo + i * kKeys;
+      f32x4 sc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+      // the key operands are read a batch of steps ahead of their products
+      constexpr int kBatch = 6, kBatches = (KS + kBatch - 1) / kBatch;
+      bf16x8 ka[2][kBatch][2];
+#pragma unroll
+      for (int b = 0; b <= kBatches; ++b) {
+        if (b < kBatches)
+#pragma unroll
+          for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+              if (b * kBatch + u < KS) ka[b & 1][u][nt] = KT::key_operand(kt, at, 16 * nt, b * kBatch + u);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b > 0)
+#pragma unroll
+          for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+            for (int nt = 0; nt < 2; ++nt)
+              if ((b - 1) * kBatch + u < KS)
+                sc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[(b - 1) & 1][u][nt], qf[(b - 1) * kBatch + u], sc[nt], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // masked online softmax (log2 domain) of row sr: lane (c, g) holds keys 16 nt + 4 g + i
+      float v[8], mx = -INFINITY;
+      if (__all(sact && j0 + kKeys - 1 <= spos && j0 >= s_lo)) {   // every row of the wave sees the whole tile
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { v[e] = sc[e >> 2][e & 3] * scale2; mx = fmaxf(mx, v[e]); }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int j = j0 + 16 * (e >> 2) + 4 * g + (e & 3);
+          v[e] = sact && j <= spos && j >= s_lo ? sc[e >> 2][e & 3] * scale2 : -INFINITY;
+          mx = fmaxf(mx, v[e]);
+        }
+      }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      const float mn = fmaxf(m_run, mx);
+      float sum = 0.f;
+      u16x8 pk;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float p = mn > -INFINITY ? __builtin_amdgcn_exp2f(v[e] - mn) : 0.f;
+        pk[e] = f32_to_bf16(p);   // rounded: what is multiplied, and its sum
+        sum += bf16_to_f32(pk[e]);
+      }
+      sum += __shfl_xor(sum, 16, 64);
+      sum += __shfl_xor(sum, 32, 64);
+      *reinterpret_cast<u16x8*>(p_lds + ((i & 1) * 64 + sr) * kPLd + 8 * g) = pk;
+      const float al = mn > -INFINITY ? __builtin_amdgcn_exp2f(m_run - mn) : 1.f;  // m_run = -inf: 0
+      if (g == 0) alpha[(i & 1) * 64 + sr] = al;
+      l_run = l_run * al + sum;
+      m_run = mn;
+    }
+    if (g == 0) {   // gate / softmax sum of the row
+      float f = 0.f;
+      if (sact && l_run > 0.f) {
+        f = 1.f / l_run;
+        if (gate_off >= 0) f *= sigmoid_f(bf16_to_f32(proj[strow * proj_ld + gate_off + shead]));
+      }
+      l_lds[sr] = f;
+    }
+    barrier_lds();
+    return;
+  }
+  f32x4 acc[4][NPW];
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+    for (int j = 0; j < NPW; ++j) acc[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i <= ntiles; ++i) {
+    if (i + 1 < ntiles) copied_but<kMainCopies>();
+    else copied_but<0>();
+    barrier_lds();
+    if (i + 2 < ntiles) {
+      copy(i + 2, page, page_rot);
+      page = page_of(i + 3, 4 * wave);
+    }
+    if (i == 0) continue;
+    unsigned char* kt = smem + ((i - 1) & 3) * KT::kBytes;
+    const unsigned short* pt = p_lds + ((i - 1) & 1) * 64 * kPLd;
+    bf16x8 pb[4], va[NPW];
+    float al[4];
+    bool rescale = false;
+#pragma unroll
+    for (int mt = 0; mt < 4; ++mt) {
+      pb[mt] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(pt + (16 * mt + c) * kPLd + 8 * g));
+      al[mt] = alpha[((i - 1) & 1) * 64 + 16 * mt + c];
+      rescale |= al[mt] != 1.f;
+    }
+#pragma unroll
+    for (int j = 0; j < NPW; ++j) va[j] = KT::value_operand(kt, at, 0, j);
+    __builtin_amdgcn_sched_barrier(0);
+    if (__any(rescale)) {   // the running maxima settle after a few tiles: most tiles skip this
+#pragma unroll
+      for (int j = 0; j < NPW; ++j)
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) acc[mt][j] *= al[mt];
+    }
+#pragma unroll
+    for (int j = 0; j < NPW; ++j)
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va[j], pb[mt], acc[mt][j], 0, 0, 0);
+  }
+  barrier_lds();
+  // lane (c, g) holds latent dims 16 nt + 4 g .. + 3 of row 16 mt + c
+#pragma unroll
+  for (int mt = 0; mt < 4; ++mt) {
+    const int r = 16 * mt + c, rt = r / hc, rh = r % hc;
+    if (rt >= ntok || rh >= nh) continue;
+    const float f = l_lds[r];
+    unsigned short* dst = o_lat + ((long)(h0 + rh) * T_rows + r0 + tok0 + rt) * DV + 16 * NPW * (wave - 4) + 4 * g;
+#pragma unroll
+    for (int j = 0; j < NPW; ++j) {
+      u16x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = f32_to_bf16(acc[mt][j][e] * f);
+      *reinterpret_cast<u16x4*>(dst + 16 * j) = o;
+    }
+  }
+}
+
+// Decode rows, one per sequence: 16 heads of sequence seq0 + blockIdx.x against the run blockIdx.z of part_keys keys,
+// 64 at a time. Wave w: scores of keys 16 w .., P . V of the latent dims DV / 4 w ... With runs the unnormalised
+// outputs and (max, sum) go to ws_acc / ws_ml.
+template <int DV>
+__global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
+    unsigned short* __restrict__ o_lat, const unsigned short* __restrict__ qc, const unsigned short* __restrict__ q,
+    const long* __restrict__ positions, const float* __restrict__ inv_freq, const unsigned short* __restrict__ proj,
+    long proj_ld, const unsigned short* __restrict__ cache, int block_size, const int* __restrict__ seq_cu,
+    const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0, int T_rows, int heads,
+    int dim, int gate_off, float scale, int window, int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
+    int row_base, int ws_rows) {
+  constexpr int kTile = 64, kPd = kTile + 8;   // kPd: row stride of P in elements
+  using KT = Tile<DV, kTile>;
+  constexpr int KS = DV / 32 + 2, NPW = DV / 64, Dk = DV + kRot;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  unsigned short* p_lds = reinterpret_cast<unsigned short*>(smem + KT::kBytes);   // [16][kPd], MFMA k order
+  float* mw = reinterpret_cast<float*>(p_lds + 16 * kPd);                         // [4][16] the waves' maxima
+  float* lw = mw + 64;                                                            // [4][16] the waves' sums
+  const int s = seq0 + blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+  const int head = blockIdx.y * 16 + c;
+  const bool act = head < heads;
+  const long trow = seq_cu[s];
+  const int pos = seq_ctx[s] - 1;
+  const int lo = (window > 0 ? max(0, pos - window + 1) : 0) + blockIdx.z * part_keys;
+  const int hi = gridDim.z > 1 ? min(pos, lo + part_keys - 1) : pos;
+  const bool partial = gridDim.z > 1;
+  const long wrow = ((long)blockIdx.z * heads + (act ? head : 0)) * ws_rows + (trow - row_base);
+  if (lo > hi) {   // an empty run: its weight in the merge is 0
+    if (partial && act && wave == 0 && g == 0) { ws_ml[2 * wrow] = -INFINITY; ws_ml[2 * wrow + 1] = 0.f; }
+    return;
+  }
+  const int* bt = seq_bt + (long)s * bt_width;
+  auto row_of = [&](int j0) {
+    const int j = min(j0 + lane, hi);
+    return ((long)bt[j / block_size] * block_size + j % block_size) * Dk;
+  };
+  auto copy = [&](int j0) {
+    const long row = row_of(j0);
+    KT::copy(smem, cache, row, 2 * wave, lane);
+    KT::copy(smem, cache, row, 2 * wave + 1, lane);
+  };
+  copy(lo);
+  bf16x8 qf[KS];
+  load_query<DV>(qf, act, qc + ((long)(act ? head : 0) * T_rows + trow) * Dk,
+                 q != nullptr ? q + trow * heads * (dim + kRot) + (long)(act ? head : 0) * (dim + kRot) + dim : nullptr,
+                 (float)positions[trow], inv_freq, g);
+  f32x4 acc[NPW];
+#pragma unroll
+  for (int j = 0; j < NPW; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;   // of row c, the same in every wave
+  const float scale2 = scale * kLog2e;
+  const typename KT::Places at = KT::places(wave, c, g);
+  for (int j0 = lo; j0 <= hi; j0 += kTile) {
+    barrier_all();
+    f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(KT::key_operand(smem, at, 16 * wave, ks), qf[ks], sc, 0, 0, 0);
+    float v[4], mx = -INFINITY;   // keys 16 wave + 4 g + i
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v[i] = act && j0 + 16 * wave + 4 * g + i <= hi ? sc[i] * scale2 : -INFINITY;
+      mx = fmaxf(mx, v[i]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (g == 0) mw[16 * wave + c] = mx;
+    barrier_lds();
+    const float mn = fmaxf(fmaxf(fmaxf(mw[c], mw[16 + c]), fmaxf(mw[32 + c], mw[48 + c])), m_run);
+    float sum = 0.f;
+    u16x4 pk;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      pk[i] = f32_to_bf16(mn > -INFINITY ? __builtin_amdgcn_exp2f(v[i] - mn) : 0.f);
+      sum += bf16_to_f32(pk[i]);
+    }
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    // key 32 kk + 16 h + 4 g + i sits at column 32 kk + 8 g + 4 h + i (kk = wave / 2, h = wave % 2)
+    *reinterpret_cast<u16x4*>(p_lds + c * kPd + 32 * (wave >> 1) + 8 * g + 4 * (wave & 1)) = pk;
+    if (g == 0) lw[16 * wave + c] = sum;
+    const float al = mn > -INFINITY ? __builtin_amdgcn_exp2f(m_run - mn) : 1.f;
+    m_run = mn;
+    barrier_lds();
+    l_run = l_run * al + (lw[c] + lw[16 + c]) + (lw[32 + c] + lw[48 + c]);
+#pragma unroll
+    for (int j = 0; j < NPW; ++j) acc[j] *= al;
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(p_lds + c * kPd + 32 * kk + 8 * g));
+#pragma unroll
+      for (int j = 0; j < NPW; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(KT::value_operand(smem, at, 32 * kk, j), pb, acc[j], 0, 0, 0);
+    }
+    if (j0 + kTile <= hi) {
+      barrier_lds();   // the tile is read
+      copy(j0 + kTile);
+    }
+  }
+  if (!act) return;
+  const int d0 = 16 * NPW * wave + 4 * g;
+  if (partial) {
+    if (wave == 0 && g == 0) { ws_ml[2 * wrow] = m_run / kLog2e; ws_ml[2 * wrow + 1] = l_run; }
+#pragma unroll
+    for (int j = 0; j < NPW; ++j) *reinterpret_cast<f32x4*>(ws_acc + wrow * DV + d0 + 16 * j) = acc[j];
+    return;
+  }
+  float f = l_run > 0.f ? 1.f / l_run : 0.f;
+  if (gate_off >= 0) f *= sigmoid_f(bf16_to_f32(proj[trow * proj_ld + gate_off + head]));
+  unsigned short* dst = o_lat + ((long)head * T_rows + trow) * DV + d0;
+#pragma unroll
+  for (int j = 0; j < NPW; ++j) {
+    u16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = f32_to_bf16(acc[j][e] * f);
+    *reinterpret_cast<u16x4*>(dst + 16 * j) = o;
+  }
+}
+
+template <typename F>
+bool allow_lds(F* fn, size_t bytes) {   // more dynamic LDS than the default limit, once per kernel
+  return bytes <= 64 * 1024 ||
+         hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
+}
+
+template <int DV>
+bool launch_dma(void* o_lat, const void* qc, const void* q, const long* positions, const float* inv_freq, const void* proj,
+                long proj_ld, const void* cache, int block_size, const int* seq_cu, const int* seq_ctx, const int* seq_bt,
+                int bt_width, int seq0, int seq1, int rows_bound, int T, int heads, int dim, int gate_off, float scale,
+                int window, bool one_row, int nparts, int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s) {
+  auto o = (unsigned short*)o_lat;
+  auto a = (const unsigned short*)qc, b = (const unsigned short*)q, p = (const unsigned short*)proj, k = (const unsigned short*)cache;
+  if (one_row) {
+    constexpr size_t smem = Tile<DV, 64>::kBytes + 16 * (64 + 8) * 2 + 128 * 4;
+    static_assert(smem <= 80 * 1024, "two workgroups per CU");
+    static const bool ok = allow_lds(&latent_dma_decode_kernel<DV>, smem);
+    if (!ok) return false;
+    latent_dma_decode_kernel<DV><<<dim3(rows_bound, (heads + 15) / 16, nparts), 256, smem, s>>>(
+        o, a, b, positions, inv_freq, p, proj_ld, k, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, T, heads, dim, gate_off,
+        scale, window, part_keys, ws_acc, ws_ml, row_base, rows_bound);
+    return true;
+  }
+  constexpr size_t smem = 4 * Tile<DV, kKeys>::kBytes + 2 * 64 * kPLd * 2 + 3 * 64 * 4;
+  static_assert(smem <= 160 * 1024, "LDS");
+  static const bool ok = allow_lds(&latent_dma_prefill_kernel<DV>, smem);
+  if (!ok) return false;
+  const int hc = min(heads, 64), tq = 64 / hc;
+  latent_dma_prefill_kernel<DV><<<dim3(rows_bound / tq + (seq1 - seq0), (heads + hc - 1) / hc), 512, smem, s>>>(
+      o, a, b, positions, inv_freq, p, proj_ld, k, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, tq, hc, T, heads, dim,
+      gate_off, scale, window);
+  return true;
+}
+
+}  // namespace
+
+bool latent_attention_dma_ok(int kv_rank, int rot_dim) {
+  return rot_dim == kRot && (kv_rank == 128 || kv_rank == 256 || kv_rank == 512);
+}
+
+bool launch_latent_attention_dma(void* o_lat, const void* qc, const void* q, const long* positions, const float* inv_freq,
+                                 const void* proj, long proj_ld, const void* cache, int block_size, const int* seq_cu,
+                                 const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int seq1, int rows_bound, int T,
+                                 int heads, int dim, int kv_rank, int gate_off, float scale, int window, bool one_row, int nparts,
+                                 int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s) {
+  if (seq1 <= seq0 || rows_bound <= 0) return true;
+#define HS_LD(DV)                                                                                                        \
+  launch_dma<DV>(o_lat, qc, q, positions, inv_freq, proj, proj_ld, cache, block_size, seq_cu, seq_ctx, seq_bt, bt_width, \
+                 seq0, seq1, rows_bound, T, heads, dim, gate_off, scale, window, one_row, nparts, part_keys, ws_acc,     \
+                 ws_ml, row_base, s)
+  return kv_rank == 128 ? HS_LD(128) : kv_rank == 256 ? HS_LD(256) : HS_LD(512);
+#undef HS_LD
+}
+
+}  // namespace hipserve

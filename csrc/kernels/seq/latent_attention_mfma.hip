@@ -298,10 +298,23 @@ __global__ __launch_bounds__(128) void latent_attention_reduce_kernel(
   }
   __syncthreads();
   const long trow = row_base + r;
-  for (int d = tid; d < kv_rank; d += 128) {
-    float o = 0.f;
-    for (int p = 0; p < nparts; ++p) o += ws_acc[(((long)p * heads + h) * ws_rows + r) * kv_rank + d] * sc[p];
-    o_lat[((long)h * T_rows + trow) * kv_rank + d] = f32_to_bf16(o);
+  for (int d = 4 * tid; d < kv_rank; d += 512) {   // kv_rank % 4 == 0
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float* src = ws_acc + ((long)h * ws_rows + r) * kv_rank + d;
+    const long step = (long)heads * ws_rows * kv_rank;
+    for (int p0 = 0; p0 < nparts; p0 += 4) {   // four runs' loads in flight; an empty run (weight 0) is not read
+      f32x4 v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        v[i] = p0 + i < nparts && sc[p0 + i] != 0.f ? *reinterpret_cast<const f32x4*>(src + (p0 + i) * step) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (p0 + i < nparts) o += v[i] * sc[p0 + i];
+    }
+    u16x4 w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w[e] = f32_to_bf16(o[e]);
+    *reinterpret_cast<u16x4*>(o_lat + ((long)h * T_rows + trow) * kv_rank + d) = w;
   }
 }
 
@@ -341,6 +354,14 @@ void launch_latent_q_cat(void* qc, const float* q_abs, const void* q, const long
   if (T <= 0) return;
   latent_q_cat_kernel<<<dim3(T, heads), 256, 0, s>>>((unsigned short*)qc, q_abs, (const unsigned short*)q, positions,
                                                      inv_freq, nfreq, T, heads, dim, rot_dim, kv_rank);
+}
+
+void launch_latent_attention_reduce(void* o_lat, const float* ws_acc, const float* ws_ml, const void* proj, long proj_ld,
+                                    int gate_off, int nparts, int heads, int rows_bound, int row_base, int T, int kv_rank,
+                                    hipStream_t s) {
+  latent_attention_reduce_kernel<<<dim3(rows_bound, heads), 128, 0, s>>>((unsigned short*)o_lat, ws_acc, ws_ml,
+                                                                       (const unsigned short*)proj, proj_ld, gate_off, nparts,
+                                                                       heads, rows_bound, row_base, T, kv_rank);
 }
 
 bool latent_attention_mfma_ok(int kv_rank, int rot_dim) {

@@ -80,6 +80,32 @@ HS_DEVICE float row_sum(float v) {
   return dpp_step<0x140, 0xf, false>(v);  // row_mirror
 }
 
+// Workgroup `wg` of those that cut every sequence seq0 .. seq1 - 1 of a step into tiles of tq rows: its sequence and first row
+// (the same in every lane); false past the last one. A lane per sequence: a walk over them would wait for every row count.
+HS_DEVICE bool find_row_tile(const int* __restrict__ seq_cu, int seq0, int seq1, int tq, int wg, int& s, int& tok0) {
+  const int lane = threadIdx.x & 63;
+  int base = 0;
+  for (int i0 = seq0; i0 < seq1; i0 += 64) {
+    const int i = i0 + lane;
+    const int nt = i < seq1 ? (seq_cu[i + 1] - seq_cu[i] + tq - 1) / tq : 0;
+    int end = nt;   // inclusive sum over the lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(end, o, 64);
+      if (lane >= o) end += v;
+    }
+    const unsigned long long mine = __ballot(wg >= base + end - nt && wg < base + end);
+    if (mine != 0) {
+      const int l = __builtin_ctzll(mine);
+      s = i0 + l;
+      tok0 = (wg - base - (__builtin_amdgcn_readlane(end, l) - __builtin_amdgcn_readlane(nt, l))) * tq;
+      return true;
+    }
+    base += __builtin_amdgcn_readlane(end, 63);
+  }
+  return false;
+}
+
 // First key (behind the kept ones) that position pos sees: its window's, its chunk's, or the sequence's first.
 HS_DEVICE int first_key(int pos, int window, int chunk) {
   return chunk > 0 ? pos - pos % chunk : window > 0 ? max(0, pos - window + 1) : 0;

@@ -126,6 +126,7 @@ TORCH_LIBRARY(hipserve_cell, m) {
         "Tensor cache, Tensor seq_cu, Tensor seq_ctx, Tensor seq_bt, int seq0, int seq1, int rows_bound, "
         "Tensor inv_freq, int heads, int dim, int rot_dim, int kv_rank, int gate_off, float scale, int window, "
         "int nparts, int part_keys, Tensor(c!)? ws_acc, Tensor(d!)? ws_ml, int row_base, bool fill_qc) -> ()");
+  m.def("latent_attention_dma_ok(int kv_rank, int rot_dim) -> bool", &latent_attention_dma_ok);
   m.def("latent_attention_mfma_ok(int kv_rank, int rot_dim) -> bool", &latent_attention_mfma_ok);
 }
 

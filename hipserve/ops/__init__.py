@@ -268,6 +268,12 @@ class KernelOps:
             if nd:
                 span = min(window, meta.max_ctx or window) if window > 0 else meta.max_ctx
                 part = self.LATENT_DECODE_RUN
+                if self._latent_lib.latent_attention_dma_ok(kv_rank, rot_dim):
+                    # a workgroup multiplies 64 keys at a time: short runs, unless the batch fills the chip several times over
+                    # (a run's unnormalised output is written and read once more)
+                    part = 64
+                    while part < 256 and nd * -(-heads // 16) * -(-span // part) > 1024:
+                        part *= 2
                 while -(-span // part) > 64:
                     part *= 2
                 nparts = max(1, -(-span // part))

@@ -194,3 +194,56 @@ def test_expert_gemm_tiles_of_few_rows(tokens, E, top, N, K, act):
     z = torch.einsum("pk,pnk->pn", xp.double(), wp.double()) * (scale.double()[:, None] if scale is not None else 1.0)
     want = act64(z, {0: None, 1: "relu2", 2: "silu_mul", 3: "clamped_glu"}[act], 1.0, 0.0)
     close_to(out[pair.long()], want, x, w.view(-1, K), scale=12.0)
+
+
+# ------------------------------------------------------------------ latent attention
+def latent_case(lens, ctxs, heads, dim, kv, rot, block, dtype, dev, seed=0):
+    """Rows of sequences with ``lens`` rows in this step and ``ctxs`` tokens after it: random queries, a random paged cache whose
+    pages lie in no order, and a meta of prompt portions first (lens > 1), single rows last."""
+    from hipserve.models.llama import AttnMeta
+
+    g = torch.Generator().manual_seed(seed)
+    T, width = sum(lens), max(-(-c // block) for c in ctxs)
+    bt = torch.randperm(len(lens) * width, generator=g).int().view(len(lens), width)
+    cache = torch.randn(len(lens) * width, block, kv + rot, generator=g).to(dtype)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    pos = torch.cat([torch.arange(c - n, c) for n, c in zip(lens, ctxs)])
+    q_abs = torch.randn(heads, T, kv + rot, generator=g).to(dtype) * 0.3
+    q = torch.randn(T, heads * (dim + rot), generator=g).to(dtype)
+    proj = torch.randn(T, heads + 3, generator=g).to(dtype)
+    nd = sum(n == 1 for n in lens)
+    meta = AttnMeta(num_prefill_tokens=T - nd, num_decode=nd, positions=pos.to(dev), slot_mapping=pos.to(dev), seq_cu=cu.to(dev),
+                    seq_ctx=torch.tensor(ctxs, dtype=torch.int32, device=dev), seq_bt=bt.to(dev), max_q=max(lens), max_ctx=max(ctxs))
+    return cache, cu, pos, bt, q_abs, q, proj, meta
+
+
+@gpu
+@pytest.mark.parametrize("kv", [128, 256, 512])
+@pytest.mark.parametrize("heads,window", [(16, 0), (5, 100), (70, 33)])
+@pytest.mark.parametrize("lens,ctxs", [([1], [1]), ([1, 1, 1], [64, 65, 700]), ([37], [37]), ([33, 5, 1], [33, 400, 129]), ([2, 190], [31, 255])])
+def test_latent_attention_dma(kv, heads, window, lens, ctxs):
+    """Tiles of 32 and 64 keys filled partly, windows that start inside a tile, rows that leave a workgroup's tiles unused, runs of
+    keys of a decode row (some empty), the rotary part formed in the kernel, in 64 bits."""
+    rot, dim, block, gate, scale = 64, 24, 16, 2, 0.11
+    cache, cu, pos, bt, q_abs, q, proj, meta = latent_case(lens, ctxs, heads, dim, kv, rot, block, torch.bfloat16, "cuda", kv + heads)
+    inv = torch.pow(torch.tensor(1e4), -2.0 * torch.arange(rot // 2) / rot)
+    T = sum(lens)
+    qr = q.double().view(T, heads, dim + rot)[..., dim:]
+    ang = pos.double()[:, None] * inv.double()
+    c, s = torch.cos(ang)[:, None], torch.sin(ang)[:, None]
+    qr = torch.cat([qr[..., :32] * c - qr[..., 32:] * s, qr[..., 32:] * c + qr[..., :32] * s], -1).bfloat16().double()
+    want = torch.empty(heads, T, kv, dtype=torch.float64)
+    for i, (n, ctx) in enumerate(zip(lens, ctxs)):
+        j = torch.arange(ctx)
+        keys = cache[bt[i, j // block].long(), j % block].double()
+        rows = slice(int(cu[i]), int(cu[i]) + n)
+        sc = (q_abs[:, rows, :kv].double() @ keys[:, :kv].T + qr[rows].transpose(0, 1) @ keys[:, kv:].T) * scale
+        back = pos[rows, None] - j
+        sc = sc.masked_fill((back < 0) | (back >= window if window else back < 0), -float("inf"))
+        want[:, rows] = (torch.softmax(sc, -1) @ keys[:, :kv]) * torch.sigmoid(proj[rows, gate:gate + heads].double().T)[..., None]
+    ops = get_ops("cuda")
+    assert ops._latent_lib.latent_attention_dma_ok(kv, rot)
+    out = torch.full((heads, T, kv), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.latent_attention(out, q_abs.cuda(), q.cuda(), proj.cuda(), cache.cuda(), meta, inv.cuda(), heads, dim, rot, kv, gate, scale, window)
+    # weights and outputs are rounded to bf16; a score is a sum of kv + rot products, exact to 2^-16 or so, before the exponential
+    assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
