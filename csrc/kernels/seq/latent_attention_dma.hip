@@ -4,7 +4,7 @@
 // That kernel loads a 32-key tile into registers, stores it to LDS and only then multiplies: a tile waits for its page
 // lookup and for its rows (about 3 us) before 0.5 us of products, its operand reads wait one by one (no registers left),
 // and the V operand of P . V is gathered from LDS two bytes at a time. Here
-//   * global_load_lds brings the rows into one of four LDS buffers, two tiles ahead of the products;
+//   * global_load_lds brings the rows into one of four LDS buffers, a tile ahead of the scores;
 //   * a buffer holds [32][latent dims] and [32][64 rotary dims]; the eight 16-byte chunks of every 128 bytes are
 //     XOR-swizzled by the key, by choosing which chunk a lane copies, so that both the row-wise operand reads of
 //     S = K . Q^T and the transposing reads below spread over the banks without padding;
@@ -15,10 +15,12 @@
 //     DV / 4 latent dims each for all 64 rows: the softmax of one tile runs beside the products of another, neither half
 //     holds the other's registers (queries 72, outputs 128 per lane), and a tile costs one barrier;
 //   * the queries' rotary part is rotated when the operands are loaded (its halves meet in one lane), no pass of its own.
-// What bounds it: LDS reads (every K row goes to four waves: 181 KB per tile of 64 rows against 1088 cycles of products).
-// @NUMBERS@
+// 8192 rows (4 prompts) x 16 heads, 512 + 64 dims, window 1024: 980 -> 416 us (540 TFLOP/s). A tile of 64 rows takes about 3700
+// cycles of its SIMDs: 1088 of products, 1400 of vector instructions (softmax, conversions), the rest waits at the one barrier
+// per tile; its LDS reads (every K row goes to four waves, 181 KB) take 1600. Counted without overlap of the scores with the next
+// tile's operand reads: 497 us; without uniform copy addresses: 437.
 // latent_dma_decode_kernel serves decode rows: a workgroup takes 16 heads of one sequence and a run of keys, 64 of them
-// at a time; its waves split the keys for S and the latent dims for P . V. @DECODE@
+// at a time; its waves split the keys for S and the latent dims for P . V. One row of 724 keys, 16 heads: 46 -> 10 us.
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
 
@@ -37,16 +39,16 @@ HS_DEVICE void barrier_all() {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
-// All but the wave's last N vector memory operations are done.
-template <int N>
-HS_DEVICE void copied_but() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"i"(N) : "memory");
-}
 // 1 KB from the lanes' addresses to LDS, 16 bytes per lane side by side, asynchronously. Written out because the compiler
-// would otherwise wait for every copy in flight before the next transposing read; the waits are the callers' copied_but.
+// would otherwise wait for every copy in flight before the next transposing read; the waits are the callers' barrier_all.
 HS_DEVICE void copy_1k(const unsigned short* src, const unsigned char* lds) {
   const unsigned at = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds;
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(at)), "v"(src) : "memory");   // nothing else in this file uses m0
+}
+// The same from a uniform base and the lanes' byte offsets.
+HS_DEVICE void copy_1k(const unsigned char* base, unsigned off, const unsigned char* lds) {
+  const unsigned at = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds;
+  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(at)), "v"(off), "s"(base) : "memory");
 }
 // The same for LDS operations alone: copies into LDS may still be in flight.
 HS_DEVICE void barrier_lds() {
@@ -55,21 +57,33 @@ HS_DEVICE void barrier_lds() {
   asm volatile("" ::: "memory");
 }
 
-// K tile rows in LDS: [KEYS][DV] then [KEYS][64]; 16-byte chunk ch of key k sits at chunk ch ^ (k & 7).
+// Largest of the values of the lanes c, c + 16, c + 32, c + 48, in all of them (row and half swaps of the vector unit).
+HS_DEVICE float max_of_rows(float x) {
+  const unsigned u = __builtin_bit_cast(unsigned, x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const float y = fmaxf(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1]));
+  const unsigned w = __builtin_bit_cast(unsigned, y);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
+}
+
+// K tile rows in LDS: [KEYS][DV] then [KEYS][64]; 16-byte chunk ch of key k sits at chunk ch ^ swizzle(k): eight keys in a
+// row use eight different chunks of a 128-byte line (the key operands), four in a row four different pairs (the values).
+HS_DEVICE int swizzle(int k) { return (k & 3) << 1 | (k >> 2 & 1); }
 template <int DV, int KEYS> struct Tile {
   static constexpr int kMain = KEYS * DV * 2, kBytes = kMain + KEYS * kRot * 2;
-  static HS_DEVICE int main_at(int k, int ch) { return k * DV * 2 + ((ch ^ (k & 7)) << 4); }
-  static HS_DEVICE int rot_at(int k, int ch) { return kMain + k * kRot * 2 + ((ch ^ (k & 7)) << 4); }
+  static HS_DEVICE int main_at(int k, int ch) { return k * DV * 2 + ((ch ^ swizzle(k)) << 4); }
+  static HS_DEVICE int rot_at(int k, int ch) { return kMain + k * kRot * 2 + ((ch ^ swizzle(k)) << 4); }
   // The wave copies keys 8 w .. 8 w + 7 of the tile; `row` = element offset of key `lane` % KEYS's cache row.
   static HS_DEVICE void copy(unsigned char* lds, const unsigned short* cache, long row, int w, int lane) {
     constexpr int kPer = 512 / DV, kChunks = DV / 8;   // keys and 16-byte chunks of a key in one 1 KB copy
 #pragma unroll
     for (int i = 0; i < 8 / kPer; ++i) {
-      const int k = 8 * w + i * kPer + lane / kChunks, ch = (lane % kChunks) ^ (k & 7);
+      const int k = 8 * w + i * kPer + lane / kChunks, ch = (lane % kChunks) ^ swizzle(k);
       const unsigned short* src = cache + __shfl(row, k, 64) + 8 * ch;
       copy_1k(src, lds + (8 * w + i * kPer) * DV * 2);
     }
-    const int k = 8 * w + lane / 8, ch = (lane & 7) ^ (k & 7);
+    const int k = 8 * w + lane / 8, ch = (lane & 7) ^ swizzle(k);
     const unsigned short* src = cache + __shfl(row, k, 64) + DV + 8 * ch;
     copy_1k(src, lds + kMain + 8 * w * kRot * 2);
   }
@@ -133,13 +147,14 @@ HS_DEVICE void load_query(bf16x8 (&qf)[DV / 32 + 2], bool act, const unsigned sh
   qf[KL + 1] = __builtin_bit_cast(bf16x8, b);
 }
 
-// 64 (token, head) rows of consecutive tokens of one sequence. Iteration i: waves 0 - 3 turn tile i into P, waves 4 - 7 add
-// tile i - 1 to the outputs, all copy tile i + 2 into the buffer that tile i - 2 has left.
+// 64 (token, head) rows of consecutive tokens of one sequence. Between two barriers waves 0 - 3 multiply tile i with the
+// queries and make P of it (the next tile's operands on their way from LDS meanwhile), waves 4 - 7 add tile i - 1 to the
+// outputs, and all copy tile i + 2 into the buffer that tile i - 2 has left.
 template <int DV>
 __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
     unsigned short* __restrict__ o_lat, const unsigned short* __restrict__ qc, const unsigned short* __restrict__ q,
     const long* __restrict__ positions, const float* __restrict__ inv_freq, const unsigned short* __restrict__ proj,
-    long proj_ld, const unsigned short* __restrict__ cache, int block_size, const int* __restrict__ seq_cu,
+    long proj_ld, const unsigned short* __restrict__ cache, int block_shift, const int* __restrict__ seq_cu,
     const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0, int seq1, int tq, int hc,
     int T_rows, int heads, int dim, int gate_off, float scale, int window) {
   using KT = Tile<DV, kKeys>;
@@ -161,21 +176,41 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
   const int lo = (window > 0 ? max(0, p_first - window + 1) : 0) & ~(kKeys - 1);
   const int ntiles = (hi - lo) / kKeys + 1;
   const int* bt = seq_bt + (long)s * bt_width;
+  const int mask = (1 << block_shift) - 1;
   // the first of the keys 4 wave .. + 3 of tile t that exists, and its page; keys past the last one are the last one again
-  auto page_of = [&](int t, int k) { return bt[min(lo + t * kKeys + k, hi) / block_size]; };
+  auto page_of = [&](int t, int k) { return bt[min(lo + t * kKeys + k, hi) >> block_shift]; };
+  constexpr int kPer = 512 / DV, kChunks = DV / 8;   // keys and 16-byte chunks of a key per copy
+  unsigned off_main[kMainCopies], off_rot;           // the lane's bytes past the row of the tile's first key (of its page)
+#pragma unroll
+  for (int i = 0; i < kMainCopies; ++i) {
+    const int k = 4 * wave + i * kPer + lane / kChunks;
+    off_main[i] = ((k & mask) * Dk + 8 * ((lane % kChunks) ^ swizzle(k))) * 2;
+  }
+  {
+    const int k = 8 * (wave & 3) + lane / 8;
+    off_rot = ((k & mask) * Dk + DV + 8 * ((lane & 7) ^ swizzle(k))) * 2;
+  }
   auto copy = [&](int t, int page, int page_rot) {
     unsigned char* lds = smem + (t & 3) * KT::kBytes;
     const int j0 = lo + t * kKeys;
-    constexpr int kPer = 512 / DV, kChunks = DV / 8;   // keys and 16-byte chunks of a key per copy
+    if (j0 + kKeys - 1 <= hi) {   // all keys exist: the addresses differ from tile to tile by uniform numbers
+      const unsigned char* base = reinterpret_cast<const unsigned char*>(cache + (((long)page << block_shift) + (j0 & mask)) * Dk);
+#pragma unroll
+      for (int i = 0; i < kMainCopies; ++i) copy_1k(base, off_main[i], lds + (4 * wave + i * kPer) * DV * 2);
+      if (wave < 4)
+        copy_1k(reinterpret_cast<const unsigned char*>(cache + (((long)page_rot << block_shift) + (j0 & mask)) * Dk), off_rot,
+                lds + KT::kMain + 8 * wave * kRot * 2);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < kMainCopies; ++i) {
-      const int k = 4 * wave + i * kPer + lane / kChunks, ch = (lane % kChunks) ^ (k & 7);
-      const unsigned short* src = cache + ((long)page * block_size + min(j0 + k, hi) % block_size) * Dk + 8 * ch;
+      const int k = 4 * wave + i * kPer + lane / kChunks, ch = (lane % kChunks) ^ swizzle(k);
+      const unsigned short* src = cache + (((long)page << block_shift) + (min(j0 + k, hi) & mask)) * Dk + 8 * ch;
       copy_1k(src, lds + (4 * wave + i * kPer) * DV * 2);
     }
     if (wave < 4) {
-      const int k = 8 * wave + lane / 8, ch = (lane & 7) ^ (k & 7);
-      const unsigned short* src = cache + ((long)page_rot * block_size + min(j0 + k, hi) % block_size) * Dk + DV + 8 * ch;
+      const int k = 8 * wave + lane / 8, ch = (lane & 7) ^ swizzle(k);
+      const unsigned short* src = cache + (((long)page_rot << block_shift) + (min(j0 + k, hi) & mask)) * Dk + DV + 8 * ch;
       copy_1k(src, lds + KT::kMain + 8 * wave * kRot * 2);
     }
   };
@@ -183,6 +218,12 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
   copy(0, page_of(0, 4 * wave), page_of(0, krot));
   if (ntiles > 1) copy(1, page_of(1, 4 * wave), page_of(1, krot));
   int page = page_of(2, 4 * wave), page_rot = page_of(2, krot);   // clamped: always an existing page
+  auto copy_next = [&](int t) {   // tile t, whose pages are at hand
+    if (t >= ntiles) return;
+    copy(t, page, page_rot);
+    page = page_of(t + 1, 4 * wave);
+    page_rot = page_of(t + 1, krot);
+  };
   const typename KT::Places at = KT::places(wave & 3, c, g);
   if (wave < 4) {
     const int sr = 16 * wave + c, srt = sr / hc, srh = sr % hc;
@@ -195,43 +236,46 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
     load_query<DV>(qf, sact, qc + ((long)shead * T_rows + strow) * Dk,
                    q != nullptr ? q + strow * heads * (dim + kRot) + (long)shead * (dim + kRot) + dim : nullptr,
                    (float)positions[strow], inv_freq, g);
-    float m_run = -INFINITY, l_run = 0.f;
+    float m_run = -INFINITY, l_run = 0.f;   // l_run: this lane's keys only
     const float scale2 = scale * kLog2e;
-    for (int i = 0; i <= ntiles; ++i) {
-      if (i + 1 < ntiles) copied_but<kMainCopies + 1>();   // tile i + 1 may still be on its way
-      else copied_but<0>();
-      barrier_lds();
-      if (i + 2 < ntiles) {
-        copy(i + 2, page, page_rot);
-        page = page_of(i + 3, 4 * wave);
-        page_rot = page_of(i + 3, krot);
-      }
-      if (i == ntiles) break;
+    constexpr int kBatch = 6, kBatches = (KS + kBatch - 1) / kBatch;   // steps whose operands are read together
+    bf16x8 ka[2][kBatch][2];
+    f32x4 sc[2];
+    auto read_keys = [&](int i, int b) {
       const unsigned char* kt = smem + (i & 3) * KT::kBytes;
-      const int j0 = lo + i * kKeys;
-      f32x4 sc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-      // the key operands are read a batch of steps ahead of their products
-      constexpr int kBatch = 6, kBatches = (KS + kBatch - 1) / kBatch;
-      bf16x8 ka[2][kBatch][2];
 #pragma unroll
-      for (int b = 0; b <= kBatches; ++b) {
-        if (b < kBatches)
+      for (int u = 0; u < kBatch; ++u)
 #pragma unroll
-          for (int u = 0; u < kBatch; ++u)
+        for (int nt = 0; nt < 2; ++nt)
+          if (b * kBatch + u < KS) ka[b & 1][u][nt] = KT::key_operand(kt, at, 16 * nt, b * kBatch + u);
+    };
+    auto multiply = [&](int i) {   // batches 0 and 1 of tile i are read
+      sc[0] = sc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt)
-              if (b * kBatch + u < KS) ka[b & 1][u][nt] = KT::key_operand(kt, at, 16 * nt, b * kBatch + u);
+      for (int b = 0; b < kBatches; ++b) {
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt)
+            if (b * kBatch + u < KS)
+              sc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[b & 1][u][nt], qf[b * kBatch + u], sc[nt], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        if (b > 0)
-#pragma unroll
-          for (int u = 0; u < kBatch; ++u)
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt)
-              if ((b - 1) * kBatch + u < KS)
-                sc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[(b - 1) & 1][u][nt], qf[(b - 1) * kBatch + u], sc[nt], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
+        if (b + 2 < kBatches) read_keys(i, b + 2);
       }
-      // masked online softmax (log2 domain) of row sr: lane (c, g) holds keys 16 nt + 4 g + i
+    };
+    barrier_all();
+    copy_next(2);
+    read_keys(0, 0);
+    if constexpr (kBatches > 1) read_keys(0, 1);
+    multiply(0);
+    for (int i = 1; i <= ntiles; ++i) {
+      if (i < ntiles) {
+        read_keys(i, 0);
+        if constexpr (kBatches > 1) read_keys(i, 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      // masked online softmax (log2 domain) of tile i - 1, row sr: lane (c, g) holds keys 16 nt + 4 g + e
+      const int j0 = lo + (i - 1) * kKeys;
       float v[8], mx = -INFINITY;
       if (__all(sact && j0 + kKeys - 1 <= spos && j0 >= s_lo)) {   // every row of the wave sees the whole tile
 #pragma unroll
@@ -244,25 +288,28 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
           mx = fmaxf(mx, v[e]);
         }
       }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+      mx = max_of_rows(mx);
       const float mn = fmaxf(m_run, mx);
+      const float off = mn > -INFINITY ? mn : 0.f;   // no key seen yet: every weight is exp2(-inf) = 0
       float sum = 0.f;
       u16x8 pk;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float p = mn > -INFINITY ? __builtin_amdgcn_exp2f(v[e] - mn) : 0.f;
-        pk[e] = f32_to_bf16(p);   // rounded: what is multiplied, and its sum
+        pk[e] = f32_to_bf16(__builtin_amdgcn_exp2f(v[e] - off));   // rounded: what is multiplied, and its sum
         sum += bf16_to_f32(pk[e]);
       }
-      sum += __shfl_xor(sum, 16, 64);
-      sum += __shfl_xor(sum, 32, 64);
-      *reinterpret_cast<u16x8*>(p_lds + ((i & 1) * 64 + sr) * kPLd + 8 * g) = pk;
+      const int pb = (i - 1) & 1;
+      *reinterpret_cast<u16x8*>(p_lds + (pb * 64 + sr) * kPLd + 8 * g) = pk;
       const float al = mn > -INFINITY ? __builtin_amdgcn_exp2f(m_run - mn) : 1.f;  // m_run = -inf: 0
-      if (g == 0) alpha[(i & 1) * 64 + sr] = al;
+      if (g == 0) alpha[pb * 64 + sr] = al;
       l_run = l_run * al + sum;
       m_run = mn;
+      barrier_all();
+      copy_next(i + 2);
+      if (i < ntiles) multiply(i);
     }
+    l_run += __shfl_xor(l_run, 16, 64);
+    l_run += __shfl_xor(l_run, 32, 64);
     if (g == 0) {   // gate / softmax sum of the row
       float f = 0.f;
       if (sact && l_run > 0.f) {
@@ -279,15 +326,11 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
   for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
     for (int j = 0; j < NPW; ++j) acc[mt][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int i = 0; i <= ntiles; ++i) {
-    if (i + 1 < ntiles) copied_but<kMainCopies>();
-    else copied_but<0>();
-    barrier_lds();
-    if (i + 2 < ntiles) {
-      copy(i + 2, page, page_rot);
-      page = page_of(i + 3, 4 * wave);
-    }
-    if (i == 0) continue;
+  barrier_all();
+  copy_next(2);
+  for (int i = 1; i <= ntiles; ++i) {
+    barrier_all();
+    copy_next(i + 2);
     unsigned char* kt = smem + ((i - 1) & 3) * KT::kBytes;
     const unsigned short* pt = p_lds + ((i - 1) & 1) * 64 * kPLd;
     bf16x8 pb[4], va[NPW];
@@ -338,7 +381,7 @@ template <int DV>
 __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
     unsigned short* __restrict__ o_lat, const unsigned short* __restrict__ qc, const unsigned short* __restrict__ q,
     const long* __restrict__ positions, const float* __restrict__ inv_freq, const unsigned short* __restrict__ proj,
-    long proj_ld, const unsigned short* __restrict__ cache, int block_size, const int* __restrict__ seq_cu,
+    long proj_ld, const unsigned short* __restrict__ cache, int block_shift, const int* __restrict__ seq_cu,
     const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0, int T_rows, int heads,
     int dim, int gate_off, float scale, int window, int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
     int row_base, int ws_rows) {
@@ -364,9 +407,10 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
     return;
   }
   const int* bt = seq_bt + (long)s * bt_width;
+  const int mask = (1 << block_shift) - 1;
   auto row_of = [&](int j0) {
     const int j = min(j0 + lane, hi);
-    return ((long)bt[j / block_size] * block_size + j % block_size) * Dk;
+    return (((long)bt[j >> block_shift] << block_shift) + (j & mask)) * Dk;
   };
   auto copy = [&](int j0) {
     const long row = row_of(j0);
@@ -396,8 +440,7 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
       v[i] = act && j0 + 16 * wave + 4 * g + i <= hi ? sc[i] * scale2 : -INFINITY;
       mx = fmaxf(mx, v[i]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = max_of_rows(mx);
     if (g == 0) mw[16 * wave + c] = mx;
     barrier_lds();
     const float mn = fmaxf(fmaxf(fmaxf(mw[c], mw[16 + c]), fmaxf(mw[32 + c], mw[48 + c])), m_run);
@@ -459,7 +502,7 @@ bool allow_lds(F* fn, size_t bytes) {   // more dynamic LDS than the default lim
 
 template <int DV>
 bool launch_dma(void* o_lat, const void* qc, const void* q, const long* positions, const float* inv_freq, const void* proj,
-                long proj_ld, const void* cache, int block_size, const int* seq_cu, const int* seq_ctx, const int* seq_bt,
+                long proj_ld, const void* cache, int block_shift, const int* seq_cu, const int* seq_ctx, const int* seq_bt,
                 int bt_width, int seq0, int seq1, int rows_bound, int T, int heads, int dim, int gate_off, float scale,
                 int window, bool one_row, int nparts, int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s) {
   auto o = (unsigned short*)o_lat;
@@ -470,7 +513,7 @@ bool launch_dma(void* o_lat, const void* qc, const void* q, const long* position
     static const bool ok = allow_lds(&latent_dma_decode_kernel<DV>, smem);
     if (!ok) return false;
     latent_dma_decode_kernel<DV><<<dim3(rows_bound, (heads + 15) / 16, nparts), 256, smem, s>>>(
-        o, a, b, positions, inv_freq, p, proj_ld, k, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, T, heads, dim, gate_off,
+        o, a, b, positions, inv_freq, p, proj_ld, k, block_shift, seq_cu, seq_ctx, seq_bt, bt_width, seq0, T, heads, dim, gate_off,
         scale, window, part_keys, ws_acc, ws_ml, row_base, rows_bound);
     return true;
   }
@@ -480,7 +523,7 @@ bool launch_dma(void* o_lat, const void* qc, const void* q, const long* position
   if (!ok) return false;
   const int hc = min(heads, 64), tq = 64 / hc;
   latent_dma_prefill_kernel<DV><<<dim3(rows_bound / tq + (seq1 - seq0), (heads + hc - 1) / hc), 512, smem, s>>>(
-      o, a, b, positions, inv_freq, p, proj_ld, k, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, tq, hc, T, heads, dim,
+      o, a, b, positions, inv_freq, p, proj_ld, k, block_shift, seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, tq, hc, T, heads, dim,
       gate_off, scale, window);
   return true;
 }
@@ -497,8 +540,9 @@ bool launch_latent_attention_dma(void* o_lat, const void* qc, const void* q, con
                                  int heads, int dim, int kv_rank, int gate_off, float scale, int window, bool one_row, int nparts,
                                  int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s) {
   if (seq1 <= seq0 || rows_bound <= 0) return true;
+  const int block_shift = __builtin_ctz(block_size);   // a power of two
 #define HS_LD(DV)                                                                                                        \
-  launch_dma<DV>(o_lat, qc, q, positions, inv_freq, proj, proj_ld, cache, block_size, seq_cu, seq_ctx, seq_bt, bt_width, \
+  launch_dma<DV>(o_lat, qc, q, positions, inv_freq, proj, proj_ld, cache, block_shift, seq_cu, seq_ctx, seq_bt, bt_width, \
                  seq0, seq1, rows_bound, T, heads, dim, gate_off, scale, window, one_row, nparts, part_keys, ws_acc,     \
                  ws_ml, row_base, s)
   return kv_rank == 128 ? HS_LD(128) : kv_rank == 256 ? HS_LD(256) : HS_LD(512);
