@@ -46,6 +46,27 @@ inline void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor
                              stream, nb > 1 ? scratch.data_ptr<int>() : nullptr);
 }
 
+// moe_align of the pairs (t, j) whose expert is table[tokens[t]][j].
+inline void moe_table_align(const at::Tensor& table, const at::Tensor& tokens, int64_t E, int64_t tile, at::Tensor& slots,
+                            at::Tensor& tile_expert, at::Tensor& pair_slot) {
+  CHECK_DEV(table); CHECK_I32(table); CHECK_I32(slots); CHECK_I32(tile_expert); CHECK_I32(pair_slot);
+  TORCH_CHECK(table.dim() == 2 && table.size(0) >= 1 && tokens.scalar_type() == at::kLong && tokens.is_contiguous());
+  TORCH_CHECK(E >= 1 && E <= 128, "moe_align: at most 128 experts");
+  TORCH_CHECK(tile == 16 || tile == 32 || tile == 64 || tile == 128 || tile == 256);
+  const long top = table.size(1), npairs = tokens.numel() * top;
+  TORCH_CHECK(top >= 1 && hipserve::moe_align_blocks(npairs) == 1, "moe_table_align: small batches");
+  TORCH_CHECK(slots.numel() >= npairs + E * (tile - 1) && slots.numel() % tile == 0,
+              "slots capacity must cover padding and be a multiple of the tile");
+  TORCH_CHECK(tile_expert.numel() * tile >= slots.numel() && pair_slot.numel() >= npairs);
+  c10::hip::HIPGuardMasqueradingAsCUDA g(table.device());
+  at::Tensor count = at::empty({1}, slots.options());
+  hipserve::launch_moe_table_align(table.data_ptr<int>(), tokens.data_ptr<long>(), top, table.size(0), npairs, E, tile,
+                                   slots.data_ptr<int>(), slots.numel(), tile_expert.data_ptr<int>(), tile_expert.numel(),
+                                   count.data_ptr<int>(), pair_slot.data_ptr<int>(), cur_stream());
+}
+
+inline bool moe_align_small(int64_t npairs) { return hipserve::moe_align_blocks(npairs) == 1; }
+
 inline void expert_gemm(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const at::Tensor& slots,
                         const at::Tensor& tile_expert, int64_t tile, int64_t gather_k, int64_t act,
                         const c10::optional<at::Tensor>& row_scale, double limit, int64_t pairs) {
@@ -100,6 +121,9 @@ inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor
 inline void def_moe_ops(torch::Library& m) {
   m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int act, float c0, float c1) -> ()");
   m.def("moe_align(Tensor ids, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, Tensor(c!) pair_slot) -> ()");
+  m.def("moe_table_align(Tensor table, Tensor tokens, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, "
+        "Tensor(c!) pair_slot) -> ()");
+  m.def("moe_align_small(int npairs) -> bool", &moe_align_small);
   m.def("expert_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor slots, Tensor tile_expert, int tile, int gather_k, "
         "int act, Tensor? row_scale=None, float limit=0.0, int pairs=0) -> ()");
 }
@@ -107,6 +131,7 @@ inline void def_moe_ops(torch::Library& m) {
 inline void impl_moe_ops(torch::Library& m) {
   m.impl("skinny_linear", &skinny_linear);
   m.impl("moe_align", &moe_align);
+  m.impl("moe_table_align", &moe_table_align);
   m.impl("expert_gemm", &expert_gemm);
 }
 

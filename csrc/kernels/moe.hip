@@ -88,16 +88,25 @@ __global__ __launch_bounds__(256) void moe_topk_softmax_kernel(const T* __restri
   }
 }
 
-__global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, int npairs, int E, int tile,
+// table (may be null): the experts come from table[tokens[t]][j] (top of them per token) instead of ids, without a
+// launch of its own for the lookup (4.5 us); a token outside the table counts as its first entry.
+__global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, const int* __restrict__ table,
+                                                         const long* __restrict__ tokens, int top, long table_rows,
+                                                         int npairs, int E, int tile,
                                                          int* __restrict__ slots, int slots_cap,
                                                          int* __restrict__ tile_expert, int tiles_cap,
                                                          int* __restrict__ num_tiles, int* __restrict__ pair_slot,
                                                          int* __restrict__ group_end) {
   __shared__ int cnt[128], off[129], cur[128];
   const int tid = threadIdx.x, lane = tid & 63;
+  auto expert_of = [&](int p) {
+    if (table == nullptr) return ids[p];
+    const long t = tokens[p / top];
+    return table[(t >= 0 && t < table_rows ? t : 0) * top + p % top];
+  };
   if (tid < 128) { cnt[tid] = 0; cur[tid] = 0; }
   __syncthreads();
-  for (int p = tid; p < npairs; p += 1024) atomicAdd(&cnt[ids[p]], 1);
+  for (int p = tid; p < npairs; p += 1024) atomicAdd(&cnt[expert_of(p)], 1);
   __syncthreads();
   if (tid < 64) {  // exclusive scan of the tile-padded counts, 2 experts per lane (E <= 128)
     const int e0 = 2 * lane, e1 = 2 * lane + 1;
@@ -130,7 +139,7 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
   for (int t = total / tile + tid; t < tiles_cap; t += 1024) tile_expert[t] = -1;
   __syncthreads();
   for (int p = tid; p < npairs; p += 1024) {
-    const int e = ids[p];
+    const int e = expert_of(p);
     const int pos = off[e] + atomicAdd(&cur[e], 1);
     slots[pos] = p;
     pair_slot[p] = pos;
@@ -456,8 +465,15 @@ void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, i
                                          num_tiles, pair_slot, group_end);
     return;
   }
-  moe_align_kernel<<<1, 1024, 0, s>>>(ids, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap, num_tiles,
-                                      pair_slot, group_end);
+  moe_align_kernel<<<1, 1024, 0, s>>>(ids, nullptr, nullptr, 1, 0, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap,
+                                      num_tiles, pair_slot, group_end);
+}
+
+void launch_moe_table_align(const int* table, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
+                            int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot,
+                            hipStream_t s) {
+  moe_align_kernel<<<1, 1024, 0, s>>>(nullptr, table, tokens, top, table_rows, npairs, E, tile, slots, slots_cap, tile_expert,
+                                      tiles_cap, num_tiles, pair_slot, nullptr);
 }
 
 // Prefill MoE input: xs[slot] = x[slots[slot] / k] (the token of the pair in that

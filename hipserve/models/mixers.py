@@ -283,16 +283,15 @@ class TableMoE:
     def forward(self, h: torch.Tensor, ids: torch.Tensor):
         s, ops = self.spec, self.ops
         T, dev = h.shape[0], h.device
-        experts = self.table.index_select(0, ids).reshape(-1)          # [T * top]
         P = T * s.top
         if self._packed_ok(h, P):
-            return self._forward_packed(h, experts, P)
+            return self._forward_packed(h, self.table.index_select(0, ids).reshape(-1), P)
         tile = MOE_TILE_LARGE if P >= 4 * MOE_TILE_LARGE * s.experts else MOE_TILE
         cap = -(-(P + s.experts * (tile - 1)) // tile) * tile
         slots = torch.empty(cap, dtype=torch.int32, device=dev)
         tile_expert = torch.empty(cap // tile, dtype=torch.int32, device=dev)
         pair_slot = torch.empty(P, dtype=torch.int32, device=dev)
-        ops.moe_align(experts, s.experts, tile, slots, tile_expert, pair_slot)
+        ops.moe_table_align(self.table, ids, s.experts, tile, slots, tile_expert, pair_slot)
         act = torch.empty(cap, s.ff, device=dev, dtype=h.dtype)
         ops.expert_gemm(act, h, self.w_up, slots, tile_expert, tile, s.top, True, pairs=P)
         y = torch.empty(cap, self.hidden, device=dev, dtype=h.dtype)

@@ -533,6 +533,13 @@ class KernelOps:
         te = torch.searchsorted(ends, t, right=True)
         tile_expert.copy_(torch.where(te < E, te, torch.full_like(te, -1)).to(torch.int32))
 
+    def moe_table_align(self, table, tokens, E, tile, slots, tile_expert, pair_slot):
+        """``moe_align`` of the experts table[tokens] [T, top]: one launch for small batches."""
+        if E <= 128 and tokens.dtype == torch.long and tokens.is_contiguous() and self._moe_lib.moe_align_small(tokens.numel() * table.shape[1]):
+            self._moe_lib.moe_table_align(table, tokens, E, tile, slots, tile_expert, pair_slot)
+        else:
+            self.moe_align(table.index_select(0, tokens).view(-1), E, tile, slots, tile_expert, pair_slot)
+
     def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0, pairs=0):
         """act: False / 0 none, True / 1 squared ReLU, 2: w = [gate rows; up rows], out = silu(gate) * up, 3: the same
         with the gate clamped at ``limit``; ``row_scale`` fp32 [pairs] multiplies each pair's product before it;
@@ -703,6 +710,9 @@ class ReferenceOps:
 
     def moe_align(self, experts, E, tile, slots, tile_expert, pair_slot):
         ref.moe_align(experts, E, tile, slots, tile_expert, pair_slot)
+
+    def moe_table_align(self, table, tokens, E, tile, slots, tile_expert, pair_slot):
+        ref.moe_align(table.index_select(0, tokens).view(-1), E, tile, slots, tile_expert, pair_slot)
 
     def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0, pairs=0):
         ref.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, int(act), row_scale, limit)

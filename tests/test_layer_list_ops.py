@@ -247,3 +247,22 @@ def test_latent_attention_dma(kv, heads, window, lens, ctxs):
     ops.latent_attention(out, q_abs.cuda(), q.cuda(), proj.cuda(), cache.cuda(), meta, inv.cuda(), heads, dim, rot, kv, gate, scale, window)
     # weights and outputs are rounded to bf16; a score is a sum of kv + rot products, exact to 2^-16 or so, before the exponential
     assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
+
+
+# ------------------------------------------------------------------ experts by token
+@gpu
+@pytest.mark.parametrize("tokens,top", [(1, 2), (48, 3), (3000, 2)])
+def test_moe_table_align(tokens, top):
+    g = torch.Generator().manual_seed(tokens)
+    E, tile, V = 9, 32, 40
+    table = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(V)]).int()
+    ids = torch.randint(0, V, (tokens,), generator=g)
+    P = tokens * top
+    cap = -(-(P + E * (tile - 1)) // tile) * tile
+    ops = get_ops("cuda")
+    slots, tiles, pair = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (cap, cap // tile, P))
+    ops.moe_table_align(table.cuda(), ids.cuda(), E, tile, slots, tiles, pair)
+    experts = table[ids].view(-1)
+    assert torch.equal(tiles.cpu()[pair.cpu().long() // tile], experts)          # a pair's slot lies in a tile of its expert
+    assert torch.equal(slots.cpu()[pair.cpu().long()], torch.arange(P).int())    # and the slot names the pair
+    assert int((slots >= 0).sum()) == P
