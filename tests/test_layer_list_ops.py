@@ -249,6 +249,30 @@ def test_latent_attention_dma(kv, heads, window, lens, ctxs):
     assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
 
 
+# ------------------------------------------------------------------ minGRU
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("width", [4, 260, 1028, 6])
+@pytest.mark.parametrize("lens", [[1], [1, 1, 1], [17], [16, 1, 256], [1, 300, 63]])
+def test_mingru_blocks(lens, width, dtype):
+    """Single rows, waves of 16 rows and blocks of 256 (full, partly filled, several), fresh and carried states, beside the reference scan."""
+    g = torch.Generator().manual_seed(sum(lens) + width)
+    T, n = sum(lens), len(lens)
+    proj = torch.randn(T, 3 * width, generator=g).to(dtype)
+    state, bz, bx = torch.randn(n + 2, width, generator=g), torch.randn(width, generator=g), torch.randn(width, generator=g)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    ctx = torch.tensor([m + (7 if i % 2 else 0) for i, m in enumerate(lens)], dtype=torch.int32)
+    slots = torch.randperm(n + 2, generator=g)[:n].int()
+    want_s, want = state.clone(), torch.empty(T, width, dtype=dtype)
+    ref.mingru_scan(want, want_s, proj, bz, bx, cu, ctx, slots)
+    got_s, got = state.cuda(), torch.empty(T, width, dtype=dtype, device="cuda")
+    get_ops("cuda")._seq.mingru_scan(got, got_s, proj.cuda(), bz.cuda(), bx.cuda(), cu.cuda(), ctx.cuda(), slots.cuda(), max(lens))
+    # every row averages the state with a bounded candidate: errors do not grow with the rows
+    assert (got_s.cpu() - want_s).abs().max() < 64 * 2.0 ** -24 * 6
+    tol = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -18
+    assert ((got.cpu().float() - want.float()).abs() <= tol * want.float().abs() + 1e-5).all()
+
+
 # ------------------------------------------------------------------ experts by token
 @gpu
 @pytest.mark.parametrize("tokens,top", [(1, 2), (48, 3), (3000, 2)])
