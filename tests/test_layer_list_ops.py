@@ -290,3 +290,36 @@ def test_moe_table_align(tokens, top):
     assert torch.equal(tiles.cpu()[pair.cpu().long() // tile], experts)          # a pair's slot lies in a tile of its expert
     assert torch.equal(slots.cpu()[pair.cpu().long()], torch.arange(P).int())    # and the slot names the pair
     assert int((slots >= 0).sum()) == P
+
+
+# ------------------------------------------------------------------ queries, keys and values of window attention
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,kv,maps,dim,vdim,nfreq", [
+    (1, 1, 1, 16, 16, 8), (4, 2, 1, 64, 128, 16), (3, 1, 2, 128, 32, 64), (32, 8, 1, 128, 128, 32), (64, 4, 1, 128, 128, 64),
+    (2, 1, 1, 1024, 256, 0), (5, 1, 1, 32, 512, 16), (2, 1, 1, 48, 64, 8), (2, 2, 1, 64, 64, 12), (130, 2, 1, 128, 128, 8)])
+@pytest.mark.parametrize("mode,v_norm,own", [(0, False, True), (1, True, True), (2, False, True), (3, True, True), (2, False, False)])
+def test_attn_prepare(heads, kv, maps, dim, vdim, nfreq, mode, v_norm, own, dtype):
+    """One item of 16 dims to two per thread, heads whose values do not start at a multiple of their size, each norm, rows
+    without a slot, and sizes of the general kernel."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(heads * dim + mode)
+    T, nq, nk, nv = 5, heads * maps * dim, kv * maps * dim, kv * vdim
+    proj = torch.randn(T, nq + (nk + nv if own else 0) + 16, generator=g).to(dtype)
+    cache = torch.zeros(2, 16, nk + nv, dtype=dtype)
+    inv = 1e4 ** (-torch.arange(nfreq).float() / max(nfreq, 1))
+    positions, slots = torch.tensor([0, 1, 77, 4000, 16000]), torch.tensor([3, -1, 31, 0, 7])
+    n = {1: (nq, nk), 2: (dim, dim)}.get(mode)
+    w = [torch.rand(m, generator=g) + 0.5 for m in n] if n else [None, None]
+    amp, eps = 1.25, 1e-5
+    sp = SimpleNamespace(q_size=nq, k_size=nk, v_size=nv, heads=heads, kv_heads=kv, maps=maps, dim=dim, vdim=vdim, kv_from=None if own else 0,
+                         qk_norm=mode == 1, head_norm=mode == 2, unit_qk=mode == 3, v_norm=v_norm, temp_coef=0.1, temp_every=64,
+                         scaling=SimpleNamespace(amplitude=amp))
+    meta = SimpleNamespace(positions=positions.cuda(), slot_mapping=slots.cuda())
+    p, c = proj.cuda(), cache.cuda()
+    get_ops("cuda").attn_prepare(p, c, meta, inv.cuda(), sp, *[v if v is None else v.cuda() for v in w], eps)
+    ref.attn_prepare(proj, cache, positions, slots, inv, sp, w[0], w[1], eps)
+    # 32-bit: sums of squares and a product or two; an angle of up to 16000 rounds to 2^-10.
+    tol = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -18
+    for got, want in ((p.cpu().float(), proj.float()), (c.cpu().float(), cache.float())):
+        assert ((got - want).abs() <= tol * want.abs() + (2.0 ** -9 if nfreq else 2.0 ** -20) * want.abs().max()).all()
