@@ -161,6 +161,15 @@ void launch_window_attention_mfma(void* out, long out_ld, const void* proj, long
                                   float lam, float post, float eps, int keep, float softcap, const float* sink_w,
                                   bool channel_gate, int chunk, hipStream_t s);
 
+// Decode rows (window_attention_decode.hip), bf16 or fp32: sequences seq0 .. seq0 + rows - 1 have one row each, batch rows
+// row_base on; blocks of a power of two of rows; proj and cache rows at multiples of 16 bytes; nparts and part_keys as above.
+bool window_attention_decode_ok(int dim, int vdim, int block_size, bool f32);
+void launch_window_attention_decode(void* out, long out_ld, const void* proj, long proj_ld, const void* cache, int block_size,
+                                    const int* seq_cu, const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int rows,
+                                    int row_base, int heads, int kv_heads, int dim, int gate_off, float scale, int window,
+                                    bool sink, float out_scale, int nparts, int part_keys, float* ws_acc, float* ws_ml, int keep,
+                                    float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, hipStream_t s);
+
 // Delta-rule recurrences over state slots (delta_scan.hip). Gated rule: proj rows = [q | k | v | ...] with beta's
 // columns from off_b on and the decay's / the gate's pre-activations from off_a / off_g on, or from `decay` (fp32
 // [T, heads * dim]: a decay per key channel) and `gate` ([T, heads * vdim], activation type); dt_bias has as many

@@ -130,6 +130,52 @@ inline void window_attention_mfma(at::Tensor& out, const at::Tensor& proj, const
                                          channel_gate, chunk, cur_stream());
 }
 
+inline bool window_attention_decode_ok(const at::Tensor& proj, const at::Tensor& cache, int64_t dim, int64_t vdim) {
+  const int64_t b = proj.element_size();
+  return (proj.scalar_type() == at::kBFloat16 || proj.scalar_type() == at::kFloat) &&
+         hipserve::window_attention_decode_ok(dim, vdim, cache.size(1), b == 4) && proj.stride(0) * b % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(proj.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(cache.data_ptr()) % 16 == 0;
+}
+
+inline void window_attention_decode(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
+                           const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t seq0, int64_t row_base, int64_t heads,
+                           int64_t kv_heads, int64_t dim, int64_t gate_off, double scale, int64_t window, bool sink,
+                           double out_scale, int64_t nparts, int64_t part_keys, const c10::optional<at::Tensor>& ws_acc,
+                           const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap,
+                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk) {
+  TORCH_CHECK(chunk >= 0 && (chunk == 0 || (window == 0 && keep == 0)), "window attention: chunks or a window");
+  CHECK_DEV(proj); CHECK_CONTIG(cache); CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_bt);
+  const bool f32 = is_f32(proj, "window_attention_decode");
+  TORCH_CHECK(out.scalar_type() == proj.scalar_type() && cache.scalar_type() == proj.scalar_type());
+  TORCH_CHECK(heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && cache.dim() == 3 && cache.size(2) == kv_heads * 2 * dim);
+  const long T = proj.size(0), nseq = seq_ctx.numel(), rows = nseq - seq0;
+  TORCH_CHECK(rows2d(proj) && proj.size(1) >= heads * dim && (gate_off < 0 || proj.size(1) >= gate_off + heads * (channel_gate ? dim : 1)) &&
+              (!channel_gate || gate_off >= 0));
+  TORCH_CHECK(rows2d(out) && out.size(0) == T && out.size(1) == heads * dim);
+  TORCH_CHECK(window_attention_decode_ok(proj, cache, dim, dim), "window_attention_decode: head size, block size or alignment");
+  TORCH_CHECK(seq_cu.numel() == nseq + 1 && seq_bt.dim() == 2 && seq_bt.size(0) >= nseq);
+  TORCH_CHECK(0 <= seq0 && rows >= 0 && window >= 0 && row_base >= 0 && row_base + rows <= T && nparts >= 1 && nparts <= 64 && part_keys > 0);
+  TORCH_CHECK(keep >= 0 && softcap >= 0.0, "window_attention_decode: kept first keys and score cap are not negative");
+  if (sink_w.has_value()) {
+    CHECK_F32(*sink_w);
+    TORCH_CHECK(sink && sink_w->numel() == heads, "window_attention_decode: one sink logit per head");
+  }
+  float *wa = nullptr, *wm = nullptr;
+  if (nparts > 1) {
+    TORCH_CHECK(ws_acc.has_value() && ws_ml.has_value());
+    CHECK_F32(*ws_acc); CHECK_F32(*ws_ml);
+    TORCH_CHECK(ws_acc->numel() >= nparts * heads * rows * dim && ws_ml->numel() >= nparts * heads * rows * 2);
+    wa = ws_acc->data_ptr<float>();
+    wm = ws_ml->data_ptr<float>();
+  }
+  c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
+  hipserve::launch_window_attention_decode(out.data_ptr(), out.stride(0), proj.data_ptr(), proj.stride(0), cache.data_ptr(),
+                                           cache.size(1), seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_bt.data_ptr<int>(),
+                                           seq_bt.size(1), seq0, rows, row_base, heads, kv_heads, dim, gate_off, (float)scale,
+                                           window, sink, (float)out_scale, nparts, part_keys, wa, wm, keep, (float)softcap,
+                                           (const float*)opt_ptr(sink_w), channel_gate, chunk, f32, cur_stream());
+}
+
 inline void activation(at::Tensor& out, const at::Tensor& x, int64_t kind, double c0, double c1) {
   CHECK_DEV(x);
   const bool f32 = is_f32(x, "activation");
@@ -222,6 +268,11 @@ inline void def_window_ops(torch::Library& m) {
         "int row_base, int maps, float lam, float post, float eps, int keep, float softcap, Tensor? sink_w, "
         "bool channel_gate=False, int chunk=0) -> ()");
   m.def("window_attention_mfma_ok(int dim, int vdim, int out_ld, int out_off, int maps) -> bool", &window_attention_mfma_ok);
+  m.def("window_attention_decode_ok(Tensor proj, Tensor cache, int dim, int vdim) -> bool");
+  m.def("window_attention_decode(Tensor(a!) out, Tensor proj, Tensor cache, Tensor seq_cu, Tensor seq_ctx, Tensor seq_bt, "
+        "int seq0, int row_base, int heads, int kv_heads, int dim, int gate_off, float scale, int window, bool sink, "
+        "float out_scale, int nparts, int part_keys, Tensor(b!)? ws_acc, Tensor(c!)? ws_ml, int keep, float softcap, "
+        "Tensor? sink_w, bool channel_gate, int chunk) -> ()");
   m.def("activation(Tensor(a!) out, Tensor x, int kind, float c0, float c1) -> ()");
   m.def("route_topk(Tensor(a!) ids, Tensor(b!) wts, Tensor logits, Tensor? correction, int top, float scale, int E, "
         "int groups, int keep, bool renorm, bool sigmoid=False, bool top2=False) -> ()");
@@ -235,6 +286,8 @@ inline void impl_window_ops(torch::Library& m) {
   m.impl("attn_prepare", &attn_prepare);
   m.impl("window_attention", &window_attention);
   m.impl("window_attention_mfma", &window_attention_mfma);
+  m.impl("window_attention_decode_ok", &window_attention_decode_ok);
+  m.impl("window_attention_decode", &window_attention_decode);
   m.impl("activation", &activation);
   m.impl("route_topk", &route_topk);
   m.impl("route_align", &route_align);

@@ -1,0 +1,315 @@
+// Window attention of decode rows (one token per sequence, one map per head; same cache, masks, sink and gates as
+// window_attention.hip), bf16 and fp32, heads of 64, 128 (and in bf16 256) dims.
+//
+// A workgroup owns up to 16 query heads of one key / value head and a run of keys. Its waves take tiles of 32 keys (fp32: 16)
+// in turn, each with its own running (max, sum) and accumulators, and meet once, at the end. Nothing is shared between the
+// waves, so nothing goes through LDS before that: every operand is loaded as the matrix instruction wants it.
+//   scores S^T = K . Q^T: a lane's part of a key row is 16 consecutive bytes of it;
+//   output O^T = V^T . P^T: the k slots of the instruction stand for the keys whose weights a lane already holds (4 g + i of
+//   each 16), and the instruction's rows for the dims that 16 consecutive bytes of a value row hold, every E-th of a block
+//   of 16 E: a lane loads whole 16-byte parts of its keys' rows, and in bf16 two byte permutations per pair of keys and pair
+//   of dims put the keys of one dim side by side.
+// What bounds it: the chain table -> cache -> scores -> output of one tile, then (many sequences) memory. All loads of a
+// tile are issued at once and no wave waits for another's. A workgroup that stages every tile for four waves of which one has
+// rows (a group of 4 heads) waits for two barriers and a transposing store per 32 keys: one sequence of 100 keys, 8 heads
+// over 2 of 128 dims, in bf16 11.5 us, this 5.8; 16 sequences of 900 keys, 16 heads over 4: 17.4, 13.3 (with the merge); 64
+// sequences of 1024 keys, 32 heads over 8: 78.6, 48.4 (5.5 TB/s). In fp32 the kernel of window_attention.hip, one wave per
+// head and no split over keys: 16 sequences 528 us, this 23.
+#include "seq_common.h"
+#include "hipserve/seq_kernels.h"
+
+namespace hipserve {
+namespace {
+
+constexpr int kMaxRuns = 64;
+constexpr float kLog2e = 1.44269504088896341f;
+
+HS_DEVICE float tanh_fast(float x) {  // 1 - 2 / (e^2x + 1); saturates cleanly at both ends
+  return 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * 2.88539008177792681f) + 1.f);
+}
+
+// Scores and their exponentials: bf16 in the log2 domain; fp32 in the natural one, exp(d) with the rounding error of d log2(e)
+// carried as in sigmoid_f.
+template <typename T> struct Softmax;
+template <> struct Softmax<unsigned short> {
+  static constexpr float kUnit = kLog2e;
+  static HS_DEVICE float exp(float d) { return __builtin_amdgcn_exp2f(d); }
+  static HS_DEVICE float tanh(float x) { return tanh_fast(x); }
+};
+template <> struct Softmax<float> {
+  static constexpr float kUnit = 1.f;
+  static HS_DEVICE float exp(float d) {   // d <= 0
+    if (!(d >= -104.f)) return d < -104.f ? 0.f : d;
+    const float t = d * 1.44269502f, lo = fmaf(d, 1.92596299e-8f, fmaf(d, 1.44269502f, -t)), e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e, lo * 0.693147182f, e);
+  }
+  static HS_DEVICE float tanh(float x) { return tanhf(x); }
+};
+
+template <bool MAX>
+HS_DEVICE float over_rows(float x) {   // over the lanes c, c + 16, c + 32, c + 48
+  const unsigned u = __builtin_bit_cast(unsigned, x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const float a0 = __builtin_bit_cast(float, (unsigned)a[0]), a1 = __builtin_bit_cast(float, (unsigned)a[1]);
+  const unsigned w = __builtin_bit_cast(unsigned, MAX ? fmaxf(a0, a1) : a0 + a1);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  const float b0 = __builtin_bit_cast(float, (unsigned)b[0]), b1 = __builtin_bit_cast(float, (unsigned)b[1]);
+  return MAX ? fmaxf(b0, b1) : b0 + b1;
+}
+
+using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
+
+template <typename T, int D>
+__global__ __launch_bounds__(512) void window_decode_kernel(
+    T* __restrict__ out, long out_ld, const T* __restrict__ proj, long proj_ld, const T* __restrict__ cache, int block_shift,
+    const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0,
+    int hc, int hchunks, int heads, int kv_heads, int gate_off, float scale, int window, bool sink, float out_scale,
+    int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml, int keep, float softcap,
+    const float* __restrict__ sink_w, bool channel_gate, int chunk) {
+  constexpr bool F32 = sizeof(T) == 4;
+  constexpr int SUB = F32 ? 1 : 2, KT = 16 * SUB;          // 16-key tiles and keys of a wave's tile
+  constexpr int QN = F32 ? D / 16 : D / 32;                // 16-byte parts of a row per lane
+  constexpr int E = F32 || D == 64 ? 4 : 8, NB = D / (16 * E);   // dims of a value row per load; loads per row
+  extern __shared__ float lds[];                           // [waves][nh][D]; [waves][16][2]
+  using S = Softmax<T>;
+  const int s = seq0 + blockIdx.x, r0 = seq_cu[s], ctx = seq_ctx[s];
+  if (seq_cu[s + 1] <= r0) return;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
+  const int group = heads / kv_heads, kvh = blockIdx.y / hchunks, h0 = (blockIdx.y % hchunks) * hc;
+  const int nh = min(hc, group - h0), head0 = kvh * group + h0;
+  const int p = ctx - 1, lo_all = first_key(max(p, 0), window, chunk);
+  const int nk = (window > 0 && keep > 0) ? min(keep, lo_all) : 0;   // kept keys below the window
+  const int total = nk + p - lo_all + 1;
+  const int lo = blockIdx.z * part_keys, hi = gridDim.z > 1 ? min(total, lo + part_keys) - 1 : total - 1;
+  const long Dc = 2L * kv_heads * D;
+  const int* bt = seq_bt + (long)s * bt_width;
+  auto row_of = [&](int u) {   // cache row of the u-th visible key; past the run's end: of its last
+    u = min(u, hi);
+    const int j = u < nk ? u : u - nk + lo_all;
+    return cache + (((long)bt[j >> block_shift] << block_shift) + (j & ((1 << block_shift) - 1))) * Dc;
+  };
+  u32x4 q[QN];
+#pragma unroll
+  for (int i = 0; i < QN; ++i) {
+    q[i] = u32x4{0, 0, 0, 0};
+    if (c < nh) q[i] = reinterpret_cast<const u32x4*>(proj + (long)r0 * proj_ld + (long)(head0 + c) * D)[4 * i + g];
+  }
+  f32x4 acc[NB][E];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int j = 0; j < E; ++j) acc[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bool sunk = sink && blockIdx.z == 0 && wave == 0;
+  float m = sunk ? (sink_w != nullptr && c < nh ? sink_w[head0 + c] * S::kUnit : 0.f) : -INFINITY, l = sunk ? 1.f : 0.f;
+  const float unit = scale * S::kUnit, cap = softcap * S::kUnit, icap = softcap > 0.f ? scale / softcap : 0.f;
+
+  for (int u0 = lo + wave * KT; u0 <= hi; u0 += nw * KT) {
+    u32x4 k[SUB][QN];
+    T v[4 * SUB][NB][E];
+#pragma unroll
+    for (int a = 0; a < SUB; ++a) {
+      const T* src = row_of(u0 + 16 * a + c) + (long)kvh * D;
+#pragma unroll
+      for (int i = 0; i < QN; ++i) k[a][i] = reinterpret_cast<const u32x4*>(src)[4 * i + g];
+    }
+#pragma unroll
+    for (int i = 0; i < 4 * SUB; ++i) {
+      const T* src = row_of(u0 + 16 * (i >> 2) + 4 * g + (i & 3)) + (long)(kv_heads + kvh) * D + E * c;
+#pragma unroll
+      for (int b = 0; b < NB; ++b) __builtin_memcpy(v[i][b], __builtin_assume_aligned(src + 16 * E * b, E * sizeof(T)), E * sizeof(T));
+    }
+    f32x4 sc[SUB];
+#pragma unroll
+    for (int a = 0; a < SUB; ++a) {
+      sc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < QN; ++i) {
+        if constexpr (F32) {
+          const f32x4 kf = __builtin_bit_cast(f32x4, k[a][i]), qf = __builtin_bit_cast(f32x4, q[i]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], sc[a], 0, 0, 0);
+        } else {
+          sc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k[a][i]), __builtin_bit_cast(bf16x8, q[i]),
+                                                          sc[a], 0, 0, 0);
+        }
+      }
+    }
+    // lane (c, g): row c against keys 16 a + 4 g + i
+    const bool whole = u0 + KT - 1 <= hi;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int a = 0; a < SUB; ++a)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float x = softcap > 0.f ? cap * S::tanh(sc[a][i] * icap) : sc[a][i] * unit;
+        if (!whole && u0 + 16 * a + 4 * g + i > hi) x = -INFINITY;
+        sc[a][i] = x;
+        mx = fmaxf(mx, x);
+      }
+    const float mn = fmaxf(m, over_rows<true>(mx)), al = mn > -INFINITY ? S::exp(m - mn) : 1.f;
+    float sum = 0.f, w[4 * SUB];
+    u16x8 pk;
+#pragma unroll
+    for (int i = 0; i < 4 * SUB; ++i) {
+      w[i] = mn > -INFINITY ? S::exp(sc[i >> 2][i & 3] - mn) : 0.f;
+      if constexpr (!F32) {
+        pk[i] = f32_to_bf16(w[i]);       // rounded to bf16: what is multiplied, and what is summed
+        w[i] = bf16_to_f32(pk[i]);
+      }
+      sum += w[i];
+    }
+    l = l * al + over_rows<false>(sum);
+    m = mn;
+    if (!whole) {   // a weight of 0 does not hide an infinity behind the run's end
+#pragma unroll
+      for (int i = 0; i < 4 * SUB; ++i)
+        if (u0 + 16 * (i >> 2) + 4 * g + (i & 3) > hi)
+#pragma unroll
+          for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[i][b][e] = 0;
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+#pragma unroll
+      for (int j = 0; j < E; ++j) acc[b][j] *= al;
+      if constexpr (F32) {
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][b][j], w[i], acc[b][j], 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+          u32x4 a;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {   // keys 2 r and 2 r + 1 of dim j
+            unsigned x, y;
+            __builtin_memcpy(&x, &v[2 * r][b][j & ~1], 4);
+            __builtin_memcpy(&y, &v[2 * r + 1][b][j & ~1], 4);
+            a[r] = __builtin_amdgcn_perm(y, x, j & 1 ? 0x07060302u : 0x05040100u);
+          }
+          acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, pk),
+                                                              acc[b][j], 0, 0, 0);
+        }
+      }
+    }
+  }
+  // lane (c, g): row c, dims 16 E b + E (4 g + i) + j
+  float* ml = lds + nw * nh * D;
+  if (c < nh) {
+    float* dst = lds + ((long)wave * nh + c) * D;
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < E; j += 4)
+          *reinterpret_cast<f32x4*>(dst + 16 * E * b + E * (4 * g + i) + j) =
+              f32x4{acc[b][j][i], acc[b][j + 1][i], acc[b][j + 2][i], acc[b][j + 3][i]};
+    if (g == 0) { ml[2 * (wave * 16 + c)] = m; ml[2 * (wave * 16 + c) + 1] = l; }
+  }
+  __syncthreads();
+  for (int it = tid; it < nh * (D / 4); it += blockDim.x) {
+    const int h = it / (D / 4), d = it % (D / 4) * 4;
+    float M = -INFINITY, L = 0.f;
+    for (int w = 0; w < nw; ++w) M = fmaxf(M, ml[2 * (w * 16 + h)]);
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    for (int w = 0; w < nw; ++w) {
+      const float mw = ml[2 * (w * 16 + h)];
+      if (mw == -INFINITY) continue;   // no key
+      const float f = S::exp(mw - M);
+      L += ml[2 * (w * 16 + h) + 1] * f;
+      o += *reinterpret_cast<const f32x4*>(lds + ((long)w * nh + h) * D + d) * f;
+    }
+    const int head = head0 + h;
+    if (gridDim.z > 1) {
+      const long wrow = ((long)blockIdx.z * heads + head) * gridDim.x + blockIdx.x;
+      *reinterpret_cast<f32x4*>(ws_acc + wrow * D + d) = o;
+      if (d == 0) { ws_ml[2 * wrow] = M; ws_ml[2 * wrow + 1] = L; }
+      continue;
+    }
+    float f = out_scale;
+    if (gate_off >= 0 && !channel_gate) f *= sigmoid_f(ldf<T>(proj, (long)r0 * proj_ld + gate_off + head));
+    f = L == 0.f ? 0.f : f / L;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float cg = channel_gate ? sigmoid_f(ldf<T>(proj, (long)r0 * proj_ld + gate_off + (long)head * D + d + e)) : 1.f;
+      stf<T>(out, (long)r0 * out_ld + (long)head * D + d + e, o[e] * f * cg);
+    }
+  }
+}
+
+// out[row_base + r, head] = sum_p acc_p e^(m_p - M) / sum_p l_p e^(m_p - M) * sigmoid(gate) * out_scale
+template <typename T>
+__global__ __launch_bounds__(128) void window_decode_reduce_kernel(
+    T* __restrict__ out, long out_ld, const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
+    const T* __restrict__ proj, long proj_ld, int gate_off, int nparts, int heads, int ws_rows, int row_base, int vdim,
+    float out_scale, bool channel_gate) {
+  using S = Softmax<T>;
+  __shared__ float sc[kMaxRuns];  // each run's weight e^(m_p - M) / L * gate * scale, 0 for empty runs
+  const int r = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const long trow = row_base + r;
+  if (tid < 64) {  // one wave: run p on lane p
+    const long w = ((long)min(tid, nparts - 1) * heads + h) * ws_rows + r;
+    const float m = tid < nparts ? ws_ml[2 * w] : -INFINITY;
+    const float l = tid < nparts ? ws_ml[2 * w + 1] : 0.f;
+    const float M = wave_max(m);
+    const float e = m == -INFINITY ? 0.f : S::exp(m - M);
+    const float L = wave_sum(l * e);
+    float f = out_scale;
+    if (gate_off >= 0 && !channel_gate) f *= sigmoid_f(ldf<T>(proj, trow * proj_ld + gate_off + h));
+    sc[tid] = L == 0.f ? 0.f : e * f / L;
+  }
+  __syncthreads();
+  for (int d = tid; d < vdim; d += 128) {
+    float o = 0.f;
+    for (int p = 0; p < nparts; ++p) o += ws_acc[(((long)p * heads + h) * ws_rows + r) * vdim + d] * sc[p];
+    if (channel_gate) o *= sigmoid_f(ldf<T>(proj, trow * proj_ld + gate_off + (long)h * vdim + d));
+    stf<T>(out, trow * out_ld + (long)h * vdim + d, o);
+  }
+}
+
+template <typename T, int D>
+void launch(T* out, long out_ld, const T* proj, long proj_ld, const T* cache, int block_size, const int* seq_cu,
+            const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int rows, int row_base, int heads, int kv_heads,
+            int gate_off, float scale, int window, bool sink, float out_scale, int nparts, int part_keys, float* ws_acc,
+            float* ws_ml, int keep, float softcap, const float* sink_w, bool channel_gate, int chunk, hipStream_t s) {
+  const int group = heads / kv_heads, hc = std::min(group, 16), hchunks = (group + hc - 1) / hc;
+  // a wave per tile of the run, as many as their accumulators fit 64 KB of LDS
+  const int kt = sizeof(T) == 4 ? 16 : 32;
+  const int nw = std::max(1, std::min({8, (part_keys + kt - 1) / kt, (1 << 14) / (hc * D)}));
+  const size_t smem = ((size_t)nw * hc * D + nw * 32) * sizeof(float);
+  window_decode_kernel<T, D><<<dim3(rows, kv_heads * hchunks, nparts), 64 * nw, smem, s>>>(
+      out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, hc, hchunks, heads,
+      kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk);
+  if (nparts > 1)
+    window_decode_reduce_kernel<T><<<dim3(rows, heads), 128, 0, s>>>(out, out_ld, ws_acc, ws_ml, proj, proj_ld, gate_off, nparts,
+                                                                    heads, rows, row_base, D, out_scale, channel_gate);
+}
+
+}  // namespace
+
+bool window_attention_decode_ok(int dim, int vdim, int block_size, bool f32) {
+  return dim == vdim && (dim == 64 || dim == 128 || (dim == 256 && !f32)) && (block_size & (block_size - 1)) == 0;
+}
+
+void launch_window_attention_decode(void* out, long out_ld, const void* proj, long proj_ld, const void* cache, int block_size,
+                                    const int* seq_cu, const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int rows,
+                                    int row_base, int heads, int kv_heads, int dim, int gate_off, float scale, int window,
+                                    bool sink, float out_scale, int nparts, int part_keys, float* ws_acc, float* ws_ml, int keep,
+                                    float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, hipStream_t s) {
+  if (rows <= 0) return;
+#define HS_WD(T, D)                                                                                                        \
+  launch<T, D>((T*)out, out_ld, (const T*)proj, proj_ld, (const T*)cache, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, \
+               rows, row_base, heads, kv_heads, gate_off, scale, window, sink, out_scale, nparts, part_keys, ws_acc, ws_ml,   \
+               keep, softcap, sink_w, channel_gate, chunk, s)
+  if (f32) { if (dim == 64) HS_WD(float, 64); else HS_WD(float, 128); }
+  else if (dim == 64) HS_WD(unsigned short, 64);
+  else if (dim == 128) HS_WD(unsigned short, 128);
+  else HS_WD(unsigned short, 256);
+#undef HS_WD
+}
+
+}  // namespace hipserve

@@ -307,6 +307,35 @@ class KernelOps:
     WINDOW_MFMA = os.environ.get("HIPSERVE_WINDOW_MFMA", "1") != "0"
     WINDOW_DECODE_RUN = 128  # keys per run of a decode row (a multiple of 32)
 
+    def _window_decode(self, out, proj, cache, meta, sp, gate_off, out_scale, sink_w) -> bool:
+        """The decode rows of ``window_attention`` by the kernel for them; False where it does not take the sizes."""
+        if sp.maps != 1 or not self.WINDOW_MFMA or not self._window_lib.window_attention_decode_ok(proj, cache, sp.dim, sp.vdim):
+            return False
+        nd = meta.num_decode
+        span = min(sp.reach, meta.max_ctx or sp.reach) if sp.reach > 0 else meta.max_ctx
+        groups = nd * sp.kv_heads * -(-(sp.heads // sp.kv_heads) // 16)   # workgroups per run
+        # One run where a second launch to merge runs costs more than it spreads: few keys (200 keys of one sequence, 8 heads
+        # over 2: 7.2 us, two runs 8.1; 400 keys: 9.2, four runs 8.5), or workgroups for half of the chip and no more than
+        # 1024 keys (41 sequences x 4 key heads: 21.3 us, in runs of 128 24.3; 16 sequences: 16.9, in runs 13.3). Longer runs
+        # where there would be many (8000 keys of one sequence, 8 key heads: runs of 256 17.6 us, of 128 22.4) or they would
+        # fill the chip several times over (their unnormalised outputs are written and read once more).
+        part = max(1, span)
+        if span > 256 and (groups < 128 or span > 1024):
+            part = self.WINDOW_DECODE_RUN
+            while -(-span // part) > 32 or groups * -(-span // part) > 1024 and part < span:
+                part *= 2
+        nparts = max(1, -(-span // part))
+        ws_acc = ws_ml = None
+        if nparts > 1:
+            ws_acc = torch.empty(nparts, sp.heads, nd, sp.vdim, device=proj.device, dtype=torch.float32)
+            ws_ml = torch.empty(nparts, sp.heads, nd, 2, device=proj.device, dtype=torch.float32)
+        self._window_lib.window_attention_decode(out, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt,
+                                                 meta.seq_ctx.shape[0] - nd, meta.num_prefill_tokens, sp.heads, sp.kv_heads, sp.dim,
+                                                 gate_off, sp.scale, sp.window, sp.sink, out_scale, nparts, part, ws_acc, ws_ml,
+                                                 sp.keep_first, sp.softcap, sink_w, sp.channel_gate, sp.chunk)
+        return True
+
+
     def window_attention(self, out, proj, cache, meta, sp, gate_off, out_scale=1.0, lam=0.0, eps=0.0, sink_w=None):
         """Prompt portions (the step's first sequences) run several tokens per workgroup, decode
         rows one token per workgroup. Two maps per head (``sp.maps`` = 2): ``lam`` weighs the second
@@ -316,6 +345,8 @@ class KernelOps:
         nd = meta.num_decode
         npf, Tp = nseq - nd, meta.num_prefill_tokens
         diff = (sp.maps, lam, 1.0 - sp.diff, eps, sp.keep_first, sp.softcap, sink_w, sp.channel_gate, sp.chunk)
+        if nd and self._window_decode(out, proj, cache, meta, sp, gate_off, out_scale, sink_w):
+            nseq, nd = npf, 0   # what is left
         if (proj.dtype == torch.bfloat16 and self.WINDOW_MFMA
                 and self._window_lib.window_attention_mfma_ok(sp.dim, sp.vdim, out.stride(0), out.storage_offset(), sp.maps)):
             # bf16: the matrix-core kernel; decode rows split their keys into runs merged by a reduce kernel

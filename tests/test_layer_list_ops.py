@@ -323,3 +323,55 @@ def test_attn_prepare(heads, kv, maps, dim, vdim, nfreq, mode, v_norm, own, dtyp
     tol = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -18
     for got, want in ((p.cpu().float(), proj.float()), (c.cpu().float(), cache.float())):
         assert ((got - want).abs() <= tol * want.abs() + (2.0 ** -9 if nfreq else 2.0 ** -20) * want.abs().max()).all()
+
+
+# ------------------------------------------------------------------ window attention of decode rows
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,kv,dim,ctxs,opts", [
+    (1, 1, 64, [1], {}), (4, 1, 128, [1, 31, 32, 33, 700], {"window": 0}), (8, 2, 128, [16, 17, 300, 257], {"window": 256, "sink": True, "gate": True}),
+    (40, 2, 64, [5, 129, 400], {"window": 100, "keep_first": 7, "softcap": 3.0, "channel_gate": True}),
+    (32, 2, 128, [64, 65, 1500], {"chunk": 64, "sink_w": True}), (16, 1, 256, [3, 290], {"window": 0})])
+def test_window_attention_decode(heads, kv, dim, ctxs, opts, dtype):
+    """One key, runs that end inside a tile, several runs, more than 16 heads per key / value head, and every mask and gate."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(heads * dim)
+    n, bs, gate = len(ctxs), 8, opts.get("gate", False) or opts.get("channel_gate", False)
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=opts.get("window", 0), scale=dim ** -0.5, sink=opts.get("sink", "sink_w" in opts),
+                         keep_first=opts.get("keep_first", 0), softcap=opts.get("softcap", 0.0), channel_gate=opts.get("channel_gate", False),
+                         chunk=opts.get("chunk", 0), diff=0.0, q_size=heads * dim, k_size=kv * dim, v_size=kv * dim, kv_from=None)
+    sp.reach = sp.window + sp.keep_first if sp.window > 0 else sp.chunk
+    width = -(-max(ctxs) // bs)
+    bt = torch.randperm(n * width, generator=g).int().view(n, width)
+    cache = torch.randn(n * width, bs, 2 * kv * dim, generator=g).to(dtype)
+    gate_off = heads * dim
+    proj = torch.randn(n, heads * dim + heads * dim, generator=g).to(dtype)
+    sink_w = torch.randn(heads, generator=g) if opts.get("sink_w") else None
+    cu, ctx = torch.arange(n + 1).int(), torch.tensor(ctxs, dtype=torch.int32)
+    want = torch.empty(n, heads * dim, dtype=torch.float64)
+    rows = cache.double().view(-1, 2 * kv, dim)
+    for s in range(n):
+        p = ctxs[s] - 1
+        lo = p - p % sp.chunk if sp.chunk else max(0, p - sp.window + 1) if sp.window else 0
+        js = sorted(set(range(lo, p + 1)) | (set(range(min(sp.keep_first, p + 1))) if sp.window else set()))
+        kv_rows = rows[[int(bt[s, j // bs]) * bs + j % bs for j in js]]
+        for h in range(heads):
+            k, v = kv_rows[:, h // (heads // kv)], kv_rows[:, kv + h // (heads // kv)]
+            x = k @ proj[s, h * dim:(h + 1) * dim].double() * sp.scale
+            if sp.softcap:
+                x = sp.softcap * torch.tanh(x / sp.softcap)
+            extra = torch.tensor([float(sink_w[h]) if sink_w is not None else 0.0]).double() if sp.sink else torch.empty(0).double()
+            w = torch.softmax(torch.cat([x, extra]), 0)[:len(js)]
+            want[s, h * dim:(h + 1) * dim] = w @ v
+    if gate:
+        gates = torch.sigmoid(proj[:, gate_off:gate_off + (heads * dim if sp.channel_gate else heads)].double())
+        want *= gates if sp.channel_gate else gates.repeat_interleave(dim, 1)
+    ops = get_ops("cuda")
+    meta = SimpleNamespace(seq_ctx=ctx.cuda(), seq_cu=cu.cuda(), seq_bt=bt.cuda(), num_decode=n, num_prefill_tokens=0, max_ctx=max(ctxs))
+    p, c, out = proj.cuda(), cache.cuda(), torch.empty(n, heads * dim, dtype=dtype, device="cuda")
+    taken = ops._window_decode(out, p, c, meta, sp, gate_off if gate else -1, 1.0, None if sink_w is None else sink_w.cuda())
+    assert taken == (dim < 256 or dtype == torch.bfloat16)
+    if taken:
+        # bf16: weights and outputs rounded to 2^-9, the largest value about 4.5; fp32: sums of up to 1500 products
+        tol, least = (2.0 ** -7, 2.0 ** -8) if dtype == torch.bfloat16 else (2.0 ** -18, 2.0 ** -19)
+        assert ((out.double().cpu() - want).abs() <= tol * want.abs() + least * rows.abs().max() * 0.5).all()
