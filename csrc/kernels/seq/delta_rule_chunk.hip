@@ -1,0 +1,354 @@
+// The generalized delta rule of prompt portions in chunks of 16 tokens, heads of 64, fp32 throughout (fp32 matrix cores):
+//   S_t = diag(w_t) S_{t-1} - a_t x_t^T + k_t v_t^T,  x_t = S_{t-1}^T u_t,  o_t = S_t^T r_t
+// (delta_scan.hip: w = exp(-e^-1/2 sigmoid(decay)), u = unit(k), a = sigmoid(a) u). With D_ij the product of the decays of
+// tokens i .. j, S the state before the chunk and strictly lower A_ij = u_i^T D_(j+1)(i-1) a_j, B_ij with k_j for a_j,
+//   X = (1 + A)^-1 (D_0(i-1) u_i S + B V)
+//   O = D_0i r_i S - Pa X + Pk V,   Pa_ij = r_i^T D_(j+1)i a_j (j <= i), Pk_ij with k_j
+//   S' = D_0,15 S - (D_(j+1),15 a_j)^T X + (D_(j+1),15 k_j)^T V
+// so that 16 dependent passes over the state become a few products. A decay is at least exp(-e^-1/2) = 0.545, a chunk's product
+// at least 6e-5: the inner ratios are quotients of products from the chunk's start, and the matrix cores form all pairs.
+//
+// delta_rule_chunk_prepare: all that does not need the state, one workgroup per (head, chunk), straight from the projection.
+// delta_rule_chunk_scan: one workgroup per (sequence, head, 32 value channels) walks the chunks as in delta_chunk.hip, with
+// U = -X: U = U0 + W S (W = -(1 + A)^-1 U), O = R S + Pa U + Pk V, S = E S + KA U + KK V.
+// A product over the chunk would carry a NaN or an infinity of one token's inputs to the tokens before it (0 times it), so such
+// a token takes part as zeros and F carries NaN to its outputs and (unless only r was not finite) all that follow.
+// What bounds it: the prepared operands (6752 floats per head and chunk) are written and read once, and the scan's products.
+// 8192 rows (4 prompts) x 32 heads: rows prepared one by one and scanned token by token (five row vectors through LDS for
+// every 4 state elements of a lane) took @START@; this @NOW@. Relative error of the outputs against 64 bits over 2048 tokens: @ERR@
+#include "seq_common.h"
+#include "hipserve/seq_kernels.h"
+
+namespace hipserve {
+namespace {
+
+constexpr int kC = 16, kD = 64, kLd = kD + 4;   // tokens per chunk; key and value channels of a head; LDS row
+
+// Buffers per (chunk, head): W, R [16][64], KA, KK [64][16], U0, V [64][16], E [64], Pa, Pk [16][16], F [32]
+struct Buf {
+  float *W, *R, *KA, *KK, *U, *V, *E, *Pa, *Pk, *F;
+};
+constexpr long kBuf = 6L * kC * kD + kD + 2 * kC * kC + 2 * kC;
+HS_DEVICE Buf buf_of(float* base, long item) {
+  float* p = base + item * kBuf;
+  constexpr int m = kC * kD;
+  return Buf{p,         p + m,          p + 2 * m,           p + 3 * m, p + 4 * m, p + 5 * m, p + 6 * m, p + 6 * m + kD,
+             p + 6 * m + kD + kC * kC, p + 6 * m + kD + 2 * kC * kC};
+}
+
+// Where a token stands in the buffers' rows and columns: a lane's four values 4 g + r are the tokens 4 r + g, so that the k steps
+// r of a sum over the tokens take the oldest four first. Their decayed parts are small, and the sum rounds to the size it
+// has by then, as token by token.
+HS_DEVICE int place(int t) { return 4 * (t & 3) + (t >> 2); }
+
+HS_DEVICE f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+HS_DEVICE f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+__global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
+    float* __restrict__ base, const unsigned short* __restrict__ proj, long ld, const float* __restrict__ wl,
+    const float* __restrict__ a_b, const float* __restrict__ w0, const int* __restrict__ seq_cu, int nseq, int heads) {
+  __shared__ __attribute__((aligned(16))) float su[kC][kLd], sr[kC][kLd], sa[kC][kLd], sk[kC][kLd], sv[kC][kLd];
+  __shared__ __attribute__((aligned(16))) float sx[kC][kLd], sy[kC][kLd];   // the decays, then KA; KK
+  __shared__ __attribute__((aligned(16))) float sA[kC][20], sB[kC][20], sM[kC][20];
+  __shared__ float sf[2][kC];   // NaN: a token's inputs, its r, are not finite
+  int s, t0;
+  if (!find_row_tile(seq_cu, 0, nseq, kC, blockIdx.y, s, t0)) return;
+  const int h = blockIdx.x, tid = threadIdx.x, row = tid >> 4, ch = 4 * (tid & 15);
+  const int r0 = seq_cu[s] + t0, nt = min(kC, seq_cu[s + 1] - r0), N = heads * kD;
+  const Buf out = buf_of(base, (long)blockIdx.y * heads + h);
+  const bool in = row < nt;
+  {
+    const long t = r0 + (in ? row : 0);
+    const int c = h * kD + ch;
+    float r[4], k[4], v[4], a[4], w[4], ab[4], wb[4], u[4];
+    const unsigned short* p = proj + t * ld + c;
+    Row<unsigned short, 4>::ld(p, r);
+    Row<unsigned short, 4>::ld(p + N, k);
+    Row<unsigned short, 4>::ld(p + 2 * N, v);
+    Row<unsigned short, 4>::ld(p + 3 * N, a);
+    Row<float, 4>::ld(wl + t * N + c, w);
+    Row<float, 4>::ld(a_b + c, ab);
+    Row<float, 4>::ld(w0 + c, wb);
+    float ss = 0.f, f = 0.f, fr = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      ss += k[e] * k[e];
+      f += (k[e] - k[e]) + (v[e] - v[e]) + (a[e] - a[e]) + (w[e] - w[e]);   // 0 or NaN
+      fr += r[e] - r[e];
+    }
+    f = in ? row_sum(f) : 0.f;
+    fr = in ? row_sum(fr) : 0.f;
+    if (ch == 0) { sf[0][row] = f; sf[1][row] = fr; }
+    const bool use = in && f == 0.f;
+    const float inv = 1.f / sqrtf(row_sum(ss) + 1e-6f);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      u[e] = use ? k[e] * inv : 0.f;
+      a[e] = use ? sigmoid_f(a[e] + ab[e]) * u[e] : 0.f;
+      w[e] = use ? expf(-0.60653065971263342f * sigmoid_f(w[e] + wb[e])) : 1.f;
+      if (!use) k[e] = v[e] = 0.f;
+      if (!use || fr != 0.f) r[e] = 0.f;
+    }
+    Row<float, 4>::st(&sx[row][ch], w);
+    __syncthreads();
+    f32x4 before = {1.f, 1.f, 1.f, 1.f}, after = before;   // the decays of the chunk's earlier and later tokens
+#pragma unroll
+    for (int m = 0; m < kC; ++m) {
+      const f32x4 x = ld4(&sx[m][ch]);
+      if (m < row) before *= x;
+      if (m > row) after *= x;
+    }
+    f32x4 ka, kk, upto, U, R, A, K, V;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      upto[e] = before[e] * w[e];
+      U[e] = u[e] * before[e];
+      R[e] = r[e] * upto[e];
+      A[e] = a[e] / upto[e];
+      K[e] = k[e] / upto[e];
+      V[e] = v[e];
+      ka[e] = a[e] * after[e];
+      kk[e] = k[e] * after[e];
+    }
+    *reinterpret_cast<f32x4*>(&su[row][ch]) = U;
+    *reinterpret_cast<f32x4*>(&sr[row][ch]) = R;
+    *reinterpret_cast<f32x4*>(&sa[row][ch]) = A;
+    *reinterpret_cast<f32x4*>(&sk[row][ch]) = K;
+    *reinterpret_cast<f32x4*>(&sv[row][ch]) = V;
+    *reinterpret_cast<f32x4*>(out.R + place(row) * kD + ch) = R;
+    if (row == kC - 1) *reinterpret_cast<f32x4*>(out.E + ch) = upto;
+    __syncthreads();
+    *reinterpret_cast<f32x4*>(&sx[row][ch]) = ka;
+    *reinterpret_cast<f32x4*>(&sy[row][ch]) = kk;
+  }
+  if (tid <= kC) {   // F[i]: added to token i's outputs; F[16]: to all after the chunk
+    float f = tid < kC ? sf[1][tid] : 0.f;
+    for (int m = 0; m < kC; ++m) f += m <= tid ? sf[0][m] : 0.f;
+    out.F[tid < kC ? place(tid) : kC] = f;
+  }
+  // all pairs of tokens: wave 0 A, 1 B, 2 Pa, 3 Pk; lane (c, g) gets rows 4 g + r of column c
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+  {
+    const float(*x)[kLd] = wave < 2 ? su : sr;
+    const float(*y)[kLd] = wave & 1 ? sk : sa;
+    f32x4 d = {0.f, 0.f, 0.f, 0.f}, d2 = d;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 a = ld4(&x[c][16 * q + 4 * g]), b = ld4(&y[c][16 * q + 4 * g]);
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        d = mfma(a[e], b[e], d);
+        d2 = mfma(a[e + 1], b[e + 1], d2);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int i = 4 * g + r;
+      const float x = wave < 2 ? (c < i ? d[r] + d2[r] : 0.f) : (c <= i ? d[r] + d2[r] : 0.f);
+      if (wave == 0) sA[i][c] = x;
+      else if (wave == 1) sB[i][c] = x;
+      else (wave == 2 ? out.Pa : out.Pk)[64 * (c >> 2) + 16 * (c & 3) + place(i)] = x;   // by k step and lane of the scan
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    if (lane < kC) {   // column `lane` of M = (1 + A)^-1
+      float x[kC];
+#pragma unroll
+      for (int i = 0; i < kC; ++i) {
+        float r = i == lane ? 1.f : 0.f;
+#pragma unroll
+        for (int j = 0; j < i; ++j) r = __builtin_fmaf(-sA[i][j], x[j], r);
+        x[i] = r;
+        sM[i][lane] = r;
+      }
+    }
+  } else {
+    for (int i = tid - 64; i < 2 * kD * 4; i += 192) {   // KA, KK transposed
+      const int k = i >> 2 & (kD - 1), q = i & 3;
+      const float(*x)[kLd] = i < kD * 4 ? sx : sy;
+      *reinterpret_cast<f32x4*>((i < kD * 4 ? out.KA : out.KK) + k * kC + 4 * q) = f32x4{x[q][k], x[q + 4][k], x[q + 8][k], x[q + 12][k]};
+    }
+  }
+  __syncthreads();
+  // W = M U, and U0 = -(M B) V with (M B)^T = B^T M^T, whose accumulators are the next product's first operand
+  const int col = 16 * wave + c;
+  const f32x4 m = ld4(&sM[place(c)][4 * g]);
+  f32x4 wv = {0.f, 0.f, 0.f, 0.f}, mb = wv, u0 = wv, v;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    wv = mfma(m[r], su[4 * g + r][col], wv);
+    mb = mfma(sB[4 * g + r][place(c)], m[r], mb);
+    v[r] = sv[4 * r + g][col];
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) u0 = mfma(-mb[r], v[r], u0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) out.W[(4 * g + r) * kD + col] = -wv[r];
+  *reinterpret_cast<f32x4*>(out.U + col * kC + 4 * g) = u0;
+  *reinterpret_cast<f32x4*>(out.V + col * kC + 4 * g) = v;
+}
+
+// Four waves with 16 state rows each, kTiles tiles of 16 value channels. What a CU can take in (about 34 KB per us) bounds it, so
+// nothing but the wave's own rows is loaded: wave 0 and 1 load U0 of a tile (the start of their sums), 2 and 3 V, which
+// goes round with the sums; each does one of the four k steps of Pa U and Pk V, and the outputs are summed with the next
+// chunk's exchange. 16 channels per workgroup with U0, V, Pa and Pk in every wave: 249 us.
+constexpr int kNW = 4, kTiles = 2, kAhead = 4;   // kAhead: chunks in flight
+__global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
+    float* __restrict__ o, float* __restrict__ S, float* __restrict__ base, const int* __restrict__ seq_cu,
+    const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads, long pad) {
+  static_assert(kNW == 2 * kTiles, "U0 and V: a wave per tile each");
+  __shared__ __attribute__((aligned(16))) f32x4 sums[2][2][kTiles][kNW][64];   // [chunk parity][U | the last chunk's O]
+  __shared__ __attribute__((aligned(16))) f32x4 vals[2][kNW][64];              // [chunk parity] U0, V
+  const int s = blockIdx.z, h = blockIdx.x;
+  const int r0 = seq_cu[s], n = seq_cu[s + 1] - r0;
+  if (n <= 0) return;
+  int first = 0;   // the sequence's first chunk in the step
+  for (int i = 0; i < s; ++i) first += (seq_cu[i + 1] - seq_cu[i] + kC - 1) / kC;
+  const int nc = (n + kC - 1) / kC;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
+  const bool odd = threadIdx.x & 64, high = threadIdx.x & 128;   // the wave's bits as lane masks: selects, not branches
+  const int N = heads * kD, k0 = 16 * wave, col0 = 16 * kTiles * blockIdx.y, mine = wave & 1, half = wave >> 1;
+  const bool carried = seq_ctx[s] - n > 0;
+  float* Sp = S + ((long)seq_state[s] * heads + h) * kD * kD + col0 + c;
+  f32x4 st[kTiles];
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) st[t][r] = carried ? Sp[(long)(k0 + 4 * g + r) * kD + 16 * t] : 0.f;
+  // Operands, each loaded kAhead chunks ahead as soon as its registers are free. The loop's loads and stores are unconditional
+  // (past the end the last chunk again, rows that do not exist behind o), so that the wait for an operand never covers the
+  // younger loads behind it.
+  struct Ops {
+    f32x4 W, R, KA, KK, E, X, F;
+    float pa, pk, later;
+  } ops[kAhead];
+  constexpr unsigned kM = kC * kD * sizeof(float);   // bytes of an operand of the buffer
+  const unsigned rows = (c * kD + k0 + 4 * g) * 4, cols = ((k0 + c) * kC + 4 * g) * 4, states = (k0 + 4 * g) * 4, toks = 4 * g * 4,
+                 vals_at = (4 + half) * kM + ((col0 + 16 * mine + c) * kC + 4 * g) * 4, pair = (64 * wave + lane) * 4;
+  auto fetch = [&](Ops& x, int ci) {
+    const char* p = reinterpret_cast<const char*>(base + ((long)(first + min(ci, nc - 1)) * heads + h) * kBuf);
+    auto get = [&](unsigned at) { return *reinterpret_cast<const f32x4*>(p + at); };
+    auto one = [&](unsigned at) { return *reinterpret_cast<const float*>(p + at); };
+    constexpr unsigned kE = 6 * kM, kP = kE + kD * 4, kF = kP + 2 * kC * kC * 4;
+    x.W = get(rows);
+    x.R = get(kM + rows);
+    x.X = get(vals_at);
+    x.F = get(kF + toks);
+    x.KK = get(3 * kM + cols);
+    x.KA = get(2 * kM + cols);
+    x.E = get(kE + states);
+    x.pa = one(kP + pair);
+    x.pk = one(kP + kC * kC * 4 + pair);
+    x.later = one(kF + kC * 4);
+  };
+  auto of_wave = [&](const f32x4& v) { return high ? (odd ? v[3] : v[2]) : odd ? v[1] : v[0]; };
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 os[kTiles] = {};
+  float bad = 0.f;   // NaN once a token's inputs were not finite
+  float* po = o + (long)(r0 + 8 * half + g) * N + h * kD + col0 + 16 * mine + c;
+  float* nowhere = o + pad + lane;
+  // the outputs of chunk ci from the sums in sums[buf]: wave w two rows of tile w % 2
+  auto read_out = [&](int ci, int buf) {
+    float y[2] = {0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kNW; ++w) {
+      const float2 v = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(&sums[buf][1][mine][w][lane]) + 2 * half);
+      y[0] += v.x;
+      y[1] += v.y;
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int i = ci * kC + 8 * half + 4 * e + g;
+      float* to = po + (long)(ci * kC + 4 * e) * N;
+      *((unsigned)i < (unsigned)n ? to : nowhere) = y[e];
+    }
+  };
+  auto step = [&](Ops& x, int ci) {
+    const int buf = ci & 1;
+    f32x4 us[kTiles], u[kTiles], v[kTiles], rs[kTiles];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      us[t] = !high && odd == t ? x.X : zero;
+      rs[t] = !high && !odd ? x.F + bad : zero;
+      sums[buf][1][t][wave][lane] = os[t];
+    }
+    vals[buf][wave][lane] = x.X;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) {
+        us[t] = mfma(x.W[r], st[t][r], us[t]);
+        rs[t] = mfma(x.R[r], st[t][r], rs[t]);
+      }
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      sums[buf][0][t][wave][lane] = us[t];
+      st[t] *= x.E;
+    }
+    __syncthreads();   // the other parity's rows are read before a wave comes here again
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      v[t] = vals[buf][kTiles + t][lane];
+      u[t] = sums[buf][0][t][0][lane];
+#pragma unroll
+      for (int w = 1; w < kNW; ++w) u[t] += sums[buf][0][t][w][lane];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) st[t] = mfma(x.KK[r], v[t][r], st[t]);
+    f32x4 sa[kTiles] = {};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) sa[t] = mfma(x.KA[r], u[t][r], sa[t]);
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) st[t] += sa[t];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      os[t] = mfma(x.pk, of_wave(v[t]), rs[t]);
+      os[t] = mfma(x.pa, of_wave(u[t]), os[t]);
+    }
+    bad += x.later;
+    fetch(x, ci + kAhead);
+    read_out(ci - 1, buf);
+  };
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) fetch(ops[i], i);
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the loop's own waits then count the loop's loads only
+  int ci = 0;
+  for (; ci + kAhead <= nc; ci += kAhead) {   // no exit in between: a wait would cover the loads of the shortest way round
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) step(ops[i], ci + i);
+  }
+#pragma unroll
+  for (int i = 0; i < kAhead - 1; ++i)
+    if (ci + i < nc) step(ops[i], ci + i);
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) sums[nc & 1][1][t][wave][lane] = os[t];
+  __syncthreads();
+  read_out(nc - 1, nc & 1);
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) Sp[(long)(k0 + 4 * g + r) * kD + 16 * t] = st[t][r] + bad;
+}
+
+}  // namespace
+
+bool delta_rule_chunk_ok(int heads, int dim, const void* proj, long ld) {
+  return dim == kD && ld % 4 == 0 && reinterpret_cast<uintptr_t>(proj) % 8 == 0;
+}
+long delta_rule_chunk_floats(int T, int nseq, int heads) { return (T / kC + nseq) * (long)heads * kBuf; }
+
+void launch_delta_rule_chunk(float* o, float* S, float* buf, const void* proj, long ld, const float* wl, const float* a_b,
+                             const float* w0, const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int T,
+                             int heads, hipStream_t s) {
+  delta_rule_chunk_prepare_kernel<<<dim3(heads, T / kC + nseq), 256, 0, s>>>(buf, (const unsigned short*)proj, ld, wl, a_b, w0,
+                                                                             seq_cu, nseq, heads);
+  delta_rule_chunk_scan_kernel<<<dim3(heads, kD / (16 * kTiles), nseq), 64 * kNW, 0, s>>>(o, S, buf, seq_cu, seq_ctx, seq_state, heads,
+                                                                               (long)T * heads * kD);
+}
+
+}  // namespace hipserve

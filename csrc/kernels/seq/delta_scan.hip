@@ -995,9 +995,14 @@ void launch_gated_delta_step(const GatedDelta& p, bool f32, hipStream_t s) {
 void launch_delta_rule(void* out, long out_ld, float* S, const void* proj, long ld, const float* wl, const float* a_b,
                        const float* w0, const float* norm_w, const int* seq_cu, const int* seq_ctx,
                        const int* seq_state, int nseq, int T, float* scratch, int heads, int dim, float eps,
-                       float out_scale, bool f32, hipStream_t s) {
+                       float out_scale, bool f32, float* chunks, hipStream_t s) {
   if (nseq <= 0 || T <= 0) return;
   const int N = heads * dim;
+  if (chunks != nullptr) {
+    launch_delta_rule_chunk(scratch, S, chunks, proj, ld, wl, a_b, w0, seq_cu, seq_ctx, seq_state, nseq, T, heads, s);
+    head_norm_gate<unsigned short>(out, out_ld, scratch, proj, ld, 4 * N, norm_w, dim, T, heads, dim, eps, false, out_scale, s);
+    return;
+  }
   float* pre = scratch;               // [T, 6 N]
   float* o = pre + (long)T * 6 * N;   // [T, N]
   dim3 grid(heads, (dim + kCols - 1) / kCols, nseq);

@@ -208,7 +208,7 @@ void sandwich_update(at::Tensor& out, at::Tensor& residual, const at::Tensor& w_
 void delta_rule(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const at::Tensor& wl, const at::Tensor& a_b,
                 const at::Tensor& w0, const at::Tensor& norm_w, const at::Tensor& seq_cu, const at::Tensor& seq_ctx,
                 const at::Tensor& seq_state, at::Tensor& scratch, int64_t heads, int64_t dim, double eps,
-                double out_scale) {
+                double out_scale, const c10::optional<at::Tensor>& chunks) {
   CHECK_DEV(proj); CHECK_F32(S); CHECK_F32(wl); CHECK_F32(a_b); CHECK_F32(w0); CHECK_F32(norm_w); CHECK_F32(scratch);
   CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_state);
   const bool f32 = is_f32(proj, "delta_rule");
@@ -219,13 +219,25 @@ void delta_rule(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const at
   TORCH_CHECK(S.dim() == 4 && S.size(1) == heads && S.size(2) == dim && S.size(3) == dim);
   TORCH_CHECK(wl.numel() == T * N && a_b.numel() == N && w0.numel() == N && norm_w.numel() == N);
   TORCH_CHECK(seq_cu.numel() == nseq + 1 && seq_state.numel() >= nseq && nseq <= 65535 &&
-              scratch.numel() >= T * 7 * N);
+              scratch.numel() >= (chunks.has_value() ? T * N + 64 : T * 7 * N));
+  if (chunks.has_value()) {
+    CHECK_F32(*chunks);
+    TORCH_CHECK(!f32 && hipserve::delta_rule_chunk_ok(heads, dim, proj.data_ptr(), proj.stride(0)) && T / 16 + nseq <= 65535 &&
+                chunks->numel() >= hipserve::delta_rule_chunk_floats(T, nseq, heads), "delta_rule: not in chunks");
+  }
   c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
   hipserve::launch_delta_rule(out.data_ptr(), out.stride(0), S.data_ptr<float>(), proj.data_ptr(), proj.stride(0),
                               wl.data_ptr<float>(), a_b.data_ptr<float>(), w0.data_ptr<float>(),
                               norm_w.data_ptr<float>(), seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(),
                               seq_state.data_ptr<int>(), nseq, T, scratch.data_ptr<float>(), heads, dim, (float)eps,
-                              (float)out_scale, f32, cur_stream());
+                              (float)out_scale, f32, (float*)opt_ptr(chunks), cur_stream());
+}
+
+// floats of delta_rule's `chunks`; 0: not for these rows
+int64_t delta_rule_chunk_floats(const at::Tensor& proj, int64_t nseq, int64_t heads, int64_t dim) {
+  return proj.scalar_type() == at::kBFloat16 && hipserve::delta_rule_chunk_ok(heads, dim, proj.data_ptr(), proj.stride(0)) &&
+                 proj.size(0) / 16 + nseq <= 65535
+             ? hipserve::delta_rule_chunk_floats(proj.size(0), nseq, heads) : 0;
 }
 
 void add_normed(at::Tensor& out, at::Tensor& residual, const at::Tensor& w, double eps,
@@ -341,7 +353,8 @@ TORCH_LIBRARY(hipserve_delta, m) {
         "float b_scale, Tensor? ye, Tensor? pair_slot, Tensor? wts, Tensor? shared, Tensor? gate) -> ()");
   m.def("delta_rule(Tensor(a!) out, Tensor(b!) S, Tensor proj, Tensor wl, Tensor a_b, Tensor w0, Tensor norm_w, "
         "Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, Tensor(c!) scratch, int heads, int dim, float eps, "
-        "float out_scale) -> ()");
+        "float out_scale, Tensor(d!)? chunks=None) -> ()");
+  m.def("delta_rule_chunk_floats(Tensor proj, int nseq, int heads, int dim) -> int");
   m.def("add_normed(Tensor(a!) out, Tensor(b!) residual, Tensor w, float eps, Tensor? y, Tensor? ye, Tensor? pair_slot, "
         "Tensor? ids, Tensor? wts, int E, Tensor? h, Tensor? shared) -> ()");
   m.def("token_shift(Tensor(a!) out, Tensor x, Tensor(b!) state, Tensor mu, Tensor seq_cu, Tensor seq_ctx, "
@@ -359,6 +372,7 @@ TORCH_LIBRARY_IMPL(hipserve_delta, CUDA, m) {
   m.impl("gated_delta_step", &gated_delta_step);
   m.impl("sandwich_update", &sandwich_update);
   m.impl("delta_rule", &delta_rule);
+  m.impl("delta_rule_chunk_floats", &delta_rule_chunk_floats);
   m.impl("add_normed", &add_normed);
   m.impl("token_shift", &token_shift);
   m.impl("wkv", &wkv);

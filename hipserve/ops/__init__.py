@@ -405,9 +405,13 @@ class KernelOps:
                                      *offs, sp.channel_decay, sp.gate_act == "silu")
 
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
-        scratch = torch.empty(proj.shape[0] * 7 * sp.size, device=proj.device, dtype=torch.float32)
+        T, n = proj.shape[0], 0
+        if self.DELTA_CHUNK and proj.dtype in self.DELTA_CHUNK_DTYPES and meta.max_q >= self.DELTA_CHUNK_ROWS:
+            n = self._delta.delta_rule_chunk_floats(proj, meta.seq_ctx.shape[0], sp.heads, sp.dim)   # 0: not for these sizes
+        chunks = torch.empty(n, device=proj.device, dtype=torch.float32) if n else None
+        scratch = torch.empty(T * sp.size + 64 if n else T * 7 * sp.size, device=proj.device, dtype=torch.float32)
         self._delta.delta_rule(out, state[0], proj, wl, a_b, w0, norm_w, meta.seq_cu, meta.seq_ctx, meta.seq_state,
-                             scratch, sp.heads, sp.dim, eps, out_scale)
+                             scratch, sp.heads, sp.dim, eps, out_scale, chunks)
 
     # ---- dense layers
     SKINNY_ROWS = 64

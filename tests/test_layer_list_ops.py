@@ -375,3 +375,43 @@ def test_window_attention_decode(heads, kv, dim, ctxs, opts, dtype):
         # bf16: weights and outputs rounded to 2^-9, the largest value about 4.5; fp32: sums of up to 1500 products
         tol, least = (2.0 ** -7, 2.0 ** -8) if dtype == torch.bfloat16 else (2.0 ** -18, 2.0 ** -19)
         assert ((out.double().cpu() - want).abs() <= tol * want.abs() + least * rows.abs().max() * 0.5).all()
+
+
+# ------------------------------------------------------------------ generalized delta rule in chunks
+@gpu
+@pytest.mark.parametrize("lens", [[32], [33, 1, 16], [40, 15, 100]])
+def test_delta_rule_chunks(lens):
+    """Whole and partly filled chunks, carried and fresh states, beside the reference; a row that is not finite poisons itself
+    and what follows, not the rows before it."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(sum(lens))
+    H, d, T, n = 3, 64, sum(lens), len(lens)
+    N, eps = H * d, 1e-5
+    proj = torch.randn(T, 5 * N + 64, generator=g).bfloat16()
+    wl, S = torch.randn(T, N, generator=g) * 2, torch.randn(n + 1, H, d, d, generator=g)
+    a_b, w0, nw = torch.randn(N, generator=g), torch.randn(N, generator=g), torch.rand(N, generator=g) + 0.5
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    ctx = torch.tensor([m + (9 if i % 2 == 0 else 0) for i, m in enumerate(lens)], dtype=torch.int32)
+    slots = torch.randperm(n + 1, generator=g)[:n].int()
+    sp = SimpleNamespace(heads=H, dim=d, size=N)
+    meta = SimpleNamespace(seq_cu=cu.cuda(), seq_ctx=ctx.cuda(), seq_state=slots.cuda(), max_q=max(lens))
+    ops = get_ops("cuda")
+    assert ops._delta.delta_rule_chunk_floats(proj.cuda(), n, H, d) > 0
+
+    def run(p):
+        out, state = torch.empty(T, N, dtype=torch.bfloat16, device="cuda"), S.cuda()
+        ops.delta_rule(out, [state], p.cuda(), wl.cuda(), a_b.cuda(), w0.cuda(), nw.cuda(), sp, eps, meta)
+        return out.cpu(), state.cpu()
+    want_s, want = S.clone(), torch.empty(T, N, dtype=torch.bfloat16)
+    ref.delta_rule(want, want_s, proj, wl, a_b, w0, nw, sp, eps, cu, ctx, slots, 1.0)
+    got, got_s = run(proj)
+    # states are sums of about 64 products of either order, 2^-24 each, that a decay of at least 0.545 per row forgets
+    assert ((got_s - want_s).abs() <= 2.0 ** -15 * want_s.abs().max()).all()
+    assert ((got.float() - want.float()).abs() <= 2.0 ** -7 * want.float().abs() + 2.0 ** -13 * want.float().abs().max()).all()
+    for col, last in ((2 * N + 5, lens[0]), (3, 21)):   # a value: the rest of the sequence; r: the row alone
+        bad = proj.clone()
+        bad[20, col] = float("nan")
+        hit = torch.zeros(T, N, dtype=torch.bool)
+        hit[20:last, :d] = True
+        out, _ = run(bad)
+        assert torch.equal(out.isnan(), hit) and torch.equal(out[~hit], got[~hit])
