@@ -161,6 +161,15 @@ void launch_window_attention_mfma(void* out, long out_ld, const void* proj, long
                                   float lam, float post, float eps, int keep, float softcap, const float* sink_w,
                                   bool channel_gate, int chunk, hipStream_t s);
 
+// Its prompt portions for heads of 64 or 128 dims without kept keys (window_attention_dma.hip); wide: 128 rows per workgroup.
+bool window_attention_dma_ok(int dim, int vdim, int block_size, int heads, int kv_heads, const void* proj, long proj_ld,
+                             const void* cache);
+void launch_window_attention_dma(void* out, long out_ld, const void* proj, long proj_ld, const void* cache, int block_size,
+                                 const int* seq_cu, const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int seq1,
+                                 int rows_bound, int heads, int kv_heads, int dim, int gate_off, float scale, int window, bool sink,
+                                 float out_scale, bool wide, float softcap, const float* sink_w, bool channel_gate, int chunk,
+                                 hipStream_t s);
+
 // Decode rows (window_attention_decode.hip), bf16 or fp32: sequences seq0 .. seq0 + rows - 1 have one row each, batch rows
 // row_base on; blocks of a power of two of rows; proj and cache rows at multiples of 16 bytes; nparts and part_keys as above.
 bool window_attention_decode_ok(int dim, int vdim, int block_size, bool f32);

@@ -21,61 +21,24 @@
 // tile's operand reads: 497 us; without uniform copy addresses: 437.
 // latent_dma_decode_kernel serves decode rows: a workgroup takes 16 heads of one sequence and a run of keys, 64 of them
 // at a time; its waves split the keys for S and the latent dims for P . V. One row of 724 keys, 16 heads: 46 -> 10 us.
+#include "lds_copy.h"
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
 
 namespace hipserve {
 namespace {
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
-
 constexpr int kKeys = 32, kRot = 64, kPLd = 40;   // kPLd: row stride of P in elements (16-byte rows, padded)
 constexpr float kLog2e = 1.44269504088896341f;
 
-// All LDS and vector memory operations issued so far are done, then every wave of the workgroup is here.
-HS_DEVICE void barrier_all() {
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-// 1 KB from the lanes' addresses to LDS, 16 bytes per lane side by side, asynchronously. Written out because the compiler
-// would otherwise wait for every copy in flight before the next transposing read; the waits are the callers' barrier_all.
-HS_DEVICE void copy_1k(const unsigned short* src, const unsigned char* lds) {
-  const unsigned at = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(at)), "v"(src) : "memory");   // nothing else in this file uses m0
-}
-// The same from a uniform base and the lanes' byte offsets.
-HS_DEVICE void copy_1k(const unsigned char* base, unsigned off, const unsigned char* lds) {
-  const unsigned at = (unsigned)(uintptr_t)(const __attribute__((address_space(3))) unsigned char*)lds;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(at)), "v"(off), "s"(base) : "memory");
-}
-// The same for LDS operations alone: copies into LDS may still be in flight.
-HS_DEVICE void barrier_lds() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Largest of the values of the lanes c, c + 16, c + 32, c + 48, in all of them (row and half swaps of the vector unit).
-HS_DEVICE float max_of_rows(float x) {
-  const unsigned u = __builtin_bit_cast(unsigned, x);
-  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  const float y = fmaxf(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1]));
-  const unsigned w = __builtin_bit_cast(unsigned, y);
-  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
-}
-
 // K tile rows in LDS: [KEYS][DV] then [KEYS][64]; 16-byte chunk ch of key k sits at chunk ch ^ swizzle(k): eight keys in a
 // row use eight different chunks of a 128-byte line (the key operands), four in a row four different pairs (the values).
-HS_DEVICE int swizzle(int k) { return (k & 3) << 1 | (k >> 2 & 1); }
 template <int DV, int KEYS> struct Tile {
   static constexpr int kMain = KEYS * DV * 2, kBytes = kMain + KEYS * kRot * 2;
   static HS_DEVICE int main_at(int k, int ch) { return k * DV * 2 + ((ch ^ swizzle(k)) << 4); }
   static HS_DEVICE int rot_at(int k, int ch) { return kMain + k * kRot * 2 + ((ch ^ swizzle(k)) << 4); }
   // The wave copies keys 8 w .. 8 w + 7 of the tile; `row` = element offset of key `lane` % KEYS's cache row.
-  static HS_DEVICE void copy(unsigned char* lds, const unsigned short* cache, long row, int w, int lane) {
+  static HS_DEVICE void copy(unsigned lds, const unsigned short* cache, long row, int w, int lane) {
     constexpr int kPer = 512 / DV, kChunks = DV / 8;   // keys and 16-byte chunks of a key in one 1 KB copy
 #pragma unroll
     for (int i = 0; i < 8 / kPer; ++i) {
@@ -190,8 +153,9 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
     const int k = 8 * (wave & 3) + lane / 8;
     off_rot = ((k & mask) * Dk + DV + 8 * ((lane & 7) ^ swizzle(k))) * 2;
   }
+  const unsigned lds0 = lds_at(smem);
   auto copy = [&](int t, int page, int page_rot) {
-    unsigned char* lds = smem + (t & 3) * KT::kBytes;
+    const unsigned lds = lds0 + (t & 3) * KT::kBytes;
     const int j0 = lo + t * kKeys;
     if (j0 + kKeys - 1 <= hi) {   // all keys exist: the addresses differ from tile to tile by uniform numbers
       const unsigned char* base = reinterpret_cast<const unsigned char*>(cache + (((long)page << block_shift) + (j0 & mask)) * Dk);
@@ -412,10 +376,11 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
     const int j = min(j0 + lane, hi);
     return (((long)bt[j >> block_shift] << block_shift) + (j & mask)) * Dk;
   };
+  const unsigned lds0 = lds_at(smem);
   auto copy = [&](int j0) {
     const long row = row_of(j0);
-    KT::copy(smem, cache, row, 2 * wave, lane);
-    KT::copy(smem, cache, row, 2 * wave + 1, lane);
+    KT::copy(lds0, cache, row, 2 * wave, lane);
+    KT::copy(lds0, cache, row, 2 * wave + 1, lane);
   };
   copy(lo);
   bf16x8 qf[KS];

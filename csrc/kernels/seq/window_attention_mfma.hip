@@ -476,6 +476,12 @@ void launch_window_attention_mfma(void* out, long out_ld, const void* proj, long
   const int ks = (dim + 31) / 32, nv = (vdim + 15) / 16;
   const bool wide = nparts == 1 && (long)rows_bound * (heads / kv_heads) >= 128 * (long)(seq1 - seq0) &&
                     (wide_wgs < 64 || wide_wgs >= 1024);
+  if (maps == 1 && nparts == 1 && keep == 0 && scale > 0.f && window_attention_dma_ok(dim, vdim, block_size, heads, kv_heads, proj, proj_ld, cache)) {
+    launch_window_attention_dma(out, out_ld, proj, proj_ld, cache, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1,
+                                rows_bound, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale, wide, softcap, sink_w,
+                                channel_gate, chunk, s);
+    return;
+  }
   if (maps == 2) {
     // row tiles come in pairs (the two maps): 64 rows per workgroup. Four tiles per wave (128 rows) measured
     // slower on 4 x 2048-row prompts (532 against 396 us with 64-dim maps and 128-dim values): too many registers.
