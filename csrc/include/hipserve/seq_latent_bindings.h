@@ -88,7 +88,7 @@ inline void latent_attention_mfma(at::Tensor& o_lat, at::Tensor& qc, const c10::
   }
   c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
   auto aligned = [](const void* p) { return (uintptr_t)p % 16 == 0; };
-  if (hipserve::latent_attention_dma_ok(kv_rank, rot_dim) && cache.size(1) >= 16 &&
+  if (hipserve::latent_attention_dma_ok(kv_rank, rot_dim) && scale > 0 && cache.size(1) >= 16 &&
       (cache.size(1) & (cache.size(1) - 1)) == 0 && aligned(cache.data_ptr()) && aligned(qc.data_ptr())) {
     // the absorbed queries lie in qc already and all 64 rotary dims rotate: the rotary part is formed by the attention itself
     const bool rotate = !q_abs.has_value() && inv_freq.numel() == 32 && dim % 8 == 0 && aligned(q.data_ptr());

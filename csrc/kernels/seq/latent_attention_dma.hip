@@ -5,9 +5,9 @@
 // lookup and for its rows (about 3 us) before 0.5 us of products, its operand reads wait one by one (no registers left),
 // and the V operand of P . V is gathered from LDS two bytes at a time. Here
 //   * global_load_lds brings the rows into one of four LDS buffers, a tile ahead of the scores;
-//   * a buffer holds [32][latent dims] and [32][64 rotary dims]; the eight 16-byte chunks of every 128 bytes are
-//     XOR-swizzled by the key, by choosing which chunk a lane copies, so that both the row-wise operand reads of
-//     S = K . Q^T and the transposing reads below spread over the banks without padding;
+//   * a buffer holds [32][latent dims] and [32][64 rotary dims]; the 16-byte chunks of a row are XOR-swizzled by the key, by
+//     choosing which chunk a lane copies, so that neither the row-wise operand reads of S = K . Q^T nor the transposing
+//     reads below meet in a bank, without padding;
 //   * the V^T operand comes from ds_read_tr16_b64: within 16 lanes, lane l gets element l % 4 of the 8 bytes that lane
 //     4 j + l / 4 addresses, j = 0 .. 3. Lane (c, g) addresses key 16 h + 4 g + c / 4, dims 4 (c % 4) .. + 3 and so
 //     receives keys 16 h + 4 g + 0 .. 3 of dim c: half of an MFMA operand in the key order of P;
@@ -15,10 +15,12 @@
 //     DV / 4 latent dims each for all 64 rows: the softmax of one tile runs beside the products of another, neither half
 //     holds the other's registers (queries 72, outputs 128 per lane), and a tile costs one barrier;
 //   * the queries' rotary part is rotated when the operands are loaded (its halves meet in one lane), no pass of its own.
-// 8192 rows (4 prompts) x 16 heads, 512 + 64 dims, window 1024: 980 -> 416 us (540 TFLOP/s). A tile of 64 rows takes about 3700
-// cycles of its SIMDs: 1088 of products, 1400 of vector instructions (softmax, conversions), the rest waits at the one barrier
-// per tile; its LDS reads (every K row goes to four waves, 181 KB) take 1600. Counted without overlap of the scores with the next
-// tile's operand reads: 497 us; without uniform copy addresses: 437.
+//   * maxima are taken of the raw products, sums come from a product with ones, and the accumulators (128 per lane) are
+//     rescaled only when a maximum grows by more than kSlack.
+// 8192 rows (4 prompts) x 16 heads, 512 + 64 dims, window 1024: 980 -> 341 us (660 TFLOP/s; 690 k cycles, of which a SIMD's matrix
+// unit is busy 220 k, the vector unit 125 k, the LDS 180 k; the rest waits for operands and at the one barrier per tile).
+// On the way, in one run: 449 with eight-way swizzles (operand rows met two to a bank) and a rescaling per tile; 386 with
+// the rescaling mended. Without overlap of the scores with the next tile's operand reads a fifth more.
 // latent_dma_decode_kernel serves decode rows: a workgroup takes 16 heads of one sequence and a run of keys, 64 of them
 // at a time; its waves split the keys for S and the latent dims for P . V. One row of 724 keys, 16 heads: 46 -> 10 us.
 #include "lds_copy.h"
@@ -31,12 +33,16 @@ namespace {
 constexpr int kKeys = 32, kRot = 64, kPLd = 40;   // kPLd: row stride of P in elements (16-byte rows, padded)
 constexpr float kLog2e = 1.44269504088896341f;
 
-// K tile rows in LDS: [KEYS][DV] then [KEYS][64]; 16-byte chunk ch of key k sits at chunk ch ^ swizzle(k): eight keys in a
-// row use eight different chunks of a 128-byte line (the key operands), four in a row four different pairs (the values).
+// K tile rows in LDS: [KEYS][DV] then [KEYS][64]; 16-byte chunk ch of key k sits at chunk ch ^ swizzle(k) (rotary part:
+// ch ^ rot_swizzle(k), rows of 128 bytes, two fill the banks): the 16 keys of an operand use 16 different chunks of 256 bytes,
+// the 8 keys of a transposing read 8 different pairs.
+// (An operand's lanes are served in groups of keys 0 - 3, 12 - 15 with chunk x and 4 - 11 with chunk x ^ 1: bit 3 goes into bit 2 too.)
+HS_DEVICE int swizzle(int k) { return ((k ^ (k >> 1 & 4)) & 7) << 1 | (k >> 3 & 1); }
+HS_DEVICE int rot_swizzle(int k) { return k >> 1 & 7; }
 template <int DV, int KEYS> struct Tile {
   static constexpr int kMain = KEYS * DV * 2, kBytes = kMain + KEYS * kRot * 2;
   static HS_DEVICE int main_at(int k, int ch) { return k * DV * 2 + ((ch ^ swizzle(k)) << 4); }
-  static HS_DEVICE int rot_at(int k, int ch) { return kMain + k * kRot * 2 + ((ch ^ swizzle(k)) << 4); }
+  static HS_DEVICE int rot_at(int k, int ch) { return kMain + k * kRot * 2 + ((ch ^ rot_swizzle(k)) << 4); }
   // The wave copies keys 8 w .. 8 w + 7 of the tile; `row` = element offset of key `lane` % KEYS's cache row.
   static HS_DEVICE void copy(unsigned lds, const unsigned short* cache, long row, int w, int lane) {
     constexpr int kPer = 512 / DV, kChunks = DV / 8;   // keys and 16-byte chunks of a key in one 1 KB copy
@@ -46,18 +52,20 @@ template <int DV, int KEYS> struct Tile {
       const unsigned short* src = cache + __shfl(row, k, 64) + 8 * ch;
       copy_1k(src, lds + (8 * w + i * kPer) * DV * 2);
     }
-    const int k = 8 * w + lane / 8, ch = (lane & 7) ^ swizzle(k);
+    const int k = 8 * w + lane / 8, ch = (lane & 7) ^ rot_swizzle(k);
     const unsigned short* src = cache + __shfl(row, k, 64) + DV + 8 * ch;
     copy_1k(src, lds + kMain + 8 * w * kRot * 2);
   }
-  // The lane's places in a tile: the swizzle touches three bits of the chunk, so two (keys) and up to four (values)
+  // The lane's places in a tile: the swizzle touches four bits of the chunk, so four (keys) and up to eight (values)
   // offsets serve all operands, with constants added.
-  static constexpr int NPW = DV / 64, JB = NPW < 4 ? NPW : 4;   // 16-dim value tiles per wave
-  struct Places { int key[2], rot[2], val[JB]; };
+  static constexpr int NPW = DV / 64, JB = NPW < 8 ? NPW : 8;   // 16-dim value tiles per wave
+  struct Places { int key[4], rot[2], val[JB]; };
   static HS_DEVICE Places places(int wave, int c, int g) {
     Places p;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) { p.key[i] = main_at(c, 4 * i + g); p.rot[i] = rot_at(c, 4 * i + g); }
+    for (int i = 0; i < 4; ++i) p.key[i] = main_at(c, 4 * i + g);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) p.rot[i] = rot_at(c, 4 * i + g);
 #pragma unroll
     for (int j = 0; j < JB; ++j)
       p.val[j] = main_at(4 * g + (c >> 2), 2 * (wave * NPW + j) + ((c & 3) >> 1)) + 8 * (c & 1);
@@ -65,7 +73,7 @@ template <int DV, int KEYS> struct Tile {
   }
   // MFMA operand of 32-dim step ks of key rows k0 + c (k0 a multiple of 16): dims 32 ks + 8 g .. + 7
   static HS_DEVICE bf16x8 key_operand(const unsigned char* lds, const Places& p, int k0, int ks) {
-    const int at = ks < DV / 32 ? p.key[ks & 1] + (ks >> 1) * 128 + k0 * DV * 2 : p.rot[ks & 1] + k0 * kRot * 2;
+    const int at = ks < DV / 32 ? p.key[ks & 3] + (ks >> 2) * 256 + k0 * DV * 2 : p.rot[ks & 1] + k0 * kRot * 2;
     return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u16x8*>(lds + at));
   }
   // MFMA operand of the wave's value tile j against keys k0 .. k0 + 31 (k0 a multiple of 32): lane (c, g) holds dim c,
@@ -75,7 +83,7 @@ template <int DV, int KEYS> struct Tile {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       h[i] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (lds_s16x4)(lds + p.val[j % JB] + (j / JB) * 128 + (k0 + 16 * i) * DV * 2));
+          (lds_s16x4)(lds + p.val[j] + (k0 + 16 * i) * DV * 2));
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5, 6, 7));
   }
 };
@@ -151,7 +159,7 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
   }
   {
     const int k = 8 * (wave & 3) + lane / 8;
-    off_rot = ((k & mask) * Dk + DV + 8 * ((lane & 7) ^ swizzle(k))) * 2;
+    off_rot = ((k & mask) * Dk + DV + 8 * ((lane & 7) ^ rot_swizzle(k))) * 2;
   }
   const unsigned lds0 = lds_at(smem);
   auto copy = [&](int t, int page, int page_rot) {
@@ -173,7 +181,7 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
       copy_1k(src, lds + (4 * wave + i * kPer) * DV * 2);
     }
     if (wave < 4) {
-      const int k = 8 * wave + lane / 8, ch = (lane & 7) ^ swizzle(k);
+      const int k = 8 * wave + lane / 8, ch = (lane & 7) ^ rot_swizzle(k);
       const unsigned short* src = cache + (((long)page_rot << block_shift) + (min(j0 + k, hi) & mask)) * Dk + DV + 8 * ch;
       copy_1k(src, lds + KT::kMain + 8 * wave * kRot * 2);
     }
@@ -200,7 +208,9 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
     load_query<DV>(qf, sact, qc + ((long)shead * T_rows + strow) * Dk,
                    q != nullptr ? q + strow * heads * (dim + kRot) + (long)shead * (dim + kRot) + dim : nullptr,
                    (float)positions[strow], inv_freq, g);
-    float m_run = -INFINITY, l_run = 0.f;   // l_run: this lane's keys only
+    float m_run = -INFINITY;   // what the weights are relative to, log2 domain
+    f32x4 lsum = {0.f, 0.f, 0.f, 0.f};   // sums of the weights that are multiplied, the same number in all four
+    const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
     const float scale2 = scale * kLog2e;
     constexpr int kBatch = 6, kBatches = (KS + kBatch - 1) / kBatch;   // steps whose operands are read together
     bf16x8 ka[2][kBatch][2];
@@ -241,43 +251,42 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
       // masked online softmax (log2 domain) of tile i - 1, row sr: lane (c, g) holds keys 16 nt + 4 g + e
       const int j0 = lo + (i - 1) * kKeys;
       float v[8], mx = -INFINITY;
-      if (__all(sact && j0 + kKeys - 1 <= spos && j0 >= s_lo)) {   // every row of the wave sees the whole tile
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { v[e] = sc[e >> 2][e & 3] * scale2; mx = fmaxf(mx, v[e]); }
-      } else {
+      for (int e = 0; e < 8; ++e) v[e] = sc[e >> 2][e & 3];
+      if (!__all(sact && j0 + kKeys - 1 <= spos && j0 >= s_lo)) {   // not every row of the wave sees the whole tile
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const int j = j0 + 16 * (e >> 2) + 4 * g + (e & 3);
-          v[e] = sact && j <= spos && j >= s_lo ? sc[e >> 2][e & 3] * scale2 : -INFINITY;
-          mx = fmaxf(mx, v[e]);
+          if (!sact || j > spos || j < s_lo) v[e] = -INFINITY;
         }
       }
-      mx = max_of_rows(mx);
-      const float mn = fmaxf(m_run, mx);
-      const float off = mn > -INFINITY ? mn : 0.f;   // no key seen yet: every weight is exp2(-inf) = 0
-      float sum = 0.f;
-      u16x8 pk;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pk[e] = f32_to_bf16(__builtin_amdgcn_exp2f(v[e] - off));   // rounded: what is multiplied, and its sum
-        sum += bf16_to_f32(pk[e]);
+      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, v[e]);
+      mx = max_of_rows(mx) * scale2;
+      float al = 1.f;
+      if (__any(mx > m_run + kSlack)) {
+        const float mn = fmaxf(m_run, mx);
+        al = mn > -INFINITY ? __builtin_amdgcn_exp2f(m_run - mn) : 1.f;  // m_run = -inf: 0
+        m_run = mn;
+        lsum *= al;
       }
+      const float off = m_run > -INFINITY ? m_run : 0.f;   // no key seen yet: every weight is exp2(-inf) = 0
+      u32x4 pk;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2)   // rounded: what is multiplied, and its sum
+        pk[e / 2] = pack2(__builtin_amdgcn_exp2f(fmaf(v[e], scale2, -off)), __builtin_amdgcn_exp2f(fmaf(v[e + 1], scale2, -off)));
       const int pb = (i - 1) & 1;
-      *reinterpret_cast<u16x8*>(p_lds + (pb * 64 + sr) * kPLd + 8 * g) = pk;
-      const float al = mn > -INFINITY ? __builtin_amdgcn_exp2f(m_run - mn) : 1.f;  // m_run = -inf: 0
+      *reinterpret_cast<u32x4*>(p_lds + (pb * 64 + sr) * kPLd + 8 * g) = pk;
       if (g == 0) alpha[pb * 64 + sr] = al;
-      l_run = l_run * al + sum;
-      m_run = mn;
+      lsum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ones), __builtin_bit_cast(bf16x8, pk), lsum, 0, 0, 0);
       barrier_all();
       copy_next(i + 2);
       if (i < ntiles) multiply(i);
     }
-    l_run += __shfl_xor(l_run, 16, 64);
-    l_run += __shfl_xor(l_run, 32, 64);
     if (g == 0) {   // gate / softmax sum of the row
       float f = 0.f;
-      if (sact && l_run > 0.f) {
-        f = 1.f / l_run;
+      if (sact && lsum[0] > 0.f) {
+        f = 1.f / lsum[0];
         if (gate_off >= 0) f *= sigmoid_f(bf16_to_f32(proj[strow * proj_ld + gate_off + shead]));
       }
       l_lds[sr] = f;
@@ -309,7 +318,7 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
 #pragma unroll
     for (int j = 0; j < NPW; ++j) va[j] = KT::value_operand(kt, at, 0, j);
     __builtin_amdgcn_sched_barrier(0);
-    if (__any(rescale)) {   // the running maxima settle after a few tiles: most tiles skip this
+    if (__any(rescale)) {   // rarely: kSlack
 #pragma unroll
       for (int j = 0; j < NPW; ++j)
 #pragma unroll

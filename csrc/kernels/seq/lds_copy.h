@@ -51,8 +51,14 @@ template <int N> HS_DEVICE void barrier_copies() {
   asm volatile("" ::: "memory");
 }
 
-// 16-byte chunk ch of row k sits at chunk ch ^ swizzle(k) of it: eight rows use eight different chunks of a 128-byte line
-// (row-wise operand reads), four rows four different pairs (transposing reads).
-HS_DEVICE int swizzle(int k) { return (k & 3) << 1 | (k >> 2 & 1); }
+// A row's softmax weights are relative to a running maximum that follows only when a score is larger by 2^kSlack: most tiles
+// need no rescaling then, and bf16 weights up to 256 are as precise as weights up to 1.
+constexpr float kSlack = 8.f;
+
+HS_DEVICE unsigned pack2(float a, float b) {
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
 
 }  // namespace hipserve

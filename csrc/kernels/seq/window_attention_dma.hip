@@ -35,16 +35,6 @@ HS_DEVICE float tanh_fast(float x) {  // 1 - 2 / (e^2x + 1); saturates cleanly a
 template <int D> HS_DEVICE int key_swizzle(int k) { return D == 128 ? k & 15 : k >> 1 & 7; }
 template <int D> HS_DEVICE int value_swizzle(int k) { return (D == 128 ? k & 7 : k >> 1 & 3) << 1; }
 
-// A row's weights are relative to a running maximum that follows only when a score is larger by 2^kSlack: most tiles
-// need no rescaling then, and bf16 weights up to 256 are as precise as weights up to 1.
-constexpr float kSlack = 8.f;
-
-HS_DEVICE unsigned pack2(float a, float b) {
-  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-  typedef float f32x2 __attribute__((ext_vector_type(2)));
-  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
-}
-
 // MT: 16-row tiles per wave; 64 MT (token, head) rows of one key / value head per workgroup.
 template <int D, int MT>
 __global__ __launch_bounds__(kThreads, 2) void window_dma_prefill_kernel(
