@@ -405,6 +405,10 @@ class KernelOps:
                                      *offs, sp.channel_decay, sp.gate_act == "silu")
 
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
+        if meta.max_q == 1 and self._delta.delta_rule_step_ok(sp.dim):   # decode steps: one launch
+            self._delta.delta_rule_step(out, state[0], proj, wl, a_b, w0, norm_w, meta.seq_cu, meta.seq_ctx, meta.seq_state,
+                                        sp.heads, sp.dim, eps, out_scale)
+            return
         T, n = proj.shape[0], 0
         if self.DELTA_CHUNK and proj.dtype in self.DELTA_CHUNK_DTYPES and meta.max_q >= self.DELTA_CHUNK_ROWS:
             n = self._delta.delta_rule_chunk_floats(proj, meta.seq_ctx.shape[0], sp.heads, sp.dim)   # 0: not for these sizes

@@ -464,3 +464,25 @@ def test_window_attention_prompts(heads, kv, dim, bs, lens, ctxs, opts):
     get_ops("cuda").window_attention(out, proj.cuda(), cache.cuda(), meta, sp, heads * dim if gate else -1, 1.0, 0.0, 0.0, None if sink_w is None else sink_w.cuda())
     # weights and outputs rounded to 2^-9, the largest value about 4.5
     assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * rows.abs().max() * 0.5).all()
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_delta_rule_step(dtype):
+    """One row per sequence, fresh and carried states, a sequence without a row, in one launch beside the reference."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(5)
+    H, d, cu = 3, 64, [0, 1, 2, 2, 3]
+    N, T, n, eps = H * d, 3, 4, 1e-5
+    proj = torch.randn(T, 5 * N + 4, generator=g).to(dtype)
+    wl, S = torch.randn(T, N, generator=g) * 2, torch.randn(n + 1, H, d, d, generator=g)
+    a_b, w0, nw = torch.randn(N, generator=g), torch.randn(N, generator=g), torch.rand(N, generator=g) + 0.5
+    cu, ctx, slots = torch.tensor(cu).int(), torch.tensor([1, 9, 4, 2]).int(), torch.tensor([4, 0, 3, 1]).int()
+    sp, meta = SimpleNamespace(heads=H, dim=d, size=N), SimpleNamespace(seq_cu=cu.cuda(), seq_ctx=ctx.cuda(), seq_state=slots.cuda(), max_q=1)
+    want_s, want = S.clone(), torch.empty(T, N, dtype=dtype)
+    ref.delta_rule(want, want_s, proj, wl, a_b, w0, nw, sp, eps, cu, ctx, slots, 1.5)
+    got_s, got = S.cuda(), torch.empty(T, N, dtype=dtype, device="cuda")
+    get_ops("cuda").delta_rule(got, [got_s], proj.cuda(), wl.cuda(), a_b.cuda(), w0.cuda(), nw.cuda(), sp, eps, meta, 1.5)
+    assert ((got_s.cpu() - want_s).abs() <= 64 * 2.0 ** -24 * want_s.abs().max()).all()   # a sum of 64 products
+    tol, least = (2.0 ** -7, 2.0 ** -13) if dtype == torch.bfloat16 else (2.0 ** -17, 2.0 ** -17)
+    assert ((got.cpu().float() - want.float()).abs() <= tol * want.float().abs() + least * want.float().abs().max()).all()
