@@ -56,6 +56,94 @@ __global__ __launch_bounds__(256) void latent_prepare_kernel(
   }
 }
 
+// The same for ranks and rotary dims that are multiples of 8 and rows at multiples of 16 bytes: the row is read once, into
+// registers, by 16-byte accesses, the last wave rotates while the others sum, and one barrier serves both norms. What bounds
+// it is that chain. Three passes of 2-byte accesses with two sums one after the other took 7.1 us for one row of 1024 + 512 +
+// 64 in bf16 and 37 for 8192 rows, this 2.6 and 19.
+template <typename T, int N>
+__global__ __launch_bounds__(1024) void latent_prepare_vec_kernel(
+    T* __restrict__ cq, T* __restrict__ cache, const T* __restrict__ proj, long ld, const long* __restrict__ positions,
+    const long* __restrict__ slots, const float* __restrict__ q_norm, const float* __restrict__ kv_norm,
+    const float* __restrict__ inv_freq, int nfreq, int q_rank, int kv_rank, int rot_dim, float eps) {
+  __shared__ float sums[2][16];
+  const long t = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = (blockDim.x >> 6) - 1;   // nw waves, and the rotating one
+  const T* row = proj + t * ld;
+  const long slot = slots[t];
+  T* dst = cache + slot * (kv_rank + rot_dim);
+  if (wave == nw) {
+    const T* kr = row + q_rank + kv_rank;
+    const float pos = (float)positions[t];
+    for (int e = lane; e < rot_dim && slot >= 0; e += 64) {
+      float v;
+      if (e < 2 * nfreq) {
+        const int i = e < nfreq ? e : e - nfreq;
+        const float u = ldf<T>(kr, i), w = ldf<T>(kr, i + nfreq);
+        float sn, cs;
+        sincosf(pos * inv_freq[i], &sn, &cs);
+        v = e < nfreq ? u * cs - w * sn : w * cs + u * sn;
+      } else {
+        v = ldf<T>(kr, e);
+      }
+      stf<T>(dst, kv_rank + e, v);
+    }
+    __syncthreads();
+    return;
+  }
+  const int nt = 64 * nw, rank = q_rank + kv_rank;
+  float x[N][8], w[N][8];
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const int e = 8 * (tid + n * nt);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[n][i] = 0.f;
+    if (e < rank) {
+      Row<T, 8>::ld(row + e, x[n]);
+      Row<float, 8>::ld(e < q_rank ? q_norm + e : kv_norm + e - q_rank, w[n]);
+    }
+  }
+  float a = 0.f, b = 0.f;
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    float v = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v += x[n][i] * x[n][i];
+    if (8 * (tid + n * nt) < q_rank) a += v; else b += v;
+  }
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if (lane == 0) { sums[0][wave] = a; sums[1][wave] = b; }
+  __syncthreads();
+  a = b = 0.f;
+  for (int i = 0; i < nw; ++i) { a += sums[0][i]; b += sums[1][i]; }
+  const float ia = 1.f / sqrtf(a / (float)q_rank + eps), ib = 1.f / sqrtf(b / (float)kv_rank + eps);
+#pragma unroll
+  for (int n = 0; n < N; ++n) {
+    const int e = 8 * (tid + n * nt);
+    if (e >= rank || (e >= q_rank && slot < 0)) continue;
+    const float f = e < q_rank ? ia : ib;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[n][i] = x[n][i] * f * w[n][i];
+    Row<T, 8>::st(e < q_rank ? cq + t * q_rank + e : dst + e - q_rank, x[n]);
+  }
+}
+
+template <typename T>
+bool prepare_vec(T* cq, T* cache, const T* proj, long ld, const long* positions, const long* slots, const float* q_norm,
+                 const float* kv_norm, const float* inv_freq, int nfreq, int T_rows, int q_rank, int kv_rank, int rot_dim, float eps,
+                 hipStream_t s) {
+  uintptr_t at = ld * sizeof(T);
+  for (const void* p : {(const void*)cq, (const void*)cache, (const void*)proj, (const void*)q_norm, (const void*)kv_norm})
+    at |= reinterpret_cast<uintptr_t>(p);
+  const int items = (q_rank + kv_rank) / 8;
+  if (q_rank % 8 != 0 || kv_rank % 8 != 0 || rot_dim % 8 != 0 || at % 16 != 0 || items > 15 * 64 * 2) return false;
+  const int n = items > 15 * 64 ? 2 : 1, nw = (items + 64 * n - 1) / (64 * n);
+  auto kern = n == 1 ? latent_prepare_vec_kernel<T, 1> : latent_prepare_vec_kernel<T, 2>;
+  kern<<<T_rows, 64 * (nw + 1), 0, s>>>(cq, cache, proj, ld, positions, slots, q_norm, kv_norm, inv_freq, nfreq, q_rank, kv_rank,
+                                        rot_dim, eps);
+  return true;
+}
+
 constexpr int kKT = 64;       // keys per tile (one per lane)
 constexpr int kDC = 64;       // cache dims per staged chunk
 constexpr int kMaxCh = 16;    // kv_rank <= kMaxCh * 64
@@ -204,6 +292,11 @@ void launch_latent_prepare(void* cq, void* cache, const void* proj, long ld, con
                            const float* q_norm, const float* kv_norm, const float* inv_freq, int nfreq, int T,
                            int q_rank, int kv_rank, int rot_dim, float eps, bool f32, hipStream_t s) {
   if (T <= 0) return;
+  if (f32 ? prepare_vec((float*)cq, (float*)cache, (const float*)proj, ld, positions, slots, q_norm, kv_norm, inv_freq, nfreq, T,
+                        q_rank, kv_rank, rot_dim, eps, s)
+          : prepare_vec((unsigned short*)cq, (unsigned short*)cache, (const unsigned short*)proj, ld, positions, slots, q_norm,
+                        kv_norm, inv_freq, nfreq, T, q_rank, kv_rank, rot_dim, eps, s))
+    return;
   if (f32)
     latent_prepare_kernel<float><<<T, 256, 0, s>>>((float*)cq, (float*)cache, (const float*)proj, ld, positions, slots,
                                                    q_norm, kv_norm, inv_freq, nfreq, q_rank, kv_rank, rot_dim, eps);

@@ -486,3 +486,26 @@ def test_delta_rule_step(dtype):
     assert ((got_s.cpu() - want_s).abs() <= 64 * 2.0 ** -24 * want_s.abs().max()).all()   # a sum of 64 products
     tol, least = (2.0 ** -7, 2.0 ** -13) if dtype == torch.bfloat16 else (2.0 ** -17, 2.0 ** -17)
     assert ((got.cpu().float() - want.float()).abs() <= tol * want.float().abs() + least * want.float().abs().max()).all()
+
+
+# ------------------------------------------------------------------ latent rows
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("q_rank,kv_rank,rot,nfreq", [(8, 8, 8, 4), (512, 128, 64, 32), (1024, 512, 64, 32), (7680, 512, 72, 20), (1536, 8192, 128, 64),
+                                                      (20, 12, 8, 4)])
+def test_latent_prepare(q_rank, kv_rank, rot, nfreq, dtype):
+    """One item of 8 to two per thread, rotary dims that do not all rotate, rows without a slot; the last two: the general kernel."""
+    g = torch.Generator().manual_seed(q_rank)
+    T, eps = 4, 1e-5
+    proj = torch.randn(T, q_rank + kv_rank + rot + 8, generator=g).to(dtype)
+    cache, cq = torch.zeros(2, 16, kv_rank + rot, dtype=dtype), torch.empty(T, q_rank, dtype=dtype)
+    pos, slots = torch.tensor([0, 5, 300, 9000]), torch.tensor([31, -1, 0, 2])
+    inv = 1e4 ** (-torch.arange(nfreq).float() / nfreq)
+    qn, kn = torch.rand(q_rank, generator=g) + 0.5, torch.rand(kv_rank, generator=g) + 0.5
+    c, q = cache.cuda(), torch.empty(T, q_rank, dtype=dtype, device="cuda")
+    get_ops("cuda").latent_prepare(q, c, proj.cuda(), pos.cuda(), slots.cuda(), qn.cuda(), kn.cuda(), inv.cuda(), q_rank, kv_rank, rot, eps)
+    ref.latent_prepare(cq, cache, proj, pos, slots, qn, kn, inv, q_rank, kv_rank, rot, eps)
+    # an angle of up to 9000 rounds to 2^-11
+    tol = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -18
+    assert ((q.cpu().float() - cq.float()).abs() <= tol * cq.float().abs() + 2.0 ** -20).all()
+    assert ((c.cpu().float() - cache.float()).abs() <= tol * cache.float().abs() + 2.0 ** -10 * 4.5).all()
