@@ -7,6 +7,9 @@
 // 16 columns per workgroup give 128 workgroups at 2048 columns. A compute unit takes in about 34 KB per us this way, so
 // the rows' own bytes (16 columns of weights serve M rows) bound the larger M: 2048 x 2048, cold weights: 1 row 4.7 us,
 // 16 rows 6.2, 32 rows 8.0, 48 rows 10.2 (the vendor's GEMM: 11.0 - 11.2); 32000 x 2048, 1 row: 26 us = 5.0 TB/s (34).
+// 32-bit operands (F32) are the same rows of twice as many 16-bit halves: a step is 64 bytes of a row, 16 numbers, and four
+// products of 4 k each; the four numbers of a lane are k 4 g + e on both sides, so nothing else differs. 3 rows, cold
+// weights, 3072 x 1024: 5.9 us (the vendor's GEMM: 11.3); 32000 x 1024: 29 us = 4.5 TB/s (34).
 #pragma once
 #include "seq_common.h"
 
@@ -32,9 +35,9 @@ HS_DEVICE void swap_steps(u16x8& s0, u16x8& s1, bool low) {
 }
 
 // acc[nt][st] += the wave's part of W[16 columns of tile nt] . x[16 rows of tile st]; lane (c, g) = (lane % 16, lane / 16)
-// ends with columns 4 g .. + 3 of row c. wr / xr: two row addresses per tile (c % 8 and c % 8 + 8), advanced by
+// ends with columns 4 g .. + 3 of row c. K in 16-bit halves. wr / xr: two row addresses per tile (c % 8 and c % 8 + 8), advanced by
 // 8 g8, g8 = g + 4 (c / 8); low = c < 8. K % 8 == 0, KU even.
-template <int ST, int NT, int KU>
+template <int ST, int NT, int KU, bool F32 = false>
 HS_DEVICE void skinny_accumulate(f32x4 (&acc)[NT][ST], const unsigned short* const (&wr)[NT][2],
                                  const unsigned short* const (&xr)[ST][2], const bool (&live)[ST][2], int K, int g8,
                                  bool low, int wave) {
@@ -62,9 +65,16 @@ HS_DEVICE void skinny_accumulate(f32x4 (&acc)[NT][ST], const unsigned short* con
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int st = 0; st < ST; ++st)
-          acc[nt][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[u][nt]),
-                                                                __builtin_bit_cast(bf16x8, b[u][st]), acc[nt][st], 0, 0, 0);
+        for (int st = 0; st < ST; ++st) {
+          if constexpr (F32) {
+            const f32x4 fa = __builtin_bit_cast(f32x4, a[u][nt]), fb = __builtin_bit_cast(f32x4, b[u][st]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[nt][st] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], acc[nt][st], 0, 0, 0);
+          } else {
+            acc[nt][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[u][nt]),
+                                                                  __builtin_bit_cast(bf16x8, b[u][st]), acc[nt][st], 0, 0, 0);
+          }
+        }
   }
 }
 

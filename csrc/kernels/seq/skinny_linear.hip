@@ -1,8 +1,11 @@
-// out[b, m, :] = act(x[b, m, :] . W[b]^T + bias) for up to 64 rows m (decode steps and short prompts): bf16 operands,
-// 32-bit accumulation, a bf16 or 32-bit result, row and batch strides of their own for x and out.
+// out[b, m, :] = act(x[b, m, :] . W[b]^T + bias) for up to 64 rows m (decode steps and short prompts): bf16 or 32-bit
+// operands, 32-bit accumulation, a result of the operands' type or in 32 bits, row and batch strides of their own for x and out.
 // act: 0 tanh, 1 xIELU, 2 squared ReLU, 3 SiLU gate, 4 clamped gate (3, 4: W = [gate rows; up rows], half as many
 // columns in out), 5 soft cap, -1 none; they see the unrounded product.
 #include "skinny.h"
+
+#include <type_traits>
+
 #include "hipserve/seq_kernels.h"
 
 namespace hipserve {
@@ -18,12 +21,14 @@ HS_DEVICE float skinny_act(float z, int act, float c0, float c1) {
 
 // ST: 16-row tiles; NT: 16-column tiles (GLU: the gate's and the up projection's of the same 16 output columns);
 // KU: k steps of 32 whose loads a wave has in flight.
-template <int ST, int NT, int KU, bool GLU, typename TO>
+// F32: 32-bit operands, x, w, their strides and K in 16-bit halves (skinny.h).
+template <int ST, int NT, int KU, bool GLU, typename TO, bool F32>
 __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
     TO* __restrict__ out, long out_ld, long out_bs, const unsigned short* __restrict__ x, long x_ld, long x_bs,
-    const unsigned short* __restrict__ w, const unsigned short* __restrict__ bias, int M, int N, int K, int act,
-    float c0, float c1) {
+    const unsigned short* __restrict__ w, const void* __restrict__ bias_, int M, int N, int K, int act, float c0, float c1) {
   static_assert(!GLU || NT == 2, "a gate tile and an up tile");
+  using TB = std::conditional_t<F32, float, unsigned short>;
+  const TB* bias = static_cast<const TB*>(bias_);
   __shared__ __attribute__((aligned(16))) float red[kSkWaves * 16 * ST * kSkLd];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
   const int No = GLU ? N / 2 : N;
@@ -52,7 +57,7 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  skinny_accumulate<ST, NT, KU>(acc, wr, xr, live, K, g8, low, wave);
+  skinny_accumulate<ST, NT, KU, F32>(acc, wr, xr, live, K, g8, low, wave);
   float v[NT][(ST + 1) / 2];
   skinny_reduce<ST, NT>(v, acc, red);
   out += (long)blockIdx.y * out_bs;
@@ -63,15 +68,15 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
     if constexpr (GLU) {
       const int n = n0 + (e & 15);
       if (n >= No) continue;
-      const float gv = v[0][i] + (bias != nullptr ? bf16_to_f32(bias[n]) : 0.f);
-      const float uv = v[1][i] + (bias != nullptr ? bf16_to_f32(bias[No + n]) : 0.f);
+      const float gv = v[0][i] + (bias != nullptr ? ldf<TB>(bias, n) : 0.f);
+      const float uv = v[1][i] + (bias != nullptr ? ldf<TB>(bias, No + n) : 0.f);
       stf<TO>(out, m * out_ld + n, act == 4 ? clamped_glu_f(gv, uv, c0) : gv * sigmoid_f(gv) * uv);
     } else {
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const int n = n0 + 16 * nt + (e & 15);
         if (n >= N) continue;
-        const float z = v[nt][i] + (bias != nullptr ? bf16_to_f32(bias[n]) : 0.f);
+        const float z = v[nt][i] + (bias != nullptr ? ldf<TB>(bias, n) : 0.f);
         stf<TO>(out, m * out_ld + n, skinny_act(z, act, c0, c1));
       }
     }
@@ -80,26 +85,30 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
 
 template <int ST, int NT, int KU, bool GLU>
 void launch_one(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs, const void* w,
-                const void* bias, int batch, int M, int N, int K, int act, float c0, float c1, hipStream_t s) {
+                const void* bias, bool f32, int batch, int M, int N, int K, int act, float c0, float c1, hipStream_t s) {
   const int cols = GLU ? N / 2 : N, per = GLU ? 16 : 16 * NT;
   const dim3 grid((cols + per - 1) / per, batch);
-  auto xi = (const unsigned short*)x, wi = (const unsigned short*)w, bi = (const unsigned short*)bias;
-  if (out_f32)
-    skinny_linear_kernel<ST, NT, KU, GLU, float><<<grid, kSkThreads, 0, s>>>((float*)out, out_ld, out_bs, xi, x_ld, x_bs,
-                                                                            wi, bi, M, N, K, act, c0, c1);
+  auto xi = (const unsigned short*)x, wi = (const unsigned short*)w;
+  if (f32)
+    skinny_linear_kernel<ST, NT, KU, GLU, float, true><<<grid, kSkThreads, 0, s>>>((float*)out, out_ld, out_bs, xi, x_ld, x_bs, wi,
+                                                                                  bias, M, N, K, act, c0, c1);
+  else if (out_f32)
+    skinny_linear_kernel<ST, NT, KU, GLU, float, false><<<grid, kSkThreads, 0, s>>>((float*)out, out_ld, out_bs, xi, x_ld, x_bs, wi,
+                                                                                   bias, M, N, K, act, c0, c1);
   else
-    skinny_linear_kernel<ST, NT, KU, GLU, unsigned short><<<grid, kSkThreads, 0, s>>>(
-        (unsigned short*)out, out_ld, out_bs, xi, x_ld, x_bs, wi, bi, M, N, K, act, c0, c1);
+    skinny_linear_kernel<ST, NT, KU, GLU, unsigned short, false><<<grid, kSkThreads, 0, s>>>(
+        (unsigned short*)out, out_ld, out_bs, xi, x_ld, x_bs, wi, bias, M, N, K, act, c0, c1);
 }
 
 }  // namespace
 
 void launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs,
-                          const void* w, const void* bias, int batch, int M, int N, int K, int act, float c0, float c1,
+                          const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, float c0, float c1,
                           hipStream_t s) {
   if (batch <= 0 || M <= 0 || N <= 0) return;
+  if (f32) { x_ld *= 2; x_bs *= 2; K *= 2; }   // in halves
 #define HS_SK(ST, NT, KU, GLU) \
-  launch_one<ST, NT, KU, GLU>(out, out_f32, out_ld, out_bs, x, x_ld, x_bs, w, bias, batch, M, N, K, act, c0, c1, s)
+  launch_one<ST, NT, KU, GLU>(out, out_f32, out_ld, out_bs, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, c0, c1, s)
   // the loads in flight per wave cover K in one go where the registers allow it: KU steps of 32 k on 8 waves
   if (act == 3 || act == 4) {
     if (M <= 16) HS_SK(1, 2, 4, true);

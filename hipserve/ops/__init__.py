@@ -422,7 +422,7 @@ class KernelOps:
     GLU_ACTS = ("silu_mul", "clamped_glu")
 
     @staticmethod
-    def skinny_pays(rows: int, cols: int, k: int, glu: bool = False) -> bool:
+    def skinny_pays(rows: int, cols: int, k: int, glu: bool = False, f32: bool = False) -> bool:
         """Whether ``skinny_linear`` is expected to be faster than the vendor's GEMM for ``rows`` x ``cols`` results (``cols``
         over all batches). Both sides in us, fitted to cold weights of 1024 .. 32000 columns and k of 1024 .. 12288: ours is
         a latency plus the weights at 5 TB/s, or what a workgroup of 16 columns reads (weights and rows) at 34 KB per us and
@@ -430,23 +430,30 @@ class KernelOps:
         Examples, ours / vendor: 2048 x 2048 with 1, 16, 32, 48 rows 4.7 / 11.0, 6.2 / 11.1, 8.0 / 11.2, 10.2 / 11.2; 6144 x
         2048 with 1, 16, 32, 48 rows 7.7 / 12.6, 10.3 / 12.3, 13.7 / 12.3, 17.8 / 12.9; 2048 x 6144 with 1, 16 rows 9.0 / 10.9,
         13.2 / 11.1; 3072 x 1024 with 1, 48 rows 3.7 / 7.3, 6.7 / 11.1; 32000 x 2048 with 1, 16, 32 rows 26 / 34, 34 / 34, 46 / 34."""
+        if f32:
+            # the same in 32 bits (twice the bytes, whole workgroups per compute unit); the vendor's is hardly ever below 10.7
+            # (8.9 for 1024 x 1024) and streams at 4.5 TB/s. 1544 x 1024 with 1, 3, 16 rows 5.6 / 10.8, 5.7 / 10.9, 6.6 / 10.9;
+            # 1024 x 3072 with 1, 16 rows 10.3 / 10.7, 13.6 / 11.0; 32000 x 1024 with 3, 16 rows 29 / 34, 35 / 33.
+            weights, per_cu = 4.0 * cols * k, -(-cols // (32 if glu else 16) // 256) * 4.0 * k * ((32 if glu else 16) + rows)
+            return 4.2 + max(weights / 5.0e6, per_cu / 34e3) < max(8.9 if max(cols, k) <= 1024 else 10.7, 3.2 + weights / 4.5e6)
         weights = 2.0 * cols * k
         per_cu = max(1.0, cols / (32 if glu else 16) / 256) * 2.0 * k * ((32 if glu else 16) + rows)
         return 3.2 + max(weights / 5.0e6, per_cu / 34e3) < max(7.5 if k <= 1024 else 10.5, 3.2 + weights / 4.2e6)
 
     def _skinny_ok(self, x, w) -> bool:
         """The shapes, types and alignment that ``skinny_linear`` takes."""
-        return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.dim() == w.dim() and 0 < x.shape[-2] <= self.SKINNY_ROWS
-                and x.shape[-1] % 8 == 0 and x.stride(-1) == 1 and x.stride(-2) % 8 == 0 and x.stride(0) % 8 == 0
+        per = 16 // x.element_size()
+        return (x.dtype in (torch.bfloat16, torch.float32) and w.dtype == x.dtype and x.dim() == w.dim() and 0 < x.shape[-2] <= self.SKINNY_ROWS
+                and x.shape[-1] % per == 0 and x.stride(-1) == 1 and x.stride(-2) % per == 0 and x.stride(0) % per == 0
                 and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
     def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0):
-        """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands. A few bf16 rows run the
+        """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands. A few rows run the
         weight-streaming kernel with the activation in its epilogue, anything else the vendor's GEMM and a second launch."""
         if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or bias.dtype == x.dtype):
             glu = act in self.GLU_ACTS
             T, N, K = x.shape[0], w.shape[0], w.shape[1]
-            if self.skinny_pays(T, N, K, glu):
+            if self.skinny_pays(T, N, K, glu, x.dtype == torch.float32):
                 out = torch.empty(T, N // 2 if glu else N, device=x.device, dtype=torch.float32 if out_f32 else x.dtype)
                 self._moe_lib.skinny_linear(out, x, w, bias, -1 if act is None else self.ACTIVATIONS[act], c0, c1)
                 return out
@@ -462,7 +469,7 @@ class KernelOps:
     def linear_heads(self, out, x, w) -> bool:
         """out[h] = x[h] . w[h]^T for a few bf16 rows (x [heads, T, K], w [heads, N, K], out [heads, T, N], strided rows);
         False, and nothing done, where the vendor's batched GEMM is the one to run."""
-        if not (x.dim() == 3 and self._skinny_ok(x, w) and self.skinny_pays(x.shape[1], w.shape[0] * w.shape[1], w.shape[2])):
+        if not (x.dim() == 3 and x.dtype == torch.bfloat16 and self._skinny_ok(x, w) and self.skinny_pays(x.shape[1], w.shape[0] * w.shape[1], w.shape[2])):
             return False
         self._moe_lib.skinny_linear(out, x, w, None, -1, 0.0, 0.0)
         return True

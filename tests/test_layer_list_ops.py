@@ -133,6 +133,23 @@ def test_skinny_linear(M, N, K):
 
 
 @gpu
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (3, 40, 36), (16, 16, 256), (17, 96, 260), (33, 33, 1024), (64, 48, 3076)])
+def test_skinny_linear_f32(M, N, K):
+    """32-bit operands: k that fills a step of 16, a wave's steps and all waves partly; bias, row strides, an activation."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w, bias = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g), torch.randn(N, generator=g)
+    wide = torch.zeros(M, K + 12, device="cuda")
+    wide[:, 4:4 + K] = x.cuda()
+    out = torch.full((M, N + 5), 7.0, device="cuda")
+    get_ops("cuda")._moe_lib.skinny_linear(out[:, :N], wide[:, 4:4 + K], w.cuda(), bias.cuda(), 2, 0.0, 0.0)
+    z = x.double() @ w.double().T + bias.double()
+    # every one of K sums and products rounds to 2^-24 of at most the sum of magnitudes; the square doubles it
+    err = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + bias.double().abs())
+    assert ((out[:, :N].double().cpu() - z.clamp_min(0) ** 2).abs() <= 2 * z.abs() * err + err ** 2 + 2.0 ** -22 * z ** 2 + 1e-9).all()
+    assert (out[:, N:] == 7.0).all()
+
+
+@gpu
 @pytest.mark.parametrize("M", [1, 16, 31, 50])
 @pytest.mark.parametrize("act,c0,c1", [("tanh", 0, 0), ("xielu", 0.8, 0.7), ("relu2", 0, 0), ("silu_mul", 0, 0), ("clamped_glu", 1.0, 0),
                                        ("softcap", 2.0, 0)])
