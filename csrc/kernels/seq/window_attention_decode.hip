@@ -277,10 +277,10 @@ void launch(T* out, long out_ld, const T* proj, long proj_ld, const T* cache, in
             int gate_off, float scale, int window, bool sink, float out_scale, int nparts, int part_keys, float* ws_acc,
             float* ws_ml, int keep, float softcap, const float* sink_w, bool channel_gate, int chunk, hipStream_t s) {
   const int group = heads / kv_heads, hc = std::min(group, 16), hchunks = (group + hc - 1) / hc;
-  // a wave per tile of the run, as many as their accumulators fit 64 KB of LDS
-  const int kt = sizeof(T) == 4 ? 16 : 32;
-  const int nw = std::max(1, std::min({8, (part_keys + kt - 1) / kt, (1 << 14) / (hc * D)}));
-  const size_t smem = ((size_t)nw * hc * D + nw * 32) * sizeof(float);
+  // a wave per tile of the run, as many as their accumulators and sums fit 64 KB of LDS
+  const int kt = sizeof(T) == 4 ? 16 : 32, wave_floats = hc * D + 32;
+  const int nw = std::max(1, std::min({8, (part_keys + kt - 1) / kt, (1 << 14) / wave_floats}));
+  const size_t smem = (size_t)nw * wave_floats * sizeof(float);
   window_decode_kernel<T, D><<<dim3(rows, kv_heads * hchunks, nparts), 64 * nw, smem, s>>>(
       out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, hc, hchunks, heads,
       kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk);

@@ -348,7 +348,7 @@ def test_attn_prepare(heads, kv, maps, dim, vdim, nfreq, mode, v_norm, own, dtyp
 @pytest.mark.parametrize("heads,kv,dim,ctxs,opts", [
     (1, 1, 64, [1], {}), (4, 1, 128, [1, 31, 32, 33, 700], {"window": 0}), (8, 2, 128, [16, 17, 300, 257], {"window": 256, "sink": True, "gate": True}),
     (40, 2, 64, [5, 129, 400], {"window": 100, "keep_first": 7, "softcap": 3.0, "channel_gate": True}),
-    (32, 2, 128, [64, 65, 1500], {"chunk": 64, "sink_w": True}), (16, 1, 256, [3, 290], {"window": 0})])
+    (32, 2, 128, [64, 65, 1500], {"chunk": 64, "sink_w": True}), (16, 1, 256, [3, 290], {"window": 0}), (16, 1, 128, [300], {"window": 0})])
 def test_window_attention_decode(heads, kv, dim, ctxs, opts, dtype):
     """One key, runs that end inside a tile, several runs, more than 16 heads per key / value head, and every mask and gate."""
     from types import SimpleNamespace
