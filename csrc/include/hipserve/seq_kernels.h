@@ -179,6 +179,13 @@ void launch_window_attention_decode(void* out, long out_ld, const void* proj, lo
                                     bool sink, float out_scale, int nparts, int part_keys, float* ws_acc, float* ws_ml, int keep,
                                     float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, hipStream_t s);
 
+// fp32 prompt portions of the sequences seq0 .. seq1 - 1 (the sizes of window_attention_decode_ok).
+void launch_window_attention_prompts_f32(float* out, long out_ld, const float* proj, long proj_ld, const float* cache, int block_size,
+                                         const int* seq_cu, const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int seq1,
+                                         int rows_bound, int heads, int kv_heads, int dim, int gate_off, float scale, int window,
+                                         bool sink, float out_scale, int keep, float softcap, const float* sink_w, bool channel_gate,
+                                         int chunk, hipStream_t s);
+
 // Delta-rule recurrences over state slots (delta_scan.hip). Gated rule: proj rows = [q | k | v | ...] with beta's
 // columns from off_b on and the decay's / the gate's pre-activations from off_a / off_g on, or from `decay` (fp32
 // [T, heads * dim]: a decay per key channel) and `gate` ([T, heads * vdim], activation type); dt_bias has as many

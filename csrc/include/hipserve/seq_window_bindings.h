@@ -176,6 +176,34 @@ inline void window_attention_decode(at::Tensor& out, const at::Tensor& proj, con
                                            (const float*)opt_ptr(sink_w), channel_gate, chunk, f32, cur_stream());
 }
 
+inline void window_attention_prompts_f32(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
+                           const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t seq0, int64_t seq1, int64_t rows_bound,
+                           int64_t heads, int64_t kv_heads, int64_t dim, int64_t gate_off, double scale, int64_t window, bool sink,
+                           double out_scale, int64_t keep, double softcap, const c10::optional<at::Tensor>& sink_w,
+                           bool channel_gate, int64_t chunk) {
+  TORCH_CHECK(chunk >= 0 && (chunk == 0 || (window == 0 && keep == 0)), "window attention: chunks or a window");
+  CHECK_F32(cache); CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_bt);
+  TORCH_CHECK(proj.is_cuda() && proj.scalar_type() == at::kFloat && out.scalar_type() == at::kFloat, "window_attention_prompts_f32: fp32");
+  TORCH_CHECK(heads >= 1 && kv_heads >= 1 && heads % kv_heads == 0 && cache.dim() == 3 && cache.size(2) == kv_heads * 2 * dim);
+  const long T = proj.size(0), nseq = seq_ctx.numel();
+  TORCH_CHECK(rows2d(proj) && proj.size(1) >= heads * dim && (gate_off < 0 || proj.size(1) >= gate_off + heads * (channel_gate ? dim : 1)) &&
+              (!channel_gate || gate_off >= 0));
+  TORCH_CHECK(rows2d(out) && out.size(0) == T && out.size(1) == heads * dim);
+  TORCH_CHECK(window_attention_decode_ok(proj, cache, dim, dim), "window_attention_prompts_f32: head size, block size or alignment");
+  TORCH_CHECK(seq_cu.numel() == nseq + 1 && seq_bt.dim() == 2 && seq_bt.size(0) >= nseq);
+  TORCH_CHECK(0 <= seq0 && seq0 <= seq1 && seq1 <= nseq && rows_bound <= T && window >= 0 && keep >= 0 && softcap >= 0.0);
+  if (sink_w.has_value()) {
+    CHECK_F32(*sink_w);
+    TORCH_CHECK(sink && sink_w->numel() == heads, "window_attention_prompts_f32: one sink logit per head");
+  }
+  c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
+  hipserve::launch_window_attention_prompts_f32(
+      out.data_ptr<float>(), out.stride(0), proj.data_ptr<float>(), proj.stride(0), cache.data_ptr<float>(), cache.size(1),
+      seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_bt.data_ptr<int>(), seq_bt.size(1), seq0, seq1, rows_bound, heads, kv_heads,
+      dim, gate_off, (float)scale, window, sink, (float)out_scale, keep, (float)softcap, (const float*)opt_ptr(sink_w), channel_gate,
+      chunk, cur_stream());
+}
+
 inline void activation(at::Tensor& out, const at::Tensor& x, int64_t kind, double c0, double c1) {
   CHECK_DEV(x);
   const bool f32 = is_f32(x, "activation");
@@ -273,6 +301,9 @@ inline void def_window_ops(torch::Library& m) {
         "int seq0, int row_base, int heads, int kv_heads, int dim, int gate_off, float scale, int window, bool sink, "
         "float out_scale, int nparts, int part_keys, Tensor(b!)? ws_acc, Tensor(c!)? ws_ml, int keep, float softcap, "
         "Tensor? sink_w, bool channel_gate, int chunk) -> ()");
+  m.def("window_attention_prompts_f32(Tensor(a!) out, Tensor proj, Tensor cache, Tensor seq_cu, Tensor seq_ctx, Tensor seq_bt, "
+        "int seq0, int seq1, int rows_bound, int heads, int kv_heads, int dim, int gate_off, float scale, int window, bool sink, "
+        "float out_scale, int keep, float softcap, Tensor? sink_w, bool channel_gate, int chunk) -> ()");
   m.def("activation(Tensor(a!) out, Tensor x, int kind, float c0, float c1) -> ()");
   m.def("route_topk(Tensor(a!) ids, Tensor(b!) wts, Tensor logits, Tensor? correction, int top, float scale, int E, "
         "int groups, int keep, bool renorm, bool sigmoid=False, bool top2=False) -> ()");
@@ -288,6 +319,7 @@ inline void impl_window_ops(torch::Library& m) {
   m.impl("window_attention_mfma", &window_attention_mfma);
   m.impl("window_attention_decode_ok", &window_attention_decode_ok);
   m.impl("window_attention_decode", &window_attention_decode);
+  m.impl("window_attention_prompts_f32", &window_attention_prompts_f32);
   m.impl("activation", &activation);
   m.impl("route_topk", &route_topk);
   m.impl("route_align", &route_align);

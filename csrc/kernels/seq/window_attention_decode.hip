@@ -9,6 +9,8 @@
 //   each 16), and the instruction's rows for the dims that 16 consecutive bytes of a value row hold, every E-th of a block
 //   of 16 E: a lane loads whole 16-byte parts of its keys' rows, and in bf16 two byte permutations per pair of keys and pair
 //   of dims put the keys of one dim side by side.
+// fp32 prompts take the same kernel with several tokens in the 16 rows and a mask per score: the eight waves share no tile, but
+// the 32-bit products are slow enough that reading the keys once per 16 rows costs less than they do.
 // What bounds it: the chain table -> cache -> scores -> output of one tile, then (many sequences) memory. All loads of a
 // tile are issued at once and no wave waits for another's. A workgroup that stages every tile for four waves of which one has
 // rows (a group of 4 heads) waits for two barriers and a transposing store per 32 keys: one sequence of 100 keys, 8 heads
@@ -59,26 +61,35 @@ HS_DEVICE float over_rows(float x) {   // over the lanes c, c + 16, c + 32, c + 
 
 using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
 
-template <typename T, int D>
+// MULTI: prompt portions, tq tokens x hc heads in the 16 rows, tiles of tokens in blockIdx.x; one run.
+template <typename T, int D, bool MULTI>
 __global__ __launch_bounds__(512) void window_decode_kernel(
     T* __restrict__ out, long out_ld, const T* __restrict__ proj, long proj_ld, const T* __restrict__ cache, int block_shift,
     const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0,
-    int hc, int hchunks, int heads, int kv_heads, int gate_off, float scale, int window, bool sink, float out_scale,
+    int seq1, int tq, int hc, int hchunks, int heads, int kv_heads, int gate_off, float scale, int window, bool sink, float out_scale,
     int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml, int keep, float softcap,
     const float* __restrict__ sink_w, bool channel_gate, int chunk) {
   constexpr bool F32 = sizeof(T) == 4;
   constexpr int SUB = F32 ? 1 : 2, KT = 16 * SUB;          // 16-key tiles and keys of a wave's tile
   constexpr int QN = F32 ? D / 16 : D / 32;                // 16-byte parts of a row per lane
   constexpr int E = F32 || D == 64 ? 4 : 8, NB = D / (16 * E);   // dims of a value row per load; loads per row
-  extern __shared__ float lds[];                           // [waves][nh][D]; [waves][16][2]
+  extern __shared__ float lds[];                           // [waves][rows][D]; [waves][16][2]
   using S = Softmax<T>;
-  const int s = seq0 + blockIdx.x, r0 = seq_cu[s], ctx = seq_ctx[s];
-  if (seq_cu[s + 1] <= r0) return;
+  int s = seq0 + blockIdx.x, tok0 = 0;
+  if (MULTI && !find_row_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) return;
+  const int seq_r0 = seq_cu[s], n = seq_cu[s + 1] - seq_r0, ctx = seq_ctx[s];
+  if (n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
   const int group = heads / kv_heads, kvh = blockIdx.y / hchunks, h0 = (blockIdx.y % hchunks) * hc;
   const int nh = min(hc, group - h0), head0 = kvh * group + h0;
-  const int p = ctx - 1, lo_all = first_key(max(p, 0), window, chunk);
+  const int ntok = MULTI ? min(tq, n - tok0) : 1, p_first = MULTI ? ctx - n + tok0 : ctx - 1, p = p_first + ntok - 1;
+  const int lo_all = first_key(max(p_first, 0), window, chunk);
+  // this lane's row
+  const int rt = MULTI ? c / hc : 0, rh = MULTI ? c % hc : c;
+  const bool act = rt < ntok && rh < nh;
+  const int head = head0 + (act ? rh : 0), spos = p_first + rt, s_lo = first_key(max(spos, 0), window, chunk);
+  const long r0 = seq_r0 + tok0 + (act ? rt : 0);
   const int nk = (window > 0 && keep > 0) ? min(keep, lo_all) : 0;   // kept keys below the window
   const int total = nk + p - lo_all + 1;
   const int lo = blockIdx.z * part_keys, hi = gridDim.z > 1 ? min(total, lo + part_keys) - 1 : total - 1;
@@ -93,7 +104,7 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
 #pragma unroll
   for (int i = 0; i < QN; ++i) {
     q[i] = u32x4{0, 0, 0, 0};
-    if (c < nh) q[i] = reinterpret_cast<const u32x4*>(proj + (long)r0 * proj_ld + (long)(head0 + c) * D)[4 * i + g];
+    if (act) q[i] = reinterpret_cast<const u32x4*>(proj + r0 * proj_ld + (long)head * D)[4 * i + g];
   }
   f32x4 acc[NB][E];
 #pragma unroll
@@ -101,7 +112,7 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
 #pragma unroll
     for (int j = 0; j < E; ++j) acc[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const bool sunk = sink && blockIdx.z == 0 && wave == 0;
-  float m = sunk ? (sink_w != nullptr && c < nh ? sink_w[head0 + c] * S::kUnit : 0.f) : -INFINITY, l = sunk ? 1.f : 0.f;
+  float m = sunk ? (sink_w != nullptr ? sink_w[head] * S::kUnit : 0.f) : -INFINITY, l = sunk ? 1.f : 0.f;
   const float unit = scale * S::kUnit, cap = softcap * S::kUnit, icap = softcap > 0.f ? scale / softcap : 0.f;
 
   for (int u0 = lo + wave * KT; u0 <= hi; u0 += nw * KT) {
@@ -136,14 +147,19 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
       }
     }
     // lane (c, g): row c against keys 16 a + 4 g + i
-    const bool whole = u0 + KT - 1 <= hi;
+    const bool whole = u0 + KT - 1 <= hi;   // a decode row sees every key of the run
+    auto hidden = [&](int u) {
+      const int j = u < nk ? u : u - nk + lo_all;
+      return u > hi || (MULTI && (j > spos || (j < s_lo && j >= keep)));
+    };
+    const bool open = MULTI ? __all(whole && u0 >= nk && u0 + KT - 1 - nk + lo_all <= spos && u0 - nk + lo_all >= s_lo) : whole;
     float mx = -INFINITY;
 #pragma unroll
     for (int a = 0; a < SUB; ++a)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float x = softcap > 0.f ? cap * S::tanh(sc[a][i] * icap) : sc[a][i] * unit;
-        if (!whole && u0 + 16 * a + 4 * g + i > hi) x = -INFINITY;
+        if (!open && hidden(u0 + 16 * a + 4 * g + i)) x = -INFINITY;
         sc[a][i] = x;
         mx = fmaxf(mx, x);
       }
@@ -197,9 +213,10 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
     }
   }
   // lane (c, g): row c, dims 16 E b + E (4 g + i) + j
-  float* ml = lds + nw * nh * D;
-  if (c < nh) {
-    float* dst = lds + ((long)wave * nh + c) * D;
+  const int nr = MULTI ? 16 : nh;   // rows
+  float* ml = lds + nw * nr * D;
+  if (c < nr) {
+    float* dst = lds + ((long)wave * nr + c) * D;
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -211,8 +228,9 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
     if (g == 0) { ml[2 * (wave * 16 + c)] = m; ml[2 * (wave * 16 + c) + 1] = l; }
   }
   __syncthreads();
-  for (int it = tid; it < nh * (D / 4); it += blockDim.x) {
-    const int h = it / (D / 4), d = it % (D / 4) * 4;
+  for (int it = tid; it < nr * (D / 4); it += blockDim.x) {
+    const int h = it / (D / 4), d = it % (D / 4) * 4, ht = MULTI ? h / hc : 0, hh = MULTI ? h % hc : h;
+    if (MULTI && (ht >= ntok || hh >= nh)) continue;
     float M = -INFINITY, L = 0.f;
     for (int w = 0; w < nw; ++w) M = fmaxf(M, ml[2 * (w * 16 + h)]);
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
@@ -221,22 +239,23 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
       if (mw == -INFINITY) continue;   // no key
       const float f = S::exp(mw - M);
       L += ml[2 * (w * 16 + h) + 1] * f;
-      o += *reinterpret_cast<const f32x4*>(lds + ((long)w * nh + h) * D + d) * f;
+      o += *reinterpret_cast<const f32x4*>(lds + ((long)w * nr + h) * D + d) * f;
     }
-    const int head = head0 + h;
+    const int hd = head0 + hh;
+    const long row = seq_r0 + tok0 + ht;
     if (gridDim.z > 1) {
-      const long wrow = ((long)blockIdx.z * heads + head) * gridDim.x + blockIdx.x;
+      const long wrow = ((long)blockIdx.z * heads + hd) * gridDim.x + blockIdx.x;
       *reinterpret_cast<f32x4*>(ws_acc + wrow * D + d) = o;
       if (d == 0) { ws_ml[2 * wrow] = M; ws_ml[2 * wrow + 1] = L; }
       continue;
     }
     float f = out_scale;
-    if (gate_off >= 0 && !channel_gate) f *= sigmoid_f(ldf<T>(proj, (long)r0 * proj_ld + gate_off + head));
+    if (gate_off >= 0 && !channel_gate) f *= sigmoid_f(ldf<T>(proj, row * proj_ld + gate_off + hd));
     f = L == 0.f ? 0.f : f / L;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float cg = channel_gate ? sigmoid_f(ldf<T>(proj, (long)r0 * proj_ld + gate_off + (long)head * D + d + e)) : 1.f;
-      stf<T>(out, (long)r0 * out_ld + (long)head * D + d + e, o[e] * f * cg);
+      const float cg = channel_gate ? sigmoid_f(ldf<T>(proj, row * proj_ld + gate_off + (long)hd * D + d + e)) : 1.f;
+      stf<T>(out, row * out_ld + (long)hd * D + d + e, o[e] * f * cg);
     }
   }
 }
@@ -281,15 +300,39 @@ void launch(T* out, long out_ld, const T* proj, long proj_ld, const T* cache, in
   const int kt = sizeof(T) == 4 ? 16 : 32, wave_floats = hc * D + 32;
   const int nw = std::max(1, std::min({8, (part_keys + kt - 1) / kt, (1 << 14) / wave_floats}));
   const size_t smem = (size_t)nw * wave_floats * sizeof(float);
-  window_decode_kernel<T, D><<<dim3(rows, kv_heads * hchunks, nparts), 64 * nw, smem, s>>>(
-      out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, hc, hchunks, heads,
-      kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk);
+  window_decode_kernel<T, D, false><<<dim3(rows, kv_heads * hchunks, nparts), 64 * nw, smem, s>>>(
+      out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq0 + rows, 1, hc,
+      hchunks, heads, kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk);
   if (nparts > 1)
     window_decode_reduce_kernel<T><<<dim3(rows, heads), 128, 0, s>>>(out, out_ld, ws_acc, ws_ml, proj, proj_ld, gate_off, nparts,
                                                                     heads, rows, row_base, D, out_scale, channel_gate);
 }
 
+template <int D>
+void launch_prompts(float* out, long out_ld, const float* proj, long proj_ld, const float* cache, int block_size, const int* seq_cu,
+                    const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int seq1, int rows_bound, int heads, int kv_heads,
+                    int gate_off, float scale, int window, bool sink, float out_scale, int keep, float softcap, const float* sink_w,
+                    bool channel_gate, int chunk, hipStream_t s) {
+  const int group = heads / kv_heads, hc = std::min(group, 16), hchunks = (group + hc - 1) / hc, tq = 16 / hc;
+  const int wave_floats = 16 * D + 32, nw = std::min(8, (1 << 14) / wave_floats);
+  window_decode_kernel<float, D, true><<<dim3(rows_bound / tq + (seq1 - seq0), kv_heads * hchunks, 1), 64 * nw,
+                                         (size_t)nw * wave_floats * sizeof(float), s>>>(
+      out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, tq, hc, hchunks,
+      heads, kv_heads, gate_off, scale, window, sink, out_scale, 0, nullptr, nullptr, keep, softcap, sink_w, channel_gate, chunk);
+}
+
 }  // namespace
+
+void launch_window_attention_prompts_f32(float* out, long out_ld, const float* proj, long proj_ld, const float* cache, int block_size,
+                                         const int* seq_cu, const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int seq1,
+                                         int rows_bound, int heads, int kv_heads, int dim, int gate_off, float scale, int window,
+                                         bool sink, float out_scale, int keep, float softcap, const float* sink_w, bool channel_gate,
+                                         int chunk, hipStream_t s) {
+  if (seq1 <= seq0 || rows_bound <= 0) return;
+  auto go = dim == 64 ? launch_prompts<64> : launch_prompts<128>;
+  go(out, out_ld, proj, proj_ld, cache, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, rows_bound, heads, kv_heads, gate_off,
+     scale, window, sink, out_scale, keep, softcap, sink_w, channel_gate, chunk, s);
+}
 
 bool window_attention_decode_ok(int dim, int vdim, int block_size, bool f32) {
   return dim == vdim && (dim == 64 || dim == 128 || (dim == 256 && !f32)) && (block_size & (block_size - 1)) == 0;

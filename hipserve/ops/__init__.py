@@ -371,7 +371,14 @@ class KernelOps:
                 self._window_lib.window_attention_mfma(out, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt, npf, nseq, nd,
                                                 *args, nparts, part, ws_acc, ws_ml, Tp, *diff)
             return
-        for s0, s1, rows, tq in ((0, npf, Tp, self.WINDOW_PREFILL_TQ), (npf, nseq, nd, 1)):
+        if npf and (proj.dtype == torch.float32 and sp.maps == 1 and self.WINDOW_MFMA
+                    and self._window_lib.window_attention_decode_ok(proj, cache, sp.dim, sp.vdim)):
+            # fp32 prompts on the 32-bit matrix cores (3 prompts, 8 heads over 2 of 128: 104 -> 28 us)
+            self._window_lib.window_attention_prompts_f32(out, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt, 0, npf, Tp,
+                                                          sp.heads, sp.kv_heads, sp.dim, gate_off, sp.scale, sp.window, sp.sink,
+                                                          out_scale, sp.keep_first, sp.softcap, sink_w, sp.channel_gate, sp.chunk)
+            npf = 0
+        for s0, s1, rows, tq in ((0, npf, Tp, self.WINDOW_PREFILL_TQ), (nseq - nd, nseq, nd, 1)):
             if s1 > s0:
                 self._window_lib.window_attention(out, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt, s0, s1, rows, tq,
                                            sp.heads, sp.kv_heads, sp.dim, sp.vdim, gate_off, sp.scale, sp.window,

@@ -436,24 +436,26 @@ def test_delta_rule_chunks(lens):
 
 # ------------------------------------------------------------------ window attention of prompts
 @gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("heads,kv,dim,bs,lens,ctxs,opts", [
     (1, 1, 64, 16, [1, 33], [1, 40], {}), (8, 2, 128, 16, [31, 32, 65], [31, 100, 65], {"window": 40, "sink": True, "gate": True}),
     (5, 1, 64, 64, [130, 7], [300, 7], {"window": 0, "softcap": 3.0, "channel_gate": True}),
     (130, 1, 64, 16, [9], [50], {"window": 20, "sink_w": True}), (4, 4, 128, 128, [200, 3], [210, 203], {"chunk": 64}),
-    (16, 4, 128, 16, [700, 300], [700, 450], {"window": 256, "sink": True}), (2, 1, 128, 8, [40], [64], {"window": 16})])
-def test_window_attention_prompts(heads, kv, dim, bs, lens, ctxs, opts):
+    (16, 4, 128, 16, [700, 300], [700, 450], {"window": 256, "sink": True}), (2, 1, 128, 8, [40], [64], {"window": 16, "keep_first": 5})])
+def test_window_attention_prompts(heads, kv, dim, bs, lens, ctxs, opts, dtype):
     """Tokens, heads and keys that do not fill a tile, windows and chunks that start inside one, pages smaller and larger than a
-    tile, one and two row tiles per wave, more than 128 heads per key / value head, and small pages, which the other kernel takes."""
+    tile, one and two row tiles per wave, more than 128 heads per key / value head, and kept keys, which the other
+    kernel takes in bf16; fp32."""
     from types import SimpleNamespace
     g = torch.Generator().manual_seed(heads * dim + sum(lens))
     n, T, gate = len(lens), sum(lens), opts.get("gate", False) or opts.get("channel_gate", False)
     sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=opts.get("window", 0), scale=dim ** -0.5, sink=opts.get("sink", "sink_w" in opts),
-                         keep_first=0, softcap=opts.get("softcap", 0.0), channel_gate=opts.get("channel_gate", False), chunk=opts.get("chunk", 0), diff=0.0)
-    sp.reach = sp.window or sp.chunk
+                         keep_first=opts.get("keep_first", 0), softcap=opts.get("softcap", 0.0), channel_gate=opts.get("channel_gate", False), chunk=opts.get("chunk", 0), diff=0.0)
+    sp.reach = sp.window + sp.keep_first if sp.window else sp.chunk
     width = -(-max(ctxs) // bs)
     bt = torch.randperm(n * width, generator=g).int().view(n, width)
-    cache = torch.randn(n * width, bs, 2 * kv * dim, generator=g).bfloat16()
-    proj = torch.randn(T, 2 * heads * dim, generator=g).bfloat16()
+    cache = torch.randn(n * width, bs, 2 * kv * dim, generator=g).to(dtype)
+    proj = torch.randn(T, 2 * heads * dim, generator=g).to(dtype)
     sink_w = torch.randn(heads, generator=g) if opts.get("sink_w") else None
     cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
     want = torch.empty(T, heads, dim, dtype=torch.float64)
@@ -463,7 +465,7 @@ def test_window_attention_prompts(heads, kv, dim, bs, lens, ctxs, opts):
         kvr = rows[bt[s].long()[j // bs] * bs + j % bs]
         p = torch.arange(ctxs[s] - lens[s], ctxs[s])[:, None]
         lo = p - p % sp.chunk if sp.chunk else p - sp.window + 1 if sp.window else torch.zeros_like(p)
-        seen = (j <= p) & (j >= lo)
+        seen = (j <= p) & ((j >= lo) | (j < sp.keep_first))
         for h in range(heads):
             q = proj[cu[s]:cu[s + 1], h * dim:(h + 1) * dim].double()
             x = q @ kvr[:, h // (heads // kv)].t() * sp.scale
@@ -477,10 +479,11 @@ def test_window_attention_prompts(heads, kv, dim, bs, lens, ctxs, opts):
         gates = torch.sigmoid(proj[:, heads * dim:heads * dim + (heads * dim if sp.channel_gate else heads)].double())
         want *= gates if sp.channel_gate else gates.repeat_interleave(dim, 1)
     meta = SimpleNamespace(seq_ctx=torch.tensor(ctxs).int().cuda(), seq_cu=cu.cuda(), seq_bt=bt.cuda(), num_decode=0, num_prefill_tokens=T, max_ctx=max(ctxs))
-    out = torch.empty(T, heads * dim, dtype=torch.bfloat16, device="cuda")
+    out = torch.empty(T, heads * dim, dtype=dtype, device="cuda")
     get_ops("cuda").window_attention(out, proj.cuda(), cache.cuda(), meta, sp, heads * dim if gate else -1, 1.0, 0.0, 0.0, None if sink_w is None else sink_w.cuda())
-    # weights and outputs rounded to 2^-9, the largest value about 4.5
-    assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * rows.abs().max() * 0.5).all()
+    # bf16: weights and outputs rounded to 2^-9, the largest value about 4.5; fp32: sums of up to 700 products
+    tol, least = (2.0 ** -7, 2.0 ** -8) if dtype == torch.bfloat16 else (2.0 ** -18, 2.0 ** -19)
+    assert ((out.double().cpu() - want).abs() <= tol * want.abs() + least * rows.abs().max() * 0.5).all()
 
 
 @gpu
