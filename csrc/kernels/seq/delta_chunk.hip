@@ -9,8 +9,8 @@
 // formed as products of the decays between the two tokens (never as a quotient), so strong decays only underflow.
 //
 // delta_chunk_prepare: everything that does not need the state, one workgroup per (head, chunk): A, P, the inverse
-// M = (1 + diag(beta) A)^-1 diag(beta) by forward substitution, and W = M (G k), U0 = M v, G q, G_15 / G k, G_15.
-// delta_chunk_scan: one workgroup per (sequence, head, 16 value channels) walks the chunks: U = U0 - W S,
+// M = (1 + diag(beta) A)^-1 diag(beta) by forward substitution, and W = -M (G k), U0 = M v, G q, G_15 / G k, G_15.
+// delta_chunk_scan: one workgroup per (sequence, head, 32 value channels) walks the chunks: U = U0 + W S,
 // o = (G q) S + P U, S = G_15 S + (G_15 / G k)^T U on mfma_f32_16x16x4f32. The state stays in registers in the
 // accumulators' layout, which is also the second operand's: lane (n, g) of a 16-row tile holds rows 4 g + r of column n,
 // and k step r of a product takes rows {4 g + r}.
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
       sMt[tid][i] = x[i];
     }
   }
-  out.P[tid] = sP[row][seg];
+  out.P[64 * (seg & 3) + 16 * (seg >> 2) + row] = sP[row][seg];   // by k step and lane of the scan
   __syncthreads();
   // W = M (G k)
   float w[NJ][VD];
@@ -192,7 +192,11 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
     }
   }
 #pragma unroll
-  for (int j = 0; j < NJ; ++j) Row<float, VD>::st(out.W + row * DP + 16 * VD * j + VD * seg, w[j]);
+  for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+    for (int e = 0; e < VD; ++e) w[j][e] = -w[j][e];
+    Row<float, VD>::st(out.W + row * DP + 16 * VD * j + VD * seg, w[j]);
+  }
   // G_15 / G k, transposed
   for (int i = tid; i < DP * (kC / 4); i += 256) {
     const int c = i >> 2, q = 4 * (i & 3);
@@ -215,120 +219,153 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
   }
 }
 
-// TPW 16-row state tiles per wave, NW waves.
-template <int TPW, int NW>
+// NW waves with TPW 16-row state tiles each, NC tiles of 16 value channels per workgroup. What a CU can take in (about 34 KB per us)
+// bounds it, so the operands of the state (W, G q, G_15 / G k) serve two tiles of channels, U0 is loaded by one wave per tile (as
+// the start of its sum) and every wave does its share of the k steps of P U; the outputs are summed with the next
+// chunk's exchange. 8192 rows (4 prompts) x 16 heads of 128 x 128: 216 us, of
+// which the matrix instructions take half; one tile per workgroup with U0 and P in every wave,
+// two chunks ahead and an exit between them: 267 us.
+constexpr int kAhead = 4;   // chunks in flight
+template <int TPW, int NW, int NC>
 __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
     float* __restrict__ o, float* __restrict__ S, float* __restrict__ base, const int* __restrict__ seq_cu,
     const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads, int dim, int vdim, int VP, long pad) {
-  constexpr int DP = 16 * TPW * NW;
-  static_assert(NW == 1 || NW == 2 || NW == 4, "the waves share the four rows of a lane");
-  __shared__ __attribute__((aligned(16))) f32x4 part[2][2][NW][64];   // [chunk parity][W S | (G q) S][wave][lane]
-  const int s = blockIdx.z, h = blockIdx.x, v0 = 16 * blockIdx.y;
+  constexpr int DP = 16 * TPW * NW, KPW = 4 / NW, RPW = 4 * NC / NW;   // k steps of P U and rows of the read-out per wave
+  static_assert((NW == 1 && NC == 1) || (NC == 2 && (NW == 2 || NW == 4)), "a wave per tile for U0, whole rows per wave");
+  __shared__ __attribute__((aligned(16))) f32x4 sums[2][2][NC][NW][64];   // [chunk parity][U | the last chunk's o][tile][wave][lane]
+  const int s = blockIdx.z, h = blockIdx.x, v0 = 16 * NC * blockIdx.y;
   const int r0 = seq_cu[s], n = seq_cu[s + 1] - r0;
   if (n <= 0) return;
   int first = 0;   // the sequence's first chunk in the step
   for (int i = 0; i < s; ++i) first += (seq_cu[i + 1] - seq_cu[i] + kC - 1) / kC;
   const int nc = (n + kC - 1) / kC;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
-  const int col = v0 + c, nv = heads * vdim;
+  const bool odd = threadIdx.x & 64, high = threadIdx.x & 128;   // the wave's bits as lane masks: selects, not branches
+  const int nv = heads * vdim, mine = wave % NC, row0 = (wave / NC) * RPW;
   const bool carried = seq_ctx[s] - n > 0;
-  float* Sp = S + ((long)seq_state[s] * heads + h) * dim * vdim + col;
-  f32x4 st[TPW];
+  float* Sp = S + ((long)seq_state[s] * heads + h) * dim * vdim + v0 + c;
+  f32x4 st[NC][TPW];
 #pragma unroll
-  for (int b = 0; b < TPW; ++b)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int k = 16 * (wave * TPW + b) + 4 * g + r;
-      st[b][r] = (carried && k < dim && col < vdim) ? Sp[(long)k * vdim] : 0.f;
-    }
-  // Two chunks' operands, each loaded two chunks ahead as soon as its registers are free. Loads and stores of the loop are
-  // unconditional (past the end the last chunk is loaded again, rows and columns that do not exist are stored behind
-  // o), so that the wait for an operand never has to cover the younger loads behind it.
-  struct Ops {
-    f32x4 W[TPW], Q[TPW], K[TPW], E[TPW], U, P;
-  } even, odd;
-  auto fetch_products = [&](Ops& x, int ci) {   // what the products with the state take
-    const ChunkBuf b = chunk_buf(base, (long)(first + min(ci, nc - 1)) * heads + h, DP, VP);
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const int at = c * DP + 16 * (wave * TPW + i) + 4 * g;
-      x.W[i] = *reinterpret_cast<const f32x4*>(b.W + at);
-      x.Q[i] = *reinterpret_cast<const f32x4*>(b.GQ + at);
-    }
-  };
-  auto fetch_update = [&](Ops& x, int ci) {     // what the state's update and the read-out take
-    const ChunkBuf b = chunk_buf(base, (long)(first + min(ci, nc - 1)) * heads + h, DP, VP);
-#pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const int k0 = 16 * (wave * TPW + i);
-      x.K[i] = *reinterpret_cast<const f32x4*>(b.KT + (k0 + c) * kC + 4 * g);
-      x.E[i] = *reinterpret_cast<const f32x4*>(b.GE + k0 + 4 * g);
-    }
-    x.U = *reinterpret_cast<const f32x4*>(b.UT + (long)col * kC + 4 * g);   // col < VP
-    x.P = *reinterpret_cast<const f32x4*>(b.P + c * kC + 4 * g);
-  };
-  auto step = [&](Ops& x, int ci) {
-    f32x4 ws = {0.f, 0.f, 0.f, 0.f}, qs = ws;
+  for (int t = 0; t < NC; ++t)
 #pragma unroll
     for (int b = 0; b < TPW; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        ws = __builtin_amdgcn_mfma_f32_16x16x4f32(x.W[b][r], st[b][r], ws, 0, 0, 0);
-        qs = __builtin_amdgcn_mfma_f32_16x16x4f32(x.Q[b][r], st[b][r], qs, 0, 0, 0);
+        const int k = 16 * (wave * TPW + b) + 4 * g + r;
+        st[t][b][r] = (carried && k < dim && v0 + 16 * t + c < vdim) ? Sp[(long)k * vdim + 16 * t] : 0.f;
       }
-    fetch_products(x, ci + 2);
-    f32x4 u = x.U;
+  // Operands, each loaded kAhead chunks ahead as soon as its registers are free. Loads and stores of the loop are
+  // unconditional (past the end the last chunk is loaded again, rows and columns that do not exist are stored behind
+  // o), so that the wait for an operand never has to cover the younger loads behind it.
+  struct Ops {
+    f32x4 W[TPW], Q[TPW], K[TPW], E[TPW], U;
+    float p[KPW];
+  } ops[kAhead];
+  const unsigned ucol = min(v0 + 16 * mine + c, VP - 1);
+  auto fetch = [&](Ops& x, int ci) {
+    const ChunkBuf b = chunk_buf(base, (long)(first + min(ci, nc - 1)) * heads + h, DP, VP);
 #pragma unroll
-    for (int b = 0; b < TPW; ++b) st[b] *= x.E[b];
-    f32x4 (*pt)[NW][64] = part[ci & 1];
-    if constexpr (NW > 1) {
-      pt[0][wave][lane] = ws;
-      pt[1][wave][lane] = qs;
-      __syncthreads();   // the other parity's rows are read before a wave comes here again
+    for (int i = 0; i < TPW; ++i) {
+      const unsigned k0 = 16 * (wave * TPW + i), at = c * DP + k0 + 4 * g;
+      x.W[i] = *reinterpret_cast<const f32x4*>(b.W + at);
+      x.Q[i] = *reinterpret_cast<const f32x4*>(b.GQ + at);
+      x.K[i] = *reinterpret_cast<const f32x4*>(b.KT + (k0 + c) * kC + 4 * g);
+      x.E[i] = *reinterpret_cast<const f32x4*>(b.GE + k0 + 4 * g);
+    }
+    x.U = *reinterpret_cast<const f32x4*>(b.UT + ucol * kC + 4 * g);
 #pragma unroll
-      for (int i = 0; i < NW; ++i) u -= pt[0][i][lane];
-    } else {
-      u -= ws;
+    for (int i = 0; i < KPW; ++i) x.p[i] = b.P[64 * (wave * KPW + i) + lane];
+  };
+  auto step_of = [&](const f32x4& v, int i) {   // the wave's i-th k step
+    if constexpr (NW == 1) return v[i];
+    else if constexpr (NW == 2) return odd ? v[2 + i] : v[i];
+    else return high ? (odd ? v[3] : v[2]) : odd ? v[1] : v[0];
+  };
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 os[NC] = {};
+  float* po = o + (long)(r0 + 4 * g + row0) * nv + h * vdim + v0 + 16 * mine + c;
+  float* nowhere = o + pad + lane;
+  const unsigned rows = v0 + 16 * mine + c < vdim ? n : 0;
+  auto read_out = [&](int ci, int buf) {   // the outputs of chunk ci from the sums in sums[buf]
+#pragma unroll
+    for (int e = 0; e < RPW; ++e) {
+      float y = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) y += reinterpret_cast<const float*>(&sums[buf][1][mine][w][lane])[row0 + e];
+      float* to = po + (long)(ci * kC + e) * nv;
+      *((unsigned)(ci * kC + 4 * g + row0 + e) < rows ? to : nowhere) = y;
+    }
+  };
+  auto step = [&](Ops& x, int ci) {
+    const int buf = ci & 1;
+    f32x4 us[NC], qs[NC], u[NC];
+#pragma unroll
+    for (int t = 0; t < NC; ++t) {
+      us[t] = NC == 1 || (!high && odd == t) ? x.U : zero;
+      qs[t] = zero;
+      sums[buf][1][t][wave][lane] = os[t];
+    }
+#pragma unroll
+    for (int b = 0; b < TPW; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < NC; ++t) {
+          us[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.W[b][r], st[t][b][r], us[t], 0, 0, 0);
+          qs[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.Q[b][r], st[t][b][r], qs[t], 0, 0, 0);
+        }
+#pragma unroll
+    for (int t = 0; t < NC; ++t) {
+      sums[buf][0][t][wave][lane] = us[t];
+#pragma unroll
+      for (int b = 0; b < TPW; ++b) st[t][b] *= x.E[b];
+    }
+    __syncthreads();   // the other parity's rows are read before a wave comes here again
+#pragma unroll
+    for (int t = 0; t < NC; ++t) {
+      u[t] = sums[buf][0][t][0][lane];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) u[t] += sums[buf][0][t][w][lane];
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int b = 0; b < TPW; ++b) st[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.K[b][r], u[r], st[b], 0, 0, 0);
-    f32x4 oo = {0.f, 0.f, 0.f, 0.f};
+      for (int b = 0; b < TPW; ++b)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) oo = __builtin_amdgcn_mfma_f32_16x16x4f32(x.P[r], u[r], oo, 0, 0, 0);
-    fetch_update(x, ci + 2);
+        for (int t = 0; t < NC; ++t) st[t][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.K[b][r], u[t][r], st[t][b], 0, 0, 0);
 #pragma unroll
-    for (int k = 0; k < 4 / NW; ++k) {   // wave w reads out the rows 4 g + w (+ NW ..)
-      const int r = wave + NW * k, i = ci * kC + 4 * g + r;
-      float y = r == 0 ? oo[0] : r == 1 ? oo[1] : r == 2 ? oo[2] : oo[3];
-      if constexpr (NW > 1) {
+    for (int t = 0; t < NC; ++t) {
+      os[t] = qs[t];
 #pragma unroll
-        for (int w = 0; w < NW; ++w) y += reinterpret_cast<const float*>(&pt[1][w][lane])[r];
-      } else {
-        y += r == 0 ? qs[0] : r == 1 ? qs[1] : r == 2 ? qs[2] : qs[3];
-      }
-      const long at = i < n && col < vdim ? (long)(r0 + i) * nv + h * vdim + col : pad + lane;
-      o[at] = y;
+      for (int i = 0; i < KPW; ++i) os[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[i], step_of(u[t], i), os[t], 0, 0, 0);
     }
+    fetch(x, ci + kAhead);
+    read_out(ci - 1, buf);
   };
-  fetch_products(even, 0);
-  fetch_update(even, 0);
-  fetch_products(odd, 1);
-  fetch_update(odd, 1);
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) fetch(ops[i], i);
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the loop's own waits then count the loop's loads only
-  for (int ci = 0; ci < nc; ci += 2) {
-    step(even, ci);
-    if (ci + 1 >= nc) break;
-    step(odd, ci + 1);
+  int ci = 0;
+  for (; ci + kAhead <= nc; ci += kAhead) {   // no exit in between: a wait would cover the loads of the shortest way round
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) step(ops[i], ci + i);
   }
 #pragma unroll
-  for (int b = 0; b < TPW; ++b)
+  for (int i = 0; i < kAhead - 1; ++i)
+    if (ci + i < nc) step(ops[i], ci + i);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int k = 16 * (wave * TPW + b) + 4 * g + r;
-      if (k < dim && col < vdim) Sp[(long)k * vdim] = st[b][r];
-    }
+  for (int t = 0; t < NC; ++t) sums[nc & 1][1][t][wave][lane] = os[t];
+  __syncthreads();
+  read_out(nc - 1, nc & 1);
+#pragma unroll
+  for (int t = 0; t < NC; ++t)
+#pragma unroll
+    for (int b = 0; b < TPW; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int k = 16 * (wave * TPW + b) + 4 * g + r;
+        if (k < dim && v0 + 16 * t + c < vdim) Sp[(long)k * vdim + 16 * t] = st[t][b][r];
+      }
 }
 
 int padded(int dim) { return dim <= 16 ? 16 : dim <= 32 ? 32 : dim <= 64 ? 64 : 128; }
@@ -347,8 +384,8 @@ void launch_delta_chunk(float* o, float* S, float* buf, const float* qk, const f
                         const float* bb, const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int T,
                         int heads, int kv_heads, int dim, int vdim, bool channel, hipStream_t s) {
   const int VP = (vdim + 15) / 16 * 16;
-  dim3 pgrid(heads, delta_chunk_bound(T, nseq)), sgrid(heads, VP / 16, nseq);
-#define HS_DC(DS, TPW, NW)                                                                                             \
+  dim3 pgrid(heads, delta_chunk_bound(T, nseq)), sgrid(heads, (VP + 31) / 32, nseq), sgrid1(heads, VP / 16, nseq);
+#define HS_DC(DS, TPW, NW, NC)                                                                                             \
   do {                                                                                                                 \
     if (channel)                                                                                                       \
       delta_chunk_prepare_kernel<DS, true><<<pgrid, 256, 0, s>>>(buf, qk, vv, gg, bb, seq_cu, nseq, heads, kv_heads, dim,  \
@@ -356,14 +393,14 @@ void launch_delta_chunk(float* o, float* S, float* buf, const float* qk, const f
     else                                                                                                               \
       delta_chunk_prepare_kernel<DS, false><<<pgrid, 256, 0, s>>>(buf, qk, vv, gg, bb, seq_cu, nseq, heads, kv_heads, dim, \
                                                                   vdim, VP);                                           \
-    delta_chunk_scan_kernel<TPW, NW><<<sgrid, 64 * NW, 0, s>>>(o, S, buf, seq_cu, seq_ctx, seq_state, heads, dim, vdim, VP,  \
+    delta_chunk_scan_kernel<TPW, NW, NC><<<NC == 1 ? sgrid1 : sgrid, 64 * NW, 0, s>>>(o, S, buf, seq_cu, seq_ctx, seq_state, heads, dim, vdim, VP,  \
                                                                (long)T * heads * vdim);                                \
   } while (0)
   switch (padded(dim)) {
-    case 16: HS_DC(1, 1, 1); break;
-    case 32: HS_DC(2, 1, 2); break;
-    case 64: HS_DC(4, 1, 4); break;
-    default: HS_DC(8, 2, 4); break;
+    case 16: HS_DC(1, 1, 1, 1); break;
+    case 32: HS_DC(2, 1, 2, 2); break;
+    case 64: HS_DC(4, 1, 4, 2); break;
+    default: HS_DC(8, 2, 4, 2); break;
   }
 #undef HS_DC
 }
