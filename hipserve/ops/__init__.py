@@ -303,7 +303,7 @@ class KernelOps:
                                  sp.scaling.amplitude if sp.scaling is not None else 1.0, sp.temp_coef, sp.temp_every)
 
     WINDOW_PREFILL_TQ = 4  # tokens per workgroup of a prompt portion (x the query heads of one key/value head)
-    # bf16 runs the MFMA kernel (HIPSERVE_WINDOW_MFMA=0: the generic kernel, as fp32 does)
+    # the matrix-core kernels where they take the sizes (HIPSERVE_WINDOW_MFMA=0: the generic kernel)
     WINDOW_MFMA = os.environ.get("HIPSERVE_WINDOW_MFMA", "1") != "0"
     WINDOW_DECODE_RUN = 128  # keys per run of a decode row (a multiple of 32)
 
@@ -384,7 +384,7 @@ class KernelOps:
                                            sp.heads, sp.kv_heads, sp.dim, sp.vdim, gate_off, sp.scale, sp.window,
                                            sp.sink, out_scale, *diff)
 
-    # bf16 prompt portions of at least this many rows run the gated delta rule in chunks on the (fp32) matrix cores
+    # bf16 prompt portions of at least this many rows run the delta rules in chunks on the (fp32) matrix cores
     # (HIPSERVE_DELTA_CHUNK=0: token by token on the scan, as fp32 does)
     DELTA_CHUNK = os.environ.get("HIPSERVE_DELTA_CHUNK", "1") != "0"
     DELTA_CHUNK_ROWS = 32
