@@ -16,12 +16,14 @@ HS_DEVICE void barrier_all() {
 }
 // 1 KB from the lanes' addresses to LDS, 16 bytes per lane side by side, asynchronously. Written out because the compiler
 // would otherwise wait for every copy in flight before the next transposing read; the waits are the callers' barrier_all.
+// A copy takes its place in LDS from m0 and must not follow a scalar write of m0 directly: one wait state, which the
+// compiler does not add inside an asm block.
 HS_DEVICE void copy_1k(const unsigned short* src, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src) : "memory");   // nothing else in those files uses m0
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src) : "m0", "memory");
 }
 // The same from a uniform base and the lanes' byte offsets.
 HS_DEVICE void copy_1k(const unsigned char* base, unsigned off, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(base) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(off), "s"(base) : "m0", "memory");
 }
 // Where a pointer into LDS points, for copy_1k: once, since turning a generic pointer into an offset costs a test.
 HS_DEVICE unsigned lds_at(const unsigned char* p) {

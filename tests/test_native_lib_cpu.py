@@ -2,10 +2,13 @@
 declared in kernels.h but left undefined fails here, not on the GPU box) and registers
 the ops the Python layer calls."""
 import os
+import re
+import subprocess
 
 import pytest
 import torch
 
+from hipserve import _build
 from hipserve.ops import library_path
 
 
@@ -17,3 +20,23 @@ def test_library_loads_and_registers_ops():
     for op in ("decode_gemm_partial", "gguf_gemm_parts", "fp8_untile", "gguf_dequant_tiled", "paged_decode",
                "splitk_add_rmsnorm", "prefill_gemm_packed", "fp8_decode_gemm"):
         assert hasattr(torch.ops.hipserve, op), op
+
+
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+@pytest.mark.parametrize("name", ["window_attention_dma", "latent_attention_dma"])
+def test_copies_into_lds_keep_their_wait_states(name, tmp_path):
+    """The copies of lds_copy.h are inline assembly, which the compiler's hazard pass does not look into: between the scalar write of
+    m0 (the place in LDS) and the copy lies another instruction, and the vector unit has not written the base address just before."""
+    asm = tmp_path / "k.s"
+    subprocess.run([_build.HIPCC, *_build.HIP_FLAGS, "-I", os.path.join(_build.CSRC, "include"), "-S", "--cuda-device-only",
+                    os.path.join(_build.CSRC, "kernels", "seq", name + ".hip"), "-o", asm], check=True, capture_output=True)
+    lines = [ln.strip() for ln in asm.read_text().splitlines()]
+    code = [ln for ln in lines if ln and ln[0] not in ".;/" and not ln.endswith(":")]
+    copies = [i for i, ln in enumerate(code) if ln.startswith("global_load_lds")]
+    assert copies
+    for i in copies:
+        assert not re.match(r"s_\w+ m0\b", code[i - 1]), code[i - 1:i + 1]
+        base = re.search(r", s\[(\d+):(\d+)\]", code[i])
+        for ln in code[i - 5:i] if base else ():
+            wrote = re.match(r"v_(?:readfirstlane|readlane|cmp)\w* s\[?(\d+)(?::(\d+))?", ln)
+            assert not wrote or int(wrote[2] or wrote[1]) < int(base[1]) or int(wrote[1]) > int(base[2]), (ln, code[i])
