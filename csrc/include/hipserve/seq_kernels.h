@@ -53,13 +53,13 @@ void launch_latent_attention_mfma(void* o_lat, const void* qc, const void* proj,
                                   float* ws_acc, float* ws_ml, int row_base, hipStream_t s);
 
 // The same for kv_rank 128 / 256 / 512 and rot_dim 64 (latent_attention_dma.hip). q (may be null): the rotary part of the
-// queries is rotated here, from q rows [heads, dim + 64], instead of read from qc (32 frequencies). one_row: every sequence
-// has one row (rows_bound of them), with or without runs; merged by launch_latent_attention_reduce.
+// queries is rotated here, from q rows [heads, dim + 64], instead of read from qc (32 frequencies). Runs (nparts > 1) are merged
+// by launch_latent_attention_reduce.
 bool latent_attention_dma_ok(int kv_rank, int rot_dim);
 bool launch_latent_attention_dma(void* o_lat, const void* qc, const void* q, const long* positions, const float* inv_freq,
                                  const void* proj, long proj_ld, const void* cache, int block_size, const int* seq_cu,
                                  const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int seq1, int rows_bound, int T,
-                                 int heads, int dim, int kv_rank, int gate_off, float scale, int window, bool one_row, int nparts,
+                                 int heads, int dim, int kv_rank, int gate_off, float scale, int window, int nparts,
                                  int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s);
 void launch_latent_attention_reduce(void* o_lat, const float* ws_acc, const float* ws_ml, const void* proj, long proj_ld,
                                     int gate_off, int nparts, int heads, int rows_bound, int row_base, int T, int kv_rank,

@@ -96,14 +96,11 @@ inline void latent_attention_mfma(at::Tensor& o_lat, at::Tensor& qc, const c10::
       hipserve::launch_latent_q_cat(qc.data_ptr(), q_abs.has_value() ? q_abs->data_ptr<float>() : nullptr, q.data_ptr(),
                                     positions.data_ptr<long>(), inv_freq.data_ptr<float>(), inv_freq.numel(), T, heads, dim,
                                     rot_dim, kv_rank, cur_stream());
-    const bool one_row = rows_bound == seq1 - seq0;   // as decode rows are
-    TORCH_CHECK(one_row || nparts == 1, "latent_attention_mfma: runs of keys are for sequences of one row");
     TORCH_CHECK(hipserve::launch_latent_attention_dma(
                     o_lat.data_ptr(), qc.data_ptr(), rotate ? q.data_ptr() : nullptr, positions.data_ptr<long>(),
                     inv_freq.data_ptr<float>(), proj.data_ptr(), proj.stride(0), cache.data_ptr(), cache.size(1),
                     seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_bt.data_ptr<int>(), seq_bt.size(1), seq0, seq1, rows_bound,
-                    T, heads, dim, kv_rank, gate_off, (float)scale, window, one_row, nparts, part_keys, wa, wm, row_base,
-                    cur_stream()),
+                    T, heads, dim, kv_rank, gate_off, (float)scale, window, nparts, part_keys, wa, wm, row_base, cur_stream()),
                 "latent attention: no LDS");
     if (nparts > 1 && seq1 > seq0 && rows_bound > 0)
       hipserve::launch_latent_attention_reduce(o_lat.data_ptr(), wa, wm, proj.data_ptr(), proj.stride(0), gate_off, nparts, heads,

@@ -21,7 +21,7 @@
 // unit is busy 220 k, the vector unit 125 k, the LDS 180 k; the rest waits for operands and at the one barrier per tile).
 // On the way, in one run: 449 with eight-way swizzles (operand rows met two to a bank) and a rescaling per tile; 386 with
 // the rescaling mended. Without overlap of the scores with the next tile's operand reads a fifth more.
-// latent_dma_decode_kernel serves decode rows: a workgroup takes 16 heads of one sequence and a run of keys, 64 of them
+// latent_dma_decode_kernel serves decode rows: a workgroup takes 16 heads of one row and a run of keys, 64 of them
 // at a time; its waves split the keys for S and the latent dims for P . V. One row of 724 keys, 16 heads: 46 -> 10 us.
 #include "lds_copy.h"
 #include "seq_common.h"
@@ -347,16 +347,16 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
   }
 }
 
-// Decode rows, one per sequence: 16 heads of sequence seq0 + blockIdx.x against the run blockIdx.z of part_keys keys,
-// 64 at a time. Wave w: scores of keys 16 w .., P . V of the latent dims DV / 4 w ... With runs the unnormalised
-// outputs and (max, sum) go to ws_acc / ws_ml.
+// 16 heads of the portion's row blockIdx.x against the run blockIdx.z of part_keys keys, 64 at a time: for portions of a row per
+// sequence, as decode rows are, and for runs. Wave w: scores of keys 16 w .., P . V of the latent dims DV / 4 w ... With
+// runs the unnormalised outputs and (max, sum) go to ws_acc / ws_ml.
 template <int DV>
 __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
     unsigned short* __restrict__ o_lat, const unsigned short* __restrict__ qc, const unsigned short* __restrict__ q,
     const long* __restrict__ positions, const float* __restrict__ inv_freq, const unsigned short* __restrict__ proj,
     long proj_ld, const unsigned short* __restrict__ cache, int block_shift, const int* __restrict__ seq_cu,
-    const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0, int T_rows, int heads,
-    int dim, int gate_off, float scale, int window, int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
+    const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0, int seq1, int T_rows,
+    int heads, int dim, int gate_off, float scale, int window, int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
     int row_base, int ws_rows) {
   constexpr int kTile = 64, kPd = kTile + 8;   // kPd: row stride of P in elements
   using KT = Tile<DV, kTile>;
@@ -365,18 +365,24 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
   unsigned short* p_lds = reinterpret_cast<unsigned short*>(smem + KT::kBytes);   // [16][kPd], MFMA k order
   float* mw = reinterpret_cast<float*>(p_lds + 16 * kPd);                         // [4][16] the waves' maxima
   float* lw = mw + 64;                                                            // [4][16] the waves' sums
-  const int s = seq0 + blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  int s, tok0;
+  if (!find_row(seq_cu, seq0, seq1, blockIdx.x, s, tok0)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
   const int head = blockIdx.y * 16 + c;
   const bool act = head < heads;
-  const long trow = seq_cu[s];
-  const int pos = seq_ctx[s] - 1;
+  const int r0 = seq_cu[s], pos = seq_ctx[s] - (seq_cu[s + 1] - r0) + tok0;
+  const long trow = r0 + tok0;
   const int lo = (window > 0 ? max(0, pos - window + 1) : 0) + blockIdx.z * part_keys;
   const int hi = gridDim.z > 1 ? min(pos, lo + part_keys - 1) : pos;
   const bool partial = gridDim.z > 1;
   const long wrow = ((long)blockIdx.z * heads + (act ? head : 0)) * ws_rows + (trow - row_base);
-  if (lo > hi) {   // an empty run: its weight in the merge is 0
+  const int d0 = 16 * NPW * wave + 4 * g;   // the lane's latent dims of the output: 16 j + d0 .. + 3
+  if (lo > hi) {   // an empty run, whose weight in the merge is 0, or a row that sees no key
     if (partial && act && wave == 0 && g == 0) { ws_ml[2 * wrow] = -INFINITY; ws_ml[2 * wrow + 1] = 0.f; }
+    if (!partial && act)
+#pragma unroll
+      for (int j = 0; j < NPW; ++j) *reinterpret_cast<u16x4*>(o_lat + ((long)head * T_rows + trow) * DV + d0 + 16 * j) = u16x4{0, 0, 0, 0};
     return;
   }
   const int* bt = seq_bt + (long)s * bt_width;
@@ -449,7 +455,6 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
     }
   }
   if (!act) return;
-  const int d0 = 16 * NPW * wave + 4 * g;
   if (partial) {
     if (wave == 0 && g == 0) { ws_ml[2 * wrow] = m_run / kLog2e; ws_ml[2 * wrow + 1] = l_run; }
 #pragma unroll
@@ -478,16 +483,16 @@ template <int DV>
 bool launch_dma(void* o_lat, const void* qc, const void* q, const long* positions, const float* inv_freq, const void* proj,
                 long proj_ld, const void* cache, int block_shift, const int* seq_cu, const int* seq_ctx, const int* seq_bt,
                 int bt_width, int seq0, int seq1, int rows_bound, int T, int heads, int dim, int gate_off, float scale,
-                int window, bool one_row, int nparts, int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s) {
+                int window, int nparts, int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s) {
   auto o = (unsigned short*)o_lat;
   auto a = (const unsigned short*)qc, b = (const unsigned short*)q, p = (const unsigned short*)proj, k = (const unsigned short*)cache;
-  if (one_row) {
+  if (nparts > 1 || rows_bound == seq1 - seq0) {   // either kernel takes any rows: a workgroup per row where they are single ones
     constexpr size_t smem = Tile<DV, 64>::kBytes + 16 * (64 + 8) * 2 + 128 * 4;
     static_assert(smem <= 80 * 1024, "two workgroups per CU");
     static const bool ok = allow_lds(&latent_dma_decode_kernel<DV>, smem);
     if (!ok) return false;
     latent_dma_decode_kernel<DV><<<dim3(rows_bound, (heads + 15) / 16, nparts), 256, smem, s>>>(
-        o, a, b, positions, inv_freq, p, proj_ld, k, block_shift, seq_cu, seq_ctx, seq_bt, bt_width, seq0, T, heads, dim, gate_off,
+        o, a, b, positions, inv_freq, p, proj_ld, k, block_shift, seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, T, heads, dim, gate_off,
         scale, window, part_keys, ws_acc, ws_ml, row_base, rows_bound);
     return true;
   }
@@ -511,13 +516,13 @@ bool latent_attention_dma_ok(int kv_rank, int rot_dim) {
 bool launch_latent_attention_dma(void* o_lat, const void* qc, const void* q, const long* positions, const float* inv_freq,
                                  const void* proj, long proj_ld, const void* cache, int block_size, const int* seq_cu,
                                  const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int seq1, int rows_bound, int T,
-                                 int heads, int dim, int kv_rank, int gate_off, float scale, int window, bool one_row, int nparts,
+                                 int heads, int dim, int kv_rank, int gate_off, float scale, int window, int nparts,
                                  int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s) {
   if (seq1 <= seq0 || rows_bound <= 0) return true;
   const int block_shift = __builtin_ctz(block_size);   // a power of two
 #define HS_LD(DV)                                                                                                        \
   launch_dma<DV>(o_lat, qc, q, positions, inv_freq, proj, proj_ld, cache, block_shift, seq_cu, seq_ctx, seq_bt, bt_width, \
-                 seq0, seq1, rows_bound, T, heads, dim, gate_off, scale, window, one_row, nparts, part_keys, ws_acc,     \
+                 seq0, seq1, rows_bound, T, heads, dim, gate_off, scale, window, nparts, part_keys, ws_acc,     \
                  ws_ml, row_base, s)
   return kv_rank == 128 ? HS_LD(128) : kv_rank == 256 ? HS_LD(256) : HS_LD(512);
 #undef HS_LD

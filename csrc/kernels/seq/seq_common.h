@@ -120,6 +120,15 @@ HS_DEVICE bool find_row_tile(const int* __restrict__ seq_cu, int seq0, int seq1,
   return false;
 }
 
+// Row `wg` of the sequences seq0 .. seq1 - 1: its sequence and its place there; false past the last row. Decode rows, one per
+// sequence, need no search.
+HS_DEVICE bool find_row(const int* __restrict__ seq_cu, int seq0, int seq1, int wg, int& s, int& tok0) {
+  s = seq0 + wg;
+  tok0 = 0;
+  if (s < seq1 && seq_cu[s] - seq_cu[seq0] == wg && seq_cu[s + 1] - seq_cu[s] == 1) return true;
+  return find_row_tile(seq_cu, seq0, seq1, 1, wg, s, tok0);
+}
+
 // First key (behind the kept ones) that position pos sees: its window's, its chunk's, or the sequence's first.
 HS_DEVICE int first_key(int pos, int window, int chunk) {
   return chunk > 0 ? pos - pos % chunk : window > 0 ? max(0, pos - window + 1) : 0;

@@ -214,9 +214,9 @@ def test_expert_gemm_tiles_of_few_rows(tokens, E, top, N, K, act):
 
 
 # ------------------------------------------------------------------ latent attention
-def latent_case(lens, ctxs, heads, dim, kv, rot, block, dtype, dev, seed=0):
+def latent_case(lens, ctxs, heads, dim, kv, rot, block, dtype, dev, seed=0, nd=None):
     """Rows of sequences with ``lens`` rows in this step and ``ctxs`` tokens after it: random queries, a random paged cache whose
-    pages lie in no order, and a meta of prompt portions first (lens > 1), single rows last."""
+    pages lie in no order, and a meta of prompt portions first (lens > 1), ``nd`` sequences of decode rows last (the single rows)."""
     from hipserve.models.llama import AttnMeta
 
     g = torch.Generator().manual_seed(seed)
@@ -228,8 +228,8 @@ def latent_case(lens, ctxs, heads, dim, kv, rot, block, dtype, dev, seed=0):
     q_abs = torch.randn(heads, T, kv + rot, generator=g).to(dtype) * 0.3
     q = torch.randn(T, heads * (dim + rot), generator=g).to(dtype)
     proj = torch.randn(T, heads + 3, generator=g).to(dtype)
-    nd = sum(n == 1 for n in lens)
-    meta = AttnMeta(num_prefill_tokens=T - nd, num_decode=nd, positions=pos.to(dev), slot_mapping=pos.to(dev), seq_cu=cu.to(dev),
+    nd = sum(n == 1 for n in lens) if nd is None else nd
+    meta = AttnMeta(num_prefill_tokens=int(cu[len(lens) - nd]), num_decode=nd, positions=pos.to(dev), slot_mapping=pos.to(dev), seq_cu=cu.to(dev),
                     seq_ctx=torch.tensor(ctxs, dtype=torch.int32, device=dev), seq_bt=bt.to(dev), max_q=max(lens), max_ctx=max(ctxs))
     return cache, cu, pos, bt, q_abs, q, proj, meta
 
@@ -237,12 +237,14 @@ def latent_case(lens, ctxs, heads, dim, kv, rot, block, dtype, dev, seed=0):
 @gpu
 @pytest.mark.parametrize("kv", [128, 256, 512])
 @pytest.mark.parametrize("heads,window", [(16, 0), (5, 100), (70, 33)])
-@pytest.mark.parametrize("lens,ctxs", [([1], [1]), ([1, 1, 1], [64, 65, 700]), ([37], [37]), ([33, 5, 1], [33, 400, 129]), ([2, 190], [31, 255])])
-def test_latent_attention_dma(kv, heads, window, lens, ctxs):
+@pytest.mark.parametrize("lens,ctxs,nd", [([1], [1], 1), ([1, 1, 1], [64, 65, 700], 3), ([37], [37], 0), ([33, 5, 1], [33, 400, 129], 1), ([2, 190], [31, 255], 0),
+                                          ([2, 0], [31, 5], 0), ([1, 0, 1], [64, 9, 700], 0), ([2, 0, 1], [31, 5, 300], 1), ([2, 0], [300, 5], 2)])
+def test_latent_attention_dma(kv, heads, window, lens, ctxs, nd):
     """Tiles of 32 and 64 keys filled partly, windows that start inside a tile, rows that leave a workgroup's tiles unused, runs of
-    keys of a decode row (some empty), the rotary part formed in the kernel, in 64 bits."""
+    keys of a decode row (some empty), as many rows as sequences, not one each (with runs too), the rotary part formed in
+    the kernel, in 64 bits."""
     rot, dim, block, gate, scale = 64, 24, 16, 2, 0.11
-    cache, cu, pos, bt, q_abs, q, proj, meta = latent_case(lens, ctxs, heads, dim, kv, rot, block, torch.bfloat16, "cuda", kv + heads)
+    cache, cu, pos, bt, q_abs, q, proj, meta = latent_case(lens, ctxs, heads, dim, kv, rot, block, torch.bfloat16, "cuda", kv + heads, nd)
     inv = torch.pow(torch.tensor(1e4), -2.0 * torch.arange(rot // 2) / rot)
     T = sum(lens)
     qr = q.double().view(T, heads, dim + rot)[..., dim:]
