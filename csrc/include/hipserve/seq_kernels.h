@@ -170,7 +170,7 @@ void launch_window_attention_dma(void* out, long out_ld, const void* proj, long 
                                  float out_scale, bool wide, float softcap, const float* sink_w, bool channel_gate, int chunk,
                                  hipStream_t s);
 
-// Decode rows (window_attention_decode.hip), bf16 or fp32: sequences seq0 .. seq0 + rows - 1 have one row each, batch rows
+// Decode rows (window_attention_decode.hip), bf16 or fp32: sequences seq0 .. seq0 + rows - 1 have up to that many rows, batch rows
 // row_base on; blocks of a power of two of rows; proj and cache rows at multiples of 16 bytes; nparts and part_keys as above.
 bool window_attention_decode_ok(int dim, int vdim, int block_size, bool f32);
 void launch_window_attention_decode(void* out, long out_ld, const void* proj, long proj_ld, const void* cache, int block_size,

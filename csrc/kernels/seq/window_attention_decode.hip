@@ -1,4 +1,4 @@
-// Window attention of decode rows (one token per sequence, one map per head; same cache, masks, sink and gates as
+// Window attention of decode rows (a workgroup per row, one map per head; same cache, masks, sink and gates as
 // window_attention.hip), bf16 and fp32, heads of 64, 128 (and in bf16 256) dims.
 //
 // A workgroup owns up to 16 query heads of one key / value head and a run of keys. Its waves take tiles of 32 keys (fp32: 16)
@@ -75,15 +75,14 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
   constexpr int E = F32 || D == 64 ? 4 : 8, NB = D / (16 * E);   // dims of a value row per load; loads per row
   extern __shared__ float lds[];                           // [waves][rows][D]; [waves][16][2]
   using S = Softmax<T>;
-  int s = seq0 + blockIdx.x, tok0 = 0;
-  if (MULTI && !find_row_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) return;
+  int s, tok0;
+  if (!(MULTI ? find_row_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0) : find_row(seq_cu, seq0, seq1, blockIdx.x, s, tok0))) return;
   const int seq_r0 = seq_cu[s], n = seq_cu[s + 1] - seq_r0, ctx = seq_ctx[s];
-  if (n <= 0) return;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
   const int group = heads / kv_heads, kvh = blockIdx.y / hchunks, h0 = (blockIdx.y % hchunks) * hc;
   const int nh = min(hc, group - h0), head0 = kvh * group + h0;
-  const int ntok = MULTI ? min(tq, n - tok0) : 1, p_first = MULTI ? ctx - n + tok0 : ctx - 1, p = p_first + ntok - 1;
+  const int ntok = MULTI ? min(tq, n - tok0) : 1, p_first = ctx - n + tok0, p = p_first + ntok - 1;
   const int lo_all = first_key(max(p_first, 0), window, chunk);
   // this lane's row
   const int rt = MULTI ? c / hc : 0, rh = MULTI ? c % hc : c;

@@ -396,6 +396,30 @@ def test_window_attention_decode(heads, kv, dim, ctxs, opts, dtype):
         assert ((out.double().cpu() - want).abs() <= tol * want.abs() + least * rows.abs().max() * 0.5).all()
 
 
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("ctx", [40, 700])   # one run of keys, several
+def test_window_attention_decode_rows_of_one_sequence(ctx, dtype):
+    """Row counts (2, 0, 1): every row sees what it would see as its sequence's last one, in the same bits."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(ctx)
+    heads, kv, dim, bs = 4, 2, 64, 16
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=0, reach=0, scale=dim ** -0.5, sink=False,
+                         keep_first=0, softcap=0.0, channel_gate=False, chunk=0)
+    width = -(-ctx // bs)
+    bt = torch.randperm(3 * width, generator=g).int().view(3, width).cuda()
+    cache, proj = torch.randn(3 * width, bs, 2 * kv * dim, generator=g).to(dtype).cuda(), torch.randn(3, heads * dim, generator=g).to(dtype).cuda()
+
+    def run(cu, ctxs, tables):
+        meta = SimpleNamespace(seq_ctx=torch.tensor(ctxs).int().cuda(), seq_cu=torch.tensor(cu).int().cuda(), seq_bt=tables.contiguous(),
+                               num_decode=3, num_prefill_tokens=0, max_ctx=ctx)
+        out = torch.full((3, heads * dim), float("nan"), dtype=dtype, device="cuda")
+        assert get_ops("cuda")._window_decode(out, proj, cache, meta, sp, -1, 1.0, None)
+        return out
+    want = run([0, 1, 2, 3], [ctx - 1, ctx, ctx - 5], bt[[0, 0, 2]])
+    assert torch.equal(run([0, 2, 2, 3], [ctx, 9, ctx - 5], bt), want) and want.isfinite().all()
+
+
 # ------------------------------------------------------------------ generalized delta rule in chunks
 @gpu
 @pytest.mark.parametrize("lens", [[32], [33, 1, 16], [40, 15, 100]])
