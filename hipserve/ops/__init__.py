@@ -466,6 +466,8 @@ class KernelOps:
                 return out
         if out_f32 and x.dtype != torch.float32:
             y = torch.mm(x, w.t(), out_dtype=torch.float32)
+            if bias is not None:
+                y += bias
         else:
             y = F.linear(x, w, bias)
         if act is None:
@@ -846,7 +848,7 @@ class ReferenceOps:
 
     def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0):
         if out_f32 and x.dtype != torch.float32:
-            x, w = x.float(), w.float()
+            x, w, bias = x.float(), w.float(), None if bias is None else bias.float()
         y = F.linear(x, w, bias)
         if act is None:
             return y

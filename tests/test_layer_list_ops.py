@@ -169,6 +169,19 @@ def test_linear_with_activation(M, act, c0, c1):
             assert ((got.double().cpu() - want).abs() <= 12 * 2.0 ** -8 * z.abs().max()).all()
 
 
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=gpu)])
+@pytest.mark.parametrize("M", [5, 70])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_linear_bias_of_32_bit_results(M, dtype, dev):
+    """The bias is added whichever product runs."""
+    (x,), (w,) = dense_case(1, M, 32, 64, M)
+    x, w = x.to(dtype), w.to(dtype)
+    bias = torch.randn(32, generator=torch.Generator().manual_seed(1)).to(dtype)
+    got = get_ops(dev).linear(x.to(dev), w.to(dev), bias.to(dev), out_f32=True)
+    assert got.dtype == torch.float32
+    close_to(got, x.double() @ w.double().T + bias.double(), x, w)
+
+
 @gpu
 @pytest.mark.parametrize("B,M,N,K", [(3, 1, 40, 16), (16, 17, 512, 128), (5, 64, 24, 520), (2, 33, 128, 512)])
 def test_skinny_heads(B, M, N, K):
