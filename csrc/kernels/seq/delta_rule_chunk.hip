@@ -12,8 +12,9 @@
 // delta_rule_chunk_scan: one workgroup per (sequence, head, 32 value channels) walks the chunks as in delta_chunk.hip, with
 // U = -X: U = U0 + W S (W = -(1 + A)^-1 U), O = R S + Pa U + Pk V, S = E S + KA U + KK V.
 // A product over the chunk would carry a NaN or an infinity of one token's inputs to the tokens before it (0 times it), so such
-// a token takes part as zeros and F carries NaN to its outputs and (unless only r was not finite) all that follow.
-// What bounds it: the prepared operands (6752 floats per head and chunk) are written and read once, and the scan's products.
+// inputs take part as zeros: F carries NaN to the outputs of a token whose r is not finite, B says from which token on a column is
+// NaN, all columns where k is not finite or a pre-activation is NaN (infinite ones saturate), one where its value is not finite.
+// What bounds it: the prepared operands (6800 floats per head and chunk) are written and read once, and the scan's products.
 // 8192 rows (4 prompts) x 32 heads: rows prepared one by one and scanned token by token (five row vectors through LDS for
 // every 4 state elements of a lane) took 126 + 700 us; this 169 + 197. Relative error of the state against 64 bits after 2048
 // tokens: 7.5e-8 (6.5e-8 token by token; outputs are rounded to bf16), with the tokens in their natural order 1.3e-7.
@@ -25,16 +26,16 @@ namespace {
 
 constexpr int kC = 16, kD = 64, kLd = kD + 4;   // tokens per chunk; key and value channels of a head; LDS row
 
-// Buffers per (chunk, head): W, R [16][64], KA, KK [64][16], U0, V [64][16], E [64], Pa, Pk [16][16], F [32]
+// Buffers per (chunk, head): W, R [16][64], KA, KK [64][16], U0, V [64][16], E [64], Pa, Pk [16][16], F [16], B [64]
 struct Buf {
-  float *W, *R, *KA, *KK, *U, *V, *E, *Pa, *Pk, *F;
+  float *W, *R, *KA, *KK, *U, *V, *E, *Pa, *Pk, *F, *B;
 };
-constexpr long kBuf = 6L * kC * kD + kD + 2 * kC * kC + 2 * kC;
+constexpr long kBuf = 6L * kC * kD + 2 * kD + 2 * kC * kC + kC;
 HS_DEVICE Buf buf_of(float* base, long item) {
   float* p = base + item * kBuf;
   constexpr int m = kC * kD;
   return Buf{p,         p + m,          p + 2 * m,           p + 3 * m, p + 4 * m, p + 5 * m, p + 6 * m, p + 6 * m + kD,
-             p + 6 * m + kD + kC * kC, p + 6 * m + kD + 2 * kC * kC};
+             p + 6 * m + kD + kC * kC, p + 6 * m + kD + 2 * kC * kC, p + 6 * m + kD + 2 * kC * kC + kC};
 }
 
 // Where a token stands in the buffers' rows and columns: a lane's four values 4 g + r are the tokens 4 r + g, so that the k steps
@@ -51,13 +52,15 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
   __shared__ __attribute__((aligned(16))) float su[kC][kLd], sr[kC][kLd], sa[kC][kLd], sk[kC][kLd], sv[kC][kLd];
   __shared__ __attribute__((aligned(16))) float sx[kC][kLd], sy[kC][kLd];   // the decays, then KA; KK
   __shared__ __attribute__((aligned(16))) float sA[kC][20], sB[kC][20], sM[kC][20];
-  __shared__ float sf[2][kC];   // NaN: a token's inputs, its r, are not finite
+  __shared__ float sf[2][kC];   // NaN: what reaches every column of a token's, its r, is not finite
+  __shared__ int sv_bad[kD];    // a column's first value that is not finite
   int s, t0;
   if (!find_row_tile(seq_cu, 0, nseq, kC, blockIdx.y, s, t0)) return;
   const int h = blockIdx.x, tid = threadIdx.x, row = tid >> 4, ch = 4 * (tid & 15);
   const int r0 = seq_cu[s] + t0, nt = min(kC, seq_cu[s + 1] - r0), N = heads * kD;
   const Buf out = buf_of(base, (long)blockIdx.y * heads + h);
   const bool in = row < nt;
+  if (tid < kD) sv_bad[tid] = kC;
   {
     const long t = r0 + (in ? row : 0);
     const int c = h * kD + ch;
@@ -71,11 +74,15 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
     Row<float, 4>::ld(a_b + c, ab);
     Row<float, 4>::ld(w0 + c, wb);
     float ss = 0.f, f = 0.f, fr = 0.f;
+    bool lost[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       ss += k[e] * k[e];
-      f += (k[e] - k[e]) + (v[e] - v[e]) + (a[e] - a[e]) + (w[e] - w[e]);   // 0 or NaN
+      a[e] = sigmoid_f(a[e] + ab[e]);
+      w[e] = expf(-0.60653065971263342f * sigmoid_f(w[e] + wb[e]));
+      f += (k[e] - k[e]) + (a[e] - a[e]) + (w[e] - w[e]);   // 0 or NaN
       fr += r[e] - r[e];
+      lost[e] = in && !(v[e] - v[e] == 0.f);
     }
     f = in ? row_sum(f) : 0.f;
     fr = in ? row_sum(fr) : 0.f;
@@ -85,13 +92,16 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       u[e] = use ? k[e] * inv : 0.f;
-      a[e] = use ? sigmoid_f(a[e] + ab[e]) * u[e] : 0.f;
-      w[e] = use ? expf(-0.60653065971263342f * sigmoid_f(w[e] + wb[e])) : 1.f;
-      if (!use) k[e] = v[e] = 0.f;
+      a[e] = use ? a[e] * u[e] : 0.f;
+      if (!use) { w[e] = 1.f; k[e] = 0.f; }
+      if (!use || lost[e]) v[e] = 0.f;
       if (!use || fr != 0.f) r[e] = 0.f;
     }
     Row<float, 4>::st(&sx[row][ch], w);
     __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (lost[e]) atomicMin(&sv_bad[ch + e], row);
     f32x4 before = {1.f, 1.f, 1.f, 1.f}, after = before;   // the decays of the chunk's earlier and later tokens
 #pragma unroll
     for (int m = 0; m < kC; ++m) {
@@ -122,10 +132,12 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
     *reinterpret_cast<f32x4*>(&sx[row][ch]) = ka;
     *reinterpret_cast<f32x4*>(&sy[row][ch]) = kk;
   }
-  if (tid <= kC) {   // F[i]: added to token i's outputs; F[16]: to all after the chunk
-    float f = tid < kC ? sf[1][tid] : 0.f;
-    for (int m = 0; m < kC; ++m) f += m <= tid ? sf[0][m] : 0.f;
-    out.F[tid < kC ? place(tid) : kC] = f;
+  if (tid < kC) out.F[place(tid)] = sf[1][tid];   // added to the token's outputs
+  if (tid < kD) {
+    int first = sv_bad[tid];
+    for (int m = kC - 1; m >= 0; --m)
+      if (sf[0][m] != 0.f) first = min(first, m);
+    out.B[tid] = (float)first;
   }
   // all pairs of tokens: wave 0 A, 1 B, 2 Pa, 3 Pk; lane (c, g) gets rows 4 g + r of column c
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
@@ -222,7 +234,7 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
   // younger loads behind it.
   struct Ops {
     f32x4 W, R, KA, KK, E, X, F;
-    float pa, pk, later;
+    float pa, pk, B[kTiles];
   } ops[kAhead];
   constexpr unsigned kM = kC * kD * sizeof(float);   // bytes of an operand of the buffer
   const unsigned rows = (c * kD + k0 + 4 * g) * 4, cols = ((k0 + c) * kC + 4 * g) * 4, states = (k0 + 4 * g) * 4, toks = 4 * g * 4,
@@ -231,7 +243,7 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
     const char* p = reinterpret_cast<const char*>(base + ((long)(first + min(ci, nc - 1)) * heads + h) * kBuf);
     auto get = [&](unsigned at) { return *reinterpret_cast<const f32x4*>(p + at); };
     auto one = [&](unsigned at) { return *reinterpret_cast<const float*>(p + at); };
-    constexpr unsigned kE = 6 * kM, kP = kE + kD * 4, kF = kP + 2 * kC * kC * 4;
+    constexpr unsigned kE = 6 * kM, kP = kE + kD * 4, kF = kP + 2 * kC * kC * 4, kB = kF + kC * 4;
     x.W = get(rows);
     x.R = get(kM + rows);
     x.X = get(vals_at);
@@ -241,12 +253,14 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
     x.E = get(kE + states);
     x.pa = one(kP + pair);
     x.pk = one(kP + kC * kC * 4 + pair);
-    x.later = one(kF + kC * 4);
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) x.B[t] = one(kB + (col0 + 16 * t + c) * 4);
   };
   auto of_wave = [&](const f32x4& v) { return high ? (odd ? v[3] : v[2]) : odd ? v[1] : v[0]; };
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 os[kTiles] = {};
-  float bad = 0.f;   // NaN once a token's inputs were not finite
+  float bad[kTiles] = {};   // NaN once a token's inputs were not finite
+  const float nan = __builtin_nanf("");
   float* po = o + (long)(r0 + 8 * half + g) * N + h * kD + col0 + 16 * mine + c;
   float* nowhere = o + pad + lane;
   // the outputs of chunk ci from the sums in sums[buf]: wave w two rows of tile w % 2
@@ -271,7 +285,8 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) {
       us[t] = !high && odd == t ? x.X : zero;
-      rs[t] = !high && !odd ? x.F + bad : zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) rs[t][r] = !high && !odd ? x.F[r] + (x.B[t] <= 4 * r + g ? nan : bad[t]) : 0.f;
       sums[buf][1][t][wave][lane] = os[t];
     }
     vals[buf][wave][lane] = x.X;
@@ -311,7 +326,8 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
       os[t] = mfma(x.pk, of_wave(v[t]), rs[t]);
       os[t] = mfma(x.pa, of_wave(u[t]), os[t]);
     }
-    bad += x.later;
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) bad[t] = x.B[t] < kC ? nan : bad[t];
     fetch(x, ci + kAhead);
     read_out(ci - 1, buf);
   };
@@ -333,7 +349,7 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
 #pragma unroll
   for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) Sp[(long)(k0 + 4 * g + r) * kD + 16 * t] = st[t][r] + bad;
+    for (int r = 0; r < 4; ++r) Sp[(long)(k0 + 4 * g + r) * kD + 16 * t] = st[t][r] + bad[t];
 }
 
 }  // namespace

@@ -473,6 +473,38 @@ def test_delta_rule_chunks(lens):
         assert torch.equal(out.isnan(), hit) and torch.equal(out[~hit], got[~hit])
 
 
+@gpu
+@pytest.mark.parametrize("what,value", [("a", "inf"), ("a", "-inf"), ("w", "inf"), ("w", "-inf"), ("a", "nan"), ("w", "nan"), ("k", "nan"), ("k", "inf"),
+                                        ("r", "nan"), ("r", "-inf"), ("v", "nan"), ("v", "inf")])
+@pytest.mark.parametrize("row", [16, 21, 38])   # a chunk's first row, one inside, one in the last chunk (the next row spreads a NaN over the state's rows)
+def test_delta_rule_chunks_not_finite(row, what, value):
+    """What one input that is not finite does to outputs and states is what it does token by token: pre-activations saturate, a
+    value reaches its column alone."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(row)
+    H, d, lens = 2, 64, [40, 7]
+    N, T, eps = H * d, sum(lens), 1e-5
+    proj, wl, S = torch.randn(T, 5 * N, generator=g).bfloat16(), torch.randn(T, N, generator=g), torch.randn(2, H, d, d, generator=g)
+    a_b, w0, nw = torch.randn(N, generator=g), torch.randn(N, generator=g), torch.rand(N, generator=g) + 0.5
+    into, col = (wl, 5) if what == "w" else (proj, {"r": 0, "k": N, "v": 2 * N, "a": 3 * N}[what] + 5)
+    into[row, col] = float(value)
+    sp = SimpleNamespace(heads=H, dim=d, size=N)
+    meta = SimpleNamespace(seq_cu=torch.tensor([0, 40, 47]).int().cuda(), seq_ctx=torch.tensor([60, 7]).int().cuda(),
+                           seq_state=torch.tensor([1, 0]).int().cuda(), max_q=40)
+    res = []
+    for chunks in (False, True):
+        ops = get_ops("cuda")
+        ops.DELTA_CHUNK = chunks
+        out, state = torch.empty(T, N, dtype=torch.bfloat16, device="cuda"), S.cuda()
+        ops.delta_rule(out, [state], proj.cuda(), wl.cuda(), a_b.cuda(), w0.cuda(), nw.cuda(), sp, eps, meta)
+        res.append((out.float(), state))
+    for (want, got), tol, least in zip(zip(*res), (2.0 ** -7, 2.0 ** -15), (2.0 ** -13, 2.0 ** -15)):
+        assert torch.equal(got.isfinite(), want.isfinite())
+        want, got = want.nan_to_num(0.0, 0.0, 0.0), got.nan_to_num(0.0, 0.0, 0.0)
+        assert ((got - want).abs() <= tol * want.abs() + least * want.abs().max()).all()
+    assert bool(res[0][1].isfinite().all()) == (what == "r" or (what in "aw" and value != "nan"))
+
+
 # ------------------------------------------------------------------ window attention of prompts
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
