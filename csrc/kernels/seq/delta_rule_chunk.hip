@@ -12,36 +12,77 @@
 // delta_rule_chunk_scan: one workgroup per (sequence, head, 32 value channels) walks the chunks as in delta_chunk.hip, with
 // U = -X: U = U0 + W S (W = -(1 + A)^-1 U), O = R S + Pa U + Pk V, S = E S + KA U + KK V.
 // A product over the chunk would carry a NaN or an infinity of one token's inputs to the tokens before it (0 times it), so such
-// inputs take part as zeros: F carries NaN to the outputs of a token whose r is not finite, B says from which token on a column is
-// NaN, all columns where k is not finite or a pre-activation is NaN (infinite ones saturate), one where its value is not finite.
-// What bounds it: the prepared operands (6800 floats per head and chunk) are written and read once, and the scan's products.
+// inputs take part as zeros, and where a chunk has some the scan ends with a walk that writes NaN: to the outputs of a token whose r
+// is not finite (F), and to the outputs and the state of a column from the token on (B) whose value is not finite, or, all columns,
+// whose k is not finite or a pre-activation of which is NaN (infinite ones saturate).
+// What bounds it: the prepared operands (6816 floats per head and chunk) are written and read once, and the scan's products.
 // 8192 rows (4 prompts) x 32 heads: rows prepared one by one and scanned token by token (five row vectors through LDS for
-// every 4 state elements of a lane) took 126 + 700 us; this 169 + 197. Relative error of the state against 64 bits after 2048
-// tokens: 7.5e-8 (6.5e-8 token by token; outputs are rounded to bf16), with the tokens in their natural order 1.3e-7.
+// every 4 state elements of a lane) took 126 + 700 us; this 190 + 204.
+// Errors against 64 bits, over 32 .. 2048 tokens, fresh and carried states, strong and weak decays: state 5.8e-8 - 6.4e-8 (token by
+// token 6.3e-8 - 7.0e-8), outputs before their norm 7.2e-8 - 7.9e-8 (9.2e-8 - 9.8e-8). What it takes: decays and their products
+// in 64 bits, rounded once into the operands (else 7.9e-8 for the state); Pa and Pk summed in 64 bits and the larger part of an output added
+// last (else 1.3e-7); tokens that go from the oldest to the newest into the state (else 1.3e-7).
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
 
 namespace hipserve {
 namespace {
 
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
 constexpr int kC = 16, kD = 64, kLd = kD + 4;   // tokens per chunk; key and value channels of a head; LDS row
 
-// Buffers per (chunk, head): W, R [16][64], KA, KK [64][16], U0, V [64][16], E [64], Pa, Pk [16][16], F [16], B [64]
+// Buffers per (chunk, head): W, R [16][64], KA, KK [64][16], U0, V [64][16], E [64], Pa, Pk [16][16], F [16], B [64], any [1]
 struct Buf {
-  float *W, *R, *KA, *KK, *U, *V, *E, *Pa, *Pk, *F, *B;
+  float *W, *R, *KA, *KK, *U, *V, *E, *Pa, *Pk, *F, *B, *any;
 };
-constexpr long kBuf = 6L * kC * kD + 2 * kD + 2 * kC * kC + kC;
+constexpr long kBuf = 6L * kC * kD + 2 * kD + 2 * kC * kC + kC + 16;
 HS_DEVICE Buf buf_of(float* base, long item) {
   float* p = base + item * kBuf;
   constexpr int m = kC * kD;
   return Buf{p,         p + m,          p + 2 * m,           p + 3 * m, p + 4 * m, p + 5 * m, p + 6 * m, p + 6 * m + kD,
-             p + 6 * m + kD + kC * kC, p + 6 * m + kD + 2 * kC * kC, p + 6 * m + kD + 2 * kC * kC + kC};
+             p + 6 * m + kD + kC * kC, p + 6 * m + kD + 2 * kC * kC, p + 6 * m + kD + 2 * kC * kC + kC,
+             p + 6 * m + 2 * kD + 2 * kC * kC + kC};
 }
 
 // Where a token stands in the buffers' rows and columns: a lane's four values 4 g + r are the tokens 4 r + g, so that the k steps
 // r of a sum over the tokens take the oldest four first. Their decayed parts are small, and the sum rounds to the size it
 // has by then, as token by token.
 HS_DEVICE int place(int t) { return 4 * (t & 3) + (t >> 2); }
+
+// exp(-e^-1/2 s) for s in 0 .. 1, a token's decay, in 64 bits: rounded to 32 bits, the decays would cost the state as much as the
+// recurrence's own roundings. Taylor polynomial of exp around the middle, up to x^7: |x| <= e^-1/2 / 2 leaves 2e-9.
+HS_DEVICE double decay_of(float s) {
+  constexpr double c[7] = {1.0, 1.0, 1.0 / 2, 1.0 / 6, 1.0 / 24, 1.0 / 120, 1.0 / 720};
+  const double x = __builtin_fma((double)s, -0.6065306597126334, 0.3032653298563167);
+  double p = 1.0 / 5040.0;
+#pragma unroll
+  for (int i = 6; i >= 0; --i) p = __builtin_fma(p, x, c[i]);
+  return p * 0.738403149974731;   // exp(-e^-1/2 / 2)
+}
+
+// Of the two rows that differ in bit 4 (bit 5) of the lane, the other's number.
+HS_DEVICE double of_row_16(double x, bool odd) {
+  const u32x2 u = __builtin_bit_cast(u32x2, x);
+  u32x2 y;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto a = __builtin_amdgcn_permlane16_swap(u[i], u[i], false, false);
+    y[i] = odd ? a[0] : a[1];
+  }
+  return __builtin_bit_cast(double, y);
+}
+HS_DEVICE double of_row_32(double x, bool high) {
+  const u32x2 u = __builtin_bit_cast(u32x2, x);
+  u32x2 y;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto a = __builtin_amdgcn_permlane32_swap(u[i], u[i], false, false);
+    y[i] = high ? a[0] : a[1];
+  }
+  return __builtin_bit_cast(double, y);
+}
 
 HS_DEVICE f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 HS_DEVICE f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
@@ -50,7 +91,8 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
     float* __restrict__ base, const unsigned short* __restrict__ proj, long ld, const float* __restrict__ wl,
     const float* __restrict__ a_b, const float* __restrict__ w0, const int* __restrict__ seq_cu, int nseq, int heads) {
   __shared__ __attribute__((aligned(16))) float su[kC][kLd], sr[kC][kLd], sa[kC][kLd], sk[kC][kLd], sv[kC][kLd];
-  __shared__ __attribute__((aligned(16))) float sx[kC][kLd], sy[kC][kLd];   // the decays, then KA; KK
+  __shared__ __attribute__((aligned(16))) float sx[kC][kLd], sy[kC][kLd];   // KA, KK
+  __shared__ __attribute__((aligned(16))) double sg[4][kD];                 // decays of four rows
   __shared__ __attribute__((aligned(16))) float sA[kC][20], sB[kC][20], sM[kC][20];
   __shared__ float sf[2][kC];   // NaN: what reaches every column of a token's, its r, is not finite
   __shared__ int sv_bad[kD];    // a column's first value that is not finite
@@ -74,13 +116,14 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
     Row<float, 4>::ld(a_b + c, ab);
     Row<float, 4>::ld(w0 + c, wb);
     float ss = 0.f, f = 0.f, fr = 0.f;
+    double dec[4];
     bool lost[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       ss += k[e] * k[e];
       a[e] = sigmoid_f(a[e] + ab[e]);
-      w[e] = expf(-0.60653065971263342f * sigmoid_f(w[e] + wb[e]));
-      f += (k[e] - k[e]) + (a[e] - a[e]) + (w[e] - w[e]);   // 0 or NaN
+      dec[e] = decay_of(sigmoid_f(w[e] + wb[e]));
+      f += (k[e] - k[e]) + (a[e] - a[e]) + (float)(dec[e] - dec[e]);   // 0 or NaN
       fr += r[e] - r[e];
       lost[e] = in && !(v[e] - v[e] == 0.f);
     }
@@ -93,33 +136,44 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
     for (int e = 0; e < 4; ++e) {
       u[e] = use ? k[e] * inv : 0.f;
       a[e] = use ? a[e] * u[e] : 0.f;
-      if (!use) { w[e] = 1.f; k[e] = 0.f; }
+      if (!use) { dec[e] = 1.0; k[e] = 0.f; }
       if (!use || lost[e]) v[e] = 0.f;
       if (!use || fr != 0.f) r[e] = 0.f;
     }
-    Row<float, 4>::st(&sx[row][ch], w);
+    // the decays of the chunk's earlier and later tokens: of the wave's four rows by row swaps, of the other waves' through LDS
+    double before[4], after[4];
+    const bool odd = row & 1, high = row & 2;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const double next = of_row_16(dec[e], odd), pair = dec[e] * next, other = of_row_32(pair, high);
+      before[e] = (odd ? next : 1.0) * (high ? other : 1.0);
+      after[e] = (odd ? 1.0 : next) * (high ? 1.0 : other);
+      if ((row & 3) == 0) sg[row >> 2][ch + e] = pair * other;
+    }
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (lost[e]) atomicMin(&sv_bad[ch + e], row);
-    f32x4 before = {1.f, 1.f, 1.f, 1.f}, after = before;   // the decays of the chunk's earlier and later tokens
+    const int group = __builtin_amdgcn_readfirstlane(row >> 2);
 #pragma unroll
-    for (int m = 0; m < kC; ++m) {
-      const f32x4 x = ld4(&sx[m][ch]);
-      if (m < row) before *= x;
-      if (m > row) after *= x;
+    for (int m = 0; m < 4; ++m) {
+      if (m == group) continue;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) (m < group ? before : after)[e] *= sg[m][ch + e];
     }
     f32x4 ka, kk, upto, U, R, A, K, V;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      upto[e] = before[e] * w[e];
-      U[e] = u[e] * before[e];
-      R[e] = r[e] * upto[e];
-      A[e] = a[e] / upto[e];
-      K[e] = k[e] / upto[e];
+    for (int e = 0; e < 4; ++e) {   // each rounded once
+      const double d = before[e] * dec[e], seed = (double)__builtin_amdgcn_rcpf((float)d);
+      const double inv = seed * __builtin_fma(-d, seed, 2.0);
+      upto[e] = (float)d;
+      U[e] = (float)(u[e] * before[e]);
+      R[e] = (float)(r[e] * d);
+      A[e] = (float)(a[e] * inv);
+      K[e] = (float)(k[e] * inv);
       V[e] = v[e];
-      ka[e] = a[e] * after[e];
-      kk[e] = k[e] * after[e];
+      ka[e] = (float)(a[e] * after[e]);
+      kk[e] = (float)(k[e] * after[e]);
     }
     *reinterpret_cast<f32x4*>(&su[row][ch]) = U;
     *reinterpret_cast<f32x4*>(&sr[row][ch]) = R;
@@ -128,39 +182,52 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
     *reinterpret_cast<f32x4*>(&sv[row][ch]) = V;
     *reinterpret_cast<f32x4*>(out.R + place(row) * kD + ch) = R;
     if (row == kC - 1) *reinterpret_cast<f32x4*>(out.E + ch) = upto;
-    __syncthreads();
     *reinterpret_cast<f32x4*>(&sx[row][ch]) = ka;
     *reinterpret_cast<f32x4*>(&sy[row][ch]) = kk;
+    __syncthreads();
   }
-  if (tid < kC) out.F[place(tid)] = sf[1][tid];   // added to the token's outputs
   if (tid < kD) {
     int first = sv_bad[tid];
-    for (int m = kC - 1; m >= 0; --m)
+    bool any = false;
+    for (int m = kC - 1; m >= 0; --m) {
       if (sf[0][m] != 0.f) first = min(first, m);
+      any |= sf[1][m] != 0.f;
+    }
     out.B[tid] = (float)first;
+    any = __any(any || first < kC);
+    if (tid < kC) out.F[tid] = sf[1][tid];
+    if (tid == 0) *out.any = any ? 1.f : 0.f;
   }
-  // all pairs of tokens: wave 0 A, 1 B, 2 Pa, 3 Pk; lane (c, g) gets rows 4 g + r of column c
+  // all pairs of tokens: wave 0 A, 1 B in four chains, 2 Pa, 3 Pk in 64 bits (in 32, the outputs' largest error; A and B in 64
+  // bits too: 18 us more and no smaller an error); lane (c, g) gets rows 4 g + r of column c, in 64 bits rows 4 r + g
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
   {
     const float(*x)[kLd] = wave < 2 ? su : sr;
     const float(*y)[kLd] = wave & 1 ? sk : sa;
-    f32x4 d = {0.f, 0.f, 0.f, 0.f}, d2 = d;
+    f32x4 xa[4], ya[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const f32x4 a = ld4(&x[c][16 * q + 4 * g]), b = ld4(&y[c][16 * q + 4 * g]);
-#pragma unroll
-      for (int e = 0; e < 4; e += 2) {
-        d = mfma(a[e], b[e], d);
-        d2 = mfma(a[e + 1], b[e + 1], d2);
-      }
+      xa[q] = ld4(&x[c][16 * q + 4 * g]);
+      ya[q] = ld4(&y[c][16 * q + 4 * g]);
     }
+    if (wave < 2) {
+      f32x4 d[4] = {};
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 4 * g + r;
-      const float x = wave < 2 ? (c < i ? d[r] + d2[r] : 0.f) : (c <= i ? d[r] + d2[r] : 0.f);
-      if (wave == 0) sA[i][c] = x;
-      else if (wave == 1) sB[i][c] = x;
-      else (wave == 2 ? out.Pa : out.Pk)[64 * (c >> 2) + 16 * (c & 3) + place(i)] = x;   // by k step and lane of the scan
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[e] = mfma(xa[q][e], ya[q][e], d[e]);
+      const f32x4 t = (d[0] + d[1]) + (d[2] + d[3]);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) (wave == 0 ? sA : sB)[4 * g + r][c] = c < 4 * g + r ? t[r] : 0.f;
+    } else {
+      f64x4 d = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d = __builtin_amdgcn_mfma_f64_16x16x4f64((double)xa[q][e], (double)ya[q][e], d, 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)   // by k step and lane of the scan
+        (wave == 2 ? out.Pa : out.Pk)[64 * (c >> 2) + 16 * (c & 3) + place(4 * r + g)] = c <= 4 * r + g ? (float)d[r] : 0.f;
     }
   }
   __syncthreads();
@@ -233,45 +300,39 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
   // (past the end the last chunk again, rows that do not exist behind o), so that the wait for an operand never covers the
   // younger loads behind it.
   struct Ops {
-    f32x4 W, R, KA, KK, E, X, F;
-    float pa, pk, B[kTiles];
+    f32x4 W, R, KA, KK, E, X;
+    float pa, pk, any;
   } ops[kAhead];
   constexpr unsigned kM = kC * kD * sizeof(float);   // bytes of an operand of the buffer
-  const unsigned rows = (c * kD + k0 + 4 * g) * 4, cols = ((k0 + c) * kC + 4 * g) * 4, states = (k0 + 4 * g) * 4, toks = 4 * g * 4,
+  const unsigned rows = (c * kD + k0 + 4 * g) * 4, cols = ((k0 + c) * kC + 4 * g) * 4, states = (k0 + 4 * g) * 4,
                  vals_at = (4 + half) * kM + ((col0 + 16 * mine + c) * kC + 4 * g) * 4, pair = (64 * wave + lane) * 4;
   auto fetch = [&](Ops& x, int ci) {
     const char* p = reinterpret_cast<const char*>(base + ((long)(first + min(ci, nc - 1)) * heads + h) * kBuf);
     auto get = [&](unsigned at) { return *reinterpret_cast<const f32x4*>(p + at); };
     auto one = [&](unsigned at) { return *reinterpret_cast<const float*>(p + at); };
-    constexpr unsigned kE = 6 * kM, kP = kE + kD * 4, kF = kP + 2 * kC * kC * 4, kB = kF + kC * 4;
+    constexpr unsigned kE = 6 * kM, kP = kE + kD * 4, kAny = kP + (2 * kC * kC + kC + kD) * 4;
     x.W = get(rows);
     x.R = get(kM + rows);
     x.X = get(vals_at);
-    x.F = get(kF + toks);
     x.KK = get(3 * kM + cols);
     x.KA = get(2 * kM + cols);
     x.E = get(kE + states);
     x.pa = one(kP + pair);
     x.pk = one(kP + kC * kC * 4 + pair);
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) x.B[t] = one(kB + (col0 + 16 * t + c) * 4);
+    x.any = one(kAny);
   };
   auto of_wave = [&](const f32x4& v) { return high ? (odd ? v[3] : v[2]) : odd ? v[1] : v[0]; };
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 os[kTiles] = {};
-  float bad[kTiles] = {};   // NaN once a token's inputs were not finite
-  const float nan = __builtin_nanf("");
+  float any = 0.f;   // 1 once a token's inputs were not finite
   float* po = o + (long)(r0 + 8 * half + g) * N + h * kD + col0 + 16 * mine + c;
   float* nowhere = o + pad + lane;
   // the outputs of chunk ci from the sums in sums[buf]: wave w two rows of tile w % 2
   auto read_out = [&](int ci, int buf) {
-    float y[2] = {0.f, 0.f};
+    float2 v[kNW];
 #pragma unroll
-    for (int w = 0; w < kNW; ++w) {
-      const float2 v = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(&sums[buf][1][mine][w][lane]) + 2 * half);
-      y[0] += v.x;
-      y[1] += v.y;
-    }
+    for (int w = 0; w < kNW; ++w) v[w] = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(&sums[buf][1][mine][w][lane]) + 2 * half);
+    const float y[2] = {(v[0].x + v[1].x) + (v[2].x + v[3].x), (v[0].y + v[1].y) + (v[2].y + v[3].y)};
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const int i = ci * kC + 8 * half + 4 * e + g;
@@ -281,12 +342,10 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
   };
   auto step = [&](Ops& x, int ci) {
     const int buf = ci & 1;
-    f32x4 us[kTiles], u[kTiles], v[kTiles], rs[kTiles];
+    f32x4 us[kTiles], u[kTiles], v[kTiles], rs[kTiles] = {};
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) {
       us[t] = !high && odd == t ? x.X : zero;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) rs[t][r] = !high && !odd ? x.F[r] + (x.B[t] <= 4 * r + g ? nan : bad[t]) : 0.f;
       sums[buf][1][t][wave][lane] = os[t];
     }
     vals[buf][wave][lane] = x.X;
@@ -323,11 +382,10 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
     for (int t = 0; t < kTiles; ++t) st[t] += sa[t];
 #pragma unroll
     for (int t = 0; t < kTiles; ++t) {
-      os[t] = mfma(x.pk, of_wave(v[t]), rs[t]);
-      os[t] = mfma(x.pa, of_wave(u[t]), os[t]);
+      os[t] = mfma(x.pa, of_wave(u[t]), rs[t]);   // the larger part last: its roundings are the outputs'
+      os[t] = mfma(x.pk, of_wave(v[t]), os[t]);
     }
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) bad[t] = x.B[t] < kC ? nan : bad[t];
+    any = fmaxf(any, x.any);
     fetch(x, ci + kAhead);
     read_out(ci - 1, buf);
   };
@@ -349,7 +407,21 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
 #pragma unroll
   for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) Sp[(long)(k0 + 4 * g + r) * kD + 16 * t] = st[t][r] + bad[t];
+    for (int r = 0; r < 4; ++r) Sp[(long)(k0 + 4 * g + r) * kD + 16 * t] = st[t][r];
+  if (any == 0.f) return;
+  __syncthreads();   // the outputs and the state are written
+  const float nan = __builtin_nanf("");
+  const int tid = threadIdx.x, col = col0 + tid % (16 * kTiles), part = tid / (16 * kTiles), parts = 64 * kNW / (16 * kTiles);
+  bool lost = false;
+  for (int ci = 0; ci < nc; ++ci) {
+    const Buf b = buf_of(base, (long)(first + ci) * heads + h);
+    const float from = b.B[col];
+    for (int i = part; i < min(kC, n - ci * kC); i += parts)
+      if (lost || i >= from || b.F[i] != 0.f) o[(long)(r0 + ci * kC + i) * N + h * kD + col] = nan;
+    lost |= from < kC;
+  }
+  if (lost)
+    for (int k = part; k < kD; k += parts) S[((long)seq_state[s] * heads + h) * kD * kD + (long)k * kD + col] = nan;
 }
 
 }  // namespace

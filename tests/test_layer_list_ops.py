@@ -474,6 +474,35 @@ def test_delta_rule_chunks(lens):
 
 
 @gpu
+@pytest.mark.parametrize("T,decay,carried", [(32, 0.6, False), (100, 0.6, True), (400, 2.0, False), (300, 0.2, True)])
+def test_delta_rule_chunks_are_as_precise(T, decay, carried):
+    """The chunks' states and outputs are no further from 64 bits than the token by token ones."""
+    g = torch.Generator().manual_seed(T)
+    H, d = 16, 64
+    N = H * d
+    proj, wl = torch.randn(T, 5 * N, generator=g).bfloat16().cuda(), (torch.randn(T, N, generator=g) * decay).cuda()
+    a_b, w0, nw = (torch.randn(N, generator=g).cuda() for _ in range(3))
+    S0 = (torch.randn(1, H, d, d, generator=g) * carried).cuda()
+    r, k, v, a = (proj[:, i * N:(i + 1) * N].double().view(T, H, d) for i in range(4))
+    w = torch.exp(-0.6065306597126334 * torch.sigmoid(wl.double() + w0.double())).view(T, H, d)
+    u = k * torch.rsqrt(k.square().sum(-1, keepdim=True) + 1e-6)
+    au = torch.sigmoid(a + a_b.double().view(H, d)) * u
+    S, o = S0[0].double(), torch.empty(T, H, d, dtype=torch.float64, device="cuda")
+    for t in range(T):
+        S = S * w[t][..., None] - au[t][..., None] * (u[t][..., None] * S).sum(1, keepdim=True) + k[t][..., None] * v[t][:, None]
+        o[t] = (r[t][..., None] * S).sum(1)
+    delta = get_ops("cuda")._delta
+    cu, ctx, slot = torch.tensor([0, T]).int().cuda(), torch.tensor([T + carried]).int().cuda(), torch.zeros(1).int().cuda()
+    errs = []
+    for floats in (0, delta.delta_rule_chunk_floats(proj, 1, H, d)):
+        out, state, scratch = torch.empty(T, N, dtype=torch.bfloat16, device="cuda"), S0.clone(), torch.empty(7 * T * N + 64, device="cuda")
+        delta.delta_rule(out, state, proj, wl, a_b, w0, nw, cu, ctx, slot, scratch, H, d, 1e-6, 1.0, torch.empty(floats, device="cuda") if floats else None)
+        raw = (scratch[:T * N] if floats else scratch[6 * T * N:7 * T * N]).view(T, H, d)   # the outputs before their norm
+        errs.append([((x.double() - y).norm() / y.norm()).item() for x, y in ((state[0], S), (raw, o))])
+    assert errs[1][0] <= errs[0][0] and errs[1][1] <= errs[0][1], errs
+
+
+@gpu
 @pytest.mark.parametrize("what,value", [("a", "inf"), ("a", "-inf"), ("w", "inf"), ("w", "-inf"), ("a", "nan"), ("w", "nan"), ("k", "nan"), ("k", "inf"),
                                         ("r", "nan"), ("r", "-inf"), ("v", "nan"), ("v", "inf")])
 @pytest.mark.parametrize("row", [16, 21, 38])   # a chunk's first row, one inside, one in the last chunk (the next row spreads a NaN over the state's rows)
