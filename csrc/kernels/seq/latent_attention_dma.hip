@@ -16,11 +16,13 @@
 //     holds the other's registers (queries 72, outputs 128 per lane), and a tile costs one barrier;
 //   * the queries' rotary part is rotated when the operands are loaded (its halves meet in one lane), no pass of its own.
 //   * maxima are taken of the raw products, sums come from a product with ones, and the accumulators (128 per lane) are
-//     rescaled only when a maximum grows by more than kSlack.
-// 8192 rows (4 prompts) x 16 heads, 512 + 64 dims, window 1024: 980 -> 341 us (660 TFLOP/s; 690 k cycles, of which a SIMD's matrix
-// unit is busy 220 k, the vector unit 125 k, the LDS 180 k; the rest waits for operands and at the one barrier per tile).
-// On the way, in one run: 449 with eight-way swizzles (operand rows met two to a bank) and a rescaling per tile; 386 with
-// the rescaling mended. Without overlap of the scores with the next tile's operand reads a fifth more.
+//     rescaled only where a row's maximum grows. (Not rarer: the largest weight is 1 then, which bf16 holds exactly. A maximum that
+//     follows only when a score is larger by 2^8 saves 20 us below, and the outputs' error against 64 bits grows by up to
+//     a tenth, 1.81e-3 -> 1.98e-3 with their own rounding.)
+// 8192 rows (4 prompts) x 16 heads, 512 + 64 dims, window 1024: 980 -> 363 us (620 TFLOP/s). Without the rescaling (341 us, 690 k
+// cycles) a SIMD's matrix unit is busy 220 k cycles, the vector unit 125 k, the LDS 180 k; the rest waits for operands and at
+// the one barrier per tile. Eight-way swizzles (operand rows met two to a bank) took 45 us more, scores without the next tile's
+// operand reads beside them a fifth more.
 // latent_dma_decode_kernel serves decode rows: a workgroup takes 16 heads of one row and a run of keys, 64 of them
 // at a time; its waves split the keys for S and the latent dims for P . V. One row of 724 keys, 16 heads: 46 -> 10 us.
 #include "lds_copy.h"
@@ -264,7 +266,7 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, v[e]);
       mx = max_of_rows(mx) * scale2;
       float al = 1.f;
-      if (__any(mx > m_run + kSlack)) {
+      if (__any(mx > m_run)) {
         const float mn = fmaxf(m_run, mx);
         al = mn > -INFINITY ? __builtin_amdgcn_exp2f(m_run - mn) : 1.f;  // m_run = -inf: 0
         m_run = mn;
@@ -318,7 +320,7 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
 #pragma unroll
     for (int j = 0; j < NPW; ++j) va[j] = KT::value_operand(kt, at, 0, j);
     __builtin_amdgcn_sched_barrier(0);
-    if (__any(rescale)) {   // rarely: kSlack
+    if (__any(rescale)) {
 #pragma unroll
       for (int j = 0; j < NPW; ++j)
 #pragma unroll

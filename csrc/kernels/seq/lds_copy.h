@@ -53,10 +53,6 @@ template <int N> HS_DEVICE void barrier_copies() {
   asm volatile("" ::: "memory");
 }
 
-// A row's softmax weights are relative to a running maximum that follows only when a score is larger by 2^kSlack: most tiles
-// need no rescaling then, and bf16 weights up to 256 are as precise as weights up to 1.
-constexpr float kSlack = 8.f;
-
 HS_DEVICE unsigned pack2(float a, float b) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   typedef float f32x2 __attribute__((ext_vector_type(2)));

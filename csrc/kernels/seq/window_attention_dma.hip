@@ -8,12 +8,14 @@
 //   * the V^T operand comes from ds_read_tr16_b64 (latent_attention_dma.hip says how), so a tile needs one barrier;
 //   * softmax costs the vector unit little more than an fma, an exponential and half a conversion per score: maxima are taken
 //     of the raw products and go round by row swaps, sums come from a product with ones, and the accumulators are rescaled
-//     only when a maximum grows by more than kSlack;
+//     only where a row's maximum grows. (Not rarer: the largest weight is 1 then, which bf16 holds exactly. A maximum that follows
+//     only when a score is larger by 2^8 saves 8 us below, and the outputs' error against 64 bits grows by up to a tenth, 1.80e-3 ->
+//     1.97e-3 with their own rounding);
 //   * the workgroups of one key / value head follow each other on the same XCD, whose L2 holds its rows, and the late
 //     tokens of the step, which see the most keys, go first.
-// 8192 rows (4 prompts) x 16 heads over 4 of 128, window 1024: 185 -> 104 us (495 TFLOP/s). Of the latter the vector unit is busy
-// 40 %, the matrix cores 27 %; waves wait at the barrier and for operands a third of their time, and a fifth of the wave
-// slots is empty at the ends. On the way: 152 with a branch per score for the score cap, 124 with the softmax of
+// 8192 rows (4 prompts) x 16 heads over 4 of 128, window 1024: 185 -> 110 us (470 TFLOP/s). Without the rescaling (104 us) the vector
+// unit is busy 40 % of the time, the matrix cores 27 %; waves wait at the barrier and for operands a third of their time, and a
+// fifth of the wave slots is empty at the ends. On the way, without it: 152 with a branch per score for the score cap, 124 with the softmax of
 // window_attention_mfma.hip, 110 with row-wise operands two to a bank, 107 with tests of LDS pointers at each copy; three
 // workgroups per CU (three buffers, 168 registers) spill: 131.
 #include "lds_copy.h"
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(kThreads, 2) void window_dma_prefill_kernel(
 #pragma unroll
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, v[e]);
       mx = max_of_rows(mx) * unit;
-      if (__any(mx > m_run[mt] + kSlack)) {
+      if (__any(mx > m_run[mt])) {
         const float mn = fmaxf(m_run[mt], mx), al = mn > -INFINITY ? __builtin_amdgcn_exp2f(m_run[mt] - mn) : 1.f;
         m_run[mt] = mn;
         lsum[mt] *= al;

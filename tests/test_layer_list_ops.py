@@ -281,6 +281,71 @@ def test_latent_attention_dma(kv, heads, window, lens, ctxs, nd):
     assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
 
 
+def tiled_softmax(sc, v, sink=False, tile=32):
+    """softmax(sc) . v as the matrix-core kernels do it, in 64 bits but for bf16 weights relative to the maximum so far."""
+    m = torch.full((sc.shape[0], 1), 0.0 if sink else -float("inf"), dtype=torch.float64)
+    l, acc = torch.full_like(m, float(sink)), torch.zeros(sc.shape[0], v.shape[1], dtype=torch.float64)
+    for j in range(0, sc.shape[1], tile):
+        s = sc[:, j:j + tile]
+        mn = torch.maximum(m, s.amax(1, keepdim=True))
+        al = torch.where(mn > -float("inf"), torch.exp(m - mn), 1.0)
+        p = torch.exp(s - torch.where(mn > -float("inf"), mn, 0.0)).bfloat16().double()
+        m, l, acc = mn, l * al + p.sum(1, keepdim=True), acc * al + p @ v[j:j + tile]
+    return acc / l
+
+
+def no_further(got, rounded, want):
+    """The kernel's bf16 outputs are as far from 64 bits as weights relative to the row's maximum make them."""
+    ours, theirs = ((x.double().cpu() - want).norm() / want.norm() for x in (got, rounded.bfloat16()))
+    assert ours <= 1.02 * theirs, (ours, theirs)   # sums in other orders, exponentials: a few of the roundings fall otherwise
+
+
+@gpu
+@pytest.mark.parametrize("kv,size", [(512, 2.0), (128, 1.0), (256, 3.0)])
+def test_latent_attention_prompt_error(kv, size):
+    rot, dim, heads, n, scale = 64, 24, 8, 300, (kv + 64) ** -0.5
+    cache, cu, pos, bt, q_abs, q, proj, meta = latent_case([n], [n], heads, dim, kv, rot, 16, torch.bfloat16, "cuda", kv)
+    q_abs, q = (q_abs.float() * size / 0.3).bfloat16(), (q.float() * size).bfloat16()
+    out = torch.empty(heads, n, kv, dtype=torch.bfloat16, device="cuda")
+    get_ops("cuda").latent_attention(out, q_abs.cuda(), q.cuda(), proj.cuda(), cache.cuda(), meta, torch.zeros(rot // 2, device="cuda"), heads, dim, rot,
+                                     kv, -1, scale, 0)
+    j = torch.arange(n)
+    keys = cache[bt[0, j // 16].long(), j % 16].double()
+    qr = q.double().view(n, heads, dim + rot)[..., dim:]
+    want, rounded = torch.empty(2, heads, n, kv, dtype=torch.float64)
+    for h in range(heads):
+        sc = (q_abs[h, :, :kv].double() @ keys[:, :kv].T + qr[:, h] @ keys[:, kv:].T) * scale
+        sc = sc.masked_fill(j > j[:, None], -float("inf"))
+        want[h], rounded[h] = torch.softmax(sc, -1) @ keys[:, :kv], tiled_softmax(sc, keys[:, :kv])
+    no_further(out, rounded, want)
+
+
+@gpu
+@pytest.mark.parametrize("dim,size,sink", [(128, 1.5, True), (128, 1.0, False), (64, 1.5, True)])
+def test_window_attention_prompt_error(dim, size, sink):
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(dim)
+    heads, kv, n, bs = 8, 2, 300, 16
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=0, reach=0, scale=dim ** -0.5, sink=sink, keep_first=0,
+                         softcap=0.0, channel_gate=False, chunk=0, diff=0.0)
+    pages = -(-n // bs)
+    cache, proj = torch.randn(pages, bs, 2 * kv * dim, generator=g), (torch.randn(n, heads * dim, generator=g) * size).bfloat16()
+    cache[..., :kv * dim] *= size
+    cache = cache.bfloat16()
+    meta = SimpleNamespace(seq_cu=torch.tensor([0, n]).int().cuda(), seq_ctx=torch.tensor([n]).int().cuda(), seq_bt=torch.arange(pages).int().view(1, -1).cuda(),
+                           num_decode=0, num_prefill_tokens=n, max_ctx=n)
+    out = torch.empty(n, heads * dim, dtype=torch.bfloat16, device="cuda")
+    get_ops("cuda").window_attention(out, proj.cuda(), cache.cuda(), meta, sp, -1)
+    rows, j = cache.double().view(-1, 2 * kv, dim)[:n], torch.arange(n)
+    want, rounded = torch.empty(2, n, heads, dim, dtype=torch.float64)
+    for h in range(heads):
+        k, v = rows[:, h // (heads // kv)], rows[:, kv + h // (heads // kv)]
+        sc = (proj[:, h * dim:(h + 1) * dim].double() @ k.T * sp.scale).masked_fill(j > j[:, None], -float("inf"))
+        full = torch.cat([sc, torch.zeros(n, 1, dtype=torch.float64)], 1) if sink else sc
+        want[:, h], rounded[:, h] = torch.softmax(full, -1)[:, :n] @ v, tiled_softmax(sc, v, sink)
+    no_further(out, rounded.view(n, -1), want.view(n, -1))
+
+
 # ------------------------------------------------------------------ minGRU
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
