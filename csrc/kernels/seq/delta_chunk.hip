@@ -220,11 +220,12 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
 }
 
 // NW waves with TPW 16-row state tiles each, NC tiles of 16 value channels per workgroup. What a CU can take in (about 34 KB per us)
-// bounds it, so the operands of the state (W, G q, G_15 / G k) serve two tiles of channels, U0 is loaded by one wave per tile (as
-// the start of its sum) and every wave does its share of the k steps of P U; the outputs are summed with the next
-// chunk's exchange. 8192 rows (4 prompts) x 16 heads of 128 x 128: 216 us, of
-// which the matrix instructions take half; one tile per workgroup with U0 and P in every wave,
-// two chunks ahead and an exit between them: 267 us.
+// bounds it, so the operands of the state (W, G q, G_15 / G k) serve two tiles of channels, U0 is loaded by one wave per tile
+// and every wave does its share of the k steps of P U; the outputs are summed with the next chunk's exchange. 8192 rows (4
+// prompts) x 16 heads of 128 x 128: 219 us, of which the matrix instructions take half; one tile per workgroup with U0 and P in
+// every wave, two chunks ahead and an exit between them: 267 us.
+// W S and P U are summed from 0, and U0 and (G q) S added to the sums: as the start of the sums they would make every product round
+// at their size (512 tokens, mean decay 0.47, against 64 bits: state 6.0e-8, with U0 as the start 1.1e-7; outputs 8.6e-8, 1.4e-7).
 constexpr int kAhead = 4;   // chunks in flight
 template <int TPW, int NW, int NC>
 __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
@@ -286,6 +287,12 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
   float* po = o + (long)(r0 + 4 * g + row0) * nv + h * vdim + v0 + 16 * mine + c;
   float* nowhere = o + pad + lane;
   const unsigned rows = v0 + 16 * mine + c < vdim ? n : 0;
+  // sum of the waves' parts, pairs first
+  auto sum_of = [&](const f32x4* p) {
+    if constexpr (NW == 1) return p[0];
+    else if constexpr (NW == 2) return p[0] + p[64];
+    else return (p[0] + p[64]) + (p[128] + p[192]);
+  };
   auto read_out = [&](int ci, int buf) {   // the outputs of chunk ci from the sums in sums[buf]
 #pragma unroll
     for (int e = 0; e < RPW; ++e) {
@@ -301,8 +308,7 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
     f32x4 us[NC], qs[NC], u[NC];
 #pragma unroll
     for (int t = 0; t < NC; ++t) {
-      us[t] = NC == 1 || (!high && odd == t) ? x.U : zero;
-      qs[t] = zero;
+      us[t] = qs[t] = zero;
       sums[buf][1][t][wave][lane] = os[t];
     }
 #pragma unroll
@@ -316,16 +322,14 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
         }
 #pragma unroll
     for (int t = 0; t < NC; ++t) {
-      sums[buf][0][t][wave][lane] = us[t];
+      sums[buf][0][t][wave][lane] = us[t] + (NC == 1 || (!high && odd == t) ? x.U : zero);
 #pragma unroll
       for (int b = 0; b < TPW; ++b) st[t][b] *= x.E[b];
     }
     __syncthreads();   // the other parity's rows are read before a wave comes here again
 #pragma unroll
     for (int t = 0; t < NC; ++t) {
-      u[t] = sums[buf][0][t][0][lane];
-#pragma unroll
-      for (int w = 1; w < NW; ++w) u[t] += sums[buf][0][t][w][lane];
+      u[t] = sum_of(&sums[buf][0][t][0][lane]);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -335,9 +339,10 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
         for (int t = 0; t < NC; ++t) st[t][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.K[b][r], u[t][r], st[t][b], 0, 0, 0);
 #pragma unroll
     for (int t = 0; t < NC; ++t) {
-      os[t] = qs[t];
+      os[t] = zero;
 #pragma unroll
       for (int i = 0; i < KPW; ++i) os[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[i], step_of(u[t], i), os[t], 0, 0, 0);
+      os[t] += qs[t];
     }
     fetch(x, ci + kAhead);
     read_out(ci - 1, buf);
