@@ -184,9 +184,10 @@ __global__ __launch_bounds__(512) void attn_prepare_vec_kernel(
     const int it = tid + n * nt;
     // mode 3: the rotated pairs count as they will be
     const float grow = norm_mode == 3 && it < nqk && (it & (per - 1)) < rot ? amp : 1.f;
-    float v = 0.f;
+    float v4[4] = {};   // four chains: a single one rounds 16 times at nearly the sum's size
 #pragma unroll
-    for (int e = 0; e < 16; ++e) { const float w = x[n][e] * grow; v += w * w; }
+    for (int e = 0; e < 16; ++e) { const float w = x[n][e] * grow; v4[e & 3] += w * w; }
+    const float v = (v4[0] + v4[1]) + (v4[2] + v4[3]);
     ss[n] = v;
     if (it < heads * per) a += v; else if (it < nqk) b += v;
   }

@@ -446,6 +446,25 @@ def test_attn_prepare(heads, kv, maps, dim, vdim, nfreq, mode, v_norm, own, dtyp
         assert ((got - want).abs() <= tol * want.abs() + (2.0 ** -9 if nfreq else 2.0 ** -20) * want.abs().max()).all()
 
 
+@gpu
+def test_attn_prepare_norm_error():
+    """How far the heads' norms are from 64 bits: their mean relative error over a head, in which its elements' own roundings cancel."""
+    from types import SimpleNamespace
+    heads, kv, dim, T = 16, 4, 128, 2000
+    proj = torch.randn(T, (heads + 2 * kv) * dim, generator=torch.Generator().manual_seed(3))
+    sp = SimpleNamespace(q_size=heads * dim, k_size=kv * dim, v_size=kv * dim, heads=heads, kv_heads=kv, maps=1, dim=dim, vdim=dim, kv_from=None,
+                         qk_norm=False, head_norm=True, unit_qk=False, v_norm=True, temp_coef=0.0, temp_every=0, scaling=None)
+    meta = SimpleNamespace(positions=torch.zeros(T, dtype=torch.long, device="cuda"), slot_mapping=torch.arange(T, device="cuda"))
+    p, cache, one = proj.cuda(), torch.zeros(T, 1, 2 * kv * dim, device="cuda"), torch.ones(dim, device="cuda")
+    get_ops("cuda").attn_prepare(p, cache, meta, torch.empty(0, device="cuda"), sp, one, one, 1e-6)
+    got = torch.cat([p[:, :heads * dim].cpu(), cache.view(T, -1).cpu()], 1).double().view(T, -1, dim)
+    want = proj.double().view(T, -1, dim)
+    want = want * torch.rsqrt(want.square().mean(-1, keepdim=True) + 1e-6)
+    off = (got * want).sum(-1) / want.square().sum(-1) - 1
+    # 4.56e-8 over 48000 heads, nearly all of it from the root and the quotient; a single chain of 16 squares per thread makes it 4.63e-8
+    assert off.square().mean().sqrt() <= 4.6e-8
+
+
 # ------------------------------------------------------------------ window attention of decode rows
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
