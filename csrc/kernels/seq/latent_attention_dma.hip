@@ -146,7 +146,7 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
   const int h0 = blockIdx.y * hc, nh = min(hc, heads - h0);
   const int p_first = ctx - n + tok0, hi = p_first + ntok - 1;
   // tiles start at multiples of 32: a wave's 4 keys (8 of the rotary part) lie on one page, looked up by the scalar unit
-  const int lo = (window > 0 ? max(0, p_first - window + 1) : 0) & ~(kKeys - 1);
+  const int lo0 = window > 0 ? max(0, p_first - window + 1) : 0, lo = lo0 & ~(kKeys - 1);
   const int ntiles = (hi - lo) / kKeys + 1;
   const int* bt = seq_bt + (long)s * bt_width;
   const int mask = (1 << block_shift) - 1;
@@ -319,6 +319,7 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
     }
 #pragma unroll
     for (int j = 0; j < NPW; ++j) va[j] = KT::value_operand(kt, at, 0, j);
+    if (i == 1 && lo < lo0) clear_below(va, lo, lo0, g);
     __builtin_amdgcn_sched_barrier(0);
     if (__any(rescale)) {
 #pragma unroll

@@ -53,6 +53,19 @@ template <int N> HS_DEVICE void barrier_copies() {
   asm volatile("" ::: "memory");
 }
 
+// The parts of a value operand (lane (c, g): keys j0 + 16 (e / 4) + 4 g + e % 4) that belong to keys before `lo`, as zeros: a weight of
+// 0 does not hide an infinity or a NaN.
+template <int N> HS_DEVICE void clear_below(bf16x8 (&va)[N], int j0, int lo, int g) {
+  u32x4 keep;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int j = j0 + 16 * (r >> 1) + 4 * g + 2 * (r & 1);
+    keep[r] = (j >= lo ? 0x0000ffffu : 0u) | (j + 1 >= lo ? 0xffff0000u : 0u);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) va[i] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, va[i]) & keep);
+}
+
 HS_DEVICE unsigned pack2(float a, float b) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   typedef float f32x2 __attribute__((ext_vector_type(2)));

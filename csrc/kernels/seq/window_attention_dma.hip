@@ -55,7 +55,7 @@ __global__ __launch_bounds__(kThreads, 2) void window_dma_prefill_kernel(
   const int group = heads / kv_heads, kvh = hy / hchunks, h0 = (hy % hchunks) * hc, nh = min(hc, group - h0);
   const int r0 = seq_cu[s], n = seq_cu[s + 1] - r0, ctx = seq_ctx[s], ntok = min(tq, n - tok0);
   const int p_first = ctx - n + tok0, hi = p_first + ntok - 1;
-  const int lo = first_key(p_first, window, chunk) & ~(kKeys - 1), ntiles = (hi - lo) / kKeys + 1;
+  const int lo0 = first_key(p_first, window, chunk), lo = lo0 & ~(kKeys - 1), ntiles = (hi - lo) / kKeys + 1;
   const long Dc = 2L * kv_heads * D;
   const int* bt = seq_bt + (long)s * bt_width;
   const int mask = (1 << block_shift) - 1;
@@ -167,6 +167,7 @@ __global__ __launch_bounds__(kThreads, 2) void window_dma_prefill_kernel(
       for (int i2 = 0; i2 < 2; ++i2) h[i2] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(tile + vat[j] + 16 * i2 * kRow));
       va[j] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(h[0], h[1], 0, 1, 2, 3, 4, 5, 6, 7));
     }
+    if (i == 0 && lo < lo0) clear_below(va, lo, lo0, g);
     __builtin_amdgcn_sched_barrier(0);
     bf16x8 pb[MT];
 #pragma unroll

@@ -281,6 +281,23 @@ def test_latent_attention_dma(kv, heads, window, lens, ctxs, nd):
     assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
 
 
+@gpu
+@pytest.mark.parametrize("kv", [128, 512])
+@pytest.mark.parametrize("n,ctx,window", [(3, 100, 40), (4, 64, 33), (2, 200, 64)])
+def test_latent_attention_hidden_keys(kv, n, ctx, window):
+    """Keys before the first row's window, which no row sees, may hold anything."""
+    heads, dim, rot = 8, 24, 64
+    cache, cu, pos, bt, q_abs, q, proj, meta = latent_case([n], [ctx], heads, dim, kv, rot, 16, torch.bfloat16, "cuda", ctx, 0)
+    j = torch.arange(ctx - n - window + 1)
+    outs = []
+    for value in (0.0, float("nan"), float("inf")):
+        cache[bt[0, j // 16].long(), j % 16] = value
+        outs.append(torch.empty(heads, n, kv, dtype=torch.bfloat16, device="cuda"))
+        get_ops("cuda").latent_attention(outs[-1], q_abs.cuda(), q.cuda(), proj.cuda(), cache.cuda(), meta, torch.zeros(rot // 2, device="cuda"), heads, dim,
+                                         rot, kv, -1, 0.1, window)
+    assert outs[0].isfinite().all() and torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
+
+
 def tiled_softmax(sc, v, sink=False, tile=32):
     """softmax(sc) . v as the matrix-core kernels do it, in 64 bits but for bf16 weights relative to the maximum so far."""
     m = torch.full((sc.shape[0], 1), 0.0 if sink else -float("inf"), dtype=torch.float64)
@@ -771,3 +788,25 @@ def test_latent_prepare(q_rank, kv_rank, rot, nfreq, dtype):
     tol = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -18
     assert ((q.cpu().float() - cq.float()).abs() <= tol * cq.float().abs() + 2.0 ** -20).all()
     assert ((c.cpu().float() - cache.float()).abs() <= tol * cache.float().abs() + 2.0 ** -10 * 4.5).all()
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("dim,n,ctx,window,chunk", [(128, 10, 100, 40, 0), (64, 20, 64, 33, 0), (128, 30, 200, 64, 0), (64, 5, 90, 0, 50)])
+def test_window_attention_hidden_keys(dim, n, ctx, window, chunk, dtype):
+    """Keys before the first row's window or chunk, which no row sees, may hold anything."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(ctx)
+    heads, kv, bs = 4, 2, 16
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=window, reach=window or chunk, scale=dim ** -0.5, sink=True, keep_first=0,
+                         softcap=0.0, channel_gate=False, chunk=chunk, diff=0.0)
+    pages = -(-ctx // bs)
+    cache, proj = torch.randn(pages * bs, 2 * kv * dim, generator=g).to(dtype), torch.randn(n, heads * dim, generator=g).to(dtype).cuda()
+    meta = SimpleNamespace(seq_cu=torch.tensor([0, n]).int().cuda(), seq_ctx=torch.tensor([ctx]).int().cuda(), seq_bt=torch.arange(pages).int().view(1, -1).cuda(),
+                           num_decode=0, num_prefill_tokens=n, max_ctx=ctx)
+    outs = []
+    for value in (0.0, float("nan"), -float("inf")):
+        cache[:(ctx - n) // chunk * chunk if chunk else ctx - n - window + 1] = value
+        outs.append(torch.empty(n, heads * dim, dtype=dtype, device="cuda"))
+        get_ops("cuda").window_attention(outs[-1], proj, cache.view(pages, bs, -1).cuda(), meta, sp, -1)
+    assert outs[0].isfinite().all() and torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
