@@ -79,6 +79,9 @@ void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, cons
                         int ntiles_cap, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
                         float limit, int pairs, bool f32, hipStream_t s);
 
+// Whether tiles of 32 slots that hold so many pairs run the kernel for few rows per tile.
+bool expert_gemm_skinny(long pairs, long ntiles_cap, long N, long K, long E, bool glu);
+
 // Norms before and after a sublayer (sandwich.hip): residual[T, H] (fp32, in place; `table` [vocab, H] in the activation
 // type: it starts as table_scale * table[ids[t]]) += mult * y / rms(y) * w_post; out = residual / rms(residual) * w_next.
 // y: rows `a` (b null); a_scale a / rms(a) * a_w + b_scale b / rms(b) * b_w; or (a null, ye not) a mixture's output

@@ -94,6 +94,10 @@ inline void expert_gemm(at::Tensor& out, const at::Tensor& x, const at::Tensor& 
                                c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
 }
 
+inline bool expert_gemm_skinny(int64_t pairs, int64_t ntiles_cap, int64_t N, int64_t K, int64_t E, bool glu) {
+  return hipserve::expert_gemm_skinny(pairs, ntiles_cap, N, K, E, glu);
+}
+
 // out = act(x . w^T + bias) of at most 64 rows: x [M, K] or [B, M, K], w [N, K] or [B, N, K], out [M, N'] or [B, M, N'].
 inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias,
                           int64_t act, double c0, double c1) {
@@ -128,6 +132,7 @@ inline void def_moe_ops(torch::Library& m) {
   m.def("moe_align_small(int npairs) -> bool", &moe_align_small);
   m.def("expert_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor slots, Tensor tile_expert, int tile, int gather_k, "
         "int act, Tensor? row_scale=None, float limit=0.0, int pairs=0) -> ()");
+  m.def("expert_gemm_skinny(int pairs, int ntiles_cap, int N, int K, int E, bool glu) -> bool", &expert_gemm_skinny);
 }
 
 inline void impl_moe_ops(torch::Library& m) {

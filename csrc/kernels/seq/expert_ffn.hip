@@ -9,6 +9,7 @@
 // computes a [32 slots x 64 columns] block, x and W staged through LDS in K-chunks of 32, fp32
 // accumulation; bf16 and fp32 element types.
 #include <algorithm>
+#include <cmath>
 
 #include "skinny.h"
 #include "hipserve/seq_kernels.h"
@@ -248,19 +249,21 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
   }
 }
 
-// Which of the two kernels serves tiles of 32 slots; cold weights, us with the launch: expert_gemm_mfma takes 10 + 0.95 per
-// step of 128 k (its steps wait for their loads) while its workgroups of 128 columns are at most 512; expert_gemm_skinny
-// 5.2 plus the weights at 5 TB/s, or what its workgroups of 16 columns read at 34 KB per us and CU. 2 of 16 experts of
-// 2048 -> 1024 -> 2048: 2 pairs 23 -> 7.2 us (up) and 18 -> 5.5 (down), 96 pairs on all 16 experts 26 -> 21 (up); 1400
-// pairs stay on the tile kernel (26 against 87 expected).
-bool skinny_tiles(int pairs, int N, int K, int E, bool glu) {
-  const double used = std::min(E, pairs), tiles = used + pairs / 32, rows = std::min(32.0, pairs / used);
-  const double wgs = std::max(1.0, tiles * N / 16 / 256);
-  const double ours = 5.2 + std::max(used * N * K * 2 / 5.0e6, wgs * 2 * K * (16 + rows / (glu ? 2 : 1)) / 34e3);
-  return ours < (10 + 0.95 * K / 128) * std::max(1.0, tiles * N / 128 / 512);
-}
-
 }  // namespace
+
+// Which of the two kernels serves tiles of 32 slots; cold weights, us with the launch, from 8 to 256 experts, K from 512 to 4096 and up
+// to 512 pairs. expert_gemm_mfma takes 5 + 1.2 per step of 128 k (its steps wait for their loads) while its workgroups of
+// 128 columns are at most 512; expert_gemm_skinny 5.2 plus the weights of the experts that so many pairs hit on average at 5 TB/s,
+// or what its workgroups of 16 columns read at 34 KB per us and CU, plus 0.3 per 1000 workgroups: it has one per 16 columns of every tile
+// of the capacity, nearly all of them empty where the experts are many. Tile kernel / this one: 16 experts, 1024 x 2048: 2 pairs 19.9 / 7.0, 64
+// pairs 26.3 / 20.9; 2048 x 1024: 2 pairs 12.8 / 5.5, 64 pairs 18.1 / 20.9; 128 experts, 1536 x 2048, gated: 8 pairs 25.1 / 14.8; 2048 x 768:
+// 8 pairs 11.8 / 13.3, 64 pairs 36.9 / 50.6; 256 experts, 2048 x 512: 8 pairs 9.4 / 19.1, 512 pairs 94 / 166; 512 x 512: 64 pairs 10.1 / 12.4.
+bool expert_gemm_skinny(long pairs, long ntiles_cap, long N, long K, long E, bool glu) {
+  const double used = E * (1 - std::pow(1 - 1.0 / E, (double)pairs)), tiles = used + pairs / 32, rows = std::min(32.0, pairs / used);
+  const double wgs = std::max(1.0, tiles * N / 16 / 256), launched = (double)((glu ? N / 2 : N) + 15) / 16 * ntiles_cap;
+  const double ours = 5.2 + std::max(used * N * K * 2 / 5.0e6, wgs * 2 * K * (16 + rows / (glu ? 2 : 1)) / 34e3) + 0.3e-3 * launched;
+  return ours < (5 + 1.2 * K / 128) * std::max(1.0, tiles * N / 128 / 512);
+}
 
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,
                         int ntiles_cap, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
@@ -273,7 +276,7 @@ void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, cons
     dim3 mg(act >= 2 ? (No + 63) / 64 : (N + 127) / 128, ntiles_cap);
     auto o = (unsigned short*)out;
     auto xi = (const unsigned short*)x, wi = (const unsigned short*)w;
-    if (tile == 32 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && skinny_tiles(pairs, N, K, E, act >= 2)) {
+    if (tile == 32 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && expert_gemm_skinny(pairs, ntiles_cap, N, K, E, act >= 2)) {
       const dim3 sg((No + 15) / 16, ntiles_cap);
 #define HS_ES(NT, KU, GLU)                                                                                          \
   expert_gemm_skinny_kernel<NT, KU, GLU><<<sg, kSkThreads, 0, s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K, \

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from hipserve import _build
-from hipserve.ops import library_path
+from hipserve.ops import _SEQ_LIBS, library_path, load_kernel_library
 
 
 @pytest.mark.skipif(not os.path.exists(library_path()), reason="hipserve/_C.so not built")
@@ -40,3 +40,16 @@ def test_copies_into_lds_keep_their_wait_states(name, tmp_path):
         for ln in code[i - 5:i] if base else ():
             wrote = re.match(r"v_(?:readfirstlane|readlane|cmp)\w* s\[?(\d+)(?::(\d+))?", ln)
             assert not wrote or int(wrote[2] or wrote[1]) < int(base[1]) or int(wrote[1]) > int(base[2]), (ln, code[i])
+
+
+@pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
+@pytest.mark.parametrize("experts,N,K,glu,by_pairs", [   # measured: whether the kernel for few rows per tile is the faster one
+    (16, 1024, 2048, False, {2: True, 16: True, 64: True}), (16, 2048, 1024, False, {2: True, 12: True, 64: False}),
+    (8, 2048, 4096, False, {2: True, 64: True}), (8, 4096, 2048, False, {4: True, 16: False, 128: False}), (128, 1536, 2048, True, {8: True}),
+    (128, 2048, 768, False, {8: False, 64: False, 512: False}), (256, 2048, 2048, False, {8: False, 64: False}),
+    (256, 2048, 512, False, {8: False, 64: False, 512: False}), (128, 512, 512, False, {1: True, 16: True, 64: False}), (32, 1024, 512, False, {8: True, 64: False})])
+def test_choice_of_the_expert_kernels(experts, N, K, glu, by_pairs):
+    load_kernel_library("seq")
+    for pairs, skinny in by_pairs.items():
+        cap = -(-(pairs + experts * 31) // 32)   # every expert's last tile partly filled
+        assert torch.ops.hipserve_seq.expert_gemm_skinny(pairs, cap, N, K, experts, glu) == skinny, pairs
