@@ -222,6 +222,8 @@ void delta_rule(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const at
               scratch.numel() >= (chunks.has_value() ? T * N + 64 : T * 7 * N));
   if (chunks.has_value()) {
     CHECK_F32(*chunks);
+    for (const at::Tensor* t : {&wl, &a_b, &w0, &*chunks})
+      TORCH_CHECK(reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 == 0, "delta_rule: chunks read 16 bytes at a time");
     TORCH_CHECK(!f32 && hipserve::delta_rule_chunk_ok(heads, dim, proj.data_ptr(), proj.stride(0)) && T / 16 + nseq <= 65535 &&
                 chunks->numel() >= hipserve::delta_rule_chunk_floats(T, nseq, heads), "delta_rule: not in chunks");
   }

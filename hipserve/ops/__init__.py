@@ -412,12 +412,14 @@ class KernelOps:
                                      *offs, sp.channel_decay, sp.gate_act == "silu")
 
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
-        if meta.max_q == 1 and self._delta.delta_rule_step_ok(sp.dim):   # decode steps: one launch
+        def aligned(*tensors):   # the kernels below read and write 16 bytes at a time
+            return all(t.data_ptr() % 16 == 0 for t in tensors)
+        if meta.max_q == 1 and self._delta.delta_rule_step_ok(sp.dim) and aligned(state[0]):   # decode steps: one launch
             self._delta.delta_rule_step(out, state[0], proj, wl, a_b, w0, norm_w, meta.seq_cu, meta.seq_ctx, meta.seq_state,
                                         sp.heads, sp.dim, eps, out_scale)
             return
         T, n = proj.shape[0], 0
-        if self.DELTA_CHUNK and proj.dtype in self.DELTA_CHUNK_DTYPES and meta.max_q >= self.DELTA_CHUNK_ROWS:
+        if self.DELTA_CHUNK and proj.dtype in self.DELTA_CHUNK_DTYPES and meta.max_q >= self.DELTA_CHUNK_ROWS and aligned(wl, a_b, w0):
             n = self._delta.delta_rule_chunk_floats(proj, meta.seq_ctx.shape[0], sp.heads, sp.dim)   # 0: not for these sizes
         chunks = torch.empty(n, device=proj.device, dtype=torch.float32) if n else None
         scratch = torch.empty(T * sp.size + 64 if n else T * 7 * sp.size, device=proj.device, dtype=torch.float32)

@@ -767,6 +767,31 @@ def test_delta_rule_step(dtype):
     assert ((got.cpu().float() - want.float()).abs() <= tol * want.float().abs() + least * want.float().abs().max()).all()
 
 
+@gpu
+@pytest.mark.parametrize("rows", [1, 40])
+def test_delta_rule_unaligned(rows):
+    """States and 32-bit rows that do not start at 16 bytes take the token by token kernels, as other sizes do."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(rows)
+    H, d, n = 2, 64, 2
+    N, T = H * d, n * rows
+    proj, wl, S = torch.randn(T, 5 * N, generator=g).bfloat16(), torch.randn(T, N, generator=g), torch.randn(n, H, d, d, generator=g)
+    a_b, w0, nw = torch.randn(N, generator=g), torch.randn(N, generator=g), torch.rand(N, generator=g) + 0.5
+    cu, ctx, slots = torch.tensor([0, rows, T]).int(), torch.tensor([rows + 4, rows]).int(), torch.tensor([1, 0]).int()
+    sp = SimpleNamespace(heads=H, dim=d, size=N)
+    meta = SimpleNamespace(seq_cu=cu.cuda(), seq_ctx=ctx.cuda(), seq_state=slots.cuda(), max_q=rows)
+    want_s, want = S.clone(), torch.empty(T, N, dtype=torch.bfloat16)
+    ref.delta_rule(want, want_s, proj, wl, a_b, w0, nw, sp, 1e-5, cu, ctx, slots, 1.0)
+
+    def shifted(t):
+        out = torch.empty(t.numel() + 1, device="cuda")[1:].view(t.shape)
+        return out.copy_(t)
+    got_s, got = shifted(S), torch.empty(T, N, dtype=torch.bfloat16, device="cuda")
+    get_ops("cuda").delta_rule(got, [got_s], proj.cuda(), shifted(wl), shifted(a_b), shifted(w0), nw.cuda(), sp, 1e-5, meta)
+    assert ((got_s.cpu() - want_s).abs() <= 2.0 ** -15 * want_s.abs().max()).all()
+    assert ((got.cpu().float() - want.float()).abs() <= 2.0 ** -7 * want.float().abs() + 2.0 ** -13 * want.float().abs().max()).all()
+
+
 # ------------------------------------------------------------------ latent rows
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
