@@ -131,8 +131,9 @@ class LatentAttention:
         self.kv_norm = None    # [kv_rank] fp32
         self.w_uq = None       # [heads * (dim + rot_dim), q_rank]
         self.w_uk = None       # [heads, dim, kv_rank]
-        self.w_uk_wide = None  # [heads, dim, kv_rank + rot_dim], zero rotary columns (made at first use)
-        self.w_uk_t = None     # [heads, kv_rank, dim] (made at first use)
+        # the same for kernels that take the absorbed queries in place:
+        self.w_uk_wide = None  # [heads, dim, kv_rank + rot_dim], zero rotary columns
+        self.w_uk_t = None     # [heads, kv_rank, dim]
         self.w_uv = None       # [heads, vdim, kv_rank]
         self.w_uv_t = None     # [heads, kv_rank, vdim]
         self.w_o = None        # [hidden, heads * vdim]
@@ -157,9 +158,16 @@ class LatentAttention:
         self.kv_norm = get(prefix + "dkv.norm").to(dev, torch.float32)
         self.w_uq = uq.to(dev, dt).contiguous()
         self.w_uk = get(prefix + "uk").to(dev, dt).view(s.heads, s.dim, s.kv_rank).contiguous()
+        if self.ops.latent_query_in_place(dt, s.kv_rank, s.rot_dim):
+            self._lay_out_queries()
         self.w_uv = get(prefix + "uv").to(dev, dt).view(s.heads, s.vdim, s.kv_rank).contiguous()
         self.w_uv_t = self.w_uv.transpose(1, 2).contiguous()
         self.w_o = get(prefix + "o").to(dev, dt).contiguous()
+
+    def _lay_out_queries(self):
+        """Both layouts of W_uk before the caches are sized, and never inside a capture, where they would hold nothing until its replay."""
+        self.w_uk_wide = F.pad(self.w_uk, (0, self.spec.rot_dim)).contiguous()
+        self.w_uk_t = self.w_uk.transpose(1, 2).contiguous()
 
     def init_random(self, gen, std: float):
         s, H = self.spec, self.hidden
@@ -196,11 +204,9 @@ class LatentAttention:
             # zero weight columns where the attention op puts the rotated part
             q_abs = torch.empty(s.heads, T, s.key_dim, device=h.device, dtype=h.dtype)
             q_heads = qh[:, :, : s.dim].transpose(0, 1)
-            if self.w_uk_t is None:
-                self.w_uk_t = self.w_uk.transpose(1, 2).contiguous()
+            if self.w_uk_t is None:   # loaded while the kernels were switched off
+                self._lay_out_queries()
             if not ops.linear_heads(q_abs[:, :, : s.kv_rank], q_heads, self.w_uk_t):
-                if self.w_uk_wide is None:
-                    self.w_uk_wide = F.pad(self.w_uk, (0, s.rot_dim)).contiguous()
                 torch.bmm(q_heads, self.w_uk_wide, out=q_abs)              # [heads, T, kv_rank + rot_dim]
         else:
             q_abs = _mm32(qh[:, :, : s.dim].transpose(0, 1), self.w_uk)            # [heads, T, kv_rank] fp32

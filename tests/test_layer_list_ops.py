@@ -281,6 +281,20 @@ def test_latent_attention_dma(kv, heads, window, lens, ctxs, nd):
     assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
 
 
+def test_latent_weights_are_laid_out_at_load():
+    from types import SimpleNamespace
+
+    from hipserve.config import LatentAttentionSpec
+    from hipserve.models.mixers import LatentAttention
+    spec = LatentAttentionSpec(heads=2, dim=8, rot_dim=4, vdim=8, q_rank=8, kv_rank=16, scale=0.1)
+    for in_place in (True, False):
+        m = LatentAttention(spec, 32, 1e-6, "cpu", torch.bfloat16, SimpleNamespace(latent_query_in_place=lambda *a: in_place))
+        m.init_random(torch.Generator().manual_seed(0), 0.02)
+        assert (m.w_uk_t is not None) == (m.w_uk_wide is not None) == in_place
+        if in_place:
+            assert torch.equal(m.w_uk_t.transpose(1, 2), m.w_uk) and torch.equal(m.w_uk_wide[..., :16], m.w_uk) and not m.w_uk_wide[..., 16:].any()
+
+
 @gpu
 @pytest.mark.parametrize("kv", [128, 512])
 @pytest.mark.parametrize("n,ctx,window", [(3, 100, 40), (4, 64, 33), (2, 200, 64)])
