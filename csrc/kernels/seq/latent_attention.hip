@@ -150,21 +150,6 @@ constexpr int kMaxCh = 16;    // kv_rank <= kMaxCh * 64
 constexpr int kMaxRows = 16;  // waves per workgroup
 
 // Finds the workgroup's (sequence, first token) among sequences seq0..seq1-1, `tq` tokens per workgroup.
-HS_DEVICE bool find_tile(const int* __restrict__ seq_cu, int seq0, int seq1, int tq, int wg, int& s, int& tok0) {
-  int acc = 0;
-  for (int i = seq0; i < seq1; ++i) {
-    const int n = seq_cu[i + 1] - seq_cu[i];
-    const int nt = (n + tq - 1) / tq;
-    if (wg < acc + nt) {
-      s = i;
-      tok0 = (wg - acc) * tq;
-      return true;
-    }
-    acc += nt;
-  }
-  return false;
-}
-
 template <typename T>
 __global__ __launch_bounds__(64 * kMaxRows) void latent_attention_kernel(
     T* __restrict__ o_lat, const float* __restrict__ q_abs, const T* __restrict__ q, const T* __restrict__ proj,
@@ -180,7 +165,7 @@ __global__ __launch_bounds__(64 * kMaxRows) void latent_attention_kernel(
   float* kc = qs + nrows * Dk;                     // [kKT][kDC + 1]
   float* ps = kc + kKT * (kDC + 1);                // [nrows][kKT]
   int s, tok0;
-  if (!find_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) return;
+  if (!find_row_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r0 = seq_cu[s], n = seq_cu[s + 1] - r0, ctx = seq_ctx[s];
   const int ntok = min(tq, n - tok0);

@@ -55,21 +55,6 @@ __global__ __launch_bounds__(256) void latent_q_cat_kernel(unsigned short* __res
 constexpr int kKeys = 32;   // keys per tile
 constexpr int kPLd = 40;    // P tile row stride (elements): 16-byte aligned rows, padded
 
-HS_DEVICE bool find_tile64(const int* __restrict__ seq_cu, int seq0, int seq1, int tq, int wg, int& s, int& tok0) {
-  int acc = 0;
-  for (int i = seq0; i < seq1; ++i) {
-    const int n = seq_cu[i + 1] - seq_cu[i];
-    const int nt = (n + tq - 1) / tq;
-    if (wg < acc + nt) {
-      s = i;
-      tok0 = (wg - acc) * tq;
-      return true;
-    }
-    acc += nt;
-  }
-  return false;
-}
-
 // K tile row stride: 32 KS + 8 elements (16-byte aligned rows; stride / 2 = 4 (mod 16) dwords keeps both the
 // row-wise 16-byte operand reads of S and the column-wise 2-byte reads of P . V at two-way bank conflicts).
 template <int KS> struct KtLd { static constexpr int v = KS * 32 + 8; };
@@ -95,7 +80,7 @@ __global__ __launch_bounds__(64 * NW, 2) void latent_attention_mfma_kernel(
   int s, tok0;
   // (workgroups are dealt to the XCDs round-robin; giving each XCD a contiguous run of token tiles was
   // measured slower, 1188 vs 1013 us at 8192 tokens x 16 heads: the causal start makes the runs unequal)
-  if (!find_tile64(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) return;
+  if (!find_row_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) return;
   const int Dk = kv_rank + rot_dim;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c = lane & 15, g = lane >> 4;

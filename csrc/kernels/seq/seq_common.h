@@ -86,6 +86,10 @@ HS_DEVICE float sigmoid_f(float x) {
   return x < 0.f ? e * r : r;
 }
 
+HS_DEVICE float tanh_fast(float x) {  // 1 - 2 / (e^2x + 1); saturates cleanly at both ends
+  return 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * 2.88539008177792681f) + 1.f);
+}
+
 // Sum over the 16 lanes of a DPP row; every lane of the row gets it.
 HS_DEVICE float row_sum(float v) {
   v = dpp_step<0xB1, 0xf, false>(v);   // quad_perm [1, 0, 3, 2]

@@ -279,21 +279,6 @@ constexpr int kDC = 64;       // key / value dims per staged chunk
 constexpr int kMaxCh = 8;     // vdim <= kMaxCh * 64
 constexpr int kMaxRows = 16;  // waves per workgroup
 
-HS_DEVICE bool find_row_tile(const int* __restrict__ seq_cu, int seq0, int seq1, int tq, int wg, int& s, int& tok0) {
-  int acc = 0;
-  for (int i = seq0; i < seq1; ++i) {
-    const int n = seq_cu[i + 1] - seq_cu[i];
-    const int nt = (n + tq - 1) / tq;
-    if (wg < acc + nt) {
-      s = i;
-      tok0 = (wg - acc) * tq;
-      return true;
-    }
-    acc += nt;
-  }
-  return false;
-}
-
 // grid.y = kv_heads * hchunks: workgroup y serves query heads g * group + c * hc .. of key/value head g.
 // MAPS = 2: the row's two maps (queries [map 1 | map 2], keys alike) run side by side with their own
 // running (max, sum) and accumulators over the same value chunks; the output is

@@ -26,10 +26,6 @@ namespace {
 constexpr int kMaxRuns = 64;
 constexpr float kLog2e = 1.44269504088896341f;
 
-HS_DEVICE float tanh_fast(float x) {  // 1 - 2 / (e^2x + 1); saturates cleanly at both ends
-  return 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * 2.88539008177792681f) + 1.f);
-}
-
 // Scores and their exponentials: bf16 in the log2 domain; fp32 in the natural one, exp(d) with the rounding error of d log2(e)
 // carried as in sigmoid_f.
 template <typename T> struct Softmax;

@@ -28,10 +28,6 @@ namespace {
 constexpr int kKeys = 32, kStages = 4, kThreads = 256;
 constexpr float kLog2e = 1.44269504088896341f;
 
-HS_DEVICE float tanh_fast(float x) {  // 1 - 2 / (e^2x + 1); saturates cleanly at both ends
-  return 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * 2.88539008177792681f) + 1.f);
-}
-
 // 16-byte chunk ch of key (value) row k sits at chunk ch ^ key_swizzle (value_swizzle) of it: the 16 rows of a key operand use
 // 16 different chunks of 256 bytes, the 8 rows of a transposing read 8 different pairs (rows of 128 bytes: two fill 256).
 template <int D> HS_DEVICE int key_swizzle(int k) { return D == 128 ? k & 15 : k >> 1 & 7; }

@@ -37,28 +37,9 @@ namespace {
 
 constexpr int kKeys = 32;   // keys per tile
 constexpr int kVLd = 40;    // transposed value tile: row stride in elements (32 keys + pad, 16-byte aligned rows)
-HS_DEVICE float tanh_fast(float x) {  // 1 - 2 / (e^2x + 1); saturates cleanly at both ends
-  return 1.f - 2.f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * 2.88539008177792681f) + 1.f);
-}
-
 constexpr int kNW = 4, kRows = 16 * kNW /* x MT */, kThreads = 64 * kNW, kFT = kThreads / kKeys;
 
 template <int KS> struct KLd { static constexpr int v = KS * 32 + 8; };
-
-HS_DEVICE bool find_tile_rows(const int* __restrict__ seq_cu, int seq0, int seq1, int tq, int wg, int& s, int& tok0) {
-  int acc = 0;
-  for (int i = seq0; i < seq1; ++i) {
-    const int n = seq_cu[i + 1] - seq_cu[i];
-    const int nt = (n + tq - 1) / tq;
-    if (wg < acc + nt) {
-      s = i;
-      tok0 = (wg - acc) * tq;
-      return true;
-    }
-    acc += nt;
-  }
-  return false;
-}
 
 // KS: 32-dim steps of a key head (dim <= 32 KS); NV: 16-dim tiles of a value head (vdim <= 16 NV); MT: 16-row
 // tiles per wave (a workgroup owns 64 MT rows; every key / value operand read from LDS feeds MT MFMAs).
@@ -83,7 +64,7 @@ __global__ __launch_bounds__(kThreads, 2) void window_attention_mfma_kernel(
     s = seq0 + blockIdx.x;
     tok0 = 0;
     if (s >= seq1) return;
-  } else if (!find_tile_rows(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) {
+  } else if (!find_row_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0)) {
     return;
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

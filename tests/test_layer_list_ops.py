@@ -251,11 +251,12 @@ def latent_case(lens, ctxs, heads, dim, kv, rot, block, dtype, dev, seed=0, nd=N
 @pytest.mark.parametrize("kv", [128, 256, 512])
 @pytest.mark.parametrize("heads,window", [(16, 0), (5, 100), (70, 33)])
 @pytest.mark.parametrize("lens,ctxs,nd", [([1], [1], 1), ([1, 1, 1], [64, 65, 700], 3), ([37], [37], 0), ([33, 5, 1], [33, 400, 129], 1), ([2, 190], [31, 255], 0),
-                                          ([2, 0], [31, 5], 0), ([1, 0, 1], [64, 9, 700], 0), ([2, 0, 1], [31, 5, 300], 1), ([2, 0], [300, 5], 2)])
+                                          ([2, 0], [31, 5], 0), ([1, 0, 1], [64, 9, 700], 0), ([2, 0, 1], [31, 5, 300], 1), ([2, 0], [300, 5], 2),
+                                          ([1] * 65 + [40] + [2] * 70, [5] * 65 + [60] + [3] * 70, 0), ([2] + [0] * 64 + [1], [9] * 66, 0)])
 def test_latent_attention_dma(kv, heads, window, lens, ctxs, nd):
     """Tiles of 32 and 64 keys filled partly, windows that start inside a tile, rows that leave a workgroup's tiles unused, runs of
-    keys of a decode row (some empty), as many rows as sequences, not one each (with runs too), the rotary part formed in
-    the kernel, in 64 bits."""
+    keys of a decode row (some empty), as many rows as sequences, not one each (with runs too), more sequences than lanes, the rotary
+    part formed in the kernel, in 64 bits."""
     rot, dim, block, gate, scale = 64, 24, 16, 2, 0.11
     cache, cu, pos, bt, q_abs, q, proj, meta = latent_case(lens, ctxs, heads, dim, kv, rot, block, torch.bfloat16, "cuda", kv + heads, nd)
     inv = torch.pow(torch.tensor(1e4), -2.0 * torch.arange(rot // 2) / rot)
@@ -574,9 +575,9 @@ def test_window_attention_decode_rows_of_one_sequence(ctx, dtype):
 
 # ------------------------------------------------------------------ generalized delta rule in chunks
 @gpu
-@pytest.mark.parametrize("lens", [[32], [33, 1, 16], [40, 15, 100]])
+@pytest.mark.parametrize("lens", [[32], [33, 1, 16], [40, 15, 100], [33] + [1] * 70 + [50] + [2] * 65])
 def test_delta_rule_chunks(lens):
-    """Whole and partly filled chunks, carried and fresh states, beside the reference; a row that is not finite poisons itself
+    """Whole and partly filled chunks, more sequences than lanes, carried and fresh states, beside the reference; a row that is not finite poisons itself
     and what follows, not the rows before it."""
     from types import SimpleNamespace
     g = torch.Generator().manual_seed(sum(lens))
@@ -714,11 +715,12 @@ def test_gated_delta_chunks_precision(lens, dim, vdim, a, carried):
     (1, 1, 64, 16, [1, 33], [1, 40], {}), (8, 2, 128, 16, [31, 32, 65], [31, 100, 65], {"window": 40, "sink": True, "gate": True}),
     (5, 1, 64, 64, [130, 7], [300, 7], {"window": 0, "softcap": 3.0, "channel_gate": True}),
     (130, 1, 64, 16, [9], [50], {"window": 20, "sink_w": True}), (4, 4, 128, 128, [200, 3], [210, 203], {"chunk": 64}),
-    (16, 4, 128, 16, [700, 300], [700, 450], {"window": 256, "sink": True}), (2, 1, 128, 8, [40], [64], {"window": 16, "keep_first": 5})])
+    (16, 4, 128, 16, [700, 300], [700, 450], {"window": 256, "sink": True}), (2, 1, 128, 8, [40], [64], {"window": 16, "keep_first": 5}),
+    (4, 2, 64, 16, [1] * 65 + [40] + [2] * 70, [5] * 65 + [60] + [3] * 70, {"window": 30})])
 def test_window_attention_prompts(heads, kv, dim, bs, lens, ctxs, opts, dtype):
     """Tokens, heads and keys that do not fill a tile, windows and chunks that start inside one, pages smaller and larger than a
-    tile, one and two row tiles per wave, more than 128 heads per key / value head, and kept keys, which the other
-    kernel takes in bf16; fp32."""
+    tile, one and two row tiles per wave, more than 128 heads per key / value head, kept keys, which the other
+    kernel takes in bf16, and more sequences than lanes; fp32."""
     from types import SimpleNamespace
     g = torch.Generator().manual_seed(heads * dim + sum(lens))
     n, T, gate = len(lens), sum(lens), opts.get("gate", False) or opts.get("channel_gate", False)
