@@ -459,7 +459,7 @@ class KernelOps:
     def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0):
         """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands. A few rows run the
         weight-streaming kernel with the activation in its epilogue, anything else the vendor's GEMM and a second launch."""
-        if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or bias.dtype == x.dtype):
+        if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())):
             glu = act in self.GLU_ACTS
             T, N, K = x.shape[0], w.shape[0], w.shape[1]
             if self.skinny_pays(T, N, K, glu, x.dtype == torch.float32):

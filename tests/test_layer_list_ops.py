@@ -182,6 +182,17 @@ def test_linear_bias_of_32_bit_results(M, dtype, dev):
     close_to(got, x.double() @ w.double().T + bias.double(), x, w)
 
 
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=gpu)])
+@pytest.mark.parametrize("M", [5, 70])
+@pytest.mark.parametrize("form", ["one number", "every other number"])
+def test_linear_bias_forms(M, form, dev):
+    """A bias that is broadcast or strided is added by either product."""
+    (x,), (w,) = dense_case(1, M, 32, 64, M)
+    bias = torch.randn(64, generator=torch.Generator().manual_seed(2)).bfloat16().to(dev)
+    bias = bias[:1] if form == "one number" else bias[::2]
+    close_to(get_ops(dev).linear(x.to(dev), w.to(dev), bias), x.double() @ w.double().T + bias.cpu().double(), x, w)
+
+
 @gpu
 @pytest.mark.parametrize("B,M,N,K", [(3, 1, 40, 16), (16, 17, 512, 128), (5, 64, 24, 520), (2, 33, 128, 512)])
 def test_skinny_heads(B, M, N, K):
