@@ -14,6 +14,7 @@ namespace hipserve_shared {
 inline hipStream_t cur_stream() { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream(); }
 
 #define CHECK_DEV(x) TORCH_CHECK((x).is_cuda(), #x " must be a GPU tensor")
+#define CHECK_SAME_DEV(x, y) TORCH_CHECK((x).device() == (y).device(), #x " must be on the device of " #y)
 #define CHECK_CONTIG(x) TORCH_CHECK((x).is_contiguous(), #x " must be contiguous")
 #define CHECK_F32(x) TORCH_CHECK((x).scalar_type() == at::kFloat && (x).is_contiguous(), #x " must be contiguous fp32")
 #define CHECK_I32(x) TORCH_CHECK((x).scalar_type() == at::kInt && (x).is_contiguous(), #x " must be contiguous int32")
@@ -50,6 +51,7 @@ inline void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor
 inline void moe_table_align(const at::Tensor& table, const at::Tensor& tokens, int64_t E, int64_t tile, at::Tensor& slots,
                             at::Tensor& tile_expert, at::Tensor& pair_slot) {
   CHECK_DEV(table); CHECK_I32(table); CHECK_I32(slots); CHECK_I32(tile_expert); CHECK_I32(pair_slot);
+  CHECK_SAME_DEV(tokens, table);
   TORCH_CHECK(table.dim() == 2 && table.size(0) >= 1 && tokens.scalar_type() == at::kLong && tokens.is_contiguous());
   TORCH_CHECK(E >= 1 && E <= 128, "moe_align: at most 128 experts");
   TORCH_CHECK(tile == 16 || tile == 32 || tile == 64 || tile == 128 || tile == 256);
@@ -101,7 +103,8 @@ inline bool expert_gemm_skinny(int64_t pairs, int64_t ntiles_cap, int64_t N, int
 // out = act(x . w^T + bias) of at most 64 rows: x [M, K] or [B, M, K], w [N, K] or [B, N, K], out [M, N'] or [B, M, N'].
 inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias,
                           int64_t act, double c0, double c1) {
-  CHECK_DEV(x); CHECK_CONTIG(w);
+  CHECK_DEV(x); CHECK_CONTIG(w); CHECK_SAME_DEV(w, x); CHECK_SAME_DEV(out, x);
+  if (bias.has_value()) CHECK_SAME_DEV(*bias, x);
   const bool f32 = x.scalar_type() == at::kFloat;
   TORCH_CHECK((f32 || x.scalar_type() == at::kBFloat16) && w.scalar_type() == x.scalar_type() &&
               (out.scalar_type() == x.scalar_type() || out.scalar_type() == at::kFloat), "skinny_linear: bf16 or fp32 operands");

@@ -43,6 +43,7 @@ void scaled_add_group_rmsnorm(at::Tensor& out, at::Tensor& residual, const at::T
   if (table.has_value()) {
     TORCH_CHECK(table->scalar_type() == out.scalar_type() && table->is_contiguous() && table->dim() == 2 && table->size(1) == H);
     TORCH_CHECK(ids.has_value() && ids->scalar_type() == at::kLong && ids->is_contiguous() && ids->numel() == T);
+    CHECK_SAME_DEV(*table, out); CHECK_SAME_DEV(*ids, out);
   }
   c10::hip::HIPGuardMasqueradingAsCUDA g(out.device());
   hipserve::launch_scaled_add_group_rmsnorm(

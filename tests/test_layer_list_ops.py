@@ -194,6 +194,28 @@ def test_linear_bias_forms(M, form, dev):
 
 
 @gpu
+@pytest.mark.parametrize("M", [5, 70])
+def test_arguments_on_another_device(M):
+    """Weights, biases, tables and ids in host memory are refused, as the products and lookups of torch refuse them."""
+    ops = get_ops("cuda")
+    (x,), (w,) = dense_case(1, M, 32, 64, M)
+    for args in ((w,), (w.cuda(), torch.zeros(32, dtype=torch.bfloat16))):
+        with pytest.raises(RuntimeError):
+            ops.linear(x.cuda(), *args)
+    ids, table = torch.zeros(M, dtype=torch.long), torch.zeros(7, 64, dtype=torch.bfloat16)
+    out, res, norm = torch.empty(M, 64, dtype=torch.bfloat16, device="cuda"), torch.empty(M, 64, device="cuda"), torch.ones(64, device="cuda")
+    for lib in ("delta", "seq"):
+        ops.norm_library = lib
+        for t, i in ((table, ids.cuda()), (table.cuda(), ids)):
+            with pytest.raises(RuntimeError):
+                ops.scaled_add_group_rmsnorm(out, res, norm, 1, 1e-6, table=t, ids=i)
+        slots, tiles, pairs = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (256, 8, M))
+        with pytest.raises(RuntimeError):
+            ops.moe_table_align(torch.zeros(7, 1, dtype=torch.int32, device="cuda"), ids, 4, 32, slots, tiles, pairs)
+    ops.norm_library = "delta"
+
+
+@gpu
 @pytest.mark.parametrize("B,M,N,K", [(3, 1, 40, 16), (16, 17, 512, 128), (5, 64, 24, 520), (2, 33, 128, 512)])
 def test_skinny_heads(B, M, N, K):
     """Batches with a stride of their own: heads side by side per row, in and out."""
