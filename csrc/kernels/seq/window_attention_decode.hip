@@ -129,17 +129,19 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
 #pragma unroll
     for (int a = 0; a < SUB; ++a) {
       sc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x4 part[4] = {};   // fp32: four chains, whose roundings are smaller than a single one's
 #pragma unroll
       for (int i = 0; i < QN; ++i) {
         if constexpr (F32) {
           const f32x4 kf = __builtin_bit_cast(f32x4, k[a][i]), qf = __builtin_bit_cast(f32x4, q[i]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) sc[a] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], sc[a], 0, 0, 0);
+          for (int e = 0; e < 4; ++e) part[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], part[e], 0, 0, 0);
         } else {
           sc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k[a][i]), __builtin_bit_cast(bf16x8, q[i]),
                                                           sc[a], 0, 0, 0);
         }
       }
+      if constexpr (F32) sc[a] = (part[0] + part[1]) + (part[2] + part[3]);
     }
     // lane (c, g): row c against keys 16 a + 4 g + i
     const bool whole = u0 + KT - 1 <= hi;   // a decode row sees every key of the run

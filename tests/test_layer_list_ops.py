@@ -606,6 +606,37 @@ def test_window_attention_decode_rows_of_one_sequence(ctx, dtype):
     assert torch.equal(run([0, 2, 2, 3], [ctx, 9, ctx - 5], bt), want) and want.isfinite().all()
 
 
+@gpu
+@pytest.mark.parametrize("dim,lens,ctx", [(64, [1] * 16, 1024), (128, [1] * 6, 500), (128, [90, 60], 150)])
+def test_window_attention_fp32_error(dim, lens, ctx, monkeypatch):
+    """fp32 rows on the matrix cores beside the kernel without them, both against 64 bits."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(dim)
+    heads, kv, bs, n, T = 8, 2, 16, len(lens), sum(lens)
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=0, reach=0, scale=dim ** -0.5, sink=False,
+                         keep_first=0, softcap=0.0, channel_gate=False, chunk=0, diff=0.0)
+    width = -(-ctx // bs)
+    cache, proj = torch.randn(n * width, bs, 2 * kv * dim, generator=g) * 1.2, torch.randn(T, heads * dim, generator=g) * 1.3
+    cu, nd = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist()).int(), n if T == n else 0
+    meta = SimpleNamespace(seq_ctx=torch.full((n,), ctx).int().cuda(), seq_cu=cu.cuda(), seq_bt=torch.arange(n * width).int().view(n, width).cuda(),
+                           num_decode=nd, num_prefill_tokens=0 if nd else T, max_ctx=ctx)
+    rows, want = cache.double().view(n, -1, 2 * kv, dim), torch.empty(T, heads, dim, dtype=torch.float64)
+    for s in range(n):
+        mine = slice(int(cu[s]), int(cu[s + 1]))
+        hidden = torch.arange(ctx) > torch.arange(ctx - lens[s], ctx)[:, None]
+        for h in range(heads):
+            k, v = rows[s, :ctx, h // (heads // kv)], rows[s, :ctx, kv + h // (heads // kv)]
+            sc = proj[mine, h * dim:(h + 1) * dim].double() @ k.T * sp.scale
+            want[mine, h] = torch.softmax(sc.masked_fill(hidden, -float("inf")), -1) @ v
+    ops, errs = get_ops("cuda"), []
+    for on in (True, False):
+        monkeypatch.setattr(type(ops), "WINDOW_MFMA", on)
+        out = torch.empty(T, heads * dim, device="cuda")
+        ops.window_attention(out, proj.cuda(), cache.cuda(), meta, sp, -1)
+        errs.append(((out.double().cpu().view(T, heads, dim) - want).norm() / want.norm()).item())
+    assert errs[0] <= 0.8 * errs[1], errs   # measured 0.42 - 0.56; scores summed in a single chain make it 0.96 - 1.02
+
+
 # ------------------------------------------------------------------ generalized delta rule in chunks
 @gpu
 @pytest.mark.parametrize("lens", [[32], [33, 1, 16], [40, 15, 100], [33] + [1] * 70 + [50] + [2] * 65])
