@@ -9,14 +9,14 @@
 //   each 16), and the instruction's rows for the dims that 16 consecutive bytes of a value row hold, every E-th of a block
 //   of 16 E: a lane loads whole 16-byte parts of its keys' rows, and in bf16 two byte permutations per pair of keys and pair
 //   of dims put the keys of one dim side by side.
-// fp32 prompts take the same kernel with several tokens in the 16 rows and a mask per score: the eight waves share no tile, but
-// the 32-bit products are slow enough that reading the keys once per 16 rows costs less than they do.
+// fp32 prompts take the same kernel with several tokens in the 16 rows and a mask per score: the waves (eight, seven at
+// 128 dims) share no tile, but the 32-bit products are slow enough that reading the keys once per 16 rows costs less than they do.
 // What bounds it: the chain table -> cache -> scores -> output of one tile, then (many sequences) memory. All loads of a
 // tile are issued at once and no wave waits for another's. A workgroup that stages every tile for four waves of which one has
 // rows (a group of 4 heads) waits for two barriers and a transposing store per 32 keys: one sequence of 100 keys, 8 heads
 // over 2 of 128 dims, in bf16 11.5 us, this 5.8; 16 sequences of 900 keys, 16 heads over 4: 17.4, 13.3 (with the merge); 64
 // sequences of 1024 keys, 32 heads over 8: 78.6, 48.4 (5.5 TB/s). In fp32 the kernel of window_attention.hip, one wave per
-// head and no split over keys: 16 sequences 528 us, this 23.
+// head and no split over keys: 16 sequences 528 us, this 19.
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
 
@@ -68,6 +68,10 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
   constexpr bool F32 = sizeof(T) == 4;
   constexpr int SUB = F32 ? 1 : 2, KT = 16 * SUB;          // 16-key tiles and keys of a wave's tile
   constexpr int QN = F32 ? D / 16 : D / 32;                // 16-byte parts of a row per lane
+  // Chains of an fp32 score. Decode rows take two: their outputs are at 0.57 - 0.71 of the error against 64 bits that the kernel without
+  // matrix cores has, with one chain 0.96 - 1.02 (over draws of 77 - 2000 keys), in the same time; four: 0.42 - 0.59 and 4 - 9 %
+  // slower. Prompts are at 0.97 - 1.0 with one, and two cost them 12 %.
+  constexpr int CH = MULTI ? 1 : 2;
   constexpr int E = F32 || D == 64 ? 4 : 8, NB = D / (16 * E);   // dims of a value row per load; loads per row
   extern __shared__ float lds[];                           // [waves][rows][D]; [waves][16][2]
   using S = Softmax<T>;
@@ -129,19 +133,19 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
 #pragma unroll
     for (int a = 0; a < SUB; ++a) {
       sc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-      f32x4 part[4] = {};   // fp32: four chains, whose roundings are smaller than a single one's
+      f32x4 part[CH] = {};
 #pragma unroll
       for (int i = 0; i < QN; ++i) {
         if constexpr (F32) {
           const f32x4 kf = __builtin_bit_cast(f32x4, k[a][i]), qf = __builtin_bit_cast(f32x4, q[i]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) part[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], part[e], 0, 0, 0);
+          for (int e = 0; e < 4; ++e) part[e % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[e], part[e % CH], 0, 0, 0);
         } else {
           sc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k[a][i]), __builtin_bit_cast(bf16x8, q[i]),
                                                           sc[a], 0, 0, 0);
         }
       }
-      if constexpr (F32) sc[a] = (part[0] + part[1]) + (part[2] + part[3]);
+      if constexpr (F32) sc[a] = CH == 2 ? part[0] + part[CH - 1] : part[0];
     }
     // lane (c, g): row c against keys 16 a + 4 g + i
     const bool whole = u0 + KT - 1 <= hi;   // a decode row sees every key of the run
