@@ -149,7 +149,6 @@ constexpr int kDC = 64;       // cache dims per staged chunk
 constexpr int kMaxCh = 16;    // kv_rank <= kMaxCh * 64
 constexpr int kMaxRows = 16;  // waves per workgroup
 
-// Finds the workgroup's (sequence, first token) among sequences seq0..seq1-1, `tq` tokens per workgroup.
 template <typename T>
 __global__ __launch_bounds__(64 * kMaxRows) void latent_attention_kernel(
     T* __restrict__ o_lat, const float* __restrict__ q_abs, const T* __restrict__ q, const T* __restrict__ proj,

@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256) void attn_prepare_kernel(
 // is read once, into registers, by 16-byte accesses: an item is two 8-dim chunks of a head (the two halves of 8 rotated
 // pairs, or 16 unrotated dims), one item per thread (N = 2: rows of more than 512 items), the heads' sums stay inside a
 // wave, and a row's angles are computed once, not once per head. 2-byte accesses, a division per element and a sine and
-// cosine per pair and head took 40 us for 8192 rows of 16 + 4 + 4 heads of 128 in bf16, this 14.8; one row of 32 + 8 + 8
+// cosine per pair and head took 40 us for 8192 rows of 16 + 4 + 4 heads of 128 in bf16, this 14.8 (25 between the products of a
+// step, whose rows are not in the cache); one row of 32 + 8 + 8
 // heads with a norm over the whole projection 5.9, this 3.2 (16 rows: 11.0, 4.9).
 template <typename T, int N>
 __global__ __launch_bounds__(512) void attn_prepare_vec_kernel(
