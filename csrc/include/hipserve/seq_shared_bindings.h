@@ -113,7 +113,7 @@ inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor
   TORCH_CHECK((d == 2 || d == 3) && w.dim() == d && out.dim() == d, "skinny_linear: rows or batches of rows");
   const long B = d == 3 ? x.size(0) : 1, M = x.size(-2), K = x.size(-1), N = w.size(-2);
   TORCH_CHECK(w.size(-1) == K && (d == 2 || (w.size(0) == B && out.size(0) == B)) && out.size(-2) == M && M <= 64 && K % per == 0 &&
-              N < (1L << 31) && K < (1L << 30) && B < 65536, "skinny_linear: shapes");
+              N < (1L << 31) && K < (1L << 24) && x.stride(-2) < (1L << 24) && B < 65536, "skinny_linear: shapes");
   const bool glu = act == 3 || act == 4;
   TORCH_CHECK(act >= -1 && act <= 5 && (!glu || N % 2 == 0) && out.size(-1) == (glu ? N / 2 : N), "skinny_linear: activation");
   auto aligned = [](const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
@@ -122,9 +122,9 @@ inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor
   if (bias.has_value())
     TORCH_CHECK(d == 2 && bias->scalar_type() == x.scalar_type() && bias->is_contiguous() && bias->numel() == N, "skinny_linear: bias");
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
-  hipserve::launch_skinny_linear(out.data_ptr(), out.scalar_type() == at::kFloat, out.stride(-2), d == 3 ? out.stride(0) : 0,
-                                 x.data_ptr(), x.stride(-2), d == 3 ? x.stride(0) : 0, w.data_ptr(), opt_ptr(bias), f32, B, M, N, K,
-                                 act, (float)c0, (float)c1, cur_stream());
+  TORCH_CHECK(hipserve::launch_skinny_linear(out.data_ptr(), out.scalar_type() == at::kFloat, out.stride(-2), d == 3 ? out.stride(0) : 0,
+                                             x.data_ptr(), x.stride(-2), d == 3 ? x.stride(0) : 0, w.data_ptr(), opt_ptr(bias), f32, B,
+                                             M, N, K, act, (float)c0, (float)c1, cur_stream()), "skinny_linear: LDS");
 }
 
 inline void def_moe_ops(torch::Library& m) {

@@ -192,45 +192,32 @@ __global__ __launch_bounds__(256) void expert_gemm_mfma_kernel(
   }
 }
 
-// bf16, tiles with few live slots (decode steps): 16 columns per workgroup, K split over its waves (skinny.h).
-template <int NT, int KU, bool GLU>
-__global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
-    unsigned short* __restrict__ out, const unsigned short* __restrict__ x, long x_ld,
-    const unsigned short* __restrict__ w, const int* __restrict__ slots, const int* __restrict__ tile_expert,
-    int gather_k, int N, int K, int act, int E, const float* __restrict__ row_scale, float limit) {
-  constexpr int ST = 2;   // a tile is 32 slots
-  __shared__ __attribute__((aligned(16))) float red[kSkWaves * 16 * ST * kSkLd];
-  const int e = tile_expert[blockIdx.y];
-  if (e < 0 || e >= E) return;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
-  const int slot0 = blockIdx.y * 16 * ST, No = GLU ? N / 2 : N, n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
-  const bool low = c < 8;
-  const int g8 = g + 4 * (c >> 3);
-  const unsigned short* wr[NT][2];
-  const unsigned short* xr[ST][2];
-  bool live[ST][2];
+// bf16, tiles with few live slots (decode steps): 16 columns per workgroup, K split over its waves (skinny.h). XG groups of 8 slots:
+// moe_align fills a tile from its first slot on, so one is enough for most.
+template <int XG, int NT, int DEPTH, bool GLU>
+HS_DEVICE void expert_rows(unsigned short* __restrict__ out, const unsigned short* __restrict__ x, long x_ld,
+                           const unsigned char* const (&wt)[NT], const unsigned (&w_row)[2 * NT], const int* __restrict__ slots, int slot0,
+                           int n0, int No, int gather_k, int K, int act, const float* __restrict__ row_scale, float limit,
+                           unsigned char* smem) {
+  using SK = Skinny<XG, NT, DEPTH>;
+  constexpr int ST = SK::ST;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  unsigned x_row[XG];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int cc = (c & 7) + 8 * h;
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      wr[nt][h] = w + ((long)e * N + (GLU ? nt * No + min(n0 + cc, No - 1) : min(n0 + 16 * nt + cc, N - 1))) * K + 8 * g8;
-#pragma unroll
-    for (int st = 0; st < ST; ++st) {
-      const int slot = slot0 + 16 * st + cc, p = slots[slot];
-      live[st][h] = p >= 0;
-      xr[st][h] = x + (p < 0 ? 0 : gather_k > 0 ? (long)(p / gather_k) : (long)slot) * x_ld + 8 * g8;
-    }
+  for (int j = 0; j < XG; ++j) {
+    const int slot = slot0 + 8 * j + (lane >> 3), p = slots[slot];
+    x_row[j] = (unsigned)(p < 0 ? 0 : gather_k > 0 ? p / gather_k : slot) * (unsigned)x_ld * 2;   // no pair: any row
   }
   f32x4 acc[NT][ST];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  skinny_accumulate<ST, NT, KU>(acc, wr, xr, live, K, g8, low, wave);
-  float v[NT][1];
-  skinny_reduce<ST, NT>(v, acc, red);
-  const int slot = slot0 + (tid >> 4), p = slots[slot];   // 512 threads: an element of the [32, 16] result each
+  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave);
+  float v[NT][(ST + 1) / 2];
+  SK::reduce(v, acc, smem);
+  if (tid >= 128 * XG) return;
+  const int slot = slot0 + (tid >> 4), p = slots[slot];   // an element of the [8 XG, 16] result per thread
   if (p < 0) return;
   const float f = row_scale != nullptr ? row_scale[p] : 1.f;
 #pragma unroll
@@ -247,6 +234,39 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
     }
     out[(long)slot * No + n] = f32_to_bf16(r);
   }
+}
+
+template <int NT> constexpr int expert_lds() {   // of the widest of the three below
+  constexpr int a = Skinny<1, NT, 2>::kLds, b = Skinny<2, NT, 1>::kLds, c = Skinny<4, NT, 1>::kLds;
+  return a > b ? (a > c ? a : c) : (b > c ? b : c);
+}
+
+template <int NT, bool GLU>
+__global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
+    unsigned short* __restrict__ out, const unsigned short* __restrict__ x, long x_ld,
+    const unsigned short* __restrict__ w, const int* __restrict__ slots, const int* __restrict__ tile_expert,
+    int gather_k, int N, int K, int act, int E, const float* __restrict__ row_scale, float limit) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int e = tile_expert[blockIdx.y];
+  if (e < 0 || e >= E) return;
+  const int lane = threadIdx.x & 63;
+  const int slot0 = blockIdx.y * 32, No = GLU ? N / 2 : N, n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
+  const unsigned char* wt[NT];
+  unsigned w_row[2 * NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int first = GLU ? n0 : min(n0 + 16 * nt, N - 1);   // of the tile's columns
+    wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)e * N + (GLU ? nt * No : 0) + first) * K);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)(min(first + 8 * h + (lane >> 3), No - 1) - first) * (unsigned)K * 2;
+  }
+#define HS_ER(XG, DEPTH) \
+  expert_rows<XG, NT, DEPTH, GLU>(out, x, x_ld, wt, w_row, slots, slot0, n0, No, gather_k, K, act, row_scale, limit, smem)
+  const unsigned long live = __ballot(slots[slot0 + (lane & 31)] >= 0);
+  if (live >> 16 & 0xffff) HS_ER(4, 1);
+  else if (live >> 8 & 0xff) HS_ER(2, 1);
+  else HS_ER(1, 2);
+#undef HS_ER
 }
 
 }  // namespace
@@ -276,15 +296,14 @@ void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, cons
     dim3 mg(act >= 2 ? (No + 63) / 64 : (N + 127) / 128, ntiles_cap);
     auto o = (unsigned short*)out;
     auto xi = (const unsigned short*)x, wi = (const unsigned short*)w;
-    if (tile == 32 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && expert_gemm_skinny(pairs, ntiles_cap, N, K, E, act >= 2)) {
+    if (tile == 32 && K < (1 << 24) && 2L * ntiles_cap * tile * x_ld < (1L << 32) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && expert_gemm_skinny(pairs, ntiles_cap, N, K, E, act >= 2)) {
       const dim3 sg((No + 15) / 16, ntiles_cap);
-#define HS_ES(NT, KU, GLU)                                                                                          \
-  expert_gemm_skinny_kernel<NT, KU, GLU><<<sg, kSkThreads, 0, s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K, \
-                                                                   act, E, row_scale, limit)
-      if (act >= 2) HS_ES(2, 4, true);
-      else if (K <= 1024) HS_ES(1, 4, false);
-      else HS_ES(1, 8, false);
-#undef HS_ES
+      if (act >= 2)
+        expert_gemm_skinny_kernel<2, true><<<sg, kSkThreads, expert_lds<2>(), s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K,
+                                                                                  act, E, row_scale, limit);
+      else
+        expert_gemm_skinny_kernel<1, false><<<sg, kSkThreads, expert_lds<1>(), s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N,
+                                                                                   K, act, E, row_scale, limit);
       return;
     }
     if (tile == 32) expert_gemm_mfma_kernel<2><<<mg, 256, 0, s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K, act, E, row_scale, limit);

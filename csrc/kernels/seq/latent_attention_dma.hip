@@ -476,12 +476,6 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
   }
 }
 
-template <typename F>
-bool allow_lds(F* fn, size_t bytes) {   // more dynamic LDS than the default limit, once per kernel
-  return bytes <= 64 * 1024 ||
-         hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
-}
-
 template <int DV>
 bool launch_dma(void* o_lat, const void* qc, const void* q, const long* positions, const float* inv_freq, const void* proj,
                 long proj_ld, const void* cache, int block_shift, const int* seq_cu, const int* seq_ctx, const int* seq_bt,

@@ -72,4 +72,10 @@ HS_DEVICE unsigned pack2(float a, float b) {
   return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
 }
 
+template <typename F>
+inline bool allow_lds(F* fn, size_t bytes) {   // more dynamic LDS than the default limit, once per kernel
+  return bytes <= 64 * 1024 ||
+         hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
+}
+
 }  // namespace hipserve

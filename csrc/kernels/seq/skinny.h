@@ -3,104 +3,150 @@
 //
 // Such a product reads every weight once and does next to nothing with it, so its time is the latency of one load
 // plus the weights over the bandwidth. A workgroup of 8 waves owns 16 columns (NT tiles of them) and splits K over its
-// waves: every wave issues the loads of its KU steps of 32 k before the first product, and the waves' sums meet in LDS.
-// 16 columns per workgroup give 128 workgroups at 2048 columns. A compute unit takes in about 34 KB per us this way, so
-// the rows' own bytes (16 columns of weights serve M rows) bound the larger M: 2048 x 2048, cold weights: 1 row 4.7 us,
-// 16 rows 6.2, 32 rows 8.0, 48 rows 10.2 (the vendor's GEMM: 11.0 - 11.2); 32000 x 2048, 1 row: 26 us = 5.0 TB/s (34).
+// waves, 64 k at a time; the waves' sums meet in LDS. 16 columns per workgroup give 128 workgroups at 2048 columns.
+//
+// What a compute unit takes in (its weights, and the rows again for every workgroup) bounds the larger M, and how a load
+// spreads its addresses decides how much that is. The matrix cores want 16 rows side by side over the lanes; a load that
+// follows them jumps to another row from lane to lane, and the addresses of its 64 lanes are looked up one by one: 34 KB per us
+// and CU, however many loads are in flight. So the rows go through LDS: global_load_lds takes 8 lanes side by side along a row
+// (whole 128-byte lines, four lanes per look-up) and the operands are read from there, without registers for loads in
+// flight: about 60 KB per us. Each wave copies into a part of LDS that is its own, DEPTH pieces of 64 k ahead, and waits for
+// its own copies alone. us, cold weights, loads in operand order -> this (the vendor's GEMM), 1 / 16 / 48 rows:
+//   1024 x 1024   3.4 -> 2.8 (5.6)    4.2 -> 3.1 (5.7)    6.5 -> 3.9 (8.1)     (columns x k)
+//   2048 x 2048   5.0 -> 4.4 (11.0)   6.4 -> 5.1 (11.1)   10.5 -> 7.1 (11.4)
+//   2048 x 6144   9.3 -> 7.8 (11.1)   13.6 -> 10.5 (11.2) 24.7 -> 16.2 (16.5)
+//   32000 x 2048  25.2 -> 25.6 (32.3) 33.7 -> 27.8 (30.9) 60 -> 33.5, four tiles per workgroup (34)
+// Deeper copies (3 or 5 pieces) changed nothing at one workgroup per CU and cost up to a fifth where they leave room for fewer.
 // 32-bit operands (F32) are the same rows of twice as many 16-bit halves: a step is 64 bytes of a row, 16 numbers, and four
-// products of 4 k each; the four numbers of a lane are k 4 g + e on both sides, so nothing else differs. 3 rows, cold
-// weights, 3072 x 1024: 5.9 us (the vendor's GEMM: 11.3); 32000 x 1024: 29 us = 4.5 TB/s (34).
+// products of 4 k each; the four numbers of a lane are k 4 g + e on both sides, so nothing else differs.
 #pragma once
+#include "lds_copy.h"
 #include "seq_common.h"
 
 namespace hipserve {
 
 constexpr int kSkWaves = 8, kSkThreads = 64 * kSkWaves, kSkLd = 20;   // kSkLd: row stride of the sums in LDS (floats)
 
-// Two k steps of 16 rows as MFMA operands: lane (c, g) wants k 8 g .. + 7 of row c of both steps (64 bytes of a row each).
-// The loads instead take whole 128-byte lines: lane (c, g) reads the part g + 4 (c / 8) of row c % 8 and of row c % 8 + 8
-// (whole lines measured 4 - 14 % faster than 64 bytes of 16 rows), and the lanes c, c ^ 8 then exchange what belongs to the other's row (a rotation by 8 within 16 lanes).
-HS_DEVICE void swap_steps(u16x8& s0, u16x8& s1, bool low) {
-  const u32x4 a = __builtin_bit_cast(u32x4, s0), b = __builtin_bit_cast(u32x4, s1);
-  u32x4 x, y;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const unsigned give = low ? b[i] : a[i];
-    const unsigned got = (unsigned)__builtin_amdgcn_update_dpp(0, (int)give, 0x128, 0xf, 0xf, true);
-    x[i] = low ? a[i] : got;
-    y[i] = low ? got : b[i];
-  }
-  s0 = __builtin_bit_cast(u16x8, x);
-  s1 = __builtin_bit_cast(u16x8, y);
-}
+template <int N> HS_DEVICE void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
-// acc[nt][st] += the wave's part of W[16 columns of tile nt] . x[16 rows of tile st]; lane (c, g) = (lane % 16, lane / 16)
-// ends with columns 4 g .. + 3 of row c. K in 16-bit halves. wr / xr: two row addresses per tile (c % 8 and c % 8 + 8), advanced by
-// 8 g8, g8 = g + 4 (c / 8); low = c < 8. K % 8 == 0, KU even.
-template <int ST, int NT, int KU, bool F32 = false>
-HS_DEVICE void skinny_accumulate(f32x4 (&acc)[NT][ST], const unsigned short* const (&wr)[NT][2],
-                                 const unsigned short* const (&xr)[ST][2], const bool (&live)[ST][2], int K, int g8,
-                                 bool low, int wave) {
-  const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int k0 = wave * 32 * KU; k0 < K; k0 += kSkWaves * 32 * KU) {
-    u16x8 a[KU][NT], b[KU][ST];
-#pragma unroll
-    for (int u = 0; u < KU; ++u) {
-      const int k = k0 + 64 * (u / 2);
-      const bool in = k + 8 * g8 < K;
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) a[u][nt] = in ? *reinterpret_cast<const u16x8*>(wr[nt][u & 1] + k) : zero;
-#pragma unroll
-      for (int st = 0; st < ST; ++st) b[u][st] = (in && live[st][u & 1]) ? *reinterpret_cast<const u16x8*>(xr[st][u & 1] + k) : zero;
-    }
-#pragma unroll
-    for (int u = 0; u < KU; u += 2) {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) swap_steps(a[u][nt], a[u + 1][nt], low);
-#pragma unroll
-      for (int st = 0; st < ST; ++st) swap_steps(b[u][st], b[u + 1][st], low);
-    }
-#pragma unroll
-    for (int u = 0; u < KU; ++u)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int st = 0; st < ST; ++st) {
-          if constexpr (F32) {
-            const f32x4 fa = __builtin_bit_cast(f32x4, a[u][nt]), fb = __builtin_bit_cast(f32x4, b[u][st]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[nt][st] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], acc[nt][st], 0, 0, 0);
-          } else {
-            acc[nt][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[u][nt]),
-                                                                  __builtin_bit_cast(bf16x8, b[u][st]), acc[nt][st], 0, 0, 0);
-          }
-        }
-  }
-}
+// One wave's part of W[NT tiles of 16 columns] . x[XG groups of 8 rows]. K in 16-bit halves, K % 8 == 0.
+// A piece (64 k) in LDS: [NT tiles][16 rows][128 bytes] of W, then [XG][8 rows][128 bytes] of x; the 16-byte part q of row r sits
+// at part q ^ (r / 2 % 8), so that the 16 rows of an operand use all banks evenly: a lane copies the part that belongs at its place.
+template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
+  static constexpr int ST = (XG + 1) / 2, kCopies = 2 * NT + XG, kPiece = kCopies * 1024;
+  // the last tile's missing 8 rows, where XG is odd, are read past the piece
+  static constexpr int kRing = kSkWaves * DEPTH * kPiece + (XG & 1) * 1024, kSums = kSkWaves * 16 * ST * kSkLd * 4;
+  static constexpr int kLds = kRing > kSums ? kRing : kSums;
+  static_assert(kLds <= 160 * 1024 && kCopies * (DEPTH - 1) < 64, "LDS; copies that a wait can count");
 
-// Sums the waves' parts: v[nt][i] = element (row, column) = (e / 16, e % 16), e = threadIdx.x + kSkThreads * i, of
-// the [16 ST, 16] result of column tile nt (threads past 256 ST get nothing). red: kSkWaves * 16 ST * kSkLd floats.
-template <int ST, int NT>
-HS_DEVICE void skinny_reduce(float (&v)[NT][(ST + 1) / 2], const f32x4 (&acc)[NT][ST], float* red) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+  static HS_DEVICE int part(int lane, int row) { return (lane & 7) ^ (row >> 1 & 7); }   // of a row, for a lane's copy
+
+  // acc[nt][st] += the products; lane (c, g) = (lane % 16, lane / 16) ends with columns 4 g .. + 3 of row 16 st + c. w[nt]: first row
+  // of the tile; w_row[i] / x_row[j]: byte offsets of the lane's row (lane / 8 of the 8) in the half tile i (of 2 NT) from w[i / 2] and in
+  // the group j of x from `x`. Every row is one that exists: what rows past the last one give is not used.
+  static HS_DEVICE void accumulate(f32x4 (&acc)[NT][ST], const unsigned char* const (&w)[NT], const unsigned (&w_row)[2 * NT],
+                                   const unsigned char* x, const unsigned (&x_row)[XG], int K, unsigned char* smem,
+                                   int lane, int wave) {
+    const int c = lane & 15, g = lane >> 4, r8 = lane >> 3;
+    unsigned char* ring = smem + wave * DEPTH * kPiece;
+    const unsigned lds0 = lds_at(ring);
+    const int pieces = (K + 63) / 64, n = (pieces - wave + kSkWaves - 1) / kSkWaves;   // this wave's: wave, wave + 8, ...
+    // the lane's bytes past the piece's first k of the first row: full pieces differ by uniform numbers
+    unsigned w_at[2 * NT], x_at[XG];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    if (nt > 0) __syncthreads();   // the previous tile's sums are read
+    for (int j = 0; j < 2 * NT; ++j) w_at[j] = w_row[j] + 16 * part(lane, 8 * (j & 1) + r8);
 #pragma unroll
-    for (int st = 0; st < ST; ++st)
-      *reinterpret_cast<f32x4*>(red + ((wave * ST + st) * 16 + c) * kSkLd + 4 * g) = acc[nt][st];
-    __syncthreads();
+    for (int j = 0; j < XG; ++j) x_at[j] = x_row[j] + 16 * part(lane, 8 * (j & 1) + r8);
+    auto copy = [&](int i) {
+      const int k0 = 64 * (wave + kSkWaves * i);
+      const unsigned to = lds0 + i % DEPTH * kPiece;
+      if (k0 + 64 <= K) {
 #pragma unroll
-    for (int i = 0; i < (ST + 1) / 2; ++i) {
-      const int e = tid + kSkThreads * i;
-      float s = 0.f;
-      if (e < 256 * ST) {
+        for (int j = 0; j < XG; ++j) copy_1k(x + 2 * k0, x_at[j], to + (2 * NT + j) * 1024);
 #pragma unroll
-        for (int w = 0; w < kSkWaves; ++w) s += red[(w * ST * 16 + (e >> 4)) * kSkLd + (e & 15)];
+        for (int j = 0; j < 2 * NT; ++j) copy_1k(w[j / 2] + 2 * k0, w_at[j], to + j * 1024);
+        return;
       }
-      v[nt][i] = s;
+#pragma unroll
+      for (int j = 0; j < XG; ++j)   // what lies past K is not used
+        copy_1k(x, x_row[j] + 2 * min(k0 + 8 * part(lane, 8 * (j & 1) + r8), K - 8), to + (2 * NT + j) * 1024);
+#pragma unroll
+      for (int j = 0; j < 2 * NT; ++j)
+        copy_1k(w[j / 2], w_row[j] + 2 * min(k0 + 8 * part(lane, 8 * (j & 1) + r8), K - 8), to + j * 1024);
+    };
+    int at[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) at[s] = c * 128 + (((4 * s + g) ^ (c >> 1)) << 4);
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i)
+      if (i < n) copy(i);
+    for (int i = 0; i < n; ++i) {
+      if (i + DEPTH <= n) wait_copies<kCopies * (DEPTH - 1)>();
+      else wait_copies<0>();
+      const unsigned char* t = ring + i % DEPTH * kPiece;
+      u16x8 a[2][NT], b[2][ST];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) a[s][nt] = *reinterpret_cast<const u16x8*>(t + nt * 2048 + at[s]);
+#pragma unroll
+        for (int st = 0; st < ST; ++st) b[s][st] = *reinterpret_cast<const u16x8*>(t + (NT + st) * 2048 + at[s]);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the piece is read
+      if (i + DEPTH < n) copy(i + DEPTH);
+      if (64 * (wave + kSkWaves * i) + 64 > K) {   // what lies past K is 0 on both sides
+        const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          if (64 * (wave + kSkWaves * i) + 32 * s + 8 * g < K) continue;
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) a[s][nt] = zero;
+#pragma unroll
+          for (int st = 0; st < ST; ++st) b[s][st] = zero;
+        }
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+          for (int st = 0; st < ST; ++st) {
+            if constexpr (F32) {
+              const f32x4 fa = __builtin_bit_cast(f32x4, a[s][nt]), fb = __builtin_bit_cast(f32x4, b[s][st]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[nt][st] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], acc[nt][st], 0, 0, 0);
+            } else {
+              acc[nt][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[s][nt]),
+                                                                    __builtin_bit_cast(bf16x8, b[s][st]), acc[nt][st], 0, 0, 0);
+            }
+          }
     }
   }
-}
+
+  // Sums the waves' parts: v[nt][i] = element (row, column) = (e / 16, e % 16), e = threadIdx.x + kSkThreads * i, of
+  // the [16 ST, 16] result of column tile nt (threads past 256 ST get nothing).
+  static HS_DEVICE void reduce(float (&v)[NT][(ST + 1) / 2], const f32x4 (&acc)[NT][ST], unsigned char* smem) {
+    float* red = reinterpret_cast<float*>(smem);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      __syncthreads();   // the pieces, or the previous tile's sums, are read
+#pragma unroll
+      for (int st = 0; st < ST; ++st)
+        *reinterpret_cast<f32x4*>(red + ((wave * ST + st) * 16 + c) * kSkLd + 4 * g) = acc[nt][st];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < (ST + 1) / 2; ++i) {
+        const int e = tid + kSkThreads * i;
+        float s = 0.f;
+        if (e < 256 * ST) {
+#pragma unroll
+          for (int w = 0; w < kSkWaves; ++w) s += red[(w * ST * 16 + (e >> 4)) * kSkLd + (e & 15)];
+        }
+        v[nt][i] = s;
+      }
+    }
+  }
+};
 
 }  // namespace hipserve

@@ -4,6 +4,8 @@
 // columns in out), 5 soft cap, -1 none; they see the unrounded product.
 #include "skinny.h"
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "hipserve/seq_kernels.h"
@@ -19,47 +21,43 @@ HS_DEVICE float skinny_act(float z, int act, float c0, float c1) {
   return z;
 }
 
-// ST: 16-row tiles; NT: 16-column tiles (GLU: the gate's and the up projection's of the same 16 output columns);
-// KU: k steps of 32 whose loads a wave has in flight.
+// XG: groups of 8 rows; NT: 16-column tiles (GLU: the gate's and the up projection's of the same 16 output columns).
 // F32: 32-bit operands, x, w, their strides and K in 16-bit halves (skinny.h).
-template <int ST, int NT, int KU, bool GLU, typename TO, bool F32>
+template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32>
 __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
     TO* __restrict__ out, long out_ld, long out_bs, const unsigned short* __restrict__ x, long x_ld, long x_bs,
     const unsigned short* __restrict__ w, const void* __restrict__ bias_, int M, int N, int K, int act, float c0, float c1) {
   static_assert(!GLU || NT == 2, "a gate tile and an up tile");
+  using SK = Skinny<XG, NT, DEPTH, F32>;
+  constexpr int ST = SK::ST;
   using TB = std::conditional_t<F32, float, unsigned short>;
   const TB* bias = static_cast<const TB*>(bias_);
-  __shared__ __attribute__((aligned(16))) float red[kSkWaves * 16 * ST * kSkLd];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int No = GLU ? N / 2 : N;
   const int n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
   x += (long)blockIdx.y * x_bs;
   w += (long)blockIdx.y * N * K;
-  const bool low = c < 8;
-  const int g8 = g + 4 * (c >> 3);
-  const unsigned short* wr[NT][2];
-  const unsigned short* xr[ST][2];
-  bool live[ST][2];
+  const unsigned char* wt[NT];
+  unsigned w_row[2 * NT];
+  unsigned x_row[XG];
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int cc = (c & 7) + 8 * h;
+  for (int nt = 0; nt < NT; ++nt) {
+    const int first = GLU ? n0 : min(n0 + 16 * nt, N - 1);   // of the tile's columns
+    wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)(GLU ? nt * No : 0) + first) * K);
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      wr[nt][h] = w + (long)(GLU ? nt * No + min(n0 + cc, No - 1) : min(n0 + 16 * nt + cc, N - 1)) * K + 8 * g8;
-#pragma unroll
-    for (int st = 0; st < ST; ++st) {
-      live[st][h] = 16 * st + cc < M;
-      xr[st][h] = x + (live[st][h] ? 16 * st + cc : 0) * x_ld + 8 * g8;
-    }
+    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)(min(first + 8 * h + (lane >> 3), No - 1) - first) * (unsigned)K * 2;
   }
+#pragma unroll
+  for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)x_ld * 2;
   f32x4 acc[NT][ST];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  skinny_accumulate<ST, NT, KU, F32>(acc, wr, xr, live, K, g8, low, wave);
+  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave);
   float v[NT][(ST + 1) / 2];
-  skinny_reduce<ST, NT>(v, acc, red);
+  SK::reduce(v, acc, smem);
   out += (long)blockIdx.y * out_bs;
 #pragma unroll
   for (int i = 0; i < (ST + 1) / 2; ++i) {
@@ -83,48 +81,58 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
   }
 }
 
-template <int ST, int NT, int KU, bool GLU>
-void launch_one(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs, const void* w,
+template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32>
+bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, const void* x, long x_ld, long x_bs, const void* w, const void* bias,
+                   int M, int N, int K, int act, float c0, float c1, hipStream_t s) {
+  constexpr int lds = Skinny<XG, NT, DEPTH, F32>::kLds;
+  static const bool ok = allow_lds(&skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32>, lds);
+  if (!ok) return false;
+  skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32><<<grid, kSkThreads, lds, s>>>(
+      (TO*)out, out_ld, out_bs, (const unsigned short*)x, x_ld, x_bs, (const unsigned short*)w, bias, M, N, K, act, c0, c1);
+  return true;
+}
+
+template <int XG, int NT, int DEPTH, bool GLU>
+bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs, const void* w,
                 const void* bias, bool f32, int batch, int M, int N, int K, int act, float c0, float c1, hipStream_t s) {
   const int cols = GLU ? N / 2 : N, per = GLU ? 16 : 16 * NT;
   const dim3 grid((cols + per - 1) / per, batch);
-  auto xi = (const unsigned short*)x, wi = (const unsigned short*)w;
-  if (f32)
-    skinny_linear_kernel<ST, NT, KU, GLU, float, true><<<grid, kSkThreads, 0, s>>>((float*)out, out_ld, out_bs, xi, x_ld, x_bs, wi,
-                                                                                  bias, M, N, K, act, c0, c1);
-  else if (out_f32)
-    skinny_linear_kernel<ST, NT, KU, GLU, float, false><<<grid, kSkThreads, 0, s>>>((float*)out, out_ld, out_bs, xi, x_ld, x_bs, wi,
-                                                                                   bias, M, N, K, act, c0, c1);
-  else
-    skinny_linear_kernel<ST, NT, KU, GLU, unsigned short, false><<<grid, kSkThreads, 0, s>>>(
-        (unsigned short*)out, out_ld, out_bs, xi, x_ld, x_bs, wi, bias, M, N, K, act, c0, c1);
+#define HS_SK(TO, F32) launch_kernel<XG, NT, DEPTH, GLU, TO, F32>(grid, out, out_ld, out_bs, x, x_ld, x_bs, w, bias, M, N, K, act, c0, c1, s)
+  return f32 ? HS_SK(float, true) : out_f32 ? HS_SK(float, false) : HS_SK(unsigned short, false);
+#undef HS_SK
+}
+
+// us of a launch with NT tiles of 16 columns per workgroup: a latency, 0.38 of the time the weights take at 5.2 TB/s (and no less
+// than that time), and what the busiest compute unit takes in at 65 / 60 / 54 KB per us. More tiles mean fewer copies of the rows and fewer workgroups. Cold weights, 1 / 2 / 4 tiles: 6144 x 2048 with 16 rows 8.2 /
+// 7.6 / -, with 48 rows 12.5 / 9.8 / 12.5; 12288 x 2048 with 16 rows 12.0 / 13.5 / -, with 48 rows 18.6 / 16.4 / 14.7; 12288 x 4096 with
+// 48 rows 32.1 / 29.3 / 23.9; 32000 x 2048 with 16 rows 26.8 / 26.8 / -, with 32 rows 38.5 / 29.7 / 30.4, with 64 50.9 / 40.4 / 34.3.
+double skinny_time(int M, long cols, int K, int nt) {
+  const long wgs = ((cols + 15) / 16 + nt - 1) / nt, rounds = (wgs + 255) / 256;
+  const double stream = 2.0 * cols * K / 5.2e6, rate = nt == 1 ? 65e3 : nt == 2 ? 60e3 : 54e3;
+  return 2.2 + std::max(stream, 0.38 * stream + rounds * 2.0 * K * (16 * nt + (M + 7) / 8 * 8) / rate);
 }
 
 }  // namespace
 
-void launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs,
+bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs,
                           const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, float c0, float c1,
                           hipStream_t s) {
-  if (batch <= 0 || M <= 0 || N <= 0) return;
+  if (batch <= 0 || M <= 0 || N <= 0) return true;
   if (f32) { x_ld *= 2; x_bs *= 2; K *= 2; }   // in halves
-#define HS_SK(ST, NT, KU, GLU) \
-  launch_one<ST, NT, KU, GLU>(out, out_f32, out_ld, out_bs, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, c0, c1, s)
-  // the loads in flight per wave cover K in one go where the registers allow it: KU steps of 32 k on 8 waves
-  if (act == 3 || act == 4) {
-    if (M <= 16) HS_SK(1, 2, 4, true);
-    else if (M <= 32) HS_SK(2, 2, 4, true);
-    else HS_SK(4, 2, 4, true);
-  } else if (K <= 512) {
-    if (M <= 16) HS_SK(1, 1, 2, false);
-    else if (M <= 32) HS_SK(2, 1, 2, false);
-    else HS_SK(4, 1, 2, false);
-  } else if (M <= 4 && K > 1024) {
-    HS_SK(1, 1, 8, false);
-  } else {
-    if (M <= 16) HS_SK(1, 1, 4, false);
-    else if (M <= 32) HS_SK(2, 1, 4, false);
-    else HS_SK(4, 1, 2, false);
-  }
+#define HS_SK(XG, NT, DEPTH, GLU)   launch_one<XG, NT, DEPTH, GLU>(out, out_f32, out_ld, out_bs, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, c0, c1, s)
+  const int xg = (M + 7) / 8;
+  if (act == 3 || act == 4)
+    return xg <= 1 ? HS_SK(1, 2, 1, true) : xg <= 2 ? HS_SK(2, 2, 1, true) : xg <= 4 ? HS_SK(4, 2, 1, true)
+         : xg <= 6 ? HS_SK(6, 2, 1, true) : HS_SK(8, 2, 1, true);
+  const double t1 = skinny_time(M, (long)N * batch, K, 1), t2 = skinny_time(M, (long)N * batch, K, 2),
+               t4 = M > 16 ? skinny_time(M, (long)N * batch, K, 4) : INFINITY;
+  // one piece ahead where the workgroups of several tiles would otherwise not fit a compute unit together (2 - 14 % faster)
+  if (t4 < t1 && t4 < t2) return xg <= 4 ? HS_SK(4, 4, 1, false) : xg <= 6 ? HS_SK(6, 4, 1, false) : HS_SK(8, 4, 1, false);
+  if (t2 < t1)
+    return xg <= 1 ? HS_SK(1, 2, 1, false) : xg <= 2 ? HS_SK(2, 2, 1, false) : xg <= 4 ? HS_SK(4, 2, 1, false)
+         : xg <= 6 ? HS_SK(6, 2, 1, false) : HS_SK(8, 2, 1, false);
+  return xg <= 1 ? HS_SK(1, 1, 2, false) : xg <= 2 ? HS_SK(2, 1, 2, false) : xg <= 3 ? HS_SK(3, 1, 2, false)
+       : xg <= 4 ? HS_SK(4, 1, 2, false) : xg <= 6 ? HS_SK(6, 1, 2, false) : HS_SK(8, 1, 2, false);
 #undef HS_SK
 }
 

@@ -433,27 +433,30 @@ class KernelOps:
     @staticmethod
     def skinny_pays(rows: int, cols: int, k: int, glu: bool = False, f32: bool = False) -> bool:
         """Whether ``skinny_linear`` is expected to be faster than the vendor's GEMM for ``rows`` x ``cols`` results (``cols``
-        over all batches). Both sides in us, fitted to cold weights of 1024 .. 32000 columns and k of 1024 .. 12288: ours is
-        a latency plus the weights at 5 TB/s, or what a workgroup of 16 columns reads (weights and rows) at 34 KB per us and
-        compute unit; the vendor's is hardly ever below 10.5 (7.5 up to k = 1024) and streams large weights at 4.2 TB/s.
-        Examples, ours / vendor: 2048 x 2048 with 1, 16, 32, 48 rows 4.7 / 11.0, 6.2 / 11.1, 8.0 / 11.2, 10.2 / 11.2; 6144 x
-        2048 with 1, 16, 32, 48 rows 7.7 / 12.6, 10.3 / 12.3, 13.7 / 12.3, 17.8 / 12.9; 2048 x 6144 with 1, 16 rows 9.0 / 10.9,
-        13.2 / 11.1; 3072 x 1024 with 1, 48 rows 3.7 / 7.3, 6.7 / 11.1; 32000 x 2048 with 1, 16, 32 rows 26 / 34, 34 / 34, 46 / 34."""
+        over all batches). Both sides in us, fitted to cold weights of 1024 .. 32000 columns and k of 1024 .. 12288: ours as the
+        kernel's choice of tiles has it (skinny_time in skinny_linear.hip); the vendor's is hardly ever below 10.5 (7.5 up to k =
+        1024), grows with k past 32 rows and streams large weights at 4.2 - 5 TB/s. Examples, ours / vendor: 2048 x 2048 with 1, 16, 48,
+        64 rows 4.4 / 11.0, 5.1 / 11.1, 7.1 / 11.4, 8.0 / 11.9; 6144 x 2048 with 1, 16, 48 rows 7.8 / 12.5, 8.1 / 12.5, 10.1 / 12.9;
+        2048 x 6144 with 1, 16, 48 rows 7.8 / 11.1, 10.5 / 11.2, 16.2 / 16.5; 12288 x 2048 with 16, 48 rows 12.6 / 15, 15.2 / 15.6;
+        32000 x 2048 with 1, 16, 48, 64 rows 26 / 32, 28 / 31, 34 / 34, 35 / 30."""
+        k *= 2 if f32 else 1   # in 16-bit halves
+        stream, tiles, padded = 2.0 * cols * k / 5.2e6, -(-cols // 16), -(-rows // 8) * 8
+
+        def intake(nt, rate):
+            return -(-(-(-tiles // nt)) // 256) * 2.0 * k * (16 * nt + padded) / rate
+
+        ours = 2.2 + max(stream, 0.38 * stream + (intake(2, 60e3) if glu else min(intake(1, 65e3), intake(2, 60e3), intake(4, 54e3))))
         if f32:
-            # the same in 32 bits (twice the bytes, whole workgroups per compute unit); the vendor's is hardly ever below 10.7
-            # (8.9 for 1024 x 1024) and streams at 4.5 TB/s. 1544 x 1024 with 1, 3, 16 rows 5.6 / 10.8, 5.7 / 10.9, 6.6 / 10.9;
-            # 1024 x 3072 with 1, 16 rows 10.3 / 10.7, 13.6 / 11.0; 32000 x 1024 with 3, 16 rows 29 / 34, 35 / 33.
-            weights, per_cu = 4.0 * cols * k, -(-cols // (32 if glu else 16) // 256) * 4.0 * k * ((32 if glu else 16) + rows)
-            return 4.2 + max(weights / 5.0e6, per_cu / 34e3) < max(8.9 if max(cols, k) <= 1024 else 10.7, 3.2 + weights / 4.5e6)
-        weights = 2.0 * cols * k
-        per_cu = max(1.0, cols / (32 if glu else 16) / 256) * 2.0 * k * ((32 if glu else 16) + rows)
-        return 3.2 + max(weights / 5.0e6, per_cu / 34e3) < max(7.5 if k <= 1024 else 10.5, 3.2 + weights / 4.2e6)
+            # the vendor's is hardly ever below 10.7 (8.9 for 1024 x 1024) and streams at 4.5 TB/s
+            return ours < max(8.9 if max(cols, k // 2) <= 1024 else 10.7, 3.2 + 2.0 * cols * k / 4.5e6)
+        least = 7.5 if k <= 1024 else 10.5 if rows <= 32 else max(10.5, 4.6 + 1.85e-3 * k)
+        return ours < max(least, 3.2 + 2.0 * cols * k / 4.2e6 if rows <= 16 else 4.2 + 2.0 * cols * k / 4.8e6)
 
     def _skinny_ok(self, x, w) -> bool:
         """The shapes, types and alignment that ``skinny_linear`` takes."""
         per = 16 // x.element_size()
         return (x.dtype in (torch.bfloat16, torch.float32) and w.dtype == x.dtype and x.dim() == w.dim() and 0 < x.shape[-2] <= self.SKINNY_ROWS
-                and x.shape[-1] % per == 0 and x.stride(-1) == 1 and x.stride(-2) % per == 0 and x.stride(0) % per == 0
+                and x.shape[-1] % per == 0 and max(x.shape[-1], x.stride(-2)) < 1 << 24 and x.stride(-1) == 1 and x.stride(-2) % per == 0 and x.stride(0) % per == 0
                 and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
     def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0):

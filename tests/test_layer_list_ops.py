@@ -133,6 +133,18 @@ def test_skinny_linear(M, N, K):
 
 
 @gpu
+@pytest.mark.parametrize("M", [8, 9, 24, 25, 40, 41, 64])
+@pytest.mark.parametrize("N", [4113, 5001, 12301])
+def test_skinny_linear_wide(M, N):
+    """More columns than one workgroup of 16 per compute unit: two (5001) or four (12301) tiles per workgroup, the last ones past N."""
+    K = 520
+    (x,), (w,) = dense_case(1, M, N, K, M + N)
+    got = torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    get_ops("cuda")._moe_lib.skinny_linear(got, x.cuda(), w.cuda(), None, -1, 0.0, 0.0)
+    close_to(got, x.double() @ w.double().T, x, w)
+
+
+@gpu
 @pytest.mark.parametrize("M,N,K", [(1, 1, 4), (3, 40, 36), (16, 16, 256), (17, 96, 260), (33, 33, 1024), (64, 48, 3076)])
 def test_skinny_linear_f32(M, N, K):
     """32-bit operands: k that fills a step of 16, a wave's steps and all waves partly; bias, row strides, an activation."""
