@@ -61,6 +61,17 @@ bool launch_latent_attention_dma(void* o_lat, const void* qc, const void* q, con
                                  const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int seq1, int rows_bound, int T,
                                  int heads, int dim, int kv_rank, int gate_off, float scale, int window, int nparts,
                                  int part_keys, float* ws_acc, float* ws_ml, int row_base, hipStream_t s);
+// Prompt steps with the heads' keys and values formed (latent_attention_prompt.hip; bf16, 128 + 64 key dims, 128 value dims):
+// lat[rows, dim] = the cache rows that the step's sequences see, side by side; off [nseq + 1] = where each one's begin. Then, with
+// kv[rows] = [keys of all heads | values of all heads] made of lat's latent part, out[T, heads * 128] from queries q[T, heads * 192];
+// rot_at: column of the rotary key part in lat. `rows` is at least the sum of the sequences' counts.
+bool latent_prompt_ok(int dim, int rot_dim, int vdim);
+void launch_latent_gather(void* lat, int* off, const void* cache, int block_size, int dim, const int* seq_cu, const int* seq_ctx,
+                          const int* seq_bt, int bt_width, int nseq, int rows, int window, hipStream_t s);
+bool launch_latent_prompt(void* out, const void* q, const void* kv, const void* lat, int lat_ld, int rot_at, const int* off, int rows,
+                          const int* seq_cu, const int* seq_ctx, int nseq, int T, const long* positions, const float* inv_freq,
+                          const void* proj, long proj_ld, int heads, int gate_off, bool channel_gate, float scale, int window,
+                          hipStream_t s);
 void launch_latent_attention_reduce(void* o_lat, const float* ws_acc, const float* ws_ml, const void* proj, long proj_ld,
                                     int gate_off, int nparts, int heads, int rows_bound, int row_base, int T, int kv_rank,
                                     hipStream_t s);

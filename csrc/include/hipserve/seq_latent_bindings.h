@@ -119,6 +119,52 @@ inline void latent_attention_mfma(at::Tensor& o_lat, at::Tensor& qc, const c10::
                                          nparts, part_keys, wa, wm, row_base, cur_stream());
 }
 
+inline void latent_gather(at::Tensor& lat, at::Tensor& off, const at::Tensor& cache, const at::Tensor& seq_cu,
+                          const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t window) {
+  CHECK_DEV(cache); CHECK_CONTIG(cache); CHECK_CONTIG(lat); CHECK_I32(off); CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_bt);
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&lat, &off, &seq_cu, &seq_ctx, &seq_bt}) CHECK_SAME_DEV(*t, cache);
+  TORCH_CHECK(cache.scalar_type() == at::kBFloat16 && lat.scalar_type() == at::kBFloat16, "latent_gather: bf16 only");
+  const long nseq = seq_ctx.numel(), block = cache.dim() == 3 ? cache.size(1) : 0;
+  TORCH_CHECK(cache.dim() == 3 && lat.dim() == 2 && lat.size(1) == cache.size(2) && cache.size(2) % 8 == 0 && block > 0 &&
+              (block & (block - 1)) == 0);
+  TORCH_CHECK(seq_cu.numel() == nseq + 1 && off.numel() == nseq + 1 && seq_bt.dim() == 2 && seq_bt.size(0) >= nseq);
+  TORCH_CHECK((uintptr_t)cache.data_ptr() % 16 == 0 && (uintptr_t)lat.data_ptr() % 16 == 0, "latent_gather: alignment");
+  c10::hip::HIPGuardMasqueradingAsCUDA g(cache.device());
+  hipserve::launch_latent_gather(lat.data_ptr(), off.data_ptr<int>(), cache.data_ptr(), block, cache.size(2), seq_cu.data_ptr<int>(),
+                                 seq_ctx.data_ptr<int>(), seq_bt.data_ptr<int>(), seq_bt.size(1), nseq, lat.size(0), window,
+                                 cur_stream());
+}
+
+inline void latent_prompt_attention(at::Tensor& out, const at::Tensor& q, const at::Tensor& kv, const at::Tensor& lat, const at::Tensor& off,
+                                    const at::Tensor& seq_cu, const at::Tensor& seq_ctx, const at::Tensor& positions,
+                                    const at::Tensor& inv_freq, const at::Tensor& proj, int64_t heads, int64_t gate_off,
+                                    bool channel_gate, double scale, int64_t window) {
+  constexpr int D = 128, R = 64;
+  CHECK_DEV(q); CHECK_CONTIG(q); CHECK_CONTIG(out); CHECK_CONTIG(kv); CHECK_CONTIG(lat); CHECK_F32(inv_freq);
+  CHECK_I32(off); CHECK_I32(seq_cu); CHECK_I32(seq_ctx);
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&out, &kv, &lat, &off, &seq_cu, &seq_ctx, &positions, &inv_freq, &proj}) CHECK_SAME_DEV(*t, q);
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&out, &q, &kv, &lat, &proj})
+    TORCH_CHECK(t->scalar_type() == at::kBFloat16 && t->dim() == 2, "latent_prompt_attention: bf16 matrices");
+  const long T = q.size(0), nseq = seq_ctx.numel(), rows = lat.size(0);
+  TORCH_CHECK(heads > 0 && q.size(1) == heads * (D + R) && out.size(0) == T && out.size(1) == heads * D);
+  TORCH_CHECK(kv.size(0) == rows && kv.size(1) == 2 * heads * D && lat.size(1) >= R && lat.size(1) % 8 == 0);
+  TORCH_CHECK(seq_cu.numel() == nseq + 1 && off.numel() == nseq + 1 && inv_freq.numel() == R / 2 && scale > 0);
+  TORCH_CHECK(positions.scalar_type() == at::kLong && positions.is_contiguous() && positions.numel() >= T);
+  TORCH_CHECK(proj.size(0) == T && proj.stride(1) == 1 && (gate_off < 0 || proj.size(1) >= gate_off + heads * (channel_gate ? D : 1)) &&
+              (gate_off >= 0 || !channel_gate));
+  TORCH_CHECK(rows < (1L << 30) && 64L * heads * D * 2 * 2 < (1L << 31) && (T / 64 + nseq) * heads < (1L << 31));   // 32-bit places
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&q, &kv, &lat, &out})
+    TORCH_CHECK((uintptr_t)t->data_ptr() % 16 == 0, "latent_prompt_attention: alignment");
+  c10::hip::HIPGuardMasqueradingAsCUDA g(q.device());
+  TORCH_CHECK(hipserve::launch_latent_prompt(
+                  out.data_ptr(), q.data_ptr(), kv.data_ptr(), lat.data_ptr(), lat.size(1), lat.size(1) - R, off.data_ptr<int>(), rows,
+                  seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), nseq, T, positions.data_ptr<long>(), inv_freq.data_ptr<float>(),
+                  proj.data_ptr(), proj.stride(0), heads, gate_off, channel_gate, (float)scale, window, cur_stream()),
+              "latent attention: no LDS");
+}
+
+inline bool latent_prompt_ok(int64_t dim, int64_t rot_dim, int64_t vdim) { return hipserve::latent_prompt_ok(dim, rot_dim, vdim); }
+
 inline bool latent_attention_dma_ok(int64_t kv_rank, int64_t rot_dim) {
   return hipserve::latent_attention_dma_ok(kv_rank, rot_dim);
 }

@@ -126,6 +126,10 @@ TORCH_LIBRARY(hipserve_cell, m) {
         "Tensor cache, Tensor seq_cu, Tensor seq_ctx, Tensor seq_bt, int seq0, int seq1, int rows_bound, "
         "Tensor inv_freq, int heads, int dim, int rot_dim, int kv_rank, int gate_off, float scale, int window, "
         "int nparts, int part_keys, Tensor(c!)? ws_acc, Tensor(d!)? ws_ml, int row_base, bool fill_qc) -> ()");
+  m.def("latent_gather(Tensor(a!) lat, Tensor(b!) off, Tensor cache, Tensor seq_cu, Tensor seq_ctx, Tensor seq_bt, int window) -> ()");
+  m.def("latent_prompt_attention(Tensor(a!) out, Tensor q, Tensor kv, Tensor lat, Tensor off, Tensor seq_cu, Tensor seq_ctx, "
+        "Tensor positions, Tensor inv_freq, Tensor proj, int heads, int gate_off, bool channel_gate, float scale, int window) -> ()");
+  m.def("latent_prompt_ok(int dim, int rot_dim, int vdim) -> bool", &latent_prompt_ok);
   m.def("latent_attention_dma_ok(int kv_rank, int rot_dim) -> bool", &latent_attention_dma_ok);
   m.def("latent_attention_mfma_ok(int kv_rank, int rot_dim) -> bool", &latent_attention_mfma_ok);
 }
@@ -139,4 +143,6 @@ TORCH_LIBRARY_IMPL(hipserve_cell, CUDA, m) {
   m.impl("latent_prepare", &latent_prepare);
   m.impl("latent_attention", &latent_attention);
   m.impl("latent_attention_mfma", &latent_attention_mfma);
+  m.impl("latent_gather", &latent_gather);
+  m.impl("latent_prompt_attention", &latent_prompt_attention);
 }

@@ -12,7 +12,8 @@ over the heads; everything between them is one op of the op set:
   up-projection -> per-head absorption of the key up-projection into the query (so the
   attention runs directly on the cached latents, one shared "key head" for all heads) ->
   ``latent_attention`` (rotary query part, sliding window, softmax, output gate) ->
-  per-head value up-projection -> output projection.
+  per-head value up-projection -> output projection. In bf16 prompt steps the keys and values of every head are formed
+  instead, one product over the cache rows that the step sees, and attended to (``latent_prompt_attention``).
 * minGRU: merged [z | x | g] projection -> ``mingru_scan`` (gates, candidate, the
   recurrence over this step's tokens from the sequence's state slot, output gate) ->
   output projection.
@@ -130,6 +131,7 @@ class LatentAttention:
         self.q_norm = None     # [q_rank] fp32
         self.kv_norm = None    # [kv_rank] fp32
         self.w_uq = None       # [heads * (dim + rot_dim), q_rank]
+        self.w_kv = None       # [heads * dim + heads * vdim, kv_rank]: w_uk and w_uv are parts of it
         self.w_uk = None       # [heads, dim, kv_rank]
         # the same for kernels that take the absorbed queries in place:
         self.w_uk_wide = None  # [heads, dim, kv_rank + rot_dim], zero rotary columns
@@ -157,10 +159,11 @@ class LatentAttention:
         self.q_norm = get(prefix + "dq.norm").to(dev, torch.float32)
         self.kv_norm = get(prefix + "dkv.norm").to(dev, torch.float32)
         self.w_uq = uq.to(dev, dt).contiguous()
-        self.w_uk = get(prefix + "uk").to(dev, dt).view(s.heads, s.dim, s.kv_rank).contiguous()
+        self.w_kv = torch.cat([get(prefix + "uk"), get(prefix + "uv")], 0).to(dev, dt).contiguous()
+        self.w_uk = self.w_kv[: s.heads * s.dim].view(s.heads, s.dim, s.kv_rank)
         if self.ops.latent_query_in_place(dt, s.kv_rank, s.rot_dim):
             self._lay_out_queries()
-        self.w_uv = get(prefix + "uv").to(dev, dt).view(s.heads, s.vdim, s.kv_rank).contiguous()
+        self.w_uv = self.w_kv[s.heads * s.dim:].view(s.heads, s.vdim, s.kv_rank)
         self.w_uv_t = self.w_uv.transpose(1, 2).contiguous()
         self.w_o = get(prefix + "o").to(dev, dt).contiguous()
 
@@ -198,6 +201,12 @@ class LatentAttention:
         ops.latent_prepare(cq, cache, proj, meta.positions, meta.slot_mapping, self.q_norm, self.kv_norm,
                            self.inv_freq, s.q_rank, s.kv_rank, s.rot_dim, self.eps)
         q = self.ops.linear(cq, self.w_uq)                             # [T, heads * (dim + rot_dim)]
+        rows = ops.latent_prompt_rows(h.dtype, s, self.inv_freq.numel(), cache, meta, T)
+        if rows:   # a prompt step: every head's keys and values are formed
+            cat = torch.empty(T, s.heads * s.vdim, device=h.device, dtype=h.dtype)
+            ops.latent_prompt_attention(cat, q, proj, cache, meta, self.inv_freq, s, self.w_kv, rows,
+                                        -1 if s.gate == "none" else gate_off)
+            return ops.linear(cat, self.w_o)
         qh = q.view(T, s.heads, s.dim + s.rot_dim)
         if ops.latent_query_in_place(h.dtype, s.kv_rank, s.rot_dim):
             # the absorption GEMM writes the attention kernel's query rows directly: bf16, the cached width,

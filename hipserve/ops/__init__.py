@@ -246,6 +246,33 @@ class KernelOps:
         ([heads, T, kv_rank + rot_dim], the rotary part left for it to fill) instead of fp32 [heads, T, kv_rank]."""
         return dtype == torch.bfloat16 and self.LATENT_MFMA and bool(self._latent_lib.latent_attention_mfma_ok(kv_rank, rot_dim))
 
+    # up to 64 rows the heads' products with W_uk and W_uv run the kernel for a few rows and the latents are faster (33 rows, one
+    # mixer, width 2048: 67 us and 74); from there on forming the keys is: 96 rows 105 and 163
+    LATENT_PROMPT_MIN_ROWS = 65
+
+    def latent_prompt_rows(self, dtype, sp, nfreq, cache, meta, T) -> int:
+        """Where the heads' keys and values of a step are formed (``latent_prompt_attention``): an upper bound of the cache rows
+        that its sequences see; 0 where the attention on the latents is the one to run: steps with decode rows, and steps that
+        see more than two cache rows per token, whose keys and values cost more than they save."""
+        if not (dtype == torch.bfloat16 and self.LATENT_MFMA and sp.scale > 0 and T >= self.LATENT_PROMPT_MIN_ROWS and meta.num_decode == 0
+                and nfreq == 32 and cache.shape[1] & (cache.shape[1] - 1) == 0 and cache.data_ptr() % 16 == 0 and sp.key_dim % 8 == 0
+                and getattr(meta, "max_q", None) and getattr(meta, "max_ctx", None) and self._latent_lib.latent_prompt_ok(sp.dim, sp.rot_dim, sp.vdim)):
+            return 0
+        rows = meta.seq_ctx.shape[0] * min(meta.max_ctx, meta.max_q + sp.window - 1 if sp.window > 0 else meta.max_ctx)
+        return rows if rows <= 2 * T else 0
+
+    def latent_prompt_attention(self, out, q, proj, cache, meta, inv_freq, sp, w_kv, rows, gate_off):
+        """out [T, heads * vdim] of a prompt step: the ``rows`` cache rows its sequences see times ``w_kv`` (keys of all heads, values
+        of all heads), then attention of every head on its own keys and the shared rotary part."""
+        lib = self._latent_lib
+        lat = torch.empty(rows, sp.key_dim, device=q.device, dtype=q.dtype)
+        off = torch.empty(meta.seq_ctx.shape[0] + 1, device=q.device, dtype=torch.int32)
+        lib.latent_gather(lat, off, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt, sp.window)
+        kv = F.linear(lat[:, :sp.kv_rank], w_kv)
+        lib.latent_prompt_attention(out, q, kv, lat, off, meta.seq_cu, meta.seq_ctx, meta.positions, inv_freq, proj, sp.heads, gate_off,
+                                    sp.gate == "channel", sp.scale, sp.window)
+        return out
+
     def latent_attention(self, o_lat, q_abs, q, proj, cache, meta, inv_freq, heads, dim, rot_dim, kv_rank,
                          gate_off, scale, window):
         """Prompt portions (the step's first sequences) run several tokens per workgroup, decode
@@ -764,6 +791,9 @@ class ReferenceOps:
 
     def latent_query_in_place(self, dtype, kv_rank, rot_dim) -> bool:
         return False
+
+    def latent_prompt_rows(self, dtype, sp, nfreq, cache, meta, T) -> int:
+        return 0
 
     def mingru_scan(self, y, state, proj, b_z, b_x, meta):
         ref.mingru_scan(y, state, proj, b_z, b_x, meta.seq_cu, meta.seq_ctx, meta.seq_state)

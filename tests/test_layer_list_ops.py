@@ -327,6 +327,52 @@ def test_latent_attention_dma(kv, heads, window, lens, ctxs, nd):
     assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
 
 
+@gpu
+@pytest.mark.parametrize("heads,gate,window,lens,ctxs", [
+    (3, "head", 0, [130], [130]), (4, "head", 50, [70, 1, 33, 200], [70, 9, 64, 331]), (2, "channel", 33, [31, 128, 129], [31, 128, 400]),
+    (2, "none", 0, [3] * 70, [5] * 70), (16, "head", 64, [2000, 0, 2097], [2000, 0, 2100]), (1, "head", 1, [65, 64], [65, 80])])
+def test_latent_prompt_attention(heads, gate, window, lens, ctxs):
+    """Cache rows side by side (all that a window shows, sequences without rows, more sequences than lanes), and attention to formed
+    keys and values: tiles filled partly, waves that leave tiles out, both row counts per wave, in 64 bits."""
+    D, rot, kv, block, scale = 128, 64, 32, 16, 0.07
+    dim = kv + rot
+    cache, cu, pos, bt, _, _, _, meta = latent_case(lens, ctxs, heads, D, kv, rot, block, torch.bfloat16, "cuda", heads + window)
+    lib, g, T = get_ops("cuda")._latent_lib, torch.Generator().manual_seed(window), sum(lens)
+    seen = [ctx - max(0, ctx - n - window + 1 if window else 0) if n else 0 for n, ctx in zip(lens, ctxs)]
+    rows = sum(seen) + 5
+    lat = torch.zeros(rows, dim, dtype=torch.bfloat16, device="cuda")
+    off = torch.empty(len(lens) + 1, dtype=torch.int32, device="cuda")
+    lib.latent_gather(lat, off, cache.cuda(), meta.seq_cu, meta.seq_ctx, meta.seq_bt, window)
+    assert off.tolist() == [sum(seen[:i]) for i in range(len(lens) + 1)]
+    q, kvs = torch.randn(T, heads * (D + rot), generator=g).bfloat16(), torch.randn(rows, 2 * heads * D, generator=g).bfloat16()
+    proj = torch.randn(T, 8 + heads * D, generator=g).bfloat16()
+    inv = torch.pow(torch.tensor(1e4), -2.0 * torch.arange(rot // 2) / rot)
+    out = torch.full((T, heads * D), float("nan"), dtype=torch.bfloat16, device="cuda")
+    lib.latent_prompt_attention(out, q.cuda(), kvs.cuda(), lat, off, meta.seq_cu, meta.seq_ctx, pos.cuda(), inv.cuda(), proj.cuda(), heads,
+                                -1 if gate == "none" else 8, gate == "channel", scale, window)
+    qh = q.double().view(T, heads, D + rot)
+    ang = pos.double()[:, None] * inv.double()
+    c, s, r = torch.cos(ang)[:, None], torch.sin(ang)[:, None], qh[..., D:]
+    qr = torch.cat([r[..., :32] * c - r[..., 32:] * s, r[..., 32:] * c + r[..., :32] * s], -1).bfloat16().double()
+    qh, lat = torch.cat([qh[..., :D], qr], -1), lat.cpu()
+    want = torch.empty(T, heads, D, dtype=torch.float64)
+    for i, (n, ctx) in enumerate(zip(lens, ctxs)):
+        j, at = torch.arange(ctx - seen[i], ctx), slice(sum(seen[:i]), sum(seen[:i + 1]))
+        assert torch.equal(lat[at], cache[bt[i, j // block].long(), j % block])
+        k, v = kvs[at].double().view(-1, 2, heads, D).unbind(1)
+        k = torch.cat([k, lat[at, None, kv:].double().expand(-1, heads, -1)], -1)
+        mine = slice(int(cu[i]), int(cu[i]) + n)
+        back = pos[mine, None] - j
+        for h in range(heads):
+            sc = (qh[mine, h] @ k[:, h].T * scale).masked_fill((back < 0) | (back >= window if window else back < 0), -float("inf"))
+            want[mine, h] = torch.softmax(sc, -1) @ v[:, h]
+    if gate != "none":
+        gates = torch.sigmoid(proj[:, 8:8 + heads * (D if gate == "channel" else 1)].double()).view(T, heads, -1)
+        want *= gates
+    # weights and outputs are rounded to bf16; a score is a sum of 192 products, exact to 2^-16 or so, before the exponential
+    assert ((out.double().cpu().view(T, heads, D) - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * kvs.double().abs().max() * 0.5).all()
+
+
 def test_latent_weights_are_laid_out_at_load():
     from types import SimpleNamespace
 
