@@ -181,3 +181,34 @@ def test_moe_align_layout(T, k, E, tile):
     for e in range(E):
         want_te[int(off[e]) // tile:int(off[e] + padded[e]) // tile] = e
     assert torch.equal(te, want_te)
+
+
+@pytest.mark.parametrize("tiles,N,K,epi", [(66, 2048, 1536, 4), (65, 2000, 1792, 0), (35, 1024, 2048, 2), (16, 2048, 1536, 4), (300, 512, 1536, 0),
+                                                 (100, 512, 1536, 4), (66, 2048, 1280, 0)])
+@pytest.mark.parametrize("gather", [False, True])
+def test_packed_grouped_left_over(tiles, N, K, epi, gather):
+    """Tiles that whole rounds leave over (quarters of K per wave, their sums in LDS): some, all, too many; a weight tile cut off; odd
+    counts of stages per wave; padding rows; K that is too short."""
+    g, op, E, M = torch.Generator(device=DEV).manual_seed(tiles + N), torch.ops.hipserve, 3, tiles * 128
+    w, x = _rnd(g, E, N, K, scale=0.05), _rnd(g, M // 2, K)
+    wp = torch.stack([_pack(w[e], epi == 2) for e in range(E)])
+    tile_expert = torch.randint(0, E, (tiles + 2,), device=DEV, generator=g, dtype=torch.int32)
+    ntiles = torch.tensor([tiles], dtype=torch.int32, device=DEV)
+    slots = torch.randperm(M + 256, device=DEV, generator=g).int()
+    slots[(slots >= M) | (slots % 97 == 5)] = -1
+    No = N // 2 if epi == 2 else N
+    out = torch.full((M + 256, No), 7.0, device=DEV, dtype=torch.bfloat16)
+    rows = torch.where((slots >= 0)[:, None], x[(slots.clamp(min=0) // 2).long()], 0.0).bfloat16()
+    if gather:
+        op.prefill_gemm_packed_grouped(out, x, wp, N, epi, tile_expert, ntiles, 1, 4, slots, 2)
+    else:
+        op.prefill_gemm_packed_grouped(out, rows, wp, N, epi, tile_expert, ntiles, 1)
+    assert bool((out[M:] == 7.0).all())   # past the counted tiles nothing is written
+    for e in range(E):
+        mine = (tile_expert[:tiles] == e).repeat_interleave(128).nonzero()[:, 0]
+        h = rows[mine].double() @ w[e].double().t()
+        want = h.clamp(min=0).square() if epi == 4 else torch.nn.functional.silu(h[:, :No]) * h[:, No:] if epi == 2 else h
+        # sums of K products in 32 bits and the result's rounding. In the gate three more: of the gate (which silu takes up at most
+        # threefold for gates above -3), of silu and of the up projection: 6 x 2^-9
+        rel = 2.0 ** -6 if epi == 2 else 2.0 ** -7
+        assert ((out[mine].double() - want).abs() <= rel * want.abs() + 2.0 ** -9 * want.abs().mean()).all()
