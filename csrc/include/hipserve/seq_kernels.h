@@ -18,10 +18,10 @@ void launch_scaled_add_group_rmsnorm(void* out, float* residual, const float* w,
 
 // out[b, m, n] = act(x[b, m] . W[b, n] + bias[n]) of up to 64 rows m (skinny_linear.hip): bf16 operands, K % 8 == 0, x rows at
 // multiples of 16 bytes; W [batch, N, K]; act 0 tanh, 1 xIELU, 2 relu^2, 3 SiLU gate, 4 clamped gate (N / 2 columns),
-// 5 soft cap, -1 none.
+// 5 soft cap, -1 none; on the columns from act_from on.
 bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs,
-                          const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, float c0, float c1,
-                          hipStream_t s);
+                          const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0,
+                          float c1, hipStream_t s);
 
 // proj[T, ld] rows = [q latent (q_rank) | kv latent (kv_rank) | rotary key (rot_dim) | ...]:
 // cq[T, q_rank] = RMSNorm(q latent) * q_norm; cache row slots[t] (>= 0) = [RMSNorm(kv latent) * kv_norm |

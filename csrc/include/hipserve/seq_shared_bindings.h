@@ -102,7 +102,7 @@ inline bool expert_gemm_skinny(int64_t pairs, int64_t ntiles_cap, int64_t N, int
 
 // out = act(x . w^T + bias) of at most 64 rows: x [M, K] or [B, M, K], w [N, K] or [B, N, K], out [M, N'] or [B, M, N'].
 inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias,
-                          int64_t act, double c0, double c1) {
+                          int64_t act, double c0, double c1, int64_t act_from) {
   CHECK_DEV(x); CHECK_CONTIG(w); CHECK_SAME_DEV(w, x); CHECK_SAME_DEV(out, x);
   if (bias.has_value()) CHECK_SAME_DEV(*bias, x);
   const bool f32 = x.scalar_type() == at::kFloat;
@@ -116,6 +116,7 @@ inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor
               N < (1L << 31) && K < (1L << 24) && x.stride(-2) < (1L << 24) && B < 65536, "skinny_linear: shapes");
   const bool glu = act == 3 || act == 4;
   TORCH_CHECK(act >= -1 && act <= 5 && (!glu || N % 2 == 0) && out.size(-1) == (glu ? N / 2 : N), "skinny_linear: activation");
+  TORCH_CHECK(act_from >= 0 && act_from <= N && (act_from == 0 || !glu), "skinny_linear: first column of the activation");
   auto aligned = [](const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
   TORCH_CHECK(x.stride(-1) == 1 && out.stride(-1) == 1 && x.stride(-2) % per == 0 && (d == 2 || x.stride(0) % per == 0) && aligned(x) &&
               aligned(w), "skinny_linear: rows at multiples of 16 bytes");
@@ -124,11 +125,11 @@ inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   TORCH_CHECK(hipserve::launch_skinny_linear(out.data_ptr(), out.scalar_type() == at::kFloat, out.stride(-2), d == 3 ? out.stride(0) : 0,
                                              x.data_ptr(), x.stride(-2), d == 3 ? x.stride(0) : 0, w.data_ptr(), opt_ptr(bias), f32, B,
-                                             M, N, K, act, (float)c0, (float)c1, cur_stream()), "skinny_linear: LDS");
+                                             M, N, K, act, act_from, (float)c0, (float)c1, cur_stream()), "skinny_linear: LDS");
 }
 
 inline void def_moe_ops(torch::Library& m) {
-  m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int act, float c0, float c1) -> ()");
+  m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int act, float c0, float c1, int act_from=0) -> ()");
   m.def("moe_align(Tensor ids, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, Tensor(c!) pair_slot) -> ()");
   m.def("moe_table_align(Tensor table, Tensor tokens, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, "
         "Tensor(c!) pair_slot) -> ()");

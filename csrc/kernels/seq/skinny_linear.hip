@@ -1,7 +1,7 @@
 // out[b, m, :] = act(x[b, m, :] . W[b]^T + bias) for up to 64 rows m (decode steps and short prompts): bf16 or 32-bit
 // operands, 32-bit accumulation, a result of the operands' type or in 32 bits, row and batch strides of their own for x and out.
 // act: 0 tanh, 1 xIELU, 2 squared ReLU, 3 SiLU gate, 4 clamped gate (3, 4: W = [gate rows; up rows], half as many
-// columns in out), 5 soft cap, -1 none; they see the unrounded product.
+// columns in out), 5 soft cap, -1 none; they see the unrounded product. act_from: the first column that it applies to (not for gates).
 #include "skinny.h"
 
 #include <algorithm>
@@ -26,7 +26,7 @@ HS_DEVICE float skinny_act(float z, int act, float c0, float c1) {
 template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32>
 __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
     TO* __restrict__ out, long out_ld, long out_bs, const unsigned short* __restrict__ x, long x_ld, long x_bs,
-    const unsigned short* __restrict__ w, const void* __restrict__ bias_, int M, int N, int K, int act, float c0, float c1) {
+    const unsigned short* __restrict__ w, const void* __restrict__ bias_, int M, int N, int K, int act, int act_from, float c0, float c1) {
   static_assert(!GLU || NT == 2, "a gate tile and an up tile");
   using SK = Skinny<XG, NT, DEPTH, F32>;
   constexpr int ST = SK::ST;
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
         const int n = n0 + 16 * nt + (e & 15);
         if (n >= N) continue;
         const float z = v[nt][i] + (bias != nullptr ? ldf<TB>(bias, n) : 0.f);
-        stf<TO>(out, m * out_ld + n, skinny_act(z, act, c0, c1));
+        stf<TO>(out, m * out_ld + n, skinny_act(z, n >= act_from ? act : -1, c0, c1));
       }
     }
   }
@@ -83,21 +83,21 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
 
 template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32>
 bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, const void* x, long x_ld, long x_bs, const void* w, const void* bias,
-                   int M, int N, int K, int act, float c0, float c1, hipStream_t s) {
+                   int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
   constexpr int lds = Skinny<XG, NT, DEPTH, F32>::kLds;
   static const bool ok = allow_lds(&skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32>, lds);
   if (!ok) return false;
   skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32><<<grid, kSkThreads, lds, s>>>(
-      (TO*)out, out_ld, out_bs, (const unsigned short*)x, x_ld, x_bs, (const unsigned short*)w, bias, M, N, K, act, c0, c1);
+      (TO*)out, out_ld, out_bs, (const unsigned short*)x, x_ld, x_bs, (const unsigned short*)w, bias, M, N, K, act, act_from, c0, c1);
   return true;
 }
 
 template <int XG, int NT, int DEPTH, bool GLU>
 bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs, const void* w,
-                const void* bias, bool f32, int batch, int M, int N, int K, int act, float c0, float c1, hipStream_t s) {
+                const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
   const int cols = GLU ? N / 2 : N, per = GLU ? 16 : 16 * NT;
   const dim3 grid((cols + per - 1) / per, batch);
-#define HS_SK(TO, F32) launch_kernel<XG, NT, DEPTH, GLU, TO, F32>(grid, out, out_ld, out_bs, x, x_ld, x_bs, w, bias, M, N, K, act, c0, c1, s)
+#define HS_SK(TO, F32) launch_kernel<XG, NT, DEPTH, GLU, TO, F32>(grid, out, out_ld, out_bs, x, x_ld, x_bs, w, bias, M, N, K, act, act_from, c0, c1, s)
   return f32 ? HS_SK(float, true) : out_f32 ? HS_SK(float, false) : HS_SK(unsigned short, false);
 #undef HS_SK
 }
@@ -115,11 +115,11 @@ double skinny_time(int M, long cols, int K, int nt) {
 }  // namespace
 
 bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs,
-                          const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, float c0, float c1,
+                          const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1,
                           hipStream_t s) {
   if (batch <= 0 || M <= 0 || N <= 0) return true;
   if (f32) { x_ld *= 2; x_bs *= 2; K *= 2; }   // in halves
-#define HS_SK(XG, NT, DEPTH, GLU)   launch_one<XG, NT, DEPTH, GLU>(out, out_f32, out_ld, out_bs, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, c0, c1, s)
+#define HS_SK(XG, NT, DEPTH, GLU)   launch_one<XG, NT, DEPTH, GLU>(out, out_f32, out_ld, out_bs, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, act_from, c0, c1, s)
   const int xg = (M + 7) / 8;
   if (act == 3 || act == 4)
     return xg <= 1 ? HS_SK(1, 2, 1, true) : xg <= 2 ? HS_SK(2, 2, 1, true) : xg <= 4 ? HS_SK(4, 2, 1, true)

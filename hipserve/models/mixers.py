@@ -41,7 +41,7 @@ over the heads; everything between them is one op of the op set:
   bottleneck | gate bottleneck | beta] and the up-projections follow as GEMMs (the decay's with a
   32-bit result); steps in which every sequence brings one row run ``gated_delta_step`` instead, the
   bottlenecks' up-projections included.
-* generalized delta rule: merged [r | k | v | a | g | decay bottleneck] projection -> tanh ->
+* generalized delta rule: merged [r | k | v | a | g | decay bottleneck] projection, tanh of the last part ->
   decay up-projection (32-bit result) -> ``delta_rule`` (decay, removal rate, unit key, the
   recurrence, per-head output norm and sigmoid gate) -> output projection.
 * linear attention with fixed decays (``Lightning``): merged [q | k | v | gate] projection ->
@@ -656,10 +656,8 @@ class DeltaRule:
 
     def mix(self, h, meta, cache, state, out, out_scale: float = 1.0):
         N, ops = self.spec.size, self.ops
-        proj = self.ops.linear(h, self.w_in)
-        low = torch.empty(h.shape[0], self.w2.shape[1], device=h.device, dtype=h.dtype)
-        ops.activation(low, proj[:, 5 * N:], "tanh")
-        wl = self.ops.linear(low, self.w2, out_f32=True)
+        proj = ops.linear(h, self.w_in, act="tanh", act_from=5 * N)
+        wl = ops.linear(proj[:, 5 * N:], self.w2, out_f32=True)
         ops.delta_rule(out, state, proj, wl, self.a_b, self.w0, self.norm, self.spec, self.eps, meta, out_scale)
         return out
 

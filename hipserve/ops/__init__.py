@@ -486,15 +486,16 @@ class KernelOps:
                 and x.shape[-1] % per == 0 and max(x.shape[-1], x.stride(-2)) < 1 << 24 and x.stride(-1) == 1 and x.stride(-2) % per == 0 and x.stride(0) % per == 0
                 and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
 
-    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0):
-        """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands. A few rows run the
-        weight-streaming kernel with the activation in its epilogue, anything else the vendor's GEMM and a second launch."""
+    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0):
+        """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands; ``act_from``: the first column that
+        the activation applies to. A few rows run the weight-streaming kernel with the activation in its epilogue, anything else the
+        vendor's GEMM and a second launch."""
         if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())):
             glu = act in self.GLU_ACTS
             T, N, K = x.shape[0], w.shape[0], w.shape[1]
             if self.skinny_pays(T, N, K, glu, x.dtype == torch.float32):
                 out = torch.empty(T, N // 2 if glu else N, device=x.device, dtype=torch.float32 if out_f32 else x.dtype)
-                self._moe_lib.skinny_linear(out, x, w, bias, -1 if act is None else self.ACTIVATIONS[act], c0, c1)
+                self._moe_lib.skinny_linear(out, x, w, bias, -1 if act is None else self.ACTIVATIONS[act], c0, c1, act_from)
                 return out
         if out_f32 and x.dtype != torch.float32:
             y = torch.mm(x, w.t(), out_dtype=torch.float32)
@@ -503,6 +504,9 @@ class KernelOps:
         else:
             y = F.linear(x, w, bias)
         if act is None:
+            return y
+        if act_from:
+            self.activation(y[:, act_from:], y[:, act_from:], act, c0, c1)
             return y
         out = torch.empty(*y.shape[:-1], y.shape[-1] // 2, device=y.device, dtype=y.dtype) if act in self.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)
@@ -881,11 +885,14 @@ class ReferenceOps:
         ref.delta_rule(out, state[0], proj, wl, a_b, w0, norm_w, sp, eps, meta.seq_cu, meta.seq_ctx,
                        meta.seq_state, out_scale)
 
-    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0):
+    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0):
         if out_f32 and x.dtype != torch.float32:
             x, w, bias = x.float(), w.float(), None if bias is None else bias.float()
         y = F.linear(x, w, bias)
         if act is None:
+            return y
+        if act_from:
+            self.activation(y[:, act_from:], y[:, act_from:], act, c0, c1)
             return y
         out = y.new_empty(*y.shape[:-1], y.shape[-1] // 2) if act in KernelOps.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)

@@ -132,6 +132,19 @@ def test_skinny_linear(M, N, K):
     close_to(half, want + bias.double(), x, w)
 
 
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("M", [1, 17, 70])
+@pytest.mark.parametrize("first", [1, 16, 39])
+def test_linear_activation_of_last_columns(dev, M, first):
+    (x,), (w,) = dense_case(1, M, 40, 64, M + first)
+    w = w * 4
+    got = get_ops(dev).linear(x.to(dev), w.to(dev), act="tanh", act_from=first)
+    want = x.double() @ w.double().T
+    want[:, first:] = torch.tanh(want[:, first:])
+    # past 64 rows the product is rounded before the activation
+    assert ((got.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 1e-3).all()
+
+
 @gpu
 @pytest.mark.parametrize("M", [8, 9, 24, 25, 40, 41, 64])
 @pytest.mark.parametrize("N", [4113, 5001, 12301])
