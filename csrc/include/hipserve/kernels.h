@@ -266,8 +266,9 @@ void launch_moe_topk_softmax(const void* logits, bool logits_f32, float* w, int*
 void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
                       int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s,
                       int* hist = nullptr);
-// the same for the pairs (t, j), expert table[tokens[t]][j] of a [table_rows, top] table: one workgroup, small batches
-void launch_moe_table_align(const int* table, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
+// the same for the pairs (t, j), expert table[i][tokens[t]][j] of `tables` tables [table_rows, top], outputs side by side (num_tiles
+// [tables]): a workgroup each, small batches
+void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
                             int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot,
                             hipStream_t s);
 // blocks of the multi-workgroup moe_align for npairs (1: the single-workgroup kernel);

@@ -47,24 +47,27 @@ inline void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor
                              stream, nb > 1 ? scratch.data_ptr<int>() : nullptr);
 }
 
-// moe_align of the pairs (t, j) whose expert is table[tokens[t]][j].
+// moe_align of the pairs (t, j) whose expert is table[tokens[t]][j], table [rows, top]; or of every table of [L, rows, top], with outputs
+// [L, slots], [L, tiles], [L, pairs].
 inline void moe_table_align(const at::Tensor& table, const at::Tensor& tokens, int64_t E, int64_t tile, at::Tensor& slots,
                             at::Tensor& tile_expert, at::Tensor& pair_slot) {
   CHECK_DEV(table); CHECK_I32(table); CHECK_I32(slots); CHECK_I32(tile_expert); CHECK_I32(pair_slot);
-  CHECK_SAME_DEV(tokens, table);
-  TORCH_CHECK(table.dim() == 2 && table.size(0) >= 1 && tokens.scalar_type() == at::kLong && tokens.is_contiguous());
+  CHECK_SAME_DEV(tokens, table); CHECK_SAME_DEV(slots, table); CHECK_SAME_DEV(tile_expert, table); CHECK_SAME_DEV(pair_slot, table);
+  const long d = table.dim(), L = d == 3 ? table.size(0) : 1;
+  TORCH_CHECK((d == 2 || d == 3) && L >= 1 && table.size(d - 2) >= 1 && tokens.scalar_type() == at::kLong && tokens.is_contiguous());
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&slots, &tile_expert, &pair_slot})
+    TORCH_CHECK(d == 2 || (t->dim() == 2 && t->size(0) == L), "moe_table_align: a row of outputs per table");
   TORCH_CHECK(E >= 1 && E <= 128, "moe_align: at most 128 experts");
   TORCH_CHECK(tile == 16 || tile == 32 || tile == 64 || tile == 128 || tile == 256);
-  const long top = table.size(1), npairs = tokens.numel() * top;
+  const long top = table.size(d - 1), npairs = tokens.numel() * top, cap = slots.numel() / L, tiles = tile_expert.numel() / L;
   TORCH_CHECK(top >= 1 && hipserve::moe_align_blocks(npairs) == 1, "moe_table_align: small batches");
-  TORCH_CHECK(slots.numel() >= npairs + E * (tile - 1) && slots.numel() % tile == 0,
-              "slots capacity must cover padding and be a multiple of the tile");
-  TORCH_CHECK(tile_expert.numel() * tile >= slots.numel() && pair_slot.numel() >= npairs);
+  TORCH_CHECK(cap >= npairs + E * (tile - 1) && cap % tile == 0, "slots capacity must cover padding and be a multiple of the tile");
+  TORCH_CHECK(tiles * tile >= cap && pair_slot.numel() / L >= npairs && (d == 2 || pair_slot.size(1) == npairs));
   c10::hip::HIPGuardMasqueradingAsCUDA g(table.device());
-  at::Tensor count = at::empty({1}, slots.options());
-  hipserve::launch_moe_table_align(table.data_ptr<int>(), tokens.data_ptr<long>(), top, table.size(0), npairs, E, tile,
-                                   slots.data_ptr<int>(), slots.numel(), tile_expert.data_ptr<int>(), tile_expert.numel(),
-                                   count.data_ptr<int>(), pair_slot.data_ptr<int>(), cur_stream());
+  at::Tensor count = at::empty({L}, slots.options());
+  hipserve::launch_moe_table_align(table.data_ptr<int>(), L, tokens.data_ptr<long>(), top, table.size(d - 2), npairs, E, tile,
+                                   slots.data_ptr<int>(), cap, tile_expert.data_ptr<int>(), tiles, count.data_ptr<int>(),
+                                   pair_slot.data_ptr<int>(), cur_stream());
 }
 
 inline bool moe_align_small(int64_t npairs) { return hipserve::moe_align_blocks(npairs) == 1; }

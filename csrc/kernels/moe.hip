@@ -89,7 +89,8 @@ __global__ __launch_bounds__(256) void moe_topk_softmax_kernel(const T* __restri
 }
 
 // table (may be null): the experts come from table[tokens[t]][j] (top of them per token) instead of ids, without a
-// launch of its own for the lookup (4.5 us); a token outside the table counts as its first entry.
+// launch of its own for the lookup (4.5 us); a token outside the table counts as its first entry. Workgroup b serves table b of as many
+// (decode steps: the tables of all layers in one launch, 3.3 - 4.4 us instead of that for each).
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, const int* __restrict__ table,
                                                          const long* __restrict__ tokens, int top, long table_rows,
                                                          int npairs, int E, int tile,
@@ -99,6 +100,12 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
                                                          int* __restrict__ group_end) {
   __shared__ int cnt[128], off[129], cur[128];
   const int tid = threadIdx.x, lane = tid & 63;
+  const long b = blockIdx.x;
+  if (table != nullptr) table += b * table_rows * top;
+  slots += b * slots_cap;
+  tile_expert += b * tiles_cap;
+  pair_slot += b * npairs;
+  num_tiles += b;
   auto expert_of = [&](int p) {
     if (table == nullptr) return ids[p];
     const long t = tokens[p / top];
@@ -469,10 +476,10 @@ void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, i
                                       num_tiles, pair_slot, group_end);
 }
 
-void launch_moe_table_align(const int* table, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
+void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
                             int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot,
                             hipStream_t s) {
-  moe_align_kernel<<<1, 1024, 0, s>>>(nullptr, table, tokens, top, table_rows, npairs, E, tile, slots, slots_cap, tile_expert,
+  moe_align_kernel<<<tables, 1024, 0, s>>>(nullptr, table, tokens, top, table_rows, npairs, E, tile, slots, slots_cap, tile_expert,
                                       tiles_cap, num_tiles, pair_slot, nullptr);
 }
 

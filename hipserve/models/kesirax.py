@@ -66,6 +66,7 @@ class KesiraxModel:
                 lw.mlp = TableMoE(spec.mlp, H, cfg.vocab_size, self.device, dtype, ops)
             self.layers.append(lw)
         self.embed = self.final_norm = self.lm_head = None
+        self.tables = None   # the expert tables of all layers, where they are of one size
         self.capture = None  # a list: the residual stream after every layer run is appended (debugging)
 
     # ---------------------------------------------------------------- weights
@@ -87,6 +88,7 @@ class KesiraxModel:
             if lw.mlp is not None:
                 lw.ls2 = get(f"l{i}.ls2").to(dev, torch.float32)
                 lw.mlp.load(get, f"l{i}.mlp.")
+        self.tables = TableMoE.stack([lw.mlp for lw in self.layers if lw.mlp is not None])
 
     def random_tensors(self, seed: int = 0, std: float = 0.05) -> dict:
         """Random checkpoint tensors (bf16-representable values) under the checkpoint's names."""
@@ -175,6 +177,9 @@ class KesiraxModel:
         # the first norm reads the embedding table itself
         ops.scaled_add_group_rmsnorm(h, residual, first.norm if first else self.final_norm, cfg.norm_groups, cfg.norm_eps,
                                      table=self.embed, ids=ids.long().contiguous())
+        experts = [i for i, lw in enumerate(self.layers) if lw.mlp is not None]
+        aligned = TableMoE.align([self.layers[i].mlp for i in experts], self.tables, h, ids) if self.tables is not None and T else None
+        aligned = dict(zip(experts, aligned)) if aligned is not None else {}
         for r, (i, _, _) in enumerate(self.runs):
             lw = self.layers[i]
             if isinstance(lw.mixer, LatentAttention):
@@ -184,7 +189,7 @@ class KesiraxModel:
             y = pair_slot = None
             top = 0
             if lw.mlp is not None:
-                y, pair_slot = lw.mlp.forward(h, ids)
+                y, pair_slot = lw.mlp.forward(h, ids, aligned.get(i))
                 top = lw.mlp.spec.top
             last = r + 1 == len(self.runs)
             nxt = self.final_norm if last else self.layers[self.runs[r + 1][0]].norm

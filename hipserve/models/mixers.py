@@ -17,7 +17,7 @@ over the heads; everything between them is one op of the op set:
 * minGRU: merged [z | x | g] projection -> ``mingru_scan`` (gates, candidate, the
   recurrence over this step's tokens from the sequence's state slot, output gate) ->
   output projection.
-* table MoE: expert ids looked up by token id -> ``moe_align`` tiles -> two
+* table MoE: expert ids looked up by token id -> ``moe_align`` tiles (of all layers at once in small steps) -> two
   ``expert_gemm`` launches (squared-ReLU in the first one's epilogue); the weighted
   combine is folded into the residual update (``scaled_add_group_rmsnorm``).
 * window attention: merged [q | k | v | gate] projection (biases in its epilogue) ->
@@ -295,18 +295,47 @@ class TableMoE:
         self.load(lambda k: t[k], "")
         return t
 
-    def forward(self, h: torch.Tensor, ids: torch.Tensor):
+    def _tables(self, P: int, dev, *layers):
+        """The tile of an expert GEMM over P pairs and empty (slots, tile_expert, pair_slot), a row per layer where they are given."""
+        E = self.spec.experts
+        tile = MOE_TILE_LARGE if P >= 4 * MOE_TILE_LARGE * E else MOE_TILE
+        cap = -(-(P + E * (tile - 1)) // tile) * tile
+        return tile, [torch.empty(*layers, n, dtype=torch.int32, device=dev) for n in (cap, cap // tile, P)]
+
+    @staticmethod
+    def stack(layers):
+        """The expert tables of layers of one size in one tensor (every layer's ``table`` becomes a part of it), or None."""
+        if len(layers) < 2 or any(m.spec != layers[0].spec or m.table.shape != layers[0].table.shape for m in layers):
+            return None
+        tables = torch.stack([m.table for m in layers])
+        for m, t in zip(layers, tables):
+            m.table = t
+        return tables
+
+    @staticmethod
+    def align(layers, tables, h: torch.Tensor, ids: torch.Tensor):
+        """(tile, slots, tile_expert, pair_slot) of every one of the ``layers``, whose tables are ``tables``, for ``forward`` to take: one
+        launch for the step; None where the layers align for themselves."""
+        m = layers[0]
+        P = h.shape[0] * m.spec.top
+        if m._packed_ok(h, P) or not m.ops.moe_tables_align_ok(tables, ids, m.spec.experts):
+            return None
+        tile, aligned = m._tables(P, h.device, len(layers))
+        m.ops.moe_table_align(tables, ids, m.spec.experts, tile, *aligned)
+        return [(tile, *a) for a in zip(*aligned)]
+
+    def forward(self, h: torch.Tensor, ids: torch.Tensor, aligned=None):
         s, ops = self.spec, self.ops
         T, dev = h.shape[0], h.device
         P = T * s.top
-        if self._packed_ok(h, P):
+        if aligned is None and self._packed_ok(h, P):
             return self._forward_packed(h, self.table.index_select(0, ids).reshape(-1), P)
-        tile = MOE_TILE_LARGE if P >= 4 * MOE_TILE_LARGE * s.experts else MOE_TILE
-        cap = -(-(P + s.experts * (tile - 1)) // tile) * tile
-        slots = torch.empty(cap, dtype=torch.int32, device=dev)
-        tile_expert = torch.empty(cap // tile, dtype=torch.int32, device=dev)
-        pair_slot = torch.empty(P, dtype=torch.int32, device=dev)
-        ops.moe_table_align(self.table, ids, s.experts, tile, slots, tile_expert, pair_slot)
+        if aligned is None:
+            tile, (slots, tile_expert, pair_slot) = self._tables(P, dev)
+            ops.moe_table_align(self.table, ids, s.experts, tile, slots, tile_expert, pair_slot)
+        else:
+            tile, slots, tile_expert, pair_slot = aligned
+        cap = slots.shape[0]
         act = torch.empty(cap, s.ff, device=dev, dtype=h.dtype)
         ops.expert_gemm(act, h, self.w_up, slots, tile_expert, tile, s.top, True, pairs=P)
         y = torch.empty(cap, self.hidden, device=dev, dtype=h.dtype)

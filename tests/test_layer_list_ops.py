@@ -549,6 +549,27 @@ def test_moe_table_align(tokens, top):
     assert int((slots >= 0).sum()) == P
 
 
+@gpu
+@pytest.mark.parametrize("tokens,top", [(1, 2), (48, 3), (1500, 2)])
+def test_moe_table_align_of_layers(tokens, top):
+    """Every table's tiles in one launch, as one by one."""
+    g = torch.Generator().manual_seed(tokens)
+    L, E, tile, V = 3, 9, 32, 40
+    tables = torch.stack([torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(V)]) for _ in range(L)]).int()
+    ids = torch.randint(0, V, (tokens,), generator=g)
+    P = tokens * top
+    cap = -(-(P + E * (tile - 1)) // tile) * tile
+    ops = get_ops("cuda")
+    assert ops.moe_tables_align_ok(tables, ids, E)
+    slots, tiles, pair = (torch.empty(L, n, dtype=torch.int32, device="cuda") for n in (cap, cap // tile, P))
+    ops.moe_table_align(tables.cuda(), ids.cuda(), E, tile, slots, tiles, pair)
+    for i in range(L):
+        experts = tables[i][ids].view(-1)
+        assert torch.equal(tiles[i].cpu()[pair[i].cpu().long() // tile], experts)
+        assert torch.equal(slots[i].cpu()[pair[i].cpu().long()], torch.arange(P).int())
+        assert int((slots[i] >= 0).sum()) == P
+
+
 # ------------------------------------------------------------------ queries, keys and values of window attention
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
