@@ -271,18 +271,22 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
 
 }  // namespace
 
-// Which of the two kernels serves tiles of 32 slots; cold weights, us with the launch, from 8 to 256 experts, K from 512 to 4096 and up
-// to 512 pairs. expert_gemm_mfma takes 5 + 1.2 per step of 128 k (its steps wait for their loads) while its workgroups of
-// 128 columns are at most 512; expert_gemm_skinny 5.2 plus the weights of the experts that so many pairs hit on average at 5 TB/s,
-// or what its workgroups of 16 columns read at 34 KB per us and CU, plus 0.3 per 1000 workgroups: it has one per 16 columns of every tile
-// of the capacity, nearly all of them empty where the experts are many. Tile kernel / this one: 16 experts, 1024 x 2048: 2 pairs 19.9 / 7.0, 64
-// pairs 26.3 / 20.9; 2048 x 1024: 2 pairs 12.8 / 5.5, 64 pairs 18.1 / 20.9; 128 experts, 1536 x 2048, gated: 8 pairs 25.1 / 14.8; 2048 x 768:
-// 8 pairs 11.8 / 13.3, 64 pairs 36.9 / 50.6; 256 experts, 2048 x 512: 8 pairs 9.4 / 19.1, 512 pairs 94 / 166; 512 x 512: 64 pairs 10.1 / 12.4.
+// Which of the two kernels serves tiles of 32 slots; cold weights, us, 8 to 256 experts, K from 512 to 4096 and up to 4000 pairs.
+// expert_gemm_skinny takes 2.2 plus the weights of the experts that so many pairs hit on average at 5.2 TB/s, or what its workgroups of
+// 16 columns read at 80 KB per us and CU, plus 0.3 per 1000 workgroups: it has one per 16 columns of every tile of the capacity, nearly all of
+// them empty where the experts are many. expert_gemm_mfma takes 3 plus 1 per step of 128 k (its steps wait for their loads), the
+// weights at 4.6 TB/s, or what its workgroups of 128 columns read at 34 KB per us and CU (rows once per wave). Both sides are true to a
+// tenth or so: this one where it is expected to be faster by more. Tile kernel / this one: 16 experts, 1024 x 2048: 2 pairs 19.8 / 4.3, 82
+// pairs 26.0 / 15.7, 512 pairs 34.2 / 23.1, 4000 pairs 142 / 83; 2048 x 1024: 82 pairs 17.4 / 15.9, 384 pairs 20.3 / 20.7, 1400 pairs 61 / 43; 8
+// experts, 4096 x 2048: 512 pairs 88.6 / 58.5; 128 experts, 1536 x 2048, gated: 8 pairs 20.9 / 13.5, 64 pairs 77.4 / 62.3; 2048 x 768: 8 pairs
+// 10.2 / 11.5, 2000 pairs 102 / 106; 256 experts, 2048 x 512: 8 pairs 8.1 / 16.8, 512 pairs 56.7 / 73.6. Two tiles of 16 columns per
+// workgroup are hardly ever faster (16 experts, 2048 x 1024, 82 pairs: 19.1, 1400 pairs: 51).
 bool expert_gemm_skinny(long pairs, long ntiles_cap, long N, long K, long E, bool glu) {
-  const double used = E * (1 - std::pow(1 - 1.0 / E, (double)pairs)), tiles = used + pairs / 32, rows = std::min(32.0, pairs / used);
-  const double wgs = std::max(1.0, tiles * N / 16 / 256), launched = (double)((glu ? N / 2 : N) + 15) / 16 * ntiles_cap;
-  const double ours = 5.2 + std::max(used * N * K * 2 / 5.0e6, wgs * 2 * K * (16 + rows / (glu ? 2 : 1)) / 34e3) + 0.3e-3 * launched;
-  return ours < (5 + 1.2 * K / 128) * std::max(1.0, tiles * N / 128 / 512);
+  const double used = E * (1 - std::pow(1 - 1.0 / E, (double)pairs)), mean = pairs / used, tiles = used * std::max(1.0, mean / 32 + 0.45);
+  const double launched = (double)((glu ? N / 2 : N) + 15) / 16 * ntiles_cap, bytes = used * N * K * 2, rows = std::min(32.0, mean);
+  auto read = [&](double cols, double rows_read, double rate) { return std::max(1.0, tiles * N / cols / 256) * 2 * K * (cols + rows_read) / rate; };
+  const double ours = 2.2 + std::max(bytes / 5.2e6, read(16, rows / (glu ? 2 : 1), 80e3)) + 0.3e-3 * launched;
+  return ours < 0.89 * (3 + std::max({K / 128.0, bytes / 4.6e6, read(128, 4 * rows, 34e3)}));
 }
 
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,
