@@ -10,16 +10,16 @@ namespace hipserve {
 
 // residual[T, H] (fp32, in place) += ls1 * mix + ls2 * (1/top) * sum_j y[pair_slot[t*top+j]] + extra;
 // out = residual normalised in `groups` consecutive parts, times w (fp32 [H]). Null inputs are skipped. With a
-// table [table_rows, H] the residual is not read: row t starts as table[ids[t]].
+// table [table_rows, H] the residual is not read: row t starts as table[ids[t]]. mix_parts > 0: mix is fp32 [mix_parts, T, H], to be summed.
 void launch_scaled_add_group_rmsnorm(void* out, float* residual, const float* w, int T, int H, int groups, float eps,
-                                     const void* mix, const float* ls1, const void* y, const int* pair_slot, int top,
+                                     const void* mix, int mix_parts, const float* ls1, const void* y, const int* pair_slot, int top,
                                      const float* ls2, const void* extra, const void* table, const long* ids,
                                      long table_rows, bool f32, hipStream_t s);
 
 // out[b, m, n] = act(x[b, m] . W[b, n] + bias[n]) of up to 64 rows m (skinny_linear.hip): bf16 operands, K % 8 == 0, x rows at
 // multiples of 16 bytes; W [batch, N, K]; act 0 tanh, 1 xIELU, 2 relu^2, 3 SiLU gate, 4 clamped gate (N / 2 columns),
-// 5 soft cap, -1 none; on the columns from act_from on.
-bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs,
+// 5 soft cap, -1 none; on the columns from act_from on. parts > 1 (no act): K in so many parts, their sums out_zs elements apart.
+bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, int parts, const void* x, long x_ld, long x_bs,
                           const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0,
                           float c1, hipStream_t s);
 

@@ -126,13 +126,33 @@ inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor
   if (bias.has_value())
     TORCH_CHECK(d == 2 && bias->scalar_type() == x.scalar_type() && bias->is_contiguous() && bias->numel() == N, "skinny_linear: bias");
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
-  TORCH_CHECK(hipserve::launch_skinny_linear(out.data_ptr(), out.scalar_type() == at::kFloat, out.stride(-2), d == 3 ? out.stride(0) : 0,
+  TORCH_CHECK(hipserve::launch_skinny_linear(out.data_ptr(), out.scalar_type() == at::kFloat, out.stride(-2), d == 3 ? out.stride(0) : 0, 0, 1,
                                              x.data_ptr(), x.stride(-2), d == 3 ? x.stride(0) : 0, w.data_ptr(), opt_ptr(bias), f32, B,
                                              M, N, K, act, act_from, (float)c0, (float)c1, cur_stream()), "skinny_linear: LDS");
 }
 
+// out [S, M, N]: 32-bit sums over S parts of K (in 64 halves) of x [M, K] . w [N, K]^T, the bias in the first.
+inline void skinny_linear_parts(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias) {
+  CHECK_DEV(x); CHECK_CONTIG(w); CHECK_F32(out); CHECK_SAME_DEV(w, x); CHECK_SAME_DEV(out, x);
+  if (bias.has_value()) CHECK_SAME_DEV(*bias, x);
+  const bool f32 = x.scalar_type() == at::kFloat;
+  TORCH_CHECK((f32 || x.scalar_type() == at::kBFloat16) && w.scalar_type() == x.scalar_type(), "skinny_linear_parts: bf16 or fp32 operands");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 3, "skinny_linear_parts: rows, and parts of rows");
+  const long per = f32 ? 4 : 8, M = x.size(0), K = x.size(1), N = w.size(0), S = out.size(0);
+  TORCH_CHECK(w.size(1) == K && out.size(1) == M && out.size(2) == N && M <= 64 && K % per == 0 && N < (1L << 31) && K < (1L << 24) &&
+              x.stride(0) < (1L << 24) && S >= 1 && S <= 64 && S <= (K * 8 / per + 63) / 64, "skinny_linear_parts: shapes");
+  auto aligned = [](const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % per == 0 && aligned(x) && aligned(w), "skinny_linear_parts: rows at multiples of 16 bytes");
+  if (bias.has_value())
+    TORCH_CHECK(bias->scalar_type() == x.scalar_type() && bias->is_contiguous() && bias->numel() == N, "skinny_linear_parts: bias");
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  TORCH_CHECK(hipserve::launch_skinny_linear(out.data_ptr(), true, N, 0, M * N, S, x.data_ptr(), x.stride(0), 0, w.data_ptr(), opt_ptr(bias),
+                                             f32, 1, M, N, K, -1, 0, 0.f, 0.f, cur_stream()), "skinny_linear_parts: LDS");
+}
+
 inline void def_moe_ops(torch::Library& m) {
   m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int act, float c0, float c1, int act_from=0) -> ()");
+  m.def("skinny_linear_parts(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias) -> ()");
   m.def("moe_align(Tensor ids, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, Tensor(c!) pair_slot) -> ()");
   m.def("moe_table_align(Tensor table, Tensor tokens, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, "
         "Tensor(c!) pair_slot) -> ()");
@@ -144,6 +164,7 @@ inline void def_moe_ops(torch::Library& m) {
 
 inline void impl_moe_ops(torch::Library& m) {
   m.impl("skinny_linear", &skinny_linear);
+  m.impl("skinny_linear_parts", &skinny_linear_parts);
   m.impl("moe_align", &moe_align);
   m.impl("moe_table_align", &moe_table_align);
   m.impl("expert_gemm", &expert_gemm);

@@ -4,7 +4,8 @@
 // The row is split into `groups` equal consecutive parts with their own mean square. The MoE
 // combine (rows of the expert-sorted y picked through pair_slot) and the embedding re-added at
 // the start of a loop pass (`extra`) ride along, so one launch sits between two layers. With a
-// table the row starts as the embedding of its id instead of the residual.
+// table the row starts as the embedding of its id instead of the residual. `mix` may be 32-bit sums over parts of a product's K
+// (mix_parts of [T, H]), which are added up first: a product of a few rows then fills the chip with workgroups of a part each.
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
 
@@ -21,14 +22,21 @@ constexpr int kNT = 256;
 template <typename T, int V, int N>
 __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
     T* __restrict__ out, float* __restrict__ residual, const float* __restrict__ w, int H, int groups, float eps,
-    const T* __restrict__ mix, const float* __restrict__ ls1, const T* __restrict__ y, const int* __restrict__ pair_slot,
-    int top, const float* __restrict__ ls2, const T* __restrict__ extra, const T* __restrict__ table,
+    const void* __restrict__ mix_, int mix_parts, const float* __restrict__ ls1, const T* __restrict__ y,
+    const int* __restrict__ pair_slot, int top, const float* __restrict__ ls2, const T* __restrict__ extra, const T* __restrict__ table,
     const long* __restrict__ ids, long table_rows) {
   extern __shared__ float sm[];  // groups > 1: [H / V] sums of squares, then [groups] inverse rms
   __shared__ float red[16];
   const long t = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const T* mix = mix_parts == 0 ? static_cast<const T*>(mix_) : nullptr;
+  const float* part = mix_parts > 0 ? static_cast<const float*>(mix_) + t * H : nullptr;
   float* r = residual + t * H;
+  int first_slot = 0, second_slot = 0;   // of the token's expert rows, known before the rows above are summed
+  if (y != nullptr) {
+    first_slot = pair_slot[t * top];
+    second_slot = pair_slot[t * top + (top > 1 ? 1 : 0)];
+  }
   long id = 0;
   if (table != nullptr) id = ids[t];
   const bool known = id >= 0 && id < table_rows;   // an id outside the table gives a row of NaN, as no row is read
@@ -61,6 +69,45 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
 #pragma unroll
         for (int k = 0; k < V; ++k) v[i][k] += ls1 != nullptr ? a[i][k] * b[i][k] : a[i][k];
   }
+  if (part != nullptr) {
+    // loads before the first use again: up to kAhead parts, the last one in place of those that do not exist
+    constexpr int kAhead = N <= 2 ? 4 : 2;
+    const long rows = (long)gridDim.x * H;   // elements of a part
+    float f[N][V], a[kAhead][N][V], b[N][V];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int e = (tid + i * kNT) * V;
+#pragma unroll
+      for (int k = 0; k < V; ++k) f[i][k] = 0.f;
+      if (e < H) {
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) Row<float, V>::ld(part + min(j, mix_parts - 1) * rows + e, a[j][i]);
+        if (ls1 != nullptr) Row<float, V>::ld(ls1 + e, b[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if ((tid + i * kNT) * V < H)
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j)
+#pragma unroll
+          for (int k = 0; k < V; ++k) f[i][k] += j < mix_parts ? a[j][i][k] : 0.f;
+    for (int j = kAhead; j < mix_parts; ++j)
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int e = (tid + i * kNT) * V;
+        if (e < H) {
+          Row<float, V>::ld(part + j * rows + e, a[0][i]);
+#pragma unroll
+          for (int k = 0; k < V; ++k) f[i][k] += a[0][i][k];
+        }
+      }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if ((tid + i * kNT) * V < H)
+#pragma unroll
+        for (int k = 0; k < V; ++k) v[i][k] += ls1 != nullptr ? f[i][k] * b[i][k] : f[i][k];
+  }
   if (y != nullptr) {
     float f[N][V], a[N][V], b[N][V];
 #pragma unroll
@@ -69,8 +116,8 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
       for (int k = 0; k < V; ++k) f[i][k] = 0.f;
     for (int j = 0; j < top; j += 2) {   // two expert rows in flight
       const bool two = j + 1 < top;
-      const T* y0 = y + (long)pair_slot[t * top + j] * H;
-      const T* y1 = two ? y + (long)pair_slot[t * top + j + 1] * H : y0;
+      const T* y0 = y + (long)(j == 0 ? first_slot : pair_slot[t * top + j]) * H;
+      const T* y1 = two ? y + (long)(j == 0 ? second_slot : pair_slot[t * top + j + 1]) * H : y0;
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         const int e = (tid + i * kNT) * V;
@@ -111,7 +158,7 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
       }
     }
   }
-  const bool changed = table != nullptr || mix != nullptr || y != nullptr || extra != nullptr;
+  const bool changed = table != nullptr || mix_ != nullptr || y != nullptr || extra != nullptr;
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
@@ -156,7 +203,7 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
 template <typename T>
 __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_kernel(
     T* __restrict__ out, float* __restrict__ residual, const float* __restrict__ w, int H, int groups, float eps,
-    const T* __restrict__ mix, const float* __restrict__ ls1, const T* __restrict__ y,
+    const void* __restrict__ mix_, int mix_parts, const float* __restrict__ ls1, const T* __restrict__ y,
     const int* __restrict__ pair_slot, int top, const float* __restrict__ ls2, const T* __restrict__ extra,
     const T* __restrict__ table, const long* __restrict__ ids, long table_rows) {
   extern __shared__ float sm[];  // [H] squares, then [groups] inverse rms
@@ -170,7 +217,11 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_kernel(
   const bool known = id >= 0 && id < table_rows;
   for (int e = tid; e < H; e += kNT) {
     float v = table == nullptr ? r[e] : known ? ldf<T>(table, id * H + e) : __builtin_nanf("");
-    if (mix != nullptr) v += ls1 != nullptr ? ldf<T>(mix, t * H + e) * ls1[e] : ldf<T>(mix, t * H + e);
+    if (mix_ != nullptr) {
+      float m = mix_parts == 0 ? ldf<T>(static_cast<const T*>(mix_), t * H + e) : 0.f;
+      for (int j = 0; j < mix_parts; ++j) m += static_cast<const float*>(mix_)[((long)j * gridDim.x + t) * H + e];
+      v += ls1 != nullptr ? m * ls1[e] : m;
+    }
     if (y != nullptr) {
       float f = 0.f;
       for (int j = 0; j < top; ++j) f += ldf<T>(y, (long)pair_slot[t * top + j] * H + e);
@@ -252,8 +303,8 @@ void launch_add_normed(void* out, float* residual, const float* w, int T, int H,
 namespace {
 
 template <typename T>
-void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, int groups, float eps, const T* mix,
-                       const float* ls1, const T* y, const int* pair_slot, int top, const float* ls2, const T* extra,
+void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, int groups, float eps, const void* mix,
+                       int mix_parts, const float* ls1, const T* y, const int* pair_slot, int top, const float* ls2, const T* extra,
                        const T* table, const long* ids, long table_rows, hipStream_t s) {
   uintptr_t at = 0;
   for (const void* p : {(const void*)out, (const void*)residual, (const void*)w, (const void*)mix, (const void*)ls1,
@@ -264,7 +315,7 @@ void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, i
   if (at % 16 == 0 && H % V == 0 && (H / groups) % V == 0 && H <= 8 * 8 * kNT) {
     const size_t smem = groups > 1 ? (size_t)(H / V + groups) * sizeof(float) : 0;
 #define HS_GN(V, N)                                                                                                  \
-  scaled_add_group_rmsnorm_vec_kernel<T, V, N><<<T_, kNT, smem, s>>>(out, residual, w, H, groups, eps, mix, ls1, y,    \
+  scaled_add_group_rmsnorm_vec_kernel<T, V, N><<<T_, kNT, smem, s>>>(out, residual, w, H, groups, eps, mix, mix_parts, ls1, y, \
                                                                      pair_slot, top, ls2, extra, table, ids, table_rows)
     if (V == 4) HS_GN(4, 1);
     else if (H <= 8 * kNT) HS_GN(8, 1);
@@ -275,21 +326,21 @@ void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, i
     return;
   }
   scaled_add_group_rmsnorm_kernel<T><<<T_, kNT, (size_t)(H + groups) * sizeof(float), s>>>(
-      out, residual, w, H, groups, eps, mix, ls1, y, pair_slot, top, ls2, extra, table, ids, table_rows);
+      out, residual, w, H, groups, eps, mix, mix_parts, ls1, y, pair_slot, top, ls2, extra, table, ids, table_rows);
 }
 
 }  // namespace
 
 void launch_scaled_add_group_rmsnorm(void* out, float* residual, const float* w, int T, int H, int groups, float eps,
-                                     const void* mix, const float* ls1, const void* y, const int* pair_slot, int top,
+                                     const void* mix, int mix_parts, const float* ls1, const void* y, const int* pair_slot, int top,
                                      const float* ls2, const void* extra, const void* table, const long* ids,
                                      long table_rows, bool f32, hipStream_t s) {
   if (T <= 0) return;
   if (f32)
-    launch_group_norm<float>((float*)out, residual, w, T, H, groups, eps, (const float*)mix, ls1, (const float*)y,
+    launch_group_norm<float>((float*)out, residual, w, T, H, groups, eps, mix, mix_parts, ls1, (const float*)y,
                              pair_slot, top, ls2, (const float*)extra, (const float*)table, ids, table_rows, s);
   else
-    launch_group_norm<unsigned short>((unsigned short*)out, residual, w, T, H, groups, eps, (const unsigned short*)mix,
+    launch_group_norm<unsigned short>((unsigned short*)out, residual, w, T, H, groups, eps, mix, mix_parts,
                                       ls1, (const unsigned short*)y, pair_slot, top, ls2, (const unsigned short*)extra,
                                       (const unsigned short*)table, ids, table_rows, s);
 }

@@ -1,5 +1,6 @@
 // out[b, m, :] = act(x[b, m, :] . W[b]^T + bias) for up to 64 rows m (decode steps and short prompts): bf16 or 32-bit
 // operands, 32-bit accumulation, a result of the operands' type or in 32 bits, row and batch strides of their own for x and out.
+// parts > 1: as many 32-bit results, each the sum over a part of K, for a next kernel to add up (the residual update).
 // act: 0 tanh, 1 xIELU, 2 squared ReLU, 3 SiLU gate, 4 clamped gate (3, 4: W = [gate rows; up rows], half as many
 // columns in out), 5 soft cap, -1 none; they see the unrounded product. act_from: the first column that it applies to (not for gates).
 #include "skinny.h"
@@ -22,22 +23,25 @@ HS_DEVICE float skinny_act(float z, int act, float c0, float c1) {
 }
 
 // XG: groups of 8 rows; NT: 16-column tiles (GLU: the gate's and the up projection's of the same 16 output columns).
-// F32: 32-bit operands, x, w, their strides and K in 16-bit halves (skinny.h).
+// F32: 32-bit operands, x, w, their strides and K in 16-bit halves (skinny.h). Workgroups z take `part` of K each (a multiple of 64) and write
+// their sums out_zs elements apart (the bias in the first).
 template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32>
 __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
-    TO* __restrict__ out, long out_ld, long out_bs, const unsigned short* __restrict__ x, long x_ld, long x_bs,
-    const unsigned short* __restrict__ w, const void* __restrict__ bias_, int M, int N, int K, int act, int act_from, float c0, float c1) {
+    TO* __restrict__ out, long out_ld, long out_bs, long out_zs, const unsigned short* __restrict__ x, long x_ld, long x_bs,
+    const unsigned short* __restrict__ w, const void* __restrict__ bias_, int M, int N, int K, int part, int act, int act_from, float c0, float c1) {
   static_assert(!GLU || NT == 2, "a gate tile and an up tile");
   using SK = Skinny<XG, NT, DEPTH, F32>;
   constexpr int ST = SK::ST;
   using TB = std::conditional_t<F32, float, unsigned short>;
-  const TB* bias = static_cast<const TB*>(bias_);
+  const TB* bias = blockIdx.z == 0 ? static_cast<const TB*>(bias_) : nullptr;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int No = GLU ? N / 2 : N;
   const int n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
-  x += (long)blockIdx.y * x_bs;
-  w += (long)blockIdx.y * N * K;
+  const int k0 = blockIdx.z * part, k1 = min(K, k0 + part);   // (no division here: it showed in the one-row times)
+  x += (long)blockIdx.y * x_bs + k0;
+  w += (long)blockIdx.y * N * K + k0;
+  out += (long)blockIdx.z * out_zs;
   const unsigned char* wt[NT];
   unsigned w_row[2 * NT];
   unsigned x_row[XG];
@@ -55,7 +59,7 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave);
+  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, k1 - k0, smem, lane, wave);
   float v[NT][(ST + 1) / 2];
   SK::reduce(v, acc, smem);
   out += (long)blockIdx.y * out_bs;
@@ -82,22 +86,22 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
 }
 
 template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32>
-bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, const void* x, long x_ld, long x_bs, const void* w, const void* bias,
+bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, long out_zs, const void* x, long x_ld, long x_bs, const void* w, const void* bias,
                    int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
   constexpr int lds = Skinny<XG, NT, DEPTH, F32>::kLds;
   static const bool ok = allow_lds(&skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32>, lds);
   if (!ok) return false;
   skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32><<<grid, kSkThreads, lds, s>>>(
-      (TO*)out, out_ld, out_bs, (const unsigned short*)x, x_ld, x_bs, (const unsigned short*)w, bias, M, N, K, act, act_from, c0, c1);
+      (TO*)out, out_ld, out_bs, out_zs, (const unsigned short*)x, x_ld, x_bs, (const unsigned short*)w, bias, M, N, K, ((K + 63) / 64 + (int)grid.z - 1) / (int)grid.z * 64, act, act_from, c0, c1);
   return true;
 }
 
 template <int XG, int NT, int DEPTH, bool GLU>
-bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs, const void* w,
-                const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
+bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, int parts, const void* x, long x_ld, long x_bs,
+                const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
   const int cols = GLU ? N / 2 : N, per = GLU ? 16 : 16 * NT;
-  const dim3 grid((cols + per - 1) / per, batch);
-#define HS_SK(TO, F32) launch_kernel<XG, NT, DEPTH, GLU, TO, F32>(grid, out, out_ld, out_bs, x, x_ld, x_bs, w, bias, M, N, K, act, act_from, c0, c1, s)
+  const dim3 grid((cols + per - 1) / per, batch, parts);
+#define HS_SK(TO, F32) launch_kernel<XG, NT, DEPTH, GLU, TO, F32>(grid, out, out_ld, out_bs, out_zs, x, x_ld, x_bs, w, bias, M, N, K, act, act_from, c0, c1, s)
   return f32 ? HS_SK(float, true) : out_f32 ? HS_SK(float, false) : HS_SK(unsigned short, false);
 #undef HS_SK
 }
@@ -106,26 +110,26 @@ bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, const void* x
 // than that time), and what the busiest compute unit takes in at 65 / 60 / 54 KB per us. More tiles mean fewer copies of the rows and fewer workgroups. Cold weights, 1 / 2 / 4 tiles: 6144 x 2048 with 16 rows 8.2 /
 // 7.6 / -, with 48 rows 12.5 / 9.8 / 12.5; 12288 x 2048 with 16 rows 12.0 / 13.5 / -, with 48 rows 18.6 / 16.4 / 14.7; 12288 x 4096 with
 // 48 rows 32.1 / 29.3 / 23.9; 32000 x 2048 with 16 rows 26.8 / 26.8 / -, with 32 rows 38.5 / 29.7 / 30.4, with 64 50.9 / 40.4 / 34.3.
-double skinny_time(int M, long cols, int K, int nt) {
-  const long wgs = ((cols + 15) / 16 + nt - 1) / nt, rounds = (wgs + 255) / 256;
+double skinny_time(int M, long cols, int K, int nt, int parts) {
+  const long wgs = ((cols + 15) / 16 + nt - 1) / nt * parts, rounds = (wgs + 255) / 256;
   const double stream = 2.0 * cols * K / 5.2e6, rate = nt == 1 ? 65e3 : nt == 2 ? 60e3 : 54e3;
-  return 2.2 + std::max(stream, 0.38 * stream + rounds * 2.0 * K * (16 * nt + (M + 7) / 8 * 8) / rate);
+  return 2.2 + std::max(stream, 0.38 * stream + rounds * 2.0 * K / parts * (16 * nt + (M + 7) / 8 * 8) / rate);
 }
 
 }  // namespace
 
-bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, const void* x, long x_ld, long x_bs,
+bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, int parts, const void* x, long x_ld, long x_bs,
                           const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1,
                           hipStream_t s) {
   if (batch <= 0 || M <= 0 || N <= 0) return true;
   if (f32) { x_ld *= 2; x_bs *= 2; K *= 2; }   // in halves
-#define HS_SK(XG, NT, DEPTH, GLU)   launch_one<XG, NT, DEPTH, GLU>(out, out_f32, out_ld, out_bs, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, act_from, c0, c1, s)
+#define HS_SK(XG, NT, DEPTH, GLU)   launch_one<XG, NT, DEPTH, GLU>(out, out_f32, out_ld, out_bs, out_zs, parts, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, act_from, c0, c1, s)
   const int xg = (M + 7) / 8;
   if (act == 3 || act == 4)
     return xg <= 1 ? HS_SK(1, 2, 1, true) : xg <= 2 ? HS_SK(2, 2, 1, true) : xg <= 4 ? HS_SK(4, 2, 1, true)
          : xg <= 6 ? HS_SK(6, 2, 1, true) : HS_SK(8, 2, 1, true);
-  const double t1 = skinny_time(M, (long)N * batch, K, 1), t2 = skinny_time(M, (long)N * batch, K, 2),
-               t4 = M > 16 ? skinny_time(M, (long)N * batch, K, 4) : INFINITY;
+  const double t1 = skinny_time(M, (long)N * batch, K, 1, parts), t2 = skinny_time(M, (long)N * batch, K, 2, parts),
+               t4 = M > 16 ? skinny_time(M, (long)N * batch, K, 4, parts) : INFINITY;
   // one piece ahead where the workgroups of several tiles would otherwise not fit a compute unit together (2 - 14 % faster)
   if (t4 < t1 && t4 < t2) return xg <= 4 ? HS_SK(4, 4, 1, false) : xg <= 6 ? HS_SK(6, 4, 1, false) : HS_SK(8, 4, 1, false);
   if (t2 < t1)

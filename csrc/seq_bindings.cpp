@@ -27,7 +27,9 @@ void scaled_add_group_rmsnorm(at::Tensor& out, at::Tensor& residual, const at::T
   const long T = residual.size(0), H = residual.size(1);
   TORCH_CHECK(groups >= 1 && H % groups == 0 && w.numel() == H && H + groups <= 15000, "group norm shape");
   if (mix.has_value()) {
-    TORCH_CHECK(mix->scalar_type() == out.scalar_type() && mix->is_contiguous() && mix->sizes() == residual.sizes());
+    TORCH_CHECK(mix->is_contiguous() && (mix->dim() == 3 ? mix->scalar_type() == at::kFloat && mix->size(0) >= 1 && mix->size(1) == T && mix->size(2) == H
+                                                         : mix->scalar_type() == out.scalar_type() && mix->sizes() == residual.sizes()));
+    CHECK_SAME_DEV(*mix, out);
     TORCH_CHECK(!ls1.has_value() || (ls1->scalar_type() == at::kFloat && ls1->is_contiguous() && ls1->numel() == H));
   }
   if (y.has_value()) {
@@ -46,6 +48,7 @@ void scaled_add_group_rmsnorm(at::Tensor& out, at::Tensor& residual, const at::T
   c10::hip::HIPGuardMasqueradingAsCUDA g(out.device());
   hipserve::launch_scaled_add_group_rmsnorm(
       out.data_ptr(), residual.data_ptr<float>(), w.data_ptr<float>(), T, H, groups, (float)eps, opt_ptr(mix),
+      mix.has_value() && mix->dim() == 3 ? (int)mix->size(0) : 0,
       (const float*)opt_ptr(ls1), opt_ptr(y), (const int*)opt_ptr(pair_slot), y.has_value() ? top : 0,
       (const float*)opt_ptr(ls2), opt_ptr(extra), opt_ptr(table), table.has_value() ? ids->data_ptr<long>() : nullptr,
       table.has_value() ? table->size(0) : 0, f32, cur_stream());

@@ -21,6 +21,13 @@ from .layer_list import LayerListModel
 
 
 class FikizenModel(LayerListModel):
+    def __init__(self, *args, **kwargs):
+        super().__init__(*args, **kwargs)
+        for lw in self.layers:
+            for m in (lw.mixer, lw.mlp) if lw is not None else ():
+                if m is not None:
+                    m.takes_parts = True   # of the residual update below
+
     # ---------------------------------------------------------------- forward
     def forward(self, ids: torch.Tensor, meta, kv_caches) -> torch.Tensor:
         ops, cfg = self.ops, self.cfg

@@ -62,6 +62,7 @@ class KesiraxModel:
                 lw.mixer = MinGRU(m, H, cfg.norm_eps, self.device, dtype, ops)
             else:
                 raise NotImplementedError(type(m).__name__)
+            lw.mixer.takes_parts = True   # of the residual update below
             if spec.mlp is not None:
                 lw.mlp = TableMoE(spec.mlp, H, cfg.vocab_size, self.device, dtype, ops)
             self.layers.append(lw)

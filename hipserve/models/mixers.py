@@ -102,6 +102,12 @@ def _side(sub, proj: torch.Tensor):
     sub.side_out = proj[:, proj.shape[1] - n:] if n else None
 
 
+def _last(sub, x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
+    """The last product of a sublayer: [T, hidden], or 32-bit parts of it [parts, T, hidden] for a model whose residual update adds
+    them up (it sets ``takes_parts``)."""
+    return sub.ops.linear_parts(x, w, b) if getattr(sub, "takes_parts", False) else sub.ops.linear(x, w, b)
+
+
 def _deinterleave(w: torch.Tensor, dims: int) -> torch.Tensor:
     """Rows [..., r, in] of a projection whose outputs are rotated in pairs (2i, 2i + 1): the first ``dims`` rows
     reordered to [even | odd], so that the rotate-half kernels (pairs i, i + dims / 2) compute the same scores."""
@@ -206,7 +212,7 @@ class LatentAttention:
             cat = torch.empty(T, s.heads * s.vdim, device=h.device, dtype=h.dtype)
             ops.latent_prompt_attention(cat, q, proj, cache, meta, self.inv_freq, s, self.w_kv, rows,
                                         -1 if s.gate == "none" else gate_off)
-            return ops.linear(cat, self.w_o)
+            return _last(self, cat, self.w_o)
         qh = q.view(T, s.heads, s.dim + s.rot_dim)
         if ops.latent_query_in_place(h.dtype, s.kv_rank, s.rot_dim):
             # the absorption GEMM writes the attention kernel's query rows directly: bf16, the cached width,
@@ -224,15 +230,15 @@ class LatentAttention:
                              s.kv_rank, gate_off if s.gate == "head" else -1, s.scale, s.window)
         cat = torch.empty(T, s.heads * s.vdim, device=h.device, dtype=h.dtype)
         if s.gate != "channel" and ops.linear_heads(cat.view(T, s.heads, s.vdim).transpose(0, 1), o_lat, self.w_uv):
-            return ops.linear(cat, self.w_o)                           # the heads were written side by side
+            return _last(self, cat, self.w_o)                          # the heads were written side by side
         o = torch.empty(s.heads, T, s.vdim, device=h.device, dtype=h.dtype)
         if not ops.linear_heads(o, o_lat, self.w_uv):
             torch.bmm(o_lat, self.w_uv_t, out=o)                       # [heads, T, vdim]
         if s.gate == "channel":
             # heads side by side per token, each element times the sigmoid of its gate column: one pass
             ops.gate_mul(cat, o, proj[:, gate_off:gate_off + s.heads * s.vdim])
-            return self.ops.linear(cat, self.w_o)
-        return self.ops.linear(o.transpose(0, 1).reshape(T, s.heads * s.vdim), self.w_o)
+            return _last(self, cat, self.w_o)
+        return _last(self, o.transpose(0, 1).reshape(T, s.heads * s.vdim), self.w_o)
 
 
 class MinGRU:
@@ -266,7 +272,7 @@ class MinGRU:
         proj = self.ops.linear(h, self.w_in)
         y = torch.empty(h.shape[0], self.spec.width, device=h.device, dtype=h.dtype)
         self.ops.mingru_scan(y, state, proj, self.b_z, self.b_x, meta)
-        return self.ops.linear(y, self.w_o)
+        return _last(self, y, self.w_o)
 
 
 class TableMoE:
@@ -484,7 +490,7 @@ class WindowAttention:
 
     def forward(self, h, meta, cache, state):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return self.ops.linear(self.mix(h, meta, cache, state, out), self.w_o, self.b_o)
+        return _last(self, self.mix(h, meta, cache, state, out), self.w_o, self.b_o)
 
 
 class Wkv:
@@ -645,7 +651,7 @@ class GatedDelta:
 
     def forward(self, h, meta, cache, state):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return self.ops.linear(self.mix(h, meta, cache, state, out), self.w_o)
+        return _last(self, self.mix(h, meta, cache, state, out), self.w_o)
 
 
 class DeltaRule:
@@ -692,7 +698,7 @@ class DeltaRule:
 
     def forward(self, h, meta, cache, state):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return self.ops.linear(self.mix(h, meta, cache, state, out), self.w_o)
+        return _last(self, self.mix(h, meta, cache, state, out), self.w_o)
 
 
 class MLstm:
@@ -865,10 +871,10 @@ class ParallelMixer:
             proj = self.ops.linear(h, self.w_in)
             self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale, proj[:, :self.split])
             self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale, proj[:, self.split:])
-            return self.ops.linear(buf, self.w_o)
+            return _last(self, buf, self.w_o)
         self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale)
         self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale)
-        return self.ops.linear(buf, self.w_o)
+        return _last(self, buf, self.w_o)
 
 
 class DenseFF:
@@ -907,7 +913,7 @@ class DenseFF:
         ff, act = self.spec.ff, self.spec.act
         c0 = self.spec.limit if act == "clamped_glu" else self.c0
         if act != "polynorm" and not self.side_rows:
-            return self.ops.linear(self.ops.linear(h, self.w_up, act=act, c0=c0, c1=self.c1), self.w_down)
+            return _last(self, self.ops.linear(h, self.w_up, act=act, c0=c0, c1=self.c1), self.w_down)
         up = self.ops.linear(h, self.w_up)
         _side(self, up)
         out = torch.empty(h.shape[0], ff, device=h.device, dtype=h.dtype)
@@ -915,7 +921,7 @@ class DenseFF:
             self.ops.polynorm(out, up[:, :ff], self.coef, self.eps)
         else:
             self.ops.activation(out, up[:, :2 * ff] if act == "clamped_glu" else up[:, :ff], act, c0, self.c1)
-        return self.ops.linear(out, self.w_down)
+        return _last(self, out, self.w_down)
 
 
 class RoutedMoE:

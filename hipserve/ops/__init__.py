@@ -226,7 +226,8 @@ class KernelOps:
     # ---- layer-list decoders (csrc/kernels/seq/*.hip; bf16 or true fp32 activations)
     def scaled_add_group_rmsnorm(self, out, residual, w, groups, eps, mix=None, ls1=None, y=None, pair_slot=None,
                                  top=0, ls2=None, extra=None, table=None, ids=None):
-        """``table`` / ``ids``: the rows start as table[ids] instead of what ``residual`` holds."""
+        """``table`` / ``ids``: the rows start as table[ids] instead of what ``residual`` holds. ``mix``: [T, H], or 32-bit parts of it
+        [parts, T, H] (``linear_parts``)."""
         lib = self._delta if self.norm_library == "delta" else self._seq
         lib.scaled_add_group_rmsnorm(out, residual, w, groups, eps, mix, ls1, y, pair_slot, top, ls2, extra, table, ids)
         return out
@@ -466,18 +467,52 @@ class KernelOps:
         64 rows 4.4 / 11.0, 5.1 / 11.1, 7.1 / 11.4, 8.0 / 11.9; 6144 x 2048 with 1, 16, 48 rows 7.8 / 12.5, 8.1 / 12.5, 10.1 / 12.9;
         2048 x 6144 with 1, 16, 48 rows 7.8 / 11.1, 10.5 / 11.2, 16.2 / 16.5; 12288 x 2048 with 16, 48 rows 12.6 / 15, 15.2 / 15.6;
         32000 x 2048 with 1, 16, 48, 64 rows 26 / 32, 28 / 31, 34 / 34, 35 / 30."""
+        return KernelOps.skinny_time(rows, cols, k, glu, f32) < KernelOps._vendor_time(rows, cols, k, f32)
+
+    @staticmethod
+    def skinny_time(rows, cols, k, glu=False, f32=False, parts=1) -> float:
         k *= 2 if f32 else 1   # in 16-bit halves
         stream, tiles, padded = 2.0 * cols * k / 5.2e6, -(-cols // 16), -(-rows // 8) * 8
 
         def intake(nt, rate):
-            return -(-(-(-tiles // nt)) // 256) * 2.0 * k * (16 * nt + padded) / rate
+            return -(-(-(-tiles // nt) * parts) // 256) * 2.0 * k / parts * (16 * nt + padded) / rate
 
-        ours = 2.2 + max(stream, 0.38 * stream + (intake(2, 60e3) if glu else min(intake(1, 65e3), intake(2, 60e3), intake(4, 54e3))))
+        return 2.2 + max(stream, 0.38 * stream + (intake(2, 60e3) if glu else min(intake(1, 65e3), intake(2, 60e3), intake(4, 54e3))))
+
+    @staticmethod
+    def _vendor_time(rows, cols, k, f32) -> float:
         if f32:
-            # the vendor's is hardly ever below 10.7 (8.9 for 1024 x 1024) and streams at 4.5 TB/s
-            return ours < max(8.9 if max(cols, k // 2) <= 1024 else 10.7, 3.2 + 2.0 * cols * k / 4.5e6)
+            # hardly ever below 10.7 (8.9 for 1024 x 1024), streams at 4.5 TB/s
+            return max(8.9 if max(cols, k) <= 1024 else 10.7, 3.2 + 4.0 * cols * k / 4.5e6)
         least = 7.5 if k <= 1024 else 10.5 if rows <= 32 else max(10.5, 4.6 + 1.85e-3 * k)
-        return ours < max(least, 3.2 + 2.0 * cols * k / 4.2e6 if rows <= 16 else 4.2 + 2.0 * cols * k / 4.8e6)
+        return max(least, 3.2 + 2.0 * cols * k / 4.2e6 if rows <= 16 else 4.2 + 2.0 * cols * k / 4.8e6)
+
+    @staticmethod
+    def skinny_parts(rows, cols, k, f32=False) -> int:
+        """Parts of k for a product whose 32-bit sums the next kernel adds up (1: none), or 0 where the vendor's GEMM is the one to run. A part
+        more gives idle compute units a share and costs 0.15 us and what it is to write and read it (fitted), and the first one 0.7 us, which
+        the update takes longer with parts in a captured step than in a loop of the two; every wave keeps a piece of 64 halves. us with the residual update and norm behind it, cold weights, vendor / one / two / four parts: 1024 x 3072 with 1, 16, 48
+        rows 14.6 / 8.0 / 7.5 / 7.5, 15.1 / 9.7 / 8.4 / 8.1, 14.7 / 12.8 / 10.2 / 9.1; 2048 x 2048 with 1, 16, 48 rows 14.0 / 7.9 / 7.7 / 8.3, 14.3 /
+        8.8 / 8.2 / 8.9, 14.3 / 10.7 / 9.6 / 10.4; 2048 x 6144 with 16, 48 rows 14.6 / 14.2 / 11.4 / 11.8, 19.9 / 20.2 / 14.6 / 14.0; 4096 x 4096
+        with 24 rows 16.7 / 13.7 / 14.7 / 15.6; 4096 x 12288 with 48 rows 35.0 / 36.7 / 32.1 / 28.8. Three or six parts were never best."""
+        def time(p):
+            return KernelOps.skinny_time(rows, cols, k, False, f32, p) + (p > 1) * 0.7 + (p - 1) * (0.15 + 0.5e-5 * rows * cols)
+
+        ours, parts = min((time(p), p) for p in (1, 2, 4) if p == 1 or p * 512 <= k * (2 if f32 else 1))
+        if ours > 0.94 * time(1):   # no more parts for what the model cannot tell
+            ours, parts = time(1), 1
+        return parts if ours < KernelOps._vendor_time(rows, cols, k, f32) else 0
+
+    def linear_parts(self, x, w, bias=None):
+        """``linear`` for a result that ``scaled_add_group_rmsnorm`` takes as ``mix``: where that is faster, 32-bit sums over parts of k,
+        [parts, T, N]."""
+        if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())):
+            parts = self.skinny_parts(x.shape[0], w.shape[0], w.shape[1], x.dtype == torch.float32)
+            if parts > 1:
+                out = torch.empty(parts, x.shape[0], w.shape[0], device=x.device, dtype=torch.float32)
+                self._moe_lib.skinny_linear_parts(out, x, w, bias)
+                return out
+        return self.linear(x, w, bias)
 
     def _skinny_ok(self, x, w) -> bool:
         """The shapes, types and alignment that ``skinny_linear`` takes."""
@@ -905,6 +940,9 @@ class ReferenceOps:
             return y
         out = y.new_empty(*y.shape[:-1], y.shape[-1] // 2) if act in KernelOps.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)
+
+    def linear_parts(self, x, w, bias=None):
+        return self.linear(x, w, bias)
 
     def linear_heads(self, out, x, w) -> bool:
         return False

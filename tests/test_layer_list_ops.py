@@ -146,6 +146,29 @@ def test_linear_activation_of_last_columns(dev, M, first):
 
 
 @gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,N,K,parts", [(1, 16, 128, 2), (3, 40, 1032, 8), (17, 2064, 1024, 3), (48, 1032, 3080, 6), (64, 16, 64, 1), (5, 5001, 1544, 4)])
+def test_product_in_parts(M, N, K, parts, dtype):
+    """Parts of k that end inside a wave's share, of a piece each, with a last piece cut off; the bias once; the residual update that
+    adds them up (its general kernel for rows that are no multiple of 4)."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x, w, bias = torch.randn(M, K, generator=g).to(dtype), (torch.randn(N, K, generator=g) / K ** 0.5).to(dtype), torch.randn(N, generator=g).to(dtype)
+    ops = get_ops("cuda")
+    out = torch.full((parts, M, N), 7.0, device="cuda")
+    ops._moe_lib.skinny_linear_parts(out, x.cuda(), w.cuda(), bias.cuda())
+    want = x.double() @ w.double().T + bias.double()
+    close_to(out.double().sum(0), want, x, w)
+    res, norm, ls = torch.randn(M, N, generator=g), torch.randn(N, generator=g), torch.randn(N, generator=g)
+    h, r = torch.empty(M, N, dtype=dtype, device="cuda"), res.cuda()
+    ops.scaled_add_group_rmsnorm(h, r, norm.cuda(), 1, 1e-6, out, ls.cuda())
+    sums = res.double() + want * ls.double()
+    # the product's sums (close_to), times ls1, added in 32 bits
+    assert ((r.double().cpu() - sums).abs() <= 2.0 ** -20 * (res.double().abs() + 4 * ls.double().abs() * (1 + want.abs())) + 1e-5).all()
+    n = sums * torch.rsqrt(sums.square().mean(-1, keepdim=True) + 1e-6) * norm.double()
+    assert ((h.double().cpu() - n).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -17) * n.abs() + 2e-5).all()
+
+
+@gpu
 @pytest.mark.parametrize("M", [8, 9, 24, 25, 40, 41, 64])
 @pytest.mark.parametrize("N", [4113, 5001, 12301])
 def test_skinny_linear_wide(M, N):
