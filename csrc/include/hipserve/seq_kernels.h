@@ -23,6 +23,19 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
                           const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0,
                           float c1, hipStream_t s);
 
+// A norm around such a product of up to 32 rows, in one part: with a residual [M, N] (fp32, updated in place), out = residual * weight
+// and squares [M, blocks = N / 16] = sums of the updated residual's squares (N % 64 == 0); without one the rows x are such an out and every
+// result is multiplied by 1 / sqrt(the row's squares / cols + eps). blocks is a multiple of 4 and at most 256.
+struct SkinnyNorm {
+  float* squares = nullptr;
+  int blocks = 0;
+  float cols = 1.f, eps = 0.f;
+  float* residual = nullptr;
+  const float* weight = nullptr;
+};
+bool launch_skinny_linear_normed(void* out, bool out_f32, const SkinnyNorm& norm, const void* x, long x_ld, const void* w, const void* bias,
+                                 bool f32, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s);
+
 // proj[T, ld] rows = [q latent (q_rank) | kv latent (kv_rank) | rotary key (rot_dim) | ...]:
 // cq[T, q_rank] = RMSNorm(q latent) * q_norm; cache row slots[t] (>= 0) = [RMSNorm(kv latent) * kv_norm |
 // RoPE(rotary key)], rotate-half over the first 2 * nfreq dims with angle pos * inv_freq[i].

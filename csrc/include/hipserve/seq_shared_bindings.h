@@ -150,9 +150,68 @@ inline void skinny_linear_parts(at::Tensor& out, const at::Tensor& x, const at::
                                              f32, 1, M, N, K, -1, 0, 0.f, 0.f, cur_stream()), "skinny_linear_parts: LDS");
 }
 
+inline void check_normed_rows(const at::Tensor& out, const at::Tensor& squares, const at::Tensor& x, const at::Tensor& w,
+                              const c10::optional<at::Tensor>& bias) {
+  CHECK_DEV(x); CHECK_CONTIG(w); CHECK_CONTIG(out); CHECK_F32(squares); CHECK_SAME_DEV(w, x); CHECK_SAME_DEV(out, x); CHECK_SAME_DEV(squares, x);
+  const bool f32 = x.scalar_type() == at::kFloat;
+  const long per = f32 ? 4 : 8, M = x.size(0), K = x.size(-1), N = w.size(0);
+  TORCH_CHECK((f32 || x.scalar_type() == at::kBFloat16) && w.scalar_type() == x.scalar_type(), "skinny_linear: bf16 or fp32 operands");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && out.dim() == 2 && squares.dim() == 2 && w.size(1) == K && out.size(0) == M && M <= 32 &&
+              K % per == 0 && N < (1L << 31) && K < (1L << 24) && x.stride(0) < (1L << 24), "skinny_linear: shapes");
+  TORCH_CHECK(squares.size(0) == M && squares.size(1) % 4 == 0 && squares.size(1) <= 256, "skinny_linear: squares");
+  auto aligned = [](const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % per == 0 && aligned(x) && aligned(w) && aligned(squares), "skinny_linear: rows at multiples of 16 bytes");
+  if (bias.has_value()) {
+    CHECK_SAME_DEV(*bias, x);
+    TORCH_CHECK(bias->scalar_type() == x.scalar_type() && bias->is_contiguous() && bias->numel() == N, "skinny_linear: bias");
+  }
+}
+
+// skinny_linear of rows x [M, K] without their norm's factor, 1 / sqrt(sum of the row's squares / K + eps).
+inline void skinny_linear_normed(at::Tensor& out, const at::Tensor& x, const at::Tensor& squares, double eps, const at::Tensor& w,
+                                 const c10::optional<at::Tensor>& bias, int64_t act, double c0, double c1, int64_t act_from) {
+  check_normed_rows(out, squares, x, w, bias);
+  const bool f32 = x.scalar_type() == at::kFloat, glu = act == 3 || act == 4;
+  const long N = w.size(0), K = x.size(1);
+  TORCH_CHECK(out.scalar_type() == x.scalar_type() || out.scalar_type() == at::kFloat, "skinny_linear: result type");
+  TORCH_CHECK(act >= -1 && act <= 5 && (!glu || N % 2 == 0) && out.size(1) == (glu ? N / 2 : N) && act_from >= 0 && act_from <= N &&
+              (act_from == 0 || !glu), "skinny_linear: activation");
+  hipserve::SkinnyNorm norm;
+  norm.squares = squares.data_ptr<float>();
+  norm.blocks = squares.size(1);
+  norm.cols = (float)K;
+  norm.eps = (float)eps;
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  TORCH_CHECK(hipserve::launch_skinny_linear_normed(out.data_ptr(), out.scalar_type() == at::kFloat, norm, x.data_ptr(), x.stride(0),
+                                                    w.data_ptr(), opt_ptr(bias), f32, x.size(0), N, K, act, act_from, (float)c0, (float)c1,
+                                                    cur_stream()), "skinny_linear: LDS");
+}
+
+// residual [M, N] += x . w^T + bias; out = residual * weight; squares [M, N / 16] = the residual's squares summed over 16 columns.
+inline void skinny_linear_update(at::Tensor& out, at::Tensor& squares, at::Tensor& residual, const at::Tensor& weight, const at::Tensor& x,
+                                 const at::Tensor& w, const c10::optional<at::Tensor>& bias) {
+  check_normed_rows(out, squares, x, w, bias);
+  CHECK_F32(residual); CHECK_F32(weight); CHECK_SAME_DEV(residual, x); CHECK_SAME_DEV(weight, x);
+  const long M = x.size(0), N = w.size(0);
+  TORCH_CHECK(out.scalar_type() == x.scalar_type() && out.size(1) == N && residual.dim() == 2 && residual.size(0) == M && residual.size(1) == N &&
+              weight.numel() == N && N % 64 == 0 && squares.size(1) == N / 16, "skinny_linear_update: shapes");
+  hipserve::SkinnyNorm norm;
+  norm.squares = squares.data_ptr<float>();
+  norm.blocks = squares.size(1);
+  norm.residual = residual.data_ptr<float>();
+  norm.weight = weight.data_ptr<float>();
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  TORCH_CHECK(hipserve::launch_skinny_linear_normed(out.data_ptr(), false, norm, x.data_ptr(), x.stride(0), w.data_ptr(), opt_ptr(bias),
+                                                    x.scalar_type() == at::kFloat, M, N, x.size(1), -1, 0, 0.f, 0.f, cur_stream()),
+              "skinny_linear: LDS");
+}
+
 inline void def_moe_ops(torch::Library& m) {
   m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int act, float c0, float c1, int act_from=0) -> ()");
   m.def("skinny_linear_parts(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias) -> ()");
+  m.def("skinny_linear_normed(Tensor(a!) out, Tensor x, Tensor squares, float eps, Tensor w, Tensor? bias, int act, float c0, float c1, "
+        "int act_from) -> ()");
+  m.def("skinny_linear_update(Tensor(a!) out, Tensor(b!) squares, Tensor(c!) residual, Tensor weight, Tensor x, Tensor w, Tensor? bias) -> ()");
   m.def("moe_align(Tensor ids, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, Tensor(c!) pair_slot) -> ()");
   m.def("moe_table_align(Tensor table, Tensor tokens, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, "
         "Tensor(c!) pair_slot) -> ()");
@@ -165,6 +224,8 @@ inline void def_moe_ops(torch::Library& m) {
 inline void impl_moe_ops(torch::Library& m) {
   m.impl("skinny_linear", &skinny_linear);
   m.impl("skinny_linear_parts", &skinny_linear_parts);
+  m.impl("skinny_linear_normed", &skinny_linear_normed);
+  m.impl("skinny_linear_update", &skinny_linear_update);
   m.impl("moe_align", &moe_align);
   m.impl("moe_table_align", &moe_table_align);
   m.impl("expert_gemm", &expert_gemm);

@@ -19,7 +19,9 @@ constexpr int kNT = 256;
 // prompt step is bound by memory, a decode step (a workgroup or two per XCD) by the latency of its loads: the element
 // loop below waits for them once per 256 elements and again for the squares. 8192 rows x 2048, bf16: 59.5 -> 41.0 us
 // (4.9 TB/s), with two expert rows 113 -> 55 us; 1 row: 5.8 -> 3.2 us, with two expert rows 8.2 -> 3.8 us (an empty kernel: 3.1).
-template <typename T, int V, int N>
+// PARTS: `mix` comes in 32-bit parts; a kernel of its own, since a decode step's launches wait for their code as well (one row of 2048
+// with two expert rows in a captured step 4.1 us, 4.8 with the parts' code in it).
+template <typename T, int V, int N, bool PARTS>
 __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
     T* __restrict__ out, float* __restrict__ residual, const float* __restrict__ w, int H, int groups, float eps,
     const void* __restrict__ mix_, int mix_parts, const float* __restrict__ ls1, const T* __restrict__ y,
@@ -29,14 +31,9 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
   __shared__ float red[16];
   const long t = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const T* mix = mix_parts == 0 ? static_cast<const T*>(mix_) : nullptr;
-  const float* part = mix_parts > 0 ? static_cast<const float*>(mix_) + t * H : nullptr;
+  const T* mix = PARTS ? nullptr : static_cast<const T*>(mix_);
+  const float* part = PARTS ? static_cast<const float*>(mix_) + t * H : nullptr;
   float* r = residual + t * H;
-  int first_slot = 0, second_slot = 0;   // of the token's expert rows, known before the rows above are summed
-  if (y != nullptr) {
-    first_slot = pair_slot[t * top];
-    second_slot = pair_slot[t * top + (top > 1 ? 1 : 0)];
-  }
   long id = 0;
   if (table != nullptr) id = ids[t];
   const bool known = id >= 0 && id < table_rows;   // an id outside the table gives a row of NaN, as no row is read
@@ -69,7 +66,7 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
 #pragma unroll
         for (int k = 0; k < V; ++k) v[i][k] += ls1 != nullptr ? a[i][k] * b[i][k] : a[i][k];
   }
-  if (part != nullptr) {
+  if constexpr (PARTS) {
     // loads before the first use again: up to kAhead parts, the last one in place of those that do not exist
     constexpr int kAhead = N <= 2 ? 4 : 2;
     const long rows = (long)gridDim.x * H;   // elements of a part
@@ -116,8 +113,8 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
       for (int k = 0; k < V; ++k) f[i][k] = 0.f;
     for (int j = 0; j < top; j += 2) {   // two expert rows in flight
       const bool two = j + 1 < top;
-      const T* y0 = y + (long)(j == 0 ? first_slot : pair_slot[t * top + j]) * H;
-      const T* y1 = two ? y + (long)(j == 0 ? second_slot : pair_slot[t * top + j + 1]) * H : y0;
+      const T* y0 = y + (long)pair_slot[t * top + j] * H;
+      const T* y1 = two ? y + (long)pair_slot[t * top + j + 1] * H : y0;
 #pragma unroll
       for (int i = 0; i < N; ++i) {
         const int e = (tid + i * kNT) * V;
@@ -314,8 +311,9 @@ void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, i
   const int V = H <= 4 * kNT ? 4 : 8;
   if (at % 16 == 0 && H % V == 0 && (H / groups) % V == 0 && H <= 8 * 8 * kNT) {
     const size_t smem = groups > 1 ? (size_t)(H / V + groups) * sizeof(float) : 0;
-#define HS_GN(V, N)                                                                                                  \
-  scaled_add_group_rmsnorm_vec_kernel<T, V, N><<<T_, kNT, smem, s>>>(out, residual, w, H, groups, eps, mix, mix_parts, ls1, y, \
+#define HS_GN(V, N) (mix_parts > 0 ? HS_GP(V, N, true) : HS_GP(V, N, false))
+#define HS_GP(V, N, PARTS)                                                                                           \
+  scaled_add_group_rmsnorm_vec_kernel<T, V, N, PARTS><<<T_, kNT, smem, s>>>(out, residual, w, H, groups, eps, mix, mix_parts, ls1, y, \
                                                                      pair_slot, top, ls2, extra, table, ids, table_rows)
     if (V == 4) HS_GN(4, 1);
     else if (H <= 8 * kNT) HS_GN(8, 1);
@@ -323,6 +321,7 @@ void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, i
     else if (H <= 32 * kNT) HS_GN(8, 4);
     else HS_GN(8, 8);
 #undef HS_GN
+#undef HS_GP
     return;
   }
   scaled_add_group_rmsnorm_kernel<T><<<T_, kNT, (size_t)(H + groups) * sizeof(float), s>>>(

@@ -8,8 +8,8 @@ layer may use another layer's weights; every layer RUN still has a paged cache a
 state tensors of its own. The logits pass ``cap * tanh(. / cap)``.
 
 The residual stream lives in 32-bit floats for every dtype; each residual update and the
-norm that follows it are one fused op (``scaled_add_group_rmsnorm`` with one group). Per
-engine step the model sees the flat token rows of all scheduled sequences (prompt portions
+norm that follows it are one fused op (``scaled_add_group_rmsnorm`` with one group), or part
+of the products around them where the step has few rows. Per engine step the model sees the flat token rows of all scheduled sequences (prompt portions
 and single decode tokens alike); attention reads and writes the paged cache through the
 step's block tables, the recurrences their sequences' state slots.
 """
@@ -41,21 +41,24 @@ class FikizenModel(LayerListModel):
         first = self.layers[self.runs[0][0]].norm1 if self.runs else self.final_norm
         # the first norm reads the embedding table itself
         ops.scaled_add_group_rmsnorm(h, residual, first, 1, cfg.norm_eps, table=self.embed, ids=ids.long().contiguous())
+        # steps of a few rows: a sublayer's last product may take the update and the next norm with it (not the last: ``forward`` returns
+        # a tensor)
+        fused = self.capture is None
         for r, (i, _, _) in enumerate(self.runs):
             lw = self.layers[i]
-            mix = lw.mixer.forward(h, meta, kv_caches[r], state[r] if state is not None else None)
-            nxt = self.final_norm if r + 1 == len(self.runs) else self.layers[self.runs[r + 1][0]].norm1
-            hn = torch.empty_like(h)
+            last = r + 1 == len(self.runs)
+            nxt = self.final_norm if last else self.layers[self.runs[r + 1][0]].norm1
+            after = nxt if lw.mlp is None else lw.norm2   # the norm after the mixer
+            h = lw.mixer.forward(h, meta, kv_caches[r], state[r] if state is not None else None,
+                                 (residual, after, cfg.norm_eps) if fused and not (last and lw.mlp is None) else None)
+            if torch.is_tensor(h):
+                h = ops.scaled_add_group_rmsnorm(torch.empty(T, H, device=ids.device, dtype=self.dtype), residual, after, 1, cfg.norm_eps, h)
             if lw.mlp is not None:
-                ops.scaled_add_group_rmsnorm(hn, residual, lw.norm2, 1, cfg.norm_eps, mix)
-                ff = lw.mlp.forward(hn)
-                hn = torch.empty_like(h)
-                ops.scaled_add_group_rmsnorm(hn, residual, nxt, 1, cfg.norm_eps, ff)
-            else:
-                ops.scaled_add_group_rmsnorm(hn, residual, nxt, 1, cfg.norm_eps, mix)
+                h = lw.mlp.forward(h, (residual, nxt, cfg.norm_eps) if fused and not last else None)
+                if torch.is_tensor(h):
+                    h = ops.scaled_add_group_rmsnorm(torch.empty(T, H, device=ids.device, dtype=self.dtype), residual, nxt, 1, cfg.norm_eps, h)
             if self.capture is not None:
                 self.capture.append(residual.clone())
-            h = hn
         return h
 
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:

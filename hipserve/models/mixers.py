@@ -102,9 +102,14 @@ def _side(sub, proj: torch.Tensor):
     sub.side_out = proj[:, proj.shape[1] - n:] if n else None
 
 
-def _last(sub, x: torch.Tensor, w: torch.Tensor, b=None) -> torch.Tensor:
+def _last(sub, x: torch.Tensor, w: torch.Tensor, b=None, update=None):
     """The last product of a sublayer: [T, hidden], or 32-bit parts of it [parts, T, hidden] for a model whose residual update adds
-    them up (it sets ``takes_parts``)."""
+    them up (it sets ``takes_parts``); with ``update`` = (residual, the next norm's weights, eps) the product may do the update
+    itself and return the next sublayer's ``NormedRows``."""
+    if update is not None:
+        rows = sub.ops.linear_update(x, w, b, *update)
+        if rows is not None:
+            return rows
     return sub.ops.linear_parts(x, w, b) if getattr(sub, "takes_parts", False) else sub.ops.linear(x, w, b)
 
 
@@ -488,9 +493,9 @@ class WindowAttention:
         ops.window_attention(out, proj, cache, meta, s, self.gate_off, out_scale, self.lam, self.eps, self.sink_w)
         return out
 
-    def forward(self, h, meta, cache, state):
+    def forward(self, h, meta, cache, state, update=None):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return _last(self, self.mix(h, meta, cache, state, out), self.w_o, self.b_o)
+        return _last(self, self.mix(h, meta, cache, state, out), self.w_o, self.b_o, update)
 
 
 class Wkv:
@@ -649,9 +654,9 @@ class GatedDelta:
         ops.gated_delta(out, state, proj, *weights, decay, gate, offs, s, self.eps, meta)
         return out
 
-    def forward(self, h, meta, cache, state):
+    def forward(self, h, meta, cache, state, update=None):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return _last(self, self.mix(h, meta, cache, state, out), self.w_o)
+        return _last(self, self.mix(h, meta, cache, state, out), self.w_o, None, update)
 
 
 class DeltaRule:
@@ -696,9 +701,9 @@ class DeltaRule:
         ops.delta_rule(out, state, proj, wl, self.a_b, self.w0, self.norm, self.spec, self.eps, meta, out_scale)
         return out
 
-    def forward(self, h, meta, cache, state):
+    def forward(self, h, meta, cache, state, update=None):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return _last(self, self.mix(h, meta, cache, state, out), self.w_o)
+        return _last(self, self.mix(h, meta, cache, state, out), self.w_o, None, update)
 
 
 class MLstm:
@@ -862,7 +867,7 @@ class ParallelMixer:
             ys.append(self.ops.linear(out, m.w_o, getattr(m, "b_o", None)))
         return NormedPair(ys[0], self.left_norm, ys[1], self.right_norm, self.spec.left_scale, self.spec.right_scale)
 
-    def forward(self, h, meta, cache, state):
+    def forward(self, h, meta, cache, state, update=None):
         if self.spec.out_norms:
             return self._forward_normed(h, meta, cache, state)
         a, b = self.left.out_size, self.right.out_size
@@ -871,10 +876,10 @@ class ParallelMixer:
             proj = self.ops.linear(h, self.w_in)
             self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale, proj[:, :self.split])
             self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale, proj[:, self.split:])
-            return _last(self, buf, self.w_o)
+            return _last(self, buf, self.w_o, None, update)
         self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale)
         self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale)
-        return _last(self, buf, self.w_o)
+        return _last(self, buf, self.w_o, None, update)
 
 
 class DenseFF:
@@ -909,11 +914,11 @@ class DenseFF:
             t["gate"] = _rand(gen, self.spec.ff, self.hidden, std=std * 4)
         return t
 
-    def forward(self, h):
+    def forward(self, h, update=None):
         ff, act = self.spec.ff, self.spec.act
         c0 = self.spec.limit if act == "clamped_glu" else self.c0
         if act != "polynorm" and not self.side_rows:
-            return _last(self, self.ops.linear(h, self.w_up, act=act, c0=c0, c1=self.c1), self.w_down)
+            return _last(self, self.ops.linear(h, self.w_up, act=act, c0=c0, c1=self.c1), self.w_down, None, update)
         up = self.ops.linear(h, self.w_up)
         _side(self, up)
         out = torch.empty(h.shape[0], ff, device=h.device, dtype=h.dtype)
@@ -921,7 +926,7 @@ class DenseFF:
             self.ops.polynorm(out, up[:, :ff], self.coef, self.eps)
         else:
             self.ops.activation(out, up[:, :2 * ff] if act == "clamped_glu" else up[:, :ff], act, c0, self.c1)
-        return _last(self, out, self.w_down)
+        return _last(self, out, self.w_down, None, update)
 
 
 class RoutedMoE:

@@ -98,6 +98,18 @@ def native_available() -> bool:
         return False
 
 
+class NormedRows:
+    """Rows [T, H] before their norm's factor: row t is to be multiplied by 1 / sqrt(sum of squares[t] / H + eps). What
+    ``KernelOps.linear_update`` leaves; ``KernelOps.linear`` takes them in place of a tensor."""
+
+    def __init__(self, rows, squares, eps: float):
+        self.rows, self.squares, self.eps = rows, squares, eps
+        self.shape, self.dtype, self.device = rows.shape, rows.dtype, rows.device
+
+    def normed(self):
+        return (self.rows.float() * torch.rsqrt(self.squares.sum(1, keepdim=True) / self.shape[1] + self.eps)).to(self.dtype)
+
+
 class KernelOps:
     """gfx950 HIP kernels (all outputs written in place; graph-capturable)."""
 
@@ -495,13 +507,17 @@ class KernelOps:
         rows 14.6 / 8.0 / 7.5 / 7.5, 15.1 / 9.7 / 8.4 / 8.1, 14.7 / 12.8 / 10.2 / 9.1; 2048 x 2048 with 1, 16, 48 rows 14.0 / 7.9 / 7.7 / 8.3, 14.3 /
         8.8 / 8.2 / 8.9, 14.3 / 10.7 / 9.6 / 10.4; 2048 x 6144 with 16, 48 rows 14.6 / 14.2 / 11.4 / 11.8, 19.9 / 20.2 / 14.6 / 14.0; 4096 x 4096
         with 24 rows 16.7 / 13.7 / 14.7 / 15.6; 4096 x 12288 with 48 rows 35.0 / 36.7 / 32.1 / 28.8. Three or six parts were never best."""
-        def time(p):
-            return KernelOps.skinny_time(rows, cols, k, False, f32, p) + (p > 1) * 0.7 + (p - 1) * (0.15 + 0.5e-5 * rows * cols)
-
-        ours, parts = min((time(p), p) for p in (1, 2, 4) if p == 1 or p * 512 <= k * (2 if f32 else 1))
-        if ours > 0.94 * time(1):   # no more parts for what the model cannot tell
-            ours, parts = time(1), 1
+        ours, parts = min((KernelOps.parts_time(rows, cols, k, f32, p), p) for p in (1, 2, 4))
+        one = KernelOps.parts_time(rows, cols, k, f32, 1)
+        if ours > 0.94 * one:   # no more parts for what the model cannot tell
+            ours, parts = one, 1
         return parts if ours < KernelOps._vendor_time(rows, cols, k, f32) else 0
+
+    @staticmethod
+    def parts_time(rows, cols, k, f32, p) -> float:
+        if p > 1 and p * 512 > k * (2 if f32 else 1):
+            return float("inf")
+        return KernelOps.skinny_time(rows, cols, k, False, f32, p) + (p > 1) * 0.7 + (p - 1) * (0.15 + 0.5e-5 * rows * cols)
 
     def linear_parts(self, x, w, bias=None):
         """``linear`` for a result that ``scaled_add_group_rmsnorm`` takes as ``mix``: where that is faster, 32-bit sums over parts of k,
@@ -525,6 +541,13 @@ class KernelOps:
         """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands; ``act_from``: the first column that
         the activation applies to. A few rows run the weight-streaming kernel with the activation in its epilogue, anything else the
         vendor's GEMM and a second launch."""
+        if isinstance(x, NormedRows):
+            if self._skinny_ok(x.rows, w) and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())):
+                N = w.shape[0] // 2 if act in self.GLU_ACTS else w.shape[0]
+                out = torch.empty(x.shape[0], N, device=x.device, dtype=torch.float32 if out_f32 else x.dtype)
+                self._moe_lib.skinny_linear_normed(out, x.rows, x.squares, x.eps, w, bias, -1 if act is None else self.ACTIVATIONS[act], c0, c1, act_from)
+                return out
+            x = x.normed()
         if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())):
             glu = act in self.GLU_ACTS
             T, N, K = x.shape[0], w.shape[0], w.shape[1]
@@ -545,6 +568,24 @@ class KernelOps:
             return y
         out = torch.empty(*y.shape[:-1], y.shape[-1] // 2, device=y.device, dtype=y.dtype) if act in self.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)
+
+    NORM_ROWS = 32   # rows that ``linear_update`` takes
+
+    def linear_update(self, x, w, bias, residual, norm_w, eps):
+        """residual += x . w^T + bias, and the rows for the next products as ``NormedRows`` of its norm; None, and nothing done, where the
+        update and norm are a launch of their own. What that launch costs in a captured step (2.5 us, and 0.05 per row and 1024 columns) is
+        weighed against k in parts (``linear_parts``), which needs it, and against the loads that both products do more."""
+        T, N, K = x.shape[0], w.shape[0], w.shape[1]
+        if not (0 < T <= self.NORM_ROWS and N % 64 == 0 and N <= 4096 and self._skinny_ok(x, w) and residual.is_contiguous() and residual.data_ptr() % 16 == 0
+                and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous()))):
+            return None
+        f32 = x.dtype == torch.float32
+        apart = min(self._vendor_time(T, N, K, f32), min(self.parts_time(T, N, K, f32, p) for p in (1, 2, 4)))
+        if self.skinny_time(T, N, K, False, f32) + 0.6 > apart + 2.5 + 0.05 * T * N / 1024:
+            return None
+        rows, squares = torch.empty(T, N, device=x.device, dtype=x.dtype), torch.empty(T, N // 16, device=x.device, dtype=torch.float32)
+        self._moe_lib.skinny_linear_update(rows, squares, residual, norm_w, x, w, bias)
+        return NormedRows(rows, squares, eps)
 
     def linear_heads(self, out, x, w) -> bool:
         """out[h] = x[h] . w[h]^T for a few bf16 rows (x [heads, T, K], w [heads, N, K], out [heads, T, N], strided rows);
@@ -943,6 +984,9 @@ class ReferenceOps:
 
     def linear_parts(self, x, w, bias=None):
         return self.linear(x, w, bias)
+
+    def linear_update(self, x, w, bias, residual, norm_w, eps):
+        return None
 
     def linear_heads(self, out, x, w) -> bool:
         return False

@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from hipserve.ops import get_ops
+from hipserve.ops import NormedRows, get_ops
 from hipserve.ops import reference as ref
 
 gpu = pytest.mark.gpu
@@ -166,6 +166,36 @@ def test_product_in_parts(M, N, K, parts, dtype):
     assert ((r.double().cpu() - sums).abs() <= 2.0 ** -20 * (res.double().abs() + 4 * ls.double().abs() * (1 + want.abs())) + 1e-5).all()
     n = sums * torch.rsqrt(sums.square().mean(-1, keepdim=True) + 1e-6) * norm.double()
     assert ((h.double().cpu() - n).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -17) * n.abs() + 2e-5).all()
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,H,K,N,act", [(1, 64, 96, 40, None), (3, 1024, 520, 96, "xielu"), (9, 2112, 1024, 130, "silu_mul"), (16, 4096, 128, 4128, "tanh"),
+                                         (17, 128, 64, 16, None), (32, 1024, 3080, 5008, None)])
+def test_norm_inside_the_products(M, H, K, N, act, dtype):
+    """The residual update in one product and the norm's factor in the next: blocks of squares that fill a row's lanes partly, one and two
+    tiles per workgroup, a bias in both, every row group."""
+    g = torch.Generator().manual_seed(M + H)
+    x, w, b = torch.randn(M, K, generator=g).to(dtype), (torch.randn(H, K, generator=g) / K ** 0.5).to(dtype), torch.randn(H, generator=g).to(dtype)
+    res, norm = torch.randn(M, H, generator=g) * 3, 1 + 0.1 * torch.randn(H, generator=g)
+    w2, b2 = (torch.randn(N, H, generator=g) / H ** 0.5).to(dtype), torch.randn(N, generator=g).to(dtype)
+    ops, r = get_ops("cuda"), res.cuda()
+    rows = torch.empty(M, H, dtype=dtype, device="cuda")
+    squares = torch.full((M, H // 16), float("nan"), device="cuda")
+    ops._moe_lib.skinny_linear_update(rows, squares, r, norm.cuda(), x.cuda(), w.cuda(), b.cuda())
+    want = res.double() + x.double() @ w.double().T + b.double()
+    close_to(r, want, x, w)
+    close_to(rows, want * norm.double(), x, w, scale=2.0)
+    assert torch.allclose(squares.double().cpu().sum(1), want.square().sum(1), rtol=1e-5)
+    h = NormedRows(rows, squares, 1e-6)
+    for first in (0, 8) if act == "tanh" else (0,):
+        got = ops.linear(h, w2.cuda(), b2.cuda(), act=act, c0=0.7, c1=0.9, act_from=first)
+        # of the rows as they are; the factor's and the product's 32-bit sums
+        n = rows.double().cpu() * torch.rsqrt(squares.double().cpu().sum(1, keepdim=True) / H + 1e-6)
+        z = n @ w2.double().T + b2.double()
+        y = act64(z, act, 0.7, 0.9)
+        close_to(got, torch.cat([z[:, :first], y[:, first:]], 1) if first else y, n, w2, scale=12.0)
+    assert torch.allclose(h.normed().double().cpu(), n, rtol=2.0 ** -7 if dtype == torch.bfloat16 else 1e-5, atol=1e-6)
 
 
 @gpu
