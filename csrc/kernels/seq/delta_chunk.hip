@@ -35,7 +35,10 @@ HS_DEVICE bool find_chunk(const int* __restrict__ seq_cu, int nseq, int id, int&
   return false;
 }
 
-// Buffers per (chunk, head): W, GQ [16][DP], KT [DP][16], GE [DP], UT [VP][16], P [16][16]
+// Buffers per (chunk, head): W, GQ [16][DP], KT [DP][16], GE [DP], UT [VP][16], P [16][16]. The first four lie as the scan's lanes take
+// them, a tile of 16 x 16 as 64 times four numbers (`in_tiles`): a load of 1 KB side by side is looked up in a quarter of the steps that
+// 64 lanes take which jump from row to row. 8192 rows (4 prompts) x 16 heads, all kernels of the rule: 424 -> 401 us, 16 prompts of 200:
+// 209 -> 198 (the same in delta_rule_chunk.hip, which loads less: 374 -> 372, not worth its longer places).
 struct ChunkBuf {
   float *W, *GQ, *KT, *GE, *UT, *P;
 };
@@ -49,6 +52,15 @@ HS_DEVICE ChunkBuf chunk_buf(float* base, long item, int DP, int VP) {
   b.UT = b.GE + DP;
   b.P = b.UT + kC * VP;
   return b;
+}
+
+// Where (a, b) of an operand lies whose lane (a % 16, g) holds b = 16 t + 4 g .. + 3 of the tile t (W, GQ: token, channel), or, with a and b
+// swapped, (channel, token): tiles go along the channels.
+HS_DEVICE int in_tiles(int token, int channel) {
+  return ((channel >> 4) * 64 + (channel >> 2 & 3) * 16 + token) * 4 + (channel & 3);
+}
+HS_DEVICE int in_tiles_t(int channel, int token) {
+  return ((channel >> 4) * 64 + (token >> 2) * 16 + (channel & 15)) * 4 + (token & 3);
 }
 
 // 16 DPP rows of 16 lanes: row i is token i; lane `seg` of a row owns channels 16 VD j + VD seg + e (DS in all).
@@ -153,7 +165,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
     Row<float, VD>::ld(&sg[0][c], g);
 #pragma unroll
     for (int e = 0; e < VD; ++e) { xk[j][e] *= g[e]; xq[j][e] *= g[e]; }   // G_i k_i, G_i q_i
-    Row<float, VD>::st(out.GQ + row * DP + c, xq[j]);
+    Row<float, VD>::st(out.GQ + in_tiles(row, c), xq[j]);
     if (row == 0) Row<float, VD>::st(out.GE + c, ge[j]);
   }
   __syncthreads();   // sk, sg are read, sA is written
@@ -195,12 +207,12 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
   for (int j = 0; j < NJ; ++j) {
 #pragma unroll
     for (int e = 0; e < VD; ++e) w[j][e] = -w[j][e];
-    Row<float, VD>::st(out.W + row * DP + 16 * VD * j + VD * seg, w[j]);
+    Row<float, VD>::st(out.W + in_tiles(row, 16 * VD * j + VD * seg), w[j]);
   }
   // G_15 / G k, transposed
   for (int i = tid; i < DP * (kC / 4); i += 256) {
     const int c = i >> 2, q = 4 * (i & 3);
-    *reinterpret_cast<f32x4*>(out.KT + 4 * i) = f32x4{sk[q][c], sk[q + 1][c], sk[q + 2][c], sk[q + 3][c]};
+    *reinterpret_cast<f32x4*>(out.KT + in_tiles_t(c, q)) = f32x4{sk[q][c], sk[q + 1][c], sk[q + 2][c], sk[q + 3][c]};
   }
   // U0 = M v, transposed, a value channel per thread
   for (int v = tid; v < VP; v += 256) {
@@ -215,7 +227,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
     }
 #pragma unroll
     for (int q = 0; q < kC; q += 4)
-      *reinterpret_cast<f32x4*>(out.UT + (long)v * kC + q) = f32x4{u[q], u[q + 1], u[q + 2], u[q + 3]};
+      *reinterpret_cast<f32x4*>(out.UT + in_tiles_t(v, q)) = f32x4{u[q], u[q + 1], u[q + 2], u[q + 3]};
   }
 }
 
@@ -262,18 +274,18 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
     f32x4 W[TPW], Q[TPW], K[TPW], E[TPW], U;
     float p[KPW];
   } ops[kAhead];
-  const unsigned ucol = min(v0 + 16 * mine + c, VP - 1);
+  const unsigned u_at = (min(v0 / 16 + mine, VP / 16 - 1) * 64 + lane) * 4;
   auto fetch = [&](Ops& x, int ci) {
     const ChunkBuf b = chunk_buf(base, (long)(first + min(ci, nc - 1)) * heads + h, DP, VP);
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
-      const unsigned k0 = 16 * (wave * TPW + i), at = c * DP + k0 + 4 * g;
+      const unsigned k0 = 16 * (wave * TPW + i), at = ((wave * TPW + i) * 64 + lane) * 4;
       x.W[i] = *reinterpret_cast<const f32x4*>(b.W + at);
       x.Q[i] = *reinterpret_cast<const f32x4*>(b.GQ + at);
-      x.K[i] = *reinterpret_cast<const f32x4*>(b.KT + (k0 + c) * kC + 4 * g);
+      x.K[i] = *reinterpret_cast<const f32x4*>(b.KT + at);
       x.E[i] = *reinterpret_cast<const f32x4*>(b.GE + k0 + 4 * g);
     }
-    x.U = *reinterpret_cast<const f32x4*>(b.UT + ucol * kC + 4 * g);
+    x.U = *reinterpret_cast<const f32x4*>(b.UT + u_at);
 #pragma unroll
     for (int i = 0; i < KPW; ++i) x.p[i] = b.P[64 * (wave * KPW + i) + lane];
   };
