@@ -89,6 +89,11 @@ void launch_latent_attention_reduce(void* o_lat, const float* ws_acc, const floa
                                     int gate_off, int nparts, int heads, int rows_bound, int row_base, int T, int kv_rank,
                                     hipStream_t s);
 
+// mingru_scan of steps of one row per sequence with the product that makes proj, x [M, K] . w [3 * width, K]^T, M <= 64: x rows and w at
+// multiples of 16 bytes.
+bool launch_mingru_product(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x,
+                           const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, bool f32,
+                           hipStream_t s);
 // minGRU over the step's rows of every sequence, from / to its fp32 state slot.
 void launch_mingru_scan(void* y, float* state, const void* proj, const float* b_z, const float* b_x,
                         const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int width, int max_q,

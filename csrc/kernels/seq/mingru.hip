@@ -9,9 +9,14 @@
 // sigmoids from a full division: 171 us for 8192 rows (4 prompts) x 4096 in bf16, now 100. Two launches over segments of
 // 64 rows (fold, replay; 4 channels per thread) fill the card whatever the sequences are, but compute z and c twice: 188.
 //
-// Decode steps (mingru_step): one row per sequence needs no folding; 4 channels per thread, 9.1 -> 5.0 us for 41 sequences.
-#include "seq_common.h"
+// Decode steps (mingru_step): one row per sequence needs no folding; 4 channels per thread, 9.1 -> 5.0 us for 41 sequences. Up to 64 of
+// them run in the epilogue of the product that makes z, x and g (mingru_product): a workgroup has all three of its 16 channels,
+// unrounded, and the states arrive beside its weights. Width 4096, K 2048, in a captured step: one row 11.6 + 4.4
+// -> 12.0 us, 48 rows 16.0 + 4.7 -> 15.4.
+#include "skinny.h"
 #include "hipserve/seq_kernels.h"
+
+#include <type_traits>
 
 namespace hipserve {
 namespace {
@@ -121,6 +126,83 @@ __global__ __launch_bounds__(256) void mingru_step_kernel(T* __restrict__ y, flo
   Row<float, kV>::st(st, S);
 }
 
+// y, state of the rows x [M, K], one per sequence, and w = [z rows; x rows; g rows]. F32: x, w, x_ld and K in 16-bit halves (skinny.h).
+template <int XG, int DEPTH, bool F32>
+__global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
+    void* __restrict__ y_, float* state, const unsigned short* __restrict__ x, long x_ld, const unsigned short* __restrict__ w,
+    const float* b_z, const float* b_x, const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K) {
+  using SK = Skinny<XG, 3, DEPTH, F32>;
+  using T = std::conditional_t<F32, float, unsigned short>;
+  constexpr int ST = SK::ST, IT = (ST + 1) / 2;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  T* y = static_cast<T*>(y_);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n0 = blockIdx.x * 16, c = min(n0 + (tid & 15), width - 1);
+  const unsigned char* wt[3];
+  unsigned w_row[6], x_row[XG];
+#pragma unroll
+  for (int nt = 0; nt < 3; ++nt) {
+    wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)nt * width + n0) * K);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)(min(n0 + 8 * h + (lane >> 3), width - 1) - n0) * (unsigned)K * 2;
+  }
+#pragma unroll
+  for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)x_ld * 2;
+  f32x4 acc[3][ST];
+#pragma unroll
+  for (int nt = 0; nt < 3; ++nt)
+#pragma unroll
+    for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float bz, bx, S[IT];
+  long at[IT];   // the channel's place in the row's state, -1: the row has no sequence
+  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave, [&] {
+    bz = b_z[c];
+    bx = b_x[c];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      const int m = (tid + kSkThreads * i) >> 4;
+      at[i] = -1;
+      S[i] = 0.f;
+      if (m >= M) continue;
+      int s = min(m, nseq - 1), ctx = seq_ctx[s], slot = seq_state[s];
+      if (seq_cu[s] != m || seq_cu[s + 1] != m + 1) {   // sequences without a row lie between
+        for (s = 0; s < nseq && !(seq_cu[s] <= m && m < seq_cu[s + 1]);) ++s;
+        if (s == nseq) continue;
+        ctx = seq_ctx[s];
+        slot = seq_state[s];
+      }
+      at[i] = (long)slot * width + c;
+      if (ctx > 1) S[i] = state[at[i]];
+    }
+  });
+  float v[3][IT];
+  SK::reduce(v, acc, smem);
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int m = (tid + kSkThreads * i) >> 4;
+    if (m >= M || n0 + (tid & 15) >= width || at[i] < 0) continue;
+    const Gru g(v[0][i], v[1][i], bz, bx);
+    const float o = (1.f - g.z) * S[i] + g.zc;
+    stf<T>(y, (long)m * width + c, o * (v[2][i] * sigmoid_f(v[2][i])));
+    state[at[i]] = o;
+  }
+}
+
+template <int XG, int DEPTH>
+bool launch_product(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x, const int* seq_cu,
+                    const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, bool f32, hipStream_t s) {
+  constexpr int lds = Skinny<XG, 3, DEPTH>::kLds;
+  auto go = [&](auto* kernel) {
+    kernel<<<(width + 15) / 16, kSkThreads, lds, s>>>(y, state, (const unsigned short*)x, x_ld, (const unsigned short*)w, b_z, b_x, seq_cu,
+                                                       seq_ctx, seq_state, nseq, M, width, K);
+  };
+  static const bool ok = allow_lds(&mingru_product_kernel<XG, DEPTH, false>, lds) && allow_lds(&mingru_product_kernel<XG, DEPTH, true>, lds);
+  if (!ok) return false;
+  if (f32) go(&mingru_product_kernel<XG, DEPTH, true>);
+  else go(&mingru_product_kernel<XG, DEPTH, false>);
+  return true;
+}
+
 // Steps of one row per sequence: widths that are multiples of 4, everything at multiples of 16 bytes.
 template <typename T>
 void launch(T* y, float* state, const T* proj, const float* b_z, const float* b_x, const int* seq_cu, const int* seq_ctx,
@@ -137,6 +219,16 @@ void launch(T* y, float* state, const T* proj, const float* b_z, const float* b_
 }
 
 }  // namespace
+
+bool launch_mingru_product(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x,
+                           const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, bool f32,
+                           hipStream_t s) {
+  if (M <= 0 || nseq <= 0 || width <= 0) return true;
+  if (f32) { x_ld *= 2; K *= 2; }   // in halves
+#define HS_MG(XG, DEPTH) launch_product<XG, DEPTH>(y, state, x, x_ld, w, b_z, b_x, seq_cu, seq_ctx, seq_state, nseq, M, width, K, f32, s)
+  return M <= 8 ? HS_MG(1, 2) : M <= 16 ? HS_MG(2, 2) : M <= 32 ? HS_MG(4, 1) : M <= 48 ? HS_MG(6, 1) : HS_MG(8, 1);
+#undef HS_MG
+}
 
 void launch_mingru_scan(void* y, float* state, const void* proj, const float* b_z, const float* b_x,
                         const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int width, int max_q,

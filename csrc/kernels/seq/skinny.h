@@ -44,9 +44,11 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
   // acc[nt][st] += the products; lane (c, g) = (lane % 16, lane / 16) ends with columns 4 g .. + 3 of row 16 st + c. w[nt]: first row
   // of the tile; w_row[i] / x_row[j]: byte offsets of the lane's row (lane / 8 of the 8) in the half tile i (of 2 NT) from w[i / 2] and in
   // the group j of x from `x`. Every row is one that exists: what rows past the last one give is not used.
+  // started(): what a kernel loads besides, once the first copies are on their way.
+  template <typename F>
   static HS_DEVICE void accumulate(f32x4 (&acc)[NT][ST], const unsigned char* const (&w)[NT], const unsigned (&w_row)[2 * NT],
                                    const unsigned char* x, const unsigned (&x_row)[XG], int K, unsigned char* smem,
-                                   int lane, int wave) {
+                                   int lane, int wave, F&& started) {
     const int c = lane & 15, g = lane >> 4, r8 = lane >> 3;
     unsigned char* ring = smem + wave * DEPTH * kPiece;
     const unsigned lds0 = lds_at(ring);
@@ -80,6 +82,7 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i)
       if (i < n) copy(i);
+    started();   // its loads are younger: the waits below cover some of them too early at most
     for (int i = 0; i < n; ++i) {
       if (i + DEPTH <= n) wait_copies<kCopies * (DEPTH - 1)>();
       else wait_copies<0>();
@@ -121,6 +124,12 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
             }
           }
     }
+  }
+
+  static HS_DEVICE void accumulate(f32x4 (&acc)[NT][ST], const unsigned char* const (&w)[NT], const unsigned (&w_row)[2 * NT],
+                                   const unsigned char* x, const unsigned (&x_row)[XG], int K, unsigned char* smem,
+                                   int lane, int wave) {
+    accumulate(acc, w, w_row, x, x_row, K, smem, lane, wave, [] {});
   }
 
   // Sums the waves' parts: v[nt][i] = element (row, column) = (e / 16, e % 16), e = threadIdx.x + kSkThreads * i, of

@@ -72,6 +72,25 @@ void mingru_scan(at::Tensor& y, at::Tensor& state, const at::Tensor& proj, const
                                seq_state.data_ptr<int>(), nseq, width, max_q, f32, cur_stream());
 }
 
+// mingru_scan of the rows x [M, K] of a step in which every sequence has one row at most, the product x . w^T included.
+void mingru_product(at::Tensor& y, at::Tensor& state, const at::Tensor& x, const at::Tensor& w, const at::Tensor& b_z,
+                    const at::Tensor& b_x, const at::Tensor& seq_cu, const at::Tensor& seq_ctx, const at::Tensor& seq_state) {
+  CHECK_DEV(x); CHECK_CONTIG(w); CHECK_CONTIG(y); CHECK_F32(state); CHECK_F32(b_z); CHECK_F32(b_x);
+  CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_state);
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&y, &state, &w, &b_z, &b_x, &seq_cu, &seq_ctx, &seq_state}) CHECK_SAME_DEV(*t, x);
+  const bool f32 = is_f32(x, "mingru_product");
+  const long per = f32 ? 4 : 8, M = x.size(0), K = x.size(-1), width = state.size(1), nseq = seq_ctx.numel();
+  TORCH_CHECK(y.scalar_type() == x.scalar_type() && w.scalar_type() == x.scalar_type());
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && state.dim() == 2 && w.size(0) == 3 * width && w.size(1) == K && y.numel() == M * width && M <= 64);
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % per == 0 && K % per == 0 && K < (1L << 24) && x.stride(0) < (1L << 24) && width < (1L << 26) &&
+              (uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0, "mingru_product: rows at multiples of 16 bytes");
+  TORCH_CHECK(b_z.numel() == width && b_x.numel() == width && seq_cu.numel() == nseq + 1 && seq_state.numel() >= nseq);
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  TORCH_CHECK(hipserve::launch_mingru_product(y.data_ptr(), state.data_ptr<float>(), x.data_ptr(), x.stride(0), w.data_ptr(),
+                                              b_z.data_ptr<float>(), b_x.data_ptr<float>(), seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(),
+                                              seq_state.data_ptr<int>(), nseq, M, width, K, f32, cur_stream()), "mingru_product: LDS");
+}
+
 }  // namespace
 
 TORCH_LIBRARY(hipserve_seq, m) {
@@ -94,6 +113,8 @@ TORCH_LIBRARY(hipserve_seq, m) {
   m.def("latent_prompt_ok(int dim, int rot_dim, int vdim) -> bool", &latent_prompt_ok);
   m.def("latent_attention_dma_ok(int kv_rank, int rot_dim) -> bool", &latent_attention_dma_ok);
   m.def("latent_attention_mfma_ok(int kv_rank, int rot_dim) -> bool", &latent_attention_mfma_ok);
+  m.def("mingru_product(Tensor(a!) y, Tensor(b!) state, Tensor x, Tensor w, Tensor b_z, Tensor b_x, Tensor seq_cu, Tensor seq_ctx, "
+        "Tensor seq_state) -> ()");
   m.def("mingru_scan(Tensor(a!) y, Tensor(b!) state, Tensor proj, Tensor b_z, Tensor b_x, Tensor seq_cu, "
         "Tensor seq_ctx, Tensor seq_state, int max_q) -> ()");
 }
@@ -107,4 +128,5 @@ TORCH_LIBRARY_IMPL(hipserve_seq, CUDA, m) {
   m.impl("latent_gather", &latent_gather);
   m.impl("latent_prompt_attention", &latent_prompt_attention);
   m.impl("mingru_scan", &mingru_scan);
+  m.impl("mingru_product", &mingru_product);
 }

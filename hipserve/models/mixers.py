@@ -16,7 +16,7 @@ over the heads; everything between them is one op of the op set:
   instead, one product over the cache rows that the step sees, and attended to (``latent_prompt_attention``).
 * minGRU: merged [z | x | g] projection -> ``mingru_scan`` (gates, candidate, the
   recurrence over this step's tokens from the sequence's state slot, output gate) ->
-  output projection.
+  output projection. In decode steps the recurrence is the merged projection's epilogue.
 * table MoE: expert ids looked up by token id -> ``moe_align`` tiles (of all layers at once in small steps) -> two
   ``expert_gemm`` launches (squared-ReLU in the first one's epilogue); the weighted
   combine is folded into the residual update (``scaled_add_group_rmsnorm``).
@@ -274,9 +274,9 @@ class MinGRU:
         return (num_slots, self.spec.width)
 
     def forward(self, h: torch.Tensor, meta, state: torch.Tensor) -> torch.Tensor:
-        proj = self.ops.linear(h, self.w_in)
         y = torch.empty(h.shape[0], self.spec.width, device=h.device, dtype=h.dtype)
-        self.ops.mingru_scan(y, state, proj, self.b_z, self.b_x, meta)
+        if not self.ops.mingru_product(y, state, h, self.w_in, self.b_z, self.b_x, meta):
+            self.ops.mingru_scan(y, state, self.ops.linear(h, self.w_in), self.b_z, self.b_x, meta)
         return _last(self, y, self.w_o)
 
 

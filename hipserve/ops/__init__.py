@@ -331,6 +331,13 @@ class KernelOps:
                                            s0, s1, rows, tq, inv_freq, heads, dim, rot_dim, kv_rank, gate_off,
                                            scale, window)
 
+    def mingru_product(self, y, state, x, w, b_z, b_x, meta) -> bool:
+        """``mingru_scan`` of the product x . w^T for a step of one row per sequence; False, and nothing done, where they are two launches."""
+        if not (meta.max_q == 1 and x.dim() == 2 and self._skinny_ok(x, w) and self.skinny_pays(x.shape[0], w.shape[0], w.shape[1], False, x.dtype == torch.float32)):
+            return False
+        self._seq.mingru_product(y, state, x, w, b_z, b_x, meta.seq_cu, meta.seq_ctx, meta.seq_state)
+        return True
+
     def mingru_scan(self, y, state, proj, b_z, b_x, meta):
         self._seq.mingru_scan(y, state, proj, b_z, b_x, meta.seq_cu, meta.seq_ctx, meta.seq_state, meta.max_q)
 
@@ -880,6 +887,9 @@ class ReferenceOps:
 
     def latent_prompt_rows(self, dtype, sp, nfreq, cache, meta, T) -> int:
         return 0
+
+    def mingru_product(self, y, state, x, w, b_z, b_x, meta) -> bool:
+        return False
 
     def mingru_scan(self, y, state, proj, b_z, b_x, meta):
         ref.mingru_scan(y, state, proj, b_z, b_x, meta.seq_cu, meta.seq_ctx, meta.seq_state)

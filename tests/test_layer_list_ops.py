@@ -538,6 +538,32 @@ def test_window_attention_prompt_error(dim, size, sink):
 # ------------------------------------------------------------------ minGRU
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,width,K,gaps", [(1, 16, 64, ()), (3, 40, 520, (0, 2)), (16, 260, 1024, ()), (17, 1028, 136, (5,)), (41, 64, 2048, (41,)), (64, 30, 256, ())])
+def test_mingru_product(M, width, K, gaps, dtype):
+    """The decode step in its product's epilogue: every row group, channels that fill no tile, sequences without a row, fresh states."""
+    g = torch.Generator().manual_seed(M + width)
+    lens = [1] * M
+    for i in gaps:
+        lens.insert(i, 0)
+    n = len(lens)
+    wide = torch.randn(M, K + 16, generator=g).to(dtype)
+    x, w = wide[:, 8:8 + K], (torch.randn(3 * width, K, generator=g) / K ** 0.5).to(dtype)
+    state, bz, bx = torch.randn(n + 2, width, generator=g), torch.randn(width, generator=g), torch.randn(width, generator=g)
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    ctx = torch.tensor([m + (7 if i % 2 else 0) for i, m in enumerate(lens)], dtype=torch.int32)
+    slots = torch.randperm(n + 2, generator=g)[:n].int()
+    want_s, want = state.clone(), torch.empty(M, width)
+    ref.mingru_scan(want, want_s, (x.double() @ w.double().T).float(), bz, bx, cu, ctx, slots)
+    got_s, got = state.cuda(), torch.empty(M, width, dtype=dtype, device="cuda")
+    get_ops("cuda")._seq.mingru_product(got, got_s, wide.cuda()[:, 8:8 + K], w.cuda(), bz.cuda(), bx.cuda(), cu.cuda(), ctx.cuda(), slots.cuda())
+    # 32-bit sums of K products, and slopes of at most a few
+    err = 16 * K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T).max() + 64 * 2.0 ** -24 * 6
+    assert (got_s.cpu() - want_s).abs().max() < err
+    assert ((got.cpu().float() - want).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -18) * want.abs() + 8 * err).all()
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("width", [4, 260, 1028, 6])
 @pytest.mark.parametrize("lens", [[1], [1, 1, 1], [17], [16, 1, 256], [1, 300, 63]])
 def test_mingru_blocks(lens, width, dtype):
