@@ -70,26 +70,26 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // asked for before the copies, which then hide them, and used after them: plain pointers, so that no copy is passed
   constexpr int IT = (ST + 1) / 2, SQ = 4;
   f32x4 sq[IT][SQ];
   float res[IT][NT];
-  if constexpr (NORM) {
+  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, k1 - k0, smem, lane, wave, [&] {
+    if constexpr (NORM) {   // used in the epilogue
 #pragma unroll
-    for (int i = 0; i < IT; ++i) {
-      const int m = (tid + kSkThreads * i) >> 4, c = tid & 15;
+      for (int i = 0; i < IT; ++i) {
+        const int m = (tid + kSkThreads * i) >> 4, c = tid & 15;
 #pragma unroll
-      for (int j = 0; j < SQ; ++j) {
-        sq[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        if (norm.residual == nullptr && m < M && 64 * j + 4 * c < norm.blocks)
-          sq[i][j] = *reinterpret_cast<f32x4*>(norm.squares + (long)m * norm.blocks + 64 * j + 4 * c);
+        for (int j = 0; j < SQ; ++j) {
+          sq[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          if (norm.residual == nullptr && m < M && 64 * j + 4 * c < norm.blocks)
+            sq[i][j] = *reinterpret_cast<f32x4*>(norm.squares + (long)m * norm.blocks + 64 * j + 4 * c);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          res[i][nt] = norm.residual != nullptr && m < M ? norm.residual[(long)m * N + n0 + 16 * nt + c] : 0.f;
       }
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-        res[i][nt] = norm.residual != nullptr && m < M ? norm.residual[(long)m * N + n0 + 16 * nt + c] : 0.f;
     }
-  }
-  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, k1 - k0, smem, lane, wave);
+  });
   float v[NT][IT];
   SK::reduce(v, acc, smem);
   out += (long)blockIdx.y * out_bs;
