@@ -262,11 +262,12 @@ long delta_rule_chunk_floats(int T, int nseq, int heads);
 void launch_delta_rule_chunk(float* o, float* S, float* buf, const void* proj, long ld, const float* wl, const float* a_b,
                              const float* w0, const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int T,
                              int heads, hipStream_t s);
-// The generalized rule of steps in which every sequence has one row, heads of 64 (delta_rule_step.hip): one launch.
+// The generalized rule of steps in which every sequence has one row, heads of 64 (delta_rule_step.hip): one launch. With w2 [heads * 64,
+// rank] (a multiple of 32; 16-byte rows) wl is not read but formed, w2 times the rank columns of proj behind the five parts.
 bool delta_rule_step_ok(int dim);
 void launch_delta_rule_step(void* out, long out_ld, float* S, const void* proj, long ld, const float* wl, const float* a_b,
                             const float* w0, const float* norm_w, const int* seq_cu, const int* seq_ctx, const int* seq_state,
-                            int nseq, int heads, float eps, float out_scale, bool f32, hipStream_t s);
+                            int nseq, int heads, float eps, float out_scale, const void* w2, int rank, bool f32, hipStream_t s);
 // Token shift: out[nb, T, H] (activation type) = x + (previous row - x) * mu[b] from the 32-bit rows x; a
 // sequence's row before the step comes from state[slot] (zeros at position 0), which then gets the step's last row.
 void launch_token_shift(void* out, const float* x, float* state, const float* mu, const int* seq_cu,

@@ -5,7 +5,8 @@
 // the state, loaded by 16 bytes side by side; every wave prepares the 64 channels for itself (a lane each), so two
 // barriers, for the sums over the rows, are all. As three launches (five row vectors written as fp32 and read back, the state
 // read by 4-byte columns, one wave per head for the norm): 16 sequences x 32 heads in bf16 27.7 us, this 6.7
-// (one sequence x 16 heads 13.0, 4.5).
+// (one sequence x 16 heads 13.0, 4.5). The decays' bottleneck (its product w2 . low, 64 of its rows per head) can come with it: each wave sums
+// a quarter of the rank for all channels, 8 KB of weights beside the state's 16. One sequence, in a captured step: 2.4 + 4.3 -> 4.7 us.
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
 
@@ -14,11 +15,14 @@ namespace {
 
 constexpr int kD = 64;
 
-template <typename T>
+// w2 (LOW): [heads * 64, rank], rank a multiple of 32; the row's bottleneck lies behind the five parts of `proj`. Else wl is the product.
+template <typename T, bool LOW>
 __global__ __launch_bounds__(256) void delta_rule_step_kernel(
     T* __restrict__ out, long out_ld, float* __restrict__ S, const T* __restrict__ proj, long ld, const float* __restrict__ wl,
     const float* __restrict__ a_b, const float* __restrict__ w0, const float* __restrict__ norm_w, const int* __restrict__ seq_cu,
-    const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads, float eps, float out_scale) {
+    const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads, float eps, float out_scale,
+    const T* __restrict__ w2, int rank) {
+  __shared__ float decay[LOW ? 4 : 1][kD];
   __shared__ __attribute__((aligned(16))) float chan[4][5][kD];   // [wave] w, a, u, k, r
   __shared__ __attribute__((aligned(16))) float sums[2][4][kD];   // x, o: [wave]
   const int h = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -35,9 +39,26 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
 #pragma unroll
   for (int e = 0; e < 4; ++e) val[e] = ldf<T>(row, 2 * N + h * kD + v0 + e);
   const float k = ldf<T>(row, N + c), r = ldf<T>(row, c), a = ldf<T>(row, 3 * N + c), gate = ldf<T>(row, 4 * N + c);
+  float d = 0.f;
+  if constexpr (LOW) {
+    const int part = rank / 4, j0 = __builtin_amdgcn_readfirstlane(wave) * part;
+    const T *wr = w2 + (long)c * rank + j0, *lr = row + 5 * N + j0;
+    for (int j = 0; j < part; j += 8) {
+      float a8[8], b8[8];
+      Row<T, 8>::ld(wr + j, a8);
+      Row<T, 8>::ld(lr + j, b8);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d = __builtin_fmaf(a8[e], b8[e], d);
+    }
+    decay[wave][lane] = d;
+    __syncthreads();
+    d = (decay[0][lane] + decay[1][lane]) + (decay[2][lane] + decay[3][lane]);
+  } else {
+    d = wl[t * N + c];
+  }
   const float u = k / sqrtf(wave_sum(k * k) + 1e-6f);
   float(*mine)[kD] = chan[wave];
-  mine[0][lane] = expf(-0.60653065971263342f * sigmoid_f(wl[t * N + c] + w0[c]));
+  mine[0][lane] = expf(-0.60653065971263342f * sigmoid_f(d + w0[c]));
   mine[1][lane] = sigmoid_f(a + a_b[c]) * u;
   mine[2][lane] = u;
   mine[3][lane] = k;
@@ -78,15 +99,16 @@ bool delta_rule_step_ok(int dim) { return dim == kD; }
 
 void launch_delta_rule_step(void* out, long out_ld, float* S, const void* proj, long ld, const float* wl, const float* a_b,
                             const float* w0, const float* norm_w, const int* seq_cu, const int* seq_ctx, const int* seq_state,
-                            int nseq, int heads, float eps, float out_scale, bool f32, hipStream_t s) {
+                            int nseq, int heads, float eps, float out_scale, const void* w2, int rank, bool f32, hipStream_t s) {
   if (nseq <= 0) return;
   const dim3 grid(heads, nseq);
-  if (f32)
-    delta_rule_step_kernel<float><<<grid, 256, 0, s>>>((float*)out, out_ld, S, (const float*)proj, ld, wl, a_b, w0, norm_w, seq_cu,
-                                                       seq_ctx, seq_state, heads, eps, out_scale);
-  else
-    delta_rule_step_kernel<unsigned short><<<grid, 256, 0, s>>>((unsigned short*)out, out_ld, S, (const unsigned short*)proj, ld, wl,
-                                                                a_b, w0, norm_w, seq_cu, seq_ctx, seq_state, heads, eps, out_scale);
+#define HS_DRS(T, LOW)                                                                                                             \
+  delta_rule_step_kernel<T, LOW><<<grid, 256, 0, s>>>((T*)out, out_ld, S, (const T*)proj, ld, wl, a_b, w0, norm_w, seq_cu, seq_ctx, \
+                                                      seq_state, heads, eps, out_scale, (const T*)w2, rank)
+  if (f32) { if (w2 != nullptr) HS_DRS(float, true); else HS_DRS(float, false); }
+  else if (w2 != nullptr) HS_DRS(unsigned short, true);
+  else HS_DRS(unsigned short, false);
+#undef HS_DRS
 }
 
 }  // namespace hipserve

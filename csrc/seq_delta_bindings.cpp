@@ -242,10 +242,11 @@ void delta_rule(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const at
 bool delta_rule_step_ok(int64_t dim) { return hipserve::delta_rule_step_ok(dim); }
 
 // delta_rule of a step in which every sequence has one row.
-void delta_rule_step(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const at::Tensor& wl, const at::Tensor& a_b,
+void delta_rule_step(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const c10::optional<at::Tensor>& wl, const at::Tensor& a_b,
                      const at::Tensor& w0, const at::Tensor& norm_w, const at::Tensor& seq_cu, const at::Tensor& seq_ctx,
-                     const at::Tensor& seq_state, int64_t heads, int64_t dim, double eps, double out_scale) {
-  CHECK_DEV(proj); CHECK_F32(S); CHECK_F32(wl); CHECK_F32(a_b); CHECK_F32(w0); CHECK_F32(norm_w);
+                     const at::Tensor& seq_state, int64_t heads, int64_t dim, double eps, double out_scale,
+                     const c10::optional<at::Tensor>& w2) {
+  CHECK_DEV(proj); CHECK_F32(S); CHECK_F32(a_b); CHECK_F32(w0); CHECK_F32(norm_w);
   CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_state);
   const bool f32 = is_f32(proj, "delta_rule_step");
   const long T = proj.size(0), nseq = seq_ctx.numel(), N = heads * dim;
@@ -253,13 +254,23 @@ void delta_rule_step(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, con
   TORCH_CHECK(rows2d(proj) && proj.size(1) >= 5 * N && rows2d(out) && out.size(0) == T && out.size(1) == N);
   TORCH_CHECK(S.dim() == 4 && S.size(1) == heads && S.size(2) == dim && S.size(3) == dim &&
               reinterpret_cast<uintptr_t>(S.data_ptr()) % 16 == 0);
-  TORCH_CHECK(wl.numel() == T * N && a_b.numel() == N && w0.numel() == N && norm_w.numel() == N);
+  TORCH_CHECK(a_b.numel() == N && w0.numel() == N && norm_w.numel() == N && (wl.has_value() != w2.has_value()));
+  if (wl.has_value()) {
+    CHECK_F32(*wl);
+    TORCH_CHECK(wl->numel() == T * N);
+  } else {
+    CHECK_CONTIG(*w2); CHECK_SAME_DEV(*w2, proj);
+    const long R = w2->size(-1), el = f32 ? 4 : 2;
+    TORCH_CHECK(w2->dim() == 2 && w2->size(0) == N && w2->scalar_type() == proj.scalar_type() && R % 32 == 0 && proj.size(1) >= 5 * N + R &&
+                proj.stride(0) * el % 16 == 0 && reinterpret_cast<uintptr_t>(proj.data_ptr()) % 16 == 0 &&
+                reinterpret_cast<uintptr_t>(w2->data_ptr()) % 16 == 0, "delta_rule_step: bottleneck");
+  }
   TORCH_CHECK(seq_cu.numel() == nseq + 1 && seq_state.numel() >= nseq && nseq <= 65535);
   c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
   hipserve::launch_delta_rule_step(out.data_ptr(), out.stride(0), S.data_ptr<float>(), proj.data_ptr(), proj.stride(0),
-                                   wl.data_ptr<float>(), a_b.data_ptr<float>(), w0.data_ptr<float>(), norm_w.data_ptr<float>(),
+                                   (const float*)opt_ptr(wl), a_b.data_ptr<float>(), w0.data_ptr<float>(), norm_w.data_ptr<float>(),
                                    seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_state.data_ptr<int>(), nseq, heads,
-                                   (float)eps, (float)out_scale, f32, cur_stream());
+                                   (float)eps, (float)out_scale, opt_ptr(w2), w2.has_value() ? w2->size(1) : 0, f32, cur_stream());
 }
 
 // floats of delta_rule's `chunks`; 0: not for these rows
@@ -384,8 +395,8 @@ TORCH_LIBRARY(hipserve_delta, m) {
         "Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, Tensor(c!) scratch, int heads, int dim, float eps, "
         "float out_scale, Tensor(d!)? chunks=None) -> ()");
   m.def("delta_rule_step_ok(int dim) -> bool", &delta_rule_step_ok);
-  m.def("delta_rule_step(Tensor(a!) out, Tensor(b!) S, Tensor proj, Tensor wl, Tensor a_b, Tensor w0, Tensor norm_w, "
-        "Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, int heads, int dim, float eps, float out_scale) -> ()");
+  m.def("delta_rule_step(Tensor(a!) out, Tensor(b!) S, Tensor proj, Tensor? wl, Tensor a_b, Tensor w0, Tensor norm_w, "
+        "Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, int heads, int dim, float eps, float out_scale, Tensor? w2=None) -> ()");
   m.def("delta_rule_chunk_floats(Tensor proj, int nseq, int heads, int dim) -> int");
   m.def("add_normed(Tensor(a!) out, Tensor(b!) residual, Tensor w, float eps, Tensor? y, Tensor? ye, Tensor? pair_slot, "
         "Tensor? ids, Tensor? wts, int E, Tensor? h, Tensor? shared) -> ()");

@@ -697,6 +697,8 @@ class DeltaRule:
     def mix(self, h, meta, cache, state, out, out_scale: float = 1.0):
         N, ops = self.spec.size, self.ops
         proj = ops.linear(h, self.w_in, act="tanh", act_from=5 * N)
+        if ops.delta_rule_low(out, state, proj, self.w2, self.a_b, self.w0, self.norm, self.spec, self.eps, meta, out_scale):
+            return out
         wl = ops.linear(proj[:, 5 * N:], self.w2, out_f32=True)
         ops.delta_rule(out, state, proj, wl, self.a_b, self.w0, self.norm, self.spec, self.eps, meta, out_scale)
         return out

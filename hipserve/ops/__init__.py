@@ -458,6 +458,19 @@ class KernelOps:
                                      meta.seq_ctx, meta.seq_state, sp.heads, sp.kv_heads, sp.dim, sp.vdim, sp.conv, eps,
                                      *offs, sp.channel_decay, sp.gate_act == "silu")
 
+    DELTA_LOW_RANK = 128   # widest bottleneck that every (sequence, head) multiplies for itself
+
+    def delta_rule_low(self, out, state, proj, w2, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0) -> bool:
+        """``delta_rule`` of a decode step with the bottleneck's product (the last columns of ``proj`` times ``w2``) in its launch; False, and
+        nothing done, where it is a product before it."""
+        per = 16 // proj.element_size()
+        if not (meta.max_q == 1 and self._delta.delta_rule_step_ok(sp.dim) and w2.shape[1] % 32 == 0 and w2.shape[1] <= self.DELTA_LOW_RANK
+                and proj.dtype == w2.dtype and w2.is_contiguous() and proj.stride(0) % per == 0 and all(t.data_ptr() % 16 == 0 for t in (state[0], proj, w2))):
+            return False
+        self._delta.delta_rule_step(out, state[0], proj, None, a_b, w0, norm_w, meta.seq_cu, meta.seq_ctx, meta.seq_state,
+                                    sp.heads, sp.dim, eps, out_scale, w2)
+        return True
+
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
         def aligned(*tensors):   # the kernels below read and write 16 bytes at a time
             return all(t.data_ptr() % 16 == 0 for t in tensors)
@@ -975,6 +988,9 @@ class ReferenceOps:
     def sandwich_update(self, out, residual, w_next, eps, y=None, w_post=None, mult=1.0, table=None):
         ref.sandwich_update(out, residual, w_next, eps, y, w_post, mult, table)
         return out
+
+    def delta_rule_low(self, out, state, proj, w2, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0) -> bool:
+        return False
 
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
         ref.delta_rule(out, state[0], proj, wl, a_b, w0, norm_w, sp, eps, meta.seq_cu, meta.seq_ctx,

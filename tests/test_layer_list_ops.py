@@ -1019,6 +1019,33 @@ def test_delta_rule_step(dtype):
 
 
 @gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rank", [32, 96, 128])
+def test_delta_rule_low(rank, dtype):
+    """The decay bottleneck's product in the decode step's launch: one load per wave and more."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(rank)
+    H, d, cu = 3, 64, torch.tensor([0, 1, 2, 2, 3]).int()
+    N, T, n, eps = H * d, 3, 4, 1e-5
+    proj, w2 = torch.randn(T, 5 * N + rank + 8, generator=g).to(dtype), (torch.randn(N, rank, generator=g) / rank ** 0.5).to(dtype)
+    proj[:, 5 * N:] = proj[:, 5 * N:].tanh()
+    S = torch.randn(n + 1, H, d, d, generator=g)
+    a_b, w0, nw = torch.randn(N, generator=g), torch.randn(N, generator=g), torch.rand(N, generator=g) + 0.5
+    ctx, slots = torch.tensor([1, 9, 4, 2]).int(), torch.tensor([4, 0, 3, 1]).int()
+    sp, meta = SimpleNamespace(heads=H, dim=d, size=N), SimpleNamespace(seq_cu=cu.cuda(), seq_ctx=ctx.cuda(), seq_state=slots.cuda(), max_q=1)
+    want_s, want = S.clone(), torch.empty(T, N, dtype=dtype)
+    wl = (proj[:, 5 * N:5 * N + rank].double() @ w2.double().T).float()
+    ref.delta_rule(want, want_s, proj, wl, a_b, w0, nw, sp, eps, cu, ctx, slots, 1.5)
+    got_s, got = S.cuda(), torch.empty(T, N, dtype=dtype, device="cuda")
+    assert get_ops("cuda").delta_rule_low(got, [got_s], proj.cuda(), w2.cuda(), a_b.cuda(), w0.cuda(), nw.cuda(), sp, eps, meta, 1.5)
+    # a sum of 64 products, and `rank` of them in a decay, whose slope is at most 0.15
+    assert ((got_s.cpu() - want_s).abs() <= (64 + rank) * 2.0 ** -24 * want_s.abs().max()).all()
+    # the outputs of test_delta_rule_step, 2^-17 = 64 x 2^-23 for sums of 64 products, with `rank` products more
+    tol, least = (2.0 ** -7, 2.0 ** -13) if dtype == torch.bfloat16 else ((64 + rank) * 2.0 ** -23,) * 2
+    assert ((got.cpu().float() - want.float()).abs() <= tol * want.float().abs() + least * want.float().abs().max()).all()
+
+
+@gpu
 @pytest.mark.parametrize("rows", [1, 40])
 def test_delta_rule_unaligned(rows):
     """States and 32-bit rows that do not start at 16 bytes take the token by token kernels, as other sizes do."""
