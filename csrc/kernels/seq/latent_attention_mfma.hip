@@ -271,10 +271,21 @@ __global__ __launch_bounds__(128) void latent_attention_reduce_kernel(
     int row_base, int T_rows, int kv_rank) {
   __shared__ float sc[kMaxRuns];  // each run's weight e^(m_p - M) / L * gate, 0 for empty runs
   const int r = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  const long step = (long)heads * ws_rows * kv_rank;   // from run to run
+  const float* first = ws_acc + ((long)h * ws_rows + r) * kv_rank;
+  // the first runs' rows are asked for behind the weights, not after them: one row of 12 runs x 16 heads 4.8 -> 4.2 us
+  constexpr int kEarly = 12;
+  float m = -INFINITY, l = 0.f;
+  if (tid < min(nparts, 64)) {
+    const long w = ((long)tid * heads + h) * ws_rows + r;
+    m = ws_ml[2 * w];
+    l = ws_ml[2 * w + 1];
+  }
+  f32x4 early[kEarly];
+#pragma unroll
+  for (int i = 0; i < kEarly; ++i)
+    if (i < nparts && 4 * tid < kv_rank) early[i] = *reinterpret_cast<const f32x4*>(first + i * step + 4 * tid);
   if (tid < 64) {  // one wave: run p on lane p
-    const long w = ((long)min(tid, nparts - 1) * heads + h) * ws_rows + r;
-    const float m = tid < nparts ? ws_ml[2 * w] : -INFINITY;
-    const float l = tid < nparts ? ws_ml[2 * w + 1] : 0.f;
     const float M = wave_max(m);
     const float e = m > -INFINITY ? __expf(m - M) : 0.f;
     const float L = wave_sum(l * e);
@@ -285,9 +296,13 @@ __global__ __launch_bounds__(128) void latent_attention_reduce_kernel(
   const long trow = row_base + r;
   for (int d = 4 * tid; d < kv_rank; d += 512) {   // kv_rank % 4 == 0
     f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
-    const float* src = ws_acc + ((long)h * ws_rows + r) * kv_rank + d;
-    const long step = (long)heads * ws_rows * kv_rank;
-    for (int p0 = 0; p0 < nparts; p0 += 4) {   // four runs' loads in flight; an empty run (weight 0) is not read
+    const float* src = first + d;
+    if (d == 4 * tid) {
+#pragma unroll
+      for (int i = 0; i < kEarly; ++i)
+        if (i < nparts && sc[i] != 0.f) o += early[i] * sc[i];   // an empty run (weight 0) holds anything
+    }
+    for (int p0 = d == 4 * tid ? kEarly : 0; p0 < nparts; p0 += 4) {   // four runs' loads in flight; an empty run is not read
       f32x4 v[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
