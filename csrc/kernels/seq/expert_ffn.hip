@@ -247,10 +247,11 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
     const unsigned short* __restrict__ w, const int* __restrict__ slots, const int* __restrict__ tile_expert,
     int gather_k, int N, int K, int act, int E, const float* __restrict__ row_scale, float limit) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x & 63, slot0 = blockIdx.y * 32;
   const int e = tile_expert[blockIdx.y];
+  const unsigned long live = __ballot(slots[slot0 + (lane & 31)] >= 0);   // before the tile's expert is looked at: both loads in flight
   if (e < 0 || e >= E) return;
-  const int lane = threadIdx.x & 63;
-  const int slot0 = blockIdx.y * 32, No = GLU ? N / 2 : N, n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
+  const int No = GLU ? N / 2 : N, n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
   const unsigned char* wt[NT];
   unsigned w_row[2 * NT];
 #pragma unroll
@@ -262,7 +263,6 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
   }
 #define HS_ER(XG, DEPTH) \
   expert_rows<XG, NT, DEPTH, GLU>(out, x, x_ld, wt, w_row, slots, slot0, n0, No, gather_k, K, act, row_scale, limit, smem)
-  const unsigned long live = __ballot(slots[slot0 + (lane & 31)] >= 0);
   if (live >> 16 & 0xffff) HS_ER(4, 1);
   else if (live >> 8 & 0xff) HS_ER(2, 1);
   else HS_ER(1, 2);
