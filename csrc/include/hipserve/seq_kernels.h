@@ -204,12 +204,23 @@ void launch_window_attention_dma(void* out, long out_ld, const void* proj, long 
 
 // Decode rows (window_attention_decode.hip), bf16 or fp32: sequences seq0 .. seq0 + rows - 1 have up to that many rows, batch rows
 // row_base on; blocks of a power of two of rows; proj and cache rows at multiples of 16 bytes; nparts and part_keys as above.
+// prep (not null): launch_attn_prepare's work in the same launch, for steps of at most one row per sequence, on rows that are left as they
+// are. Heads of at most 128 dims (at 256 the registers spill), nfreq a multiple of 8, norms at multiples of 16 bytes; cache, positions and slots by batch row; own_kv false: only queries.
+struct WindowPrep {
+  void* cache;
+  const long *positions, *slots;
+  const float *inv_freq, *q_norm, *k_norm;
+  int nfreq, norm_mode, temp_every;
+  float eps, amp, temp_coef;
+  bool own_kv, v_norm;
+};
 bool window_attention_decode_ok(int dim, int vdim, int block_size, bool f32);
 void launch_window_attention_decode(void* out, long out_ld, const void* proj, long proj_ld, const void* cache, int block_size,
                                     const int* seq_cu, const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int rows,
                                     int row_base, int heads, int kv_heads, int dim, int gate_off, float scale, int window,
                                     bool sink, float out_scale, int nparts, int part_keys, float* ws_acc, float* ws_ml, int keep,
-                                    float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, hipStream_t s);
+                                    float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, const WindowPrep* prep,
+                                    hipStream_t s);
 
 // fp32 prompt portions of the sequences seq0 .. seq1 - 1 (the sizes of window_attention_decode_ok).
 void launch_window_attention_prompts_f32(float* out, long out_ld, const float* proj, long proj_ld, const float* cache, int block_size,

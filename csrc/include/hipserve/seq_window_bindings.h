@@ -137,12 +137,12 @@ inline bool window_attention_decode_ok(const at::Tensor& proj, const at::Tensor&
          reinterpret_cast<uintptr_t>(proj.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(cache.data_ptr()) % 16 == 0;
 }
 
-inline void window_attention_decode(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
+inline void window_decode(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
                            const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t seq0, int64_t row_base, int64_t heads,
                            int64_t kv_heads, int64_t dim, int64_t gate_off, double scale, int64_t window, bool sink,
                            double out_scale, int64_t nparts, int64_t part_keys, const c10::optional<at::Tensor>& ws_acc,
                            const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap,
-                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk) {
+                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk, const hipserve::WindowPrep* prep) {
   TORCH_CHECK(chunk >= 0 && (chunk == 0 || (window == 0 && keep == 0)), "window attention: chunks or a window");
   CHECK_DEV(proj); CHECK_CONTIG(cache); CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_bt);
   const bool f32 = is_f32(proj, "window_attention_decode");
@@ -173,7 +173,48 @@ inline void window_attention_decode(at::Tensor& out, const at::Tensor& proj, con
                                            cache.size(1), seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_bt.data_ptr<int>(),
                                            seq_bt.size(1), seq0, rows, row_base, heads, kv_heads, dim, gate_off, (float)scale,
                                            window, sink, (float)out_scale, nparts, part_keys, wa, wm, keep, (float)softcap,
-                                           (const float*)opt_ptr(sink_w), channel_gate, chunk, f32, cur_stream());
+                                           (const float*)opt_ptr(sink_w), channel_gate, chunk, f32, prep, cur_stream());
+}
+
+inline void window_attention_decode(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
+                           const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t seq0, int64_t row_base, int64_t heads,
+                           int64_t kv_heads, int64_t dim, int64_t gate_off, double scale, int64_t window, bool sink,
+                           double out_scale, int64_t nparts, int64_t part_keys, const c10::optional<at::Tensor>& ws_acc,
+                           const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap,
+                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk) {
+  window_decode(out, proj, cache, seq_cu, seq_ctx, seq_bt, seq0, row_base, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale,
+                nparts, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, nullptr);
+}
+
+// The two ops above for steps of at most one row per sequence; the queries in proj stay as they are.
+inline void window_attention_step(at::Tensor& out, const at::Tensor& proj, at::Tensor& cache, const at::Tensor& positions,
+                           const at::Tensor& slots, const at::Tensor& inv_freq, bool own_kv, const c10::optional<at::Tensor>& q_norm,
+                           const c10::optional<at::Tensor>& k_norm, int64_t norm_mode, bool v_norm, double eps, double amp,
+                           double temp_coef, int64_t temp_every, const at::Tensor& seq_cu,
+                           const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t heads,
+                           int64_t kv_heads, int64_t dim, int64_t gate_off, double scale, int64_t window, bool sink,
+                           double out_scale, int64_t nparts, int64_t part_keys, const c10::optional<at::Tensor>& ws_acc,
+                           const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap,
+                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk) {
+  CHECK_DEV(proj); CHECK_F32(inv_freq);
+  TORCH_CHECK(heads >= 1 && kv_heads >= 1 && temp_every >= 0 && temp_every < (1LL << 31) && norm_mode >= 0 && norm_mode <= 3);
+  const long T = proj.size(0), nq = heads * dim, nk = kv_heads * dim;
+  TORCH_CHECK(proj.dim() == 2 && dim <= 128 && proj.size(1) >= nq + (own_kv ? 2 * nk : 0));
+  TORCH_CHECK(positions.scalar_type() == at::kLong && slots.scalar_type() == at::kLong && positions.numel() >= T &&
+              slots.numel() >= T && positions.is_contiguous() && slots.is_contiguous());
+  TORCH_CHECK(2 * inv_freq.numel() <= dim && inv_freq.numel() % 8 == 0, "window_attention_step: rotated dims");
+  TORCH_CHECK((norm_mode == 1 || norm_mode == 2) == q_norm.has_value() && (!own_kv || q_norm.has_value() == k_norm.has_value()));
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&cache, &positions, &slots, &inv_freq}) CHECK_SAME_DEV(*t, proj);
+  for (const auto* w : {&q_norm, &k_norm})
+    if (w->has_value() && (own_kv || w == &q_norm)) {
+      CHECK_F32(**w); CHECK_SAME_DEV(**w, proj);
+      TORCH_CHECK((*w)->numel() == (norm_mode == 2 ? dim : w == &q_norm ? nq : nk) && (uintptr_t)(*w)->data_ptr() % 16 == 0);
+    }
+  const hipserve::WindowPrep prep{cache.data_ptr(), positions.data_ptr<long>(), slots.data_ptr<long>(), inv_freq.data_ptr<float>(),
+                                  (const float*)opt_ptr(q_norm), own_kv ? (const float*)opt_ptr(k_norm) : nullptr, (int)inv_freq.numel(),
+                                  (int)norm_mode, (int)temp_every, (float)eps, (float)amp, (float)temp_coef, own_kv, v_norm};
+  window_decode(out, proj, cache, seq_cu, seq_ctx, seq_bt, 0, 0, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale,
+                nparts, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, &prep);
 }
 
 inline void window_attention_prompts_f32(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
@@ -301,6 +342,11 @@ inline void def_window_ops(torch::Library& m) {
         "int seq0, int row_base, int heads, int kv_heads, int dim, int gate_off, float scale, int window, bool sink, "
         "float out_scale, int nparts, int part_keys, Tensor(b!)? ws_acc, Tensor(c!)? ws_ml, int keep, float softcap, "
         "Tensor? sink_w, bool channel_gate, int chunk) -> ()");
+  m.def("window_attention_step(Tensor(a!) out, Tensor proj, Tensor(b!) cache, Tensor positions, Tensor slots, Tensor inv_freq, "
+        "bool own_kv, Tensor? q_norm, Tensor? k_norm, int norm_mode, bool v_norm, float eps, float amp, float temp_coef, "
+        "int temp_every, Tensor seq_cu, Tensor seq_ctx, Tensor seq_bt, int heads, int kv_heads, int dim, int gate_off, float scale, "
+        "int window, bool sink, float out_scale, int nparts, int part_keys, Tensor(c!)? ws_acc, Tensor(d!)? ws_ml, int keep, "
+        "float softcap, Tensor? sink_w, bool channel_gate, int chunk) -> ()");
   m.def("window_attention_prompts_f32(Tensor(a!) out, Tensor proj, Tensor cache, Tensor seq_cu, Tensor seq_ctx, Tensor seq_bt, "
         "int seq0, int seq1, int rows_bound, int heads, int kv_heads, int dim, int gate_off, float scale, int window, bool sink, "
         "float out_scale, int keep, float softcap, Tensor? sink_w, bool channel_gate, int chunk) -> ()");
@@ -319,6 +365,7 @@ inline void impl_window_ops(torch::Library& m) {
   m.impl("window_attention_mfma", &window_attention_mfma);
   m.impl("window_attention_decode_ok", &window_attention_decode_ok);
   m.impl("window_attention_decode", &window_attention_decode);
+  m.impl("window_attention_step", &window_attention_step);
   m.impl("window_attention_prompts_f32", &window_attention_prompts_f32);
   m.impl("activation", &activation);
   m.impl("route_topk", &route_topk);

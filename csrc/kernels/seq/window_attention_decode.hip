@@ -57,14 +57,188 @@ HS_DEVICE float over_rows(float x) {   // over the lanes c, c + 16, c + 32, c + 
 
 using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
 
+struct NoPrep {};
+
+// 8 elements of a row as they lie in memory.
+template <typename T> struct Raw8 {
+  u32x4 w[sizeof(T) / 2];
+  HS_DEVICE void ld(const T* p) {
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 2; ++i) w[i] = reinterpret_cast<const u32x4*>(p)[i];
+  }
+  HS_DEVICE void get(float* f) const {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const unsigned u = sizeof(T) == 4 ? w[e / 4 % (sizeof(T) / 2)][e % 4] : (e & 1) ? w[0][e / 2] & 0xffff0000u : w[0][e / 2] << 16;
+      f[e] = __builtin_bit_cast(float, u);
+    }
+  }
+};
+
+// attn_prepare_vec_kernel's work for one workgroup of a decode step: its query heads, and the new key and value of their
+// key / value head, from the projection row into LDS (`heads` [nh][D], then key [D], value [D]), the latter two into the cache
+// row as well where `keep_row` says so. What is normed over the whole projection is summed by every workgroup of the row: 5 KB
+// for 16 + 4 heads of 128 in bf16, while the keys' addresses are on their way. `rows` asks for the first tile's places, `early` for the tile.
+template <typename T, int D, typename F, typename G>
+HS_DEVICE void prepare_row(const WindowPrep& pr, const T* __restrict__ row, long at, long slot, int head0, int nh, int kvh, int heads,
+                           int kv_heads, bool keep_row, T* hs, float* angles, F&& rows, G&& early) {
+  __shared__ float red[2][8];
+  constexpr int PER = D / 16, NS = sizeof(T) == 4 ? 4 : 8;   // NS: loads of the sums in flight beside the tile's, within the registers
+  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6;
+  const int nq = heads * D, nk = pr.own_kv ? kv_heads * D : 0, rot = pr.nfreq / 8, items = (nh + (pr.own_kv ? 2 : 0)) * PER;
+  const int chunks = pr.norm_mode == 1 ? (nq + nk) / 8 : 0;
+  int o0 = 0, o1 = 0;
+  auto place = [&](int it) {   // of an item: two 8-dim chunks of a head, as rotated pairs have them
+    const int h = it / PER, j = it % PER;
+    const bool pair = j < rot && h <= nh;
+    o0 = pair ? 8 * j : h <= nh ? 2 * pr.nfreq + 16 * (j - rot) : 16 * j;
+    o1 = o0 + (pair ? pr.nfreq : 8);
+    return row + (h < nh ? (head0 + h) * D : h == nh ? nq + kvh * D : nq + nk + kvh * D);
+  };
+  Raw8<T> lo{}, hi{}, sum[NS];
+  if (tid < items) {
+    const T* src = place(tid);
+    lo.ld(src + o0);
+    hi.ld(src + o1);
+  }
+#pragma unroll
+  for (int b = 0; b < NS; ++b)
+    if (b * nt < chunks) sum[b].ld(row + 8L * min(tid + b * nt, chunks - 1));
+  // Loads return in order, and a wait behind a branch is for all of them: what the preparation needs stands before the tile, and has
+  // landed when the tile's loads are issued (their addresses come from the block table, asked for at the same time).
+  auto landed = [] { __builtin_amdgcn_s_waitcnt(0x0f70); };   // vmcnt(0)
+  const bool weighed = pr.norm_mode == 1 || pr.norm_mode == 2;
+  float wl[8], wh[8];
+  auto weights = [&](int it) {   // place(it) is the last one
+    const int h = it / PER;
+    const float* w = (h < nh ? pr.q_norm : pr.k_norm) + (pr.norm_mode == 2 ? 0 : h < nh ? (head0 + h) * D : kvh * D);
+    Row<float, 8>::ld(w + o0, wl);
+    Row<float, 8>::ld(w + o1, wh);
+  };
+  if (weighed && tid < items && tid / PER <= nh) weights(tid);
+  const float freq = tid < pr.nfreq ? pr.inv_freq[tid] : 0.f;
+  rows();
+  landed();
+  float a = 0.f, b = 0.f;
+  for (int i0 = 0; i0 < chunks; i0 += NS * nt) {
+    if (i0 > 0) {
+#pragma unroll
+      for (int n = 0; n < NS; ++n)
+        if (i0 + n * nt < chunks) sum[n].ld(row + 8L * min(tid + i0 + n * nt, chunks - 1));
+      landed();
+    }
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+      const int i = tid + i0 + n * nt;
+      if (i0 + n * nt >= chunks || i >= chunks) continue;
+      float x[8], v[4] = {};
+      sum[n].get(x);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e & 3] += x[e] * x[e];
+      const float t = (v[0] + v[1]) + (v[2] + v[3]);
+      if (8 * i < nq) a += t; else b += t;
+    }
+  }
+  early();   // nothing that was asked for before is waited for behind this
+  const float pos = (float)at;
+  for (int i = tid; i < pr.nfreq; i += nt) {
+    float sn, cs;
+    float w = freq;
+    if (i >= nt) {
+      w = pr.inv_freq[i];
+      landed();
+    }
+    sincosf(pos * w, &sn, &cs);
+    angles[i] = cs * pr.amp;
+    angles[pr.nfreq + i] = sn * pr.amp;
+  }
+  if (pr.norm_mode == 1) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if (lane == 0) { red[0][wave] = a; red[1][wave] = b; }
+  }
+  __syncthreads();
+  float iq = 1.f, ik = 1.f;
+  if (pr.norm_mode == 1) {
+    a = b = 0.f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {   // one wait for all of them
+      const float u = red[0][w], t = red[1][w];
+      a += w < nt / 64 ? u : 0.f;
+      b += w < nt / 64 ? t : 0.f;
+    }
+    iq = 1.f / sqrtf(a / (float)nq + pr.eps);
+    ik = 1.f / sqrtf(b / (float)max(nk, 1) + pr.eps);
+  }
+  const float temp = pr.temp_every > 0 ? 1.f + pr.temp_coef * logf((float)((at + 1) / pr.temp_every) + 1.f) : 1.f;
+  T* dst = reinterpret_cast<T*>(pr.cache) + slot * (2L * kv_heads * D) + kvh * D;
+  for (int it = tid; (it & ~63) < items; it += nt) {   // whole waves: a head's sum is over its lanes
+    const bool live = it < items;
+    const T* src = place(min(it, items - 1));
+    if (it >= nt && live) {
+      lo.ld(src + o0);
+      hi.ld(src + o1);
+      if (weighed && it / PER <= nh) weights(it);
+      landed();
+    }
+    const int h = it / PER, j = it % PER;
+    const bool qk = h <= nh, isq = h < nh;
+    float x[8], y[8], v[4] = {};
+    lo.get(x);
+    hi.get(y);
+    const float grow = pr.norm_mode == 3 && j < rot && qk ? pr.amp : 1.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { const float w = x[e] * grow; v[e & 3] += w * w; }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { const float w = y[e] * grow; v[e & 3] += w * w; }
+    float f = isq ? iq : qk ? ik : 1.f, ss = (v[0] + v[1]) + (v[2] + v[3]);
+    if (pr.norm_mode >= 2 || pr.v_norm) {
+#pragma unroll
+      for (int o = 1; o < PER; o <<= 1) ss += __shfl_xor(ss, o, 64);
+      if (qk ? pr.norm_mode >= 2 : pr.v_norm) f = 1.f / sqrtf(ss / (float)D + pr.eps);
+    }
+    if (!live) continue;
+    if (isq) f *= temp;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) { x[e] *= f; y[e] *= f; }
+    if (qk && weighed) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) { x[e] *= wl[e]; y[e] *= wh[e]; }
+    }
+    if (qk && j < rot) {
+      float cs[8], sn[8];
+      Row<float, 8>::ld(angles + 8 * j, cs);
+      Row<float, 8>::ld(angles + pr.nfreq + 8 * j, sn);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float p = x[e], q = y[e];
+        x[e] = p * cs[e] - q * sn[e];
+        y[e] = q * cs[e] + p * sn[e];
+      }
+    }
+    Row<T, 8>::st(hs + h * D + o0, x);
+    Row<T, 8>::st(hs + h * D + o1, y);
+    if (!isq && keep_row) {
+      T* to = dst + (qk ? 0 : kv_heads * D);
+      Row<T, 8>::st(to + o0, x);
+      Row<T, 8>::st(to + o1, y);
+    }
+  }
+  __syncthreads();
+}
+
 // MULTI: prompt portions, tq tokens x hc heads in the 16 rows, tiles of tokens in blockIdx.x; one run.
-template <typename T, int D, bool MULTI>
+// PREP: the projection rows come as the product leaves them (one row per sequence), and the new key and value of a row reach its
+// own tile through LDS. Preparation and attention in captured steps, two launches -> this, in bf16 at 128 dims: one row of 8 heads over 2
+// 3.4 + 5.5 -> 7.7 us, 16 rows of 16 over 4 4.3 + 9.0 -> 11.0, 16 rows of 32 over 8 and 2000 keys 5.0 + 23.9 -> 27.6; fp32, 4 rows of 8
+// over 2 3.3 + 9.6 -> 11.6. With the tile's loads waited for before the sums 8.9, 11.4, 25.9 and 11.4.
+template <typename T, int D, bool MULTI, bool PREP = false>
 __global__ __launch_bounds__(512) void window_decode_kernel(
     T* __restrict__ out, long out_ld, const T* __restrict__ proj, long proj_ld, const T* __restrict__ cache, int block_shift,
     const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0,
     int seq1, int tq, int hc, int hchunks, int heads, int kv_heads, int gate_off, float scale, int window, bool sink, float out_scale,
     int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml, int keep, float softcap,
-    const float* __restrict__ sink_w, bool channel_gate, int chunk) {
+    const float* __restrict__ sink_w, bool channel_gate, int chunk, std::conditional_t<PREP, WindowPrep, NoPrep> prep) {
   constexpr bool F32 = sizeof(T) == 4;
   constexpr int SUB = F32 ? 1 : 2, KT = 16 * SUB;          // 16-key tiles and keys of a wave's tile
   constexpr int QN = F32 ? D / 16 : D / 32;                // 16-byte parts of a row per lane
@@ -99,11 +273,45 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
     const int j = u < nk ? u : u - nk + lo_all;
     return cache + (((long)bt[j >> block_shift] << block_shift) + (j & ((1 << block_shift) - 1))) * Dc;
   };
+  using Keys = u32x4[SUB][QN];
+  // as they lie in memory: 16-bit elements of their own are taken apart, and waited for, where they are loaded
+  using Part = __attribute__((ext_vector_type(E * sizeof(T) / 4))) unsigned;
+  using Values = Part[4 * SUB][NB];
+  using Rows = const T*[5 * SUB];
+  auto rows_of = [&](int u0, Rows& src) {
+#pragma unroll
+    for (int a = 0; a < SUB; ++a) src[a] = row_of(u0 + 16 * a + c) + (long)kvh * D;
+#pragma unroll
+    for (int i = 0; i < 4 * SUB; ++i) src[SUB + i] = row_of(u0 + 16 * (i >> 2) + 4 * g + (i & 3)) + (long)(kv_heads + kvh) * D + E * c;
+  };
+  auto load = [&](const Rows& src, Keys& k, Values& v) {
+#pragma unroll
+    for (int a = 0; a < SUB; ++a)
+#pragma unroll
+      for (int i = 0; i < QN; ++i) k[a][i] = reinterpret_cast<const u32x4*>(src[a])[4 * i + g];
+#pragma unroll
+    for (int i = 0; i < 4 * SUB; ++i)
+#pragma unroll
+      for (int b = 0; b < NB; ++b) v[i][b] = *reinterpret_cast<const Part*>(src[SUB + i] + 16 * E * b);
+  };
+  const int first = lo + wave * KT;
+  constexpr bool EARLY = PREP && D * sizeof(T) <= 256;      // the first tile fits the registers beside the preparation
+  T* hs = reinterpret_cast<T*>(lds + nw * (hc * D + 32));   // PREP: the prepared heads, key and value
+  bool fresh = false;                                       // the run ends with the row's own key
+  [[maybe_unused]] Keys k0;
+  [[maybe_unused]] Values v0;
+  [[maybe_unused]] Rows src0;
+  if constexpr (PREP) {
+    const long slot = prep.own_kv ? prep.slots[r0] : -1;
+    fresh = slot >= 0 && hi >= lo && hi == total - 1;
+    prepare_row<T, D>(prep, proj + r0 * proj_ld, prep.positions[r0], slot, head0, nh, kvh, heads, kv_heads, fresh && h0 == 0, hs,
+                      reinterpret_cast<float*>(hs + (hc + 2) * D), [&] { if (EARLY) rows_of(first, src0); }, [&] { if (EARLY && first <= hi) load(src0, k0, v0); });
+  }
   u32x4 q[QN];
 #pragma unroll
   for (int i = 0; i < QN; ++i) {
     q[i] = u32x4{0, 0, 0, 0};
-    if (act) q[i] = reinterpret_cast<const u32x4*>(proj + r0 * proj_ld + (long)head * D)[4 * i + g];
+    if (act) q[i] = reinterpret_cast<const u32x4*>(PREP ? hs + rh * D : proj + r0 * proj_ld + (long)head * D)[4 * i + g];
   }
   f32x4 acc[NB][E];
 #pragma unroll
@@ -114,20 +322,28 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
   float m = sunk ? (sink_w != nullptr ? sink_w[head] * S::kUnit : 0.f) : -INFINITY, l = sunk ? 1.f : 0.f;
   const float unit = scale * S::kUnit, cap = softcap * S::kUnit, icap = softcap > 0.f ? scale / softcap : 0.f;
 
-  for (int u0 = lo + wave * KT; u0 <= hi; u0 += nw * KT) {
-    u32x4 k[SUB][QN];
-    T v[4 * SUB][NB][E];
-#pragma unroll
-    for (int a = 0; a < SUB; ++a) {
-      const T* src = row_of(u0 + 16 * a + c) + (long)kvh * D;
-#pragma unroll
-      for (int i = 0; i < QN; ++i) k[a][i] = reinterpret_cast<const u32x4*>(src)[4 * i + g];
+  for (int u0 = first; u0 <= hi; u0 += nw * KT) {
+    Keys kl;
+    Values vl;
+    Keys& k = EARLY ? k0 : kl;
+    Values& v = EARLY ? v0 : vl;
+    if (!EARLY || u0 != first) {
+      Rows src;
+      rows_of(u0, src);
+      load(src, k, v);
     }
+    if (PREP && fresh && hi - u0 < KT) {   // the cache row is being written: its key and value are in LDS
+      const T* key = hs + nh * D;
 #pragma unroll
-    for (int i = 0; i < 4 * SUB; ++i) {
-      const T* src = row_of(u0 + 16 * (i >> 2) + 4 * g + (i & 3)) + (long)(kv_heads + kvh) * D + E * c;
+      for (int a = 0; a < SUB; ++a)
+        if (u0 + 16 * a + c == hi)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) __builtin_memcpy(v[i][b], __builtin_assume_aligned(src + 16 * E * b, E * sizeof(T)), E * sizeof(T));
+          for (int i = 0; i < QN; ++i) k[a][i] = reinterpret_cast<const u32x4*>(key)[4 * i + g];
+#pragma unroll
+      for (int i = 0; i < 4 * SUB; ++i)
+        if (u0 + 16 * (i >> 2) + 4 * g + (i & 3) == hi)
+#pragma unroll
+          for (int b = 0; b < NB; ++b) v[i][b] = *reinterpret_cast<const Part*>(key + D + E * c + 16 * E * b);
     }
     f32x4 sc[SUB];
 #pragma unroll
@@ -183,9 +399,7 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
       for (int i = 0; i < 4 * SUB; ++i)
         if (u0 + 16 * (i >> 2) + 4 * g + (i & 3) > hi)
 #pragma unroll
-          for (int b = 0; b < NB; ++b)
-#pragma unroll
-            for (int e = 0; e < E; ++e) v[i][b][e] = 0;
+          for (int b = 0; b < NB; ++b) v[i][b] = Part{};
     }
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
@@ -195,18 +409,14 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
 #pragma unroll
         for (int j = 0; j < E; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i][b][j], w[i], acc[b][j], 0, 0, 0);
+          for (int i = 0; i < 4; ++i) acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(float, (unsigned)v[i][b][j]), w[i], acc[b][j], 0, 0, 0);
       } else {
 #pragma unroll
         for (int j = 0; j < E; ++j) {
           u32x4 a;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {   // keys 2 r and 2 r + 1 of dim j
-            unsigned x, y;
-            __builtin_memcpy(&x, &v[2 * r][b][j & ~1], 4);
-            __builtin_memcpy(&y, &v[2 * r + 1][b][j & ~1], 4);
-            a[r] = __builtin_amdgcn_perm(y, x, j & 1 ? 0x07060302u : 0x05040100u);
-          }
+          for (int r = 0; r < 4; ++r)   // keys 2 r and 2 r + 1 of dim j
+            a[r] = __builtin_amdgcn_perm(v[2 * r + 1][b][j / 2], v[2 * r][b][j / 2], j & 1 ? 0x07060302u : 0x05040100u);
           acc[b][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, pk),
                                                               acc[b][j], 0, 0, 0);
         }
@@ -295,15 +505,25 @@ template <typename T, int D>
 void launch(T* out, long out_ld, const T* proj, long proj_ld, const T* cache, int block_size, const int* seq_cu,
             const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int rows, int row_base, int heads, int kv_heads,
             int gate_off, float scale, int window, bool sink, float out_scale, int nparts, int part_keys, float* ws_acc,
-            float* ws_ml, int keep, float softcap, const float* sink_w, bool channel_gate, int chunk, hipStream_t s) {
+            float* ws_ml, int keep, float softcap, const float* sink_w, bool channel_gate, int chunk, const WindowPrep* prep,
+            hipStream_t s) {
   const int group = heads / kv_heads, hc = std::min(group, 16), hchunks = (group + hc - 1) / hc;
-  // a wave per tile of the run, as many as their accumulators and sums fit 64 KB of LDS
+  // a wave per tile of the run, as many as their accumulators and sums (and the prepared heads and angles) fit 64 KB of LDS
   const int kt = sizeof(T) == 4 ? 16 : 32, wave_floats = hc * D + 32;
-  const int nw = std::max(1, std::min({8, (part_keys + kt - 1) / kt, (1 << 14) / wave_floats}));
-  const size_t smem = (size_t)nw * wave_floats * sizeof(float);
-  window_decode_kernel<T, D, false><<<dim3(rows, kv_heads * hchunks, nparts), 64 * nw, smem, s>>>(
-      out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq0 + rows, 1, hc,
-      hchunks, heads, kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk);
+  const int prepared = prep != nullptr ? ((hc + 2) * D * (int)sizeof(T) + 3) / 4 + 2 * prep->nfreq : 0, room = (1 << 14) - 16 - prepared;
+  const int nw = std::max(1, std::min({8, (part_keys + kt - 1) / kt, room / wave_floats}));
+  const size_t smem = ((size_t)nw * wave_floats + prepared) * sizeof(float);
+  const dim3 grid(rows, kv_heads * hchunks, nparts);
+  if constexpr (D <= 128) {
+    if (prep != nullptr)
+      window_decode_kernel<T, D, false, true><<<grid, 64 * nw, smem, s>>>(
+          out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq0 + rows, 1, hc, hchunks,
+          heads, kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, *prep);
+  }
+  if (prep == nullptr)
+    window_decode_kernel<T, D, false><<<grid, 64 * nw, smem, s>>>(
+        out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq0 + rows, 1, hc, hchunks,
+        heads, kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, NoPrep{});
   if (nparts > 1)
     window_decode_reduce_kernel<T><<<dim3(rows, heads), 128, 0, s>>>(out, out_ld, ws_acc, ws_ml, proj, proj_ld, gate_off, nparts,
                                                                     heads, rows, row_base, D, out_scale, channel_gate);
@@ -319,7 +539,7 @@ void launch_prompts(float* out, long out_ld, const float* proj, long proj_ld, co
   window_decode_kernel<float, D, true><<<dim3(rows_bound / tq + (seq1 - seq0), kv_heads * hchunks, 1), 64 * nw,
                                          (size_t)nw * wave_floats * sizeof(float), s>>>(
       out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, tq, hc, hchunks,
-      heads, kv_heads, gate_off, scale, window, sink, out_scale, 0, nullptr, nullptr, keep, softcap, sink_w, channel_gate, chunk);
+      heads, kv_heads, gate_off, scale, window, sink, out_scale, 0, nullptr, nullptr, keep, softcap, sink_w, channel_gate, chunk, NoPrep{});
 }
 
 }  // namespace
@@ -343,12 +563,13 @@ void launch_window_attention_decode(void* out, long out_ld, const void* proj, lo
                                     const int* seq_cu, const int* seq_ctx, const int* seq_bt, int bt_width, int seq0, int rows,
                                     int row_base, int heads, int kv_heads, int dim, int gate_off, float scale, int window,
                                     bool sink, float out_scale, int nparts, int part_keys, float* ws_acc, float* ws_ml, int keep,
-                                    float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, hipStream_t s) {
+                                    float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, const WindowPrep* prep,
+                                    hipStream_t s) {
   if (rows <= 0) return;
 #define HS_WD(T, D)                                                                                                        \
   launch<T, D>((T*)out, out_ld, (const T*)proj, proj_ld, (const T*)cache, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, \
                rows, row_base, heads, kv_heads, gate_off, scale, window, sink, out_scale, nparts, part_keys, ws_acc, ws_ml,   \
-               keep, softcap, sink_w, channel_gate, chunk, s)
+               keep, softcap, sink_w, channel_gate, chunk, prep, s)
   if (f32) { if (dim == 64) HS_WD(float, 64); else HS_WD(float, 128); }
   else if (dim == 64) HS_WD(unsigned short, 64);
   else if (dim == 128) HS_WD(unsigned short, 128);

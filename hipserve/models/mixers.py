@@ -23,7 +23,8 @@ over the heads; everything between them is one op of the op set:
 * window attention: merged [q | k | v | gate] projection (biases in its epilogue) ->
   ``attn_prepare`` (whole-projection or per-head q / k norm, rotation, value norm, paged cache
   write) -> ``window_attention`` (sliding window, softmax with a sink, per-head output gate; with
-  two maps per head the differential combination and its norm) -> output projection. A layer
+  two maps per head the differential combination and its norm) -> output projection. Both are one
+  launch in decode steps (``window_step``: one map, heads of 64 or 128 dims). A layer
   that reads another layer's cache projects only its queries.
 * linear attention with per-channel decays (``Wkv``): ``token_shift`` (five blends of the token's
   and the previous token's 32-bit input) -> one batched projection for r / k / v / gate and the
@@ -489,6 +490,8 @@ class WindowAttention:
         if proj is None:
             proj = self.ops.linear(h, self.w_in, self.b_in)
             _side(self, proj)
+        if ops.window_step(out, proj, cache, meta, self.inv_freq, s, self.q_norm, self.k_norm, self.eps, self.gate_off, out_scale, self.sink_w):
+            return out
         ops.attn_prepare(proj, cache, meta, self.inv_freq, s, self.q_norm, self.k_norm, self.eps)
         ops.window_attention(out, proj, cache, meta, s, self.gate_off, out_scale, self.lam, self.eps, self.sink_w)
         return out

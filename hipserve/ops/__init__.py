@@ -354,8 +354,20 @@ class KernelOps:
     WINDOW_MFMA = os.environ.get("HIPSERVE_WINDOW_MFMA", "1") != "0"
     WINDOW_DECODE_RUN = 128  # keys per run of a decode row (a multiple of 32)
 
-    def _window_decode(self, out, proj, cache, meta, sp, gate_off, out_scale, sink_w) -> bool:
-        """The decode rows of ``window_attention`` by the kernel for them; False where it does not take the sizes."""
+    def window_step(self, out, proj, cache, meta, inv_freq, sp, q_norm, k_norm, eps, gate_off, out_scale=1.0, sink_w=None) -> bool:
+        """``attn_prepare`` and ``window_attention`` of a decode step (one row per sequence) in one launch; False, and nothing done, where they
+        are two."""
+        if not (meta.max_q == 1 and meta.num_prefill_tokens == 0 and meta.num_decode == meta.seq_ctx.shape[0] > 0 and inv_freq.numel() % 8 == 0
+                and 2 * inv_freq.numel() <= sp.dim <= 128 and all(w is None or w.data_ptr() % 16 == 0 for w in (q_norm, k_norm))):
+            return False
+        mode, own_kv = 1 if sp.qk_norm else 2 if sp.head_norm else 3 if sp.unit_qk else 0, sp.kv_from is None
+        prep = (meta.positions, meta.slot_mapping, inv_freq, own_kv, q_norm if mode in (1, 2) else None, k_norm if mode in (1, 2) and own_kv else None,
+                mode, sp.v_norm, eps, sp.scaling.amplitude if sp.scaling is not None else 1.0, sp.temp_coef, sp.temp_every)
+        return self._window_decode(out, proj, cache, meta, sp, gate_off, out_scale, sink_w, prep)
+
+    def _window_decode(self, out, proj, cache, meta, sp, gate_off, out_scale, sink_w, prep=None) -> bool:
+        """The decode rows of ``window_attention`` by the kernel for them; False where it does not take the sizes. ``prep``: what is between
+        the cache and the table in ``window_attention_step``."""
         if sp.maps != 1 or not self.WINDOW_MFMA or not self._window_lib.window_attention_decode_ok(proj, cache, sp.dim, sp.vdim):
             return False
         nd = meta.num_decode
@@ -376,10 +388,13 @@ class KernelOps:
         if nparts > 1:
             ws_acc = torch.empty(nparts, sp.heads, nd, sp.vdim, device=proj.device, dtype=torch.float32)
             ws_ml = torch.empty(nparts, sp.heads, nd, 2, device=proj.device, dtype=torch.float32)
-        self._window_lib.window_attention_decode(out, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt,
-                                                 meta.seq_ctx.shape[0] - nd, meta.num_prefill_tokens, sp.heads, sp.kv_heads, sp.dim,
-                                                 gate_off, sp.scale, sp.window, sp.sink, out_scale, nparts, part, ws_acc, ws_ml,
-                                                 sp.keep_first, sp.softcap, sink_w, sp.channel_gate, sp.chunk)
+        rest = (sp.heads, sp.kv_heads, sp.dim, gate_off, sp.scale, sp.window, sp.sink, out_scale, nparts, part, ws_acc, ws_ml,
+                sp.keep_first, sp.softcap, sink_w, sp.channel_gate, sp.chunk)
+        if prep is not None:
+            self._window_lib.window_attention_step(out, proj, cache, *prep, meta.seq_cu, meta.seq_ctx, meta.seq_bt, *rest)
+        else:
+            self._window_lib.window_attention_decode(out, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt,
+                                                     meta.seq_ctx.shape[0] - nd, meta.num_prefill_tokens, *rest)
         return True
 
 
@@ -990,6 +1005,9 @@ class ReferenceOps:
         return out
 
     def delta_rule_low(self, out, state, proj, w2, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0) -> bool:
+        return False
+
+    def window_step(self, out, proj, cache, meta, inv_freq, sp, q_norm, k_norm, eps, gate_off, out_scale=1.0, sink_w=None) -> bool:
         return False
 
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):

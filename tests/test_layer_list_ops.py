@@ -1113,3 +1113,53 @@ def test_window_attention_hidden_keys(dim, n, ctx, window, chunk, dtype):
         outs.append(torch.empty(n, heads * dim, dtype=dtype, device="cuda"))
         get_ops("cuda").window_attention(outs[-1], proj, cache.view(pages, bs, -1).cuda(), meta, sp, -1)
     assert outs[0].isfinite().all() and torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,kv,dim,ctxs,nfreq,mode,own,opts", [
+    (1, 1, 64, [1], 0, 0, True, {}), (16, 4, 128, [1, 31, 32, 33, 700], 64, 1, True, {"v_norm": True}),
+    (40, 2, 64, [5, 129, 400], 16, 2, True, {"window": 100, "keep_first": 7, "temp_every": 64}), (64, 8, 128, [2, 20], 64, 1, True, {}),
+    (32, 2, 128, [64, 65, 1500], 32, 3, True, {"chunk": 64}), (16, 1, 256, [3, 290], 128, 2, True, {}), (8, 2, 128, [16, 300], 64, 1, False, {})])
+def test_window_step(heads, kv, dim, ctxs, nfreq, mode, own, opts, dtype):
+    """The launch for a decode step beside the two it takes the place of: one key, runs that end before, at and behind a tile's end, several
+    runs, more than 16 heads per key / value head, more than one round of items and sums (one wave, 72 heads), each norm, a
+    row without a slot, queries alone, and a sequence without a row."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(heads * dim + mode)
+    n, bs, nq, nk = len(ctxs), 8, heads * dim, kv * dim
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=opts.get("window", 0), scale=dim ** -0.5, sink=False,
+                         keep_first=opts.get("keep_first", 0), softcap=0.0, channel_gate=False, chunk=opts.get("chunk", 0), diff=0.0, q_size=nq,
+                         k_size=nk, v_size=nk, kv_from=None if own else 0, qk_norm=mode == 1, head_norm=mode == 2, unit_qk=mode == 3,
+                         v_norm=opts.get("v_norm", False), temp_coef=0.1, temp_every=opts.get("temp_every", 0), scaling=SimpleNamespace(amplitude=1.25))
+    sp.reach = sp.window + sp.keep_first if sp.window > 0 else sp.chunk
+    width = -(-max(ctxs) // bs)
+    bt = torch.randperm((n + 1) * width, generator=g).int().view(n + 1, width)
+    cache = torch.randn((n + 1) * width, bs, 2 * nk, generator=g).to(dtype).cuda()
+    proj = torch.randn(n + 1, nq + (2 * nk if own else 0) + 16, generator=g).to(dtype).cuda()   # a padding row at the end
+    w = [torch.rand(m, generator=g).cuda() + 0.5 for m in {1: (nq, nk), 2: (dim, dim)}[mode]] if mode in (1, 2) else [None, None]
+    pos = torch.tensor([c - 1 for c in ctxs] + [0])
+    slots = torch.tensor([int(bt[s, (c - 1) // bs]) * bs + (c - 1) % bs for s, c in enumerate(ctxs)] + [-1])
+    if n > 2:
+        slots[1] = -1   # its key and value stay what the cache holds
+    cu, ctx = torch.tensor([*range(n + 1), n]).int(), torch.tensor(ctxs + [0]).int()
+    meta = SimpleNamespace(seq_ctx=ctx.cuda(), seq_cu=cu.cuda(), seq_bt=bt.cuda(), num_decode=n + 1, num_prefill_tokens=0, max_ctx=max(ctxs), max_q=1,
+                           positions=pos.cuda(), slot_mapping=slots.cuda())
+    inv = (1e4 ** (-torch.arange(nfreq).float() / max(nfreq, 1))).cuda()
+    ops = get_ops("cuda")
+    p, c, out, want = proj.clone(), cache.clone(), torch.zeros(n + 1, nq, dtype=dtype, device="cuda"), torch.zeros(n + 1, nq, dtype=dtype, device="cuda")
+    taken = ops.window_step(out, p, c, meta, inv, sp, *w, 1e-5, -1)
+    assert taken == (dim < 256)
+    if not taken:
+        return
+    assert torch.equal(p, proj)
+    ops.attn_prepare(p, cache, meta, inv, sp, *w, 1e-5)
+    ops.window_attention(want, p, cache, meta, sp, -1)
+    # sums of squares in another order: 2^-22 of a head's factor, so that an element of the cache, and of the queries, may round the other way:
+    # 2^-8 in bf16; in fp32 that factor and three more roundings. A score of up to about 60 (queries and keys times 1.25 and weights of up to 1.5, sums
+    # of 256 products at 16 standard deviations) moves by 60 x 2^-8 x 3 / sqrt(128) at the most, an output by that share and its own rounding.
+    tol = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -20
+    assert ((c.float() - cache.float()).abs() <= tol * cache.float().abs() + 2.0 ** -20).all()
+    tol = 0.08 if dtype == torch.bfloat16 else 60 * 2.0 ** -20
+    out, want = out[:n].float(), want[:n].float()   # the padding row's is nobody's
+    assert (out - want).abs().max() <= tol * max(1.0, float(want.abs().max()))
