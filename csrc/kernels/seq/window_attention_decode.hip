@@ -305,7 +305,7 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
     const long slot = prep.own_kv ? prep.slots[r0] : -1;
     fresh = slot >= 0 && hi >= lo && hi == total - 1;
     prepare_row<T, D>(prep, proj + r0 * proj_ld, prep.positions[r0], slot, head0, nh, kvh, heads, kv_heads, fresh && h0 == 0, hs,
-                      reinterpret_cast<float*>(hs + (hc + 2) * D), [&] { if (EARLY) rows_of(first, src0); }, [&] { if (EARLY && first <= hi) load(src0, k0, v0); });
+                      reinterpret_cast<float*>(hs + (hc + 2) * D), [&] { if (EARLY && first <= hi) rows_of(first, src0); }, [&] { if (EARLY && first <= hi) load(src0, k0, v0); });
   }
   u32x4 q[QN];
 #pragma unroll
