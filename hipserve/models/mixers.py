@@ -171,7 +171,9 @@ class LatentAttention:
         self.q_norm = get(prefix + "dq.norm").to(dev, torch.float32)
         self.kv_norm = get(prefix + "dkv.norm").to(dev, torch.float32)
         self.w_uq = uq.to(dev, dt).contiguous()
-        self.w_kv = torch.cat([get(prefix + name).to(dev, dt).reshape(-1, s.kv_rank) for name in ("uk", "uv")], 0)
+        # of their own sizes each, before they share one allocation
+        uk, uv = (get(prefix + name).to(dev, dt).reshape(s.heads, d, s.kv_rank) for name, d in (("uk", s.dim), ("uv", s.vdim)))
+        self.w_kv = torch.cat([uk.flatten(0, 1), uv.flatten(0, 1)], 0)
         self.w_uk = self.w_kv[: s.heads * s.dim].view(s.heads, s.dim, s.kv_rank)
         if self.ops.latent_query_in_place(dt, s.kv_rank, s.rot_dim):
             self._lay_out_queries()

@@ -453,6 +453,24 @@ def test_latent_weights_are_laid_out_at_load():
             assert torch.equal(m.w_uk_t.transpose(1, 2), m.w_uk) and torch.equal(m.w_uk_wide[..., :16], m.w_uk) and not m.w_uk_wide[..., 16:].any()
 
 
+def test_latent_weights_of_other_sizes_are_refused():
+    """W_uk and W_uv lie side by side in one allocation: rows that one has too many must not become the other's."""
+    from types import SimpleNamespace
+
+    from hipserve.config import LatentAttentionSpec
+    from hipserve.models.mixers import LatentAttention
+    spec = LatentAttentionSpec(heads=2, dim=8, rot_dim=4, vdim=12, q_rank=8, kv_rank=16, scale=0.1)
+    m = LatentAttention(spec, 32, 1e-6, "cpu", torch.float32, SimpleNamespace(latent_query_in_place=lambda *a: False))
+    t = m.init_random(torch.Generator().manual_seed(0), 0.02)
+    m.load(t.__getitem__, "")
+    assert torch.equal(m.w_uk.flatten(0, 1), t["uk"].view(-1, 16)) and torch.equal(m.w_uv.flatten(0, 1), t["uv"].view(-1, 16))
+    both = torch.cat([t["uk"].view(-1, 16), t["uv"].view(-1, 16)])
+    for rows in (24, 17):   # the two exchanged, a row of one with the other
+        wrong = dict(t, uk=both[:rows], uv=both[rows:])
+        with pytest.raises(RuntimeError):
+            m.load(wrong.__getitem__, "")
+
+
 @gpu
 @pytest.mark.parametrize("kv", [128, 512])
 @pytest.mark.parametrize("n,ctx,window", [(3, 100, 40), (4, 64, 33), (2, 200, 64)])
