@@ -329,9 +329,12 @@ class TableMoE:
     @staticmethod
     def align(layers, tables, h: torch.Tensor, ids: torch.Tensor):
         """(tile, slots, tile_expert, pair_slot) of every one of the ``layers``, whose tables are ``tables``, for ``forward`` to take: one
-        launch for the step; None where the layers align for themselves."""
+        launch for the step; None where the layers align for themselves, as they do once one of them has loaded a table of its own."""
         m = layers[0]
         P = h.shape[0] * m.spec.top
+        first, size = tables.data_ptr(), tables.stride(0) * tables.element_size()
+        if any(l.table.data_ptr() != first + i * size for i, l in enumerate(layers)):
+            return None
         if m._packed_ok(h, P) or not m.ops.moe_tables_align_ok(tables, ids, m.spec.experts):
             return None
         tile, aligned = m._tables(P, h.device, len(layers))

@@ -667,6 +667,31 @@ def test_moe_table_align_of_layers(tokens, top):
         assert int((slots[i] >= 0).sum()) == P
 
 
+def test_moe_tables_of_layers_after_a_reload():
+    """A layer that loads another table after the tables were stacked is not aligned by what it had before."""
+    from types import SimpleNamespace
+
+    from hipserve.config import TableMoESpec
+    from hipserve.models.mixers import TableMoE
+    calls = []
+    ops = SimpleNamespace(name="stub", moe_tables_align_ok=lambda *a: True, moe_table_align=lambda tables, *a: calls.append(tables.clone()))
+    layers = [TableMoE(TableMoESpec(experts=4, top=2, ff=8), 16, 40, "cpu", torch.float32, ops) for _ in range(3)]
+    g = torch.Generator().manual_seed(0)
+    for m in layers:
+        m.init_random(g, 0.02)
+    tables = TableMoE.stack(layers)
+    h, ids = torch.zeros(5, 16), torch.arange(5)
+    assert len(TableMoE.align(layers, tables, h, ids)) == 3 and torch.equal(calls[0], torch.stack([m.table for m in layers]))
+    for i in range(3):
+        TableMoE.stack(layers)   # of its own: `tables` is no longer what the layers hold
+        assert TableMoE.align(layers, tables, h, ids) is None
+        tables = TableMoE.stack(layers)
+        assert TableMoE.align(layers, tables, h, ids) is not None
+        layers[i].init_random(g, 0.02)
+        assert TableMoE.align(layers, tables, h, ids) is None
+    assert len(calls) == 4
+
+
 # ------------------------------------------------------------------ queries, keys and values of window attention
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
