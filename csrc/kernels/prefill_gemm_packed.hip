@@ -201,26 +201,142 @@ HS_DEVICE void pw_epilogue(f32x4 (&acc)[8][8], int own, int t, int mb, int fq, i
   }
 }
 
-// kGroup (MoE prefill experts): X rows are expert-sorted slots in BM-row tiles
-// (moe_align with tile BM, moe_gather); m-tile tm multiplies expert grp.tile_expert[tm]'s
-// packed weight (Wp + e * estride) and only the first *grp.num_tiles m-tiles (the
-// device-side count: no host round trip, graph-capturable) are walked. rest > 0: only whole
-// rounds of `rest` tiles, where pw_tail_kernel takes what is left over (pw_whole).
-template <int WM, int EPI, bool kGroup, int RW, bool LDLY = false, bool kGather = false>
-__global__ __launch_bounds__(PW_T) __attribute__((amdgpu_waves_per_eu(1, 1))) void pgw_kernel(
-    const unsigned short* __restrict__ X, long ldx, const unsigned short* __restrict__ Wp,
-    unsigned short* __restrict__ C, long ldc, int M, int N, int K, int tiles_m, int tiles_n,
-    const unsigned short* __restrict__ bias, PwGroup grp, int rest) {
+// The tiles that whole rounds leave over (WM = 1, grouped): 272 tiles on 256 compute units took two rounds, the second on 16 of them.
+// A workgroup takes one 128 x 128 weight tile of such a tile, each of its waves a quarter of K with X rows of its own in LDS (no
+// barriers; loads a 64-deep stage ahead), and the waves' sums meet in LDS, in the order of K. A stage is bound by what a compute unit
+// takes in (X and weights 1 : 1 instead of 1 : 4: 40 KB per us), so that a quarter costs about 9 + 12.5 us per 1024 of K where
+// the round that it replaces costs 24 us per 1024, as it has the memory to itself: nothing is gained below K = 1536 (1024: 24 -> 22 us),
+// and two rounds of quarters never pay. Whole rounds alone -> with quarters, 8 experts: 1024 x 2048, 260 tiles 102 -> 80 us; 2048 x 4096, 520
+// tiles 290 -> 247; 4096 x 2048, 560 tiles 160 -> 141. The quarters follow in the launch of the whole rounds: one of its own, which has to come
+// whatever the device's counts are, cost 2 - 3 us of products that leave nothing over (1024 x 2048, 400 tiles: 114, 117 with it, 114 now).
+constexpr int PW_TAIL_LDS = 4 * 2 * 128 * 128;   // [wave][2][128 rows of 128 bytes], then the sums [owner][other][8 KB]
+template <int EPI, bool kGather>
+HS_DEVICE void pw_tail(unsigned char* lds, int r, const unsigned short* __restrict__ X, long ldx, const unsigned short* __restrict__ Wp,
+                       unsigned short* __restrict__ C, long ldc, int M, int N, int K, int tiles_m, int tiles_n, const PwGroup& grp,
+                       int whole) {
+  constexpr int BUF = 128 * 128, XP = 16;   // a wave's stage: 128 rows of 128 bytes, 8 rows a load
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ntiles = (N + 127) >> 7, KS = K >> 8;
+  const int units = 4 * (tiles_m * tiles_n - whole);
+  const int nst = K >> 8, q0 = wave * 2 * nst;   // the wave's stages, its first 32-deep slot
+  const int fr = lane & 15, fq = lane >> 4, sw = (fr >> 1) & 7;
+  const int foff = wave * 2 * BUF + fr * 128;
+  const int ch[2] = {(fq ^ sw) * 16, ((4 + fq) ^ sw) * 16};
+  // staging: lane -> rows 8 p + lane / 8, 16-byte chunk c of row r at chunk c ^ ((r >> 1) & 7): r / 2 % 8 = 4 (p % 2) + lane / 16
+  const int xd = wave * 2 * BUF + (lane >> 3) * 128;
+  const int xdo[2] = {xd + (((lane & 7) ^ (lane >> 4)) * 16), xd + (((lane & 7) ^ (4 + (lane >> 4))) * 16)};
+  for (int u = r; u < units; u += gridDim.x) {
+    int tm, tn;
+    pw_tile(whole + (u >> 2), tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * 128, t = 4 * tn + (u & 3);
+    if (t >= ntiles) continue;
+    const unsigned short* wp = Wp + (long)__builtin_amdgcn_readfirstlane(grp.tile_expert[tm]) * grp.estride + (long)t * KS * 32768;
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)wp, 0, KS * 65536, 0x00020000);
+    // rows that do not exist lie past the buffer and read as zero (pw_make)
+    const int bytes = kGather ? (int)((long)grp.x_rows * ldx * 2) : (int)((long)min(128, M - m0) * ldx * 2);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)(kGather ? X : X + (long)m0 * ldx), 0, bytes, 0x00020000);
+    int xo[XP];
+#pragma unroll
+    for (int p = 0; p < XP; ++p) {
+      const int r = 8 * p + (lane >> 3);
+      if constexpr (kGather) {
+        const int s = m0 + r < M ? grp.gather_slots[m0 + r] : -1;
+        xo[p] = (s >= 0 ? (s / grp.gather_k) * (int)ldx * 2 : bytes) + (lane & 7) * 16;
+      } else {
+        xo[p] = r * (int)ldx * 2 + (lane & 7) * 16;
+      }
+    }
+    u32x4 xst[XP], w[2][8], xa[8], xb[8];
+    f32x4 acc[8][8];
+    auto wload = [&](int q, int rg) -> u32x4 {   // slot q of the wave's
+      q += q0;
+      return __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16, (q >> 3) * 65536 + rg * 8192 + (q & 7) * 1024, 0);
+    };
+    auto xload = [&](int st) {
+#pragma unroll
+      for (int p = 0; p < XP; ++p) xst[p] = __builtin_amdgcn_raw_buffer_load_b128(xr, xo[p], q0 * 64 + st * 128, 0);
+    };
+    auto xstore = [&](int buf) {
+#pragma unroll
+      for (int p = 0; p < XP; ++p) *reinterpret_cast<u32x4*>(lds + buf * BUF + p * 1024 + xdo[p & 1]) = xst[p];
+    };
+    auto xfrag = [&](int buf, int h, int i) -> u32x4 {
+      return *reinterpret_cast<const u32x4*>(lds + buf * BUF + foff + i * 2048 + ch[h]);
+    };
+    xload(0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int rg = 0; rg < 8; ++rg) w[j][rg] = wload(j, rg);
+#pragma unroll
+    for (int rg = 0; rg < 8; ++rg)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[rg][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    xstore(0);
+    xload(min(1, nst - 1));
+#pragma unroll
+    for (int i = 0; i < 8; ++i) xa[i] = xfrag(0, 0, i);
+    for (int st = 0; st < nst; ++st) {
+      const int buf = st & 1, nq = 2 * min(st + 1, nst - 1);
+#pragma unroll
+      for (int rg = 0; rg < 8; ++rg) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pw_mfma(acc[rg][i], w[0][rg], xa[i]);
+        w[0][rg] = wload(nq, rg);
+        xb[rg] = xfrag(buf, 1, rg);
+        if (rg == 2) xstore(buf ^ 1);
+        if (rg == 3) xload(min(st + 2, nst - 1));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int rg = 0; rg < 8; ++rg) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) pw_mfma(acc[rg][i], w[1][rg], xb[i]);
+        w[1][rg] = wload(nq + 1, rg);
+        xa[rg] = xfrag(buf ^ 1, 0, rg);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");  // last MFMA -> VALU reads
+    // wave w ends with the row groups w and w + 4: the others' parts through LDS, half of the rows at a time, added in the order of K
+    f32x4* sums = reinterpret_cast<f32x4*>(lds);   // [owner][wave][2][4][64 lanes]
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      __syncthreads();
+#pragma unroll
+      for (int rg = 0; rg < 8; ++rg)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sums[((((rg & 3) * 4 + wave) * 2 + (rg >> 2)) * 4 + i) * 64 + lane] = acc[rg][4 * half + i];
+      __syncthreads();
+#pragma unroll
+      for (int rg = 0; rg < 8; ++rg) {
+        if ((rg & 3) != wave) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int o = 0; o < 4; ++o) a += sums[(((wave * 4 + o) * 2 + (rg >> 2)) * 4 + i) * 64 + lane];
+          acc[rg][4 * half + i] = a;
+        }
+      }
+    }
+    pw_epilogue<EPI>(acc, wave, t, m0 + fr, fq, ntiles, C, ldc, M, N, nullptr, grp);
+    __syncthreads();   // the sums are read before the next unit's rows come
+  }
+}
+
+// The tiles r, r + G, .. < total of a workgroup.
+template <int WM, int EPI, bool kGroup, int RW, bool LDLY, bool kGather>
+HS_DEVICE void pw_tiles(unsigned char* lds, int r, int G, int total, const unsigned short* __restrict__ X, long ldx,
+                        const unsigned short* __restrict__ Wp, unsigned short* __restrict__ C, long ldc, int M, int N, int K,
+                        int tiles_m, int tiles_n, const unsigned short* __restrict__ bias, const PwGroup& grp) {
   constexpr int WN = 4 / WM, BM = 128 * WM, STAGE = BM * 128, XP = BM / 32;
-  __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * STAGE];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave - (wave / WN) * WN;
   const int ntiles = (N + 127) >> 7;
   const int KS = K >> 8, nq = K >> 5, nst = K >> 6;
-  if constexpr (kGroup) tiles_m = min(tiles_m, __builtin_amdgcn_readfirstlane(*grp.num_tiles));
-  const int total = rest > 0 ? pw_whole(tiles_m * tiles_n, rest) : tiles_m * tiles_n, G = gridDim.x;
-  const int r = xcd_remap(blockIdx.x, G);
   if (r >= total) return;
 
   // cur: the tile whose MFMAs run; nxt: the one the loads past cur's end stream in, so
@@ -355,156 +471,28 @@ __global__ __launch_bounds__(PW_T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
   }
 }
 
-// The tiles that whole rounds leave over (WM = 1, grouped): 272 tiles on 256 compute units took two rounds, the second on 16 of them.
-// A workgroup takes one 128 x 128 weight tile of such a tile, each of its waves a quarter of K with X rows of its own in LDS (no
-// barriers; loads a 64-deep stage ahead), and the waves' sums meet in LDS, in the order of K. A stage is bound by what a compute unit
-// takes in (X and weights 1 : 1 instead of 1 : 4: 40 KB per us), so that a quarter costs about 9 + 12.5 us per 1024 of K where
-// the round that it replaces costs 24 us per 1024, as it has the memory to itself: nothing is gained below K = 1536 (1024: 24 -> 22 us
-// and a launch), and two rounds of quarters never pay. 16 experts, 16384 rows, 1024 x 2048 each: 123 -> 73 + 35 us; 8 experts, 2048 x 4096:
-// 253 -> 175 + 51, 4096 x 2048: 230 -> 190 + 31.
-template <int EPI, bool kGather>
-__global__ __launch_bounds__(PW_T) __attribute__((amdgpu_waves_per_eu(1, 1))) void pgw_tail_kernel(
-    const unsigned short* __restrict__ X, long ldx, const unsigned short* __restrict__ Wp, unsigned short* __restrict__ C, long ldc,
-    int M, int N, int K, int tiles_m, int tiles_n, PwGroup grp, int ncu) {
-  constexpr int BUF = 128 * 128, XP = 16;   // a wave's stage: 128 rows of 128 bytes, 8 rows a load
-  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];   // [wave][2][BUF], then the sums [owner][other][8 KB]
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ntiles = (N + 127) >> 7, KS = K >> 8;
-  tiles_m = min(tiles_m, __builtin_amdgcn_readfirstlane(*grp.num_tiles));
-  const int total = tiles_m * tiles_n, whole = pw_whole(total, ncu), units = 4 * (total - whole);
-  const int nst = K >> 8, q0 = wave * 2 * nst;   // the wave's stages, its first 32-deep slot
-  const int fr = lane & 15, fq = lane >> 4, sw = (fr >> 1) & 7;
-  const int foff = wave * 2 * BUF + fr * 128;
-  const int ch[2] = {(fq ^ sw) * 16, ((4 + fq) ^ sw) * 16};
-  // staging: lane -> rows 8 p + lane / 8, 16-byte chunk c of row r at chunk c ^ ((r >> 1) & 7): r / 2 % 8 = 4 (p % 2) + lane / 16
-  const int xd = wave * 2 * BUF + (lane >> 3) * 128;
-  const int xdo[2] = {xd + (((lane & 7) ^ (lane >> 4)) * 16), xd + (((lane & 7) ^ (4 + (lane >> 4))) * 16)};
-  for (int u = xcd_remap(blockIdx.x, gridDim.x); u < units; u += gridDim.x) {
-    int tm, tn;
-    pw_tile(whole + (u >> 2), tiles_m, tiles_n, tm, tn);
-    const int m0 = tm * 128, t = 4 * tn + (u & 3);
-    if (t >= ntiles) continue;
-    const unsigned short* wp = Wp + (long)__builtin_amdgcn_readfirstlane(grp.tile_expert[tm]) * grp.estride + (long)t * KS * 32768;
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)wp, 0, KS * 65536, 0x00020000);
-    // rows that do not exist lie past the buffer and read as zero (pw_make)
-    const int bytes = kGather ? (int)((long)grp.x_rows * ldx * 2) : (int)((long)min(128, M - m0) * ldx * 2);
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)(kGather ? X : X + (long)m0 * ldx), 0, bytes, 0x00020000);
-    int xo[XP];
-#pragma unroll
-    for (int p = 0; p < XP; ++p) {
-      const int r = 8 * p + (lane >> 3);
-      if constexpr (kGather) {
-        const int s = m0 + r < M ? grp.gather_slots[m0 + r] : -1;
-        xo[p] = (s >= 0 ? (s / grp.gather_k) * (int)ldx * 2 : bytes) + (lane & 7) * 16;
-      } else {
-        xo[p] = r * (int)ldx * 2 + (lane & 7) * 16;
-      }
-    }
-    u32x4 xst[XP], w[2][8], xa[8], xb[8];
-    f32x4 acc[8][8];
-    auto wload = [&](int q, int rg) -> u32x4 {   // slot q of the wave's
-      q += q0;
-      return __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16, (q >> 3) * 65536 + rg * 8192 + (q & 7) * 1024, 0);
-    };
-    auto xload = [&](int st) {
-#pragma unroll
-      for (int p = 0; p < XP; ++p) xst[p] = __builtin_amdgcn_raw_buffer_load_b128(xr, xo[p], q0 * 64 + st * 128, 0);
-    };
-    auto xstore = [&](int buf) {
-#pragma unroll
-      for (int p = 0; p < XP; ++p) *reinterpret_cast<u32x4*>(lds + buf * BUF + p * 1024 + xdo[p & 1]) = xst[p];
-    };
-    auto xfrag = [&](int buf, int h, int i) -> u32x4 {
-      return *reinterpret_cast<const u32x4*>(lds + buf * BUF + foff + i * 2048 + ch[h]);
-    };
-    xload(0);
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int rg = 0; rg < 8; ++rg) w[j][rg] = wload(j, rg);
-#pragma unroll
-    for (int rg = 0; rg < 8; ++rg)
-#pragma unroll
-      for (int i = 0; i < 8; ++i) acc[rg][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    xstore(0);
-    xload(min(1, nst - 1));
-#pragma unroll
-    for (int i = 0; i < 8; ++i) xa[i] = xfrag(0, 0, i);
-    for (int st = 0; st < nst; ++st) {
-      const int buf = st & 1, nq = 2 * min(st + 1, nst - 1);
-#pragma unroll
-      for (int rg = 0; rg < 8; ++rg) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pw_mfma(acc[rg][i], w[0][rg], xa[i]);
-        w[0][rg] = wload(nq, rg);
-        xb[rg] = xfrag(buf, 1, rg);
-        if (rg == 2) xstore(buf ^ 1);
-        if (rg == 3) xload(min(st + 2, nst - 1));
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int rg = 0; rg < 8; ++rg) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pw_mfma(acc[rg][i], w[1][rg], xb[i]);
-        w[1][rg] = wload(nq + 1, rg);
-        xa[rg] = xfrag(buf ^ 1, 0, rg);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");  // last MFMA -> VALU reads
-    // wave w ends with the row groups w and w + 4: the others' parts through LDS, half of the rows at a time, added in the order of K
-    f32x4* sums = reinterpret_cast<f32x4*>(lds);   // [owner][wave][2][4][64 lanes]
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      __syncthreads();
-#pragma unroll
-      for (int rg = 0; rg < 8; ++rg)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) sums[((((rg & 3) * 4 + wave) * 2 + (rg >> 2)) * 4 + i) * 64 + lane] = acc[rg][4 * half + i];
-      __syncthreads();
-#pragma unroll
-      for (int rg = 0; rg < 8; ++rg) {
-        if ((rg & 3) != wave) continue;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int o = 0; o < 4; ++o) a += sums[(((wave * 4 + o) * 2 + (rg >> 2)) * 4 + i) * 64 + lane];
-          acc[rg][4 * half + i] = a;
-        }
-      }
-    }
-    pw_epilogue<EPI>(acc, wave, t, m0 + fr, fq, ntiles, C, ldc, M, N, nullptr, grp);
-    __syncthreads();   // the sums are read before the next unit's rows come
+// kGroup (MoE prefill experts): X rows are expert-sorted slots in BM-row tiles
+// (moe_align with tile BM, moe_gather); m-tile tm multiplies expert grp.tile_expert[tm]'s
+// packed weight (Wp + e * estride) and only the first *grp.num_tiles m-tiles (the
+// device-side count: no host round trip, graph-capturable) are walked. TAIL: whole rounds of
+// `ncu` tiles, then what they leave over (pw_whole, pw_tail).
+template <int WM, int EPI, bool kGroup, int RW, bool LDLY = false, bool kGather = false, bool TAIL = false>
+__global__ __launch_bounds__(PW_T) __attribute__((amdgpu_waves_per_eu(1, 1))) void pgw_kernel(
+    const unsigned short* __restrict__ X, long ldx, const unsigned short* __restrict__ Wp,
+    unsigned short* __restrict__ C, long ldc, int M, int N, int K, int tiles_m, int tiles_n,
+    const unsigned short* __restrict__ bias, PwGroup grp, int ncu) {
+  static_assert(!TAIL || (WM == 1 && kGroup), "pw_tail");
+  __shared__ __attribute__((aligned(1024))) unsigned char lds[TAIL ? PW_TAIL_LDS : 2 * 128 * WM * 128];
+  // TAIL: of the grid, as many as there can be whole tiles for, which the XCDs share evenly that way
+  const int G = TAIL ? min((int)gridDim.x, tiles_m * tiles_n) : gridDim.x;
+  if constexpr (kGroup) tiles_m = min(tiles_m, __builtin_amdgcn_readfirstlane(*grp.num_tiles));
+  const int total = TAIL ? pw_whole(tiles_m * tiles_n, ncu) : tiles_m * tiles_n;
+  const int r = (int)blockIdx.x < G ? xcd_remap(blockIdx.x, G) : total;
+  pw_tiles<WM, EPI, kGroup, RW, LDLY, kGather>(lds, r, G, total, X, ldx, Wp, C, ldc, M, N, K, tiles_m, tiles_n, bias, grp);
+  if constexpr (TAIL) {
+    __syncthreads();   // the last tile's rows are read
+    pw_tail<EPI, kGather>(lds, xcd_remap(blockIdx.x, gridDim.x), X, ldx, Wp, C, ldc, M, N, K, tiles_m, tiles_n, grp, total);
   }
-}
-
-// pgw_tail_kernel after the whole rounds; false where its LDS is refused
-template <int EPI>
-bool launch_tail(const unsigned short* X, long ldx, const unsigned short* Wp, unsigned short* C, long ldc, int M, int N, int K,
-                 int tiles_m, int tiles_n, const PwGroup& grp, int ncu, hipStream_t s) {
-  constexpr int smem = 4 * 2 * 128 * 128;
-  const int wgs = std::min(ncu, 4 * tiles_m * tiles_n);
-  auto go = [&](auto* kernel) {
-    kernel<<<wgs, PW_T, smem, s>>>(X, ldx, Wp, C, ldc, M, N, K, tiles_m, tiles_n, grp, ncu);
-  };
-  if (grp.gather_slots != nullptr) go(&pgw_tail_kernel<EPI, true>);
-  else if constexpr (EPI != PW_EPI_CGLU) go(&pgw_tail_kernel<EPI, false>);
-  return true;
-}
-
-template <int EPI> bool tail_ok() {
-  static const bool ok = [] {
-    auto allow = [](auto* kernel) {
-      return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 2 * 128 * 128) ==
-             hipSuccess;
-    };
-    if constexpr (EPI != PW_EPI_CGLU)
-      if (!allow(&pgw_tail_kernel<EPI, false>)) return false;
-    return allow(&pgw_tail_kernel<EPI, true>);
-  }();
-  return ok;
 }
 
 bool launch_prefill_gemm_packed(int epi, void* C, long ldc, const void* X, long ldx, const void* Wp, int M, int N,
@@ -534,7 +522,6 @@ bool launch_prefill_gemm_packed(int epi, void* C, long ldc, const void* X, long 
   }
   const int total = tiles_m * tiles_n;
   const dim3 grid(min(total, grid_req > 0 ? grid_req : ncu));
-  int rest = 0;   // > 0: the tiles that whole rounds of so many leave over are pgw_tail_kernel's
   auto* x = static_cast<const unsigned short*>(X);
   auto* w = static_cast<const unsigned short*>(Wp);
   auto* c = static_cast<unsigned short*>(C);
@@ -542,11 +529,11 @@ bool launch_prefill_gemm_packed(int epi, void* C, long ldc, const void* X, long 
 #define PW_LAUNCH1(WM_, E_, RW_)                                                                               \
   do {                                                                                                         \
     if (gather)                                                                                                \
-      pgw_kernel<WM_, E_, true, 4, false, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, rest); \
+      pgw_kernel<WM_, E_, true, 4, false, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu); \
     else if (grouped)                                                                                          \
-      pgw_kernel<WM_, E_, true, RW_><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, rest);  \
+      pgw_kernel<WM_, E_, true, RW_><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu);  \
     else                                                                                                       \
-      pgw_kernel<WM_, E_, false, RW_><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, rest); \
+      pgw_kernel<WM_, E_, false, RW_><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu); \
   } while (0)
 #define PW_LAUNCH(WM_, E_)                                                                                   \
   do {                                                                                                       \
@@ -555,28 +542,34 @@ bool launch_prefill_gemm_packed(int epi, void* C, long ldc, const void* X, long 
     else if (rw == 2)                                                                                        \
       PW_LAUNCH1(WM_, E_, 2);                                                                                \
     else if (grouped)                                                                                        \
-      pgw_kernel<WM_, E_, true, 4, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, rest);  \
+      pgw_kernel<WM_, E_, true, 4, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu);  \
     else                                                                                                     \
-      pgw_kernel<WM_, E_, false, 4, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, rest); \
+      pgw_kernel<WM_, E_, false, 4, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu); \
   } while (0)
   if (grouped && wm == 1 && grid_req <= 0 && K >= 1536) {
-#define PW_TAIL(E_) \
-  if (tail_ok<E_>()) rest = launch_tail<E_>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, grp, ncu, s) ? ncu : 0
+    const dim3 tg(std::min(4 * total, ncu));   // fewer tiles than compute units may come in quarters
+#define PW_TAIL(E_)                                                                                                                  \
+  do {                                                                                                                               \
+    if (gather) pgw_kernel<1, E_, true, 4, false, true, true><<<tg, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu); \
+    else if constexpr (E_ != PW_EPI_CGLU)                                                                                             \
+      pgw_kernel<1, E_, true, 4, false, false, true><<<tg, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu);   \
+    return true;                                                                                                                     \
+  } while (0)
     switch (epi) {
-      case PW_EPI_STORE: PW_TAIL(PW_EPI_STORE); break;
-      case PW_EPI_GLU: PW_TAIL(PW_EPI_GLU); break;
-      case PW_EPI_GEGLU: PW_TAIL(PW_EPI_GEGLU); break;
-      case PW_EPI_RELU2: PW_TAIL(PW_EPI_RELU2); break;
-      case PW_EPI_CGLU: PW_TAIL(PW_EPI_CGLU); break;
+      case PW_EPI_STORE: PW_TAIL(PW_EPI_STORE);
+      case PW_EPI_GLU: PW_TAIL(PW_EPI_GLU);
+      case PW_EPI_GEGLU: PW_TAIL(PW_EPI_GEGLU);
+      case PW_EPI_RELU2: PW_TAIL(PW_EPI_RELU2);
+      case PW_EPI_CGLU: PW_TAIL(PW_EPI_CGLU);
       default: return false;
     }
 #undef PW_TAIL
   }
   if (epi == PW_EPI_CGLU) {   // instantiated in the gather form only
     if (wm == 1)
-      pgw_kernel<1, PW_EPI_CGLU, true, 4, false, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, rest);
+      pgw_kernel<1, PW_EPI_CGLU, true, 4, false, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu);
     else
-      pgw_kernel<2, PW_EPI_CGLU, true, 4, false, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, rest);
+      pgw_kernel<2, PW_EPI_CGLU, true, 4, false, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu);
     return true;
   }
 #define PW_EPIS(WM_)                                          \

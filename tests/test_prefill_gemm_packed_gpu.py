@@ -212,3 +212,28 @@ def test_packed_grouped_left_over(tiles, N, K, epi, gather):
         # threefold for gates above -3), of silu and of the up projection: 6 x 2^-9
         rel = 2.0 ** -6 if epi == 2 else 2.0 ** -7
         assert ((out[mine].double() - want).abs() <= rel * want.abs() + 2.0 ** -9 * want.abs().mean()).all()
+
+
+@pytest.mark.parametrize("tiles,counted,N", [(5, 0, 512), (300, 3, 1024), (40, 40, 1024), (64, 33, 2048)])
+def test_packed_grouped_in_one_launch(tiles, counted, N, tmp_path):
+    """Whatever is counted on the device, a grouped product is one launch; of a bound far above the count, and of a grid of which some
+    workgroups have no whole tile, every counted row is written and no other."""
+    g, op, E, K, M = torch.Generator(device=DEV).manual_seed(tiles), torch.ops.hipserve, 2, 1536, tiles * 128
+    w, x = _rnd(g, E, N, K, scale=0.05), _rnd(g, M, K)
+    wp = torch.stack([_pack(w[e]) for e in range(E)])
+    tile_expert = torch.randint(0, E, (tiles,), device=DEV, generator=g, dtype=torch.int32)
+    ntiles = torch.tensor([counted], dtype=torch.int32, device=DEV)
+    out = torch.full((M, N), 7.0, device=DEV, dtype=torch.bfloat16)
+    op.prefill_gemm_packed_grouped(out, x, wp, N, 0, tile_expert, ntiles, 1)
+    got = out.clone()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    graph.enable_debug_mode()
+    with torch.cuda.graph(graph):
+        op.prefill_gemm_packed_grouped(out, x, wp, N, 0, tile_expert, ntiles, 1)
+    graph.debug_dump(str(tmp_path / "graph.dot"))
+    assert (tmp_path / "graph.dot").read_text().count("KERNEL") == 1
+    rows = counted * 128
+    assert bool((got[rows:] == 7.0).all())
+    want = torch.cat([x[t * 128:(t + 1) * 128].double() @ w[int(tile_expert[t])].double().t() for t in range(counted)] + [x.new_zeros(0, N).double()])
+    # sums of K products in 32 bits and the result's rounding
+    assert ((got[:rows].double() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -9 * K ** 0.5 * 0.05).all()
