@@ -11,6 +11,7 @@ falling back to PyTorch.
 """
 from __future__ import annotations
 
+import functools
 import os
 import threading
 
@@ -505,7 +506,10 @@ class KernelOps:
     SKINNY_ROWS = 64
     GLU_ACTS = ("silu_mul", "clamped_glu")
 
+    # The rules below are arithmetic on sizes, 3 - 10 us of Python each, and a step asks for every product: what they
+    # said of the last sizes is kept (a step that is not captured, of four layers and a few rows, took 20 - 40 us longer).
     @staticmethod
+    @functools.lru_cache(maxsize=4096)
     def skinny_pays(rows: int, cols: int, k: int, glu: bool = False, f32: bool = False) -> bool:
         """Whether ``skinny_linear`` is expected to be faster than the vendor's GEMM for ``rows`` x ``cols`` results (``cols``
         over all batches). Both sides in us, fitted to cold weights of 1024 .. 32000 columns and k of 1024 .. 12288: ours as the
@@ -535,6 +539,7 @@ class KernelOps:
         return max(least, 3.2 + 2.0 * cols * k / 4.2e6 if rows <= 16 else 4.2 + 2.0 * cols * k / 4.8e6)
 
     @staticmethod
+    @functools.lru_cache(maxsize=4096)
     def skinny_parts(rows, cols, k, f32=False) -> int:
         """Parts of k for a product whose 32-bit sums the next kernel adds up (1: none), or 0 where the vendor's GEMM is the one to run. A part
         more gives idle compute units a share and costs 0.15 us and what it is to write and read it (fitted), and the first one 0.7 us, which
@@ -557,39 +562,41 @@ class KernelOps:
     def linear_parts(self, x, w, bias=None):
         """``linear`` for a result that ``scaled_add_group_rmsnorm`` takes as ``mix``: where that is faster, 32-bit sums over parts of k,
         [parts, T, N]."""
-        if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())):
-            parts = self.skinny_parts(x.shape[0], w.shape[0], w.shape[1], x.dtype == torch.float32)
+        if x.dim() == 2 and x.shape[0] <= self.SKINNY_ROWS and self._skinny_ok(x, w, bias):
+            T, N, K = x.shape[0], w.shape[0], w.shape[1]
+            parts = self.skinny_parts(T, N, K, x.dtype == torch.float32)
             if parts > 1:
-                out = torch.empty(parts, x.shape[0], w.shape[0], device=x.device, dtype=torch.float32)
+                out = torch.empty(parts, T, N, device=x.device, dtype=torch.float32)
                 self._moe_lib.skinny_linear_parts(out, x, w, bias)
                 return out
+            if parts:
+                return self._skinny_linear(x, w, bias)
         return self.linear(x, w, bias)
 
-    def _skinny_ok(self, x, w) -> bool:
-        """The shapes, types and alignment that ``skinny_linear`` takes."""
-        per = 16 // x.element_size()
-        return (x.dtype in (torch.bfloat16, torch.float32) and w.dtype == x.dtype and x.dim() == w.dim() and 0 < x.shape[-2] <= self.SKINNY_ROWS
-                and x.shape[-1] % per == 0 and max(x.shape[-1], x.stride(-2)) < 1 << 24 and x.stride(-1) == 1 and x.stride(-2) % per == 0 and x.stride(0) % per == 0
-                and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0)
+    def _skinny_ok(self, x, w, bias=None) -> bool:
+        """The shapes, types, alignment and bias that ``skinny_linear`` takes."""
+        if x.dim() != w.dim() or not 0 < x.shape[-2] <= self.SKINNY_ROWS:
+            return False
+        per, K, stride = 16 // x.element_size(), x.shape[-1], x.stride()
+        return (x.dtype in (torch.bfloat16, torch.float32) and w.dtype == x.dtype and K % per == 0 and max(K, stride[-2]) < 1 << 24
+                and stride[-1] == 1 and stride[-2] % per == 0 and stride[0] % per == 0
+                and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())))
 
     def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0):
         """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands; ``act_from``: the first column that
         the activation applies to. A few rows run the weight-streaming kernel with the activation in its epilogue, anything else the
         vendor's GEMM and a second launch."""
         if isinstance(x, NormedRows):
-            if self._skinny_ok(x.rows, w) and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())):
+            if self._skinny_ok(x.rows, w, bias):
                 N = w.shape[0] // 2 if act in self.GLU_ACTS else w.shape[0]
                 out = torch.empty(x.shape[0], N, device=x.device, dtype=torch.float32 if out_f32 else x.dtype)
                 self._moe_lib.skinny_linear_normed(out, x.rows, x.squares, x.eps, w, bias, -1 if act is None else self.ACTIVATIONS[act], c0, c1, act_from)
                 return out
             x = x.normed()
-        if x.dim() == 2 and self._skinny_ok(x, w) and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())):
-            glu = act in self.GLU_ACTS
-            T, N, K = x.shape[0], w.shape[0], w.shape[1]
-            if self.skinny_pays(T, N, K, glu, x.dtype == torch.float32):
-                out = torch.empty(T, N // 2 if glu else N, device=x.device, dtype=torch.float32 if out_f32 else x.dtype)
-                self._moe_lib.skinny_linear(out, x, w, bias, -1 if act is None else self.ACTIVATIONS[act], c0, c1, act_from)
-                return out
+        if (x.dim() == 2 and x.shape[0] <= self.SKINNY_ROWS and self._skinny_ok(x, w, bias)
+                and self.skinny_pays(x.shape[0], w.shape[0], w.shape[1], act in self.GLU_ACTS, x.dtype == torch.float32)):
+            return self._skinny_linear(x, w, bias, out_f32, act, c0, c1, act_from)
         if out_f32 and x.dtype != torch.float32:
             y = torch.mm(x, w.t(), out_dtype=torch.float32)
             if bias is not None:
@@ -604,19 +611,28 @@ class KernelOps:
         out = torch.empty(*y.shape[:-1], y.shape[-1] // 2, device=y.device, dtype=y.dtype) if act in self.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)
 
+    def _skinny_linear(self, x, w, bias, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0):
+        out = torch.empty(x.shape[0], w.shape[0] // 2 if act in self.GLU_ACTS else w.shape[0], device=x.device,
+                          dtype=torch.float32 if out_f32 else x.dtype)
+        self._moe_lib.skinny_linear(out, x, w, bias, -1 if act is None else self.ACTIVATIONS[act], c0, c1, act_from)
+        return out
+
     NORM_ROWS = 32   # rows that ``linear_update`` takes
+
+    @staticmethod
+    @functools.lru_cache(maxsize=4096)
+    def update_pays(rows, cols, k, f32) -> bool:
+        """Whether a residual update and norm go into the products around them: what their launch costs in a captured step (2.5 us, and 0.05 per
+        row and 1024 columns) is weighed against k in parts (``linear_parts``), which needs it, and against the loads that both products do more."""
+        apart = min(KernelOps._vendor_time(rows, cols, k, f32), min(KernelOps.parts_time(rows, cols, k, f32, p) for p in (1, 2, 4)))
+        return KernelOps.skinny_time(rows, cols, k, False, f32) + 0.6 <= apart + 2.5 + 0.05 * rows * cols / 1024
 
     def linear_update(self, x, w, bias, residual, norm_w, eps):
         """residual += x . w^T + bias, and the rows for the next products as ``NormedRows`` of its norm; None, and nothing done, where the
-        update and norm are a launch of their own. What that launch costs in a captured step (2.5 us, and 0.05 per row and 1024 columns) is
-        weighed against k in parts (``linear_parts``), which needs it, and against the loads that both products do more."""
+        update and norm are a launch of their own (``update_pays``)."""
         T, N, K = x.shape[0], w.shape[0], w.shape[1]
-        if not (0 < T <= self.NORM_ROWS and N % 64 == 0 and N <= 4096 and self._skinny_ok(x, w) and residual.is_contiguous() and residual.data_ptr() % 16 == 0
-                and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous()))):
-            return None
-        f32 = x.dtype == torch.float32
-        apart = min(self._vendor_time(T, N, K, f32), min(self.parts_time(T, N, K, f32, p) for p in (1, 2, 4)))
-        if self.skinny_time(T, N, K, False, f32) + 0.6 > apart + 2.5 + 0.05 * T * N / 1024:
+        if not (0 < T <= self.NORM_ROWS and N % 64 == 0 and N <= 4096 and self.update_pays(T, N, K, x.dtype == torch.float32)
+                and self._skinny_ok(x, w, bias) and residual.is_contiguous() and residual.data_ptr() % 16 == 0):
             return None
         rows, squares = torch.empty(T, N, device=x.device, dtype=x.dtype), torch.empty(T, N // 16, device=x.device, dtype=torch.float32)
         self._moe_lib.skinny_linear_update(rows, squares, residual, norm_w, x, w, bias)
