@@ -23,6 +23,8 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
                           const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0,
                           float c1, hipStream_t s);
 
+// us that such a launch takes, cold weights; k in numbers of the operands' type
+double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts);
 // A norm around such a product of up to 32 rows, in one part: with a residual [M, N] (fp32, updated in place), out = residual * weight
 // and squares [M, blocks = N / 16] = sums of the updated residual's squares (N % 64 == 0); without one the rows x are such an out and every
 // result is multiplied by 1 / sqrt(the row's squares / cols + eps). blocks is a multiple of 4 and at most 256.
@@ -94,6 +96,7 @@ void launch_latent_attention_reduce(void* o_lat, const float* ws_acc, const floa
 bool launch_mingru_product(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x,
                            const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, bool f32,
                            hipStream_t s);
+double mingru_product_time(int M, int width, int k, bool f32);   // us, cold weights
 // minGRU over the step's rows of every sequence, from / to its fp32 state slot.
 void launch_mingru_scan(void* y, float* state, const void* proj, const float* b_z, const float* b_x,
                         const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int width, int max_q,

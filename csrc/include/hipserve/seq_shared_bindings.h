@@ -131,6 +131,11 @@ inline void skinny_linear(at::Tensor& out, const at::Tensor& x, const at::Tensor
                                              M, N, K, act, act_from, (float)c0, (float)c1, cur_stream()), "skinny_linear: LDS");
 }
 
+inline double skinny_time(int64_t rows, int64_t cols, int64_t k, bool glu, bool f32, int64_t parts) {
+  TORCH_CHECK(rows >= 0 && rows <= 64 && cols >= 0 && cols < (1L << 40) && k >= 0 && k < (1L << 30) && parts >= 1 && parts <= 64, "skinny_time: sizes");
+  return hipserve::skinny_time(rows, cols, k, glu, f32, parts);
+}
+
 // out [S, M, N]: 32-bit sums over S parts of K (in 64 halves) of x [M, K] . w [N, K]^T, the bias in the first.
 inline void skinny_linear_parts(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const c10::optional<at::Tensor>& bias) {
   CHECK_DEV(x); CHECK_CONTIG(w); CHECK_F32(out); CHECK_SAME_DEV(w, x); CHECK_SAME_DEV(out, x);
@@ -208,6 +213,7 @@ inline void skinny_linear_update(at::Tensor& out, at::Tensor& squares, at::Tenso
 
 inline void def_moe_ops(torch::Library& m) {
   m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int act, float c0, float c1, int act_from=0) -> ()");
+  m.def("skinny_time(int rows, int cols, int k, bool glu, bool f32, int parts) -> float", &skinny_time);
   m.def("skinny_linear_parts(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias) -> ()");
   m.def("skinny_linear_normed(Tensor(a!) out, Tensor x, Tensor squares, float eps, Tensor w, Tensor? bias, int act, float c0, float c1, "
         "int act_from) -> ()");

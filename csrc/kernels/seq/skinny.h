@@ -10,13 +10,14 @@
 // follows them jumps to another row from lane to lane, and the addresses of its 64 lanes are looked up one by one: 34 KB per us
 // and CU, however many loads are in flight. So the rows go through LDS: global_load_lds takes 8 lanes side by side along a row
 // (whole 128-byte lines, four lanes per look-up) and the operands are read from there, without registers for loads in
-// flight: about 60 KB per us. Each wave copies into a part of LDS that is its own, DEPTH pieces of 64 k ahead, and waits for
+// flight: 60 - 80 KB per us. Each wave copies into a part of LDS that is its own, DEPTH pieces of 64 k ahead, and waits for
 // its own copies alone. us, cold weights, loads in operand order -> this (the vendor's GEMM), 1 / 16 / 48 rows:
 //   1024 x 1024   3.4 -> 2.8 (5.6)    4.2 -> 3.1 (5.7)    6.5 -> 3.9 (8.1)     (columns x k)
 //   2048 x 2048   5.0 -> 4.4 (11.0)   6.4 -> 5.1 (11.1)   10.5 -> 7.1 (11.4)
 //   2048 x 6144   9.3 -> 7.8 (11.1)   13.6 -> 10.5 (11.2) 24.7 -> 16.2 (16.5)
 //   32000 x 2048  25.2 -> 25.6 (32.3) 33.7 -> 27.8 (30.9) 60 -> 33.5, four tiles per workgroup (34)
-// Deeper copies (3 or 5 pieces) changed nothing at one workgroup per CU and cost up to a fifth where they leave room for fewer.
+// Deeper copies (3 or 5 pieces) changed nothing at one workgroup per CU and cost up to a fifth where they leave room for fewer; so do two
+// pieces but for up to 16 rows and more than a piece per wave (skinny_linear.hip).
 // 32-bit operands (F32) are the same rows of twice as many 16-bit halves: a step is 64 bytes of a row, 16 numbers, and four
 // products of 4 k each; the four numbers of a lane are k 4 g + e on both sides, so nothing else differs.
 #pragma once

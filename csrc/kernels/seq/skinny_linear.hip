@@ -158,17 +158,39 @@ bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, 
 #undef HS_SK
 }
 
-// us of a launch with NT tiles of 16 columns per workgroup: a latency, 0.38 of the time the weights take at 5.2 TB/s (and no less
-// than that time), and what the busiest compute unit takes in at 65 / 60 / 54 KB per us. More tiles mean fewer copies of the rows and fewer workgroups. Cold weights, 1 / 2 / 4 tiles: 6144 x 2048 with 16 rows 8.2 /
-// 7.6 / -, with 48 rows 12.5 / 9.8 / 12.5; 12288 x 2048 with 16 rows 12.0 / 13.5 / -, with 48 rows 18.6 / 16.4 / 14.7; 12288 x 4096 with
-// 48 rows 32.1 / 29.3 / 23.9; 32000 x 2048 with 16 rows 26.8 / 26.8 / -, with 32 rows 38.5 / 29.7 / 30.4, with 64 50.9 / 40.4 / 34.3.
-double skinny_time(int M, long cols, int K, int nt, int parts) {
+// How many tiles of 16 columns a workgroup takes. One, unless their workgroups are more than the compute units (or a few of them hold
+// many k each): then two or four share what they copy of the rows; up to 16 rows there is too little of that. Cold weights, us with 1 / 2 / 4
+// tiles: 6144 x 4096, 16 rows 14.5 / 15.1 / 21, 48 rows 20.9 / 18.7 / 26; 16384 x 2048, 16 rows 17.0 / 15.5 / 15.5, 24 rows 18.3 / 16.4 /
+// 16.2, 48 rows 22.6 / 19.4 / 18.8; 32000 x 512, 24 rows 10.4 / 10.0 / 11.9; 16384 x 4096, 64 rows 41.6 / 35.9 / 29.3.
+// Of 2541 sizes (1 - 64 rows, 64 - 65536 columns, k 128 - 12288, both types) the choice is 0.6 % slower than the best on average, at most 21 %.
+int skinny_tiles(int M, long tiles, int K) {
+  if (tiles <= 256) return 1;
+  if (M <= 16) return M > 8 && tiles <= 512 && K >= 8192 ? 2 : 1;
+  if (tiles <= 512) return K >= 1024 ? 2 : 1;
+  if (M > 48) return K >= 1024 ? 4 : 1;
+  return K >= 4096 ? 4 : 2;
+}
+
+// us of a launch (K in halves, over `parts`): a latency, the results, and the time the weights take at 5.2 TB/s, or, where that is more, at 9 TB/s and with it
+// what the busiest compute unit takes in (80 KB per us), its sums in LDS and its products of 32-bit operands. 9 % off over the sizes above.
+double skinny_time_of(int M, long cols, double K, int nt, int parts, bool f32, double out_bytes) {
   const long wgs = ((cols + 15) / 16 + nt - 1) / nt * parts, rounds = (wgs + 255) / 256;
-  const double stream = 2.0 * cols * K / 5.2e6, rate = nt == 1 ? 65e3 : nt == 2 ? 60e3 : 54e3;
-  return 2.2 + std::max(stream, 0.38 * stream + rounds * 2.0 * K / parts * (16 * nt + (M + 7) / 8 * 8) / rate);
+  const double bytes = 2.0 * cols * K, rows = (M + 7) / 8 * 8, k = K / parts, st = nt * ((M + 15) / 16);
+  const double each = 2.0 * k * (16 * nt + rows) / 80e3 + st * (0.09 + (f32 ? 8.5e-5 * k : 0));
+  return 2.16 + std::max(bytes / 5.2e6, bytes / 9e6 + rounds * each) + 0.7e-6 * out_bytes;
 }
 
 }  // namespace
+
+double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts) {
+  const int K = f32 ? 2 * k : k;
+  const double out = (double)M * (glu ? cols / 2 : cols) * (f32 ? 4 : 2);
+  return skinny_time_of(M, cols, K, glu ? 2 : skinny_tiles(M, (cols + 15) / 16 * parts, K / parts), parts, f32, out);
+}
+
+double mingru_product_time(int M, int width, int k, bool f32) {   // a workgroup's three tiles (mingru.hip)
+  return skinny_time_of(M, 3L * width, f32 ? 2 * k : k, 3, 1, f32, (double)M * width * (f32 ? 4 : 2));
+}
 
 bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, int parts, const void* x, long x_ld, long x_bs,
                           const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1,
@@ -180,15 +202,16 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
   if (act == 3 || act == 4)
     return xg <= 1 ? HS_SK(1, 2, 1, true) : xg <= 2 ? HS_SK(2, 2, 1, true) : xg <= 4 ? HS_SK(4, 2, 1, true)
          : xg <= 6 ? HS_SK(6, 2, 1, true) : HS_SK(8, 2, 1, true);
-  const double t1 = skinny_time(M, (long)N * batch, K, 1, parts), t2 = skinny_time(M, (long)N * batch, K, 2, parts),
-               t4 = M > 16 ? skinny_time(M, (long)N * batch, K, 4, parts) : INFINITY;
-  // one piece ahead where the workgroups of several tiles would otherwise not fit a compute unit together (2 - 14 % faster)
-  if (t4 < t1 && t4 < t2) return xg <= 4 ? HS_SK(4, 4, 1, false) : xg <= 6 ? HS_SK(6, 4, 1, false) : HS_SK(8, 4, 1, false);
-  if (t2 < t1)
-    return xg <= 1 ? HS_SK(1, 2, 1, false) : xg <= 2 ? HS_SK(2, 2, 1, false) : xg <= 4 ? HS_SK(4, 2, 1, false)
-         : xg <= 6 ? HS_SK(6, 2, 1, false) : HS_SK(8, 2, 1, false);
-  return xg <= 1 ? HS_SK(1, 1, 2, false) : xg <= 2 ? HS_SK(2, 1, 2, false) : xg <= 3 ? HS_SK(3, 1, 2, false)
-       : xg <= 4 ? HS_SK(4, 1, 2, false) : xg <= 6 ? HS_SK(6, 1, 2, false) : HS_SK(8, 1, 2, false);
+  const long tiles = ((long)N * batch + 15) / 16 * parts;
+  const int nt = skinny_tiles(M, tiles, K / parts);
+  // One piece ahead: two are faster (up to 40 %) where a wave waits for its few copies, up to 16 rows and more than a piece per wave, and slower
+  // where they leave room for fewer workgroups (33 - 64 rows, 16384 x 256: 19 -> 13 us; 32 heads of 512 x 128, one row 4.1 -> 3.4).
+  if (nt == 4) return xg <= 4 ? HS_SK(4, 4, 1, false) : xg <= 6 ? HS_SK(6, 4, 1, false) : HS_SK(8, 4, 1, false);
+  if (nt == 2) return xg <= 2 ? HS_SK(2, 2, 1, false) : xg <= 4 ? HS_SK(4, 2, 1, false) : xg <= 6 ? HS_SK(6, 2, 1, false) : HS_SK(8, 2, 1, false);
+  const bool ahead = xg <= 2 && K / parts > 1024 && !(xg == 1 && tiles > 256 && tiles <= 512);
+  if (ahead) return xg <= 1 ? HS_SK(1, 1, 2, false) : HS_SK(2, 1, 2, false);
+  return xg <= 1 ? HS_SK(1, 1, 1, false) : xg <= 2 ? HS_SK(2, 1, 1, false) : xg <= 3 ? HS_SK(3, 1, 1, false)
+       : xg <= 4 ? HS_SK(4, 1, 1, false) : xg <= 6 ? HS_SK(6, 1, 1, false) : HS_SK(8, 1, 1, false);
 #undef HS_SK
 }
 
@@ -201,13 +224,13 @@ bool launch_skinny_linear_normed(void* out, bool out_f32, const SkinnyNorm& norm
 #define HS_SN(XG, NT, DEPTH, GLU, TO, F32)                                                                                                    \
   launch_kernel<XG, NT, DEPTH, GLU, TO, F32, true>(dim3((No + (GLU ? 16 : 16 * NT) - 1) / (GLU ? 16 : 16 * NT)), out, No, 0, 0, x, x_ld, 0, w,  \
                                                    bias, M, N, K, act, act_from, c0, c1, s, norm)
-#define HS_SX(NT, D1, D, GLU, TO, F32) (M <= 8 ? HS_SN(1, NT, D1, GLU, TO, F32) : M <= 16 ? HS_SN(2, NT, D, GLU, TO, F32) : HS_SN(4, NT, D, GLU, TO, F32))
-#define HS_ST(NT, D1, D, GLU) \
-  (f32 ? HS_SX(NT, D1, D, GLU, float, true) : out_f32 ? HS_SX(NT, D1, D, GLU, float, false) : HS_SX(NT, D1, D, GLU, unsigned short, false))
-  if (glu) return HS_ST(2, 1, 1, true);
-  // whole tiles only where squares are written
-  const bool two = skinny_time(M, N, K, 2, 1) < skinny_time(M, N, K, 1, 1) && (norm.residual == nullptr || N % 32 == 0);
-  return two ? HS_ST(2, 1, 1, false) : HS_ST(1, 2, 2, false);
+#define HS_SX(NT, D, GLU, TO, F32) (M <= 8 ? HS_SN(1, NT, D, GLU, TO, F32) : M <= 16 ? HS_SN(2, NT, D, GLU, TO, F32) : HS_SN(4, NT, 1, GLU, TO, F32))
+#define HS_ST(NT, D, GLU) (f32 ? HS_SX(NT, D, GLU, float, true) : out_f32 ? HS_SX(NT, D, GLU, float, false) : HS_SX(NT, D, GLU, unsigned short, false))
+#define HS_S4() (f32 ? HS_SN(4, 4, 1, false, float, true) : out_f32 ? HS_SN(4, 4, 1, false, float, false) : HS_SN(4, 4, 1, false, unsigned short, false))
+  if (glu) return HS_ST(2, 1, true);
+  const int nt = skinny_tiles(M, (N + 15) / 16, K);   // 4 above 16 rows alone; where squares are written, N is a multiple of 64
+  return nt == 4 ? HS_S4() : nt == 2 ? HS_ST(2, 1, false) : HS_ST(1, 2, false);
+#undef HS_S4
 #undef HS_ST
 #undef HS_SX
 #undef HS_SN

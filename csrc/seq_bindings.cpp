@@ -113,6 +113,10 @@ TORCH_LIBRARY(hipserve_seq, m) {
   m.def("latent_prompt_ok(int dim, int rot_dim, int vdim) -> bool", &latent_prompt_ok);
   m.def("latent_attention_dma_ok(int kv_rank, int rot_dim) -> bool", &latent_attention_dma_ok);
   m.def("latent_attention_mfma_ok(int kv_rank, int rot_dim) -> bool", &latent_attention_mfma_ok);
+  m.def("mingru_product_time(int rows, int width, int k, bool f32) -> float", [](int64_t rows, int64_t width, int64_t k, bool f32) {
+    TORCH_CHECK(rows >= 0 && rows <= 64 && width >= 0 && width < (1L << 26) && k >= 0 && k < (1L << 30), "mingru_product_time: sizes");
+    return hipserve::mingru_product_time(rows, width, k, f32);
+  });
   m.def("mingru_product(Tensor(a!) y, Tensor(b!) state, Tensor x, Tensor w, Tensor b_z, Tensor b_x, Tensor seq_cu, Tensor seq_ctx, "
         "Tensor seq_state) -> ()");
   m.def("mingru_scan(Tensor(a!) y, Tensor(b!) state, Tensor proj, Tensor b_z, Tensor b_x, Tensor seq_cu, "

@@ -12,6 +12,7 @@ falling back to PyTorch.
 from __future__ import annotations
 
 import functools
+import math
 import os
 import threading
 
@@ -122,6 +123,10 @@ class KernelOps:
         # the library whose copy of the shared kernels runs ("seq" / "delta" / "cell" / "stream"): a model sets it to
         # the one its mixers load anyway, so it never builds or loads another
         self.norm_library = "seq"
+        # the rules of products of a few rows: arithmetic on sizes, a few us each, and a step asks for every product. What they said of
+        # the last sizes is kept (a step that is not captured, of four layers and a few rows, took 20 - 40 us longer)
+        self.skinny_pays, self.skinny_parts, self.update_pays, self.mingru_pays = (
+            functools.lru_cache(maxsize=4096)(rule) for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._mingru_pays))
 
     @property
     def _op(self):
@@ -332,9 +337,16 @@ class KernelOps:
                                            s0, s1, rows, tq, inv_freq, heads, dim, rot_dim, kv_rank, gate_off,
                                            scale, window)
 
+    def _mingru_pays(self, rows, width, k, f32) -> bool:
+        """Whether the step in its product's epilogue is expected to take less than the faster product of the two and its launch, 2 us (1 in 32 bits)
+        as the rules' times go: of 1209 sizes (1 - 64 rows, widths 256 - 8192, k 256 - 4096) the choice takes 1 % longer than the faster of the two.
+        us, product and step / this: width 4096, k 2048, 1 and 48 rows 14.8 / 12.6, 20.6 / 16.4; in 32 bits width 512, k 4096, 33 rows 18.5 / 41.2."""
+        apart = min(self._skinny_time(rows, 3 * width, k, False, f32), 1.2 * self._vendor_time(rows, 3 * width, k, f32))
+        return self._seq.mingru_product_time(rows, width, k, f32) < apart + (1.0 if f32 else 2.0)
+
     def mingru_product(self, y, state, x, w, b_z, b_x, meta) -> bool:
         """``mingru_scan`` of the product x . w^T for a step of one row per sequence; False, and nothing done, where they are two launches."""
-        if not (meta.max_q == 1 and x.dim() == 2 and self._skinny_ok(x, w) and self.skinny_pays(x.shape[0], w.shape[0], w.shape[1], False, x.dtype == torch.float32)):
+        if not (meta.max_q == 1 and x.dim() == 2 and self._skinny_ok(x, w) and self.mingru_pays(x.shape[0], y.shape[-1], w.shape[1], x.dtype == torch.float32)):
             return False
         self._seq.mingru_product(y, state, x, w, b_z, b_x, meta.seq_cu, meta.seq_ctx, meta.seq_state)
         return True
@@ -506,58 +518,55 @@ class KernelOps:
     SKINNY_ROWS = 64
     GLU_ACTS = ("silu_mul", "clamped_glu")
 
-    # The rules below are arithmetic on sizes, 3 - 10 us of Python each, and a step asks for every product: what they
-    # said of the last sizes is kept (a step that is not captured, of four layers and a few rows, took 20 - 40 us longer).
-    @staticmethod
-    @functools.lru_cache(maxsize=4096)
-    def skinny_pays(rows: int, cols: int, k: int, glu: bool = False, f32: bool = False) -> bool:
-        """Whether ``skinny_linear`` is expected to be faster than the vendor's GEMM for ``rows`` x ``cols`` results (``cols``
-        over all batches). Both sides in us, fitted to cold weights of 1024 .. 32000 columns and k of 1024 .. 12288: ours as the
-        kernel's choice of tiles has it (skinny_time in skinny_linear.hip); the vendor's is hardly ever below 10.5 (7.5 up to k =
-        1024), grows with k past 32 rows and streams large weights at 4.2 - 5 TB/s. Examples, ours / vendor: 2048 x 2048 with 1, 16, 48,
-        64 rows 4.4 / 11.0, 5.1 / 11.1, 7.1 / 11.4, 8.0 / 11.9; 6144 x 2048 with 1, 16, 48 rows 7.8 / 12.5, 8.1 / 12.5, 10.1 / 12.9;
-        2048 x 6144 with 1, 16, 48 rows 7.8 / 11.1, 10.5 / 11.2, 16.2 / 16.5; 12288 x 2048 with 16, 48 rows 12.6 / 15, 15.2 / 15.6;
-        32000 x 2048 with 1, 16, 48, 64 rows 26 / 32, 28 / 31, 34 / 34, 35 / 30."""
-        return KernelOps.skinny_time(rows, cols, k, glu, f32) < KernelOps._vendor_time(rows, cols, k, f32)
+    def _skinny_pays(self, rows: int, cols: int, k: int, glu: bool = False, f32: bool = False, act: bool = False) -> bool:
+        """Whether ``skinny_linear`` is expected to be faster than the vendor's GEMM for ``rows`` x ``cols`` results (``cols`` over all
+        batches), both sides in us for cold weights: ours as the kernel's choice of tiles has it (skinny_time in skinny_linear.hip), the vendor's as
+        the choice between them comes out best. Over 2541 sizes (1 - 64 rows, 64 - 65536 columns, k 128 - 12288, both types) it takes 1 % longer
+        than the faster of the two. Examples, ours / vendor: 2048 x 2048 with 1, 16, 48, 64 rows 4.2 / 10.1, 4.9 / 10.2, 6.8 / 10.7, 7.6 / 11.1; 6144 x
+        2048 with 1, 16, 48 rows 7.7 / 12.4, 8.4 / 12.3, 10.9 / 13.4; 4096 x 12288 with 1, 16, 48 rows 19.4 / 21.1, 23.8 / 22.3, 33.9 / 32.5; 512 x
+        8192 with 48 rows 16.3 / 11.1; 32000 x 2048 with 1, 16, 48, 64 rows 24.3 / 28.2, 25.0 / 28.6, 30.3 / 31.4, 33.9 / 26.6; in 32 bits 1024 x
+        1024 with 3, 16, 48 rows 4.2 / 8.3, 4.4 / 8.3, 7.3 / 8.3; 32000 x 2048 with 1, 16, 64 rows 44 / 57, 48 / 59, 82 / 68."""
+        # an activation is a launch more there (48 x 32000: 6 - 8 us)
+        launch = 2.5 + 2.5e-6 * rows * cols if act and not glu else 0.0
+        return self._skinny_time(rows, cols, k, glu, f32) < self._vendor_time(rows, cols, k, f32, glu) + launch
+
+    def _skinny_time(self, rows, cols, k, glu=False, f32=False, parts=1) -> float:
+        return self._moe_lib.skinny_time(rows, cols, k, glu, f32, parts)
+
+    # [f32, gate][up to 16, 32, 48, 64 rows]: us that the vendor's product takes at least, that per 1000 k, that per doubling of more than 1024 columns;
+    # us and TB/s of large weights
+    VENDOR = {(False, False): ((6.58, 0.52, 0.07, 1.54, 3.04), (5.88, 0.64, 0.09, 6.1, 4.8), (3.0, 1.09, 0.02, 9.87, 5.11), (6.09, 1.47, 0.21, 6.49, 5.41)),
+              (True, False): ((4.67, 1.71, 0.14, 4.79, 3.32), (3.86, 2.0, 1.5, 9.6, 6.02), (4.25, 1.98, 1.21, 6.76, 2.58), (4.34, 2.0, 1.1, 7.25, 4.82)),
+              (False, True): ((6.07, 0.66, 1.22, 4.64, 5.03), (8.06, 0.84, 0.12, 8.17, 5.03), (8.81, 0.97, 0.03, 8.9, 4.27), (8.78, 1.8, 0.24, 9.17, 4.51)),
+              (True, True): ((4.67, 2.0, 1.5, 7.69, 5.25), (6.04, 2.0, 1.18, 9.15, 4.51), (8.32, 1.99, 0.98, 5.85, 3.31), (6.83, 2.0, 0.89, 8.72, 4.09))}
 
     @staticmethod
-    def skinny_time(rows, cols, k, glu=False, f32=False, parts=1) -> float:
-        k *= 2 if f32 else 1   # in 16-bit halves
-        stream, tiles, padded = 2.0 * cols * k / 5.2e6, -(-cols // 16), -(-rows // 8) * 8
+    def _vendor_time(rows, cols, k, f32, glu=False) -> float:
+        """us of the vendor's GEMM (and of the gate's launch), which are by turns a fifth above and below any smooth rule: the constants are those
+        that made the fewest and smallest wrong choices beside ``skinny_time``, not the closest ones."""
+        least, per_k, per_cols, start, rate = KernelOps.VENDOR[f32, glu][(min(rows, 64) - 1) // 16]
+        least += per_k * 1e-3 * k + (per_cols * math.log2(cols / 1024) if cols > 1024 else 0.0)
+        return max(least, start + (4.0 if f32 else 2.0) * cols * k / 1e6 / rate)
 
-        def intake(nt, rate):
-            return -(-(-(-tiles // nt) * parts) // 256) * 2.0 * k / parts * (16 * nt + padded) / rate
-
-        return 2.2 + max(stream, 0.38 * stream + (intake(2, 60e3) if glu else min(intake(1, 65e3), intake(2, 60e3), intake(4, 54e3))))
-
-    @staticmethod
-    def _vendor_time(rows, cols, k, f32) -> float:
-        if f32:
-            # hardly ever below 10.7 (8.9 for 1024 x 1024), streams at 4.5 TB/s
-            return max(8.9 if max(cols, k) <= 1024 else 10.7, 3.2 + 4.0 * cols * k / 4.5e6)
-        least = 7.5 if k <= 1024 else 10.5 if rows <= 32 else max(10.5, 4.6 + 1.85e-3 * k)
-        return max(least, 3.2 + 2.0 * cols * k / 4.2e6 if rows <= 16 else 4.2 + 2.0 * cols * k / 4.8e6)
-
-    @staticmethod
-    @functools.lru_cache(maxsize=4096)
-    def skinny_parts(rows, cols, k, f32=False) -> int:
+    def _skinny_parts(self, rows, cols, k, f32=False) -> int:
         """Parts of k for a product whose 32-bit sums the next kernel adds up (1: none), or 0 where the vendor's GEMM is the one to run. A part
         more gives idle compute units a share and costs 0.15 us and what it is to write and read it (fitted), and the first one 0.7 us, which
-        the update takes longer with parts in a captured step than in a loop of the two; every wave keeps a piece of 64 halves. us with the residual update and norm behind it, cold weights, vendor / one / two / four parts: 1024 x 3072 with 1, 16, 48
-        rows 14.6 / 8.0 / 7.5 / 7.5, 15.1 / 9.7 / 8.4 / 8.1, 14.7 / 12.8 / 10.2 / 9.1; 2048 x 2048 with 1, 16, 48 rows 14.0 / 7.9 / 7.7 / 8.3, 14.3 /
-        8.8 / 8.2 / 8.9, 14.3 / 10.7 / 9.6 / 10.4; 2048 x 6144 with 16, 48 rows 14.6 / 14.2 / 11.4 / 11.8, 19.9 / 20.2 / 14.6 / 14.0; 4096 x 4096
-        with 24 rows 16.7 / 13.7 / 14.7 / 15.6; 4096 x 12288 with 48 rows 35.0 / 36.7 / 32.1 / 28.8. Three or six parts were never best."""
-        ours, parts = min((KernelOps.parts_time(rows, cols, k, f32, p), p) for p in (1, 2, 4))
-        one = KernelOps.parts_time(rows, cols, k, f32, 1)
+        the update takes longer with parts in a captured step than in a loop of the two; every wave keeps a piece of 64 halves. The vendor's 1.2: it
+        is the slower one by more than ``_vendor_time`` says where parts pay, many k. us with the residual update and norm behind it, cold weights,
+        vendor / one / two / four parts: 1024 x 3072 with 1, 16, 48 rows 14.6 / 8.0 / 7.5 / 7.5, 15.1 / 9.7 / 8.4 / 8.1, 14.7 / 12.8 / 10.2 / 9.1; 2048
+        x 2048 with 1, 16, 48 rows 14.0 / 7.9 / 7.7 / 8.3, 14.3 / 8.8 / 8.2 / 8.9, 14.3 / 10.7 / 9.6 / 10.4; 2048 x 6144 with 16, 48 rows 14.6 / 14.2
+        / 11.4 / 11.8, 19.9 / 20.2 / 14.6 / 14.0; 4096 x 4096 with 24 rows 16.7 / 13.7 / 14.7 / 15.6; 4096 x 12288 with 48 rows 35.0 / 36.7 / 32.1 /
+        28.8. Over 855 sizes (1 - 64 rows, 512 - 6144 columns, k 512 - 12288) the choice takes 1 % longer than the best of the four."""
+        ours, parts = min((self._parts_time(rows, cols, k, f32, p), p) for p in (1, 2, 4))
+        one = self._parts_time(rows, cols, k, f32, 1)
         if ours > 0.94 * one:   # no more parts for what the model cannot tell
             ours, parts = one, 1
-        return parts if ours < KernelOps._vendor_time(rows, cols, k, f32) else 0
+        return parts if ours < 1.2 * self._vendor_time(rows, cols, k, f32) else 0
 
-    @staticmethod
-    def parts_time(rows, cols, k, f32, p) -> float:
+    def _parts_time(self, rows, cols, k, f32, p) -> float:
         if p > 1 and p * 512 > k * (2 if f32 else 1):
             return float("inf")
-        return KernelOps.skinny_time(rows, cols, k, False, f32, p) + (p > 1) * 0.7 + (p - 1) * (0.15 + 0.5e-5 * rows * cols)
+        return self._skinny_time(rows, cols, k, False, f32, p) + (p > 1) * 0.7 + (p - 1) * (0.15 + 0.2e-5 * rows * cols)
 
     def linear_parts(self, x, w, bias=None):
         """``linear`` for a result that ``scaled_add_group_rmsnorm`` takes as ``mix``: where that is faster, 32-bit sums over parts of k,
@@ -595,7 +604,7 @@ class KernelOps:
                 return out
             x = x.normed()
         if (x.dim() == 2 and x.shape[0] <= self.SKINNY_ROWS and self._skinny_ok(x, w, bias)
-                and self.skinny_pays(x.shape[0], w.shape[0], w.shape[1], act in self.GLU_ACTS, x.dtype == torch.float32)):
+                and self.skinny_pays(x.shape[0], w.shape[0], w.shape[1], act in self.GLU_ACTS, x.dtype == torch.float32, act is not None)):
             return self._skinny_linear(x, w, bias, out_f32, act, c0, c1, act_from)
         if out_f32 and x.dtype != torch.float32:
             y = torch.mm(x, w.t(), out_dtype=torch.float32)
@@ -619,13 +628,11 @@ class KernelOps:
 
     NORM_ROWS = 32   # rows that ``linear_update`` takes
 
-    @staticmethod
-    @functools.lru_cache(maxsize=4096)
-    def update_pays(rows, cols, k, f32) -> bool:
+    def _update_pays(self, rows, cols, k, f32) -> bool:
         """Whether a residual update and norm go into the products around them: what their launch costs in a captured step (2.5 us, and 0.05 per
         row and 1024 columns) is weighed against k in parts (``linear_parts``), which needs it, and against the loads that both products do more."""
-        apart = min(KernelOps._vendor_time(rows, cols, k, f32), min(KernelOps.parts_time(rows, cols, k, f32, p) for p in (1, 2, 4)))
-        return KernelOps.skinny_time(rows, cols, k, False, f32) + 0.6 <= apart + 2.5 + 0.05 * rows * cols / 1024
+        apart = min(self._vendor_time(rows, cols, k, f32), min(self._parts_time(rows, cols, k, f32, p) for p in (1, 2, 4)))
+        return self._skinny_time(rows, cols, k, False, f32) + 0.6 <= apart + 2.5 + 0.05 * rows * cols / 1024
 
     def linear_update(self, x, w, bias, residual, norm_w, eps):
         """residual += x . w^T + bias, and the rows for the next products as ``NormedRows`` of its norm; None, and nothing done, where the
@@ -931,6 +938,13 @@ class ReferenceOps:
 
     def latent_prompt_rows(self, dtype, sp, nfreq, cache, meta, T) -> int:
         return 0
+
+    def _mingru_pays(self, rows, width, k, f32) -> bool:
+        """Whether the step in its product's epilogue is expected to take less than the faster product of the two and its launch, 2 us (1 in 32 bits)
+        as the rules' times go: of 1209 sizes (1 - 64 rows, widths 256 - 8192, k 256 - 4096) the choice takes 1 % longer than the faster of the two.
+        us, product and step / this: width 4096, k 2048, 1 and 48 rows 14.8 / 12.6, 20.6 / 16.4; in 32 bits width 512, k 4096, 33 rows 18.5 / 41.2."""
+        apart = min(self._skinny_time(rows, 3 * width, k, False, f32), 1.2 * self._vendor_time(rows, 3 * width, k, f32))
+        return self._seq.mingru_product_time(rows, width, k, f32) < apart + (1.0 if f32 else 2.0)
 
     def mingru_product(self, y, state, x, w, b_z, b_x, meta) -> bool:
         return False

@@ -132,15 +132,14 @@ def test_skinny_linear(M, N, K):
     close_to(half, want + bias.double(), x, w)
 
 
-def test_rules_of_a_few_rows_are_asked_once_per_size(monkeypatch):
+def test_rules_of_a_few_rows_are_asked_once_per_size():
     """Every product of every step asks; a step that is not captured waits for the answers."""
     from types import SimpleNamespace
 
     from hipserve.ops import KernelOps
-    ops, asked, time_of = KernelOps(), [], KernelOps.skinny_time
-    lib = SimpleNamespace(skinny_linear=lambda *a: None, skinny_linear_parts=lambda *a: None, skinny_linear_update=lambda *a: None)
-    ops._lib_ops = {"seq": lib}
-    monkeypatch.setattr(KernelOps, "skinny_time", staticmethod(lambda *a: asked.append(a) or time_of(*a)))
+    ops, asked = KernelOps(), []
+    ops._lib_ops = {"seq": SimpleNamespace(skinny_linear=lambda *a: None, skinny_linear_parts=lambda *a: None, skinny_linear_update=lambda *a: None,
+                                           skinny_time=lambda *a: asked.append(a) or 3.0)}
     x, w, residual = torch.zeros(7, 1048), torch.zeros(1088, 1048), torch.zeros(7, 1088)
     for _ in range(2):
         seen = len(asked)

@@ -53,3 +53,26 @@ def test_choice_of_the_expert_kernels(experts, N, K, glu, by_pairs):
     for pairs, skinny in by_pairs.items():
         cap = -(-(pairs + experts * 31) // 32)   # every expert's last tile partly filled
         assert torch.ops.hipserve_seq.expert_gemm_skinny(pairs, cap, N, K, experts, glu) == skinny, pairs
+
+
+@pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
+@pytest.mark.parametrize("rows,cols,k,f32,glu,pays", [
+    (1, 2048, 2048, False, False, True), (48, 2048, 2048, False, False, True), (64, 6144, 1024, False, False, True), (16, 32000, 1024, True, False, True),
+    (48, 512, 8192, False, False, False), (40, 576, 12288, False, False, False), (64, 32768, 128, False, False, False), (64, 65536, 512, False, False, False),
+    (56, 12288, 2048, True, False, False), (64, 12288, 512, True, False, False), (48, 576, 2048, True, False, False),
+    (16, 2048, 6144, True, True, False), (16, 4096, 12288, False, True, False), (1, 12288, 2048, False, True, True)])
+def test_products_of_a_few_rows_take_the_faster_kernel(rows, cols, k, f32, glu, pays):
+    """Sizes at which one of the two was measured to be at least 10 % faster (the weight-streaming kernel where ``pays``), among them few columns
+    of many k, many columns of few k and matrix products that are bound by their 32-bit arithmetic."""
+    from hipserve.ops import KernelOps
+
+    assert KernelOps().skinny_pays(rows, cols, k, glu, f32) == pays
+
+
+@pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
+@pytest.mark.parametrize("rows,width,k,f32,pays", [(1, 4096, 2048, False, True), (48, 4096, 2048, False, True), (17, 6000, 1024, False, True),
+                                                   (33, 512, 4096, True, False), (64, 256, 3072, True, False)])
+def test_mingru_product_where_it_is_faster(rows, width, k, f32, pays):
+    from hipserve.ops import KernelOps
+
+    assert KernelOps().mingru_pays(rows, width, k, f32) == pays
