@@ -23,7 +23,7 @@ def test_library_loads_and_registers_ops():
 
 
 @pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
-@pytest.mark.parametrize("name", ["window_attention_dma", "latent_attention_dma", "skinny_linear", "expert_ffn"])
+@pytest.mark.parametrize("name", ["window_attention_dma", "latent_attention_dma", "skinny_linear", "expert_ffn", "mingru", "latent_attention_prompt"])
 def test_copies_into_lds_keep_their_wait_states(name, tmp_path):
     """The copies of lds_copy.h are inline assembly, which the compiler's hazard pass does not look into: between the scalar write of
     m0 (the place in LDS) and the copy lies another instruction, and the vector unit has not written the base address just before."""
