@@ -276,22 +276,26 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
 
 }  // namespace
 
-// Which of the two kernels serves tiles of 32 slots; cold weights, us, 8 to 256 experts, K from 512 to 4096 and up to 4000 pairs.
-// expert_gemm_skinny takes 2.2 plus the weights of the experts that so many pairs hit on average at 5.2 TB/s, or what its workgroups of
-// 16 columns read at 80 KB per us and CU, plus 0.3 per 1000 workgroups: it has one per 16 columns of every tile of the capacity, nearly all of
-// them empty where the experts are many. expert_gemm_mfma takes 3 plus 1 per step of 128 k (its steps wait for their loads), the
-// weights at 4.6 TB/s, or what its workgroups of 128 columns read at 34 KB per us and CU (rows once per wave). Both sides are true to a
-// tenth or so: this one where it is expected to be faster by more. Tile kernel / this one: 16 experts, 1024 x 2048: 2 pairs 19.8 / 4.3, 82
-// pairs 26.0 / 15.7, 512 pairs 34.2 / 23.1, 4000 pairs 142 / 83; 2048 x 1024: 82 pairs 17.4 / 15.9, 384 pairs 20.3 / 20.7, 1400 pairs 61 / 43; 8
-// experts, 4096 x 2048: 512 pairs 88.6 / 58.5; 128 experts, 1536 x 2048, gated: 8 pairs 20.9 / 13.5, 64 pairs 77.4 / 62.3; 2048 x 768: 8 pairs
-// 10.2 / 11.5, 2000 pairs 102 / 106; 256 experts, 2048 x 512: 8 pairs 8.1 / 16.8, 512 pairs 56.7 / 73.6. Two tiles of 16 columns per
-// workgroup are hardly ever faster (16 experts, 2048 x 1024, 82 pairs: 19.1, 1400 pairs: 51).
+// Which of the two kernels serves tiles of 32 slots; cold weights, us, 462 sizes of 4 to 256 experts, K from 512 to 4096 and up to 1600
+// pairs. Both read the weights of the experts that so many pairs hit on average. expert_gemm_skinny takes 3.1 plus them at 7 TB/s and what its
+// workgroups of 16 columns (gated 32) take in, the rows at 86 KB per us and CU, over K in whole rounds of its eight waves, and 0.37 per 1000
+// workgroups: it has one per 16 columns of every tile of the capacity. expert_gemm_mfma takes 4.2 plus the weights at 11 TB/s and the longest of
+// its steps of 128 k (they wait for their loads), the weights at 7.7 TB/s, and what its workgroups of 128 columns read at 37 KB per us and CU (rows once
+// per wave). Both are true to 8 %. Ungated products of few pairs per expert, where the two are close, keep the tile kernel until this one is a fifth
+// ahead. The choice takes 1.2 % longer than the faster one on average. Tile kernel / this one: 16 experts, 1024 x 2048: 2 pairs
+// 19.8 / 4.3, 82 pairs 26.0 / 15.7, 512 pairs 34.2 / 23.1; 2048 x 1024: 66 pairs 18.8 / 16.8, 400 pairs 33.6 / 22.2; 8 experts, 4096 x 2048:
+// 128 pairs 39.1 / 32.9; 64 experts, 2816 x 2048, gated: 4 pairs 23.0 / 12.3, 96 pairs 134 / 101; 128 experts, 1536 x 2048, gated: 16 pairs
+// 23.6 / 21.1; 2048 x 768: 8 pairs 12.2 / 14.6, 400 pairs 83 / 86; 256 experts, 2048 x 512: 8 pairs 10.2 / 19.6, 66 pairs 25.5 / 39.7. Two tiles of 16
+// columns per workgroup are hardly ever faster (16 experts, 2048 x 1024, 82 pairs: 19.1, 1400 pairs: 51).
 bool expert_gemm_skinny(long pairs, long ntiles_cap, long N, long K, long E, bool glu) {
   const double used = E * (1 - std::pow(1 - 1.0 / E, (double)pairs)), mean = pairs / used, tiles = used * std::max(1.0, mean / 32 + 0.45);
   const double launched = (double)((glu ? N / 2 : N) + 15) / 16 * ntiles_cap, bytes = used * N * K * 2, rows = std::min(32.0, mean);
-  auto read = [&](double cols, double rows_read, double rate) { return std::max(1.0, tiles * N / cols / 256) * 2 * K * (cols + rows_read) / rate; };
-  const double ours = 2.2 + std::max(bytes / 5.2e6, read(16, rows / (glu ? 2 : 1), 80e3)) + 0.3e-3 * launched;
-  return ours < 0.89 * (3 + std::max({K / 128.0, bytes / 4.6e6, read(128, 4 * rows, 34e3)}));
+  const double cols = glu ? 32 : 16, whole = (K + 511) / 512 * 512;
+  const double mine = std::max(1.0, tiles * N / cols / 256) * (2 * whole * (cols / 300e3 + rows / 86e3) + 0.22);
+  const double ours = 3.1 + std::max(bytes / 5.7e6, 0.81 * bytes / 5.7e6 + mine) + 0.37e-3 * launched;
+  const double theirs = 4.2 + 0.7 * bytes / 7.7e6 +
+                        std::max({0.97 * K / 128, bytes / 7.7e6, std::max(1.0, tiles * N / 128 / 256) * 2 * K * (128 + 4 * rows) / 37.5e3});
+  return ours < (glu || mean > 17 ? 1.0 : 0.8) * theirs;
 }
 
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,

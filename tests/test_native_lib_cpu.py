@@ -56,6 +56,17 @@ def test_choice_of_the_expert_kernels(experts, N, K, glu, by_pairs):
 
 
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
+@pytest.mark.parametrize("experts,N,K,glu,by_pairs", [   # measured, as above: gated products, a part of a round of the waves, many pairs per expert
+    (64, 2816, 2048, True, {4: True, 96: True, 1600: True}), (256, 512, 2048, True, {4: True, 32: True}), (32, 1024, 1024, True, {128: True, 264: True}),
+    (32, 1000, 520, False, {1200: False, 1600: False}), (64, 2048, 704, False, {1600: False}), (16, 2048, 1024, False, {400: True, 600: True})])
+def test_choice_of_the_expert_kernels_by_load(experts, N, K, glu, by_pairs):
+    load_kernel_library("seq")
+    for pairs, skinny in by_pairs.items():
+        cap = -(-(pairs + experts * 31) // 32)
+        assert torch.ops.hipserve_seq.expert_gemm_skinny(pairs, cap, N, K, experts, glu) == skinny, pairs
+
+
+@pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
 @pytest.mark.parametrize("rows,cols,k,f32,glu,pays", [
     (1, 2048, 2048, False, False, True), (48, 2048, 2048, False, False, True), (64, 6144, 1024, False, False, True), (16, 32000, 1024, True, False, True),
     (48, 512, 8192, False, False, False), (40, 576, 12288, False, False, False), (64, 32768, 128, False, False, False), (64, 65536, 512, False, False, False),
