@@ -719,14 +719,14 @@ __global__ __launch_bounds__(kStepThreads) void gated_delta_step_kernel(const Ga
   // All that is small before the state: loads come back in order, and the chain (convolution, unit vectors, decays) runs while the state's
   // 64 KB arrive. One launch of 16 sequences x 16 heads 13.3 -> 11.8 us, of one x 8 9.2 -> 8.0 (each tap waited
   // for the one before it, all of them for the state, and gates and weights were asked for where they are used).
-  constexpr int kConvIt = 1, kTaps = 4;
+  constexpr int kTaps = 4;
   const int channels = 2 * dim + vdim;
-  const bool quick = taps <= kTaps && channels <= kConvIt * kStepThreads;
+  const bool quick = taps <= kTaps && channels <= kStepThreads;
   float* cs = p.conv_state + (long)p.seq_state[s] * max(hist, 1) * C;
   auto channel_of = [&](int i) {
     return i < dim ? kh * dim + i : i < 2 * dim ? nqk + kh * dim + i - dim : 2 * nqk + h * vdim + i - 2 * dim;
   };
-  float now[kConvIt], old[kConvIt][kTaps - 1], cwt[kConvIt][kTaps];
+  float now = 0.f, old[kTaps - 1], cwt[kTaps];
   const float beta_in = ldf<T>(row, p.off_b + h), weight = tid < vdim ? p.norm_w[tid] : 0.f;   // vdim <= 256
   float decay_in = 0.f, bias_in = 0.f, rate = 0.f, gate_in = 0.f;
   if constexpr (!CH) {
@@ -736,15 +736,12 @@ __global__ __launch_bounds__(kStepThreads) void gated_delta_step_kernel(const Ga
     if (tid < vdim) gate_in = ldf<T>(row, p.off_g + h * vdim + tid);
   }
   if (quick) {
+    const int c = channel_of(min(tid, channels - 1));
+    now = ldf<T>(row, c);
 #pragma unroll
-    for (int q = 0; q < kConvIt; ++q) {
-      const int c = channel_of(min(tid + q * kStepThreads, channels - 1));
-      now[q] = ldf<T>(row, c);
-#pragma unroll
-      for (int j = 0; j < kTaps; ++j) {
-        cwt[q][j] = j < taps ? p.conv_w[(long)c * taps + j] : 0.f;
-        if (j < kTaps - 1) old[q][j] = carried && j < hist ? cs[(long)j * C + c] : 0.f;
-      }
+    for (int j = 0; j < kTaps; ++j) {
+      cwt[j] = j < taps ? p.conv_w[(long)c * taps + j] : 0.f;
+      if (j < kTaps - 1) old[j] = carried && j < hist ? cs[(long)j * C + c] : 0.f;
     }
   }
   f32x4 st[VEC == 4 ? kStepIt : 1];
@@ -774,21 +771,18 @@ __global__ __launch_bounds__(kStepThreads) void gated_delta_step_kernel(const Ga
       low[j] = j < p.ra ? ldf<T>(row, p.off_a + j) : ldf<T>(row, p.off_g + j - p.ra);
   }
   // the convolution of the head's channels; with heads of their own queries and keys the kept inputs move on here
-  if (quick) {
+  if (quick && tid < channels) {
+    const int c = channel_of(tid);
+    float a = 0.f, last = 0.f;
 #pragma unroll
-    for (int q = 0; q < kConvIt; ++q) {
-      const int i = tid + q * kStepThreads, c = channel_of(min(i, channels - 1));
-      float a = 0.f, last = 0.f;
-#pragma unroll
-      for (int j = 0; j < kTaps - 1; ++j) {
-        if (j < hist) a = __builtin_fmaf(cwt[q][j], old[q][j], a);
-        last = j + 1 == hist ? cwt[q][j + 1] : hist == 0 ? cwt[q][0] : last;
-        if (own_conv && j > 0 && j < hist && i < channels) cs[(long)(j - 1) * C + c] = old[q][j];
-      }
-      if (own_conv && hist > 0 && i < channels) cs[(long)(hist - 1) * C + c] = now[q];
-      a = __builtin_fmaf(last, now[q], a);
-      if (i < channels) xs[i] = a * sigmoid_f(a);
+    for (int j = 0; j < kTaps - 1; ++j) {
+      if (j < hist) a = __builtin_fmaf(cwt[j], old[j], a);
+      last = j + 1 == hist ? cwt[j + 1] : hist == 0 ? cwt[0] : last;
+      if (own_conv && j > 0 && j < hist) cs[(long)(j - 1) * C + c] = old[j];
     }
+    if (own_conv && hist > 0) cs[(long)(hist - 1) * C + c] = now;
+    a = __builtin_fmaf(last, now, a);
+    xs[tid] = a * sigmoid_f(a);
   }
   for (int i = quick ? channels : tid; i < channels; i += kStepThreads) {
     const int c = channel_of(i);

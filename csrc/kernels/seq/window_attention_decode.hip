@@ -141,16 +141,11 @@ HS_DEVICE void prepare_row(const WindowPrep& pr, const T* __restrict__ row, long
   }
   early();   // nothing that was asked for before is waited for behind this
   const float pos = (float)at;
-  for (int i = tid; i < pr.nfreq; i += nt) {
+  if (tid < pr.nfreq) {   // at most 64 frequencies, at least 64 threads
     float sn, cs;
-    float w = freq;
-    if (i >= nt) {
-      w = pr.inv_freq[i];
-      landed();
-    }
-    sincosf(pos * w, &sn, &cs);
-    angles[i] = cs * pr.amp;
-    angles[pr.nfreq + i] = sn * pr.amp;
+    sincosf(pos * freq, &sn, &cs);
+    angles[tid] = cs * pr.amp;
+    angles[pr.nfreq + tid] = sn * pr.amp;
   }
   if (pr.norm_mode == 1) {
     a = wave_sum(a);
