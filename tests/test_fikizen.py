@@ -490,3 +490,79 @@ def test_preset_and_cli_model_resolution(tmp_path):
     m = resolve_model_config(path)
     assert isinstance(m, FikizenConfig) and model_class(m).__name__ == "FikizenModel"
     assert isinstance(resolve_model_config("tiny-fikizen"), FikizenConfig)
+
+# ---------------------------------------------------------------- decode steps of a few rows
+def batch_meta(lens, ctxs, dev, state, width, block_size=4):
+    """Step metadata of one sequence per entry, ``lens`` rows that end at ``ctxs`` tokens each; a sequence's pages and slot do not depend on
+    the others."""
+    n, cu = len(lens), [0]
+    for l in lens:
+        cu.append(cu[-1] + l)
+    order = torch.randperm(n * width, generator=torch.Generator().manual_seed(n)).int().view(n, width).to(dev)
+    pos = torch.cat([torch.arange(c - l, c) for l, c in zip(lens, ctxs)]).to(dev)
+    req = torch.cat([torch.full((l,), i) for i, l in enumerate(lens)]).to(dev)
+    decode = max(lens) == 1
+    m = AttnMeta(num_prefill_tokens=0 if decode else cu[-1], num_decode=n if decode else 0, positions=pos,
+                 slot_mapping=order[req, pos // block_size].long() * block_size + pos % block_size)
+    m.seq_cu, m.seq_ctx = torch.tensor(cu, dtype=torch.int32, device=dev), torch.tensor(ctxs, dtype=torch.int32, device=dev)
+    m.seq_bt, m.seq_state, m.state = order, torch.arange(n, dtype=torch.int32, device=dev), state
+    m.max_q, m.max_ctx = max(lens), max(ctxs)
+    return m
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("last_ff", [True, False])
+@pytest.mark.parametrize("n,everywhere", [(1, True), (1, False), (16, True), (16, False), (17, True), (32, True), (32, False), (33, False)])
+def test_decode_steps_with_updates_inside_the_products(n, everywhere, last_ff, dtype):
+    """The residual updates and norms of decode steps inside the products around them (up to 32 rows: all, or those that the rule says), or beside
+    products in parts of k, layers with and without a feed-forward, a shared one, the last without one or with: eager against the oracle, captured
+    against eager."""
+    from hipserve.models.registry import build_model
+    from hipserve.ops import NormedRows
+    f = O.dense(ff=6144)
+    a = dict(heads=4, kv_heads=2, dim=64, vdim=64, window=6, rot_dims=32)
+    layers = [O.attn_layer(mlp=f, **a), O.delta_layer(heads=4, kv_heads=2, dim=32, vdim=64)]
+    layers += [O.shared(layers, 0), O.parallel_layer(left=a, heads=2, dim=64, mlp=f), O.delta_layer(heads=2, kv_heads=2, dim=5, vdim=70, mlp=f if last_ff else None)]
+    cfg = O.make_config(layers, width=128)
+    W = O.make_weights(cfg, seed=n, rank=32)
+    dev, ops = torch.device("cuda", 0), get_ops("cuda")
+    model = build_model(FikizenConfig.from_dict(cfg), TPGroup(0, 1, None, dev), dev, getattr(torch, dtype), ops, max_pos=64)
+    model.load_tensors(lambda k: W[k])
+    kv, state = model.allocate_kv_cache(n * 5, 4), model.allocate_state(n)
+    new, lens = 3, [4 + i % 5 for i in range(n)]
+    toks = [tokens(l + new, cfg["vocab"], 100 + i) for i, l in enumerate(lens)]
+    refs = [O.forward(cfg, W, t) for t in toks]
+    meta = batch_meta(lens, lens, dev, state, 5)
+    model.forward(torch.tensor(sum((t[:l] for t, l in zip(toks, lens)), []), device=dev), meta, kv)
+    updates, parts = [], []
+    update_of, parts_of = ops.linear_update, ops.linear_parts
+    if everywhere:
+        ops.update_pays = lambda *x: True
+    pays = lambda k: n <= 32 and k * (4 if dtype == "float32" else 2) % 16 == 0 and ops.update_pays(n, 128, k, dtype == "float32")   # rows of 16 bytes
+    ops.linear_update = lambda *x: updates.append((x[0].shape[1], update_of(*x))) or updates[-1][1]
+    ops.linear_parts = lambda *x: parts.append(parts_of(*x)) or parts[-1]
+    flat = [t for run in [*kv, *(state or [])] if run is not None for t in (run if isinstance(run, (list, tuple)) else [run])]
+    ends = 9 if last_ff else 8   # sublayers
+    try:
+        for step in range(new):
+            meta = batch_meta([1] * n, [l + step + 1 for l in lens], dev, state, 5)
+            ids = torch.tensor([t[l + step] for t, l in zip(toks, lens)], device=dev)
+            before = [t.clone() for t in flat]
+            updates.clear(), parts.clear()
+            got = model.compute_logits(model.forward(ids, meta, kv)).cpu()
+            assert len(updates) == ends - 1 and all(isinstance(u, NormedRows) == pays(k) for k, u in updates)
+            assert len(parts) == 1 + sum(u is None for _, u in updates) and sum(p.dim() == 3 for p in parts) >= 3 * (n > 32)
+            want = torch.stack([r[l + step] for r, l in zip(refs, lens)])
+            check_all({("a", i): got[i] for i in range(n)}, "a", want, TOL[dtype])
+            after = [t.clone() for t in flat]
+            side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                logits = model.compute_logits(model.forward(ids, meta, kv))
+            for _ in range(2):
+                for t, b in zip(flat, before):
+                    t.copy_(b)
+                graph.replay()
+                assert torch.equal(logits.cpu(), got) and all(torch.equal(t, b) for t, b in zip(flat, after))
+    finally:
+        del ops.linear_update, ops.linear_parts

@@ -420,6 +420,52 @@ def test_latent_attention_long_prompt_gpu(kv_rank, window):
     assert rel_err(got, want) < TOL["bfloat16"]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("window", [0, 40, 5000])
+@pytest.mark.parametrize("before,lens", [([0], [64]), ([0], [65]), ([70], [70]), ([71], [70]), ([0, 30, 128, 5, 0], [33, 100, 1, 64, 257]),
+                                         ([0, 30, 100, 5, 0], [150, 100, 131, 164, 257]), ([200, 0], [90, 310])])
+def test_latent_attention_with_formed_keys_gpu(before, lens, window):
+    """Prompt steps whose rows and visible cache rows lie just below and above what the formed keys and values are for, behind tokens of earlier
+    steps or none: the path that is meant runs, and is as close to the oracle as the one on the latents."""
+    dev, dt, ops = torch.device("cuda"), torch.bfloat16, get_ops("cuda")
+    l = O.attn_layer(heads=3, dim=128, rot_dim=64, vdim=128, q_rank=40, kv_rank=512, window=window)
+    cfg = O.make_config([l], width=64)
+    W = O.make_weights(cfg, seed=37)
+    g = torch.Generator().manual_seed(sum(lens) + window)
+    ctx = [b + n for b, n in zip(before, lens)]
+    hs = [torch.randn(c, 64, generator=g).bfloat16().float() for c in ctx]
+    want = torch.cat([O.latent_attention(h, W, "l0.mix.", l["mixer"], 1e-6)[b:] for h, b in zip(hs, before)])
+    mix = LatentAttention(HybridConfig.from_dict(cfg).layers[0].mixer, 64, 1e-6, dev, dt, ops)
+    mix.load(lambda k: W[k], "l0.mix.")
+    bs, n = 16, len(lens)
+    nb = -(-max(ctx) // bs)
+    bt = torch.randperm(n * nb, generator=g).int().view(n, nb)
+
+    def step(a, b, cache):   # rows a[i] .. b[i] - 1 of every sequence
+        m = [y - x for x, y in zip(a, b)]
+        pos = torch.cat([torch.arange(x, y) for x, y in zip(a, b)])
+        seq = torch.cat([torch.full((k,), i) for i, k in enumerate(m)])
+        cu = torch.tensor([0] + torch.tensor(m).cumsum(0).tolist(), dtype=torch.int32)
+        meta = AttnMeta(num_prefill_tokens=sum(m), num_decode=0, positions=pos.to(dev), slot_mapping=(bt.long()[seq, pos // bs] * bs + pos % bs).to(dev),
+                        seq_cu=cu.to(dev), seq_ctx=torch.tensor(b, dtype=torch.int32, device=dev), seq_bt=bt.to(dev), max_q=max(m), max_ctx=max(b))
+        return mix.forward(torch.cat([h[x:y] for h, x, y in zip(hs, a, b)]).to(dev, dt), meta, cache)
+
+    formed, run = [], ops.latent_prompt_attention
+    ops.latent_prompt_attention = lambda *x: formed.append(x[8]) or run(*x)
+    errors = []
+    for least in (type(ops).LATENT_PROMPT_MIN_ROWS, 1 << 30):
+        ops.LATENT_PROMPT_MIN_ROWS = least
+        cache = torch.full(mix.cache_shape(n * nb, bs), float("nan"), device=dev, dtype=dt)
+        if sum(before):
+            step([0] * n, before, cache)
+        formed.clear()
+        got = step(before, ctx, cache)
+        T, seen = sum(lens), max(ctx) if not window else min(max(ctx), max(lens) + window - 1)
+        assert formed == ([n * seen] if T >= least and n * seen <= 2 * T else [])
+        errors.append(float((got.double().cpu() - want).norm() / want.double().norm()))
+    assert errors[1] < 2e-2 and errors[0] < 1.25 * errors[1], errors
+
+
 def test_openai_server_and_cli_config(tmp_path):
     """The engine command line resolves a checkpoint folder of this design (model class by config.json) and
     the OpenAI server completes, streams and samples with penalties and logprobs on it."""

@@ -1223,3 +1223,66 @@ def test_window_step(heads, kv, dim, ctxs, nfreq, mode, own, opts, dtype):
     tol = 0.08 if dtype == torch.bfloat16 else 60 * 2.0 ** -20
     out, want = out[:n].float(), want[:n].float()   # the padding row's is nobody's
     assert (out - want).abs().max() <= tol * max(1.0, float(want.abs().max()))
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,kv,dim,ctxs,opts", [
+    (8, 2, 128, [1, 5, 33], {"sink": True}), (8, 2, 128, [2, 300, 600], {"sink": True}), (8, 2, 128, [1, 31, 200], {"sink_w": True, "gate": True}),
+    (8, 2, 128, [129, 500], {"sink_w": True, "softcap": 3.0}), (40, 2, 64, [5, 129, 400], {"window": 100, "keep_first": 7, "channel_gate": True, "scale": 0.5}),
+    (4, 4, 64, [40, 257], {"softcap": 2.0, "channel_gate": True, "scale": 1.5}), (16, 2, 64, [64, 65, 300], {"chunk": 64, "gate": True, "scale": 0.25})])
+def test_window_step_options(heads, kv, dim, ctxs, opts, dtype):
+    """Sinks, gates, the cap and the factor of the launch for a decode step, in one run and in several, against 64 bits. Projections that are neither
+    normed nor turned go through unaltered, so that the bound holds the attention's own roundings alone: it sees any one key left out (asserted on
+    the 64-bit side), and any sink but one of weight 1 among hundreds of keys in bf16."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(heads * dim + sum(ctxs))
+    n, bs, nq, nk = len(ctxs), 8, heads * dim, kv * dim
+    gated, factor = opts.get("gate", False) or opts.get("channel_gate", False), opts.get("scale", 1.0)
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=opts.get("window", 0), scale=dim ** -0.5, sink=opts.get("sink", "sink_w" in opts),
+                         keep_first=opts.get("keep_first", 0), softcap=opts.get("softcap", 0.0), channel_gate=opts.get("channel_gate", False),
+                         chunk=opts.get("chunk", 0), diff=0.0, q_size=nq, k_size=nk, v_size=nk, kv_from=None, qk_norm=False, head_norm=False, unit_qk=False,
+                         v_norm=False, temp_coef=0.0, temp_every=0, scaling=None)
+    sp.reach = sp.window + sp.keep_first if sp.window > 0 else sp.chunk
+    width = -(-max(ctxs) // bs)
+    bt = torch.randperm(n * width, generator=g).int().view(n, width)
+    cache, proj = torch.randn(n * width * bs, 2 * kv, dim, generator=g), torch.randn(n, nq + 2 * nk + nq, generator=g)
+    for s, c in enumerate(ctxs):   # an element of every key's value that tells it from its neighbours
+        for j in range(c):
+            cache[int(bt[s, j // bs]) * bs + j % bs, kv:, j % dim] += 16
+        proj[s, nq + nk:].view(-1, dim)[:kv, (c - 1) % dim] += 16
+    cache, proj = cache.view(n * width, bs, 2 * nk).to(dtype), proj.to(dtype)
+    slots = torch.tensor([int(bt[s, (c - 1) // bs]) * bs + (c - 1) % bs for s, c in enumerate(ctxs)])
+    after = cache.clone()   # with every step's own key and value
+    after.view(-1, 2 * nk)[slots] = proj[:, nq:nq + 2 * nk]
+    sink_w = torch.randn(heads, generator=g) + 4 if opts.get("sink_w") else None
+    rows, gate_off = after.double().view(-1, 2 * kv, dim), nq + 2 * nk
+    want, size = torch.empty(n, heads, dim, dtype=torch.float64), torch.empty(n, heads, dim, dtype=torch.float64)   # size: sum of weight x |value|
+    unit = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -17   # weights and outputs rounded to 8 bits, 2^-8 each; in fp32 scores of sums of up to 128 products
+    for s in range(n):
+        p = ctxs[s] - 1
+        lo = p - p % sp.chunk if sp.chunk else max(0, p - sp.window + 1) if sp.window else 0
+        js = sorted(set(range(lo, p + 1)) | (set(range(min(sp.keep_first, p + 1))) if sp.window else set()))
+        kv_rows = rows[[int(bt[s, j // bs]) * bs + j % bs for j in js]].repeat_interleave(heads // kv, 1)
+        k, v = kv_rows[:, :heads], kv_rows[:, heads:]
+        x = torch.einsum("jhd,hd->hj", k, proj[s, :nq].double().view(heads, dim)) * sp.scale
+        x = sp.softcap * torch.tanh(x / sp.softcap) if sp.softcap else x
+        extra = torch.zeros(heads, int(sp.sink), dtype=torch.float64) if sink_w is None else sink_w.double()[:, None]
+        w = torch.softmax(torch.cat([x, extra], 1), 1)[:, :len(js), None]
+        v = v.transpose(0, 1)
+        want[s], size[s] = (w * v).sum(1), (w * v.abs()).sum(1)
+        if len(js) > 1:   # what any one key left out would change
+            change = (w / (1 - w) * (want[s][:, None] - v)).abs() / (unit * size[s])[:, None]
+            assert float(change.amax((0, 2)).min()) > 1
+    if gated:
+        gates = torch.sigmoid(proj[:, gate_off:gate_off + (nq if sp.channel_gate else heads)].double()).view(n, heads, -1)
+        want, size = want * gates, size * gates
+    ops = get_ops("cuda")
+    meta = SimpleNamespace(seq_ctx=torch.tensor(ctxs).int().cuda(), seq_cu=torch.arange(n + 1).int().cuda(), seq_bt=bt.cuda(), num_decode=n, num_prefill_tokens=0,
+                           max_ctx=max(ctxs), max_q=1, positions=torch.tensor(ctxs).cuda() - 1, slot_mapping=slots.cuda())
+    c, out = cache.cuda(), torch.empty(n, nq, dtype=dtype, device="cuda")
+    assert ops.window_step(out, proj.cuda(), c, meta, torch.empty(0, device="cuda"), sp, None, None, 1e-5, gate_off if gated else -1, factor,
+                           None if sink_w is None else sink_w.cuda())
+    assert torch.equal(c.cpu(), after)
+    wrong = (out.double().cpu().view(n, heads, dim) - factor * want).abs() / (unit * factor * size)
+    assert wrong.max() < 1, wrong.max()
