@@ -10,9 +10,9 @@
 // buffers (20 KB: keys, values, rotary parts), three tiles ahead; one barrier per tile; V^T by transposing reads. What differs:
 // the key rows lie side by side, so that tiles start at the first key a workgroup's rows see and no page is looked up; a wave
 // leaves out the tiles that its own rows do not see (of 128 rows x 1024 keys every tenth).
-// 8192 rows (4 prompts of 2048) x 16 heads, window 1024: 374 -> 142 us (450 TFLOP/s of the products with visible keys; the LDS is read
-// about as long as the matrix units work: 20 KB per 32 rows and tile), the mixer with its products 676 -> 355 us; 41 prompts of 150
-// 393 -> 279. Errors of the mixer's output against 64 bits, both ways: 7.0e-3 - 7.4e-3.
+// 8192 rows (4 prompts of 2048) x 16 heads, window 1024: 363 -> 131 us (490 TFLOP/s of the products with visible keys; the LDS is read
+// about as long as the matrix units work: 20 KB per 32 rows and tile), the mixer with its products 680 -> 349 us; 41 prompts of 150
+// 388 -> 274. Errors of the mixer's output against 64 bits, both ways: 7.0e-3 - 7.4e-3.
 #include "lds_copy.h"
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"

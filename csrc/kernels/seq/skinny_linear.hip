@@ -70,7 +70,7 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int IT = (ST + 1) / 2, SQ = 4;
+  constexpr int IT = (ST + 1) / 2, SQ = 4;   // 16 threads x SQ loads x 4 sums of 16 columns each: rows of up to 4096
   f32x4 sq[IT][SQ];
   float res[IT][NT];
   SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, k1 - k0, smem, lane, wave, [&] {

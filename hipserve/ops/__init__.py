@@ -939,13 +939,6 @@ class ReferenceOps:
     def latent_prompt_rows(self, dtype, sp, nfreq, cache, meta, T) -> int:
         return 0
 
-    def _mingru_pays(self, rows, width, k, f32) -> bool:
-        """Whether the step in its product's epilogue is expected to take less than the faster product of the two and its launch, 2 us (1 in 32 bits)
-        as the rules' times go: of 1209 sizes (1 - 64 rows, widths 256 - 8192, k 256 - 4096) the choice takes 1 % longer than the faster of the two.
-        us, product and step / this: width 4096, k 2048, 1 and 48 rows 14.8 / 12.6, 20.6 / 16.4; in 32 bits width 512, k 4096, 33 rows 18.5 / 41.2."""
-        apart = min(self._skinny_time(rows, 3 * width, k, False, f32), 1.2 * self._vendor_time(rows, 3 * width, k, f32))
-        return self._seq.mingru_product_time(rows, width, k, f32) < apart + (1.0 if f32 else 2.0)
-
     def mingru_product(self, y, state, x, w, b_z, b_x, meta) -> bool:
         return False
 
