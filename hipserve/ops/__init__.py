@@ -323,7 +323,13 @@ class KernelOps:
                 while -(-span // part) > 64:
                     part *= 2
                 nparts = max(1, -(-span // part))
-                ws_acc = ws_ml = None
+                # Two launches where a compute unit would prepare several workgroups' rows one behind the other: its registers hold one workgroup of 128
+        # dims at a time, two of fp32 without the preparation. us, one launch / two, 8 key heads: fp32, 48 and 64 rows of 70 keys 20.1 / 16.1, 21.7 /
+        # 17.4, of 900 keys 86.5 / 85.3, 119 / 96.5, 8 rows in runs 26.2 / 24.0, 32 rows (256 workgroups) 51.9 / 62.6; bf16, 48 and 64 rows of 70
+        # keys 10.2 / 11.3, 10.6 / 11.7, 48 of 300 22.4 / 21.2, of 900 50.2 / 48.7; 32 key heads, 64 rows of 300 88.6 / 84.6.
+        if prep is not None and sp.dim == 128 and (groups * nparts > 256 if proj.dtype == torch.float32 else groups > 256 and span > 256):
+            return False
+        ws_acc = ws_ml = None
                 if nparts > 1:
                     ws_acc = torch.empty(nparts, heads, nd, kv_rank, device=q.device, dtype=torch.float32)
                     ws_ml = torch.empty(nparts, heads, nd, 2, device=q.device, dtype=torch.float32)
