@@ -636,9 +636,11 @@ class KernelOps:
 
     def _update_pays(self, rows, cols, k, f32) -> bool:
         """Whether a residual update and norm go into the products around them: what their launch costs in a captured step (2.5 us, and 0.05 per
-        row and 1024 columns) is weighed against k in parts (``linear_parts``), which needs it, and against the loads that both products do more."""
+        row and 1024 columns) is weighed against k in parts (``linear_parts``), which needs it, against the loads that both products do more, and
+        against what the next product, taken to be of three times the columns, loses where the vendor's GEMM would be the one to run."""
         apart = min(self._vendor_time(rows, cols, k, f32), min(self._parts_time(rows, cols, k, f32, p) for p in (1, 2, 4)))
-        return self._skinny_time(rows, cols, k, False, f32) + 0.6 <= apart + 2.5 + 0.05 * rows * cols / 1024
+        after = max(0.0, self._skinny_time(rows, 3 * cols, cols, False, f32) - self._vendor_time(rows, 3 * cols, cols, f32))
+        return self._skinny_time(rows, cols, k, False, f32) + 0.6 + after <= apart + 2.5 + 0.05 * rows * cols / 1024
 
     def linear_update(self, x, w, bias, residual, norm_w, eps):
         """residual += x . w^T + bias, and the rows for the next products as ``NormedRows`` of its norm; None, and nothing done, where the
