@@ -323,13 +323,7 @@ class KernelOps:
                 while -(-span // part) > 64:
                     part *= 2
                 nparts = max(1, -(-span // part))
-                # Two launches where a compute unit would prepare several workgroups' rows one behind the other: its registers hold one workgroup of 128
-        # dims at a time, two of fp32 without the preparation. us, one launch / two, 8 key heads: fp32, 48 and 64 rows of 70 keys 20.1 / 16.1, 21.7 /
-        # 17.4, of 900 keys 86.5 / 85.3, 119 / 96.5, 8 rows in runs 26.2 / 24.0, 32 rows (256 workgroups) 51.9 / 62.6; bf16, 48 and 64 rows of 70
-        # keys 10.2 / 11.3, 10.6 / 11.7, 48 of 300 22.4 / 21.2, of 900 50.2 / 48.7; 32 key heads, 64 rows of 300 88.6 / 84.6.
-        if prep is not None and sp.dim == 128 and (groups * nparts > 256 if proj.dtype == torch.float32 else groups > 256 and span > 256):
-            return False
-        ws_acc = ws_ml = None
+                ws_acc = ws_ml = None
                 if nparts > 1:
                     ws_acc = torch.empty(nparts, heads, nd, kv_rank, device=q.device, dtype=torch.float32)
                     ws_ml = torch.empty(nparts, heads, nd, 2, device=q.device, dtype=torch.float32)
@@ -403,6 +397,12 @@ class KernelOps:
             while -(-span // part) > 32 or groups * -(-span // part) > 1024 and part < span:
                 part *= 2
         nparts = max(1, -(-span // part))
+        # Two launches where a compute unit would prepare several workgroups' rows one behind the other: its registers hold one workgroup of 128
+        # dims at a time, two of fp32 without the preparation. us, one launch / two, 8 key heads: fp32, 48 and 64 rows of 70 keys 20.1 / 16.1, 21.7 /
+        # 17.4, of 900 keys 86.5 / 85.3, 119 / 96.5, 8 rows in runs 26.2 / 24.0, 32 rows (256 workgroups) 51.9 / 62.6; bf16, 48 and 64 rows of 70
+        # keys 10.2 / 11.3, 10.6 / 11.7, 48 of 300 22.4 / 21.2, of 900 50.2 / 48.7; 32 key heads, 64 rows of 300 88.6 / 84.6.
+        if prep is not None and sp.dim == 128 and (groups * nparts > 256 if proj.dtype == torch.float32 else groups > 256 and span > 256):
+            return False
         ws_acc = ws_ml = None
         if nparts > 1:
             ws_acc = torch.empty(nparts, sp.heads, nd, sp.vdim, device=proj.device, dtype=torch.float32)
@@ -497,7 +497,12 @@ class KernelOps:
     def delta_rule_low(self, out, state, proj, w2, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0) -> bool:
         """``delta_rule`` of a decode step with the bottleneck's product (the last columns of ``proj`` times ``w2``) in its launch; False, and
         nothing done, where it is a product before it."""
-        per = 16 // proj.element_size()
+        # Every workgroup (a head of a row) reads its 64 rows of w2 again, from its compute unit's 32 KB of cache where they fit: a launch saved
+        # (1.9 us) against that. us, one launch / two: rank 64 in bf16 1024 workgroups 10.6 / 12.1, 4096 33.2 / 33.0, in fp32 2048 19.7 / 20.6, 3072
+        # 28.9 / 27.8; rank 128 in bf16 2048 19.6 / 20.2, 3072 31.2 / 27.4, 16384 137 / 111, in fp32 512 7.9 / 8.7, 1024 13.1 / 12.3, 16384 176 / 117.
+        per, row = 16 // proj.element_size(), w2.shape[1] * w2.element_size()
+        if proj.shape[0] * sp.heads * row > (1 << 19 if row <= 256 else 1 << 18):
+            return False
         if not (meta.max_q == 1 and self._delta.delta_rule_step_ok(sp.dim) and w2.shape[1] % 32 == 0 and w2.shape[1] <= self.DELTA_LOW_RANK
                 and proj.dtype == w2.dtype and w2.is_contiguous() and proj.stride(0) % per == 0 and all(t.data_ptr() % 16 == 0 for t in (state[0], proj, w2))):
             return False

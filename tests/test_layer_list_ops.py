@@ -167,6 +167,21 @@ def test_window_step_in_one_launch_by_its_workgroups(dtype, kv, dim, n, keys, on
     assert ops.window_step(torch.zeros_like(proj), proj, proj, meta, torch.zeros(dim // 2), sp, None, None, 1e-6, -1) == one and len(ran) == one
 
 
+@pytest.mark.parametrize("dtype,rank,most", [(torch.bfloat16, 64, 64), (torch.bfloat16, 128, 32), (torch.float32, 64, 32), (torch.float32, 128, 8)])
+def test_bottleneck_in_the_rules_launch_by_its_workgroups(dtype, rank, most):
+    """Up to ``most`` rows of 64 heads; a product of its own where its rows would be read too often."""
+    from types import SimpleNamespace
+
+    from hipserve.ops import KernelOps
+    ops, ran = KernelOps(), []
+    ops._lib_ops = {"delta": SimpleNamespace(delta_rule_step_ok=lambda *a: True, delta_rule_step=lambda *a: ran.append(a))}
+    sp, w2 = SimpleNamespace(heads=64, dim=64), torch.zeros(4096, rank, dtype=dtype)
+    for n in (1, most, most + 1):
+        meta, proj = SimpleNamespace(max_q=1, seq_cu=None, seq_ctx=None, seq_state=None), torch.zeros(n, 8, dtype=dtype)
+        ran.clear()
+        assert ops.delta_rule_low(None, [torch.zeros(4)], proj, w2, None, None, None, sp, 1e-6, meta) == (n <= most) == bool(ran)
+
+
 @pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
 @pytest.mark.parametrize("M", [1, 17, 70])
 @pytest.mark.parametrize("first", [1, 16, 39])
