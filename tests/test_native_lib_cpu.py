@@ -42,6 +42,17 @@ def test_copies_into_lds_keep_their_wait_states(name, tmp_path):
             assert not wrote or int(wrote[2] or wrote[1]) < int(base[1]) or int(wrote[1]) > int(base[2]), (ln, code[i])
 
 
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+def test_a_carried_state_is_asked_for_at_once(tmp_path):
+    """The chunked gated rule's scan loads its 16 numbers per lane with no wait between them."""
+    asm = tmp_path / "k.s"
+    subprocess.run([_build.HIPCC, *_build.HIP_FLAGS, "-I", os.path.join(_build.CSRC, "include"), "-S", "--cuda-device-only",
+                    os.path.join(_build.CSRC, "kernels", "seq", "delta_chunk.hip"), "-o", asm], check=True, capture_output=True)
+    code = re.split(r"^_ZN\S*delta_chunk_scan_kernelILi2ELi4ELi2E\S*:", asm.read_text(), maxsplit=1, flags=re.M)[1].split("s_endpgm")[0].split("v_mfma")[0]
+    between = code.split("global_load_dword ")   # the operands are loaded sixteen bytes at a time, P alone by single numbers
+    assert max(len(run) for run in "".join("w" if "s_waitcnt" in x else "l" for x in between[1:-1]).split("w")) >= 15
+
+
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
 @pytest.mark.parametrize("experts,N,K,glu,by_pairs", [   # measured: whether the kernel for few rows per tile is the faster one
     (16, 1024, 2048, False, {2: True, 16: True, 64: True}), (16, 2048, 1024, False, {2: True, 12: True, 64: False}),
