@@ -397,11 +397,13 @@ class KernelOps:
             while -(-span // part) > 32 or groups * -(-span // part) > 1024 and part < span:
                 part *= 2
         nparts = max(1, -(-span // part))
-        # Two launches where a compute unit would prepare several workgroups' rows one behind the other: its registers hold one workgroup of 128
-        # dims at a time, two of fp32 without the preparation. us, one launch / two, 8 key heads: fp32, 48 and 64 rows of 70 keys 20.1 / 16.1, 21.7 /
-        # 17.4, of 900 keys 86.5 / 85.3, 119 / 96.5, 8 rows in runs 26.2 / 24.0, 32 rows (256 workgroups) 51.9 / 62.6; bf16, 48 and 64 rows of 70
-        # keys 10.2 / 11.3, 10.6 / 11.7, 48 of 300 22.4 / 21.2, of 900 50.2 / 48.7; 32 key heads, 64 rows of 300 88.6 / 84.6.
-        if prep is not None and sp.dim == 128 and (groups * nparts > 256 if proj.dtype == torch.float32 else groups > 256 and span > 256):
+        # Two launches in fp32 of 128 dims, whose registers hold one workgroup per compute unit (two without the preparation), where the compute
+        # units take several: few keys each, or many key heads and rounds that two at a time halve. us, one launch / two, 8 key heads: 48 and 64
+        # rows of 70 keys 20.1 / 16.1, 21.7 / 17.4, of 900 keys 86.5 / 85.3, 119 / 96.5, 8 rows in runs of 128 26.2 / 24.0; but 32 rows (256
+        # workgroups) 51.9 / 62.6, 96 rows (768) 158 / 169, with 4 key heads 128 and 192 rows 92.6 / 92.4, 137 / 159. bf16 holds one either way.
+        wgs = groups * nparts
+        if prep is not None and proj.dtype == torch.float32 and sp.dim == 128 and wgs > 256 and (
+                min(part, span) <= 128 or sp.kv_heads >= 8 and (wgs - 1) % 512 >= 256):
             return False
         ws_acc = ws_ml = None
         if nparts > 1:

@@ -149,10 +149,13 @@ def test_rules_of_a_few_rows_are_asked_once_per_size():
     assert seen > 0 and len(asked) == seen
 
 
-@pytest.mark.parametrize("dtype,kv,dim,n,keys,one", [
-    (torch.float32, 8, 128, 32, 70, True), (torch.float32, 8, 128, 33, 70, False), (torch.float32, 8, 128, 4, 900, True), (torch.float32, 8, 128, 5, 900, False),
-    (torch.float32, 8, 64, 64, 900, True), (torch.bfloat16, 8, 128, 32, 900, True), (torch.bfloat16, 8, 128, 33, 257, False), (torch.bfloat16, 8, 128, 64, 256, True)])
-def test_window_step_in_one_launch_by_its_workgroups(dtype, kv, dim, n, keys, one):
+@pytest.mark.parametrize("dtype,kv,dim,n,keys,normed,one", [
+    (torch.float32, 8, 128, 32, 70, True, True), (torch.float32, 8, 128, 33, 70, False, False), (torch.float32, 8, 128, 4, 900, False, True),
+    (torch.float32, 8, 128, 5, 900, False, False), (torch.float32, 8, 128, 33, 900, True, False), (torch.float32, 8, 128, 64, 900, False, False),
+    (torch.float32, 8, 128, 65, 900, True, True), (torch.float32, 4, 128, 128, 900, True, True), (torch.float32, 4, 128, 128, 128, True, False),
+    (torch.float32, 4, 128, 128, 129, True, True), (torch.float32, 8, 64, 64, 900, True, True), (torch.bfloat16, 8, 128, 64, 70, True, True),
+    (torch.bfloat16, 8, 128, 64, 900, True, True)])
+def test_window_step_in_one_launch_by_its_workgroups(dtype, kv, dim, n, keys, normed, one):
     """A decode step's preparation is a launch of its own where a compute unit would take several workgroups with it in turn."""
     from types import SimpleNamespace
 
@@ -160,11 +163,11 @@ def test_window_step_in_one_launch_by_its_workgroups(dtype, kv, dim, n, keys, on
     ops, ran = KernelOps(), []
     ops._lib_ops = {"delta": SimpleNamespace(window_attention_decode_ok=lambda *a: True, window_attention_step=lambda *a: ran.append(a))}
     sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=4 * kv, kv_heads=kv, window=1024, reach=1024, scale=1.0, sink=False, keep_first=0, softcap=0.0,
-                         channel_gate=False, chunk=0, kv_from=None, qk_norm=False, head_norm=False, unit_qk=False, v_norm=False, scaling=None, temp_coef=0.0,
+                         channel_gate=False, chunk=0, kv_from=None, qk_norm=normed, head_norm=False, unit_qk=False, v_norm=False, scaling=None, temp_coef=0.0,
                          temp_every=0)
     meta = SimpleNamespace(max_q=1, num_prefill_tokens=0, num_decode=n, seq_ctx=torch.zeros(n), seq_cu=None, seq_bt=None, positions=None, slot_mapping=None, max_ctx=keys)
-    proj = torch.zeros(n, 8, dtype=dtype)
-    assert ops.window_step(torch.zeros_like(proj), proj, proj, meta, torch.zeros(dim // 2), sp, None, None, 1e-6, -1) == one and len(ran) == one
+    proj, norm_w = torch.zeros(n, 8, dtype=dtype), torch.zeros(4) if normed else None
+    assert ops.window_step(torch.zeros_like(proj), proj, proj, meta, torch.zeros(dim // 2), sp, *(2 * [norm_w]), 1e-6, -1) == one and len(ran) == one
 
 
 @pytest.mark.parametrize("dtype,rank,most", [(torch.bfloat16, 64, 64), (torch.bfloat16, 128, 32), (torch.float32, 64, 32), (torch.float32, 128, 8)])
