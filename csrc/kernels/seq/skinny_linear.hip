@@ -204,11 +204,12 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
          : xg <= 6 ? HS_SK(6, 2, 1, true) : HS_SK(8, 2, 1, true);
   const long tiles = ((long)N * batch + 15) / 16 * parts;
   const int nt = skinny_tiles(M, tiles, K / parts);
-  // One piece ahead: two are faster (up to 40 %) where a wave waits for its few copies, up to 16 rows and more than a piece per wave, and slower
+  // One piece ahead: two are faster (up to 40 %) where a wave waits for its few copies, up to 16 rows and more than a piece per wave (more than
+  // two where a compute unit holds several workgroups: 12288 x 1024, 16 rows 9 % slower; 3072 x 1024, one row 4 % faster), and slower
   // where they leave room for fewer workgroups (33 - 64 rows, 16384 x 256: 19 -> 13 us; 32 heads of 512 x 128, one row 4.1 -> 3.4).
   if (nt == 4) return xg <= 4 ? HS_SK(4, 4, 1, false) : xg <= 6 ? HS_SK(6, 4, 1, false) : HS_SK(8, 4, 1, false);
   if (nt == 2) return xg <= 2 ? HS_SK(2, 2, 1, false) : xg <= 4 ? HS_SK(4, 2, 1, false) : xg <= 6 ? HS_SK(6, 2, 1, false) : HS_SK(8, 2, 1, false);
-  const bool ahead = xg <= 2 && K / parts > 1024 && !(xg == 1 && tiles > 256 && tiles <= 512);
+  const bool ahead = xg <= 2 && K / parts > (tiles <= 256 ? 512 : 1024) && !(xg == 1 && tiles > 256 && tiles <= 512);
   if (ahead) return xg <= 1 ? HS_SK(1, 1, 2, false) : HS_SK(2, 1, 2, false);
   return xg <= 1 ? HS_SK(1, 1, 1, false) : xg <= 2 ? HS_SK(2, 1, 1, false) : xg <= 3 ? HS_SK(3, 1, 1, false)
        : xg <= 4 ? HS_SK(4, 1, 1, false) : xg <= 6 ? HS_SK(6, 1, 1, false) : HS_SK(8, 1, 1, false);
