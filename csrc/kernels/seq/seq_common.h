@@ -10,6 +10,16 @@ template <typename T> HS_DEVICE void stf(T* p, long i, float v);
 template <> HS_DEVICE void stf<unsigned short>(unsigned short* p, long i, float v) { p[i] = f32_to_bf16(v); }
 template <> HS_DEVICE void stf<float>(float* p, long i, float v) { p[i] = v; }
 
+// Kernel arguments from byte `at` of the argument block on, loaded where this stands and not before: the compiler loads arguments
+// at the kernel's entry and waits for them there, which takes 0.26 us of a small launch (a second, dependent load of them 0.34). The ones that the first loads need come first and reach
+// the kernel in scalar registers (the build's flags ask for it).
+template <typename T> using LateArgs = const __attribute__((address_space(4))) T*;
+template <typename T> HS_DEVICE LateArgs<T> late_args(int at) {
+  unsigned long p = reinterpret_cast<unsigned long>(__builtin_amdgcn_kernarg_segment_ptr()) + at;
+  asm volatile("" : "+s"(p));
+  return reinterpret_cast<LateArgs<T>>(p);
+}
+
 // V consecutive elements of a row as fp32 (V > 1: the address is aligned to V elements)
 template <typename T, int V> struct Row;
 template <> struct Row<float, 1> {

@@ -26,7 +26,7 @@
 
 namespace hipserve {
 
-constexpr int kSkWaves = 8, kSkThreads = 64 * kSkWaves, kSkLd = 20;   // kSkLd: row stride of the sums in LDS (floats)
+constexpr int kSkWaves = 8 /* 1 << 3 */, kSkThreads = 64 * kSkWaves, kSkLd = 20;   // kSkLd: row stride of the sums in LDS (floats)
 
 template <int N> HS_DEVICE void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
@@ -53,7 +53,7 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
     const int c = lane & 15, g = lane >> 4, r8 = lane >> 3;
     unsigned char* ring = smem + wave * DEPTH * kPiece;
     const unsigned lds0 = lds_at(ring);
-    const int pieces = (K + 63) / 64, n = (pieces - wave + kSkWaves - 1) / kSkWaves;   // this wave's: wave, wave + 8, ...
+    const int pieces = (K + 63) >> 6, n = (pieces - wave + kSkWaves - 1) >> 3;   // this wave's: wave, wave + 8, ...
     // the lane's bytes past the piece's first k of the first row: full pieces differ by uniform numbers
     unsigned w_at[2 * NT], x_at[XG];
 #pragma unroll

@@ -29,122 +29,186 @@ HS_DEVICE float skinny_act(float z, int act, float c0, float c1) {
   return z;
 }
 
+enum { kPlain, kNormed, kUpdate };   // SkinnyNorm: none; rows without their norm's factor; a result that goes into the residual stream
 struct NoNorm {};
+// The kernel's arguments: the parameters are what its first loads need, the rest is loaded once the copies are on their way (seq_common.h), and
+// nothing is asked for after the product any more. us of four products in a captured loop (square, 3 x wider, back, 1.5 x wider), cold weights,
+// 1 and 16 rows: width 1024 15.1 -> 13.6, 17.4 -> 16.0, width 2048 24.4 -> 22.8, 29.4 -> 27.8.
+template <int NORM> struct SkinnyRest {
+  long x_bs, out_ld, out_bs, out_zs;
+  int act, act_from;
+  float c0, c1, cols, eps;
+  void* out;
+  float* squares;      // kUpdate
+  const void* bias;
+};
+template <int NORM> struct SkinnyArgs {
+  const void *x, *w, *p, *q;
+  int x_ld, M, N, K, i;
+  SkinnyRest<NORM> rest;
+};
 
 // XG: groups of 8 rows; NT: 16-column tiles (GLU: the gate's and the up projection's of the same 16 output columns).
 // F32: 32-bit operands, x, w, their strides and K in 16-bit halves (skinny.h). Workgroups z take `part` of K each (a multiple of 64) and write
 // their sums out_zs elements apart (the bias in the first).
-// NORM: the rows come without their norm's factor, or the result goes into the residual stream (SkinnyNorm; K in one part).
-template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, bool NORM>
+// p, q, i: kPlain - , bias, part; kNormed squares, bias, blocks; kUpdate residual, weight, blocks (K in one part for both).
+template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM>
 __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
-    TO* __restrict__ out, long out_ld, long out_bs, long out_zs, const unsigned short* __restrict__ x, long x_ld, long x_bs,
-    const unsigned short* __restrict__ w, const void* __restrict__ bias_, int M, int N, int K, int part, int act, int act_from, float c0, float c1,
-    std::conditional_t<NORM, SkinnyNorm, NoNorm> norm) {
+    const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, void* p, const void* q, int x_ld, int M, int N, int K, int ni,
+    const SkinnyRest<NORM>) {
   static_assert(!GLU || NT == 2, "a gate tile and an up tile");
   using SK = Skinny<XG, NT, DEPTH, F32>;
   constexpr int ST = SK::ST;
   using TB = std::conditional_t<F32, float, unsigned short>;
-  const TB* bias = blockIdx.z == 0 ? static_cast<const TB*>(bias_) : nullptr;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int No = GLU ? N / 2 : N;
   const int n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
-  const int k0 = blockIdx.z * part, k1 = min(K, k0 + part);   // (no division here: it showed in the one-row times)
-  x += (long)blockIdx.y * x_bs + k0;
-  w += (long)blockIdx.y * N * K + k0;
-  out += (long)blockIdx.z * out_zs;
+  const int k0 = NORM == kPlain ? blockIdx.z * ni : 0, k1 = NORM == kPlain ? min(K, k0 + ni) : K;
+  const int rest_at = offsetof(SkinnyArgs<NORM>, rest);
+  if (NORM == kPlain && blockIdx.y != 0) {
+    x += (long)blockIdx.y * late_args<SkinnyRest<NORM>>(rest_at)->x_bs;
+    w += (long)blockIdx.y * N * K;
+  }
   const unsigned char* wt[NT];
   unsigned w_row[2 * NT];
   unsigned x_row[XG];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int first = GLU ? n0 : min(n0 + 16 * nt, N - 1);   // of the tile's columns
-    wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)(GLU ? nt * No : 0) + first) * K);
+    wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)(GLU ? nt * No : 0) + first) * K + k0);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)(min(first + 8 * h + (lane >> 3), No - 1) - first) * (unsigned)K * 2;
+    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), No - 1 - first) * (unsigned)(2 * K);
   }
 #pragma unroll
-  for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)x_ld * 2;
+  for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)(2 * x_ld);
   f32x4 acc[NT][ST];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
   constexpr int IT = (ST + 1) / 2, SQ = 4;   // 16 threads x SQ loads x 4 sums of 16 columns each: rows of up to 4096
-  f32x4 sq[IT][SQ];
-  float res[IT][NT];
-  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, k1 - k0, smem, lane, wave, [&] {
-    if constexpr (NORM) {   // used in the epilogue
+  [[maybe_unused]] f32x4 sq[IT][SQ];
+  [[maybe_unused]] float res[IT][NT], wgt[NT];
+  [[maybe_unused]] TB bs[NT];
+  // for the epilogue, ahead of the copies: without branches, behind which the copies would be waited for, and first, since loads return in
+  // order and a wait for the copies would be one for these too
+  const int c = tid & 15;
+  const bool biased = NORM != kUpdate && q != nullptr && blockIdx.z == 0;
+  const TB* bias = static_cast<const TB*>(biased ? q : x);
 #pragma unroll
-      for (int i = 0; i < IT; ++i) {
-        const int m = (tid + kSkThreads * i) >> 4, c = tid & 15;
+  for (int i = 0; i < IT; ++i) {
+    [[maybe_unused]] const long m = min((tid + kSkThreads * i) >> 4, M - 1);
+    if constexpr (NORM == kNormed) {
 #pragma unroll
-        for (int j = 0; j < SQ; ++j) {
-          sq[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-          if (norm.residual == nullptr && m < M && 64 * j + 4 * c < norm.blocks)
-            sq[i][j] = *reinterpret_cast<f32x4*>(norm.squares + (long)m * norm.blocks + 64 * j + 4 * c);
-        }
+      for (int j = 0; j < SQ; ++j) sq[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p) + m * ni + min(64 * j + 4 * c, ni - 4));
+    }
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-          res[i][nt] = norm.residual != nullptr && m < M ? norm.residual[(long)m * N + n0 + 16 * nt + c] : 0.f;
+    for (int nt = 0; nt < NT; ++nt) {
+      const int n = (GLU ? nt * No : 0) + min(n0 + (GLU ? 0 : 16 * nt) + c, No - 1);
+      if constexpr (NORM == kUpdate) res[i][nt] = static_cast<const float*>(p)[m * N + n];
+      if (i == 0) {
+        if constexpr (NORM == kUpdate) wgt[nt] = static_cast<const float*>(q)[n];
+        else bs[nt] = bias[biased ? n : 0];
+      }
+    }
+  }
+  int act = 0, act_from = 0;
+  float c0 = 0.f, c1 = 0.f, cols = 1.f, eps = 0.f;
+  long out_ld = 0;
+  TO* out = nullptr;
+  [[maybe_unused]] float* squares = nullptr;
+  [[maybe_unused]] const TB* late_bias = nullptr;
+  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x + k0), x_row, k1 - k0, smem, lane, wave, [&] {
+    const auto rest = late_args<SkinnyRest<NORM>>(rest_at);
+    out = static_cast<TO*>(rest->out);
+    out_ld = NORM == kPlain ? rest->out_ld : GLU ? No : N;
+    if constexpr (NORM == kPlain) out += (long)blockIdx.y * rest->out_bs + (long)blockIdx.z * rest->out_zs;
+    if constexpr (NORM == kUpdate) squares = rest->squares;
+    act = rest->act;
+    act_from = rest->act_from;
+    c0 = rest->c0;
+    c1 = rest->c1;
+    cols = rest->cols;
+    eps = rest->eps;
+    asm volatile("" ::"s"(act), "s"(act_from), "s"(c0), "s"(c1), "s"(cols), "s"(eps), "s"(out), "s"(out_ld), "s"(squares));
+    if constexpr (NORM == kUpdate) {
+      late_bias = static_cast<const TB*>(rest->bias);
+      if (late_bias != nullptr) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) bs[nt] = late_bias[n0 + 16 * nt + c];
       }
     }
   });
   float v[NT][IT];
   SK::reduce(v, acc, smem);
-  out += (long)blockIdx.y * out_bs;
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
     const int e = tid + kSkThreads * i, m = e >> 4;
     if (m >= M) continue;   // a row's 16 lanes together
-    if constexpr (NORM) {
-      if (norm.residual != nullptr) {   // N is a multiple of the workgroup's columns
+    if constexpr (NORM == kUpdate) {   // N is a multiple of the workgroup's columns
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          const int n = n0 + 16 * nt + (e & 15);
-          const float r = res[i][nt] + (v[nt][i] + (bias != nullptr ? ldf<TB>(bias, n) : 0.f));
-          norm.residual[(long)m * N + n] = r;
-          stf<TO>(out, m * out_ld + n, r * norm.weight[n]);
-          const float s = row_sum(r * r);
-          if ((e & 15) == 0) norm.squares[(long)m * norm.blocks + (n >> 4)] = s;
-        }
-        continue;
+      for (int nt = 0; nt < NT; ++nt) {
+        const int n = n0 + 16 * nt + (e & 15);
+        const float r = res[i][nt] + (v[nt][i] + (late_bias != nullptr ? ldf<TB>(&bs[nt], 0) : 0.f));
+        static_cast<float*>(p)[(long)m * N + n] = r;
+        stf<TO>(out, m * out_ld + n, r * wgt[nt]);
+        const float s = row_sum(r * r);
+        if ((e & 15) == 0) squares[(long)m * ni + (n >> 4)] = s;
       }
+      continue;
+    }
+    if constexpr (NORM == kNormed) {
       float s = 0.f;
 #pragma unroll
-      for (int j = 0; j < SQ; ++j) s += (sq[i][j][0] + sq[i][j][1]) + (sq[i][j][2] + sq[i][j][3]);
-      const float inv = 1.f / sqrtf(row_sum(s) / norm.cols + norm.eps);
+      for (int j = 0; j < SQ; ++j)
+        if (64 * j + 4 * c < ni) s += (sq[i][j][0] + sq[i][j][1]) + (sq[i][j][2] + sq[i][j][3]);
+      const float inv = 1.f / sqrtf(row_sum(s) / cols + eps);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) v[nt][i] *= inv;
     }
     if constexpr (GLU) {
       const int n = n0 + (e & 15);
       if (n >= No) continue;
-      const float gv = v[0][i] + (bias != nullptr ? ldf<TB>(bias, n) : 0.f);
-      const float uv = v[1][i] + (bias != nullptr ? ldf<TB>(bias, No + n) : 0.f);
+      const float gv = v[0][i] + (biased ? ldf<TB>(&bs[0], 0) : 0.f);
+      const float uv = v[1][i] + (biased ? ldf<TB>(&bs[1], 0) : 0.f);
       stf<TO>(out, m * out_ld + n, act == 4 ? clamped_glu_f(gv, uv, c0) : gv * sigmoid_f(gv) * uv);
     } else {
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const int n = n0 + 16 * nt + (e & 15);
         if (n >= N) continue;
-        const float z = v[nt][i] + (bias != nullptr ? ldf<TB>(bias, n) : 0.f);
+        const float z = v[nt][i] + (biased ? ldf<TB>(&bs[nt], 0) : 0.f);
         stf<TO>(out, m * out_ld + n, skinny_act(z, n >= act_from ? act : -1, c0, c1));
       }
     }
   }
 }
 
-template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, bool NORM = false>
+template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM = kPlain>
 bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, long out_zs, const void* x, long x_ld, long x_bs, const void* w, const void* bias,
                    int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s,
-                   const std::conditional_t<NORM, SkinnyNorm, NoNorm>& norm = {}) {
+                   const std::conditional_t<NORM != kPlain, SkinnyNorm, NoNorm>& norm = {}) {
   constexpr int lds = Skinny<XG, NT, DEPTH, F32>::kLds;
   static const bool ok = allow_lds(&skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM>, lds);
   if (!ok) return false;
-  skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM><<<grid, kSkThreads, lds, s>>>(
-      (TO*)out, out_ld, out_bs, out_zs, (const unsigned short*)x, x_ld, x_bs, (const unsigned short*)w, bias, M, N, K, ((K + 63) / 64 + (int)grid.z - 1) / (int)grid.z * 64, act,
-      act_from, c0, c1, norm);
+  SkinnyRest<NORM> rest{x_bs, out_ld, out_bs, out_zs, act, act_from, c0, c1, 1.f, 0.f, out, nullptr, bias};
+  void* p = nullptr;
+  const void* q = bias;
+  int i = ((K + 63) / 64 + (int)grid.z - 1) / (int)grid.z * 64;
+  if constexpr (NORM != kPlain) {
+    rest.cols = norm.cols;
+    rest.eps = norm.eps;
+    i = norm.blocks;
+    p = norm.squares;
+    if constexpr (NORM == kUpdate) {
+      p = norm.residual;
+      q = norm.weight;
+      rest.squares = norm.squares;
+    }
+  }
+  skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM><<<grid, kSkThreads, lds, s>>>((const unsigned short*)x, (const unsigned short*)w, p, q,
+                                                                                        (int)x_ld, M, N, K, i, rest);
   return true;
 }
 
@@ -216,27 +280,36 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
 #undef HS_SK
 }
 
-bool launch_skinny_linear_normed(void* out, bool out_f32, const SkinnyNorm& norm, const void* x, long x_ld, const void* w, const void* bias,
-                                 bool f32, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
-  if (M <= 0 || N <= 0) return true;
+template <int NORM>
+static bool launch_normed(void* out, bool out_f32, const SkinnyNorm& norm, const void* x, long x_ld, const void* w, const void* bias,
+                          bool f32, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
   if (f32) { x_ld *= 2; K *= 2; }   // in halves
   const bool glu = act == 3 || act == 4;
   const long No = glu ? N / 2 : N;
 #define HS_SN(XG, NT, DEPTH, GLU, TO, F32)                                                                                                    \
-  launch_kernel<XG, NT, DEPTH, GLU, TO, F32, true>(dim3((No + (GLU ? 16 : 16 * NT) - 1) / (GLU ? 16 : 16 * NT)), out, No, 0, 0, x, x_ld, 0, w,  \
+  launch_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM>(dim3((No + (GLU ? 16 : 16 * NT) - 1) / (GLU ? 16 : 16 * NT)), out, No, 0, 0, x, x_ld, 0, w,  \
                                                    bias, M, N, K, act, act_from, c0, c1, s, norm)
 #define HS_SX(NT, D, GLU, TO, F32) (M <= 8 ? HS_SN(1, NT, D, GLU, TO, F32) : M <= 16 ? HS_SN(2, NT, D, GLU, TO, F32) : HS_SN(4, NT, F32 ? 1 : D, GLU, TO, F32))
-#define HS_ST(NT, D, GLU) (f32 ? HS_SX(NT, D, GLU, float, true) : out_f32 ? HS_SX(NT, D, GLU, float, false) : HS_SX(NT, D, GLU, unsigned short, false))
-#define HS_S4() (f32 ? HS_SN(4, 4, 1, false, float, true) : out_f32 ? HS_SN(4, 4, 1, false, float, false) : HS_SN(4, 4, 1, false, unsigned short, false))
+  using Wide = std::conditional_t<NORM == kNormed, float, unsigned short>;   // an update writes rows of the operands' type
+#define HS_ST(NT, D, GLU) (f32 ? HS_SX(NT, D, GLU, float, true) : out_f32 ? HS_SX(NT, D, GLU, Wide, false) : HS_SX(NT, D, GLU, unsigned short, false))
+#define HS_S4() (f32 ? HS_SN(4, 4, 1, false, float, true) : out_f32 ? HS_SN(4, 4, 1, false, Wide, false) : HS_SN(4, 4, 1, false, unsigned short, false))
   // Two pieces ahead for one tile, but for more than 16 rows of 32 bits: a decode step of 20 rows (width 1024) 122.4 us with two, 124.2 with
   // one, in 32 bits 167.1 and 166.0, of 32 rows 128.4 and 130.0, 173.7 and 170.0.
-  if (glu) return HS_ST(2, 1, true);
+  if constexpr (NORM == kNormed)
+    if (glu) return HS_ST(2, 1, true);
   const int nt = skinny_tiles(M, (N + 15) / 16, K);   // 4 above 16 rows alone; where squares are written, N is a multiple of 64
   return nt == 4 ? HS_S4() : nt == 2 ? HS_ST(2, 1, false) : HS_ST(1, 2, false);
 #undef HS_S4
 #undef HS_ST
 #undef HS_SX
 #undef HS_SN
+}
+
+bool launch_skinny_linear_normed(void* out, bool out_f32, const SkinnyNorm& norm, const void* x, long x_ld, const void* w, const void* bias,
+                                 bool f32, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
+  if (M <= 0 || N <= 0) return true;
+  auto go = norm.residual != nullptr ? launch_normed<kUpdate> : launch_normed<kNormed>;
+  return go(out, out_f32, norm, x, x_ld, w, bias, f32, M, N, K, act, act_from, c0, c1, s);
 }
 
 }  // namespace hipserve

@@ -35,6 +35,8 @@ HIP_FLAGS = [
     "-Wno-unused-variable",
     # no packed-fp32 instructions from ordinary float code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # the first 14 words of a kernel's arguments in scalar registers when it starts (whole parameters; a struct and what follows it are loaded)
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
 
 # kernel libraries: name -> (shared object, kernel sources, host bindings). "core" is every
