@@ -216,6 +216,7 @@ struct WindowPrep {
   int nfreq, norm_mode, temp_every;
   float eps, amp, temp_coef;
   bool own_kv, v_norm;
+  int rows;   // of the batch
 };
 bool window_attention_decode_ok(int dim, int vdim, int block_size, bool f32);
 void launch_window_attention_decode(void* out, long out_ld, const void* proj, long proj_ld, const void* cache, int block_size,

@@ -212,7 +212,7 @@ inline void window_attention_step(at::Tensor& out, const at::Tensor& proj, at::T
     }
   const hipserve::WindowPrep prep{cache.data_ptr(), positions.data_ptr<long>(), slots.data_ptr<long>(), inv_freq.data_ptr<float>(),
                                   (const float*)opt_ptr(q_norm), own_kv ? (const float*)opt_ptr(k_norm) : nullptr, (int)inv_freq.numel(),
-                                  (int)norm_mode, (int)temp_every, (float)eps, (float)amp, (float)temp_coef, own_kv, v_norm};
+                                  (int)norm_mode, (int)temp_every, (float)eps, (float)amp, (float)temp_coef, own_kv, v_norm, (int)T};
   window_decode(out, proj, cache, seq_cu, seq_ctx, seq_bt, 0, 0, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale,
                 nparts, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, &prep);
 }

@@ -59,17 +59,19 @@ using u32x4 = __attribute__((ext_vector_type(4))) unsigned;
 
 struct NoPrep {};
 
-// 8 elements of a row as they lie in memory.
-template <typename T> struct Raw8 {
-  u32x4 w[sizeof(T) / 2];
+// N elements of a row as they lie in memory (4 or 8).
+template <typename T, int N> struct Raw {
+  using V = __attribute__((ext_vector_type(N * sizeof(T) >= 16 ? 4 : 2))) unsigned;
+  static constexpr int PER = sizeof(V) / sizeof(T);
+  V w[N / PER];
   HS_DEVICE void ld(const T* p) {
 #pragma unroll
-    for (unsigned i = 0; i < sizeof(T) / 2; ++i) w[i] = reinterpret_cast<const u32x4*>(p)[i];
+    for (int i = 0; i < N / PER; ++i) w[i] = reinterpret_cast<const V*>(p)[i];
   }
   HS_DEVICE void get(float* f) const {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const unsigned u = sizeof(T) == 4 ? w[e / 4 % (sizeof(T) / 2)][e % 4] : (e & 1) ? w[0][e / 2] & 0xffff0000u : w[0][e / 2] << 16;
+    for (int e = 0; e < N; ++e) {
+      const unsigned u = sizeof(T) == 4 ? w[e / PER][e % PER] : (e & 1) ? w[0][e / 2] & 0xffff0000u : w[0][e / 2 % 4] << 16;
       f[e] = __builtin_bit_cast(float, u);
     }
   }
@@ -77,84 +79,104 @@ template <typename T> struct Raw8 {
 
 // attn_prepare_vec_kernel's work for one workgroup of a decode step: its query heads, and the new key and value of their
 // key / value head, from the projection row into LDS (`heads` [nh][D], then key [D], value [D]), the latter two into the cache
-// row as well where `keep_row` says so. What is normed over the whole projection is summed by every workgroup of the row: 5 KB
-// for 16 + 4 heads of 128 in bf16, while the keys' addresses are on their way. `rows` asks for the first tile's places, `early` for the tile.
-template <typename T, int D, typename F, typename G>
-HS_DEVICE void prepare_row(const WindowPrep& pr, const T* __restrict__ row, long at, long slot, int head0, int nh, int kvh, int heads,
-                           int kv_heads, bool keep_row, T* hs, float* angles, F&& rows, G&& early) {
+// row as well where `keep_row` says so. What is normed over the whole projection (MODE 1) is summed by every workgroup of the row: 5 KB
+// for 16 + 4 heads of 128 in bf16, while the keys' addresses are on their way. `places` asks for the first tile's places, `early` for the tile.
+// Loads return in order and nothing here branches between them: the angles' frequencies, the places, the row, then, once the places are there,
+// the tile, which is on its way while the row is worked on. MODE: WindowPrep's norm_mode, 0 for 3 too.
+template <typename T, int D, int MODE, typename F, typename G>
+HS_DEVICE void prepare_row(const WindowPrep& pr, int waves, const T* __restrict__ row, long at, long slot, int head0, int nh, int kvh, int heads,
+                           int kv_heads, bool keep_row, T* hs, float* angles, F&& places, G&& early) {
   __shared__ float red[2][8];
-  constexpr int PER = D / 16, NS = sizeof(T) == 4 ? 4 : 8;   // NS: loads of the sums in flight beside the tile's, within the registers
-  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wave = tid >> 6;
-  const int nq = heads * D, nk = pr.own_kv ? kv_heads * D : 0, rot = pr.nfreq / 8, items = (nh + (pr.own_kv ? 2 : 0)) * PER;
-  const int chunks = pr.norm_mode == 1 ? (nq + nk) / 8 : 0;
+  constexpr int PER = D / 8, NS = sizeof(T) == 4 ? 4 : 8;   // NS: loads of the sums in flight beside the tile's, within the registers
+  const int tid = threadIdx.x, nt = 64 * waves, lane = tid & 63, wave = tid >> 6;
+  const int nq = heads * D, nk = pr.own_kv ? kv_heads * D : 0, rot = pr.nfreq / 4, items = (nh + (pr.own_kv ? 2 : 0)) * PER;
+  const int chunks = (nq + nk) / 8;
   int o0 = 0, o1 = 0;
-  auto place = [&](int it) {   // of an item: two 8-dim chunks of a head, as rotated pairs have them
+  auto place = [&](int it) {   // of an item: two 4-dim chunks of a head, as rotated pairs have them
     const int h = it / PER, j = it % PER;
     const bool pair = j < rot && h <= nh;
-    o0 = pair ? 8 * j : h <= nh ? 2 * pr.nfreq + 16 * (j - rot) : 16 * j;
-    o1 = o0 + (pair ? pr.nfreq : 8);
+    o0 = pair ? 4 * j : h <= nh ? 2 * pr.nfreq + 8 * (j - rot) : 8 * j;
+    o1 = o0 + (pair ? pr.nfreq : 4);
     return row + (h < nh ? (head0 + h) * D : h == nh ? nq + kvh * D : nq + nk + kvh * D);
   };
-  Raw8<T> lo{}, hi{}, sum[NS];
-  if (tid < items) {
-    const T* src = place(tid);
+  Raw<T, 4> lo{}, hi{};
+  Raw<T, 8> sum[NS];
+  f32x4 wl, wh;
+  using Weights = const __attribute__((address_space(1))) f32x4*;
+  using Weight = const __attribute__((address_space(1))) float*;
+  auto qn = reinterpret_cast<Weight>(reinterpret_cast<unsigned long>(pr.q_norm));
+  auto kn = reinterpret_cast<Weight>(reinterpret_cast<unsigned long>(pr.own_kv ? pr.k_norm : pr.q_norm));
+  if constexpr (MODE != 0) asm volatile("" : "+s"(qn), "+s"(kn));   // two pointers to choose from, not a place in the arguments
+  auto weights = [&](int it) {   // place(it) is the last one; the new value has none, and takes any
+    const int h = it / PER;
+    const auto w = (h < nh ? qn : kn) + (MODE == 2 ? 0 : h < nh ? (head0 + h) * D : kvh * D);
+    wl = *reinterpret_cast<Weights>(w + o0);
+    wh = *reinterpret_cast<Weights>(w + o1);
+  };
+  const float freq = *(pr.nfreq > 0 ? pr.inv_freq + min(lane, pr.nfreq - 1) : reinterpret_cast<const float*>(row));
+  places();
+  {
+    const int it = min(tid, items - 1);
+    const T* src = place(it);
     lo.ld(src + o0);
     hi.ld(src + o1);
+    if constexpr (MODE != 0) weights(it);
   }
+  if constexpr (MODE == 1) {
 #pragma unroll
-  for (int b = 0; b < NS; ++b)
-    if (b * nt < chunks) sum[b].ld(row + 8L * min(tid + b * nt, chunks - 1));
-  // Loads return in order, and a wait behind a branch is for all of them: what the preparation needs stands before the tile, and has
-  // landed when the tile's loads are issued (their addresses come from the block table, asked for at the same time).
-  auto landed = [] { __builtin_amdgcn_s_waitcnt(0x0f70); };   // vmcnt(0)
-  const bool weighed = pr.norm_mode == 1 || pr.norm_mode == 2;
-  float wl[8], wh[8];
-  auto weights = [&](int it) {   // place(it) is the last one
-    const int h = it / PER;
-    const float* w = (h < nh ? pr.q_norm : pr.k_norm) + (pr.norm_mode == 2 ? 0 : h < nh ? (head0 + h) * D : kvh * D);
-    Row<float, 8>::ld(w + o0, wl);
-    Row<float, 8>::ld(w + o1, wh);
-  };
-  if (weighed && tid < items && tid / PER <= nh) weights(tid);
-  const float freq = tid < pr.nfreq ? pr.inv_freq[tid] : 0.f;
-  rows();
-  landed();
-  float a = 0.f, b = 0.f;
-  for (int i0 = 0; i0 < chunks; i0 += NS * nt) {
-    if (i0 > 0) {
-#pragma unroll
-      for (int n = 0; n < NS; ++n)
-        if (i0 + n * nt < chunks) sum[n].ld(row + 8L * min(tid + i0 + n * nt, chunks - 1));
-      landed();
-    }
-#pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      const int i = tid + i0 + n * nt;
-      if (i0 + n * nt >= chunks || i >= chunks) continue;
-      float x[8], v[4] = {};
-      sum[n].get(x);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e & 3] += x[e] * x[e];
-      const float t = (v[0] + v[1]) + (v[2] + v[3]);
-      if (8 * i < nq) a += t; else b += t;
-    }
+    for (int b = 0; b < NS; ++b) sum[b].ld(row + 8L * min(tid + b * nt, chunks - 1));
   }
-  early();   // nothing that was asked for before is waited for behind this
-  const float pos = (float)at;
-  if (tid < pr.nfreq) {   // at most 64 frequencies, at least 64 threads
+  early();
+  if (tid >= nt - 64 && lane < pr.nfreq) {   // at most 64 frequencies, by the last wave, which has the fewest items
     float sn, cs;
-    sincosf(pos * freq, &sn, &cs);
-    angles[tid] = cs * pr.amp;
-    angles[pr.nfreq + tid] = sn * pr.amp;
+    sincosf((float)at * freq, &sn, &cs);
+    angles[lane] = cs * pr.amp;
+    angles[pr.nfreq + lane] = sn * pr.amp;
   }
-  if (pr.norm_mode == 1) {
+  float a = 0.f, b = 0.f;
+  if constexpr (MODE == 1) {
+    auto add = [&](int i0) {
+#pragma unroll
+      for (int n = 0; n < NS; ++n) {
+        const int i = tid + i0 + n * nt;
+        float x[8], v[4] = {};
+        sum[n].get(x);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e & 3] += x[e] * x[e];
+        const float t = i < chunks ? (v[0] + v[1]) + (v[2] + v[3]) : 0.f;
+        a += 8 * i < nq ? t : 0.f;
+        b += 8 * i < nq ? 0.f : t;
+      }
+    };
+    add(0);   // apart from the others, whose loads would have this one wait for the tile
+    for (int i0 = NS * nt; i0 < chunks; i0 += NS * nt) {
+#pragma unroll
+      for (int n = 0; n < NS; ++n) sum[n].ld(row + 8L * min(tid + i0 + n * nt, chunks - 1));
+      add(i0);
+    }
     a = wave_sum(a);
     b = wave_sum(b);
     if (lane == 0) { red[0][wave] = a; red[1][wave] = b; }
   }
+  float x[4], y[4], ss = 0.f;   // an item's elements and the sum of its head's squares
+  auto take = [&](int it) {   // place(it) is the last one
+    const int h = it / PER, j = it % PER;
+    lo.get(x);
+    hi.get(y);
+    if (pr.norm_mode >= 2 || pr.v_norm) {
+      const float grow = pr.norm_mode == 3 && j < rot && h <= nh ? pr.amp : 1.f;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { const float p = x[e] * grow, q = y[e] * grow; v[e] = p * p + q * q; }
+      ss = (v[0] + v[1]) + (v[2] + v[3]);
+#pragma unroll
+      for (int o = 1; o < PER; o <<= 1) ss += __shfl_xor(ss, o, 64);
+    }
+  };
+  if ((tid & ~63) < items) take(min(tid, items - 1));   // whole waves: a head's sum is over its lanes
   __syncthreads();
   float iq = 1.f, ik = 1.f;
-  if (pr.norm_mode == 1) {
+  if constexpr (MODE == 1) {
     a = b = 0.f;
 #pragma unroll
     for (int w = 0; w < 8; ++w) {   // one wait for all of them
@@ -167,73 +189,75 @@ HS_DEVICE void prepare_row(const WindowPrep& pr, const T* __restrict__ row, long
   }
   const float temp = pr.temp_every > 0 ? 1.f + pr.temp_coef * logf((float)((at + 1) / pr.temp_every) + 1.f) : 1.f;
   T* dst = reinterpret_cast<T*>(pr.cache) + slot * (2L * kv_heads * D) + kvh * D;
-  for (int it = tid; (it & ~63) < items; it += nt) {   // whole waves: a head's sum is over its lanes
-    const bool live = it < items;
-    const T* src = place(min(it, items - 1));
-    if (it >= nt && live) {
-      lo.ld(src + o0);
-      hi.ld(src + o1);
-      if (weighed && it / PER <= nh) weights(it);
-      landed();
-    }
+  auto item = [&](int it) {
+    if (it >= items) return;
     const int h = it / PER, j = it % PER;
     const bool qk = h <= nh, isq = h < nh;
-    float x[8], y[8], v[4] = {};
-    lo.get(x);
-    hi.get(y);
-    const float grow = pr.norm_mode == 3 && j < rot && qk ? pr.amp : 1.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { const float w = x[e] * grow; v[e & 3] += w * w; }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { const float w = y[e] * grow; v[e & 3] += w * w; }
-    float f = isq ? iq : qk ? ik : 1.f, ss = (v[0] + v[1]) + (v[2] + v[3]);
-    if (pr.norm_mode >= 2 || pr.v_norm) {
-#pragma unroll
-      for (int o = 1; o < PER; o <<= 1) ss += __shfl_xor(ss, o, 64);
-      if (qk ? pr.norm_mode >= 2 : pr.v_norm) f = 1.f / sqrtf(ss / (float)D + pr.eps);
-    }
-    if (!live) continue;
+    float f = isq ? iq : qk ? ik : 1.f;
+    if (qk ? pr.norm_mode >= 2 : pr.v_norm) f = 1.f / sqrtf(ss / (float)D + pr.eps);
     if (isq) f *= temp;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { x[e] *= f; y[e] *= f; }
-    if (qk && weighed) {
+    for (int e = 0; e < 4; ++e) { x[e] *= f; y[e] *= f; }
+    if (MODE != 0 && qk) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) { x[e] *= wl[e]; y[e] *= wh[e]; }
+      for (int e = 0; e < 4; ++e) { x[e] *= wl[e]; y[e] *= wh[e]; }
     }
     if (qk && j < rot) {
-      float cs[8], sn[8];
-      Row<float, 8>::ld(angles + 8 * j, cs);
-      Row<float, 8>::ld(angles + pr.nfreq + 8 * j, sn);
+      float cs[4], sn[4];
+      Row<float, 4>::ld(angles + 4 * j, cs);
+      Row<float, 4>::ld(angles + pr.nfreq + 4 * j, sn);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < 4; ++e) {
         const float p = x[e], q = y[e];
         x[e] = p * cs[e] - q * sn[e];
         y[e] = q * cs[e] + p * sn[e];
       }
     }
-    Row<T, 8>::st(hs + h * D + o0, x);
-    Row<T, 8>::st(hs + h * D + o1, y);
+    Row<T, 4>::st(hs + h * D + o0, x);
+    Row<T, 4>::st(hs + h * D + o1, y);
     if (!isq && keep_row) {
       T* to = dst + (qk ? 0 : kv_heads * D);
-      Row<T, 8>::st(to + o0, x);
-      Row<T, 8>::st(to + o1, y);
+      Row<T, 4>::st(to + o0, x);
+      Row<T, 4>::st(to + o1, y);
     }
+  };
+  if ((tid & ~63) < items) item(tid);
+  for (int it = tid + nt; (it & ~63) < items; it += nt) {
+    const T* src = place(min(it, items - 1));
+    lo.ld(src + o0);
+    hi.ld(src + o1);
+    if constexpr (MODE != 0) weights(min(it, items - 1));
+    take(min(it, items - 1));
+    item(it);
   }
   __syncthreads();
 }
 
 // MULTI: prompt portions, tq tokens x hc heads in the 16 rows, tiles of tokens in blockIdx.x; one run.
 // PREP: the projection rows come as the product leaves them (one row per sequence), and the new key and value of a row reach its
-// own tile through LDS. Preparation and attention in captured steps, two launches -> this, in bf16 at 128 dims: one row of 8 heads over 2
-// 3.4 + 5.5 -> 7.7 us, 16 rows of 16 over 4 4.3 + 9.0 -> 11.0, 16 rows of 32 over 8 and 2000 keys 5.0 + 23.9 -> 27.6; fp32, 4 rows of 8
-// over 2 3.3 + 9.6 -> 11.6. With the tile's loads waited for before the sums 8.9, 11.4, 25.9 and 11.4.
-template <typename T, int D, bool MULTI, bool PREP = false>
+// own tile through LDS. What bounds a short step is the number of instructions that one wave issues in turn, some 5 cycles each, more than
+// memory: the scalars that places and lengths need are asked for in one batch with the arguments, a row's elements are spread over more lanes, the angles
+// are the last wave's, and the waves' results are read side by side at the end. us behind a copy of the row, before / with these, keys not in the L2:
+// one row of 8 heads over 2, 45 keys 5.9 / 5.1 (normed over the projection 6.9 / 6.2), 16 rows of 16 over 4, 230 keys 9.2 / 8.2, 16 rows of 32 over 8,
+// 1000 keys 25.9 / 23.5; fp32, 4 rows of 8 over 2, 300 keys 12.4 / 11.9.
+template <typename T, bool PREP> struct WindowRest {
+  T* out;
+  long out_ld, proj_ld;
+  const T* cache;
+  float *ws_acc, *ws_ml;
+  const float* sink_w;
+  int block_shift, seq0, seq1, tq, hc, hchunks, heads, kv_heads, group, gate_off, window, part_keys, keep, chunk, waves, nparts;
+  float scale, out_scale, softcap;
+  bool sink, channel_gate;
+  std::conditional_t<PREP, WindowPrep, NoPrep> prep;
+};
+
+// MODE: 3 without the preparation, else prepare_row's. The parameters before `rest` reach the kernel in scalar registers.
+template <typename T, int D, bool MULTI, int MODE = 3>
 __global__ __launch_bounds__(512) void window_decode_kernel(
-    T* __restrict__ out, long out_ld, const T* __restrict__ proj, long proj_ld, const T* __restrict__ cache, int block_shift,
-    const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0,
-    int seq1, int tq, int hc, int hchunks, int heads, int kv_heads, int gate_off, float scale, int window, bool sink, float out_scale,
-    int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml, int keep, float softcap,
-    const float* __restrict__ sink_w, bool channel_gate, int chunk, std::conditional_t<PREP, WindowPrep, NoPrep> prep) {
+    const T* __restrict__ proj, const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt,
+    const long* __restrict__ positions, const long* __restrict__ slots, int bt_width, int T_rows, const WindowRest<T, (MODE < 3)> rest) {
+  constexpr bool PREP = MODE < 3;
   constexpr bool F32 = sizeof(T) == 4;
   constexpr int SUB = F32 ? 1 : 2, KT = 16 * SUB;          // 16-key tiles and keys of a wave's tile
   constexpr int QN = F32 ? D / 16 : D / 32;                // 16-byte parts of a row per lane
@@ -244,12 +268,48 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
   constexpr int E = F32 || D == 64 ? 4 : 8, NB = D / (16 * E);   // dims of a value row per load; loads per row
   extern __shared__ float lds[];                           // [waves][rows][D]; [waves][16][2]
   using S = Softmax<T>;
-  int s, tok0;
-  if (!(MULTI ? find_row_tile(seq_cu, seq0, seq1, tq, blockIdx.x, s, tok0) : find_row(seq_cu, seq0, seq1, blockIdx.x, s, tok0))) return;
-  const int seq_r0 = seq_cu[s], n = seq_cu[s + 1] - seq_r0, ctx = seq_ctx[s];
+  T* __restrict__ const out = rest.out;
+  const T* __restrict__ const cache = rest.cache;
+  float *__restrict__ const ws_acc = rest.ws_acc, *__restrict__ const ws_ml = rest.ws_ml;
+  const float* __restrict__ const sink_w = rest.sink_w;
+  const long out_ld = rest.out_ld, proj_ld = rest.proj_ld;
+  const int block_shift = rest.block_shift, tq = rest.tq, hc = rest.hc, hchunks = rest.hchunks, heads = rest.heads, kv_heads = rest.kv_heads;
+  const int group = rest.group, gate_off = rest.gate_off, window = rest.window, part_keys = rest.part_keys, keep = rest.keep, chunk = rest.chunk;
+  const float scale = rest.scale, out_scale = rest.out_scale, softcap = rest.softcap;
+  const bool sink = rest.sink, channel_gate = rest.channel_gate;
+  int s, tok0, seq_r0, n, ctx;
+  [[maybe_unused]] long at = 0, new_slot = -1;
+  if constexpr (PREP) {
+    // asked for together, with the arguments, as if every sequence had a row, as they have in nearly every step
+    const int x = blockIdx.x, row = min(x, T_rows - 1);
+    int cu1 = seq_cu[x + 1];
+    seq_r0 = seq_cu[x];
+    ctx = seq_ctx[x];
+    at = positions[row];
+    new_slot = slots[row];
+    s = x;
+    tok0 = 0;
+    n = 1;
+    asm volatile("" ::"s"(rest.prep.q_norm), "s"(rest.prep.k_norm), "s"(rest.prep.inv_freq), "s"(rest.prep.nfreq), "s"(rest.prep.norm_mode),
+                 "s"(rest.prep.amp), "s"(rest.prep.eps), "s"(proj_ld), "s"(cache), "s"(heads), "s"(kv_heads), "s"(group), "s"(gate_off), "s"(window),
+                 "s"(part_keys), "s"(keep), "s"(chunk), "s"(rest.waves), "s"(rest.nparts), "s"(block_shift), "s"(hc), "s"(hchunks));
+    if (seq_r0 != x || cu1 != x + 1) {
+      if (!find_row(seq_cu, 0, rest.seq1, x, s, tok0)) return;
+      seq_r0 = seq_cu[s];
+      n = seq_cu[s + 1] - seq_r0;
+      ctx = seq_ctx[s];
+      at = positions[seq_r0 + tok0];
+      new_slot = slots[seq_r0 + tok0];
+    }
+  } else {
+    if (!(MULTI ? find_row_tile(seq_cu, rest.seq0, rest.seq1, tq, blockIdx.x, s, tok0) : find_row(seq_cu, rest.seq0, rest.seq1, blockIdx.x, s, tok0))) return;
+    seq_r0 = seq_cu[s];
+    n = seq_cu[s + 1] - seq_r0;
+    ctx = seq_ctx[s];
+  }
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = blockDim.x >> 6;
-  const int group = heads / kv_heads, kvh = blockIdx.y / hchunks, h0 = (blockIdx.y % hchunks) * hc;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = rest.waves, nparts = rest.nparts;   // (not from the launch's sizes: one more load)
+  const int kvh = hchunks == 1 ? blockIdx.y : blockIdx.y / hchunks, h0 = hchunks == 1 ? 0 : blockIdx.y % hchunks * hc;
   const int nh = min(hc, group - h0), head0 = kvh * group + h0;
   const int ntok = MULTI ? min(tq, n - tok0) : 1, p_first = ctx - n + tok0, p = p_first + ntok - 1;
   const int lo_all = first_key(max(p_first, 0), window, chunk);
@@ -260,24 +320,40 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
   const long r0 = seq_r0 + tok0 + (act ? rt : 0);
   const int nk = (window > 0 && keep > 0) ? min(keep, lo_all) : 0;   // kept keys below the window
   const int total = nk + p - lo_all + 1;
-  const int lo = blockIdx.z * part_keys, hi = gridDim.z > 1 ? min(total, lo + part_keys) - 1 : total - 1;
-  const long Dc = 2L * kv_heads * D;
+  const int lo = blockIdx.z * part_keys, hi = nparts > 1 ? min(total, lo + part_keys) - 1 : total - 1;
   const int* bt = seq_bt + (long)s * bt_width;
-  auto row_of = [&](int u) {   // cache row of the u-th visible key; past the run's end: of its last
-    u = min(u, hi);
-    const int j = u < nk ? u : u - nk + lo_all;
-    return cache + (((long)bt[j >> block_shift] << block_shift) + (j & ((1 << block_shift) - 1))) * Dc;
+  // The u-th visible key (past the run's end: its last) is row key_of(u) of the sequence, which lies in block bt[key_of(u) >> block_shift].
+  const int last = max(hi, 0), in_block = (1 << block_shift) - 1;
+  auto key_of = [&](int u) {
+    u = min(u, last);
+    return u < nk ? u : u - nk + lo_all;
+  };
+  auto row_of = [&](int block, int key) {
+    return cache + (unsigned long)(unsigned)((block << block_shift) + (key & in_block)) * (unsigned)(2 * kv_heads * D);
   };
   using Keys = u32x4[SUB][QN];
   // as they lie in memory: 16-bit elements of their own are taken apart, and waited for, where they are loaded
   using Part = __attribute__((ext_vector_type(E * sizeof(T) / 4))) unsigned;
   using Values = Part[4 * SUB][NB];
+  // A decode row's 16 keys side by side lie in at most two blocks, which are the same in every lane, unless blocks are smaller or keys are kept:
+  // ten rows per lane, each with a load and a 64-bit address of its own, were a quarter of a short step's time.
+  const bool near = !MULTI && nk == 0 && block_shift >= 4;
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  using Blocks = i32x2[SUB];
+  auto blocks_of = [&](int u0, Blocks& block) {
+#pragma unroll
+    for (int a = 0; a < SUB; ++a) block[a] = i32x2{bt[key_of(u0 + 16 * a) >> block_shift], bt[key_of(u0 + 16 * a + 15) >> block_shift]};
+  };
   using Rows = const T*[5 * SUB];
-  auto rows_of = [&](int u0, Rows& src) {
+  auto rows_of = [&](int u0, const Blocks& block, Rows& src) {
+    auto all = [&](auto&& row) {
 #pragma unroll
-    for (int a = 0; a < SUB; ++a) src[a] = row_of(u0 + 16 * a + c) + (long)kvh * D;
+      for (int a = 0; a < SUB; ++a) src[a] = row(a, key_of(u0 + 16 * a + c)) + kvh * D;
 #pragma unroll
-    for (int i = 0; i < 4 * SUB; ++i) src[SUB + i] = row_of(u0 + 16 * (i >> 2) + 4 * g + (i & 3)) + (long)(kv_heads + kvh) * D + E * c;
+      for (int i = 0; i < 4 * SUB; ++i) src[SUB + i] = row(i >> 2, key_of(u0 + 16 * (i >> 2) + 4 * g + (i & 3))) + (kv_heads + kvh) * D + E * c;
+    };
+    if (near) all([&](int a, int key) { return row_of(key >> block_shift == key_of(u0 + 16 * a) >> block_shift ? block[a][0] : block[a][1], key); });
+    else all([&](int, int key) { return row_of(bt[key >> block_shift], key); });
   };
   auto load = [&](const Rows& src, Keys& k, Values& v) {
 #pragma unroll
@@ -295,12 +371,22 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
   bool fresh = false;                                       // the run ends with the row's own key
   [[maybe_unused]] Keys k0;
   [[maybe_unused]] Values v0;
-  [[maybe_unused]] Rows src0;
+  [[maybe_unused]] Blocks block0;
+  [[maybe_unused]] T gate0{};   // of the thread's first results
   if constexpr (PREP) {
-    const long slot = prep.own_kv ? prep.slots[r0] : -1;
+    const long slot = rest.prep.own_kv ? new_slot : -1;
+    const T* row = proj + r0 * proj_ld;
     fresh = slot >= 0 && hi >= lo && hi == total - 1;
-    prepare_row<T, D>(prep, proj + r0 * proj_ld, prep.positions[r0], slot, head0, nh, kvh, heads, kv_heads, fresh && h0 == 0, hs,
-                      reinterpret_cast<float*>(hs + (hc + 2) * D), [&] { if (EARLY && first <= hi) rows_of(first, src0); }, [&] { if (EARLY && first <= hi) load(src0, k0, v0); });
+    prepare_row<T, D, MODE>(rest.prep, nw, row, at, slot, head0, nh, kvh, heads, kv_heads, fresh && h0 == 0, hs, reinterpret_cast<float*>(hs + (hc + 2) * D), [&] {
+      if (EARLY) blocks_of(first, block0);
+      gate0 = row[gate_off >= 0 && !channel_gate ? gate_off + head0 + min(tid / (D / 4), nh - 1) : 0];
+    }, [&] {
+      if constexpr (EARLY) {
+        Rows src;
+        rows_of(first, block0, src);
+        load(src, k0, v0);
+      }
+    });
   }
   u32x4 q[QN];
 #pragma unroll
@@ -323,8 +409,10 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
     Keys& k = EARLY ? k0 : kl;
     Values& v = EARLY ? v0 : vl;
     if (!EARLY || u0 != first) {
+      Blocks block;
       Rows src;
-      rows_of(u0, src);
+      blocks_of(u0, block);
+      rows_of(u0, block, src);
       load(src, k, v);
     }
     if (PREP && fresh && hi - u0 < KT) {   // the cache row is being written: its key and value are in LDS
@@ -431,32 +519,40 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
         for (int j = 0; j < E; j += 4)
           *reinterpret_cast<f32x4*>(dst + 16 * E * b + E * (4 * g + i) + j) =
               f32x4{acc[b][j][i], acc[b][j + 1][i], acc[b][j + 2][i], acc[b][j + 3][i]};
-    if (g == 0) { ml[2 * (wave * 16 + c)] = m; ml[2 * (wave * 16 + c) + 1] = l; }
+    if (g == 0) *reinterpret_cast<float2*>(ml + 2 * (c * nw + wave)) = float2{m, l};
   }
   __syncthreads();
-  for (int it = tid; it < nr * (D / 4); it += blockDim.x) {
+  for (int it = tid; it < nr * (D / 4); it += 64 * nw) {
     const int h = it / (D / 4), d = it % (D / 4) * 4, ht = MULTI ? h / hc : 0, hh = MULTI ? h % hc : h;
     if (MULTI && (ht >= ntok || hh >= nh)) continue;
-    float M = -INFINITY, L = 0.f;
-    for (int w = 0; w < nw; ++w) M = fmaxf(M, ml[2 * (w * 16 + h)]);
+    float2 mw[8];
+    f32x4 part[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {   // at most eight waves: what there is of them is asked for at once
+      mw[w] = *reinterpret_cast<const float2*>(ml + 2 * (h * nw + min(w, nw - 1)));
+      part[w] = *reinterpret_cast<const f32x4*>(lds + ((long)min(w, nw - 1) * nr + h) * D + d);
+    }
+    float M = mw[0].x, L = 0.f;
+#pragma unroll
+    for (int w = 1; w < 8; ++w) M = fmaxf(M, mw[w].x);
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    for (int w = 0; w < nw; ++w) {
-      const float mw = ml[2 * (w * 16 + h)];
-      if (mw == -INFINITY) continue;   // no key
-      const float f = S::exp(mw - M);
-      L += ml[2 * (w * 16 + h) + 1] * f;
-      o += *reinterpret_cast<const f32x4*>(lds + ((long)w * nr + h) * D + d) * f;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+      if (w >= nw) break;
+      const float f = mw[w].x == -INFINITY ? 0.f : S::exp(mw[w].x - M);   // no key: sums and outputs are 0
+      L += mw[w].y * f;
+      o += part[w] * f;
     }
     const int hd = head0 + hh;
     const long row = seq_r0 + tok0 + ht;
-    if (gridDim.z > 1) {
-      const long wrow = ((long)blockIdx.z * heads + hd) * gridDim.x + blockIdx.x;
+    if (nparts > 1) {
+      const long wrow = ((long)blockIdx.z * heads + hd) * (rest.seq1 - rest.seq0) + blockIdx.x;
       *reinterpret_cast<f32x4*>(ws_acc + wrow * D + d) = o;
       if (d == 0) { ws_ml[2 * wrow] = M; ws_ml[2 * wrow + 1] = L; }
       continue;
     }
     float f = out_scale;
-    if (gate_off >= 0 && !channel_gate) f *= sigmoid_f(ldf<T>(proj, row * proj_ld + gate_off + hd));
+    if (gate_off >= 0 && !channel_gate) f *= sigmoid_f(PREP && it == tid ? ldf<T>(&gate0, 0) : ldf<T>(proj, row * proj_ld + gate_off + hd));
     f = L == 0.f ? 0.f : f / L;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -509,16 +605,26 @@ void launch(T* out, long out_ld, const T* proj, long proj_ld, const T* cache, in
   const int nw = std::max(1, std::min({8, (part_keys + kt - 1) / kt, room / wave_floats}));
   const size_t smem = ((size_t)nw * wave_floats + prepared) * sizeof(float);
   const dim3 grid(rows, kv_heads * hchunks, nparts);
+  auto go = [&](auto* kernel, auto rest) {
+    rest.out = out; rest.out_ld = out_ld; rest.proj_ld = proj_ld; rest.cache = cache; rest.ws_acc = ws_acc; rest.ws_ml = ws_ml; rest.sink_w = sink_w;
+    rest.block_shift = __builtin_ctz(block_size); rest.seq0 = seq0; rest.seq1 = seq0 + rows; rest.tq = 1; rest.hc = hc; rest.hchunks = hchunks;
+    rest.heads = heads; rest.kv_heads = kv_heads; rest.group = group; rest.gate_off = gate_off; rest.window = window; rest.part_keys = part_keys;
+    rest.keep = keep; rest.chunk = chunk; rest.scale = scale; rest.out_scale = out_scale; rest.softcap = softcap; rest.sink = sink;
+    rest.channel_gate = channel_gate; rest.waves = nw; rest.nparts = nparts;
+    const WindowPrep none{};
+    const WindowPrep& pr = prep != nullptr ? *prep : none;
+    kernel<<<grid, 64 * nw, smem, s>>>(proj, seq_cu, seq_ctx, seq_bt, pr.positions, pr.slots, bt_width, pr.rows, rest);
+  };
+  if (prep == nullptr) go(&window_decode_kernel<T, D, false>, WindowRest<T, false>{});
   if constexpr (D <= 128) {
-    if (prep != nullptr)
-      window_decode_kernel<T, D, false, true><<<grid, 64 * nw, smem, s>>>(
-          out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq0 + rows, 1, hc, hchunks,
-          heads, kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, *prep);
+    if (prep != nullptr) {
+      WindowRest<T, true> rest{};
+      rest.prep = *prep;
+      if (prep->norm_mode == 1) go(&window_decode_kernel<T, D, false, 1>, rest);
+      else if (prep->norm_mode == 2) go(&window_decode_kernel<T, D, false, 2>, rest);
+      else go(&window_decode_kernel<T, D, false, 0>, rest);
+    }
   }
-  if (prep == nullptr)
-    window_decode_kernel<T, D, false><<<grid, 64 * nw, smem, s>>>(
-        out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq0 + rows, 1, hc, hchunks,
-        heads, kv_heads, gate_off, scale, window, sink, out_scale, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, NoPrep{});
   if (nparts > 1)
     window_decode_reduce_kernel<T><<<dim3(rows, heads), 128, 0, s>>>(out, out_ld, ws_acc, ws_ml, proj, proj_ld, gate_off, nparts,
                                                                     heads, rows, row_base, D, out_scale, channel_gate);
@@ -531,10 +637,13 @@ void launch_prompts(float* out, long out_ld, const float* proj, long proj_ld, co
                     bool channel_gate, int chunk, hipStream_t s) {
   const int group = heads / kv_heads, hc = std::min(group, 16), hchunks = (group + hc - 1) / hc, tq = 16 / hc;
   const int wave_floats = 16 * D + 32, nw = std::min(8, (1 << 14) / wave_floats);
+  WindowRest<float, false> rest{};
+  rest.out = out; rest.out_ld = out_ld; rest.proj_ld = proj_ld; rest.cache = cache; rest.sink_w = sink_w; rest.block_shift = __builtin_ctz(block_size);
+  rest.seq0 = seq0; rest.seq1 = seq1; rest.tq = tq; rest.hc = hc; rest.hchunks = hchunks; rest.heads = heads; rest.kv_heads = kv_heads;
+  rest.group = group; rest.gate_off = gate_off; rest.window = window; rest.keep = keep; rest.chunk = chunk; rest.scale = scale;
+  rest.out_scale = out_scale; rest.softcap = softcap; rest.sink = sink; rest.channel_gate = channel_gate; rest.waves = nw; rest.nparts = 1;
   window_decode_kernel<float, D, true><<<dim3(rows_bound / tq + (seq1 - seq0), kv_heads * hchunks, 1), 64 * nw,
-                                         (size_t)nw * wave_floats * sizeof(float), s>>>(
-      out, out_ld, proj, proj_ld, cache, __builtin_ctz(block_size), seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, tq, hc, hchunks,
-      heads, kv_heads, gate_off, scale, window, sink, out_scale, 0, nullptr, nullptr, keep, softcap, sink_w, channel_gate, chunk, NoPrep{});
+                                         (size_t)nw * wave_floats * sizeof(float), s>>>(proj, seq_cu, seq_ctx, seq_bt, nullptr, nullptr, bt_width, 0, rest);
 }
 
 }  // namespace
@@ -560,7 +669,7 @@ void launch_window_attention_decode(void* out, long out_ld, const void* proj, lo
                                     bool sink, float out_scale, int nparts, int part_keys, float* ws_acc, float* ws_ml, int keep,
                                     float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, const WindowPrep* prep,
                                     hipStream_t s) {
-  if (rows <= 0) return;
+  if (rows <= 0 || (prep != nullptr && prep->rows <= 0)) return;
 #define HS_WD(T, D)                                                                                                        \
   launch<T, D>((T*)out, out_ld, (const T*)proj, proj_ld, (const T*)cache, block_size, seq_cu, seq_ctx, seq_bt, bt_width, seq0, \
                rows, row_base, heads, kv_heads, gate_off, scale, window, sink, out_scale, nparts, part_keys, ws_acc, ws_ml,   \
