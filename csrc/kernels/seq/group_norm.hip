@@ -196,6 +196,95 @@ __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_vec_kernel(
   }
 }
 
+// The same for sizes that the compiler knows: rows of WAVES * 256, 4 elements per thread, groups of whole waves, TOP expert rows. A decode step's
+// rows are bound by the instructions that a wave issues in turn, of which there are half as many, a prompt's by memory; arguments that are
+// there at the start, every load before the first use, one barrier. us in a captured loop, rows not in the L2, bf16, the kernel above / this, 1, 48,
+// 512, 8192 rows: 2048, two expert rows 3.1 / 2.2, 4.3 / 2.8, 6.5 / 5.1, 58.9 / 55.0, with four parts 3.8 / 2.4, 5.2 / 3.3, 9.8 / 8.4, 98.2 / 95.9;
+// 4096, a row alone 3.0 / 2.6, 4.0 / 3.1, 8.6 / 7.7, 80.6 / 75.3; 1024, a row alone 2.3 / 2.0, 2.5 / 2.1, 3.9 / 3.2, 20.7 / 18.3.
+enum { kMixRow, kMixTwoParts, kMixFourParts, kFromTable };   // where the rows' addend (or the rows) come from
+
+struct KnownNormRest {
+  void* out;
+  int parts, rows, per;   // of mix; 1 << per waves share a group
+  float icols, eps;       // 1 / columns of a group (a power of two)
+  long table_rows;
+};
+struct KnownNormArgs {
+  const void *residual, *mix, *y, *pair_slot, *w, *ls1, *ls2;
+  KnownNormRest rest;
+};
+
+template <typename T, int WAVES, int KIND, int TOP>
+__global__ __launch_bounds__(64 * WAVES) void scaled_add_group_rmsnorm_known_kernel(
+    float* residual, const void* __restrict__ mix, const T* __restrict__ y, const int* __restrict__ pair_slot, const float* __restrict__ w,
+    const float* __restrict__ ls1, const float* __restrict__ ls2, const KnownNormRest) {
+  __shared__ float sums[WAVES];
+  constexpr int H = 256 * WAVES, P = KIND == kMixFourParts ? 4 : 2;
+  const int t = blockIdx.x, tid = threadIdx.x, e = 4 * tid, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const auto rest = late_args<KnownNormRest>(offsetof(KnownNormArgs, rest));
+  float* r = residual + (long)t * H + e;
+  float v[4], a[4], wv[4], l1[4], l2[4], part[P][4], ye[TOP > 0 ? TOP : 1][4];
+  int slot[TOP > 0 ? TOP : 1];
+#pragma unroll
+  for (int j = 0; j < TOP; ++j) slot[j] = pair_slot[t * TOP + j];
+  [[maybe_unused]] bool known = true;
+  if constexpr (KIND == kFromTable) {   // y: the table, pair_slot: the ids (an id outside the table gives a row of NaN, as no row is read)
+    const long id = reinterpret_cast<const long*>(pair_slot)[t];
+    known = id >= 0 && id < rest->table_rows;
+    Row<T, 4>::ld((known ? y + id * H : reinterpret_cast<const T*>(w)) + e, v);
+  } else {
+    Row<float, 4>::ld(r, v);
+  }
+  if constexpr (KIND == kMixRow) Row<T, 4>::ld(static_cast<const T*>(mix) + (long)t * H + e, a);
+  Row<float, 4>::ld(w + e, wv);
+  if constexpr (KIND != kFromTable) Row<float, 4>::ld((ls1 != nullptr ? ls1 : w) + e, l1);
+  if constexpr (TOP > 0) Row<float, 4>::ld(ls2 + e, l2);
+#pragma unroll
+  for (int j = 0; j < TOP; ++j) Row<T, 4>::ld(y + (long)slot[j] * H + e, ye[j]);
+  const int parts = rest->parts;
+  if constexpr (KIND == kMixTwoParts || KIND == kMixFourParts) {   // the last part in place of one that does not exist
+#pragma unroll
+    for (int j = 0; j < P; ++j) Row<float, 4>::ld(static_cast<const float*>(mix) + ((long)min(j, parts - 1) * rest->rows + t) * H + e, part[j]);
+  }
+  T* out = static_cast<T*>(rest->out);
+  const int per = rest->per;
+  const float icols = rest->icols, eps = rest->eps;
+  asm volatile("" ::"s"(out), "s"(per), "s"(icols), "s"(eps));
+  float q = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    if constexpr (KIND == kFromTable) {
+      if (!known) v[k] = __builtin_nanf("");
+    } else {
+      float m = 0.f;
+      if constexpr (KIND == kMixRow) m = a[k];
+      else {
+#pragma unroll
+        for (int j = 0; j < P; ++j) m += j < parts ? part[j][k] : 0.f;
+      }
+      v[k] += ls1 != nullptr ? m * l1[k] : m;
+    }
+    if constexpr (TOP > 0) {
+      float f = 0.f;
+#pragma unroll
+      for (int j = 0; j < TOP; ++j) f += ye[j][k];
+      v[k] += f * (1.f / (float)TOP) * l2[k];
+    }
+    q += v[k] * v[k];
+  }
+  Row<float, 4>::st(r, v);
+  q = wave_sum(q);
+  if ((tid & 63) == 0) sums[wave] = q;
+  __syncthreads();
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < WAVES; ++i) s += i >> per == wave >> per ? sums[i] : 0.f;
+  const float inv = 1.f / sqrtf(s * icols + eps);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = v[k] * inv * wv[k];
+  Row<T, 4>::st(out + (long)t * H + e, v);
+}
+
 // Any length and grouping, element by element.
 template <typename T>
 __global__ __launch_bounds__(kNT) void scaled_add_group_rmsnorm_kernel(
@@ -307,6 +396,25 @@ void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, i
   for (const void* p : {(const void*)out, (const void*)residual, (const void*)w, (const void*)mix, (const void*)ls1,
                         (const void*)y, (const void*)ls2, (const void*)extra, (const void*)table})
     at |= reinterpret_cast<uintptr_t>(p);
+  const int waves = H / 256;
+  if (at % 16 == 0 && extra == nullptr && H % 256 == 0 && (waves == 4 || waves == 8 || waves == 16) && groups > 0 &&
+      waves % groups == 0 && (y == nullptr || (top == 2 && ls2 != nullptr)) && (table != nullptr ? mix == nullptr && y == nullptr : mix != nullptr) &&
+      mix_parts <= 4) {
+    const KnownNormRest rest{out, mix_parts, T_, __builtin_ctz(waves / groups), (float)groups / (float)H, eps, table_rows};
+    auto go = [&](auto* kernel) {
+      if (table != nullptr) kernel<<<T_, 64 * waves, 0, s>>>(residual, nullptr, table, reinterpret_cast<const int*>(ids), w, ls1, ls2, rest);
+      else kernel<<<T_, 64 * waves, 0, s>>>(residual, mix, y, pair_slot, w, ls1, ls2, rest);
+    };
+#define HS_GS(W, KIND) (y != nullptr ? go(&scaled_add_group_rmsnorm_known_kernel<T, W, KIND, 2>) : go(&scaled_add_group_rmsnorm_known_kernel<T, W, KIND, 0>))
+#define HS_GW(W) (table != nullptr ? go(&scaled_add_group_rmsnorm_known_kernel<T, W, kFromTable, 0>) \
+                  : mix_parts == 0 ? HS_GS(W, kMixRow) : mix_parts <= 2 ? HS_GS(W, kMixTwoParts) : HS_GS(W, kMixFourParts))
+    if (waves == 4) HS_GW(4);
+    else if (waves == 8) HS_GW(8);
+    else HS_GW(16);
+#undef HS_GW
+#undef HS_GS
+    return;
+  }
   // 8 elements per thread and step, or 4 for rows that would leave half of the threads idle
   const int V = H <= 4 * kNT ? 4 : 8;
   if (at % 16 == 0 && H % V == 0 && (H / groups) % V == 0 && H <= 8 * 8 * kNT) {

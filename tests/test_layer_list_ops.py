@@ -73,6 +73,43 @@ def test_group_norm_unknown_id_and_unaligned_rows():
     assert torch.equal(ra, rb) and torch.allclose(a, b, rtol=2e-6, atol=0)
 
 
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,groups", [(1024, 4), (2048, 1), (2048, 8), (4096, 16), (4096, 2), (1280, 5), (3072, 3)])
+@pytest.mark.parametrize("T", [1, 3, 300])
+@pytest.mark.parametrize("kind", [0, 1, 2, 3, 4, "table"])
+def test_group_norm_of_known_sizes(H, groups, T, kind, dtype):
+    """Rows and groups of whole waves, and sizes beside them: ``mix`` as a row, in one to four parts, with two expert rows; ids inside and outside the table."""
+    g = torch.Generator().manual_seed(H + T)
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    res, w, kw, mix = rnd(T, H), 1 + 0.1 * rnd(H), {}, None
+    if kind == "table":
+        ids = torch.randint(0, 7, (T,), generator=g)
+        ids[T // 2] = 7 if T > 1 else 6
+        kw = dict(table=rnd(7, H).to(dtype), ids=ids)
+    else:
+        mix = rnd(T, H).to(dtype) if kind == 0 else rnd(kind, T, H)
+        kw = dict(ls1=0.5 + 0.1 * rnd(H), y=rnd(2 * T + 3, H).to(dtype), pair_slot=torch.randperm(2 * T + 3, generator=g)[:2 * T].int(), top=2, ls2=0.5 + 0.1 * rnd(H))
+    if kind == "table":
+        x = torch.where((ids < 7)[:, None], kw["table"][ids.clamp(max=6)].double(), float("nan"))
+    else:
+        x = res.double() + (mix.double() if kind == 0 else mix.double().sum(0)) * kw["ls1"].double()
+        x += kw["y"][kw["pair_slot"].long().view(T, 2)].double().sum(1) / 2 * kw["ls2"].double()
+    want = (x.view(T, groups, -1) * torch.rsqrt(x.view(T, groups, -1).square().mean(-1, keepdim=True) + 1e-6)).view(T, H) * w.double()
+    dev = lambda v: v.cuda() if isinstance(v, torch.Tensor) else v  # noqa: E731
+    got_res, got = res.cuda(), torch.empty(T, H, dtype=dtype, device="cuda")
+    ops = get_ops("cuda")
+    ops.norm_library = "delta"
+    ops.scaled_add_group_rmsnorm(got, got_res, w.cuda(), groups, 1e-6, dev(mix), **{k: dev(v) for k, v in kw.items()})
+    ok = ~x.isnan()
+    assert torch.equal(got_res.cpu().isnan(), ~ok) and torch.equal(got.cpu().isnan(), ~ok)
+    err = 8 * 16 * 2.0 ** -24   # eight additions of numbers below 16 in 32 bits
+    assert (got_res.cpu().double() - x)[ok].abs().max() <= err
+    # a neighbouring bf16 number; the norm's 32-bit sum and root; where the addends cancel, their error times 1 / rms (below 2) and w (below 1.5)
+    tol = 2.0 ** -8 if dtype == torch.bfloat16 else 2e-6
+    assert ((got.cpu().double() - want).abs()[ok] <= tol * want.abs()[ok] + 3 * err).all()
+
+
 # ------------------------------------------------------------------ soft cap
 @pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=gpu)])
 @pytest.mark.parametrize("shape", [(1, 5), (3, 2048), (2, 32001)])
