@@ -24,7 +24,7 @@
 // the one barrier per tile. Eight-way swizzles (operand rows met two to a bank) took 45 us more, scores without the next tile's
 // operand reads beside them a fifth more.
 // latent_dma_decode_kernel serves decode rows: a workgroup takes 16 heads of one row and a run of keys, 64 of them
-// at a time; its waves split the keys for S and the latent dims for P . V. One row of 724 keys, 16 heads: 46 -> 10 us.
+// at a time; its waves split the keys for S and the latent dims for P . V. One row of 724 keys, 16 heads, with the merge: 46 -> 10 us.
 #include "lds_copy.h"
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
@@ -50,6 +50,12 @@ template <int DV, int KEYS> struct Tile {
     constexpr int kPer = 512 / DV, kChunks = DV / 8;   // keys and 16-byte chunks of a key in one 1 KB copy
 #pragma unroll
     for (int i = 0; i < 8 / kPer; ++i) {
+      if constexpr (kPer == 1) {   // one key, the same for all lanes
+        const int k = 8 * w + i;
+        const unsigned lo = __builtin_amdgcn_readlane((int)row, k), hi = __builtin_amdgcn_readlane((int)(row >> 32), k);
+        copy_1k(reinterpret_cast<const unsigned char*>(cache + (long)((unsigned long)hi << 32 | lo)), 16 * (lane ^ swizzle(k)), lds + k * DV * 2);
+        continue;
+      }
       const int k = 8 * w + i * kPer + lane / kChunks, ch = (lane % kChunks) ^ swizzle(k);
       const unsigned short* src = cache + __shfl(row, k, 64) + 8 * ch;
       copy_1k(src, lds + (8 * w + i * kPer) * DV * 2);
@@ -91,10 +97,10 @@ template <int DV, int KEYS> struct Tile {
 };
 
 // Query operands of one (token, head) row: the latent part from qc, the last 64 dims from qc too, or rotated here from
-// the projection's rotary part (q_rot: its 64 numbers; entry i pairs with i + 32, angle pos * inv_freq[i]).
-template <int DV>
-HS_DEVICE void load_query(bf16x8 (&qf)[DV / 32 + 2], bool act, const unsigned short* qc, const unsigned short* q_rot, float pos,
-                          const float* __restrict__ inv_freq, int g) {
+// the projection's rotary part (q_rot: its 64 numbers; entry i pairs with i + 32, angle pos * inv_freq[i]). angle(i, sn, cs): of entry i, after
+// asked(), which runs behind the loads.
+template <int DV, typename F, typename G>
+HS_DEVICE void load_query(bf16x8 (&qf)[DV / 32 + 2], bool act, const unsigned short* qc, const unsigned short* q_rot, int g, G&& asked, F&& angle) {
   constexpr int KL = DV / 32;
   const u16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
@@ -106,11 +112,12 @@ HS_DEVICE void load_query(bf16x8 (&qf)[DV / 32 + 2], bool act, const unsigned sh
     a = *reinterpret_cast<const u16x8*>(src + 8 * g);
     b = *reinterpret_cast<const u16x8*>(src + 32 + 8 * g);
   }
+  asked();
   if (q_rot != nullptr && act) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       float sn, cs;
-      sincosf(pos * inv_freq[8 * g + e], &sn, &cs);
+      angle(8 * g + e, sn, cs);
       const float u = bf16_to_f32(a[e]), w = bf16_to_f32(b[e]);
       a[e] = f32_to_bf16(u * cs - w * sn);
       b[e] = f32_to_bf16(w * cs + u * sn);
@@ -209,7 +216,7 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
     bf16x8 qf[KS];
     load_query<DV>(qf, sact, qc + ((long)shead * T_rows + strow) * Dk,
                    q != nullptr ? q + strow * heads * (dim + kRot) + (long)shead * (dim + kRot) + dim : nullptr,
-                   (float)positions[strow], inv_freq, g);
+                   g, [] {}, [&, pos = (float)positions[strow]](int i, float& sn, float& cs) { sincosf(pos * inv_freq[i], &sn, &cs); });
     float m_run = -INFINITY;   // what the weights are relative to, log2 domain
     f32x4 lsum = {0.f, 0.f, 0.f, 0.f};   // sums of the weights that are multiplied, the same number in all four
     const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
@@ -353,33 +360,60 @@ __global__ __launch_bounds__(512, 2) void latent_dma_prefill_kernel(
 // 16 heads of the portion's row blockIdx.x against the run blockIdx.z of part_keys keys, 64 at a time: for portions of a row per
 // sequence, as decode rows are, and for runs. Wave w: scores of keys 16 w .., P . V of the latent dims DV / 4 w ... With
 // runs the unnormalised outputs and (max, sum) go to ws_acc / ws_ml.
+// What bounds it where the keys are few: the instructions of one wave in turn. The scalars that places and lengths need are asked for in one batch
+// with the arguments, the row's 32 angles are made once, a lane each, and a copy takes its key's row from a scalar
+// register, the scores are two chains. us with the merge of runs (latent_attention_mfma.hip), 16 heads, before / this: one row of 64 keys 8.4 / 6.9, of 256 11.1 /
+// 9.3, of 1024 11.4 / 9.7, 13 rows of 1300 15.6 / 14.2, 48 rows of 182 12.4 / 10.6.
+struct LatentDecodeRest {
+  unsigned short* o_lat;
+  const unsigned short *qc, *q, *proj;
+  const float* inv_freq;
+  float *ws_acc, *ws_ml;
+  long proj_ld;
+  int T_rows, heads, dim, gate_off, window, part_keys, row_base, ws_rows, nparts;
+  float scale;
+};
+
 template <int DV>
 __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
-    unsigned short* __restrict__ o_lat, const unsigned short* __restrict__ qc, const unsigned short* __restrict__ q,
-    const long* __restrict__ positions, const float* __restrict__ inv_freq, const unsigned short* __restrict__ proj,
-    long proj_ld, const unsigned short* __restrict__ cache, int block_shift, const int* __restrict__ seq_cu,
-    const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, int bt_width, int seq0, int seq1, int T_rows,
-    int heads, int dim, int gate_off, float scale, int window, int part_keys, float* __restrict__ ws_acc, float* __restrict__ ws_ml,
-    int row_base, int ws_rows) {
+    const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_bt, const long* __restrict__ positions,
+    const unsigned short* __restrict__ cache, int seq0, int seq1, int bt_width, int block_shift, const LatentDecodeRest rest) {
   constexpr int kTile = 64, kPd = kTile + 8;   // kPd: row stride of P in elements
   using KT = Tile<DV, kTile>;
   constexpr int KS = DV / 32 + 2, NPW = DV / 64, Dk = DV + kRot;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  __shared__ float2 angles[kRot / 2];
   unsigned short* p_lds = reinterpret_cast<unsigned short*>(smem + KT::kBytes);   // [16][kPd], MFMA k order
   float* mw = reinterpret_cast<float*>(p_lds + 16 * kPd);                         // [4][16] the waves' maxima
   float* lw = mw + 64;                                                            // [4][16] the waves' sums
-  int s, tok0;
-  if (!find_row(seq_cu, seq0, seq1, blockIdx.x, s, tok0)) return;
+  const int x = blockIdx.x;
+  int s = min(seq0 + x, seq1 - 1), tok0 = 0;
+  int first = seq_cu[seq0], r0 = seq_cu[s], r1 = seq_cu[s + 1], ctx = seq_ctx[s];
+  unsigned short* __restrict__ const o_lat = rest.o_lat;
+  const unsigned short *__restrict__ const qc = rest.qc, *__restrict__ const q = rest.q, *__restrict__ const proj = rest.proj;
+  const float* __restrict__ const inv_freq = rest.inv_freq;
+  float *__restrict__ const ws_acc = rest.ws_acc, *__restrict__ const ws_ml = rest.ws_ml;
+  const int T_rows = rest.T_rows, heads = rest.heads, dim = rest.dim, gate_off = rest.gate_off, window = rest.window, part_keys = rest.part_keys;
+  const long proj_ld = rest.proj_ld;
+  const float scale = rest.scale;
+  const bool partial = rest.nparts > 1;
+  asm volatile("" ::"s"(qc), "s"(q), "s"(inv_freq), "s"(ws_ml), "s"(T_rows), "s"(heads), "s"(dim), "s"(window), "s"(part_keys), "s"(rest.row_base),
+               "s"(rest.ws_rows), "s"(rest.nparts));
+  if (seq0 + x >= seq1 || r0 - first != x || r1 - r0 != 1) {   // not one row per sequence up to here
+    if (!find_row(seq_cu, seq0, seq1, x, s, tok0)) return;
+    r0 = seq_cu[s];
+    r1 = seq_cu[s + 1];
+    ctx = seq_ctx[s];
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
   const int head = blockIdx.y * 16 + c;
   const bool act = head < heads;
-  const int r0 = seq_cu[s], pos = seq_ctx[s] - (seq_cu[s + 1] - r0) + tok0;
+  const int pos = ctx - (r1 - r0) + tok0;
   const long trow = r0 + tok0;
   const int lo = (window > 0 ? max(0, pos - window + 1) : 0) + blockIdx.z * part_keys;
-  const int hi = gridDim.z > 1 ? min(pos, lo + part_keys - 1) : pos;
-  const bool partial = gridDim.z > 1;
-  const long wrow = ((long)blockIdx.z * heads + (act ? head : 0)) * ws_rows + (trow - row_base);
+  const int hi = partial ? min(pos, lo + part_keys - 1) : pos;
+  const long wrow = ((long)blockIdx.z * heads + (act ? head : 0)) * rest.ws_rows + (trow - rest.row_base);
   const int d0 = 16 * NPW * wave + 4 * g;   // the lane's latent dims of the output: 16 j + d0 .. + 3
   if (lo > hi) {   // an empty run, whose weight in the merge is 0, or a row that sees no key
     if (partial && act && wave == 0 && g == 0) { ws_ml[2 * wrow] = -INFINITY; ws_ml[2 * wrow + 1] = 0.f; }
@@ -392,7 +426,7 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
   const int mask = (1 << block_shift) - 1;
   auto row_of = [&](int j0) {
     const int j = min(j0 + lane, hi);
-    return (((long)bt[j >> block_shift] << block_shift) + (j & mask)) * Dk;
+    return (long)((unsigned long)(unsigned)((bt[j >> block_shift] << block_shift) + (j & mask)) * Dk);
   };
   const unsigned lds0 = lds_at(smem);
   auto copy = [&](int j0) {
@@ -400,11 +434,22 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
     KT::copy(lds0, cache, row, 2 * wave, lane);
     KT::copy(lds0, cache, row, 2 * wave + 1, lane);
   };
+  const bool rotate = q != nullptr;
+  const float at_pos = (float)positions[trow], freq = rotate ? inv_freq[lane & (kRot / 2 - 1)] : 0.f;
   copy(lo);
   bf16x8 qf[KS];
   load_query<DV>(qf, act, qc + ((long)(act ? head : 0) * T_rows + trow) * Dk,
-                 q != nullptr ? q + trow * heads * (dim + kRot) + (long)(act ? head : 0) * (dim + kRot) + dim : nullptr,
-                 (float)positions[trow], inv_freq, g);
+                 rotate ? q + trow * heads * (dim + kRot) + (long)(act ? head : 0) * (dim + kRot) + dim : nullptr, g,
+                 [&] {
+                   if (!rotate) return;
+                   if (tid < kRot / 2) {
+                     float sn, cs;
+                     sincosf(at_pos * freq, &sn, &cs);
+                     angles[tid] = float2{sn, cs};
+                   }
+                   barrier_lds();
+                 },
+                 [&](int i, float& sn, float& cs) { const float2 a = angles[i]; sn = a.x; cs = a.y; });
   f32x4 acc[NPW];
 #pragma unroll
   for (int j = 0; j < NPW; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -413,10 +458,11 @@ __global__ __launch_bounds__(256, 2) void latent_dma_decode_kernel(
   const typename KT::Places at = KT::places(wave, c, g);
   for (int j0 = lo; j0 <= hi; j0 += kTile) {
     barrier_all();
-    f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 half[2] = {};   // two chains
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks)
-      sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(KT::key_operand(smem, at, 16 * wave, ks), qf[ks], sc, 0, 0, 0);
+      half[ks & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(KT::key_operand(smem, at, 16 * wave, ks), qf[ks], half[ks & 1], 0, 0, 0);
+    const f32x4 sc = half[0] + half[1];
     float v[4], mx = -INFINITY;   // keys 16 wave + 4 g + i
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -489,8 +535,8 @@ bool launch_dma(void* o_lat, const void* qc, const void* q, const long* position
     static const bool ok = allow_lds(&latent_dma_decode_kernel<DV>, smem);
     if (!ok) return false;
     latent_dma_decode_kernel<DV><<<dim3(rows_bound, (heads + 15) / 16, nparts), 256, smem, s>>>(
-        o, a, b, positions, inv_freq, p, proj_ld, k, block_shift, seq_cu, seq_ctx, seq_bt, bt_width, seq0, seq1, T, heads, dim, gate_off,
-        scale, window, part_keys, ws_acc, ws_ml, row_base, rows_bound);
+        seq_cu, seq_ctx, seq_bt, positions, k, seq0, seq1, bt_width, block_shift,
+        LatentDecodeRest{o, a, b, p, inv_freq, ws_acc, ws_ml, proj_ld, T, heads, dim, gate_off, window, part_keys, row_base, rows_bound, nparts, scale});
     return true;
   }
   constexpr size_t smem = 4 * Tile<DV, kKeys>::kBytes + 2 * 64 * kPLd * 2 + 3 * 64 * 4;

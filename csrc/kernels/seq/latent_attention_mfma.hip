@@ -265,59 +265,69 @@ __global__ __launch_bounds__(64 * NW, 2) void latent_attention_mfma_kernel(
 
 // o_lat[h, row_base + r, :] = sum_p acc_p e^(m_p - M) / sum_p l_p e^(m_p - M) * sigmoid(gate)
 constexpr int kMaxRuns = 64;
+struct LatentReduceRest { long proj_ld; int gate_off, T_rows; };
+
+// EARLY runs' rows are asked for behind the weights, not after them: as many runs of 64 keys as a window of 1024 has, or 4 where there are no more; those
+// beyond are asked for below, four at a time. Both waves hold the runs' weights, a lane each, and take them from there: nothing goes through LDS, and the
+// gate's load does not wait behind a branch (figures: latent_attention_dma.hip).
+template <int EARLY>
 __global__ __launch_bounds__(128) void latent_attention_reduce_kernel(
-    unsigned short* __restrict__ o_lat, const float* __restrict__ ws_acc, const float* __restrict__ ws_ml,
-    const unsigned short* __restrict__ proj, long proj_ld, int gate_off, int nparts, int heads, int ws_rows,
-    int row_base, int T_rows, int kv_rank) {
-  __shared__ float sc[kMaxRuns];  // each run's weight e^(m_p - M) / L * gate, 0 for empty runs
-  const int r = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+    const float* __restrict__ ws_ml, const float* __restrict__ ws_acc, const unsigned short* __restrict__ proj, unsigned short* __restrict__ o_lat,
+    int nparts, int heads, int ws_rows, int row_base, int kv_rank, const LatentReduceRest rest) {
+  const int r = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const long step = (long)heads * ws_rows * kv_rank;   // from run to run
   const float* first = ws_acc + ((long)h * ws_rows + r) * kv_rank;
-  // The first runs' rows are asked for behind the weights, not after them (one row of 12 runs x 16 heads 4.8 -> 4.2 us): as many runs of 64
-  // keys as a window of 1024 has, in 64 registers; those beyond are asked for below, four at a time. With the attention before it, 12 / 16
-  // asked for: one row of 16 runs 12.1 / 11.5 us, of 12 runs 11.3 / 11.3, of 2 runs 10.9 / 11.0.
-  constexpr int kEarly = 16;
-  float m = -INFINITY, l = 0.f;
-  if (tid < min(nparts, 64)) {
-    const long w = ((long)tid * heads + h) * ws_rows + r;
-    m = ws_ml[2 * w];
-    l = ws_ml[2 * w + 1];
-  }
-  f32x4 early[kEarly];
+  const float2 run = *reinterpret_cast<const float2*>(ws_ml + 2 * (((long)min(lane, nparts - 1) * heads + h) * ws_rows + r));
+  f32x4 early[EARLY];
+  const int d0 = min(4 * tid, kv_rank - 4);
+  const float* at = first;
 #pragma unroll
-  for (int i = 0; i < kEarly; ++i)
-    if (i < nparts && 4 * tid < kv_rank) early[i] = *reinterpret_cast<const f32x4*>(first + i * step + 4 * tid);
-  if (tid < 64) {  // one wave: run p on lane p
-    const float M = wave_max(m);
-    const float e = m > -INFINITY ? __expf(m - M) : 0.f;
-    const float L = wave_sum(l * e);
-    const float gate = gate_off >= 0 ? sigmoid_f(bf16_to_f32(proj[(long)(row_base + r) * proj_ld + gate_off + h])) : 1.f;
-    sc[tid] = L > 0.f ? e * gate / L : 0.f;
+  for (int i = 0; i < EARLY; ++i) {   // the last one in place of those that do not exist
+    early[i] = *reinterpret_cast<const f32x4*>(at + d0);
+    at += i + 1 < nparts ? step : 0;
   }
-  __syncthreads();
   const long trow = row_base + r;
+  const int gate_off = rest.gate_off;
+  const float gate_in = bf16_to_f32(proj[trow * rest.proj_ld + (gate_off >= 0 ? gate_off + h : 0)]);   // (a branch around it would wait for all of the above)
+  const float m = lane < nparts ? run.x : -INFINITY, l = lane < nparts ? run.y : 0.f;
+  const float M = wave_max(m);
+  const float e = m > -INFINITY ? __expf(m - M) : 0.f;
+  const float L = wave_sum(l * e);
+  const float gate = gate_off >= 0 ? sigmoid_f(gate_in) : 1.f;
+  const float weight = L > 0.f ? e * gate / L : 0.f;   // of run `lane`, 0 for an empty one
+  auto weight_of = [&](int p) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), p)); };
   for (int d = 4 * tid; d < kv_rank; d += 512) {   // kv_rank % 4 == 0
     f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
     const float* src = first + d;
     if (d == 4 * tid) {
 #pragma unroll
-      for (int i = 0; i < kEarly; ++i)
-        if (i < nparts && sc[i] != 0.f) o += early[i] * sc[i];   // an empty run (weight 0) holds anything
+      for (int i = 0; i < EARLY; ++i) {
+        const float f = weight_of(i);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] += f != 0.f ? early[i][k] * f : 0.f;   // an empty run (weight 0) holds anything
+      }
     }
-    for (int p0 = d == 4 * tid ? kEarly : 0; p0 < nparts; p0 += 4) {   // four runs' loads in flight; an empty run is not read
+    for (int p0 = d == 4 * tid ? EARLY : 0; p0 < nparts; p0 += 4) {   // four runs' loads in flight; an empty run is not read
       f32x4 v[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        v[i] = p0 + i < nparts && sc[p0 + i] != 0.f ? *reinterpret_cast<const f32x4*>(src + (p0 + i) * step) : f32x4{0.f, 0.f, 0.f, 0.f};
+        v[i] = p0 + i < nparts && weight_of((p0 + i) & 63) != 0.f ? *reinterpret_cast<const f32x4*>(src + (p0 + i) * step) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (p0 + i < nparts) o += v[i] * sc[p0 + i];
+        if (p0 + i < nparts) o += v[i] * weight_of((p0 + i) & 63);
     }
     u16x4 w;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w[e] = f32_to_bf16(o[e]);
-    *reinterpret_cast<u16x4*>(o_lat + ((long)h * T_rows + trow) * kv_rank + d) = w;
+    for (int k = 0; k < 4; ++k) w[k] = f32_to_bf16(o[k]);
+    *reinterpret_cast<u16x4*>(o_lat + ((long)h * rest.T_rows + trow) * kv_rank + d) = w;
   }
+}
+
+void reduce_runs(unsigned short* o_lat, const float* ws_acc, const float* ws_ml, const unsigned short* proj, long proj_ld, int gate_off, int nparts,
+                 int heads, int ws_rows, int row_base, int T, int kv_rank, hipStream_t s) {
+  auto fn = nparts <= 4 ? &latent_attention_reduce_kernel<4> : nparts <= 8 ? &latent_attention_reduce_kernel<8>
+            : nparts <= 12 ? &latent_attention_reduce_kernel<12> : &latent_attention_reduce_kernel<16>;
+  fn<<<dim3(ws_rows, heads), 128, 0, s>>>(ws_ml, ws_acc, proj, o_lat, nparts, heads, ws_rows, row_base, kv_rank, LatentReduceRest{proj_ld, gate_off, T});
 }
 
 template <int KS, int NPW, int NW>
@@ -343,9 +353,7 @@ bool launch_mfma(unsigned short* o_lat, const unsigned short* qc, const unsigned
                                 tq, hc, T, heads, rot_dim, kv_rank, gate_off, scale, window, part_keys, ws_acc, ws_ml,
                                 row_base, rows_bound);
   if (nparts > 1)
-    latent_attention_reduce_kernel<<<dim3(rows_bound, heads), 128, 0, s>>>(o_lat, ws_acc, ws_ml, proj, proj_ld, gate_off,
-                                                                         nparts, heads, rows_bound, row_base, T,
-                                                                         kv_rank);
+    reduce_runs(o_lat, ws_acc, ws_ml, proj, proj_ld, gate_off, nparts, heads, rows_bound, row_base, T, kv_rank, s);
   return true;
 }
 
@@ -361,9 +369,7 @@ void launch_latent_q_cat(void* qc, const float* q_abs, const void* q, const long
 void launch_latent_attention_reduce(void* o_lat, const float* ws_acc, const float* ws_ml, const void* proj, long proj_ld,
                                     int gate_off, int nparts, int heads, int rows_bound, int row_base, int T, int kv_rank,
                                     hipStream_t s) {
-  latent_attention_reduce_kernel<<<dim3(rows_bound, heads), 128, 0, s>>>((unsigned short*)o_lat, ws_acc, ws_ml,
-                                                                       (const unsigned short*)proj, proj_ld, gate_off, nparts,
-                                                                       heads, rows_bound, row_base, T, kv_rank);
+  reduce_runs((unsigned short*)o_lat, ws_acc, ws_ml, (const unsigned short*)proj, proj_ld, gate_off, nparts, heads, rows_bound, row_base, T, kv_rank, s);
 }
 
 bool latent_attention_mfma_ok(int kv_rank, int rot_dim) {
