@@ -12,7 +12,8 @@
 // Decode steps (mingru_step): one row per sequence needs no folding; 4 channels per thread, 9.1 -> 5.0 us for 41 sequences. Up to 64 of
 // them run in the epilogue of the product that makes z, x and g (mingru_product): a workgroup has all three of its 16 channels,
 // unrounded, and the states arrive beside its weights. Width 4096, K 2048, in a captured step: one row 11.6 + 4.4
-// -> 12.0 us, 48 rows 16.0 + 4.7 -> 15.4.
+// -> 12.0 us, 48 rows 16.0 + 4.7 -> 15.4. The copies need no arguments that have to be loaded, and the rows' sequences come through the scalar unit:
+// 1, 16, 48, 64 rows 12.4 -> 11.5, 12.5 -> 11.8, 15.4 -> 14.6, 16.8 -> 15.7 (in a loop), width 2048, K 1024 5.0 -> 4.4, 5.2 -> 4.5, 7.4 -> 6.8, 8.3 -> 7.5.
 #include "skinny.h"
 #include "hipserve/seq_kernels.h"
 
@@ -126,16 +127,27 @@ __global__ __launch_bounds__(256) void mingru_step_kernel(T* __restrict__ y, flo
   Row<float, kV>::st(st, S);
 }
 
+struct MinGruRest {
+  void* y;
+  float* state;
+  const float *b_z, *b_x;
+  int nseq;
+};
+struct MinGruArgs {
+  const void *x, *w, *seq_cu, *seq_ctx, *seq_state;
+  int x_ld, M, width, K;
+  MinGruRest rest;
+};
+
 // y, state of the rows x [M, K], one per sequence, and w = [z rows; x rows; g rows]. F32: x, w, x_ld and K in 16-bit halves (skinny.h).
 template <int XG, int DEPTH, bool F32>
 __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
-    void* __restrict__ y_, float* state, const unsigned short* __restrict__ x, long x_ld, const unsigned short* __restrict__ w,
-    const float* b_z, const float* b_x, const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K) {
+    const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx,
+    const int* __restrict__ seq_state, int x_ld, int M, int width, int K, const MinGruRest) {
   using SK = Skinny<XG, 3, DEPTH, F32>;
   using T = std::conditional_t<F32, float, unsigned short>;
   constexpr int ST = SK::ST, IT = (ST + 1) / 2;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  T* y = static_cast<T*>(y_);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n0 = blockIdx.x * 16, c = min(n0 + (tid & 15), width - 1);
   const unsigned char* wt[3];
@@ -144,7 +156,7 @@ __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
   for (int nt = 0; nt < 3; ++nt) {
     wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)nt * width + n0) * K);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)(min(n0 + 8 * h + (lane >> 3), width - 1) - n0) * (unsigned)K * 2;
+    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), width - 1 - n0) * (unsigned)K * 2;
   }
 #pragma unroll
   for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)x_ld * 2;
@@ -153,26 +165,38 @@ __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
   for (int nt = 0; nt < 3; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
+  T* y = nullptr;
+  float* state = nullptr;
   float bz, bx, S[IT];
   long at[IT];   // the channel's place in the row's state, -1: the row has no sequence
+  bool fresh[IT];
   SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave, [&] {
-    bz = b_z[c];
-    bx = b_x[c];
+    const auto rest = late_args<MinGruRest>(offsetof(MinGruArgs, rest));
+    const int nseq = rest->nseq;
+    y = static_cast<T*>(rest->y);
+    state = rest->state;
+    bz = rest->b_z[c];
+    bx = rest->b_x[c];
+    // A wave's four rows' sequences through the scalar unit, whose loads the copies in flight are not waited for with.
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
-      const int m = (tid + kSkThreads * i) >> 4;
-      at[i] = -1;
-      S[i] = 0.f;
-      if (m >= M) continue;
-      int s = min(m, nseq - 1), ctx = seq_ctx[s], slot = seq_state[s];
-      if (seq_cu[s] != m || seq_cu[s + 1] != m + 1) {   // sequences without a row lie between
-        for (s = 0; s < nseq && !(seq_cu[s] <= m && m < seq_cu[s + 1]);) ++s;
-        if (s == nseq) continue;
-        ctx = seq_ctx[s];
-        slot = seq_state[s];
+      int slot = -1, ctx = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int m = 4 * wave + 32 * i + k;
+        if (m >= M) continue;
+        int s = min(m, nseq - 1), ctx_k = seq_ctx[s], slot_k = seq_state[s];
+        const int first = seq_cu[s], end = seq_cu[s + 1];
+        if ((first ^ m) | (end ^ (m + 1))) {   // sequences without a row lie between
+          for (s = 0; s < nseq && !(seq_cu[s] <= m && m < seq_cu[s + 1]);) ++s;
+          ctx_k = s < nseq ? seq_ctx[s] : 0;
+          slot_k = s < nseq ? seq_state[s] : -1;
+        }
+        if (lane >> 4 == k) { slot = slot_k; ctx = ctx_k; }
       }
-      at[i] = (long)slot * width + c;
-      if (ctx > 1) S[i] = state[at[i]];
+      at[i] = slot < 0 ? -1 : (long)slot * width + c;
+      fresh[i] = ctx <= 1;
+      S[i] = state[at[i] < 0 ? c : at[i]];
     }
   });
   float v[3][IT];
@@ -182,7 +206,7 @@ __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
     const int m = (tid + kSkThreads * i) >> 4;
     if (m >= M || n0 + (tid & 15) >= width || at[i] < 0) continue;
     const Gru g(v[0][i], v[1][i], bz, bx);
-    const float o = (1.f - g.z) * S[i] + g.zc;
+    const float o = (1.f - g.z) * (fresh[i] ? 0.f : S[i]) + g.zc;
     stf<T>(y, (long)m * width + c, o * (v[2][i] * sigmoid_f(v[2][i])));
     state[at[i]] = o;
   }
@@ -193,8 +217,8 @@ bool launch_product(void* y, float* state, const void* x, long x_ld, const void*
                     const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, bool f32, hipStream_t s) {
   constexpr int lds = Skinny<XG, 3, DEPTH>::kLds;
   auto go = [&](auto* kernel) {
-    kernel<<<(width + 15) / 16, kSkThreads, lds, s>>>(y, state, (const unsigned short*)x, x_ld, (const unsigned short*)w, b_z, b_x, seq_cu,
-                                                       seq_ctx, seq_state, nseq, M, width, K);
+    kernel<<<(width + 15) / 16, kSkThreads, lds, s>>>((const unsigned short*)x, (const unsigned short*)w, seq_cu, seq_ctx, seq_state, (int)x_ld, M,
+                                                       width, K, MinGruRest{y, state, b_z, b_x, nseq});
   };
   static const bool ok = allow_lds(&mingru_product_kernel<XG, DEPTH, false>, lds) && allow_lds(&mingru_product_kernel<XG, DEPTH, true>, lds);
   if (!ok) return false;
