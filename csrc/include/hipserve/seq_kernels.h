@@ -106,10 +106,11 @@ void launch_mingru_scan(void* y, float* state, const void* proj, const float* b_
 // expert is < 0 or >= E (no weights) are skipped. act 0: none, 1: squared ReLU, 2: W[e] = [gate rows; up rows]
 // and out[slot, N / 2] = silu(gate) * up, 3: the same with g sigmoid(1.702 g) (u + 1), g = min(gate, limit),
 // u = clamp(up, -limit, limit). row_scale (may be null): the products of pair p are multiplied by row_scale[p] first.
-// pairs: how many (token, choice) pairs the tiles hold (0: guessed from their capacity).
+// pairs: how many (token, choice) pairs the tiles hold (0: guessed from their capacity). ntiles: tiles to launch, all of the capacity, or
+// fewer where those in use are known to be among them (bounded: they are counted, the alignments leave a pair in each).
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,
-                        int ntiles_cap, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
-                        float limit, int pairs, bool f32, hipStream_t s);
+                        int ntiles_cap, int ntiles, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
+                        float limit, int pairs, bool bounded, bool f32, hipStream_t s);
 
 // Whether tiles of 32 slots that hold so many pairs run the kernel for few rows per tile.
 bool expert_gemm_skinny(long pairs, long ntiles_cap, long N, long K, long E, bool glu);

@@ -74,7 +74,7 @@ inline bool moe_align_small(int64_t npairs) { return hipserve::moe_align_blocks(
 
 inline void expert_gemm(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const at::Tensor& slots,
                         const at::Tensor& tile_expert, int64_t tile, int64_t gather_k, int64_t act,
-                        const c10::optional<at::Tensor>& row_scale, double limit, int64_t pairs) {
+                        const c10::optional<at::Tensor>& row_scale, double limit, int64_t pairs, int64_t tiles) {
   auto i32 = [](const at::Tensor& t) { return t.scalar_type() == at::kInt && t.is_contiguous(); };
   TORCH_CHECK(x.is_cuda() && out.is_contiguous() && w.is_contiguous() && i32(slots) && i32(tile_expert));
   TORCH_CHECK(x.scalar_type() == at::kFloat || x.scalar_type() == at::kBFloat16, "expert_gemm: bf16 or fp32 activations");
@@ -92,10 +92,12 @@ inline void expert_gemm(at::Tensor& out, const at::Tensor& x, const at::Tensor& 
   TORCH_CHECK(tile % 32 == 0 && cap % tile == 0 && tile_expert.numel() * tile >= cap, "tiles of a multiple of 32 slots");
   TORCH_CHECK(gather_k > 0 || x.size(0) >= cap, "ungathered x needs one row per slot");
   TORCH_CHECK(pairs >= 0 && pairs <= cap, "expert_gemm: at most a pair per slot");
+  TORCH_CHECK(tiles >= 0, "expert_gemm: tiles in use");   // 0: not known; else they are among the first so many
+  const long ntiles = tiles > 0 ? std::min<long>(tiles, cap / tile) : cap / tile;
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   hipserve::launch_expert_gemm(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), slots.data_ptr<int>(),
-                               tile_expert.data_ptr<int>(), cap / tile, tile, gather_k, N, K, act, w.size(0),
-                               (const float*)opt_ptr(row_scale), (float)limit, pairs, f32,
+                               tile_expert.data_ptr<int>(), cap / tile, ntiles, tile, gather_k, N, K, act, w.size(0),
+                               (const float*)opt_ptr(row_scale), (float)limit, pairs, tiles > 0, f32,
                                c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
 }
 
@@ -223,7 +225,7 @@ inline void def_moe_ops(torch::Library& m) {
         "Tensor(c!) pair_slot) -> ()");
   m.def("moe_align_small(int npairs) -> bool", &moe_align_small);
   m.def("expert_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor slots, Tensor tile_expert, int tile, int gather_k, "
-        "int act, Tensor? row_scale=None, float limit=0.0, int pairs=0) -> ()");
+        "int act, Tensor? row_scale=None, float limit=0.0, int pairs=0, int tiles=0) -> ()");
   m.def("expert_gemm_skinny(int pairs, int ntiles_cap, int N, int K, int E, bool glu) -> bool", &expert_gemm_skinny);
 }
 

@@ -192,33 +192,56 @@ __global__ __launch_bounds__(256) void expert_gemm_mfma_kernel(
   }
 }
 
+struct ExpertRest {
+  unsigned short* out;
+  const float* row_scale;
+  int act;
+  float limit;
+};
+struct ExpertArgs {
+  const void *slots, *tile_expert, *x, *w;
+  int x_ld, N, K, E, gather_k, gather_shift;
+  ExpertRest rest;
+};
+
 // bf16, tiles with few live slots (decode steps): 16 columns per workgroup, K split over its waves (skinny.h). XG groups of 8 slots:
-// moe_align fills a tile from its first slot on, so one is enough for most.
+// moe_align fills a tile from its first slot on, so one is enough for most. mine: the pair in the tile's slot lane % 32: asked for once, together with
+// the tile's expert. What bounds it is the memory, and for a few rows the start of its workgroups: one row of 16 experts, two of them hit, 1024 x 2048
+// and 2048 x 1024 4.0 -> 3.7 and 3.9 -> 3.6 us with two of 16 tiles launched and without loads of arguments ahead of the copies.
 template <int XG, int NT, int DEPTH, bool GLU>
-HS_DEVICE void expert_rows(unsigned short* __restrict__ out, const unsigned short* __restrict__ x, long x_ld,
-                           const unsigned char* const (&wt)[NT], const unsigned (&w_row)[2 * NT], const int* __restrict__ slots, int slot0,
-                           int n0, int No, int gather_k, int K, int act, const float* __restrict__ row_scale, float limit,
-                           unsigned char* smem) {
+HS_DEVICE void expert_rows(const unsigned short* __restrict__ x, unsigned x_ld, const unsigned char* const (&wt)[NT], const unsigned (&w_row)[2 * NT],
+                           int mine, int slot0, int n0, int No, int gather_k, int gather_shift, int K, unsigned char* smem) {
   using SK = Skinny<XG, NT, DEPTH>;
   constexpr int ST = SK::ST;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   unsigned x_row[XG];
 #pragma unroll
   for (int j = 0; j < XG; ++j) {
-    const int slot = slot0 + 8 * j + (lane >> 3), p = slots[slot];
-    x_row[j] = (unsigned)(p < 0 ? 0 : gather_k > 0 ? p / gather_k : slot) * (unsigned)x_ld * 2;   // no pair: any row
+    const int r = 8 * j + (lane >> 3), p = __shfl(mine, r, 64);
+    const int from = gather_shift >= 0 ? p >> gather_shift : gather_k > 0 ? p / gather_k : slot0 + r;
+    x_row[j] = (unsigned)(p < 0 ? 0 : from) * x_ld * 2;   // no pair: any row
   }
   f32x4 acc[NT][ST];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave);
+  unsigned short* out = nullptr;
+  const float* row_scale = nullptr;
+  int act = 0;
+  float limit = 0.f;
+  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave, [&] {
+    const auto rest = late_args<ExpertRest>(offsetof(ExpertArgs, rest));
+    out = rest->out;
+    row_scale = rest->row_scale;
+    act = rest->act;
+    limit = rest->limit;
+    asm volatile("" ::"s"(out), "s"(row_scale), "s"(act), "s"(limit));
+  });
   float v[NT][(ST + 1) / 2];
   SK::reduce(v, acc, smem);
-  if (tid >= 128 * XG) return;
-  const int slot = slot0 + (tid >> 4), p = slots[slot];   // an element of the [8 XG, 16] result per thread
-  if (p < 0) return;
+  const int slot = slot0 + (tid >> 4), p = __shfl(mine, tid >> 4 & 31, 64);   // an element of the [8 XG, 16] result per thread
+  if (tid >= 128 * XG || p < 0) return;
   const float f = row_scale != nullptr ? row_scale[p] : 1.f;
 #pragma unroll
   for (int nt = 0; nt < (GLU ? 1 : NT); ++nt) {
@@ -248,13 +271,12 @@ template <int NT> constexpr int expert_lds() {
 
 template <int NT, bool GLU>
 __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
-    unsigned short* __restrict__ out, const unsigned short* __restrict__ x, long x_ld,
-    const unsigned short* __restrict__ w, const int* __restrict__ slots, const int* __restrict__ tile_expert,
-    int gather_k, int N, int K, int act, int E, const float* __restrict__ row_scale, float limit) {
+    const int* __restrict__ slots, const int* __restrict__ tile_expert, const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
+    int x_ld, int N, int K, int E, int gather_k, int gather_shift, const ExpertRest) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, slot0 = blockIdx.y * 32;
-  const int e = tile_expert[blockIdx.y];
-  const unsigned long live = __ballot(slots[slot0 + (lane & 31)] >= 0);   // before the tile's expert is looked at: both loads in flight
+  const int e = tile_expert[blockIdx.y], mine = slots[slot0 + (lane & 31)];   // both loads in flight
+  const unsigned long live = __ballot(mine >= 0);
   if (e < 0 || e >= E) return;
   const int No = GLU ? N / 2 : N, n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
   const unsigned char* wt[NT];
@@ -264,10 +286,9 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
     const int first = GLU ? n0 : min(n0 + 16 * nt, N - 1);   // of the tile's columns
     wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)e * N + (GLU ? nt * No : 0) + first) * K);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)(min(first + 8 * h + (lane >> 3), No - 1) - first) * (unsigned)K * 2;
+    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), No - 1 - first) * (unsigned)K * 2;
   }
-#define HS_ER(XG, DEPTH) \
-  expert_rows<XG, NT, DEPTH, GLU>(out, x, x_ld, wt, w_row, slots, slot0, n0, No, gather_k, K, act, row_scale, limit, smem)
+#define HS_ER(XG, DEPTH) expert_rows<XG, NT, DEPTH, GLU>(x, x_ld, wt, w_row, mine, slot0, n0, No, gather_k, gather_shift, K, smem)
   if (live >> 16 & 0xffff) HS_ER(4, 1);
   else if (live >> 8 & 0xff) HS_ER(2, 1);
   else HS_ER(1, GLU ? 1 : 2);
@@ -276,7 +297,14 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
 
 }  // namespace
 
-// Which of the two kernels serves tiles of 32 slots; cold weights, us, 462 sizes of 4 to 256 experts, K from 512 to 4096 and up to 1600
+// Which of the two kernels serves tiles of 32 slots, where the caller says how many tiles are in use at most (`ntiles` of them are launched): the one for
+// few rows but for thousands of workgroups of 512 k and fewer, whose start costs more than their products. Of 280 sizes (4 to 256 experts, k 512 - 4096,
+// up to 200 pairs per expert, gated and not) it is the slower one in two others, by 3 % and 1 %. us, tile kernel / this one: 16 experts, 2048 x 1024: 22, 96
+// and 200 pairs 16.7 / 12.0, 17.1 / 14.7, 19.1 / 15.8; 8 experts, 4096 x 2048, 22 pairs 34.1 / 25.8; 64 experts, 704 x 2048, 96 pairs 47.0 / 25.8; 128 experts,
+// 2048 x 768, 64 pairs 39.5 / 30.5; but 256 experts, 2048 x 512, 256 pairs 64.5 / 78.9, 72 pairs 27.3 / 28.1.
+static bool expert_rows_pay(long ntiles, long No, long K) { return K >= 640 || (No + 15) / 16 * ntiles <= 8192; }
+
+// The same where the whole capacity is launched, as the two were before a tile's slots came to a workgroup with its expert; us, cold weights, 462 sizes of 4 to 256 experts, K from 512 to 4096 and up to 1600
 // pairs. Both read the weights of the experts that so many pairs hit on average. expert_gemm_skinny takes 3.1 plus them at 7 TB/s and what its
 // workgroups of 16 columns (gated 32) take in, the rows at 86 KB per us and CU, over K in whole rounds of its eight waves, and 0.37 per 1000
 // workgroups: it has one per 16 columns of every tile of the capacity. expert_gemm_mfma takes 4.2 plus the weights at 11 TB/s and the longest of
@@ -299,31 +327,33 @@ bool expert_gemm_skinny(long pairs, long ntiles_cap, long N, long K, long E, boo
 }
 
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,
-                        int ntiles_cap, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
-                        float limit, int pairs, bool f32, hipStream_t s) {
+                        int ntiles_cap, int ntiles, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
+                        float limit, int pairs, bool bounded, bool f32, hipStream_t s) {
   if (ntiles_cap <= 0) return;
   // the capacity covers a partly filled tile per expert
   pairs = pairs > 0 ? pairs : std::max(1, ntiles_cap * tile - E * (tile - 1));
   const int No = act >= 2 ? N / 2 : N;
   if (!f32 && K % 8 == 0 && No % 8 == 0 && x_ld % 8 == 0 && (tile == 32 || tile == 64)) {
-    dim3 mg(act >= 2 ? (No + 63) / 64 : (N + 127) / 128, ntiles_cap);
+    dim3 mg(act >= 2 ? (No + 63) / 64 : (N + 127) / 128, ntiles);
     auto o = (unsigned short*)out;
     auto xi = (const unsigned short*)x, wi = (const unsigned short*)w;
-    if (tile == 32 && K < (1 << 24) && 2L * ntiles_cap * tile * x_ld < (1L << 32) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && expert_gemm_skinny(pairs, ntiles_cap, N, K, E, act >= 2)) {
-      const dim3 sg((No + 15) / 16, ntiles_cap);
+    if (tile == 32 && K < (1 << 24) && 2L * ntiles_cap * tile * x_ld < (1L << 32) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 &&
+        (bounded ? expert_rows_pay(ntiles, No, K) : expert_gemm_skinny(pairs, ntiles_cap, N, K, E, act >= 2))) {
+      const dim3 sg((No + 15) / 16, ntiles);
+      const int shift = gather_k > 0 && (gather_k & (gather_k - 1)) == 0 ? __builtin_ctz(gather_k) : -1;
       if (act >= 2)
-        expert_gemm_skinny_kernel<2, true><<<sg, kSkThreads, expert_lds<2>(), s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K,
-                                                                                  act, E, row_scale, limit);
+        expert_gemm_skinny_kernel<2, true><<<sg, kSkThreads, expert_lds<2>(), s>>>(slots, tile_expert, xi, wi, (int)x_ld, N, K, E, gather_k, shift,
+                                                                                  ExpertRest{o, row_scale, act, limit});
       else
-        expert_gemm_skinny_kernel<1, false><<<sg, kSkThreads, expert_lds<1>(), s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N,
-                                                                                   K, act, E, row_scale, limit);
+        expert_gemm_skinny_kernel<1, false><<<sg, kSkThreads, expert_lds<1>(), s>>>(slots, tile_expert, xi, wi, (int)x_ld, N, K, E, gather_k, shift,
+                                                                                   ExpertRest{o, row_scale, act, limit});
       return;
     }
     if (tile == 32) expert_gemm_mfma_kernel<2><<<mg, 256, 0, s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K, act, E, row_scale, limit);
     else expert_gemm_mfma_kernel<4><<<mg, 256, 0, s>>>(o, xi, x_ld, wi, slots, tile_expert, gather_k, N, K, act, E, row_scale, limit);
     return;
   }
-  dim3 grid(act >= 2 ? (No + kTN / 2 - 1) / (kTN / 2) : (N + kTN - 1) / kTN, (long)ntiles_cap * tile / kTM);
+  dim3 grid(act >= 2 ? (No + kTN / 2 - 1) / (kTN / 2) : (N + kTN - 1) / kTN, (long)ntiles * tile / kTM);
   if (f32)
     expert_gemm_kernel<float><<<grid, 256, 0, s>>>((float*)out, (const float*)x, x_ld, (const float*)w, slots,
                                                    tile_expert, tile, gather_k, N, K, act, E, row_scale, limit);

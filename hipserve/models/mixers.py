@@ -354,9 +354,9 @@ class TableMoE:
             tile, slots, tile_expert, pair_slot = aligned
         cap = slots.shape[0]
         act = torch.empty(cap, s.ff, device=dev, dtype=h.dtype)
-        ops.expert_gemm(act, h, self.w_up, slots, tile_expert, tile, s.top, True, pairs=P)
+        ops.expert_gemm(act, h, self.w_up, slots, tile_expert, tile, s.top, True, pairs=P, tiles=P)
         y = torch.empty(cap, self.hidden, device=dev, dtype=h.dtype)
-        ops.expert_gemm(y, act, self.w_down, slots, tile_expert, tile, 0, False, pairs=P)
+        ops.expert_gemm(y, act, self.w_down, slots, tile_expert, tile, 0, False, pairs=P, tiles=P)
         return y, pair_slot
 
     def _packed_ok(self, h: torch.Tensor, P: int) -> bool:
@@ -1020,9 +1020,9 @@ class RoutedMoE:
         ops.route_align(ids, wts, slots, tile_expert, pair_slot, *router, nb, tile, *options)
         act = torch.empty(cap, s.ff, device=dev, dtype=h.dtype)
         # the gate and the pair's input weight in the epilogue
-        ops.expert_gemm(act, h, self.w_gu, slots, tile_expert, tile, s.top, self.epilogue, scale, s.limit, pairs=P)
+        ops.expert_gemm(act, h, self.w_gu, slots, tile_expert, tile, s.top, self.epilogue, scale, s.limit, pairs=P, tiles=P)
         ye = torch.empty(cap, self.hidden, device=dev, dtype=h.dtype)
-        ops.expert_gemm(ye, act, self.w_down, slots, tile_expert, tile, 0, 0, pairs=P)
+        ops.expert_gemm(ye, act, self.w_down, slots, tile_expert, tile, 0, 0, pairs=P, tiles=P)
         return ye, pair_slot, ids, wts, s.experts, h, self._shared(h)
 
     def _shared(self, h: torch.Tensor):

@@ -786,11 +786,12 @@ class KernelOps:
             assert table.dim() == 2, "the tables of several layers: small batches"
             self.moe_align(table.index_select(0, tokens).view(-1), E, tile, slots, tile_expert, pair_slot)
 
-    def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0, pairs=0):
+    def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0, pairs=0, tiles=0):
         """act: False / 0 none, True / 1 squared ReLU, 2: w = [gate rows; up rows], out = silu(gate) * up, 3: the same
         with the gate clamped at ``limit``; ``row_scale`` fp32 [pairs] multiplies each pair's product before it;
-        ``pairs``: how many (token, choice) pairs the tiles hold, where the caller knows (the choice of kernel)."""
-        self._moe_lib.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, int(act), row_scale, limit, pairs)
+        ``pairs``: how many (token, choice) pairs the tiles hold, where the caller knows (the choice of kernel); ``tiles``: the tiles in use are
+        among the first so many, as the alignments leave them with a pair in each (the rest is not launched)."""
+        self._moe_lib.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, int(act), row_scale, limit, pairs, tiles)
 
     # ---- norms before and after every sublayer (csrc/kernels/seq/sandwich.hip)
     def sandwich_update(self, out, residual, w_next, eps, y=None, w_post=None, mult=1.0, table=None):
@@ -969,7 +970,7 @@ class ReferenceOps:
     def moe_table_align(self, table, tokens, E, tile, slots, tile_expert, pair_slot):
         ref.moe_align(table.index_select(0, tokens).view(-1), E, tile, slots, tile_expert, pair_slot)
 
-    def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0, pairs=0):
+    def expert_gemm(self, out, x, w, slots, tile_expert, tile, gather_k, act, row_scale=None, limit=0.0, pairs=0, tiles=0):
         ref.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, int(act), row_scale, limit)
 
     def stream_update(self, out, dst, src, coef, w, eps, y1=None, y2=None):

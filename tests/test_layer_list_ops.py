@@ -1359,3 +1359,33 @@ def test_window_step_options(heads, kv, dim, ctxs, opts, dtype):
     assert torch.equal(c.cpu(), after)
     wrong = (out.double().cpu().view(n, heads, dim) - factor * want).abs() / (unit * factor * size)
     assert wrong.max() < 1, wrong.max()
+
+
+# ------------------------------------------------------------------ experts whose used tiles are known
+@gpu
+@pytest.mark.parametrize("E,top,N,K,T", [(16, 2, 1024, 2048, 1), (16, 2, 2048, 1024, 3), (4, 3, 40, 648, 5), (5, 2, 24, 640, 70), (8, 1, 264, 632, 9), (3, 2, 16, 1032, 120)])
+@pytest.mark.parametrize("act", [0, 1, 2])
+def test_expert_gemm_of_known_tiles(E, top, N, K, T, act):
+    """Tiles of one to 32 rows, as many as there are pairs launched at most; k and columns with remainders, choices that are no power of two, rows by slot."""
+    g = torch.Generator().manual_seed(E * N + T)
+    P, tile = T * top, 32
+    x = torch.randn(T, K, generator=g).bfloat16().cuda()
+    w = (torch.randn(E, N, K, generator=g) / K ** 0.5).bfloat16().cuda()
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(T)]).int().cuda()
+    ops, cap = get_ops("cuda"), -(-(P + E * (tile - 1)) // tile) * tile
+    slots, te, ps = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (cap, cap // tile, P))
+    ops.moe_align(ids.view(-1), E, tile, slots, te, ps)
+    y = torch.einsum("pk,pnk->pn", x.double().repeat_interleave(top, 0), w.double()[ids.view(-1).long()])
+    size = torch.einsum("pk,pnk->pn", x.double().abs().repeat_interleave(top, 0), w.double().abs()[ids.view(-1).long()])   # bounds the sums' rounding
+    if act == 1:
+        y, size = y.clamp(min=0) ** 2, 2 * y.abs() * size
+    if act == 2:
+        a, b = y.chunk(2, 1)
+        y, size = a * torch.sigmoid(a) * b, (2 * size[:, : N // 2] * b.abs() + size[:, N // 2:] * a.abs())
+    rows = torch.zeros(cap, K, dtype=torch.bfloat16, device="cuda")
+    rows[ps.long()] = x.repeat_interleave(top, 0)
+    for src, k in ((x, top), (rows, 0)):
+        for tiles in (0, P):
+            out = torch.full((cap, y.shape[1]), float("nan"), dtype=torch.bfloat16, device="cuda")
+            ops.expert_gemm(out, src, w, slots, te, tile, k, act, pairs=P, tiles=tiles)
+            assert ((out[ps.long()].double() - y).abs() <= 2.0 ** -8 * y.abs() + K * 2.0 ** -23 * size + 1e-30).all()
