@@ -16,22 +16,36 @@ namespace {
 constexpr int kD = 64;
 
 // w2 (LOW): [heads * 64, rank], rank a multiple of 32; the row's bottleneck lies behind the five parts of `proj`. Else wl is the product.
+// The sequence's numbers and the arguments that are no parameters of the first 14 words are asked for in one batch: 1 and
+// 16 rows of 32 heads with the bottleneck 3.75 -> 3.67, 6.62 -> 6.30 us in a loop.
+struct DeltaRuleRest {
+  void* out;
+  long out_ld;
+  const float *w0, *norm_w;
+  float eps, out_scale;
+};
 template <typename T, bool LOW>
 __global__ __launch_bounds__(256) void delta_rule_step_kernel(
-    T* __restrict__ out, long out_ld, float* __restrict__ S, const T* __restrict__ proj, long ld, const float* __restrict__ wl,
-    const float* __restrict__ a_b, const float* __restrict__ w0, const float* __restrict__ norm_w, const int* __restrict__ seq_cu,
-    const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads, float eps, float out_scale,
-    const T* __restrict__ w2, int rank) {
+    const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, const T* __restrict__ proj,
+    float* __restrict__ S, const void* __restrict__ low, int heads, int rank, const float* __restrict__ a_b, long ld, const DeltaRuleRest rest) {
   __shared__ float decay[LOW ? 4 : 1][kD];
   __shared__ __attribute__((aligned(16))) float chan[4][5][kD];   // [wave] w, a, u, k, r
   __shared__ __attribute__((aligned(16))) float sums[2][4][kD];   // x, o: [wave]
   const int h = blockIdx.x, s = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const long t = seq_cu[s];
-  if (seq_cu[s + 1] <= t) return;
+  const long t = seq_cu[s], after = seq_cu[s + 1];
+  const int ctx = seq_ctx[s], slot = seq_state[s];
+  const float *__restrict__ const w0 = rest.w0, *__restrict__ const norm_w = rest.norm_w;
+  const float eps = rest.eps, out_scale = rest.out_scale;
+  T* __restrict__ const out = static_cast<T*>(rest.out);
+  const long out_ld = rest.out_ld;
+  [[maybe_unused]] const T* __restrict__ const w2 = static_cast<const T*>(low);           // LOW
+  [[maybe_unused]] const float* __restrict__ const wl = static_cast<const float*>(low);   // not LOW
+  asm volatile("" ::"s"(t), "s"(after), "s"(ctx), "s"(slot), "s"(a_b), "s"(ld), "s"(w0), "s"(norm_w), "s"(eps), "s"(out_scale), "s"(out), "s"(out_ld));
+  if (after <= t) return;
   const int N = heads * kD, c = h * kD + lane, v0 = 4 * (tid & 15), k0 = 4 * (tid >> 4);
   const T* row = proj + t * ld;
-  float* Sp = S + (((long)seq_state[s] * heads + h) * kD + k0) * kD + v0;
-  const bool carried = seq_ctx[s] > 1;
+  float* Sp = S + (((long)slot * heads + h) * kD + k0) * kD + v0;
+  const bool carried = ctx > 1;
   f32x4 st[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) st[i] = carried ? *reinterpret_cast<const f32x4*>(Sp + i * kD) : f32x4{0.f, 0.f, 0.f, 0.f};
@@ -39,6 +53,7 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
 #pragma unroll
   for (int e = 0; e < 4; ++e) val[e] = ldf<T>(row, 2 * N + h * kD + v0 + e);
   const float k = ldf<T>(row, N + c), r = ldf<T>(row, c), a = ldf<T>(row, 3 * N + c), gate = ldf<T>(row, 4 * N + c);
+  const float w0_c = w0[c], a_b_c = a_b[c], norm_c = norm_w[c];
   float d = 0.f;
   if constexpr (LOW) {
     const int part = rank / 4, j0 = __builtin_amdgcn_readfirstlane(wave) * part;
@@ -58,8 +73,8 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
   }
   const float u = k / sqrtf(wave_sum(k * k) + 1e-6f);
   float(*mine)[kD] = chan[wave];
-  mine[0][lane] = expf(-0.60653065971263342f * sigmoid_f(d + w0[c]));
-  mine[1][lane] = sigmoid_f(a + a_b[c]) * u;
+  mine[0][lane] = expf(-0.60653065971263342f * sigmoid_f(d + w0_c));
+  mine[1][lane] = sigmoid_f(a + a_b_c) * u;
   mine[2][lane] = u;
   mine[3][lane] = k;
   mine[4][lane] = r;
@@ -90,7 +105,7 @@ __global__ __launch_bounds__(256) void delta_rule_step_kernel(
   if (wave != 0) return;
   const float o = (sums[1][0][lane] + sums[1][1][lane]) + (sums[1][2][lane] + sums[1][3][lane]);
   const float inv = out_scale / sqrtf(wave_sum(o * o) / (float)kD + eps);
-  stf<T>(out, t * out_ld + c, o * inv * norm_w[c] * sigmoid_f(gate));
+  stf<T>(out, t * out_ld + c, o * inv * norm_c * sigmoid_f(gate));
 }
 
 }  // namespace
@@ -103,8 +118,8 @@ void launch_delta_rule_step(void* out, long out_ld, float* S, const void* proj, 
   if (nseq <= 0) return;
   const dim3 grid(heads, nseq);
 #define HS_DRS(T, LOW)                                                                                                             \
-  delta_rule_step_kernel<T, LOW><<<grid, 256, 0, s>>>((T*)out, out_ld, S, (const T*)proj, ld, wl, a_b, w0, norm_w, seq_cu, seq_ctx, \
-                                                      seq_state, heads, eps, out_scale, (const T*)w2, rank)
+  delta_rule_step_kernel<T, LOW><<<grid, 256, 0, s>>>(seq_cu, seq_ctx, seq_state, (const T*)proj, S, LOW ? w2 : (const void*)wl, heads, rank, a_b, ld, \
+                                                      DeltaRuleRest{out, out_ld, w0, norm_w, eps, out_scale})
   if (f32) { if (w2 != nullptr) HS_DRS(float, true); else HS_DRS(float, false); }
   else if (w2 != nullptr) HS_DRS(unsigned short, true);
   else HS_DRS(unsigned short, false);
