@@ -10,7 +10,7 @@
 //
 // delta_chunk_prepare: everything that does not need the state, one workgroup per (head, chunk): A, P, the inverse
 // M = (1 + diag(beta) A)^-1 diag(beta) by forward substitution, and W = -M (G k), U0 = M v, G q, G_15 / G k, G_15.
-// delta_chunk_scan: one workgroup per (sequence, head, 32 value channels) walks the chunks: U = U0 + W S,
+// delta_chunk_scan: one workgroup per (sequence, head, 16 or 32 value channels) walks the chunks: U = U0 + W S,
 // o = (G q) S + P U, S = G_15 S + (G_15 / G k)^T U on mfma_f32_16x16x4f32. The state stays in registers in the
 // accumulators' layout, which is also the second operand's: lane (n, g) of a 16-row tile holds rows 4 g + r of column n,
 // and k step r of a product takes rows {4 g + r}.
@@ -231,20 +231,23 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
   }
 }
 
-// NW waves with TPW 16-row state tiles each, NC tiles of 16 value channels per workgroup. What a CU can take in (about 34 KB per us)
-// bounds it, so the operands of the state (W, G q, G_15 / G k) serve two tiles of channels, U0 is loaded by one wave per tile
-// and every wave does its share of the k steps of P U; the outputs are summed with the next chunk's exchange. 8192 rows (4
-// prompts) x 16 heads of 128 x 128: 219 us, of which the matrix instructions take half; one tile per workgroup with U0 and P in
-// every wave, two chunks ahead and an exit between them: 267 us.
+// NW waves with TPW 16-row state tiles each, NC tiles of 16 value channels per workgroup. U0 is loaded by one wave per tile, every wave does
+// its share of the k steps of P U, and the outputs are summed with the next chunk's exchange. What bounds it is the chain from chunk to
+// chunk: a wave's matrix instructions (50 of 32 cycles at 128 x 128 and two tiles, 0.67 us) and the exchange of W S through LDS, which
+// goes round while (G q) S runs; loads go out among the products, two chunks ahead (four: 184 us for 169). Prompts x tokens, 16 heads of
+// 128 x 128: 4 x 2048 197 -> 167 us, 6 x 1300 243 -> 169, 16 x 200 92 -> 59. One tile per workgroup where two leave CUs idle, and of smaller heads
+// always: 1 x 300 30 -> 16 us (two tiles: 25), 2 x 600 57 -> 30, 4 x 2048 of 64 x 64 128 -> 76 (103), of 32 x 32 122 -> 57 (87). A tile's U0 is
+// added in the same wave either way, so that the bits do not depend on it.
 // W S and P U are summed from 0, and U0 and (G q) S added to the sums: as the start of the sums they would make every product round
 // at their size (512 tokens, mean decay 0.47, against 64 bits: state 6.0e-8, with U0 as the start 1.1e-7; outputs 8.6e-8, 1.4e-7).
-constexpr int kAhead = 4;   // chunks in flight
+constexpr int kAhead = 2;   // chunks in flight
 template <int TPW, int NW, int NC>
-__global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
+__global__ __launch_bounds__(64 * NW, 2) void delta_chunk_scan_kernel(
     float* __restrict__ o, float* __restrict__ S, float* __restrict__ base, const int* __restrict__ seq_cu,
-    const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads, int dim, int vdim, int VP, long pad) {
+    const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads, int dim, int vdim, int VP) {
   constexpr int DP = 16 * TPW * NW, KPW = 4 / NW, RPW = 4 * NC / NW;   // k steps of P U and rows of the read-out per wave
-  static_assert((NW == 1 && NC == 1) || (NC == 2 && (NW == 2 || NW == 4)), "a wave per tile for U0, whole rows per wave");
+  static_assert(NW % NC == 0 && 4 * NC % NW == 0, "a wave per tile for U0, whole rows per wave");
+  static_assert(kAhead % 2 == 0, "a place of the ring has one parity");
   __shared__ __attribute__((aligned(16))) f32x4 sums[2][2][NC][NW][64];   // [chunk parity][U | the last chunk's o][tile][wave][lane]
   const int s = blockIdx.z, h = blockIdx.x, v0 = 16 * NC * blockIdx.y;
   const int r0 = seq_cu[s], n = seq_cu[s + 1] - r0;
@@ -253,32 +256,45 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
   for (int i = 0; i < s; ++i) first += (seq_cu[i + 1] - seq_cu[i] + kC - 1) / kC;
   const int nc = (n + kC - 1) / kC;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
+  const unsigned starts = NC == 1 ? blockIdx.y & 1 : 0;   // U0 of an even tile is added to the first wave's sums, of an odd one to the second's
   const bool odd = threadIdx.x & 64, high = threadIdx.x & 128;   // the wave's bits as lane masks: selects, not branches
   const int nv = heads * vdim, mine = wave % NC, row0 = (wave / NC) * RPW;
   const bool carried = seq_ctx[s] - n > 0;
   float* Sp = S + ((long)seq_state[s] * heads + h) * dim * vdim;
   f32x4 st[NC][TPW] = {};
   // Operands, each loaded kAhead chunks ahead as soon as its registers are free. Loads and stores of the loop are
-  // unconditional (past the end the last chunk is loaded again, rows and columns that do not exist are stored behind
-  // o), so that the wait for an operand never has to cover the younger loads behind it.
+  // unconditional (past the end the last chunk is loaded again, rows and columns that do not exist are outside the
+  // store's bounds), so that the wait for an operand never has to cover the younger loads behind it.
   struct Ops {
     f32x4 W[TPW], Q[TPW], K[TPW], E[TPW], U;
     float p[KPW];
   } ops[kAhead];
-  const unsigned u_at = (min(v0 / 16 + mine, VP / 16 - 1) * 64 + lane) * 4;
-  auto fetch = [&](Ops& x, int ci) {
-    const ChunkBuf b = chunk_buf(base, (long)(first + min(ci, nc - 1)) * heads + h, DP, VP);
+  const unsigned kE = 3 * kC * DP * 4, kU = kE + DP * 4, kP = kU + kC * VP * 4, bytes = kP + kC * kC * 4;   // where GE, UT, P start
+  const unsigned w_at = (wave * TPW * 64 + lane) * 16, e_at = kE + (16 * wave * TPW + 4 * g) * 4,
+                 u_at = kU + (min(v0 / 16 + mine, VP / 16 - 1) * 64 + lane) * 16, p_at = kP + (64 * wave * KPW + lane) * 4;
+  const char* next = reinterpret_cast<const char*>(base) + ((long)first * heads + h) * bytes;   // the next chunk to be loaded
+  int left = nc - 1;
+  auto from = [&] { return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(next), 0, bytes, 0x00020000); };
+  auto get = [&](unsigned at) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from(), at, 0, 0)); };
+  auto fetch = [&](Ops& x, int part) {
+    if (part == 0) {
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-      const unsigned k0 = 16 * (wave * TPW + i), at = ((wave * TPW + i) * 64 + lane) * 4;
-      x.W[i] = *reinterpret_cast<const f32x4*>(b.W + at);
-      x.Q[i] = *reinterpret_cast<const f32x4*>(b.GQ + at);
-      x.K[i] = *reinterpret_cast<const f32x4*>(b.KT + at);
-      x.E[i] = *reinterpret_cast<const f32x4*>(b.GE + k0 + 4 * g);
+      for (int i = 0; i < TPW; ++i) x.W[i] = get(w_at + 1024 * i);
+      x.U = get(u_at);
+    } else if (part == 1) {
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) {
+        x.Q[i] = get(kC * DP * 4 + w_at + 1024 * i);
+        x.E[i] = get(e_at + 64 * i);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < TPW; ++i) x.K[i] = get(2 * kC * DP * 4 + w_at + 1024 * i);
+#pragma unroll
+      for (int i = 0; i < KPW; ++i) x.p[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from(), p_at + 256 * i, 0, 0));
+      next += left > 0 ? (long)heads * bytes : 0;
+      --left;
     }
-    x.U = *reinterpret_cast<const f32x4*>(b.UT + u_at);
-#pragma unroll
-    for (int i = 0; i < KPW; ++i) x.p[i] = b.P[64 * (wave * KPW + i) + lane];
   };
   auto step_of = [&](const f32x4& v, int i) {   // the wave's i-th k step
     if constexpr (NW == 1) return v[i];
@@ -287,9 +303,7 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
   };
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 os[NC] = {};
-  float* po = o + (long)(r0 + 4 * g + row0) * nv + h * vdim + v0 + 16 * mine + c;
-  float* nowhere = o + pad + lane;
-  const unsigned rows = v0 + 16 * mine + c < vdim ? n : 0;
+  const unsigned out_at = v0 + 16 * mine + c < vdim ? ((4 * g + row0) * nv + h * vdim + v0 + 16 * mine + c) * 4 : 0x80000000u;
   // sum of the waves' parts, pairs first
   auto sum_of = [&](const f32x4* p) {
     if constexpr (NW == 1) return p[0];
@@ -297,43 +311,55 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
     else return (p[0] + p[64]) + (p[128] + p[192]);
   };
   auto read_out = [&](int ci, int buf) {   // the outputs of chunk ci from the sums in sums[buf]
+    const auto to = __builtin_amdgcn_make_buffer_rsrc(o + (long)(r0 + ci * kC) * nv, 0, (min(kC, n - ci * kC) & ~(ci >> 31)) * nv * 4, 0x00020000);
 #pragma unroll
     for (int e = 0; e < RPW; ++e) {
       float y = 0.f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) y += reinterpret_cast<const float*>(&sums[buf][1][mine][w][lane])[row0 + e];
-      float* to = po + (long)(ci * kC + e) * nv;
-      *((unsigned)(ci * kC + 4 * g + row0 + e) < rows ? to : nowhere) = y;
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, y), to, out_at + 4 * e * nv, 0, 0);
     }
   };
-  auto step = [&](Ops& x, int ci) {
-    const int buf = ci & 1;
+  auto step = [&](Ops& x, int ci, int buf) {
     f32x4 us[NC], qs[NC], u[NC];
 #pragma unroll
-    for (int t = 0; t < NC; ++t) {
-      us[t] = qs[t] = zero;
-      sums[buf][1][t][wave][lane] = os[t];
-    }
+    for (int t = 0; t < NC; ++t) us[t] = qs[t] = zero;
 #pragma unroll
     for (int b = 0; b < TPW; ++b)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int t = 0; t < NC; ++t) {
-          us[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.W[b][r], st[t][b][r], us[t], 0, 0, 0);
-          qs[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.Q[b][r], st[t][b][r], qs[t], 0, 0, 0);
-        }
+        for (int t = 0; t < NC; ++t) us[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.W[b][r], st[t][b][r], us[t], 0, 0, 0);
 #pragma unroll
-    for (int t = 0; t < NC; ++t) {
-      sums[buf][0][t][wave][lane] = us[t] + (NC == 1 || (!high && odd == t) ? x.U : zero);
+    for (int t = 0; t < NC; ++t) sums[buf][1][t][wave][lane] = os[t];
+    __builtin_amdgcn_sched_barrier(0);
+    auto queries = [&](int b, int r) {
+#pragma unroll
+      for (int t = 0; t < NC; ++t) qs[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.Q[b][r], st[t][b][r], qs[t], 0, 0, 0);
+    };
+    queries(0, 0);
+    queries(0, 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < NC; ++t) sums[buf][0][t][wave][lane] = us[t] + (NW == 1 || (!high && odd == (starts + t)) ? x.U : zero);
+    fetch(x, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    queries(0, 2);
+    queries(0, 3);
+#pragma unroll
+    for (int b = 1; b < TPW; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) queries(b, r);
+#pragma unroll
+    for (int t = 0; t < NC; ++t)
 #pragma unroll
       for (int b = 0; b < TPW; ++b) st[t][b] *= x.E[b];
-    }
+    fetch(x, 1);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();   // the other parity's rows are read before a wave comes here again
 #pragma unroll
-    for (int t = 0; t < NC; ++t) {
-      u[t] = sum_of(&sums[buf][0][t][0][lane]);
-    }
+    for (int t = 0; t < NC; ++t) u[t] = sum_of(&sums[buf][0][t][0][lane]);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -347,11 +373,13 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
       for (int i = 0; i < KPW; ++i) os[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.p[i], step_of(u[t], i), os[t], 0, 0, 0);
       os[t] += qs[t];
     }
-    fetch(x, ci + kAhead);
+    fetch(x, 2);
     read_out(ci - 1, buf);
+    __builtin_amdgcn_sched_barrier(0);
   };
 #pragma unroll
-  for (int i = 0; i < kAhead; ++i) fetch(ops[i], i);
+  for (int i = 0; i < kAhead; ++i)
+    for (int part = 0; part < 3; ++part) fetch(ops[i], part);
   // The carried state, rows and columns that do not exist as zeros of a place that does: a branch for each element came with a wait for the one
   // before (200 sequences of one row x 16 heads in a step, all kernels of the rule, 792 -> 638 us; 50 of 64 rows 287 -> 258).
   if (carried) {
@@ -372,13 +400,14 @@ __global__ __launch_bounds__(64 * NW) void delta_chunk_scan_kernel(
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the loop's own waits then count the loop's loads only
   int ci = 0;
+#pragma nounroll
   for (; ci + kAhead <= nc; ci += kAhead) {   // no exit in between: a wait would cover the loads of the shortest way round
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) step(ops[i], ci + i);
+    for (int i = 0; i < kAhead; ++i) step(ops[i], ci + i, i & 1);
   }
 #pragma unroll
   for (int i = 0; i < kAhead - 1; ++i)
-    if (ci + i < nc) step(ops[i], ci + i);
+    if (ci + i < nc) step(ops[i], ci + i, i & 1);
 #pragma unroll
   for (int t = 0; t < NC; ++t) sums[nc & 1][1][t][wave][lane] = os[t];
   __syncthreads();
@@ -410,7 +439,7 @@ void launch_delta_chunk(float* o, float* S, float* buf, const float* qk, const f
                         const float* bb, const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int T,
                         int heads, int kv_heads, int dim, int vdim, bool channel, hipStream_t s) {
   const int VP = (vdim + 15) / 16 * 16;
-  dim3 pgrid(heads, delta_chunk_bound(T, nseq)), sgrid(heads, (VP + 31) / 32, nseq), sgrid1(heads, VP / 16, nseq);
+  dim3 pgrid(heads, delta_chunk_bound(T, nseq));
 #define HS_DC(DS, TPW, NW, NC)                                                                                             \
   do {                                                                                                                 \
     if (channel)                                                                                                       \
@@ -419,14 +448,16 @@ void launch_delta_chunk(float* o, float* S, float* buf, const float* qk, const f
     else                                                                                                               \
       delta_chunk_prepare_kernel<DS, false><<<pgrid, 256, 0, s>>>(buf, qk, vv, gg, bb, seq_cu, nseq, heads, kv_heads, dim, \
                                                                   vdim, VP);                                           \
-    delta_chunk_scan_kernel<TPW, NW, NC><<<NC == 1 ? sgrid1 : sgrid, 64 * NW, 0, s>>>(o, S, buf, seq_cu, seq_ctx, seq_state, heads, dim, vdim, VP,  \
-                                                               (long)T * heads * vdim);                                \
+    delta_chunk_scan_kernel<TPW, NW, NC><<<dim3(heads, (VP + 16 * NC - 1) / (16 * NC), nseq), 64 * NW, 0, s>>>(            \
+        o, S, buf, seq_cu, seq_ctx, seq_state, heads, dim, vdim, VP);                                                      \
   } while (0)
   switch (padded(dim)) {
     case 16: HS_DC(1, 1, 1, 1); break;
-    case 32: HS_DC(2, 1, 2, 2); break;
-    case 64: HS_DC(4, 1, 4, 2); break;
-    default: HS_DC(8, 2, 4, 2); break;
+    case 32: HS_DC(2, 1, 2, 1); break;
+    case 64: HS_DC(4, 1, 4, 1); break;
+    default:
+      if (heads * ((VP + 31) / 32) * nseq < 256) HS_DC(8, 2, 4, 1);
+      else HS_DC(8, 2, 4, 2);   // two tiles per workgroup where such workgroups are one per CU
   }
 #undef HS_DC
 }

@@ -9,7 +9,7 @@
 // at least 6e-5: the inner ratios are quotients of products from the chunk's start, and the matrix cores form all pairs.
 //
 // delta_rule_chunk_prepare: all that does not need the state, one workgroup per (head, chunk), straight from the projection.
-// delta_rule_chunk_scan: one workgroup per (sequence, head, 32 value channels) walks the chunks as in delta_chunk.hip, with
+// delta_rule_chunk_scan: one workgroup per (sequence, head, 16 or 32 value channels) walks the chunks as in delta_chunk.hip, with
 // U = -X: U = U0 + W S (W = -(1 + A)^-1 U), O = R S + Pa U + Pk V, S = E S + KA U + KK V.
 // A product over the chunk would carry a NaN or an infinity of one token's inputs to the tokens before it (0 times it), so such
 // inputs take part as zeros, and where a chunk has some the scan ends with a walk that writes NaN: to the outputs of a token whose r
@@ -17,7 +17,7 @@
 // whose k is not finite or a pre-activation of which is NaN (infinite ones saturate).
 // What bounds it: the prepared operands (6816 floats per head and chunk) are written and read once, and the scan's products.
 // 8192 rows (4 prompts) x 32 heads: rows prepared one by one and scanned token by token (five row vectors through LDS for
-// every 4 state elements of a lane) took 126 + 700 us; this 190 + 204.
+// every 4 state elements of a lane) took 126 + 700 us; this 177 + 144.
 // Errors against 64 bits, over 32 .. 2048 tokens, fresh and carried states, strong and weak decays: state 5.8e-8 - 6.4e-8 (token by
 // token 6.3e-8 - 7.0e-8), outputs before their norm 7.2e-8 - 7.9e-8 (9.2e-8 - 9.8e-8). What it takes: decays and their products
 // in 64 bits, rounded once into the operands (else 7.9e-8 for the state); Pa and Pk summed in 64 bits and the larger part of an output added
@@ -269,15 +269,21 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
   *reinterpret_cast<f32x4*>(out.V + col * kC + 4 * g) = v;
 }
 
-// Four waves with 16 state rows each, kTiles tiles of 16 value channels. What a CU can take in (about 34 KB per us) bounds it, so
-// nothing but the wave's own rows is loaded: wave 0 and 1 load U0 of a tile (the start of their sums), 2 and 3 V, which
-// goes round with the sums; each does one of the four k steps of Pa U and Pk V, and the outputs are summed with the next
-// chunk's exchange. 16 channels per workgroup with U0, V, Pa and Pk in every wave: 249 us.
-constexpr int kNW = 4, kTiles = 2, kAhead = 4;   // kAhead: chunks in flight
-__global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
+// Four waves with 16 state rows each, kTiles tiles of 16 value channels. Nothing but the wave's own rows is loaded: of U0 (the start of
+// a tile's sums) and V each one tile per wave, which goes round with the sums; each wave does one of the four k steps of Pa U and Pk V, and
+// the outputs are summed with the next chunk's exchange. What bounds it is the chain from chunk to chunk: 36 matrix instructions of
+// a wave's own (0.5 us), the exchange of W S through LDS, and the loads' way into the CU. So W S comes first and goes round
+// while R S and KK V run, V is exchanged a chunk early, loads go out among the products, and two chunks ahead are enough (four: 256
+// registers and 146 us). 4 prompts of 2048 x 32 heads: 186 -> 144 us, 6 of 1300: 225 -> 142, 16 of 200: 83 -> 53.
+// One tile per workgroup where two leave CUs idle: 1 prompt of 300 26 -> 15 us (two tiles: 21), 2 of 600 50 -> 27, 4 of 2048 166. A tile's
+// sums start in the same wave either way, so that the bits do not depend on it.
+constexpr int kNW = 4, kAhead = 2;   // kAhead: chunks in flight
+template <int kTiles>
+__global__ __launch_bounds__(64 * kNW, 2) void delta_rule_chunk_scan_kernel(
     float* __restrict__ o, float* __restrict__ S, float* __restrict__ base, const int* __restrict__ seq_cu,
-    const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads, long pad) {
-  static_assert(kNW == 2 * kTiles, "U0 and V: a wave per tile each");
+    const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads) {
+  static_assert(kNW == 4 && kTiles <= 2, "U0 and V: a wave per tile each");
+  static_assert(kAhead % 2 == 0, "a place of the ring has one parity");
   __shared__ __attribute__((aligned(16))) f32x4 sums[2][2][kTiles][kNW][64];   // [chunk parity][U | the last chunk's O]
   __shared__ __attribute__((aligned(16))) f32x4 vals[2][kNW][64];              // [chunk parity] U0, V
   const int s = blockIdx.z, h = blockIdx.x;
@@ -288,121 +294,158 @@ __global__ __launch_bounds__(64 * kNW) void delta_rule_chunk_scan_kernel(
   const int nc = (n + kC - 1) / kC;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
   const bool odd = threadIdx.x & 64, high = threadIdx.x & 128;   // the wave's bits as lane masks: selects, not branches
-  const int N = heads * kD, k0 = 16 * wave, col0 = 16 * kTiles * blockIdx.y, mine = wave & 1, half = wave >> 1;
+  const int N = heads * kD, k0 = 16 * wave, col0 = 16 * kTiles * blockIdx.y, half = wave >> 1;
+  const int mine = kTiles == 2 ? wave & 1 : 0, row0 = kTiles == 2 ? 2 * half : wave;
+  const unsigned starts = kTiles == 2 ? 0 : blockIdx.y & 1;   // a tile's sums start with U0 in wave (column / 16) % 2
   const bool carried = seq_ctx[s] - n > 0;
   float* Sp = S + ((long)seq_state[s] * heads + h) * kD * kD + col0 + c;
-  f32x4 st[kTiles];
+  f32x4 st[kTiles] = {};
+  if (carried)
 #pragma unroll
-  for (int t = 0; t < kTiles; ++t)
+    for (int t = 0; t < kTiles; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) st[t][r] = carried ? Sp[(long)(k0 + 4 * g + r) * kD + 16 * t] : 0.f;
+      for (int r = 0; r < 4; ++r) st[t][r] = Sp[(k0 + 4 * g + r) * kD + 16 * t];
   // Operands, each loaded kAhead chunks ahead as soon as its registers are free. The loop's loads and stores are unconditional
-  // (past the end the last chunk again, rows that do not exist behind o), so that the wait for an operand never covers the
-  // younger loads behind it.
+  // (past the end the last chunk again, rows that do not exist outside the store's bounds), so that the wait for an operand never
+  // covers the younger loads behind it.
   struct Ops {
     f32x4 W, R, KA, KK, E, X;
-    float pa, pk, any;
+    float pa, pk;
   } ops[kAhead];
-  constexpr unsigned kM = kC * kD * sizeof(float);   // bytes of an operand of the buffer
-  const unsigned rows = (c * kD + k0 + 4 * g) * 4, cols = ((k0 + c) * kC + 4 * g) * 4, states = (k0 + 4 * g) * 4,
-                 vals_at = (4 + half) * kM + ((col0 + 16 * mine + c) * kC + 4 * g) * 4, pair = (64 * wave + lane) * 4;
-  auto fetch = [&](Ops& x, int ci) {
-    const char* p = reinterpret_cast<const char*>(base + ((long)(first + min(ci, nc - 1)) * heads + h) * kBuf);
-    auto get = [&](unsigned at) { return *reinterpret_cast<const f32x4*>(p + at); };
-    auto one = [&](unsigned at) { return *reinterpret_cast<const float*>(p + at); };
-    constexpr unsigned kE = 6 * kM, kP = kE + kD * 4, kAny = kP + (2 * kC * kC + kC + kD) * 4;
-    x.W = get(rows);
-    x.R = get(kM + rows);
-    x.X = get(vals_at);
-    x.KK = get(3 * kM + cols);
-    x.KA = get(2 * kM + cols);
-    x.E = get(kE + states);
-    x.pa = one(kP + pair);
-    x.pk = one(kP + kC * kC * 4 + pair);
-    x.any = one(kAny);
+  constexpr unsigned kM = kC * kD * sizeof(float), kE = 6 * kM, kP = kE + kD * 4;   // bytes of an operand, where E and Pa start
+  const unsigned rows = (c * kD + k0 + 4 * g) * 4, cols = ((k0 + c) * kC + 4 * g) * 4, states = kE + (k0 + 4 * g) * 4,
+                 vals_at = (4 + half) * kM + ((col0 + 16 * mine + c) * kC + 4 * g) * 4, pair = kP + (64 * wave + lane) * 4;
+  const long stride = heads * kBuf * (long)sizeof(float);
+  const char* chunks = reinterpret_cast<const char*>(base + ((long)first * heads + h) * kBuf);
+  const char* next = chunks;   // the next chunk to be loaded
+  int left = nc - 1;
+  auto from = [&] { return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(next), 0, kBuf * (int)sizeof(float), 0x00020000); };
+  auto get = [&](unsigned at) { return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from(), at, 0, 0)); };
+  auto one = [&](unsigned at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from(), at, 0, 0)); };
+  auto fetch = [&](Ops& x, int part) {
+    if (part == 0) { x.W = get(rows); x.X = get(vals_at); }
+    if (part == 1) { x.R = get(kM + rows); x.E = get(states); }
+    if (part == 2) x.KK = get(3 * kM + cols);
+    if (part == 3) {
+      x.KA = get(2 * kM + cols);
+      x.pa = one(pair);
+      x.pk = one(kC * kC * 4 + pair);
+      next += left > 0 ? stride : 0;
+      --left;
+    }
   };
   auto of_wave = [&](const f32x4& v) { return high ? (odd ? v[3] : v[2]) : odd ? v[1] : v[0]; };
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 os[kTiles] = {};
-  float any = 0.f;   // 1 once a token's inputs were not finite
-  float* po = o + (long)(r0 + 8 * half + g) * N + h * kD + col0 + 16 * mine + c;
-  float* nowhere = o + pad + lane;
-  // the outputs of chunk ci from the sums in sums[buf]: wave w two rows of tile w % 2
+  f32x4 os[kTiles] = {}, v[kTiles];
+  float vr[kTiles];   // the wave's k step of v
+  // the outputs of chunk ci from the sums in sums[buf]: every wave kTiles rows of four
+  const unsigned out_at = ((4 * row0 + g) * N + h * kD + col0 + 16 * mine + c) * 4;
   auto read_out = [&](int ci, int buf) {
-    float2 v[kNW];
+    float x[kNW][kTiles];
 #pragma unroll
-    for (int w = 0; w < kNW; ++w) v[w] = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(&sums[buf][1][mine][w][lane]) + 2 * half);
-    const float y[2] = {(v[0].x + v[1].x) + (v[2].x + v[3].x), (v[0].y + v[1].y) + (v[2].y + v[3].y)};
+    for (int w = 0; w < kNW; ++w)
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const int i = ci * kC + 8 * half + 4 * e + g;
-      float* to = po + (long)(ci * kC + 4 * e) * N;
-      *((unsigned)i < (unsigned)n ? to : nowhere) = y[e];
-    }
+      for (int e = 0; e < kTiles; ++e) x[w][e] = reinterpret_cast<const float*>(&sums[buf][1][mine][w][lane])[row0 + e];
+    const auto to = __builtin_amdgcn_make_buffer_rsrc(o + (long)(r0 + ci * kC) * N, 0, (min(kC, n - ci * kC) & ~(ci >> 31)) * N * 4, 0x00020000);
+#pragma unroll
+    for (int e = 0; e < kTiles; ++e)
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (x[0][e] + x[1][e]) + (x[2][e] + x[3][e])), to, out_at + 16 * e * N, 0, 0);
   };
-  auto step = [&](Ops& x, int ci) {
-    const int buf = ci & 1;
-    f32x4 us[kTiles], u[kTiles], v[kTiles], rs[kTiles] = {};
+  auto step = [&](Ops& x, const Ops& y, int ci, int buf) {
+    f32x4 us[kTiles], u[kTiles], rs[kTiles] = {}, sa[kTiles] = {};
+    float pv[kTiles];
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      us[t] = !high && odd == t ? x.X : zero;
-      sums[buf][1][t][wave][lane] = os[t];
-    }
-    vals[buf][wave][lane] = x.X;
+    for (int t = 0; t < kTiles; ++t) pv[t] = vr[t];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) us[t] = !high && odd == (starts + t) ? x.X : zero;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int t = 0; t < kTiles; ++t) {
-        us[t] = mfma(x.W[r], st[t][r], us[t]);
-        rs[t] = mfma(x.R[r], st[t][r], rs[t]);
-      }
+      for (int t = 0; t < kTiles; ++t) us[t] = mfma(x.W[r], st[t][r], us[t]);
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      sums[buf][0][t][wave][lane] = us[t];
-      st[t] *= x.E;
-    }
-    __syncthreads();   // the other parity's rows are read before a wave comes here again
+    for (int t = 0; t < kTiles; ++t) sums[buf][1][t][wave][lane] = os[t];
+    vals[buf ^ 1][wave][lane] = y.X;   // the next chunk's
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      v[t] = vals[buf][kTiles + t][lane];
-      u[t] = sums[buf][0][t][0][lane];
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
-      for (int w = 1; w < kNW; ++w) u[t] += sums[buf][0][t][w][lane];
-    }
+      for (int t = 0; t < kTiles; ++t) rs[t] = mfma(x.R[r], st[t][r], rs[t]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) sums[buf][0][t][wave][lane] = us[t];
+    fetch(x, 0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 2; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < kTiles; ++t) rs[t] = mfma(x.R[r], st[t][r], rs[t]);
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) st[t] *= x.E;
+    fetch(x, 1);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int t = 0; t < kTiles; ++t) st[t] = mfma(x.KK[r], v[t][r], st[t]);
-    f32x4 sa[kTiles] = {};
+    fetch(x, 2);
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();   // the other parity's rows are read before a wave comes here again
+    f32x4 part[kTiles][kNW];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t)
+#pragma unroll
+      for (int w = 0; w < kNW; ++w) part[t][w] = sums[buf][0][t][w][lane];
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      u[t] = part[t][0];
+#pragma unroll
+      for (int w = 1; w < kNW; ++w) u[t] += part[t][w];
+    }
+#pragma unroll
+    for (int t = 0; t < kTiles; ++t) {
+      v[t] = vals[buf ^ 1][2 + t][lane];
+      vr[t] = reinterpret_cast<const float*>(&vals[buf ^ 1][2 + t][lane])[wave];
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int t = 0; t < kTiles; ++t) sa[t] = mfma(x.KA[r], u[t][r], sa[t]);
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) st[t] += sa[t];
-#pragma unroll
     for (int t = 0; t < kTiles; ++t) {
       os[t] = mfma(x.pa, of_wave(u[t]), rs[t]);   // the larger part last: its roundings are the outputs'
-      os[t] = mfma(x.pk, of_wave(v[t]), os[t]);
+      os[t] = mfma(x.pk, pv[t], os[t]);
     }
-    any = fmaxf(any, x.any);
-    fetch(x, ci + kAhead);
+    fetch(x, 3);
     read_out(ci - 1, buf);
-  };
 #pragma unroll
-  for (int i = 0; i < kAhead; ++i) fetch(ops[i], i);
+    for (int t = 0; t < kTiles; ++t) st[t] += sa[t];
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // 1 if a token's inputs were not finite
+  float any = 0.f;
+  for (int ci = threadIdx.x; ci < nc; ci += 64 * kNW) any = fmaxf(any, *reinterpret_cast<const float*>(chunks + ci * stride + kP + (2 * kC * kC + kC + kD) * 4));
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) for (int part = 0; part < 4; ++part) fetch(ops[i], part);
   __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0): the loop's own waits then count the loop's loads only
+  vals[0][wave][lane] = ops[0].X;
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < kTiles; ++t) {
+    v[t] = vals[0][2 + t][lane];
+    vr[t] = reinterpret_cast<const float*>(&vals[0][2 + t][lane])[wave];
+  }
   int ci = 0;
+#pragma nounroll
   for (; ci + kAhead <= nc; ci += kAhead) {   // no exit in between: a wait would cover the loads of the shortest way round
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) step(ops[i], ci + i);
+    for (int i = 0; i < kAhead; ++i) step(ops[i], ops[(i + 1) % kAhead], ci + i, i & 1);
   }
 #pragma unroll
   for (int i = 0; i < kAhead - 1; ++i)
-    if (ci + i < nc) step(ops[i], ci + i);
+    if (ci + i < nc) step(ops[i], ops[i + 1], ci + i, i & 1);
 #pragma unroll
   for (int t = 0; t < kTiles; ++t) sums[nc & 1][1][t][wave][lane] = os[t];
-  __syncthreads();
+  any = __syncthreads_or(any != 0.f);
   read_out(nc - 1, nc & 1);
 #pragma unroll
   for (int t = 0; t < kTiles; ++t)
@@ -436,8 +479,9 @@ void launch_delta_rule_chunk(float* o, float* S, float* buf, const void* proj, l
                              int heads, hipStream_t s) {
   delta_rule_chunk_prepare_kernel<<<dim3(heads, T / kC + nseq), 256, 0, s>>>(buf, (const unsigned short*)proj, ld, wl, a_b, w0,
                                                                              seq_cu, nseq, heads);
-  delta_rule_chunk_scan_kernel<<<dim3(heads, kD / (16 * kTiles), nseq), 64 * kNW, 0, s>>>(o, S, buf, seq_cu, seq_ctx, seq_state, heads,
-                                                                               (long)T * heads * kD);
+  const bool few = heads * (kD / 32) * nseq < 256;   // two tiles per workgroup where such workgroups are one per CU
+  (few ? delta_rule_chunk_scan_kernel<1> : delta_rule_chunk_scan_kernel<2>)<<<dim3(heads, kD / (few ? 16 : 32), nseq), 64 * kNW, 0, s>>>(
+      o, S, buf, seq_cu, seq_ctx, seq_state, heads);
 }
 
 }  // namespace hipserve

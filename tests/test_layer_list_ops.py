@@ -1043,6 +1043,41 @@ def test_delta_rule_chunks_not_finite(row, what, value):
 
 
 @gpu
+@pytest.mark.parametrize("rule,heads,vdim", [("gated", 16, 128), ("gated", 13, 100), ("generalized", 32, 64)])
+def test_delta_chunks_of_one_and_two_tiles(rule, heads, vdim):
+    """Eight sequences in one step (two tiles of value channels per workgroup) and each by itself (one): the same bits; the last rows of a
+    sequence's last chunk, and columns past a tile's end, belong to others."""
+    g = torch.Generator().manual_seed(heads)
+    lens, dim = [33, 1, 16, 50, 64, 17, 5, 100], 128 if rule == "gated" else 64
+    T, n, N, nq = sum(lens), len(lens), heads * vdim, heads * dim
+    cols = 2 * nq + N
+    delta = get_ops("cuda")._delta
+    proj = torch.randn(T, cols + 2 * heads + N if rule == "gated" else 5 * N, generator=g).bfloat16().cuda()
+    wl, conv, S0 = torch.randn(T, N, generator=g).cuda(), torch.randn(cols, 4, generator=g).cuda(), torch.randn(n, heads, dim, vdim, generator=g).cuda()
+    a, b, nw = (torch.randn(max(heads, N), generator=g).cuda() for _ in range(3))
+    start = [0] + torch.tensor(lens).cumsum(0).tolist()
+
+    def run(first, last):
+        rows, m = slice(start[first], start[last]), last - first
+        t, state, out = start[last] - start[first], S0[first:last].clone(), torch.empty(start[last] - start[first], N, dtype=torch.bfloat16, device="cuda")
+        cu = torch.tensor([c - start[first] for c in start[first:last + 1]]).int().cuda()
+        ctx, slots = torch.tensor([k + (i % 2) for i, k in enumerate(lens)][first:last]).int().cuda(), torch.arange(m).int().cuda()
+        if rule == "gated":
+            scratch, chunks = torch.empty(t * (2 * nq + 2 * N + 2 * heads) + 64, device="cuda"), torch.empty(delta.delta_chunk_floats(t, m, heads, dim, vdim), device="cuda")
+            delta.gated_delta(out, state, torch.zeros(m, 3, cols, device="cuda"), proj[rows], conv, a[:heads], b[:heads], nw[:vdim], None, None, cu, ctx, slots,
+                              scratch, heads, heads, dim, vdim, 4, 1e-6, cols + heads, cols + 2 * heads, cols, False, True, chunks)
+        else:
+            scratch, chunks = torch.empty(t * N + 64, device="cuda"), torch.empty(delta.delta_rule_chunk_floats(proj[rows], m, heads, dim), device="cuda")
+            delta.delta_rule(out, state, proj[rows], wl[rows], a, b, nw, cu, ctx, slots, scratch, heads, dim, 1e-6, 1.0, chunks)
+        return out, state
+    out, state = run(0, n)
+    for i in range(n):
+        alone, its = run(i, i + 1)
+        assert torch.equal(alone, out[start[i]:start[i + 1]]) and torch.equal(its, state[i:i + 1]), i
+    assert out.isfinite().all()
+
+
+@gpu
 @pytest.mark.parametrize("lens,dim,vdim,a,carried", [([40, 33], 128, 128, 0.0, False), ([300], 128, 128, -2.0, True), ([200], 64, 48, -1.0, True), ([100, 64], 32, 64, 0.0, False)])
 def test_gated_delta_chunks_precision(lens, dim, vdim, a, carried):
     """States and outputs of the chunked gated rule beside the scan's, both against 64 bits from the same prepared rows."""
