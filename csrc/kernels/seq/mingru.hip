@@ -4,10 +4,13 @@
 // all in fp32, from the sequence's state slot (zero when the step starts at position 0) and back
 // into it. A workgroup owns 64 channels of one sequence. Its waves hold 16 consecutive rows each: a wave folds its rows into
 // (A, B) with S_out = A S_in + B, the waves' pairs are chained through LDS, and the rows are replayed from their true S_in.
-// z and z c stay in registers in between: the arithmetic (three sigmoids per element, about 90 instruction slots) bounds
-// it, so nothing is computed twice. Waves that fold and then replay one long segment each, reading z and x again, with
-// sigmoids from a full division: 171 us for 8192 rows (4 prompts) x 4096 in bf16, now 100. Two launches over segments of
-// 64 rows (fold, replay; 4 channels per thread) fill the card whatever the sequences are, but compute z and c twice: 188.
+// 1 - z and z c stay in registers in between: the arithmetic (three sigmoids per element, 60 instructions in all) and, in 32 bits, the
+// bytes bound it. Nothing is computed twice, rows are addressed by buffers whose bounds stand for the last block's missing rows
+// and the columns past the width, and the next block's rows are loaded while this one's are folded and replayed. 8192 rows (4 prompts)
+// x 4096 in bf16: with 64-bit addresses, a branch per element and loads at the head of the block (110 instructions) 95 us, now 71 (float32 112, 115:
+// 4.7 TB/s); 7 prompts, 8100 rows x 8192 223 -> 176 (241 -> 231), 700 rows x 4096 29.7 -> 23.3. Waves that fold and then replay one long
+// segment each, reading z and x again: 171 us. Two launches over segments of 64 rows (fold, replay; 4 channels per
+// thread) fill the card whatever the sequences are, but compute z and c twice: 188. z and x loaded in turns: 74.
 //
 // Decode steps (mingru_step): one row per sequence needs no folding; 4 channels per thread, 9.1 -> 5.0 us for 41 sequences. Up to 64 of
 // them run in the epilogue of the product that makes z, x and g (mingru_product): a workgroup has all three of its 16 channels,
@@ -25,23 +28,35 @@ namespace {
 constexpr int kMaxWaves = 16, kRows = 16;   // waves of a workgroup; rows that a wave holds at a time
 
 struct Gru {
-  float z, zc;   // S <- (1 - z) S + zc
+  float keep, zc;   // S <- keep S + zc, keep = 1 - z
   HS_DEVICE Gru() {}
   HS_DEVICE Gru(float zp, float xp, float bz, float bx) {
-    z = sigmoid_f(zp + bz);
+    const float z = sigmoid_f(zp + bz);
+    keep = 1.f - z;
     const float u = xp + bx;
-    zc = z * (u >= 0.f ? u + 0.5f : sigmoid_f(u));
+    float e;
+    const float r = sigmoid_of_abs(u, e);
+    zc = z * (u >= 0.f ? u + 0.5f : e * r);
   }
 };
+
+// A number of a row as it is in memory, a register each: packed in pairs, they would be waited for where they are loaded.
+template <typename T>
+HS_DEVICE unsigned ld_raw(__amdgpu_buffer_rsrc_t from, unsigned at) {
+  if constexpr (sizeof(T) == 4) return __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0);
+  else return __builtin_amdgcn_raw_buffer_load_b16(from, at, 0, 0);
+}
+template <typename T>
+HS_DEVICE float of_raw(unsigned x) { return __builtin_bit_cast(float, sizeof(T) == 4 ? x : x << 16); }
 
 template <typename T>
 __global__ __launch_bounds__(64 * kMaxWaves) void mingru_scan_kernel(
     T* __restrict__ y, float* __restrict__ state, const T* __restrict__ proj, const float* __restrict__ b_z,
     const float* __restrict__ b_x, const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx,
     const int* __restrict__ seq_state, int width) {
-  __shared__ float sa[2][kMaxWaves][64], sb[2][kMaxWaves][64];
+  __shared__ float2 fold[2][kMaxWaves][64];
   const int s = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
   const int c = blockIdx.y * 64 + lane;
   const int r0 = seq_cu[s], n = seq_cu[s + 1] - r0;
   if (n <= 0) return;
@@ -49,49 +64,70 @@ __global__ __launch_bounds__(64 * kMaxWaves) void mingru_scan_kernel(
   const int cc = live ? c : 0;
   const float bz = b_z[cc], bx = b_x[cc];
   const long ld = 3L * width, slot = (long)seq_state[s] * width + cc;
+  const unsigned at0 = live ? c * sizeof(T) : 0x80000000u;   // outside every row
   // every wave reads the carried state before the first barrier; the slot is rewritten only after the last, by the wave that
   // replays the last row (the chained pairs round once more: 5.3e-8 from 64 bits instead of 5.0e-8 after 2048 rows)
   float last = 0.f;
   bool holds = false;
   float S = (seq_ctx[s] - n > 0) ? state[slot] : 0.f;
-  for (int b0 = 0, buf = 0; b0 < n; b0 += nw * kRows, buf ^= 1) {
-    const int a = b0 + wave * kRows, rows = min(kRows, n - a);   // of this wave; none or fewer in the last block
-    Gru g[kRows];
-    float gp[kRows], A = 1.f, B = 0.f;
-    if (rows > 0) {
-      float zp[kRows], xp[kRows];
+  // The wave's rows of the next block are loaded while this one is replayed; rows that do not exist are outside the buffers.
+  auto rows_of = [&](int b0) { return min(kRows, n - b0 - wave * kRows); };
+  unsigned zp[kRows], xp[kRows], gp[kRows];
+  auto load = [&](unsigned* to, int b0, int which) {
+    const int rows = rows_of(b0);
+    const auto from = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(proj) + (long)(r0 + b0 + wave * kRows) * ld + (long)which * width, 0,
+                                                        rows > 0 ? ((rows - 1) * 3 + 1) * width * (int)sizeof(T) : 0, 0x00020000);
+    unsigned at = at0;
 #pragma unroll
-      for (int i = 0; i < kRows; ++i) {
-        const long base = (long)(r0 + a + min(i, rows - 1)) * ld + cc;
-        zp[i] = ldf<T>(proj, base);
-        xp[i] = ldf<T>(proj, base + width);
-        gp[i] = ldf<T>(proj, base + 2 * width);
+    for (int i = 0; i < kRows; ++i, at += 3 * width * sizeof(T)) to[i] = ld_raw<T>(from, at);
+  };
+  load(zp, 0, 0);
+  load(xp, 0, 1);
+  load(gp, 0, 2);
+#pragma nounroll
+  for (int b0 = 0, buf = 0; b0 < n; b0 += nw * kRows, buf ^= 1) {
+    const int rows = rows_of(b0);   // of this wave; none or fewer in the last block
+    Gru g[kRows];
+    float A = 1.f, B = 0.f;
+    if (rows > 0) {
+#pragma unroll
+      for (int i = 0; i < kRows; ++i) g[i] = Gru(of_raw<T>(zp[i]), of_raw<T>(xp[i]), bz, bx);
+      if (rows < kRows) {
+        asm volatile("");   // a branch, not selects
+#pragma unroll
+        for (int i = 0; i < kRows; ++i)
+          if (i >= rows) { g[i].keep = 1.f; g[i].zc = 0.f; }
       }
 #pragma unroll
       for (int i = 0; i < kRows; ++i) {
-        g[i] = Gru(zp[i], xp[i], bz, bx);
-        if (i < rows) {
-          A *= 1.f - g[i].z;
-          B = (1.f - g[i].z) * B + g[i].zc;
-        }
+        A *= g[i].keep;
+        B = g[i].keep * B + g[i].zc;
       }
     }
-    sa[buf][wave][lane] = A;
-    sb[buf][wave][lane] = B;
+    load(zp, b0 + nw * kRows, 0);
+    load(xp, b0 + nw * kRows, 1);
+    fold[buf][wave][lane] = float2{A, B};
     __syncthreads();
     float mine = S;
+#pragma unroll 4
     for (int k = 0; k < nw; ++k) {
       if (k == wave) mine = S;
-      S = sa[buf][k][lane] * S + sb[buf][k][lane];
+      const float2 f = fold[buf][k][lane];
+      S = f.x * S + f.y;
     }
-    if (live)
+    if (rows > 0) {
+      const auto to = __builtin_amdgcn_make_buffer_rsrc(y + (long)(r0 + b0 + wave * kRows) * width, 0, rows * width * (int)sizeof(T), 0x00020000);
+      unsigned at = at0;
 #pragma unroll
-      for (int i = 0; i < kRows; ++i)
-        if (i < rows) {
-          mine = (1.f - g[i].z) * mine + g[i].zc;
-          stf<T>(y, (long)(r0 + a + i) * width + c, mine * (gp[i] * sigmoid_f(gp[i])));
-        }
-    if (rows > 0 && a + rows == n) { last = mine; holds = true; }
+      for (int i = 0; i < kRows; ++i, at += width * sizeof(T)) {
+        mine = g[i].keep * mine + g[i].zc;
+        const float gate = of_raw<T>(gp[i]), out = mine * (gate * sigmoid_f(gate));
+        if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, out), to, at, 0, 0);
+        else __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(out), to, at, 0, 0);
+      }
+      if (b0 + wave * kRows + rows == n) { last = mine; holds = true; }
+    }
+    load(gp, b0 + nw * kRows, 2);
   }
   if (live && holds) state[slot] = last;
 }
@@ -120,7 +156,7 @@ __global__ __launch_bounds__(256) void mingru_step_kernel(T* __restrict__ y, flo
 #pragma unroll
   for (int v = 0; v < kV; ++v) {
     const Gru g(zp[v], xp[v], bz[v], bx[v]);
-    S[v] = (1.f - g.z) * S[v] + g.zc;
+    S[v] = g.keep * S[v] + g.zc;
     o[v] = S[v] * (gp[v] * sigmoid_f(gp[v]));
   }
   Row<T, kV>::st(y + row * width + c, o);
@@ -206,7 +242,7 @@ __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
     const int m = (tid + kSkThreads * i) >> 4;
     if (m >= M || n0 + (tid & 15) >= width || at[i] < 0) continue;
     const Gru g(v[0][i], v[1][i], bz, bx);
-    const float o = (1.f - g.z) * (fresh[i] ? 0.f : S[i]) + g.zc;
+    const float o = g.keep * (fresh[i] ? 0.f : S[i]) + g.zc;
     stf<T>(y, (long)m * width + c, o * (v[2][i] * sigmoid_f(v[2][i])));
     state[at[i]] = o;
   }
