@@ -537,7 +537,7 @@ class KernelOps:
         the choice between them comes out best. Over 2541 sizes (1 - 64 rows, 64 - 65536 columns, k 128 - 12288, both types) it takes 1 % longer
         than the faster of the two. Examples, ours / vendor: 2048 x 2048 with 1, 16, 48, 64 rows 4.2 / 10.1, 4.9 / 10.2, 6.8 / 10.7, 7.6 / 11.1; 6144 x
         2048 with 1, 16, 48 rows 7.7 / 12.4, 8.4 / 12.3, 10.9 / 13.4; 4096 x 12288 with 1, 16, 48 rows 19.4 / 21.1, 23.8 / 22.3, 33.9 / 32.5; 512 x
-        8192 with 48 rows 16.3 / 11.1; 32000 x 2048 with 1, 16, 48, 64 rows 24.3 / 28.2, 25.0 / 28.6, 30.3 / 31.4, 33.9 / 26.6; in 32 bits 1024 x
+        8192 with 48 rows 16.3 / 11.1; 32000 x 2048 with 9, 16, 48, 64 rows 24.8 / 31.6, 26.8 / 31.5, 32.3 / 35.6, 36.8 / 32.2; in 32 bits 1024 x
         1024 with 3, 16, 48 rows 4.2 / 8.3, 4.4 / 8.3, 7.3 / 8.3; 32000 x 2048 with 1, 16, 64 rows 44 / 57, 48 / 59, 82 / 68."""
         # an activation is a launch more there (48 x 32000: 6 - 8 us)
         launch = 2.5 + 2.5e-6 * rows * cols if act and not glu else 0.0
