@@ -37,7 +37,7 @@ HS_DEVICE int find_seq(const int* __restrict__ seq_cu, int nseq, int row) {
   return -1;
 }
 
-// What enters the gated rule, as fp32 rows. One wave per item and run of kPrepTokens rows; the items of a row are
+// What enters the gated rule, as fp32 rows. One wave per item and `run` rows (prep_run); the items of a row are
 //   the query heads: unit(silu(conv q)) dim^-1/2,  the key heads: unit(silu(conv k))      -> qk[t] = [q | k]
 //   the value channels in parts of 256: silu(conv v)                                       -> vv[t]
 //   the heads' decays: exp(-exp(a_log) softplus(. + dt_bias)), one per head or (CH) per head and key channel
@@ -45,7 +45,17 @@ HS_DEVICE int find_seq(const int* __restrict__ seq_cu, int nseq, int row) {
 //   beta: sigmoid                                                                          -> bb[t]
 // Lane l owns channels l, l + 64, ... of its item and keeps their last TAPS - 1 inputs in registers while it walks
 // the rows (TAPS 0: any number of taps, inputs read again per row).
-constexpr int kPrepTokens = 16, kPrepCh = 4;   // kPrepCh * 64: most channels of an item
+constexpr int kPrepCh = 4;   // kPrepCh * 64: most channels of an item
+
+// Rows that a wave of gated_delta_prepare walks, one after the other: 16, or, of steps that leave the card room, 2 - 8: a row takes
+// about 1 us, the TAPS - 1 rows read again cost bytes. The whole rule in us with 2 / 4 / 8 / 16 rows (workgroups with 16): 33 rows of 8 heads of 128 (9)
+// 24.8 / 26.5 / 29.9 / 36.8; 3 prompts of 300 (171) 46.7 / 47.7 / 52.4 / 62.8; 16 of 200 (600) 96 / 91 / 94 / 103; 4 of 2048 (1536) 217 / 204 / 200 /
+// 212; of 16 heads (2560) 407 / 383 / 368 / 368.
+int prep_run(int T, int groups) {
+  int run = 2;
+  while (run < 16 && (long)((T + run - 1) / run) * groups > 3600) run *= 2;
+  return run;
+}
 
 template <typename T, int TAPS, bool CH>
 __global__ __launch_bounds__(256) void gated_delta_prepare_kernel(
@@ -53,12 +63,12 @@ __global__ __launch_bounds__(256) void gated_delta_prepare_kernel(
     const T* __restrict__ proj, long ld, const float* __restrict__ dec, const float* __restrict__ conv_state,
     const float* __restrict__ conv_w, const float* __restrict__ a_log, const float* __restrict__ dt_bias,
     const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int nseq, int T_,
-    int heads, int kv_heads, int dim, int vdim, int taps_, int off_a, int off_b) {
+    int heads, int kv_heads, int dim, int vdim, int taps_, int off_a, int off_b, int run) {
   const int lane = threadIdx.x & 63;
   const int nqk = kv_heads * dim, nv = heads * vdim, C = 2 * nqk + nv;
   const int vparts = (nv + 64 * kPrepCh - 1) / (64 * kPrepCh), dparts = CH ? heads : 1;
   int item = blockIdx.y * 4 + (threadIdx.x >> 6);
-  const int t0 = blockIdx.x * kPrepTokens, t1 = min(t0 + kPrepTokens, T_);
+  const int t0 = blockIdx.x * run, t1 = min(t0 + run, T_);
   if (item >= 2 * kv_heads + vparts) {
     item -= 2 * kv_heads + vparts;
     if (item < dparts) {
@@ -1024,12 +1034,13 @@ void gated_delta(const GatedDelta& p, float* scratch, hipStream_t s) {
   float* bb = vv + T_ * nv;       // [T, heads]
   float* o = bb + T_ * p.heads;   // [T, nv]
   const int items = 2 * p.kv_heads + (nv + 64 * kPrepCh - 1) / (64 * kPrepCh) + (CH ? p.heads : 1) + 1;
-  dim3 pgrid((p.T + kPrepTokens - 1) / kPrepTokens, (items + 3) / 4);
+  const int run = prep_run(p.T, (items + 3) / 4);
+  dim3 pgrid((p.T + run - 1) / run, (items + 3) / 4);
 #define HS_GP(N)                                                                                                       \
   gated_delta_prepare_kernel<T, N, CH><<<pgrid, 256, 0, s>>>(qk, vv, gg, bb, (const T*)p.proj, p.ld, p.decay,           \
                                                              p.conv_state, p.conv_w, p.a_log, p.dt_bias, p.seq_cu,      \
                                                              p.seq_ctx, p.seq_state, p.nseq, p.T, p.heads, p.kv_heads,  \
-                                                             p.dim, p.vdim, p.taps, p.off_a, p.off_b)
+                                                             p.dim, p.vdim, p.taps, p.off_a, p.off_b, run)
   if (p.taps == 4) HS_GP(4); else if (p.taps == 3) HS_GP(3); else if (p.taps == 2) HS_GP(2); else HS_GP(0);
 #undef HS_GP
   conv_state_update<T>(p, s);

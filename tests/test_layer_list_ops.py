@@ -1043,6 +1043,32 @@ def test_delta_rule_chunks_not_finite(row, what, value):
 
 
 @gpu
+@pytest.mark.parametrize("n", [6, 12, 37])
+def test_gated_delta_rows_of_a_run(n):
+    """What enters the rule, prepared in runs of 4, 8 and 16 rows (by the size of the step) and, a sequence by itself, of 2: the same bits."""
+    g = torch.Generator().manual_seed(n)
+    H, dim, one = 32, 32, 100
+    N = H * dim
+    cols, T = 3 * N, n * one
+    delta = get_ops("cuda")._delta
+    proj = torch.randn(T, cols + 2 * H + N, generator=g).bfloat16().cuda()
+    conv, kept = torch.randn(cols, 4, generator=g).cuda(), torch.randn(n, 3, cols, generator=g).cuda()
+    a, b, nw = (torch.randn(H, generator=g).cuda() for _ in range(3))
+
+    def run(rows, kept):
+        t, m = rows.shape[0], kept.shape[0]
+        scratch = torch.empty(t * (4 * N + 2 * H) + 64, device="cuda")
+        delta.gated_delta(torch.empty(t, N, dtype=torch.bfloat16, device="cuda"), torch.zeros(m, H, dim, dim, device="cuda"), kept.clone(), rows, conv, a, b,
+                          nw, None, None, (torch.arange(m + 1) * one).int().cuda(), torch.full((m,), one + 1).int().cuda(), torch.arange(m).int().cuda(), scratch, H,
+                          H, dim, dim, 4, 1e-6, cols + H, cols + 2 * H, cols, False, True, torch.empty(delta.delta_chunk_floats(t, m, H, dim, dim), device="cuda"))
+        return [x.view(t, -1) for x in scratch[:-64].split([t * 2 * N, t * H, t * N, t * H, t * N])[:4]]
+    whole = run(proj, kept)
+    for i in (0, 1, n - 1):
+        rows = slice(i * one, (i + 1) * one)
+        assert all(torch.equal(x, y[rows]) for x, y in zip(run(proj[rows], kept[i:i + 1]), whole)), i
+
+
+@gpu
 @pytest.mark.parametrize("rule,heads,vdim", [("gated", 16, 128), ("gated", 13, 100), ("generalized", 32, 64)])
 def test_delta_chunks_of_one_and_two_tiles(rule, heads, vdim):
     """Eight sequences in one step (two tiles of value channels per workgroup) and each by itself (one): the same bits; the last rows of a
