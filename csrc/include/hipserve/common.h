@@ -45,9 +45,10 @@ HS_DEVICE unsigned int pack_bf16x2(float lo, float hi) {
 // ds_bpermute round trips through the LDS crossbar. The result is wave-uniform.
 template <int kCtrl, int kRowMask, bool kMax>
 HS_DEVICE float dpp_step(float x) {
+  // a sum over whole rows, whose every lane has a partner: with no old value to keep, the permutation is part of the addition
+  constexpr bool kWhole = !kMax && kRowMask == 0xf;
   const float y = __builtin_bit_cast(
-      float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), kCtrl, kRowMask, 0xf,
-                                         false));
+      float, __builtin_amdgcn_update_dpp(kWhole ? 0 : __builtin_bit_cast(int, x), __builtin_bit_cast(int, x), kCtrl, kRowMask, 0xf, kWhole));
   return kMax ? fmaxf(x, y) : x + y;
 }
 template <bool kMax>
