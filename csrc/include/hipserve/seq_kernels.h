@@ -25,8 +25,10 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
 
 // us that such a launch takes, cold weights; k in numbers of the operands' type
 double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts);
+// Whether its workgroups take 8 columns for 16; tiles of 16 columns, over all batches and parts, K in 16-bit halves
+bool skinny_half(int M, long tiles, int K);
 // A norm around such a product of up to 32 rows, in one part: with a residual [M, N] (fp32, updated in place), out = residual * weight
-// and squares [M, blocks = N / 16] = sums of the updated residual's squares (N % 64 == 0); without one the rows x are such an out and every
+// and squares [M, blocks = N / 16 or N / 8] = sums of the updated residual's squares (N % 64 == 0); without one the rows x are such an out and every
 // result is multiplied by 1 / sqrt(the row's squares / cols + eps). blocks is a multiple of 4 and at most 256.
 struct SkinnyNorm {
   float* squares = nullptr;

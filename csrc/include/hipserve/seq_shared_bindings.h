@@ -194,14 +194,15 @@ inline void skinny_linear_normed(at::Tensor& out, const at::Tensor& x, const at:
                                                     cur_stream()), "skinny_linear: LDS");
 }
 
-// residual [M, N] += x . w^T + bias; out = residual * weight; squares [M, N / 16] = the residual's squares summed over 16 columns.
+// residual [M, N] += x . w^T + bias; out = residual * weight; squares [M, N / 16] or [M, N / 8] = the residual's squares summed over 16 or 8 columns,
+// which is what a workgroup then takes (skinny_half).
 inline void skinny_linear_update(at::Tensor& out, at::Tensor& squares, at::Tensor& residual, const at::Tensor& weight, const at::Tensor& x,
                                  const at::Tensor& w, const c10::optional<at::Tensor>& bias) {
   check_normed_rows(out, squares, x, w, bias);
   CHECK_F32(residual); CHECK_F32(weight); CHECK_SAME_DEV(residual, x); CHECK_SAME_DEV(weight, x);
   const long M = x.size(0), N = w.size(0);
   TORCH_CHECK(out.scalar_type() == x.scalar_type() && out.size(1) == N && residual.dim() == 2 && residual.size(0) == M && residual.size(1) == N &&
-              weight.numel() == N && N % 64 == 0 && squares.size(1) == N / 16, "skinny_linear_update: shapes");
+              weight.numel() == N && N % 64 == 0 && (squares.size(1) == N / 16 || squares.size(1) == N / 8), "skinny_linear_update: shapes");
   hipserve::SkinnyNorm norm;
   norm.squares = squares.data_ptr<float>();
   norm.blocks = squares.size(1);
@@ -213,9 +214,15 @@ inline void skinny_linear_update(at::Tensor& out, at::Tensor& squares, at::Tenso
               "skinny_linear: LDS");
 }
 
+inline bool skinny_half(int64_t rows, int64_t cols, int64_t k, bool f32) {
+  TORCH_CHECK(rows >= 0 && rows <= 64 && cols >= 0 && cols < (1L << 40) && k >= 0 && k < (1L << 30), "skinny_half: sizes");
+  return hipserve::skinny_half(rows, (cols + 15) / 16, f32 ? 2 * k : k);
+}
+
 inline void def_moe_ops(torch::Library& m) {
   m.def("skinny_linear(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias, int act, float c0, float c1, int act_from=0) -> ()");
   m.def("skinny_time(int rows, int cols, int k, bool glu, bool f32, int parts) -> float", &skinny_time);
+  m.def("skinny_half(int rows, int cols, int k, bool f32) -> bool", &skinny_half);
   m.def("skinny_linear_parts(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias) -> ()");
   m.def("skinny_linear_normed(Tensor(a!) out, Tensor x, Tensor squares, float eps, Tensor w, Tensor? bias, int act, float c0, float c1, "
         "int act_from) -> ()");

@@ -33,8 +33,10 @@ template <int N> HS_DEVICE void wait_copies() { asm volatile("s_waitcnt vmcnt(%0
 // One wave's part of W[NT tiles of 16 columns] . x[XG groups of 8 rows]. K in 16-bit halves, K % 8 == 0.
 // A piece (64 k) in LDS: [NT tiles][16 rows][128 bytes] of W, then [XG][8 rows][128 bytes] of x; the 16-byte part q of row r sits
 // at part q ^ (r / 2 % 8), so that the 16 rows of an operand use all banks evenly: a lane copies the part that belongs at its place.
-template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
-  static constexpr int ST = (XG + 1) / 2, kCopies = 2 * NT + XG, kPiece = kCopies * 1024;
+template <int XG, int NT, int DEPTH, bool F32 = false, bool HALF = false> struct Skinny {
+  static_assert(!HALF || NT == 1, "eight columns");
+  static constexpr int WG = HALF ? 1 : 2 * NT;   // groups of 8 rows of W
+  static constexpr int ST = (XG + 1) / 2, kCopies = WG + XG, kPiece = kCopies * 1024;
   // the last tile's missing 8 rows, where XG is odd, are read past the piece
   static constexpr int kRing = kSkWaves * DEPTH * kPiece + (XG & 1) * 1024, kSums = kSkWaves * 16 * ST * kSkLd * 4;
   static constexpr int kLds = kRing > kSums ? kRing : kSums;
@@ -47,7 +49,7 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
   // the group j of x from `x`. Every row is one that exists: what rows past the last one give is not used.
   // started(): what a kernel loads besides, once the first copies are on their way.
   template <typename F>
-  static HS_DEVICE void accumulate(f32x4 (&acc)[NT][ST], const unsigned char* const (&w)[NT], const unsigned (&w_row)[2 * NT],
+  static HS_DEVICE void accumulate(f32x4 (&acc)[NT][ST], const unsigned char* const (&w)[NT], const unsigned (&w_row)[WG],
                                    const unsigned char* x, const unsigned (&x_row)[XG], int K, unsigned char* smem,
                                    int lane, int wave, F&& started) {
     const int c = lane & 15, g = lane >> 4, r8 = lane >> 3;
@@ -55,9 +57,9 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
     const unsigned lds0 = lds_at(ring);
     const int pieces = (K + 63) >> 6, n = (pieces - wave + kSkWaves - 1) >> 3;   // this wave's: wave, wave + 8, ...
     // the lane's bytes past the piece's first k of the first row: full pieces differ by uniform numbers
-    unsigned w_at[2 * NT], x_at[XG];
+    unsigned w_at[WG], x_at[XG];
 #pragma unroll
-    for (int j = 0; j < 2 * NT; ++j) w_at[j] = w_row[j] + 16 * part(lane, 8 * (j & 1) + r8);
+    for (int j = 0; j < WG; ++j) w_at[j] = w_row[j] + 16 * part(lane, 8 * (j & 1) + r8);
 #pragma unroll
     for (int j = 0; j < XG; ++j) x_at[j] = x_row[j] + 16 * part(lane, 8 * (j & 1) + r8);
     auto copy = [&](int i) {
@@ -65,21 +67,24 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
       const unsigned to = lds0 + i % DEPTH * kPiece;
       if (k0 + 64 <= K) {
 #pragma unroll
-        for (int j = 0; j < XG; ++j) copy_1k(x + 2 * k0, x_at[j], to + (2 * NT + j) * 1024);
+        for (int j = 0; j < XG; ++j) copy_1k(x + 2 * k0, x_at[j], to + (WG + j) * 1024);
 #pragma unroll
-        for (int j = 0; j < 2 * NT; ++j) copy_1k(w[j / 2] + 2 * k0, w_at[j], to + j * 1024);
+        for (int j = 0; j < WG; ++j) copy_1k(w[j / 2] + 2 * k0, w_at[j], to + j * 1024);
         return;
       }
 #pragma unroll
       for (int j = 0; j < XG; ++j)   // what lies past K is not used
-        copy_1k(x, x_row[j] + 2 * min(k0 + 8 * part(lane, 8 * (j & 1) + r8), K - 8), to + (2 * NT + j) * 1024);
+        copy_1k(x, x_row[j] + 2 * min(k0 + 8 * part(lane, 8 * (j & 1) + r8), K - 8), to + (WG + j) * 1024);
 #pragma unroll
-      for (int j = 0; j < 2 * NT; ++j)
+      for (int j = 0; j < WG; ++j)
         copy_1k(w[j / 2], w_row[j] + 2 * min(k0 + 8 * part(lane, 8 * (j & 1) + r8), K - 8), to + j * 1024);
     };
     int at[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) at[s] = c * 128 + (((4 * s + g) ^ (c >> 1)) << 4);
+    int w_of[2];   // HALF: both halves of the tile are the same eight rows
+#pragma unroll
+    for (int s = 0; s < 2; ++s) w_of[s] = HALF ? (c & 7) * 128 + (((4 * s + g) ^ ((c & 7) >> 1)) << 4) : at[s];
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i)
       if (i < n) copy(i);
@@ -92,9 +97,9 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) a[s][nt] = *reinterpret_cast<const u16x8*>(t + nt * 2048 + at[s]);
+        for (int nt = 0; nt < NT; ++nt) a[s][nt] = *reinterpret_cast<const u16x8*>(t + nt * 2048 + w_of[s]);
 #pragma unroll
-        for (int st = 0; st < ST; ++st) b[s][st] = *reinterpret_cast<const u16x8*>(t + (NT + st) * 2048 + at[s]);
+        for (int st = 0; st < ST; ++st) b[s][st] = *reinterpret_cast<const u16x8*>(t + WG * 1024 + st * 2048 + at[s]);
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the piece is read
       if (i + DEPTH < n) copy(i + DEPTH);
@@ -127,15 +132,16 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
     }
   }
 
-  static HS_DEVICE void accumulate(f32x4 (&acc)[NT][ST], const unsigned char* const (&w)[NT], const unsigned (&w_row)[2 * NT],
+  static HS_DEVICE void accumulate(f32x4 (&acc)[NT][ST], const unsigned char* const (&w)[NT], const unsigned (&w_row)[WG],
                                    const unsigned char* x, const unsigned (&x_row)[XG], int K, unsigned char* smem,
                                    int lane, int wave) {
     accumulate(acc, w, w_row, x, x_row, K, smem, lane, wave, [] {});
   }
 
-  // Sums the waves' parts: v[nt][i] = element (row, column) = (e / 16, e % 16), e = threadIdx.x + kSkThreads * i, of
-  // the [16 ST, 16] result of column tile nt (threads past 256 ST get nothing).
-  static HS_DEVICE void reduce(float (&v)[NT][(ST + 1) / 2], const f32x4 (&acc)[NT][ST], unsigned char* smem) {
+  // Sums the waves' parts: v[nt][i] = element (row, column) = (e / kCols, e % kCols), e = threadIdx.x + kSkThreads * i, of
+  // the [16 ST, kCols] result of column tile nt (threads past it get nothing).
+  static constexpr int kCols = HALF ? 8 : 16, kElems = (16 * ST * kCols + kSkThreads - 1) / kSkThreads;
+  static HS_DEVICE void reduce(float (&v)[NT][kElems], const f32x4 (&acc)[NT][ST], unsigned char* smem) {
     float* red = reinterpret_cast<float*>(smem);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;
 #pragma unroll
@@ -146,12 +152,12 @@ template <int XG, int NT, int DEPTH, bool F32 = false> struct Skinny {
         *reinterpret_cast<f32x4*>(red + ((wave * ST + st) * 16 + c) * kSkLd + 4 * g) = acc[nt][st];
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < (ST + 1) / 2; ++i) {
+      for (int i = 0; i < kElems; ++i) {
         const int e = tid + kSkThreads * i;
         float s = 0.f;
-        if (e < 256 * ST) {
+        if (e < 16 * kCols * ST) {
 #pragma unroll
-          for (int w = 0; w < kSkWaves; ++w) s += red[(w * ST * 16 + (e >> 4)) * kSkLd + (e & 15)];
+          for (int w = 0; w < kSkWaves; ++w) s += red[(w * ST * 16 + e / kCols) * kSkLd + e % kCols];
         }
         v[nt][i] = s;
       }

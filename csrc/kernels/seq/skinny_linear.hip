@@ -29,6 +29,14 @@ HS_DEVICE float skinny_act(float z, int act, float c0, float c1) {
   return z;
 }
 
+// Sum over the lanes of a row's columns; every one of them gets it.
+template <int COLS> HS_DEVICE float cols_sum(float v) {
+  if constexpr (COLS == 16) return row_sum(v);
+  v = dpp_step<0xB1, 0xf, false>(v);      // quad_perm [1, 0, 3, 2]
+  v = dpp_step<0x4E, 0xf, false>(v);      // quad_perm [2, 3, 0, 1]
+  return dpp_step<0x141, 0xf, false>(v);  // row_half_mirror
+}
+
 enum { kPlain, kNormed, kUpdate };   // SkinnyNorm: none; rows without their norm's factor; a result that goes into the residual stream
 struct NoNorm {};
 // The kernel's arguments: the parameters are what its first loads need, the rest is loaded once the copies are on their way (seq_common.h), and
@@ -52,18 +60,18 @@ template <int NORM> struct SkinnyArgs {
 // F32: 32-bit operands, x, w, their strides and K in 16-bit halves (skinny.h). Workgroups z take `part` of K each (a multiple of 64) and write
 // their sums out_zs elements apart (the bias in the first).
 // p, q, i: kPlain - , bias, part; kNormed squares, bias, blocks; kUpdate residual, weight, blocks (K in one part for both).
-template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM>
+template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM, bool HALF>
 __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, void* p, const void* q, int x_ld, int M, int N, int K, int ni,
     const SkinnyRest<NORM>) {
   static_assert(!GLU || NT == 2, "a gate tile and an up tile");
-  using SK = Skinny<XG, NT, DEPTH, F32>;
-  constexpr int ST = SK::ST;
+  using SK = Skinny<XG, NT, DEPTH, F32, HALF>;
+  constexpr int ST = SK::ST, kCols = SK::kCols;
   using TB = std::conditional_t<F32, float, unsigned short>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int No = GLU ? N / 2 : N;
-  const int n0 = blockIdx.x * (GLU ? 16 : 16 * NT);
+  const int n0 = blockIdx.x * (GLU ? 16 : kCols * NT);
   const int k0 = NORM == kPlain ? blockIdx.z * ni : 0, k1 = NORM == kPlain ? min(K, k0 + ni) : K;
   const int rest_at = offsetof(SkinnyArgs<NORM>, rest);
   if (NORM == kPlain && blockIdx.y != 0) {
@@ -71,14 +79,14 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
     w += (long)blockIdx.y * N * K;
   }
   const unsigned char* wt[NT];
-  unsigned w_row[2 * NT];
+  unsigned w_row[SK::WG];
   unsigned x_row[XG];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int first = GLU ? n0 : min(n0 + 16 * nt, N - 1);   // of the tile's columns
     wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)(GLU ? nt * No : 0) + first) * K + k0);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), No - 1 - first) * (unsigned)(2 * K);
+    for (int h = 0; h < (HALF ? 1 : 2); ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), No - 1 - first) * (unsigned)(2 * K);
   }
 #pragma unroll
   for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)(2 * x_ld);
@@ -87,21 +95,21 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int IT = (ST + 1) / 2, SQ = 4;   // 16 threads x SQ loads x 4 sums of 16 columns each: rows of up to 4096
+  constexpr int IT = SK::kElems, SQ = HALF ? 8 : 4;   // kCols threads x SQ loads x 4 sums: 256 of them, rows of up to 4096 at 16 columns each
   [[maybe_unused]] f32x4 sq[IT][SQ];
   [[maybe_unused]] float res[IT][NT], wgt[NT];
   [[maybe_unused]] TB bs[NT];
   // for the epilogue, ahead of the copies: without branches, behind which the copies would be waited for, and first, since loads return in
   // order and a wait for the copies would be one for these too
-  const int c = tid & 15;
+  const int c = tid % kCols;
   const bool biased = NORM != kUpdate && q != nullptr && blockIdx.z == 0;
   const TB* bias = static_cast<const TB*>(biased ? q : x);
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
-    [[maybe_unused]] const long m = min((tid + kSkThreads * i) >> 4, M - 1);
+    [[maybe_unused]] const long m = min((tid + kSkThreads * i) / kCols, M - 1);
     if constexpr (NORM == kNormed) {
 #pragma unroll
-      for (int j = 0; j < SQ; ++j) sq[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p) + m * ni + min(64 * j + 4 * c, ni - 4));
+      for (int j = 0; j < SQ; ++j) sq[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p) + m * ni + min(4 * kCols * j + 4 * c, ni - 4));
     }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -144,17 +152,17 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
   SK::reduce(v, acc, smem);
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
-    const int e = tid + kSkThreads * i, m = e >> 4;
-    if (m >= M) continue;   // a row's 16 lanes together
+    const int e = tid + kSkThreads * i, m = e / kCols;
+    if (m >= M) continue;   // a row's lanes together
     if constexpr (NORM == kUpdate) {   // N is a multiple of the workgroup's columns
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        const int n = n0 + 16 * nt + (e & 15);
+        const int n = n0 + 16 * nt + e % kCols;
         const float r = res[i][nt] + (v[nt][i] + (late_bias != nullptr ? ldf<TB>(&bs[nt], 0) : 0.f));
         static_cast<float*>(p)[(long)m * N + n] = r;
         stf<TO>(out, m * out_ld + n, r * wgt[nt]);
-        const float s = row_sum(r * r);
-        if ((e & 15) == 0) squares[(long)m * ni + (n >> 4)] = s;
+        const float s = cols_sum<kCols>(r * r);
+        if (e % kCols == 0) squares[(long)m * ni + n / kCols] = s;
       }
       continue;
     }
@@ -162,8 +170,8 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
       float s = 0.f;
 #pragma unroll
       for (int j = 0; j < SQ; ++j)
-        if (64 * j + 4 * c < ni) s += (sq[i][j][0] + sq[i][j][1]) + (sq[i][j][2] + sq[i][j][3]);
-      const float inv = 1.f / sqrtf(row_sum(s) / cols + eps);
+        if (4 * kCols * j + 4 * c < ni) s += (sq[i][j][0] + sq[i][j][1]) + (sq[i][j][2] + sq[i][j][3]);
+      const float inv = 1.f / sqrtf(cols_sum<kCols>(s) / cols + eps);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) v[nt][i] *= inv;
     }
@@ -176,7 +184,7 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
     } else {
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        const int n = n0 + 16 * nt + (e & 15);
+        const int n = n0 + 16 * nt + e % kCols;
         if (n >= N) continue;
         const float z = v[nt][i] + (biased ? ldf<TB>(&bs[nt], 0) : 0.f);
         stf<TO>(out, m * out_ld + n, skinny_act(z, n >= act_from ? act : -1, c0, c1));
@@ -185,12 +193,12 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
   }
 }
 
-template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM = kPlain>
+template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM = kPlain, bool HALF = false>
 bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, long out_zs, const void* x, long x_ld, long x_bs, const void* w, const void* bias,
                    int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s,
                    const std::conditional_t<NORM != kPlain, SkinnyNorm, NoNorm>& norm = {}) {
-  constexpr int lds = Skinny<XG, NT, DEPTH, F32>::kLds;
-  static const bool ok = allow_lds(&skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM>, lds);
+  constexpr int lds = Skinny<XG, NT, DEPTH, F32, HALF>::kLds;
+  static const bool ok = allow_lds(&skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM, HALF>, lds);
   if (!ok) return false;
   SkinnyRest<NORM> rest{x_bs, out_ld, out_bs, out_zs, act, act_from, c0, c1, 1.f, 0.f, out, nullptr, bias};
   void* p = nullptr;
@@ -207,17 +215,17 @@ bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, long out_zs, 
       rest.squares = norm.squares;
     }
   }
-  skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM><<<grid, kSkThreads, lds, s>>>((const unsigned short*)x, (const unsigned short*)w, p, q,
+  skinny_linear_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM, HALF><<<grid, kSkThreads, lds, s>>>((const unsigned short*)x, (const unsigned short*)w, p, q,
                                                                                         (int)x_ld, M, N, K, i, rest);
   return true;
 }
 
-template <int XG, int NT, int DEPTH, bool GLU>
+template <int XG, int NT, int DEPTH, bool GLU, bool HALF = false>
 bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, int parts, const void* x, long x_ld, long x_bs,
                 const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
-  const int cols = GLU ? N / 2 : N, per = GLU ? 16 : 16 * NT;
+  const int cols = GLU ? N / 2 : N, per = GLU ? 16 : HALF ? 8 : 16 * NT;
   const dim3 grid((cols + per - 1) / per, batch, parts);
-#define HS_SK(TO, F32) launch_kernel<XG, NT, DEPTH, GLU, TO, F32>(grid, out, out_ld, out_bs, out_zs, x, x_ld, x_bs, w, bias, M, N, K, act, act_from, c0, c1, s)
+#define HS_SK(TO, F32) launch_kernel<XG, NT, DEPTH, GLU, TO, F32, kPlain, HALF>(grid, out, out_ld, out_bs, out_zs, x, x_ld, x_bs, w, bias, M, N, K, act, act_from, c0, c1, s)
   return f32 ? HS_SK(float, true) : out_f32 ? HS_SK(float, false) : HS_SK(unsigned short, false);
 #undef HS_SK
 }
@@ -240,20 +248,31 @@ int skinny_tiles(int M, long tiles, int K) {
 // From the third round on two workgroups of two tiles share a compute unit and hide a quarter of it, measured where the choice turns on it: 32000 x
 // 2048 with 32, 48 rows 28.5, 32.7 us (32.7, 37.4 without that, so that the vendor's 35.6 was taken for 48), 65536 x 2048 with 32 55.5 (vendor 66.9);
 // with fewer k or more than 48 rows the vendor's is the faster one there (50000 x 1024 with 40 rows 26.8 / 22.6, 65536 x 2048 with 56 75 / 72).
-double skinny_time_of(int M, long cols, double K, int nt, int parts, bool f32, double out_bytes) {
-  const long wgs = ((cols + 15) / 16 + nt - 1) / nt * parts, rounds = (wgs + 255) / 256;
+double skinny_time_of(int M, long cols, double K, int nt, int parts, bool f32, double out_bytes, bool half = false) {
+  const long wgs = ((cols + 15) / 16 + nt - 1) / nt * parts, rounds = (wgs + 255) / 256;   // of whole tiles; halves are one round
   const double bytes = 2.0 * cols * K, rows = (M + 7) / 8 * 8, k = K / parts, st = nt * ((M + 15) / 16);
-  const double each = 2.0 * k * (16 * nt + rows) / 80e3 + st * (0.09 + (f32 ? 8.5e-5 * k : 0));
+  const double each = 2.0 * k * ((half ? 8 : 16 * nt) + rows) / 80e3 + st * (0.09 + (f32 ? 8.5e-5 * k : 0));
   const double hidden = nt == 2 && wgs > 512 && parts == 1 && !f32 && M <= 48 && K >= 2048 && K < 4096 ? 0.25 : 0.0;
   return 2.16 + std::max(bytes / 5.2e6, bytes / 9e6 + (1.0 - hidden) * rounds * each) + 0.7e-6 * out_bytes;
 }
 
 }  // namespace
 
+// Whether a workgroup takes half a tile, 8 columns: where whole ones leave half of the compute units idle, and K (in halves) is long enough for what
+// a workgroup takes in to matter. Two pieces ahead (three for up to 8 rows of more than 4096). The sums are the same. Cold weights, us, whole ->
+// half: 2048 x 2048 with 1, 16, 24 rows 3.6 -> 3.4, 3.8 -> 3.65, 4.25 -> 3.85; 2048 x 6144 with 1, 16, 48 rows 7.3 -> 6.4, 10.1 -> 8.25, 16.2 ->
+// 14.0; 1024 x 3072 with 1, 16, 48 rows 3.6 -> 3.6, 4.2 -> 3.9, 6.4 -> 5.9; in 32 bits, 16 rows, 2048 x 2048 7.2 -> 6.3, 1024 x 3072 9.0 -> 7.6. 2048
+// x 1024 with 1, 16 rows 2.85 -> 2.95, 2.95 -> 3.0; 2048 x 2048 with 48 rows 5.2 -> 5.35. 1024 x 3072 with one row: no gain, and the sums of squares of an
+// update are twice as many (a decode step of width 1024 116 -> 118).
+bool skinny_half(int M, long tiles, int K) {
+  return tiles <= 128 && (M <= 8 && tiles <= 64 ? K > 4096 : K > 1024) && (M <= 32 || tiles <= 104 || K > 2048);
+}
+
 double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts) {
   const int K = f32 ? 2 * k : k;
   const double out = (double)M * (glu ? cols / 2 : cols) * (f32 ? 4 : 2);
-  return skinny_time_of(M, cols, K, glu ? 2 : skinny_tiles(M, (cols + 15) / 16 * parts, K / parts), parts, f32, out);
+  const long tiles = (cols + 15) / 16 * parts;
+  return skinny_time_of(M, cols, K, glu ? 2 : skinny_tiles(M, tiles, K / parts), parts, f32, out, !glu && skinny_half(M, tiles, K / parts));
 }
 
 double mingru_product_time(int M, int width, int k, bool f32) {   // a workgroup's three tiles (mingru.hip)
@@ -265,12 +284,17 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
                           hipStream_t s) {
   if (batch <= 0 || M <= 0 || N <= 0) return true;
   if (f32) { x_ld *= 2; x_bs *= 2; K *= 2; }   // in halves
-#define HS_SK(XG, NT, DEPTH, GLU)   launch_one<XG, NT, DEPTH, GLU>(out, out_f32, out_ld, out_bs, out_zs, parts, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, act_from, c0, c1, s)
+#define HS_SK(XG, NT, DEPTH, ...)   launch_one<XG, NT, DEPTH, __VA_ARGS__>(out, out_f32, out_ld, out_bs, out_zs, parts, x, x_ld, x_bs, w, bias, f32, batch, M, N, K, act, act_from, c0, c1, s)
   const int xg = (M + 7) / 8;
   if (act == 3 || act == 4)
     return xg <= 1 ? HS_SK(1, 2, 1, true) : xg <= 2 ? HS_SK(2, 2, 1, true) : xg <= 4 ? HS_SK(4, 2, 1, true)
          : xg <= 6 ? HS_SK(6, 2, 1, true) : HS_SK(8, 2, 1, true);
   const long tiles = ((long)N * batch + 15) / 16 * parts;
+  if (skinny_half(M, tiles, K / parts)) {
+    if (xg <= 1) return K / parts > 4096 ? HS_SK(1, 1, 3, false, true) : HS_SK(1, 1, 2, false, true);
+    return xg <= 2 ? HS_SK(2, 1, 2, false, true) : xg <= 3 ? HS_SK(3, 1, 2, false, true) : xg <= 4 ? HS_SK(4, 1, 2, false, true)
+         : xg <= 6 ? HS_SK(6, 1, 2, false, true) : HS_SK(8, 1, 2, false, true);
+  }
   const int nt = skinny_tiles(M, tiles, K / parts);
   // One piece ahead: two are faster (up to 40 %) where a wave waits for its few copies, up to 16 rows and more than a piece per wave (more than
   // two where a compute unit holds several workgroups: 12288 x 1024, 16 rows 9 % slower; 3072 x 1024, one row 4 % faster), and slower
@@ -290,20 +314,29 @@ static bool launch_normed(void* out, bool out_f32, const SkinnyNorm& norm, const
   if (f32) { x_ld *= 2; K *= 2; }   // in halves
   const bool glu = act == 3 || act == 4;
   const long No = glu ? N / 2 : N;
-#define HS_SN(XG, NT, DEPTH, GLU, TO, F32)                                                                                                    \
-  launch_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM>(dim3((No + (GLU ? 16 : 16 * NT) - 1) / (GLU ? 16 : 16 * NT)), out, No, 0, 0, x, x_ld, 0, w,  \
-                                                   bias, M, N, K, act, act_from, c0, c1, s, norm)
-#define HS_SX(NT, D, GLU, TO, F32) (M <= 8 ? HS_SN(1, NT, D, GLU, TO, F32) : M <= 16 ? HS_SN(2, NT, D, GLU, TO, F32) : HS_SN(4, NT, F32 ? 1 : D, GLU, TO, F32))
+#define HS_SN(XG, NT, DEPTH, GLU, TO, F32, HALF)                                                                                              \
+  launch_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM, HALF>(dim3((No + (GLU ? 16 : HALF ? 8 : 16 * NT) - 1) / (GLU ? 16 : HALF ? 8 : 16 * NT)), out, No, \
+                                                         0, 0, x, x_ld, 0, w, bias, M, N, K, act, act_from, c0, c1, s, norm)
+#define HS_SX(NT, D, GLU, TO, F32) \
+  (M <= 8 ? HS_SN(1, NT, D, GLU, TO, F32, false) : M <= 16 ? HS_SN(2, NT, D, GLU, TO, F32, false) : HS_SN(4, NT, F32 ? 1 : D, GLU, TO, F32, false))
+#define HS_SH(TO, F32)                                                                                                              \
+  (M <= 8 ? K > 4096 ? HS_SN(1, 1, 3, false, TO, F32, true) : HS_SN(1, 1, 2, false, TO, F32, true)                                  \
+          : M <= 16 ? HS_SN(2, 1, 2, false, TO, F32, true) : HS_SN(4, 1, 2, false, TO, F32, true))
   using Wide = std::conditional_t<NORM == kNormed, float, unsigned short>;   // an update writes rows of the operands' type
 #define HS_ST(NT, D, GLU) (f32 ? HS_SX(NT, D, GLU, float, true) : out_f32 ? HS_SX(NT, D, GLU, Wide, false) : HS_SX(NT, D, GLU, unsigned short, false))
-#define HS_S4() (f32 ? HS_SN(4, 4, 1, false, float, true) : out_f32 ? HS_SN(4, 4, 1, false, Wide, false) : HS_SN(4, 4, 1, false, unsigned short, false))
+#define HS_S4() \
+  (f32 ? HS_SN(4, 4, 1, false, float, true, false) : out_f32 ? HS_SN(4, 4, 1, false, Wide, false, false) : HS_SN(4, 4, 1, false, unsigned short, false, false))
   // Two pieces ahead for one tile, but for more than 16 rows of 32 bits: a decode step of 20 rows (width 1024) 122.4 us with two, 124.2 with
   // one, in 32 bits 167.1 and 166.0, of 32 rows 128.4 and 130.0, 173.7 and 170.0.
   if constexpr (NORM == kNormed)
     if (glu) return HS_ST(2, 1, true);
+  // where squares are written, their number says what the workgroups are to take
+  if (NORM == kUpdate ? norm.blocks == N / 8 : skinny_half(M, (N + 15) / 16, K))
+    return f32 ? HS_SH(float, true) : out_f32 ? HS_SH(Wide, false) : HS_SH(unsigned short, false);
   const int nt = skinny_tiles(M, (N + 15) / 16, K);   // 4 above 16 rows alone; where squares are written, N is a multiple of 64
   return nt == 4 ? HS_S4() : nt == 2 ? HS_ST(2, 1, false) : HS_ST(1, 2, false);
 #undef HS_S4
+#undef HS_SH
 #undef HS_ST
 #undef HS_SX
 #undef HS_SN

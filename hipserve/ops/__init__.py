@@ -125,8 +125,9 @@ class KernelOps:
         self.norm_library = "seq"
         # the rules of products of a few rows: arithmetic on sizes, a few us each, and a step asks for every product. What they said of
         # the last sizes is kept (a step that is not captured, of four layers and a few rows, took 20 - 40 us longer)
-        self.skinny_pays, self.skinny_parts, self.update_pays, self.mingru_pays = (
-            functools.lru_cache(maxsize=4096)(rule) for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._mingru_pays))
+        self.skinny_pays, self.skinny_parts, self.update_pays, self.update_cols, self.mingru_pays = (
+            functools.lru_cache(maxsize=4096)(rule)
+            for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._update_cols, self._mingru_pays))
 
     @property
     def _op(self):
@@ -649,6 +650,10 @@ class KernelOps:
         after = max(0.0, self._skinny_time(rows, 3 * cols, cols, False, f32) - self._vendor_time(rows, 3 * cols, cols, f32))
         return self._skinny_time(rows, cols, k, False, f32) + 0.6 + after <= apart + 2.5 + 0.05 * rows * cols / 1024
 
+    def _update_cols(self, rows, cols, k, f32) -> int:
+        """Columns that a workgroup of the update takes, and that a sum of squares is over."""
+        return 8 if cols <= 2048 and self._moe_lib.skinny_half(rows, cols, k, f32) else 16
+
     def linear_update(self, x, w, bias, residual, norm_w, eps):
         """residual += x . w^T + bias, and the rows for the next products as ``NormedRows`` of its norm; None, and nothing done, where the
         update and norm are a launch of their own (``update_pays``)."""
@@ -656,7 +661,7 @@ class KernelOps:
         if not (0 < T <= self.NORM_ROWS and N % 64 == 0 and N <= 4096 and self.update_pays(T, N, K, x.dtype == torch.float32)
                 and self._skinny_ok(x, w, bias) and residual.is_contiguous() and residual.data_ptr() % 16 == 0):
             return None
-        rows, squares = torch.empty(T, N, device=x.device, dtype=x.dtype), torch.empty(T, N // 16, device=x.device, dtype=torch.float32)
+        rows, squares = torch.empty(T, N, device=x.device, dtype=x.dtype), torch.empty(T, N // self.update_cols(T, N, K, x.dtype == torch.float32), device=x.device, dtype=torch.float32)
         self._moe_lib.skinny_linear_update(rows, squares, residual, norm_w, x, w, bias)
         return NormedRows(rows, squares, eps)
 

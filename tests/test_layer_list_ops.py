@@ -289,6 +289,47 @@ def test_norm_inside_the_products(M, H, K, N, act, dtype):
 
 
 @gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 25, 33, 49])
+@pytest.mark.parametrize("N,K", [(1, 1032), (9, 2056), (1660, 1096), (2048, 4104)])
+def test_products_in_half_tiles(M, N, K, dtype):
+    """Workgroups of 8 columns: the same bits as those of 16, which the same columns among more of them take; a last workgroup that is partly
+    filled, k past a whole piece, two and three pieces ahead, a bias, an activation."""
+    g = torch.Generator().manual_seed(M + N)
+    x, b = torch.randn(M, K, generator=g).to(dtype).cuda(), torch.randn(N + 2064, generator=g).to(dtype).cuda()
+    w = torch.randn(N + 2064, K, generator=g).to(dtype).cuda()
+    lib = get_ops("cuda")._moe_lib
+    f32 = dtype == torch.float32
+    assert not lib.skinny_half(M, N + 2064, K, f32) and lib.skinny_half(M, N, K, f32) == (M > 8 or N > 1024 or K * (1 + f32) > 4096)
+    for act in (-1, 0):
+        got, want = torch.empty(M, N, dtype=dtype, device="cuda"), torch.empty(M, N + 2064, dtype=dtype, device="cuda")
+        lib.skinny_linear(got, x, w[:N], b[:N], act, 0.0, 0.0)
+        lib.skinny_linear(want, x, w, b, act, 0.0, 0.0)
+        assert torch.equal(got, want[:, :N])
+
+
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("M,H,K", [(1, 64, 2056), (8, 2048, 4104), (9, 192, 1032), (16, 1024, 3072), (17, 2048, 520), (32, 832, 2048)])
+def test_updates_in_half_tiles(M, H, K, dtype):
+    """A residual update of 8 columns per workgroup: its sums, rows and squares, and the norm's factor from twice as many of them."""
+    g = torch.Generator().manual_seed(M + H)
+    x, w, b = torch.randn(M, K, generator=g).to(dtype), (torch.randn(H, K, generator=g) / K ** 0.5).to(dtype), torch.randn(H, generator=g).to(dtype)
+    res, norm, w2 = torch.randn(M, H, generator=g) * 3, 1 + 0.1 * torch.randn(H, generator=g), (torch.randn(80, H, generator=g) / H ** 0.5).to(dtype)
+    ops, out = get_ops("cuda"), []
+    for cols in (8, 16):
+        r, rows = res.cuda(), torch.empty(M, H, dtype=dtype, device="cuda")
+        squares = torch.full((M, H // cols), float("nan"), device="cuda")
+        ops._moe_lib.skinny_linear_update(rows, squares, r, norm.cuda(), x.cuda(), w.cuda(), b.cuda())
+        out.append((r, rows, squares, ops.linear(NormedRows(rows, squares, 1e-6), w2.cuda())))
+    (r8, rows8, s8, y8), (r16, rows16, s16, y16) = out
+    assert torch.equal(r8, r16) and torch.equal(rows8, rows16)
+    assert torch.allclose(s8.double().cpu().sum(1), r16.double().cpu().square().sum(1), rtol=1e-5)
+    # the factors from the same squares in another order: 2^-22 of a result, which may round the other way
+    assert ((y8.double() - y16.double()).abs() <= (2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -20) * y16.double().abs()).all()
+
+
+@gpu
 @pytest.mark.parametrize("M", [8, 9, 24, 25, 40, 41, 64])
 @pytest.mark.parametrize("N", [4113, 5001, 12301])
 def test_skinny_linear_wide(M, N):
