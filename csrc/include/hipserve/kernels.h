@@ -267,13 +267,14 @@ void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, i
                       int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s,
                       int* hist = nullptr);
 // the same for the pairs (t, j), expert table[i][tokens[t]][j] of `tables` tables [table_rows, top], outputs side by side (num_tiles
-// [tables]): a workgroup each, small batches
+// [tables]): a workgroup each, or many for a large step of one table (hist as below)
 void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
                             int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot,
-                            hipStream_t s);
+                            int* hist, hipStream_t s);
 // blocks of the multi-workgroup moe_align for npairs (1: the single-workgroup kernel);
 // it needs hist = int32 [blocks * 128] scratch
 int moe_align_blocks(int npairs);
+bool moe_align_small(int npairs);   // what moe_table_align takes
 // xs[slot, H] = x[slots[slot] / k] (zeros for padding slots): grouped-GEMM input rows
 void launch_moe_gather(void* out, const void* x, long x_stride, const int* slots, int nslots, int k, int H,
                        hipStream_t s);

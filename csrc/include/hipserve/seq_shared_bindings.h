@@ -48,9 +48,9 @@ inline void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor
 }
 
 // moe_align of the pairs (t, j) whose expert is table[tokens[t]][j], table [rows, top]; or of every table of [L, rows, top], with outputs
-// [L, slots], [L, tiles], [L, pairs].
+// [L, slots], [L, tiles], [L, pairs]; num_tiles [L]: the tiles in use.
 inline void moe_table_align(const at::Tensor& table, const at::Tensor& tokens, int64_t E, int64_t tile, at::Tensor& slots,
-                            at::Tensor& tile_expert, at::Tensor& pair_slot) {
+                            at::Tensor& tile_expert, at::Tensor& pair_slot, const c10::optional<at::Tensor>& num_tiles) {
   CHECK_DEV(table); CHECK_I32(table); CHECK_I32(slots); CHECK_I32(tile_expert); CHECK_I32(pair_slot);
   CHECK_SAME_DEV(tokens, table); CHECK_SAME_DEV(slots, table); CHECK_SAME_DEV(tile_expert, table); CHECK_SAME_DEV(pair_slot, table);
   const long d = table.dim(), L = d == 3 ? table.size(0) : 1;
@@ -60,17 +60,23 @@ inline void moe_table_align(const at::Tensor& table, const at::Tensor& tokens, i
   TORCH_CHECK(E >= 1 && E <= 128, "moe_align: at most 128 experts");
   TORCH_CHECK(tile == 16 || tile == 32 || tile == 64 || tile == 128 || tile == 256);
   const long top = table.size(d - 1), npairs = tokens.numel() * top, cap = slots.numel() / L, tiles = tile_expert.numel() / L;
-  TORCH_CHECK(top >= 1 && hipserve::moe_align_blocks(npairs) == 1, "moe_table_align: small batches");
+  TORCH_CHECK(top >= 1 && hipserve::moe_align_small(npairs), "moe_table_align: small batches");
   TORCH_CHECK(cap >= npairs + E * (tile - 1) && cap % tile == 0, "slots capacity must cover padding and be a multiple of the tile");
   TORCH_CHECK(tiles * tile >= cap && pair_slot.numel() / L >= npairs && (d == 2 || pair_slot.size(1) == npairs));
   c10::hip::HIPGuardMasqueradingAsCUDA g(table.device());
-  at::Tensor count = at::empty({L}, slots.options());
+  if (num_tiles.has_value()) {
+    CHECK_I32(*num_tiles); CHECK_SAME_DEV(*num_tiles, table);
+    TORCH_CHECK(num_tiles->numel() == L, "moe_table_align: a count per table");
+  }
+  const int nb = L == 1 ? hipserve::moe_align_blocks(npairs) : 1;
+  at::Tensor hist = at::empty({nb > 1 ? nb * 128L : 0}, slots.options());
+  at::Tensor count = num_tiles.has_value() ? *num_tiles : at::empty({L}, slots.options());
   hipserve::launch_moe_table_align(table.data_ptr<int>(), L, tokens.data_ptr<long>(), top, table.size(d - 2), npairs, E, tile,
                                    slots.data_ptr<int>(), cap, tile_expert.data_ptr<int>(), tiles, count.data_ptr<int>(),
-                                   pair_slot.data_ptr<int>(), cur_stream());
+                                   pair_slot.data_ptr<int>(), hist.data_ptr<int>(), cur_stream());
 }
 
-inline bool moe_align_small(int64_t npairs) { return hipserve::moe_align_blocks(npairs) == 1; }
+inline bool moe_align_small(int64_t npairs) { return hipserve::moe_align_small(npairs); }
 
 inline void expert_gemm(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const at::Tensor& slots,
                         const at::Tensor& tile_expert, int64_t tile, int64_t gather_k, int64_t act,
@@ -229,7 +235,7 @@ inline void def_moe_ops(torch::Library& m) {
   m.def("skinny_linear_update(Tensor(a!) out, Tensor(b!) squares, Tensor(c!) residual, Tensor weight, Tensor x, Tensor w, Tensor? bias) -> ()");
   m.def("moe_align(Tensor ids, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, Tensor(c!) pair_slot) -> ()");
   m.def("moe_table_align(Tensor table, Tensor tokens, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, "
-        "Tensor(c!) pair_slot) -> ()");
+        "Tensor(c!) pair_slot, Tensor(d!)? num_tiles=None) -> ()");
   m.def("moe_align_small(int npairs) -> bool", &moe_align_small);
   m.def("expert_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor slots, Tensor tile_expert, int tile, int gather_k, "
         "int act, Tensor? row_scale=None, float limit=0.0, int pairs=0, int tiles=0) -> ()");

@@ -88,153 +88,166 @@ __global__ __launch_bounds__(256) void moe_topk_softmax_kernel(const T* __restri
   }
 }
 
+HS_DEVICE int pair_expert(int p, const int* ids, const int* table, const long* tokens, int top, int top_shift, long table_rows) {
+  if (table == nullptr) return ids[p];
+  const int t = top_shift >= 0 ? p >> top_shift : p / top;
+  const long row = tokens[t];
+  return table[(row >= 0 && row < table_rows ? row : 0) * top + (p - t * top)];
+}
+
+// Exclusive scan of the tile-padded counts by one wave, 2 experts per lane (E <= 128); off[128]: all of them.
+HS_DEVICE void padded_offsets(const int* cnt, int* off, int E, int tile_shift, int* num_tiles, int* group_end, bool first) {
+  const int lane = threadIdx.x & 63, e0 = 2 * lane, e1 = 2 * lane + 1, tile = 1 << tile_shift;
+  const int a = e0 < E ? (cnt[e0] + tile - 1) >> tile_shift << tile_shift : 0;
+  const int b = e1 < E ? (cnt[e1] + tile - 1) >> tile_shift << tile_shift : 0;
+  int incl = a + b;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += v;
+  }
+  const int excl = incl - a - b;
+  off[e0] = excl;
+  off[e1] = excl + a;
+  if (first && group_end != nullptr) {  // per-expert end row of the padded expert-sorted slots (grouped GEMM offsets)
+    if (e0 < E) group_end[e0] = excl + a;
+    if (e1 < E) group_end[e1] = incl;
+  }
+  if (lane == 63) {
+    off[128] = incl;
+    if (first) *num_tiles = incl >> tile_shift;
+  }
+}
+
 // table (may be null): the experts come from table[tokens[t]][j] (top of them per token) instead of ids, without a
-// launch of its own for the lookup (4.5 us); a token outside the table counts as its first entry. Workgroup b serves table b of as many
-// (decode steps: the tables of all layers in one launch, 3.3 - 4.4 us instead of that for each).
+// launch of its own for the lookup (4.5 - 6.3 us); a token outside the table counts as its first entry. Workgroup b serves table b of as many
+// (decode steps: the tables of all layers in one launch, 2.6 - 3.8 us instead of that for each).
+// PER: pairs per thread at most, all looked up at once; a pair's place among its expert's is what the count gives it, and only slots that hold
+// no pair are cleared (96 pairs 3.2 -> 2.6 us beside a second pass that counts again).
+template <int PER>
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, const int* __restrict__ table,
-                                                         const long* __restrict__ tokens, int top, long table_rows,
-                                                         int npairs, int E, int tile,
+                                                         const long* __restrict__ tokens, int top, int top_shift, long table_rows,
+                                                         int npairs, int E, int tile_shift,
                                                          int* __restrict__ slots, int slots_cap,
                                                          int* __restrict__ tile_expert, int tiles_cap,
                                                          int* __restrict__ num_tiles, int* __restrict__ pair_slot,
                                                          int* __restrict__ group_end) {
-  __shared__ int cnt[128], off[129], cur[128];
-  const int tid = threadIdx.x, lane = tid & 63;
+  __shared__ int cnt[128], off[129];
+  const int tid = threadIdx.x;
   const long b = blockIdx.x;
   if (table != nullptr) table += b * table_rows * top;
   slots += b * slots_cap;
   tile_expert += b * tiles_cap;
   pair_slot += b * npairs;
   num_tiles += b;
-  auto expert_of = [&](int p) {
-    if (table == nullptr) return ids[p];
-    const long t = tokens[p / top];
-    return table[(t >= 0 && t < table_rows ? t : 0) * top + p % top];
-  };
-  if (tid < 128) { cnt[tid] = 0; cur[tid] = 0; }
-  __syncthreads();
-  for (int p = tid; p < npairs; p += 1024) atomicAdd(&cnt[expert_of(p)], 1);
-  __syncthreads();
-  if (tid < 64) {  // exclusive scan of the tile-padded counts, 2 experts per lane (E <= 128)
-    const int e0 = 2 * lane, e1 = 2 * lane + 1;
-    const int a = e0 < E ? (cnt[e0] + tile - 1) / tile * tile : 0;
-    const int b = e1 < E ? (cnt[e1] + tile - 1) / tile * tile : 0;
-    int incl = a + b;
+  int e[PER], rank[PER];
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
-    const int excl = incl - a - b;
-    off[e0] = excl;
-    off[e1] = excl + a;
-    if (group_end != nullptr) {  // per-expert end row of the padded expert-sorted slots (grouped GEMM offsets)
-      if (e0 < E) group_end[e0] = excl + a;
-      if (e1 < E) group_end[e1] = incl;
-    }
-    if (lane == 63) {
-      off[128] = incl;
-      *num_tiles = incl / tile;
-    }
-  }
-  __syncthreads();
-  const int total = off[128];
-  for (int s = tid; s < slots_cap; s += 1024) slots[s] = -1;
-  // each expert labels its own tiles; tiles past the used range are -1
-  if (tid < E)
-    for (int t = off[tid] / tile; t < (off[tid] + (cnt[tid] + tile - 1) / tile * tile) / tile; ++t) tile_expert[t] = tid;
-  for (int t = total / tile + tid; t < tiles_cap; t += 1024) tile_expert[t] = -1;
-  __syncthreads();
-  for (int p = tid; p < npairs; p += 1024) {
-    const int e = expert_of(p);
-    const int pos = off[e] + atomicAdd(&cur[e], 1);
-    slots[pos] = p;
-    pair_slot[p] = pos;
-  }
-}
-
-// Multi-workgroup moe_align for prefill-sized pair counts (one workgroup scatters ~0.6 ns
-// per pair: 157 us per layer at 262K pairs). Pass 1: per-block expert histograms
-// hist[b][E]. Pass 2: every block sums the table (nb x E ints) into the padded expert
-// offsets and its own prefix, then scatters its chunk; block 0 also writes the tile table,
-// the tile count and the padding slots (disjoint from every real slot, so no ordering
-// between blocks is needed).
-constexpr int kAlignChunk = 4096;
-__global__ __launch_bounds__(1024) void moe_count_kernel(const int* __restrict__ ids, int npairs,
-                                                         int* __restrict__ hist) {
-  __shared__ int cnt[128];
-  const int tid = threadIdx.x, b = blockIdx.x;
+  for (int i = 0; i < PER; ++i) e[i] = npairs > 0 ? pair_expert(min(tid + 1024 * i, npairs - 1), ids, table, tokens, top, top_shift, table_rows) : 0;
   if (tid < 128) cnt[tid] = 0;
   __syncthreads();
-  const int end = min(npairs, (b + 1) * kAlignChunk);
-  for (int p = b * kAlignChunk + tid; p < end; p += 1024) atomicAdd(&cnt[ids[p]], 1);
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+    if (tid + 1024 * i < npairs) rank[i] = atomicAdd(&cnt[e[i]], 1);
+  __syncthreads();
+  if (tid < 64) padded_offsets(cnt, off, E, tile_shift, num_tiles, group_end, true);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int p = tid + 1024 * i;
+    if (p < npairs) {
+      const int pos = off[e[i]] + rank[i];
+      slots[pos] = p;
+      pair_slot[p] = pos;
+    }
+  }
+  const int total = off[128];
+  for (int x = tid >> 6; x < E; x += 16)   // the rest of every expert's last tile
+    for (int s = off[x] + cnt[x] + (tid & 63); s < off[x + 1]; s += 64) slots[s] = -1;
+  for (int s = total + tid; s < slots_cap; s += 1024) slots[s] = -1;
+  // each expert labels its own tiles; tiles past the used range are -1
+  if (tid < E)
+    for (int t = off[tid] >> tile_shift; t < off[tid + 1] >> tile_shift; ++t) tile_expert[t] = tid;
+  for (int t = (total >> tile_shift) + tid; t < tiles_cap; t += 1024) tile_expert[t] = -1;
+}
+
+// moe_align over many workgroups, for prefill-sized pair counts (one workgroup is bound by its compute unit's lookups and stores). Pass 1: a
+// workgroup counts the experts of its PER * 1024 pairs, hist[b][E], and leaves each pair's expert and place among them in pair_slot. Pass
+// 2: every workgroup sums the table (nb x E ints) into the padded expert offsets and its own prefix, then scatters its pairs; the padding slots
+// (disjoint from every real slot, so no ordering between workgroups is needed) and tile tables of the experts go round the workgroups.
+// us, one workgroup -> many, in brackets with the lookup of table[token]: 8000 pairs, 16 experts 7.2 -> 5.0 (13.4 -> 5.4), 16384 pairs 11.9 -> 5.2
+// (24.4 -> 5.6), of 128 experts 13.8 -> 6.4 (25.4 -> 6.8); 4096 pairs 4.0 (5.5) on one.
+template <int PER>
+__global__ __launch_bounds__(1024) void moe_count_kernel(const int* __restrict__ ids, const int* __restrict__ table, const long* __restrict__ tokens,
+                                                         int top, int top_shift, long table_rows, int npairs, int* __restrict__ pair_slot,
+                                                         int* __restrict__ hist) {
+  __shared__ int cnt[128];
+  const int tid = threadIdx.x, b = blockIdx.x, p0 = b * PER * 1024 + tid;
+  int e[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) e[i] = pair_expert(min(p0 + 1024 * i, npairs - 1), ids, table, tokens, top, top_shift, table_rows);
+  if (tid < 128) cnt[tid] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+    if (p0 + 1024 * i < npairs) pair_slot[p0 + 1024 * i] = e[i] << 16 | atomicAdd(&cnt[e[i]], 1);
   __syncthreads();
   if (tid < 128) hist[b * 128 + tid] = cnt[tid];
 }
 
-__global__ __launch_bounds__(1024) void moe_place_kernel(const int* __restrict__ ids, int npairs, int E, int tile,
-                                                         const int* __restrict__ hist, int nb,
+template <int PER>
+__global__ __launch_bounds__(1024) void moe_place_kernel(int npairs, int E, int tile_shift, const int* __restrict__ hist, int nb,
                                                          int* __restrict__ slots, int slots_cap,
                                                          int* __restrict__ tile_expert, int tiles_cap,
                                                          int* __restrict__ num_tiles, int* __restrict__ pair_slot,
                                                          int* __restrict__ group_end) {
-  __shared__ int cnt[128], pre[128], off[129], cur[128];
-  const int tid = threadIdx.x, lane = tid & 63, b = blockIdx.x;
-  if (tid < 128) {  // expert totals and this block's prefix over the blocks before it
+  __shared__ int cnt[128], pre[128], off[129], part[2][8][128];
+  const int tid = threadIdx.x, b = blockIdx.x, tile = 1 << tile_shift, p0 = b * PER * 1024 + tid;
+  int mine[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) mine[i] = pair_slot[min(p0 + 1024 * i, npairs - 1)];
+  {  // expert totals and this workgroup's prefix over those before it
+    const int x = tid & 127, g = tid >> 7;
     int c = 0, q = 0;
-    for (int j = 0; j < nb; ++j) {
-      const int h = hist[j * 128 + tid];
+#pragma unroll 4
+    for (int j = g; j < nb; j += 8) {
+      const int h = hist[j * 128 + x];
       c += h;
       q += j < b ? h : 0;
     }
-    cnt[tid] = c;
-    pre[tid] = q;
-    cur[tid] = 0;
+    part[0][g][x] = c;
+    part[1][g][x] = q;
   }
   __syncthreads();
-  if (tid < 64) {  // exclusive scan of the tile-padded counts, 2 experts per lane (E <= 128)
-    const int e0 = 2 * lane, e1 = 2 * lane + 1;
-    const int a = e0 < E ? (cnt[e0] + tile - 1) / tile * tile : 0;
-    const int c = e1 < E ? (cnt[e1] + tile - 1) / tile * tile : 0;
-    int incl = a + c;
+  if (tid < 256) {
+    int c = 0;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
-    const int excl = incl - a - c;
-    off[e0] = excl;
-    off[e1] = excl + a;
-    if (b == 0 && group_end != nullptr) {
-      if (e0 < E) group_end[e0] = excl + a;
-      if (e1 < E) group_end[e1] = incl;
-    }
-    if (lane == 63) {
-      off[128] = incl;
-      if (b == 0) *num_tiles = incl / tile;
-    }
+    for (int g = 0; g < 8; ++g) c += part[tid >> 7][g][tid & 127];
+    (tid < 128 ? cnt : pre)[tid & 127] = c;
   }
   __syncthreads();
-  if (b == 0) {
-    const int total = off[128];
-    for (int e = 0; e < E; ++e) {  // padding slots of each expert, then the unused tail
-      const int lo = off[e] + cnt[e], hi = off[e] + (cnt[e] + tile - 1) / tile * tile;
-      for (int s = lo + tid; s < hi; s += 1024) slots[s] = -1;
-      for (int t = off[e] / tile + tid; t < hi / tile; t += 1024) tile_expert[t] = e;
+  if (tid < 64) padded_offsets(cnt, off, E, tile_shift, num_tiles, group_end, b == 0);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int p = p0 + 1024 * i, x = mine[i] >> 16;
+    if (p < npairs) {
+      const int pos = off[x] + pre[x] + (mine[i] & 0xffff);
+      slots[pos] = p;
+      pair_slot[p] = pos;
     }
-    for (int s = total + tid; s < slots_cap; s += 1024) slots[s] = -1;
-    for (int t = total / tile + tid; t < tiles_cap; t += 1024) tile_expert[t] = -1;
   }
-  const int end = min(npairs, (b + 1) * kAlignChunk);
-  for (int p = b * kAlignChunk + tid; p < end; p += 1024) {
-    const int e = ids[p];
-    const int pos = off[e] + pre[e] + atomicAdd(&cur[e], 1);
-    slots[pos] = p;
-    pair_slot[p] = pos;
+  const int total = off[128];
+  for (int x = b; x < E; x += nb) {   // the rest of the experts' last tiles, their tiles' labels
+    for (int s = off[x] + cnt[x] + tid; s < off[x + 1]; s += 1024) slots[s] = -1;
+    for (int t = (off[x] >> tile_shift) + tid; t < off[x + 1] >> tile_shift; t += 1024) tile_expert[t] = x;
   }
+  for (int s = total + b * 1024 + tid; s < slots_cap; s += nb * 1024) slots[s] = -1;
+  for (int t = (total >> tile_shift) + b * 1024 + tid; t < tiles_cap; t += nb * 1024) tile_expert[t] = -1;
 }
 
-int moe_align_blocks(int npairs) { return npairs > 4 * kAlignChunk ? (npairs + kAlignChunk - 1) / kAlignChunk : 1; }
+static int align_chunk(int npairs) { return npairs > 65536 ? 4096 : 1024; }
+int moe_align_blocks(int npairs) { return npairs > 4096 ? (npairs + align_chunk(npairs) - 1) / align_chunk(npairs) : 1; }
+bool moe_align_small(int npairs) { return npairs <= 16384; }
 
 // out[slot, N] = x[row(slot), K] . W[e, N, K]^T; row(slot) = pair / k (gather) or slot.
 // A tile = 16*MT consecutive slots of one expert; each W fragment feeds MT MFMAs.
@@ -463,24 +476,29 @@ void launch_moe_topk_softmax(const void* logits, bool logits_f32, float* w, int*
                                                                    T, E, k, renorm ? 1 : 0);
 }
 
-void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
-                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist) {
-  const int nb = moe_align_blocks(npairs);
-  if (nb > 1 && hist != nullptr) {
-    moe_count_kernel<<<nb, 1024, 0, s>>>(ids, npairs, hist);
-    moe_place_kernel<<<nb, 1024, 0, s>>>(ids, npairs, E, tile, hist, nb, slots, slots_cap, tile_expert, tiles_cap,
-                                         num_tiles, pair_slot, group_end);
+// tiles of a power of two; hist: [moe_align_blocks, 128] where that is more than one and there is one table
+static void align(int tables, const int* ids, const int* table, const long* tokens, int top, long table_rows, int npairs, int E, int tile, int* slots,
+                  int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, int* hist, hipStream_t s) {
+  const int top_shift = (top & (top - 1)) == 0 ? __builtin_ctz(top) : -1, shift = __builtin_ctz(tile), nb = moe_align_blocks(npairs);
+  if (nb > 1 && tables == 1) {
+    const bool wide = align_chunk(npairs) > 1024;
+    (wide ? moe_count_kernel<4> : moe_count_kernel<1>)<<<nb, 1024, 0, s>>>(ids, table, tokens, top, top_shift, table_rows, npairs, pair_slot, hist);
+    (wide ? moe_place_kernel<4> : moe_place_kernel<1>)<<<nb, 1024, 0, s>>>(npairs, E, shift, hist, nb, slots, slots_cap, tile_expert, tiles_cap,
+                                                                           num_tiles, pair_slot, group_end);
     return;
   }
-  moe_align_kernel<<<1, 1024, 0, s>>>(ids, nullptr, nullptr, 1, 0, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap,
-                                      num_tiles, pair_slot, group_end);
+  (npairs <= 1024 ? moe_align_kernel<1> : npairs <= 4096 ? moe_align_kernel<4> : moe_align_kernel<16>)<<<tables, 1024, 0, s>>>(
+      ids, table, tokens, top, top_shift, table_rows, npairs, E, shift, slots, slots_cap, tile_expert, tiles_cap, num_tiles, pair_slot, group_end);
+}
+
+void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
+                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist) {
+  align(1, ids, nullptr, nullptr, 1, 0, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap, num_tiles, pair_slot, group_end, hist, s);
 }
 
 void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
-                            int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot,
-                            hipStream_t s) {
-  moe_align_kernel<<<tables, 1024, 0, s>>>(nullptr, table, tokens, top, table_rows, npairs, E, tile, slots, slots_cap, tile_expert,
-                                      tiles_cap, num_tiles, pair_slot, nullptr);
+                            int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot, int* hist, hipStream_t s) {
+  align(tables, nullptr, table, tokens, top, table_rows, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap, num_tiles, pair_slot, nullptr, hist, s);
 }
 
 // Prefill MoE input: xs[slot] = x[slots[slot] / k] (the token of the pair in that

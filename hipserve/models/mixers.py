@@ -346,7 +346,7 @@ class TableMoE:
         T, dev = h.shape[0], h.device
         P = T * s.top
         if aligned is None and self._packed_ok(h, P):
-            return self._forward_packed(h, self.table.index_select(0, ids).reshape(-1), P)
+            return self._forward_packed(h, ids, P)
         if aligned is None:
             tile, (slots, tile_expert, pair_slot) = self._tables(P, dev)
             ops.moe_table_align(self.table, ids, s.experts, tile, slots, tile_expert, pair_slot)
@@ -365,7 +365,7 @@ class TableMoE:
                 and self.hidden % 256 == 0 and s.ff % 256 == 0
                 and P >= MOE_PACKED_MIN_PAIRS_PER_EXPERT * s.experts and not torch.cuda.is_current_stream_capturing())
 
-    def _forward_packed(self, h: torch.Tensor, experts: torch.Tensor, P: int):
+    def _forward_packed(self, h: torch.Tensor, ids: torch.Tensor, P: int):
         """Large bf16 batches: the experts as two launches of the packed-layout grouped GEMM (token rows
         gathered through the slot table inside the first one, squared ReLU in its epilogue)."""
         from ..ops import gemm
@@ -385,7 +385,10 @@ class TableMoE:
         tile_expert = torch.empty(cap // tile, dtype=torch.int32, device=dev)
         ntiles = torch.empty(1, dtype=torch.int32, device=dev)
         pair_slot = torch.empty(P, dtype=torch.int32, device=dev)
-        op.moe_align(experts, E, tile, slots, tile_expert, ntiles, pair_slot, None)
+        if self.ops.moe_tables_align_ok(self.table, ids, E):
+            self.ops.moe_table_align(self.table, ids, E, tile, slots, tile_expert, pair_slot, ntiles)
+        else:
+            op.moe_align(self.table.index_select(0, ids).reshape(-1), E, tile, slots, tile_expert, ntiles, pair_slot, None)
         pu, pd = self.packed
         act = torch.empty(cap, ff, dtype=h.dtype, device=dev)
         op.prefill_gemm_packed_grouped(act, h, pu, ff, 4, tile_expert, ntiles, gemm.PW_WM, gemm.PW_RW, slots, s.top)

@@ -778,6 +778,38 @@ def test_moe_table_align(tokens, top):
 
 
 @gpu
+@pytest.mark.parametrize("P", [1024, 1025, 4096, 4097, 16383, 65536, 65537])
+@pytest.mark.parametrize("E,tile", [(5, 128), (128, 16)])
+def test_moe_align_sizes(P, E, tile):
+    """One pair per thread and more, many workgroups of 1024 and 4096 pairs: the pairs of an expert in its tiles, the experts' tiles in order, nothing
+    else; looked up in a table as well, its tiles counted, and several tables by a workgroup each."""
+    g = torch.Generator().manual_seed(P + E)
+    table, tokens = torch.randint(0, E, (50, 1), generator=g).int(), torch.randint(0, 50, (P,), generator=g)
+    experts, ops = table[tokens].view(-1), get_ops("cuda")
+    counts = torch.bincount(experts.long(), minlength=E)
+    labels = torch.repeat_interleave(torch.arange(E), (counts + tile - 1) // tile).int()
+    cap = -(-(P + E * (tile - 1)) // tile) * tile
+
+    def check(slots, tiles, pair):
+        slots, tiles, pair = slots.cpu(), tiles.cpu(), pair.cpu().long()
+        assert torch.equal(slots[pair], torch.arange(P).int()) and int((slots == -1).sum()) == cap - P
+        assert torch.equal(tiles[:len(labels)], labels) and bool((tiles[len(labels):] == -1).all()) and torch.equal(tiles[pair // tile], experts)
+    made = lambda *n: [torch.full((*n, k), 7, dtype=torch.int32, device="cuda") for k in (cap, cap // tile, P)]  # noqa: E731
+    out = made()
+    ops.moe_align(experts.cuda(), E, tile, *out)
+    check(*out)
+    if P <= 16384:
+        out, count = made(), torch.empty(1, dtype=torch.int32, device="cuda")
+        ops.moe_table_align(table.cuda(), tokens.cuda(), E, tile, *out, count)
+        check(*out)
+        assert int(count) == len(labels)
+        out = made(2)
+        ops.moe_table_align(torch.stack([table] * 2).cuda(), tokens.cuda(), E, tile, *out)
+        for i in range(2):
+            check(*(x[i] for x in out))
+
+
+@gpu
 @pytest.mark.parametrize("tokens,top", [(1, 2), (48, 3), (1500, 2)])
 def test_moe_table_align_of_layers(tokens, top):
     """Every table's tiles in one launch, as one by one."""
