@@ -17,7 +17,8 @@
 // whose k is not finite or a pre-activation of which is NaN (infinite ones saturate).
 // What bounds it: the prepared operands (6816 floats per head and chunk) are written and read once, and the scan's products.
 // 8192 rows (4 prompts) x 32 heads: rows prepared one by one and scanned token by token (five row vectors through LDS for
-// every 4 state elements of a lane) took 126 + 700 us; this 177 + 144.
+// every 4 state elements of a lane) took 126 + 700 us; this 171 + 144 (188 before the products of the
+// decays were a channel per lane of one wave, three swaps and seven selects for each).
 // Errors against 64 bits, over 32 .. 2048 tokens, fresh and carried states, strong and weak decays: state 5.8e-8 - 6.4e-8 (token by
 // token 6.3e-8 - 7.0e-8), outputs before their norm 7.2e-8 - 7.9e-8 (9.2e-8 - 9.8e-8). What it takes: decays and their products
 // in 64 bits, rounded once into the operands (else 7.9e-8 for the state); Pa and Pk summed in 64 bits and the larger part of an output added
@@ -29,7 +30,6 @@ namespace hipserve {
 namespace {
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
-typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kC = 16, kD = 64, kLd = kD + 4;   // tokens per chunk; key and value channels of a head; LDS row
 
@@ -62,28 +62,6 @@ HS_DEVICE double decay_of(float s) {
   return p * 0.738403149974731;   // exp(-e^-1/2 / 2)
 }
 
-// Of the two rows that differ in bit 4 (bit 5) of the lane, the other's number.
-HS_DEVICE double of_row_16(double x, bool odd) {
-  const u32x2 u = __builtin_bit_cast(u32x2, x);
-  u32x2 y;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const auto a = __builtin_amdgcn_permlane16_swap(u[i], u[i], false, false);
-    y[i] = odd ? a[0] : a[1];
-  }
-  return __builtin_bit_cast(double, y);
-}
-HS_DEVICE double of_row_32(double x, bool high) {
-  const u32x2 u = __builtin_bit_cast(u32x2, x);
-  u32x2 y;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const auto a = __builtin_amdgcn_permlane32_swap(u[i], u[i], false, false);
-    y[i] = high ? a[0] : a[1];
-  }
-  return __builtin_bit_cast(double, y);
-}
-
 HS_DEVICE f32x4 ld4(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
 HS_DEVICE f32x4 mfma(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -91,18 +69,23 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
     float* __restrict__ base, const unsigned short* __restrict__ proj, long ld, const float* __restrict__ wl,
     const float* __restrict__ a_b, const float* __restrict__ w0, const int* __restrict__ seq_cu, int nseq, int heads) {
   __shared__ __attribute__((aligned(16))) float su[kC][kLd], sr[kC][kLd], sa[kC][kLd], sk[kC][kLd], sv[kC][kLd];
-  __shared__ __attribute__((aligned(16))) float sx[kC][kLd], sy[kC][kLd];   // KA, KK
-  __shared__ __attribute__((aligned(16))) double sg[4][kD];                 // decays of four rows
-  __shared__ __attribute__((aligned(16))) float sA[kC][20], sB[kC][20], sM[kC][20];
+  // The products of the decays before and after a token, then, where those are, KA and KK, and A, B and M: 39 KB for four workgroups per CU.
+  constexpr int kBytes = kC * kD * 8, kAt = 2 * kC * kLd * 4;
+  __shared__ __attribute__((aligned(16))) unsigned char pool[kAt + kBytes];
+  static_assert(kAt >= kBytes && 3 * kC * 20 * 4 <= kBytes, "two regions");
+  auto sbefore = reinterpret_cast<double(*)[kD]>(pool), safter = reinterpret_cast<double(*)[kD]>(pool + kAt);
+  auto sx = reinterpret_cast<float(*)[kLd]>(pool), sy = sx + kC;   // KA, KK
+  auto sA = reinterpret_cast<float(*)[20]>(pool + kAt), sB = sA + kC, sM = sB + kC;
   __shared__ float sf[2][kC];   // NaN: what reaches every column of a token's, its r, is not finite
   __shared__ int sv_bad[kD];    // a column's first value that is not finite
   int s, t0;
   if (!find_row_tile(seq_cu, 0, nseq, kC, blockIdx.y, s, t0)) return;
-  const int h = blockIdx.x, tid = threadIdx.x, row = tid >> 4, ch = 4 * (tid & 15);
+  const int h = blockIdx.x, tid = threadIdx.x, row = tid >> 4, ch = 4 * (tid & 15), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r0 = seq_cu[s] + t0, nt = min(kC, seq_cu[s + 1] - r0), N = heads * kD;
   const Buf out = buf_of(base, (long)blockIdx.y * heads + h);
   const bool in = row < nt;
   if (tid < kD) sv_bad[tid] = kC;
+  f32x4 ka, kk;
   {
     const long t = r0 + (in ? row : 0);
     const int c = h * kD + ch;
@@ -140,28 +123,37 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
       if (!use || lost[e]) v[e] = 0.f;
       if (!use || fr != 0.f) r[e] = 0.f;
     }
-    // the decays of the chunk's earlier and later tokens: of the wave's four rows by row swaps, of the other waves' through LDS
-    double before[4], after[4];
-    const bool odd = row & 1, high = row & 2;
+    // the products of the decays of the chunk's earlier and later tokens, a channel per lane of a wave that has little else to do
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const double next = of_row_16(dec[e], odd), pair = dec[e] * next, other = of_row_32(pair, high);
-      before[e] = (odd ? next : 1.0) * (high ? other : 1.0);
-      after[e] = (odd ? 1.0 : next) * (high ? 1.0 : other);
-      if ((row & 3) == 0) sg[row >> 2][ch + e] = pair * other;
-    }
+    for (int e = 0; e < 4; ++e) sbefore[row][ch + e] = dec[e];
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (lost[e]) atomicMin(&sv_bad[ch + e], row);
-    const int group = __builtin_amdgcn_readfirstlane(row >> 2);
+    if (wave == 1) {
+      double d[kC], p = 1.0;
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      if (m == group) continue;
+      for (int i = 0; i < kC; ++i) d[i] = sbefore[i][lane];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) (m < group ? before : after)[e] *= sg[m][ch + e];
+      for (int i = 0; i < kC; ++i) {
+        sbefore[i][lane] = p;
+        p *= d[i];
+      }
+      p = 1.0;
+#pragma unroll
+      for (int i = kC - 1; i >= 0; --i) {
+        safter[i][lane] = p;
+        p *= d[i];
+      }
     }
-    f32x4 ka, kk, upto, U, R, A, K, V;
+    __syncthreads();
+    double before[4], after[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      before[e] = sbefore[row][ch + e];
+      after[e] = safter[row][ch + e];
+    }
+    f32x4 upto, U, R, A, K, V;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {   // each rounded once
       const double d = before[e] * dec[e], seed = (double)__builtin_amdgcn_rcpf((float)d);
@@ -182,25 +174,21 @@ __global__ __launch_bounds__(256) void delta_rule_chunk_prepare_kernel(
     *reinterpret_cast<f32x4*>(&sv[row][ch]) = V;
     *reinterpret_cast<f32x4*>(out.R + place(row) * kD + ch) = R;
     if (row == kC - 1) *reinterpret_cast<f32x4*>(out.E + ch) = upto;
+    __syncthreads();   // the products are read
     *reinterpret_cast<f32x4*>(&sx[row][ch]) = ka;
     *reinterpret_cast<f32x4*>(&sy[row][ch]) = kk;
-    __syncthreads();
   }
-  if (tid < kD) {
-    int first = sv_bad[tid];
-    bool any = false;
-    for (int m = kC - 1; m >= 0; --m) {
-      if (sf[0][m] != 0.f) first = min(first, m);
-      any |= sf[1][m] != 0.f;
-    }
-    out.B[tid] = (float)first;
-    any = __any(any || first < kC);
-    if (tid < kC) out.F[tid] = sf[1][tid];
-    if (tid == 0) *out.any = any ? 1.f : 0.f;
+  if (wave == 1) {
+    const unsigned long all = __ballot(lane < kC && sf[0][lane & 15] != 0.f), rs = __ballot(lane < kC && sf[1][lane & 15] != 0.f);
+    const int first = min(sv_bad[lane], all ? __builtin_ctzll(all) : kC);
+    out.B[lane] = (float)first;
+    const bool any = __any(first < kC) || rs != 0;
+    if (lane < kC) out.F[lane] = sf[1][lane];
+    if (lane == 0) *out.any = any ? 1.f : 0.f;
   }
   // all pairs of tokens: wave 0 A, 1 B in four chains, 2 Pa, 3 Pk in 64 bits (in 32, the outputs' largest error; A and B in 64
   // bits too: 18 us more and no smaller an error); lane (c, g) gets rows 4 g + r of column c, in 64 bits rows 4 r + g
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+  const int c = lane & 15, g = lane >> 4;
   {
     const float(*x)[kLd] = wave < 2 ? su : sr;
     const float(*y)[kLd] = wave & 1 ? sk : sa;
