@@ -8,7 +8,7 @@
 // so a chunk costs a few small matrix products instead of 16 dependent passes over the state. The ratios G_i / G_j are
 // formed as products of the decays between the two tokens (never as a quotient), so strong decays only underflow.
 //
-// delta_chunk_prepare: everything that does not need the state, one workgroup per (head, chunk): A, P, the inverse
+// delta_chunk_prepare (a decay per channel), delta_chunk_prepare_head: everything that does not need the state, one workgroup per (head, chunk): A, P, the inverse
 // M = (1 + diag(beta) A)^-1 diag(beta) by forward substitution, and W = -M (G k), U0 = M v, G q, G_15 / G k, G_15.
 // delta_chunk_scan: one workgroup per (sequence, head, 16 or 32 value channels) walks the chunks: U = U0 + W S,
 // o = (G q) S + P U, S = G_15 S + (G_15 / G k)^T U on mfma_f32_16x16x4f32. The state stays in registers in the
@@ -19,6 +19,8 @@
 
 namespace hipserve {
 namespace {
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kC = 16;   // tokens per chunk
 
@@ -63,8 +65,8 @@ HS_DEVICE int in_tiles_t(int channel, int token) {
   return ((channel >> 4) * 64 + (token >> 2) * 16 + (channel & 15)) * 4 + (token & 3);
 }
 
-// 16 DPP rows of 16 lanes: row i is token i; lane `seg` of a row owns channels 16 VD j + VD seg + e (DS in all).
-template <int DS, bool CH>
+// A decay per key channel. 16 DPP rows of 16 lanes: row i is token i; lane `seg` of a row owns channels 16 VD j + VD seg + e (DS in all).
+template <int DS>
 __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
     float* __restrict__ base, const float* __restrict__ qk, const float* __restrict__ vv, const float* __restrict__ gg,
     const float* __restrict__ bb, const int* __restrict__ seq_cu, int nseq, int heads, int kv_heads, int dim, int vdim,
@@ -89,14 +91,13 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
   for (int j = 0; j < NJ; ++j) {
     const int c = 16 * VD * j + VD * seg;
     const float* pq = qk + t * 2 * nqk + kh * dim + c;
-    const float* pg = CH ? gg + (t * heads + h) * dim + c : gg + t * heads + h;
+    const float* pg = gg + (t * heads + h) * dim + c;
     if (VD == 4 && dim % 4 == 0) {   // four channels are inside together, rows are 16-byte aligned
       f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a, g = {1.f, 1.f, 1.f, 1.f};
       if (in && c < dim) {
         a = *reinterpret_cast<const f32x4*>(pq + nqk);
         b = *reinterpret_cast<const f32x4*>(pq);
-        if constexpr (CH) g = *reinterpret_cast<const f32x4*>(pg);
-        else g = f32x4{*pg, *pg, *pg, *pg};
+        g = *reinterpret_cast<const f32x4*>(pg);
       }
 #pragma unroll
       for (int e = 0; e < VD; ++e) { xk[j][e] = a[e]; xq[j][e] = b[e]; g0[j][e] = g[e]; }
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
         const bool ok = in && c + e < dim;
         xk[j][e] = ok ? pq[nqk + e] : 0.f;
         xq[j][e] = ok ? pq[e] : 0.f;
-        g0[j][e] = ok ? pg[CH ? e : 0] : 1.f;
+        g0[j][e] = ok ? pg[e] : 1.f;
       }
     }
     Row<float, VD>::st(&sk[row][c], xk[j]);
@@ -228,6 +229,145 @@ __global__ __launch_bounds__(256) void delta_chunk_prepare_kernel(
 #pragma unroll
     for (int q = 0; q < kC; q += 4)
       *reinterpret_cast<f32x4*>(out.UT + in_tiles_t(v, q)) = f32x4{u[q], u[q + 1], u[q + 2], u[q + 3]};
+  }
+}
+
+// The same for a decay per head, where all that the channels differ in are products of matrices: the pairs k_i k_j and q_i k_j on the
+// matrix cores, a quarter of the channels per wave, times the decays between the two tokens; W and U0 with M as an operand, whose results lie as
+// the scan's lanes take them. What bounds it are the bytes, 34 KB written per head and chunk: 8192 rows (4 prompts) x 16 heads of 128 x 128 with a
+// walk through the tokens per row, as above, 126 us, now 90; 16 prompts of 200 56 -> 39. Errors against 64 bits beside the token by token scan's, over
+// 100 - 700 tokens, weak and strong decays: states 0.82 - 1.33 of them (0.87 - 1.34 before), outputs 0.96 - 1.28 (1.11 - 1.40): the pairs of
+// queries and keys and the products of decays are formed in 64 bits and rounded once (in 32 bits, four chains per wave, 0.99 - 1.43 and 5 us less).
+template <int DS>
+__global__ __launch_bounds__(256) void delta_chunk_prepare_head_kernel(
+    float* __restrict__ base, const float* __restrict__ qk, const float* __restrict__ vv, const float* __restrict__ gg,
+    const float* __restrict__ bb, const int* __restrict__ seq_cu, int nseq, int heads, int kv_heads, int dim, int vdim, int VP) {
+  constexpr int DP = 16 * DS, LD = DP + 4, NK = DS < 4 ? DS : 4, KS = DP / 4 / NK;   // waves that share the channels; k steps of each
+  __shared__ __attribute__((aligned(16))) float sk[kC][LD], sq[kC][LD];
+  __shared__ __attribute__((aligned(16))) f32x4 part[NK][64];
+  __shared__ __attribute__((aligned(16))) f64x4 partq[NK][64];
+  __shared__ float sA[kC][kC + 1], sM[kC][kC + 4], sMG[kC][kC + 4];
+  __shared__ float sg[kC], sb[kC], sG[kC], sE[kC];   // decays, rates, products up to a token and after it
+  int s, t0;
+  if (!find_chunk(seq_cu, nseq, blockIdx.y, s, t0)) return;
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+  const int r0 = seq_cu[s] + t0, nt = min(kC, seq_cu[s + 1] - r0);
+  const int nqk = kv_heads * dim, nv = heads * vdim, kh = h / (heads / kv_heads);
+  const ChunkBuf out = chunk_buf(base, (long)blockIdx.y * heads + h, DP, VP);
+  // a value tile's second operand: four tokens of a channel
+  auto values = [&](int t, f32x4& v) {
+    const int ch = 16 * t + c;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = vv[(long)(r0 + min(4 * r + g, nt - 1)) * nv + h * vdim + min(ch, vdim - 1)];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = 4 * r + g < nt && ch < vdim ? v[r] : 0.f;
+  };
+  f32x4 v0 = {0.f, 0.f, 0.f, 0.f}, v1 = v0;   // of the wave's first two tiles, loaded early
+  if (16 * wave < VP) values(wave, v0);
+  if (16 * (wave + 4) < VP) values(wave + 4, v1);
+  const bool vec = dim % 4 == 0;
+  for (int i = tid; i < kC * DP / 4; i += 256) {
+    const int row = i / (DP / 4), ch = i % (DP / 4) * 4;
+    f32x4 k = {0.f, 0.f, 0.f, 0.f}, q = k;
+    if (row < nt && ch < dim) {
+      const float* p = qk + (long)(r0 + row) * 2 * nqk + kh * dim + ch;
+      if (vec) {
+        q = *reinterpret_cast<const f32x4*>(p);
+        k = *reinterpret_cast<const f32x4*>(p + nqk);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (ch + e < dim) { q[e] = p[e]; k[e] = p[nqk + e]; }
+      }
+    }
+    *reinterpret_cast<f32x4*>(&sk[row][ch]) = k;
+    *reinterpret_cast<f32x4*>(&sq[row][ch]) = q;
+  }
+  if (tid < kC) {
+    const long at = (long)(r0 + min(tid, nt - 1)) * heads + h;
+    const float d = gg[at], beta = bb[at];
+    sg[tid] = tid < nt ? d : 1.f;
+    sb[tid] = tid < nt ? beta : 0.f;
+  }
+  __syncthreads();
+  if (wave < NK) {   // lane (c, g): rows 4 g + r of column c, in 64 bits rows 4 r + g
+    f32x4 a[4] = {};
+    f64x4 p = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int st = 0; st < KS; ++st) {
+      const int ch = 4 * (wave * KS + st) + g;
+      const float k = sk[c][ch], q = sq[c][ch];
+      a[st & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(k, k, a[st & 3], 0, 0, 0);
+      p = __builtin_amdgcn_mfma_f64_16x16x4f64((double)q, (double)k, p, 0, 0, 0);
+    }
+    part[wave][lane] = (a[0] + a[1]) + (a[2] + a[3]);
+    partq[wave][lane] = p;
+  }
+  // the products of the decays between two tokens, never a quotient; row i, column j
+  const int i = tid >> 4, j = tid & 15;
+  double exact = 1.0;   // rounded once: a factor that all channels share
+#pragma unroll
+  for (int m = kC - 1; m > 0; --m) exact *= m <= i && m > j ? (double)sg[m] : 1.0;
+  const float ratio = (float)exact;
+  if (j == 0) sG[i] = (float)(exact * (double)sg[0]);
+  if (i == kC - 1) sE[j] = ratio;
+  __syncthreads();
+  {
+    float a = 0.f;
+    double p = 0.0;
+#pragma unroll
+    for (int w = 0; w < NK; ++w) {
+      a += reinterpret_cast<const float*>(&part[w][(i >> 2) * 16 + j])[i & 3];
+      p += reinterpret_cast<const double*>(&partq[w][(i & 3) * 16 + j])[i >> 2];
+    }
+    sA[i][j] = j < i ? a * ratio : 0.f;
+    out.P[64 * (j & 3) + 16 * (j >> 2) + i] = j <= i ? (float)(p * exact) : 0.f;   // by k step and lane of the scan
+  }
+  __syncthreads();
+  if (tid < kC) {   // column tid of M: (1 + diag(beta) A) x = beta e
+    float x[kC];
+    const float G = sG[tid];
+#pragma unroll
+    for (int i = 0; i < kC; ++i) {
+      float r = 0.f;
+#pragma unroll
+      for (int j = 0; j < i; ++j) r = __builtin_fmaf(sA[i][j], x[j], r);
+      x[i] = sb[i] * ((i == tid ? 1.f : 0.f) - r);
+      sM[i][tid] = x[i];
+      sMG[i][tid] = -x[i] * G;
+    }
+  } else if (tid >= 64) {   // G q, G_15 / G k as they lie in tiles, by the other waves
+    for (int t = wave - 1; t < DS; t += 3) {
+      f32x4 q = *reinterpret_cast<const f32x4*>(&sq[c][16 * t + 4 * g]), k;
+      q *= sG[c];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) k[r] = sk[4 * g + r][16 * t + c] * sE[4 * g + r];
+      *reinterpret_cast<f32x4*>(out.GQ + (t * 64 + lane) * 4) = q;
+      *reinterpret_cast<f32x4*>(out.KT + (t * 64 + lane) * 4) = k;
+    }
+    for (int ch = tid - 64; ch < DP; ch += 192) out.GE[ch] = sG[kC - 1];
+  }
+  __syncthreads();
+  float mg[4], m[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    mg[r] = sMG[c][4 * r + g];
+    m[r] = sM[c][4 * r + g];
+  }
+  for (int t = wave; t < DS; t += 4) {
+    f32x4 w = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; ++r) w = __builtin_amdgcn_mfma_f32_16x16x4f32(sk[4 * r + g][16 * t + c], mg[r], w, 0, 0, 0);
+    *reinterpret_cast<f32x4*>(out.W + (t * 64 + lane) * 4) = w;
+  }
+  for (int t = wave; 16 * t < VP; t += 4) {
+    f32x4 v, u = {0.f, 0.f, 0.f, 0.f};
+    if (t == wave) v = v0;
+    else if (t == wave + 4) v = v1;
+    else values(t, v);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) u = __builtin_amdgcn_mfma_f32_16x16x4f32(m[r], v[r], u, 0, 0, 0);
+    *reinterpret_cast<f32x4*>(out.UT + (t * 64 + lane) * 4) = u;
   }
 }
 
@@ -443,11 +583,10 @@ void launch_delta_chunk(float* o, float* S, float* buf, const float* qk, const f
 #define HS_DC(DS, TPW, NW, NC)                                                                                             \
   do {                                                                                                                 \
     if (channel)                                                                                                       \
-      delta_chunk_prepare_kernel<DS, true><<<pgrid, 256, 0, s>>>(buf, qk, vv, gg, bb, seq_cu, nseq, heads, kv_heads, dim,  \
+      delta_chunk_prepare_kernel<DS><<<pgrid, 256, 0, s>>>(buf, qk, vv, gg, bb, seq_cu, nseq, heads, kv_heads, dim,  \
                                                                  vdim, VP);                                            \
     else                                                                                                               \
-      delta_chunk_prepare_kernel<DS, false><<<pgrid, 256, 0, s>>>(buf, qk, vv, gg, bb, seq_cu, nseq, heads, kv_heads, dim, \
-                                                                  vdim, VP);                                           \
+      delta_chunk_prepare_head_kernel<DS><<<pgrid, 256, 0, s>>>(buf, qk, vv, gg, bb, seq_cu, nseq, heads, kv_heads, dim, vdim, VP); \
     delta_chunk_scan_kernel<TPW, NW, NC><<<dim3(heads, (VP + 16 * NC - 1) / (16 * NC), nseq), 64 * NW, 0, s>>>(            \
         o, S, buf, seq_cu, seq_ctx, seq_state, heads, dim, vdim, VP);                                                      \
   } while (0)
