@@ -274,7 +274,7 @@ void launch_delta_rule(void* out, long out_ld, float* S, const void* proj, long 
                        const int* seq_state, int nseq, int T, float* scratch, int heads, int dim, float eps,
                        float out_scale, bool f32, float* chunks, hipStream_t s);
 // The generalized rule in chunks (delta_rule_chunk.hip), bf16 rows, heads of 64: launch_delta_rule with
-// delta_rule_chunk_floats() floats in `chunks` (scratch then holds o [T, heads * 64] and 64 floats behind it).
+// delta_rule_chunk_floats() floats in `chunks` (scratch then holds o [T, heads * 64]; 64 floats behind it are not used).
 bool delta_rule_chunk_ok(int heads, int dim, const void* proj, long ld);
 long delta_rule_chunk_floats(int T, int nseq, int heads);
 void launch_delta_rule_chunk(float* o, float* S, float* buf, const void* proj, long ld, const float* wl, const float* a_b,
