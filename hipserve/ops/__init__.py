@@ -650,9 +650,11 @@ class KernelOps:
         after = max(0.0, self._skinny_time(rows, 3 * cols, cols, False, f32) - self._vendor_time(rows, 3 * cols, cols, f32))
         return self._skinny_time(rows, cols, k, False, f32) + 0.6 + after <= apart + 2.5 + 0.05 * rows * cols / 1024
 
-    def _update_cols(self, rows, cols, k, f32) -> int:
-        """Columns that a workgroup of the update takes, and that a sum of squares is over."""
-        return 8 if cols <= 2048 and self._moe_lib.skinny_half(rows, cols, k, f32) else 16
+    @staticmethod
+    def _update_cols(rows, cols, k, f32) -> int:
+        """Columns that a workgroup of the update takes, and that a sum of squares is over: as skinny_half (skinny_linear.hip) has it for
+        up to 32 rows."""
+        return 8 if cols <= 2048 and k * (2 if f32 else 1) > (4096 if rows <= 8 and cols <= 1024 else 1024) else 16
 
     def linear_update(self, x, w, bias, residual, norm_w, eps):
         """residual += x . w^T + bias, and the rows for the next products as ``NormedRows`` of its norm; None, and nothing done, where the

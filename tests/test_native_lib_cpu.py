@@ -78,6 +78,18 @@ def test_choice_of_the_expert_kernels_by_load(experts, N, K, glu, by_pairs):
 
 
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
+def test_an_update_takes_the_columns_that_its_product_would():
+    from hipserve.ops import KernelOps
+    load_kernel_library("seq")
+    half = torch.ops.hipserve_seq.skinny_half
+    for rows in (1, 8, 9, 32):
+        for cols in (64, 1024, 1088, 2048, 2112, 4096):
+            for k in (512, 520, 1024, 1032, 2048, 2056, 4096, 4104):
+                for f32 in (False, True):
+                    assert (KernelOps._update_cols(rows, cols, k, f32) == 8) == half(rows, cols, k, f32), (rows, cols, k, f32)
+
+
+@pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
 @pytest.mark.parametrize("rows,cols,k,f32,glu,pays", [
     (1, 2048, 2048, False, False, True), (48, 2048, 2048, False, False, True), (64, 6144, 1024, False, False, True), (16, 32000, 1024, True, False, True),
     (48, 512, 8192, False, False, False), (40, 576, 12288, False, False, False), (64, 32768, 128, False, False, False), (64, 65536, 512, False, False, False),
