@@ -506,6 +506,14 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
       }
     }
   }
+  // A wave that sees none of a row's keys leaves zeros: a hidden key's weight of 0 does not hide an infinity or a NaN among its values.
+  if (__any(m == -INFINITY)) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int j = 0; j < E; ++j)
+        if (m == -INFINITY) acc[b][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   // lane (c, g): row c, dims 16 E b + E (4 g + i) + j
   const int nr = MULTI ? 16 : nh;   // rows
   float* ml = lds + nw * nr * D;
@@ -539,7 +547,7 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
 #pragma unroll
     for (int w = 0; w < 8; ++w) {
       if (w >= nw) break;
-      const float f = mw[w].x == -INFINITY ? 0.f : S::exp(mw[w].x - M);   // no key: sums and outputs are 0
+      const float f = mw[w].x == -INFINITY ? 0.f : S::exp(mw[w].x - M);   // no key: its sums and outputs are 0 (above)
       L += mw[w].y * f;
       o += part[w] * f;
     }

@@ -1383,6 +1383,29 @@ def test_window_attention_hidden_keys(dim, n, ctx, window, chunk, dtype):
 
 
 @gpu
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("chunk,at,rows", [(0, 23, slice(0, 8)), (16, 3, slice(8, 16))])
+def test_window_attention_fp32_values_of_hidden_tiles(dim, chunk, at, rows):
+    """Positions 8 .. 23 share a tile of rows, and two waves their keys 0 .. 15 and 16 .. 23: what a row's wave holds that sees none of its
+    keys, those after it or of the chunk before it, stays out of the row whatever their values are."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(dim + chunk)
+    n, ctx, heads = 16, 24, 2
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=heads, window=0, reach=chunk, scale=dim ** -0.5, sink=False, keep_first=0,
+                         softcap=0.0, channel_gate=False, chunk=chunk, diff=0.0)
+    cache, proj = torch.randn(2, 16, 2 * heads * dim, generator=g), torch.randn(n, heads * dim, generator=g).cuda()
+    meta = SimpleNamespace(seq_cu=torch.tensor([0, n]).int().cuda(), seq_ctx=torch.tensor([ctx]).int().cuda(), seq_bt=torch.arange(2).int().view(1, -1).cuda(),
+                           num_decode=0, num_prefill_tokens=n, max_ctx=ctx)
+    outs = []
+    for value in (0.0, float("nan"), -float("inf")):
+        cache[at // 16, at % 16, heads * dim:] = value
+        outs.append(torch.empty(n, heads * dim, device="cuda"))
+        get_ops("cuda").window_attention(outs[-1], proj, cache.cuda(), meta, sp, -1)
+    assert outs[0].isfinite().all() and not outs[1][n - 1 if chunk == 0 else 0].isfinite().any()
+    assert torch.equal(outs[1][rows], outs[0][rows]) and torch.equal(outs[2][rows], outs[0][rows])
+
+
+@gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("heads,kv,dim,ctxs,nfreq,mode,own,opts", [
     (1, 1, 64, [1], 0, 0, True, {}), (16, 4, 128, [1, 31, 32, 33, 700], 64, 1, True, {"v_norm": True}),
