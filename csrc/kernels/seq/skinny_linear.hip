@@ -244,16 +244,13 @@ int skinny_tiles(int M, long tiles, int K) {
 }
 
 // us of a launch (K in halves, over `parts`): a latency, the results, and the time the weights take at 5.2 TB/s, or, where that is more, at 9 TB/s and with it
-// what the busiest compute unit takes in (80 KB per us), its sums in LDS and its products of 32-bit operands. 9 % off over the sizes above.
-// From the third round on two workgroups of two tiles share a compute unit and hide a quarter of it, measured where the choice turns on it: 32000 x
-// 2048 with 32, 48 rows 28.5, 32.7 us (32.7, 37.4 without that, so that the vendor's 35.6 was taken for 48), 65536 x 2048 with 32 55.5 (vendor 66.9);
-// with fewer k or more than 48 rows the vendor's is the faster one there (50000 x 1024 with 40 rows 26.8 / 22.6, 65536 x 2048 with 56 75 / 72).
+// what the busiest compute unit takes in (80 KB per us), its sums in LDS and its products of 32-bit operands. 9 % off on average over 5127 sizes (1 -
+// 64 rows, 64 - 65536 columns, k 128 - 12288, plain and gated, 32 bits).
 double skinny_time_of(int M, long cols, double K, int nt, int parts, bool f32, double out_bytes, bool half = false) {
   const long wgs = ((cols + 15) / 16 + nt - 1) / nt * parts, rounds = (wgs + 255) / 256;   // of whole tiles; halves are one round
   const double bytes = 2.0 * cols * K, rows = (M + 7) / 8 * 8, k = K / parts, st = nt * ((M + 15) / 16);
   const double each = 2.0 * k * ((half ? 8 : 16 * nt) + rows) / 80e3 + st * (0.09 + (f32 ? 8.5e-5 * k : 0));
-  const double hidden = nt == 2 && wgs > 512 && parts == 1 && !f32 && M <= 48 && K >= 2048 && K < 4096 ? 0.25 : 0.0;
-  return 2.16 + std::max(bytes / 5.2e6, bytes / 9e6 + (1.0 - hidden) * rounds * each) + 0.7e-6 * out_bytes;
+  return 2.16 + std::max(bytes / 5.2e6, bytes / 9e6 + rounds * each) + 0.7e-6 * out_bytes;
 }
 
 }  // namespace

@@ -535,11 +535,11 @@ class KernelOps:
     def _skinny_pays(self, rows: int, cols: int, k: int, glu: bool = False, f32: bool = False, act: bool = False) -> bool:
         """Whether ``skinny_linear`` is expected to be faster than the vendor's GEMM for ``rows`` x ``cols`` results (``cols`` over all
         batches), both sides in us for cold weights: ours as the kernel's choice of tiles has it (skinny_time in skinny_linear.hip), the vendor's as
-        the choice between them comes out best. Over 2541 sizes (1 - 64 rows, 64 - 65536 columns, k 128 - 12288, both types) it takes 1 % longer
-        than the faster of the two. Examples, ours / vendor: 2048 x 2048 with 1, 16, 48, 64 rows 4.2 / 10.1, 4.9 / 10.2, 6.8 / 10.7, 7.6 / 11.1; 6144 x
-        2048 with 1, 16, 48 rows 7.7 / 12.4, 8.4 / 12.3, 10.9 / 13.4; 4096 x 12288 with 1, 16, 48 rows 19.4 / 21.1, 23.8 / 22.3, 33.9 / 32.5; 512 x
-        8192 with 48 rows 16.3 / 11.1; 32000 x 2048 with 9, 16, 48, 64 rows 24.8 / 31.6, 26.8 / 31.5, 32.3 / 35.6, 36.8 / 32.2; in 32 bits 1024 x
-        1024 with 3, 16, 48 rows 4.2 / 8.3, 4.4 / 8.3, 7.3 / 8.3; 32000 x 2048 with 1, 16, 64 rows 44 / 57, 48 / 59, 82 / 68."""
+        the choice between them comes out best. Over 5127 sizes (1 - 64 rows, 64 - 65536 columns, k 128 - 12288, plain and gated, 32 bits) it takes
+        1.2 % longer than the faster of the two. Examples, ours / vendor: 2048 x 2048 with 1, 16, 48, 64 rows 4.0 / 11.0, 4.3 / 11.0, 7.0 / 11.1, 7.7 /
+        11.7; 6144 x 2048 with 1, 16, 48 rows 7.0 / 12.5, 8.0 / 12.5, 10.2 / 13.1; 4096 x 12288 with 1, 16, 48 rows 20.4 / 22.0, 22.0 / 22.5, 33.6 /
+        32.1; 512 x 8192 with 48 rows 14.9 / 11.4; 32000 x 2048 with 1, 16, 48, 64 rows 25.0 / 32.3, 27.5 / 32.7, 33.3 / 37.4, 37.5 / 34.2; in 32 bits
+        1024 x 1024 with 1, 16, 48 rows 3.7 / 8.3, 3.8 / 8.8, 6.4 / 8.8; 32000 x 2048 with 1, 16, 64 rows 44 / 63, 51 / 65, 84 / 72."""
         # an activation is a launch more there (48 x 32000: 6 - 8 us)
         launch = 2.5 + 2.5e-6 * rows * cols if act and not glu else 0.0
         return self._skinny_time(rows, cols, k, glu, f32) < self._vendor_time(rows, cols, k, f32, glu) + launch
@@ -557,8 +557,13 @@ class KernelOps:
     @staticmethod
     def _vendor_time(rows, cols, k, f32, glu=False) -> float:
         """us of the vendor's GEMM (and of the gate's launch), which are by turns a fifth above and below any smooth rule: the constants are those
-        that made the fewest and smallest wrong choices beside ``skinny_time``, not the closest ones."""
+        that made the fewest and smallest wrong choices beside ``skinny_time``, not the closest ones. 16-bit weights whose rows lie a multiple of
+        4096 bytes apart come slower, up to k of 8192: 17 - 48 rows, TB/s at k of 1536, 2048, 2304, 3072, 3584, 4096, 5120, 6144 (mean of 16384 - 65536
+        columns) 3.8, 3.7, 4.6, 4.7, 4.9, 4.2, 5.1, 4.4. A tenth of the rate is what chooses best (0.07 - 0.1 alike; 5127 sizes: 1.33 % longer than the
+        faster one without it, 1.24 with it): 32000 x 2048 with 48 rows 33.3 / 37.4, 24576 x 4096 gated with 32 rows 40.1 / 49.0."""
         least, per_k, per_cols, start, rate = KernelOps.VENDOR[f32, glu][(min(rows, 64) - 1) // 16]
+        if not f32 and k % 2048 == 0 and k < 8192:
+            rate *= 0.91
         least += per_k * 1e-3 * k + (per_cols * math.log2(cols / 1024) if cols > 1024 else 0.0)
         return max(least, start + (4.0 if f32 else 2.0) * cols * k / 1e6 / rate)
 

@@ -94,10 +94,12 @@ def test_an_update_takes_the_columns_that_its_product_would():
     (1, 2048, 2048, False, False, True), (48, 2048, 2048, False, False, True), (64, 6144, 1024, False, False, True), (16, 32000, 1024, True, False, True),
     (48, 512, 8192, False, False, False), (40, 576, 12288, False, False, False), (64, 32768, 128, False, False, False), (64, 65536, 512, False, False, False),
     (56, 12288, 2048, True, False, False), (64, 12288, 512, True, False, False), (48, 576, 2048, True, False, False),
-    (16, 2048, 6144, True, True, False), (16, 4096, 12288, False, True, False), (1, 12288, 2048, False, True, True)])
+    (16, 2048, 6144, True, True, False), (16, 4096, 12288, False, True, False), (1, 12288, 2048, False, True, True),
+    (40, 25600, 3072, False, False, False), (40, 65536, 2560, False, False, False), (40, 25600, 3584, False, False, False), (48, 32000, 2048, False, False, True),
+    (32, 65536, 2048, False, False, True), (24, 50000, 2048, False, False, True), (32, 49152, 4096, False, True, True)])
 def test_products_of_a_few_rows_take_the_faster_kernel(rows, cols, k, f32, glu, pays):
     """Sizes at which one of the two was measured to be at least 10 % faster (the weight-streaming kernel where ``pays``), among them few columns
-    of many k, many columns of few k and matrix products that are bound by their 32-bit arithmetic."""
+    of many k, many columns of few k, matrix products that are bound by their 32-bit arithmetic and weights whose rows lie a multiple of 4096 bytes apart."""
     from hipserve.ops import KernelOps
 
     assert KernelOps().skinny_pays(rows, cols, k, glu, f32) == pays
