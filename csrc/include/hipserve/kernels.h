@@ -264,15 +264,14 @@ namespace hipserve {
 void launch_moe_topk_softmax(const void* logits, bool logits_f32, float* w, int* ids, int T, int E, int k,
                              bool renorm, hipStream_t s, int splits = 0);
 void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
-                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s,
-                      int* hist = nullptr);
+                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist);
 // the same for the pairs (t, j), expert table[i][tokens[t]][j] of `tables` tables [table_rows, top], outputs side by side (num_tiles
 // [tables]): a workgroup each, or many for a large step of one table (hist as below)
 void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
                             int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot,
                             int* hist, hipStream_t s);
-// blocks of the multi-workgroup moe_align for npairs (1: the single-workgroup kernel);
-// it needs hist = int32 [blocks * 128] scratch
+// Workgroups of moe_align for npairs. More than one need hist, int32 [moe_align_blocks(npairs) * 128] scratch (of one table; else it is not
+// looked at). The number does not grow with npairs (65536: 64, 65537: 17): it is asked for at every call.
 int moe_align_blocks(int npairs);
 bool moe_align_small(int npairs);   // what moe_table_align takes
 // xs[slot, H] = x[slots[slot] / k] (zeros for padding slots): grouped-GEMM input rows

@@ -23,6 +23,18 @@ def test_library_loads_and_registers_ops():
 
 
 @pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+@pytest.mark.parametrize("hist", ["", ", p"])
+def test_the_alignment_asks_for_its_scratch(hist, tmp_path):
+    """From 4097 pairs on many workgroups write counts there: a call without it does not compile."""
+    src = tmp_path / "k.cpp"
+    src.write_text('#include "hipserve/kernels.h"\n'
+                   f"void f(int* p, hipStream_t s) {{ hipserve::launch_moe_align(p, 5000, 8, 32, p, 6000, p, 200, p, p, nullptr, s{hist}); }}\n")
+    r = subprocess.run(["g++", "-std=c++17", "-fsyntax-only", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(_build.ROCM, "include"),
+                        "-I", os.path.join(_build.CSRC, "include"), src], capture_output=True, text=True)
+    assert (r.returncode == 0) == bool(hist), r.stderr
+
+
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
 @pytest.mark.parametrize("name", ["window_attention_dma", "latent_attention_dma", "skinny_linear", "expert_ffn", "mingru", "latent_attention_prompt"])
 def test_copies_into_lds_keep_their_wait_states(name, tmp_path):
     """The copies of lds_copy.h are inline assembly, which the compiler's hazard pass does not look into: between the scalar write of
