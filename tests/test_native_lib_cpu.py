@@ -65,6 +65,18 @@ def test_a_carried_state_is_asked_for_at_once(tmp_path):
     assert max(len(run) for run in "".join("w" if "s_waitcnt" in x else "l" for x in between[1:-1]).split("w")) >= 15
 
 
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+def test_a_gate_is_asked_for_beside_the_weights_of_the_runs(tmp_path):
+    """The merge of latent decode runs waits for the weights and the gate while the runs' rows are on their way."""
+    asm = tmp_path / "k.s"
+    subprocess.run([_build.HIPCC, *_build.HIP_FLAGS, "-I", os.path.join(_build.CSRC, "include"), "-S", "--cuda-device-only",
+                    os.path.join(_build.CSRC, "kernels", "seq", "latent_attention_mfma.hip"), "-o", asm], check=True, capture_output=True)
+    for rows in (4, 8, 12, 16):
+        code = re.split(rf"^_ZN\S*latent_attention_reduce_kernelILi{rows}E\S*:", asm.read_text(), maxsplit=1, flags=re.M)[1].split("s_endpgm")[0]
+        before, after = code.split("s_waitcnt vmcnt", 1)
+        assert after.startswith(f"({rows})") and before.count("global_load_ushort") == 1 and before.count("global_load_dwordx4") == rows, rows
+
+
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
 @pytest.mark.parametrize("experts,N,K,glu,by_pairs", [   # measured: whether the kernel for few rows per tile is the faster one
     (16, 1024, 2048, False, {2: True, 16: True, 64: True}), (16, 2048, 1024, False, {2: True, 12: True, 64: False}),
