@@ -108,14 +108,14 @@ void launch_mingru_scan(void* y, float* state, const void* proj, const float* b_
 // expert is < 0 or >= E (no weights) are skipped. act 0: none, 1: squared ReLU, 2: W[e] = [gate rows; up rows]
 // and out[slot, N / 2] = silu(gate) * up, 3: the same with g sigmoid(1.702 g) (u + 1), g = min(gate, limit),
 // u = clamp(up, -limit, limit). row_scale (may be null): the products of pair p are multiplied by row_scale[p] first.
-// pairs: how many (token, choice) pairs the tiles hold (0: guessed from their capacity). ntiles: tiles to launch, all of the capacity, or
-// fewer where those in use are known to be among them (bounded: they are counted, the alignments leave a pair in each).
+// pairs: how many (token, choice) pairs the tiles hold (0: guessed from their capacity; for the choice of kernel). ntiles: tiles to launch, all of the
+// capacity, or fewer where those in use are known to be among them (the alignments leave a pair in each of the first tiles).
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,
                         int ntiles_cap, int ntiles, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
-                        float limit, int pairs, bool bounded, bool f32, hipStream_t s);
+                        float limit, int pairs, bool f32, hipStream_t s);
 
-// Whether tiles of 32 slots that hold so many pairs run the kernel for few rows per tile.
-bool expert_gemm_skinny(long pairs, long ntiles_cap, long N, long K, long E, bool glu);
+// Whether so many launched tiles of 32 slots with so many pairs run the kernel for few rows per tile (cols of the result).
+bool expert_rows_pay(long ntiles, long pairs, long cols, long K);
 
 // Norms before and after a sublayer (sandwich.hip): residual[T, H] (fp32, in place; `table` [vocab, H] in the activation
 // type: it starts as table_scale * table[ids[t]]) += mult * y / rms(y) * w_post; out = residual / rms(residual) * w_next.

@@ -103,12 +103,14 @@ inline void expert_gemm(at::Tensor& out, const at::Tensor& x, const at::Tensor& 
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   hipserve::launch_expert_gemm(out.data_ptr(), x.data_ptr(), x.stride(0), w.data_ptr(), slots.data_ptr<int>(),
                                tile_expert.data_ptr<int>(), cap / tile, ntiles, tile, gather_k, N, K, act, w.size(0),
-                               (const float*)opt_ptr(row_scale), (float)limit, pairs, tiles > 0, f32,
+                               (const float*)opt_ptr(row_scale), (float)limit, pairs, f32,
                                c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream());
 }
 
-inline bool expert_gemm_skinny(int64_t pairs, int64_t ntiles_cap, int64_t N, int64_t K, int64_t E, bool glu) {
-  return hipserve::expert_gemm_skinny(pairs, ntiles_cap, N, K, E, glu);
+inline bool expert_rows_pay(int64_t tiles, int64_t pairs, int64_t cols, int64_t k) {
+  constexpr int64_t kMost = 1LL << 31;
+  TORCH_CHECK(tiles >= 0 && tiles < kMost && pairs >= 0 && pairs < kMost && cols >= 0 && cols < kMost && k >= 0, "expert_rows_pay: sizes");
+  return hipserve::expert_rows_pay(tiles, pairs, cols, k);
 }
 
 // out = act(x . w^T + bias) of at most 64 rows: x [M, K] or [B, M, K], w [N, K] or [B, N, K], out [M, N'] or [B, M, N'].
@@ -239,7 +241,7 @@ inline void def_moe_ops(torch::Library& m) {
   m.def("moe_align_small(int npairs) -> bool", &moe_align_small);
   m.def("expert_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor slots, Tensor tile_expert, int tile, int gather_k, "
         "int act, Tensor? row_scale=None, float limit=0.0, int pairs=0, int tiles=0) -> ()");
-  m.def("expert_gemm_skinny(int pairs, int ntiles_cap, int N, int K, int E, bool glu) -> bool", &expert_gemm_skinny);
+  m.def("expert_rows_pay(int tiles, int pairs, int cols, int k) -> bool", &expert_rows_pay);
 }
 
 inline void impl_moe_ops(torch::Library& m) {

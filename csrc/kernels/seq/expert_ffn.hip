@@ -9,7 +9,6 @@
 // computes a [32 slots x 64 columns] block, x and W staged through LDS in K-chunks of 32, fp32
 // accumulation; bf16 and fp32 element types.
 #include <algorithm>
-#include <cmath>
 
 #include "skinny.h"
 #include "hipserve/seq_kernels.h"
@@ -297,38 +296,22 @@ __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
 
 }  // namespace
 
-// Which of the two kernels serves tiles of 32 slots, where the caller says how many tiles are in use at most (`ntiles` of them are launched): the one for
-// few rows but for thousands of workgroups of 512 k and fewer, whose start costs more than their products. Of 280 sizes (4 to 256 experts, k 512 - 4096,
-// up to 200 pairs per expert, gated and not) it is the slower one in two others, by 3 % and 1 %. us, tile kernel / this one: 16 experts, 2048 x 1024: 22, 96
-// and 200 pairs 16.7 / 12.0, 17.1 / 14.7, 19.1 / 15.8; 8 experts, 4096 x 2048, 22 pairs 34.1 / 25.8; 64 experts, 704 x 2048, 96 pairs 47.0 / 25.8; 128 experts,
-// 2048 x 768, 64 pairs 39.5 / 30.5; but 256 experts, 2048 x 512, 256 pairs 64.5 / 78.9, 72 pairs 27.3 / 28.1.
-static bool expert_rows_pay(long ntiles, long No, long K) { return K >= 640 || (No + 15) / 16 * ntiles <= 8192; }
-
-// The same where the whole capacity is launched, as the two were before a tile's slots came to a workgroup with its expert; us, cold weights, 462 sizes of 4 to 256 experts, K from 512 to 4096 and up to 1600
-// pairs. Both read the weights of the experts that so many pairs hit on average. expert_gemm_skinny takes 3.1 plus them at 7 TB/s and what its
-// workgroups of 16 columns (gated 32) take in, the rows at 86 KB per us and CU, over K in whole rounds of its eight waves, and 0.37 per 1000
-// workgroups: it has one per 16 columns of every tile of the capacity. expert_gemm_mfma takes 4.2 plus the weights at 11 TB/s and the longest of
-// its steps of 128 k (they wait for their loads), the weights at 7.7 TB/s, and what its workgroups of 128 columns read at 37 KB per us and CU (rows once
-// per wave). Both are true to 8 %. Ungated products of few pairs per expert, where the two are close, keep the tile kernel until this one is a fifth
-// ahead. The choice takes 1.2 % longer than the faster one on average. Tile kernel / this one: 16 experts, 1024 x 2048: 2 pairs
-// 19.8 / 4.3, 82 pairs 26.0 / 15.7, 512 pairs 34.2 / 23.1; 2048 x 1024: 66 pairs 18.8 / 16.8, 400 pairs 33.6 / 22.2; 8 experts, 4096 x 2048:
-// 128 pairs 39.1 / 32.9; 64 experts, 2816 x 2048, gated: 4 pairs 23.0 / 12.3, 96 pairs 134 / 101; 128 experts, 1536 x 2048, gated: 16 pairs
-// 23.6 / 21.1; 2048 x 768: 8 pairs 12.2 / 14.6, 400 pairs 83 / 86; 256 experts, 2048 x 512: 8 pairs 10.2 / 19.6, 66 pairs 25.5 / 39.7. Two tiles of 16
-// columns per workgroup are hardly ever faster (16 experts, 2048 x 1024, 82 pairs: 19.1, 1400 pairs: 51).
-bool expert_gemm_skinny(long pairs, long ntiles_cap, long N, long K, long E, bool glu) {
-  const double used = E * (1 - std::pow(1 - 1.0 / E, (double)pairs)), mean = pairs / used, tiles = used * std::max(1.0, mean / 32 + 0.45);
-  const double launched = (double)((glu ? N / 2 : N) + 15) / 16 * ntiles_cap, bytes = used * N * K * 2, rows = std::min(32.0, mean);
-  const double cols = glu ? 32 : 16, whole = (K + 511) / 512 * 512;
-  const double mine = std::max(1.0, tiles * N / cols / 256) * (2 * whole * (cols / 300e3 + rows / 86e3) + 0.22);
-  const double ours = 3.1 + std::max(bytes / 5.7e6, 0.81 * bytes / 5.7e6 + mine) + 0.37e-3 * launched;
-  const double theirs = 4.2 + 0.7 * bytes / 7.7e6 +
-                        std::max({0.97 * K / 128, bytes / 7.7e6, std::max(1.0, tiles * N / 128 / 256) * 2 * K * (128 + 4 * rows) / 37.5e3});
-  return ours < (glu || mean > 17 ? 1.0 : 0.8) * theirs;
+// Which of the two kernels serves `ntiles` launched tiles of 32 slots that hold so many pairs: the one for few rows, but for thousands of workgroups of
+// 512 k and fewer, whose start costs more than their products, and where thousands of workgroups find no pair (0.37 us per 1000; only a launch of the
+// whole capacity has so many). 244 sizes of 4 to 256 experts, k 512 - 4096, 1 to 255 pairs per expert, gated and not, cold weights: 0.4 % longer than the
+// faster one on average, at most 15 %, with the whole capacity launched 0.4 and 17 %. us, tile kernel / this one: 16 experts, 2048 x 1024: 32, 128 and 4080
+// pairs 17.5 / 12.8, 18.0 / 16.0, 131 / 93; 8 experts, 4096 x 2048, 16 pairs 35.1 / 27.5; 64 experts, 2048 x 704, 128 and 16320 pairs 37.6 / 31.7, 344 /
+// 287; 128 experts, 2048 x 768, 64 pairs 40.2 / 31.1; but 32 experts, 1000 x 520, 4096 pairs 36 / 45, 256 experts, 2048 x 512, 512 and 65280 pairs 91 / 107, 987 /
+// 1086, and with all of 125 tiles launched for 4 pairs, 128 experts, 4096 x 1024, 14 / 27. Two tiles of 16 columns per workgroup are hardly ever
+// faster (16 experts, 2048 x 1024, 82 pairs: 19.1, 1400 pairs: 51).
+bool expert_rows_pay(long ntiles, long pairs, long cols, long K) {
+  const long per_tile = (cols + 15) / 16;
+  return (K >= 640 || per_tile * ntiles <= 8192) && per_tile * (ntiles - pairs) <= 8192;
 }
 
 void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, const int* slots, const int* tile_expert,
                         int ntiles_cap, int ntiles, int tile, int gather_k, int N, int K, int act, int E, const float* row_scale,
-                        float limit, int pairs, bool bounded, bool f32, hipStream_t s) {
+                        float limit, int pairs, bool f32, hipStream_t s) {
   if (ntiles_cap <= 0) return;
   // the capacity covers a partly filled tile per expert
   pairs = pairs > 0 ? pairs : std::max(1, ntiles_cap * tile - E * (tile - 1));
@@ -338,7 +321,7 @@ void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, cons
     auto o = (unsigned short*)out;
     auto xi = (const unsigned short*)x, wi = (const unsigned short*)w;
     if (tile == 32 && K < (1 << 24) && 2L * ntiles_cap * tile * x_ld < (1L << 32) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 &&
-        (bounded ? expert_rows_pay(ntiles, No, K) : expert_gemm_skinny(pairs, ntiles_cap, N, K, E, act >= 2))) {
+        expert_rows_pay(ntiles, pairs, No, K)) {
       const dim3 sg((No + 15) / 16, ntiles);
       const int shift = gather_k > 0 && (gather_k & (gather_k - 1)) == 0 ? __builtin_ctz(gather_k) : -1;
       if (act >= 2)

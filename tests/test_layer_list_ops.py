@@ -1546,3 +1546,30 @@ def test_expert_gemm_of_known_tiles(E, top, N, K, T, act):
             out = torch.full((cap, y.shape[1]), float("nan"), dtype=torch.bfloat16, device="cuda")
             ops.expert_gemm(out, src, w, slots, te, tile, k, act, pairs=P, tiles=tiles)
             assert ((out[ps.long()].double() - y).abs() <= 2.0 ** -8 * y.abs() + K * 2.0 ** -23 * size + 1e-30).all()
+
+
+@gpu
+@pytest.mark.parametrize("tile,dtype,E,top,N,K,T", [(64, torch.bfloat16, 5, 2, 264, 640, 70), (32, torch.bfloat16, 70, 1, 2048, 512, 70), (32, torch.bfloat16, 3, 2, 20, 72, 40),
+                                                    (32, torch.float32, 4, 2, 40, 652, 9), (64, torch.float32, 3, 1, 72, 100, 150)])
+def test_expert_gemm_of_known_tiles_by_the_other_kernels(tile, dtype, E, top, N, K, T):
+    """Fewer tiles launched than the capacity has, by the kernels for larger tiles, for thousands of workgroups of few k, for odd columns and for 32 bits:
+    the rows of all pairs, the same bits as with all tiles."""
+    g = torch.Generator().manual_seed(E + N)
+    P = T * top
+    x, w = torch.randn(T, K, generator=g).to(dtype).cuda(), (torch.randn(E, N, K, generator=g) / K ** 0.5).to(dtype).cuda()
+    ids = torch.arange(P).remainder(E).int().cuda()
+    ops, cap = get_ops("cuda"), -(-(P + E * (tile - 1)) // tile) * tile
+    slots, te, ps = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (cap, cap // tile, P))
+    ops.moe_align(ids, E, tile, slots, te, ps)
+    used = int((te >= 0).sum())
+    assert used <= P and ops._moe_lib.expert_rows_pay(used, P, N, K) == (K != 512)
+    outs = []
+    for tiles in (0, used, P):
+        out = torch.full((cap, N), float("nan"), dtype=dtype, device="cuda")
+        ops.expert_gemm(out, x, w, slots, te, tile, top, 0, pairs=P, tiles=tiles)
+        outs.append(out[ps.long()])
+    rows, mine = x.double().repeat_interleave(top, 0), w.double()[ids.long()]
+    y, size = (torch.matmul(m, r[:, :, None])[..., 0] for m, r in ((mine, rows), (mine.abs(), rows.abs())))
+    # a result of its type, and the sums' rounding
+    assert ((outs[0].double() - y).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * y.abs() + K * 2.0 ** -23 * size).all()
+    assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])

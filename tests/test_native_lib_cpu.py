@@ -78,27 +78,25 @@ def test_a_gate_is_asked_for_beside_the_weights_of_the_runs(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
-@pytest.mark.parametrize("experts,N,K,glu,by_pairs", [   # measured: whether the kernel for few rows per tile is the faster one
-    (16, 1024, 2048, False, {2: True, 16: True, 64: True}), (16, 2048, 1024, False, {2: True, 12: True, 64: False}),
-    (8, 2048, 4096, False, {2: True, 64: True}), (8, 4096, 2048, False, {4: True, 16: False, 128: False}), (128, 1536, 2048, True, {8: True}),
-    (128, 2048, 768, False, {8: False, 64: False, 512: False}), (256, 2048, 2048, False, {8: False, 64: False}),
-    (256, 2048, 512, False, {8: False, 64: False, 512: False}), (128, 512, 512, False, {1: True, 16: True, 64: False}), (32, 1024, 512, False, {8: True, 64: False})])
-def test_choice_of_the_expert_kernels(experts, N, K, glu, by_pairs):
+@pytest.mark.parametrize("cols,k,tiles_and_pairs", [   # measured: whether the kernel for few rows per tile is at least 10 % faster, or slower
+    (2048, 1024, {(1, 1): True, (17, 32): True, (143, 4080): True}), (512, 512, {(1, 1): True, (64, 64): True, (36, 1020): True}),
+    (2048, 704, {(4, 4): True, (66, 128): True, (572, 16320): True}), (1024, 640, {(16, 16): True, (132, 256): True}), (4096, 1024, {(64, 64): True, (1144, 32640): True}),
+    (512, 1024, {(33, 64): True, (286, 8160): True}), (2048, 768, {(16, 16): True, (125, 1): False, (125, 16): False}), (4096, 640, {(16, 16): True, (63, 4): False}),
+    (2048, 512, {(16, 16): True, (249, 16): False, (264, 512): False, (2288, 65280): False}), (1000, 520, {(39, 256): True, (159, 4096): False, (286, 8160): False}),
+    (2048, 2048, {(249, 4): False})])
+def test_choice_of_the_expert_kernels(cols, k, tiles_and_pairs):
     load_kernel_library("seq")
-    for pairs, skinny in by_pairs.items():
-        cap = -(-(pairs + experts * 31) // 32)   # every expert's last tile partly filled
-        assert torch.ops.hipserve_seq.expert_gemm_skinny(pairs, cap, N, K, experts, glu) == skinny, pairs
+    for (tiles, pairs), rows in tiles_and_pairs.items():
+        assert torch.ops.hipserve_seq.expert_rows_pay(tiles, pairs, cols, k) == rows, (tiles, pairs)
 
 
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
-@pytest.mark.parametrize("experts,N,K,glu,by_pairs", [   # measured, as above: gated products, a part of a round of the waves, many pairs per expert
-    (64, 2816, 2048, True, {4: True, 96: True, 1600: True}), (256, 512, 2048, True, {4: True, 32: True}), (32, 1024, 1024, True, {128: True, 264: True}),
-    (32, 1000, 520, False, {1200: False, 1600: False}), (64, 2048, 704, False, {1600: False}), (16, 2048, 1024, False, {400: True, 600: True})])
-def test_choice_of_the_expert_kernels_by_load(experts, N, K, glu, by_pairs):
+@pytest.mark.parametrize("cols,per_tile", [(16, 1), (17, 2), (2048, 128)])
+def test_choice_of_the_expert_kernels_at_its_edges(cols, per_tile):
     load_kernel_library("seq")
-    for pairs, skinny in by_pairs.items():
-        cap = -(-(pairs + experts * 31) // 32)
-        assert torch.ops.hipserve_seq.expert_gemm_skinny(pairs, cap, N, K, experts, glu) == skinny, pairs
+    pay, most = torch.ops.hipserve_seq.expert_rows_pay, 8192 // per_tile
+    assert pay(most, 10 * most, cols, 512) and not pay(most + 1, 10 * most, cols, 512) and not pay(most + 1, 10 * most, cols, 639) and pay(most + 1, 10 * most, cols, 640)
+    assert pay(most + 5, 5, cols, 4096) and not pay(most + 6, 5, cols, 4096)
 
 
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
