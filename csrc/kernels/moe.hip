@@ -247,6 +247,8 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(int npairs, int E, int 
 
 static int align_chunk(int npairs) { return npairs > 65536 ? 4096 : 1024; }
 int moe_align_blocks(int npairs) { return npairs > 4096 ? (npairs + align_chunk(npairs) - 1) / align_chunk(npairs) : 1; }
+// The tables of several layers go through one workgroup each, 16 pairs per thread at most. One table alone has no such bound; the same line is kept for it, and
+// beyond it the experts are gathered first.
 bool moe_align_small(int npairs) { return npairs <= 16384; }
 
 // out[slot, N] = x[row(slot), K] . W[e, N, K]^T; row(slot) = pair / k (gather) or slot.

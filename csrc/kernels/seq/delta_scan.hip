@@ -1096,7 +1096,7 @@ void gated_delta_step(const GatedDelta& p, hipStream_t s) {
     if (early) go(&gated_delta_step_kernel<T, CH, 4, true>);
   }
   if (early) {
-  } else if (!CH && p.dim == 128 && p.vdim == 128) {
+  } else if (!CH && p.dim == 128 && p.vdim == 128) {   // the head size of this package's own configurations (both sides: at the kernel)
     if constexpr (!CH) go(&gated_delta_step_kernel<T, CH, 4, false, 128>);
   } else if (p.vdim % 4 == 0) {
     go(&gated_delta_step_kernel<T, CH, 4, false>);

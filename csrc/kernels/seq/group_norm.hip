@@ -396,6 +396,8 @@ void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, i
   for (const void* p : {(const void*)out, (const void*)residual, (const void*)w, (const void*)mix, (const void*)ls1,
                         (const void*)y, (const void*)ls2, (const void*)extra, (const void*)table})
     at |= reinterpret_cast<uintptr_t>(p);
+  // 4, 8 and 16 waves, two expert rows or none: the widths and the choices per token of this package's own layer-list configurations, 1024, 2048 and 4096
+  // (both sides: at the kernel). Powers of two, so that a wave's group is a shift and 1 / columns exact; other sizes take the kernels below.
   const int waves = H / 256;
   if (at % 16 == 0 && extra == nullptr && H % 256 == 0 && (waves == 4 || waves == 8 || waves == 16) && groups > 0 &&
       waves % groups == 0 && (y == nullptr || (top == 2 && ls2 != nullptr)) && (table != nullptr ? mix == nullptr && y == nullptr : mix != nullptr) &&

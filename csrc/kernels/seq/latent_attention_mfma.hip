@@ -264,7 +264,6 @@ __global__ __launch_bounds__(64 * NW, 2) void latent_attention_mfma_kernel(
 }
 
 // o_lat[h, row_base + r, :] = sum_p acc_p e^(m_p - M) / sum_p l_p e^(m_p - M) * sigmoid(gate)
-constexpr int kMaxRuns = 64;
 
 // EARLY runs' rows are asked for behind the weights, not after them: as many runs of 64 keys as a window of 1024 has, or 4 where there are no more; those
 // beyond are asked for below, four at a time. Both waves hold the runs' weights, a lane each, and take them from there: nothing goes through LDS. All

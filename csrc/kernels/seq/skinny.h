@@ -2,8 +2,8 @@
 // (skinny_linear.hip) and the experts (expert_ffn.hip) share.
 //
 // Such a product reads every weight once and does next to nothing with it, so its time is the latency of one load
-// plus the weights over the bandwidth. A workgroup of 8 waves owns 16 columns (NT tiles of them) and splits K over its
-// waves, 64 k at a time; the waves' sums meet in LDS. 16 columns per workgroup give 128 workgroups at 2048 columns.
+// plus the weights over the bandwidth. A workgroup of 8 waves owns 16 columns (NT tiles of them, or HALF a tile) and splits K over its
+// waves, 64 k at a time; the waves' sums meet in LDS. At 2048 columns that is 128 workgroups, or 256 of half tiles.
 //
 // What a compute unit takes in (its weights, and the rows again for every workgroup) bounds the larger M, and how a load
 // spreads its addresses decides how much that is. The matrix cores want 16 rows side by side over the lanes; a load that
@@ -12,12 +12,13 @@
 // (whole 128-byte lines, four lanes per look-up) and the operands are read from there, without registers for loads in
 // flight: 60 - 80 KB per us. Each wave copies into a part of LDS that is its own, DEPTH pieces of 64 k ahead, and waits for
 // its own copies alone. us, cold weights, loads in operand order -> this (the vendor's GEMM), 1 / 16 / 48 rows:
-//   1024 x 1024   3.4 -> 2.8 (5.6)    4.2 -> 3.1 (5.7)    6.5 -> 3.9 (8.1)     (columns x k)
-//   2048 x 2048   5.0 -> 4.4 (11.0)   6.4 -> 5.1 (11.1)   10.5 -> 7.1 (11.4)
-//   2048 x 6144   9.3 -> 7.8 (11.1)   13.6 -> 10.5 (11.2) 24.7 -> 16.2 (16.5)
-//   32000 x 2048  25.2 -> 25.6 (32.3) 33.7 -> 27.8 (30.9) 60 -> 33.5, four tiles per workgroup (34)
-// Deeper copies (3 or 5 pieces) changed nothing at one workgroup per CU and cost up to a fifth where they leave room for fewer; so do two
-// pieces but for up to 16 rows and more than a piece per wave (skinny_linear.hip).
+//   1024 x 1024   3.4 -> 2.6 (5.7)    4.2 -> 2.8 (5.8)    6.5 -> 3.8 (8.0)     (columns x k)
+//   2048 x 2048   5.0 -> 4.0 (11.0)   6.4 -> 4.3 (11.0)   10.5 -> 7.0 (11.1)   (half tiles but for 48 rows)
+//   2048 x 6144   9.3 -> 6.7 (11.2)   13.6 -> 8.4 (11.4)  24.7 -> 14.0 (16.8)  (half tiles)
+//   32000 x 2048  25.2 -> 25.0 (32.3) 33.7 -> 27.5 (32.7) 60 -> 33.3, two tiles per workgroup (37.4)
+// Deeper copies of whole tiles (3 or 5 pieces) changed nothing at one workgroup per CU and cost up to a fifth where they leave room for fewer; so do two
+// pieces but for up to 16 rows and more than a piece per wave. Half tiles, one workgroup per CU, run two for any rows, three for up to 8 rows of more
+// than 4096 k (skinny_linear.hip).
 // 32-bit operands (F32) are the same rows of twice as many 16-bit halves: a step is 64 bytes of a row, 16 numbers, and four
 // products of 4 k each; the four numbers of a lane are k 4 g + e on both sides, so nothing else differs.
 #pragma once
@@ -26,7 +27,7 @@
 
 namespace hipserve {
 
-constexpr int kSkWaves = 8 /* 1 << 3 */, kSkThreads = 64 * kSkWaves, kSkLd = 20;   // kSkLd: row stride of the sums in LDS (floats)
+constexpr int kSkWaves = 8, kSkThreads = 64 * kSkWaves, kSkLd = 20;   // kSkLd: row stride of the sums in LDS (floats)
 
 template <int N> HS_DEVICE void wait_copies() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
@@ -55,7 +56,7 @@ template <int XG, int NT, int DEPTH, bool F32 = false, bool HALF = false> struct
     const int c = lane & 15, g = lane >> 4, r8 = lane >> 3;
     unsigned char* ring = smem + wave * DEPTH * kPiece;
     const unsigned lds0 = lds_at(ring);
-    const int pieces = (K + 63) >> 6, n = (pieces - wave + kSkWaves - 1) >> 3;   // this wave's: wave, wave + 8, ...
+    const int pieces = (K + 63) >> 6, n = (pieces - wave + kSkWaves - 1) >> 3;   // (kSkWaves is 1 << 3) this wave's: wave, wave + 8, ...
     // the lane's bytes past the piece's first k of the first row: full pieces differ by uniform numbers
     unsigned w_at[WG], x_at[XG];
 #pragma unroll

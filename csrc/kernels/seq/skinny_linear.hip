@@ -6,7 +6,7 @@
 //
 // Norms between such products cost a launch of their own, 2.5 - 4 us of a decode step each, nearly all of it latency. A product whose
 // result goes into the residual stream therefore can take the update with it (SkinnyNorm with a residual): it adds its result to the
-// 32-bit stream, writes the rows times the next norm's weights, and leaves the sums of squares of its 16 columns; the products that
+// 32-bit stream, writes the rows times the next norm's weights, and leaves the sums of squares of its 16 or 8 columns; the products that
 // read these rows (SkinnyNorm without one) sum the squares and scale their results, of which a norm's factor per row is part
 // as well. The rows are rounded once either way, and the update sees the unrounded product. Six norms less in a decode step of Fikizen: one
 // row, width 1024, 2450 -> 2328 us (17 steps), 16 rows, width 2048, 9271 -> 8957 (33 steps); both products take about 0.3 us longer.
@@ -234,7 +234,6 @@ bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, 
 // many k each): then two or four share what they copy of the rows; up to 16 rows there is too little of that. Cold weights, us with 1 / 2 / 4
 // tiles: 6144 x 4096, 16 rows 14.5 / 15.1 / 21, 48 rows 20.9 / 18.7 / 26; 16384 x 2048, 16 rows 17.0 / 15.5 / 15.5, 24 rows 18.3 / 16.4 /
 // 16.2, 48 rows 22.6 / 19.4 / 18.8; 32000 x 512, 24 rows 10.4 / 10.0 / 11.9; 16384 x 4096, 64 rows 41.6 / 35.9 / 29.3.
-// Of 2541 sizes (1 - 64 rows, 64 - 65536 columns, k 128 - 12288, both types) the choice is 0.6 % slower than the best on average, at most 21 %.
 int skinny_tiles(int M, long tiles, int K) {
   if (tiles <= 256) return 1;
   if (M <= 16) return M > 8 && tiles <= 512 && K >= 8192 ? 2 : 1;
