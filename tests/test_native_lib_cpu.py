@@ -66,6 +66,19 @@ def test_a_carried_state_is_asked_for_at_once(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+def test_short_prompts_of_mingru_leave_room_for_twice_the_waves(tmp_path):
+    """Sequences of one block of rows: no registers for a next block's, and no loads of it."""
+    asm = tmp_path / "k.s"
+    subprocess.run([_build.HIPCC, *_build.HIP_FLAGS, "-I", os.path.join(_build.CSRC, "include"), "-S", "--cuda-device-only",
+                    os.path.join(_build.CSRC, "kernels", "seq", "mingru.hip"), "-o", asm], check=True, capture_output=True)
+    text = asm.read_text()
+    for t, load in (("f", "buffer_load_dword "), ("t", "buffer_load_ushort ")):
+        code = re.split(rf"^_ZN\S*mingru_scan_kernelI{t}Lb0E\S*:", text, maxsplit=1, flags=re.M)[1].split("s_endpgm")[0]
+        regs = re.search(rf"\.name:\s+_ZN\S*mingru_scan_kernelI{t}Lb0E.*?\.vgpr_count:\s+(\d+)", text, flags=re.S)
+        assert int(regs[1]) <= 64 and code.count(load) == 3 * 16
+
+
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
 def test_a_gate_is_asked_for_beside_the_weights_of_the_runs(tmp_path):
     """The merge of latent decode runs waits for the weights and the gate while the runs' rows are on their way."""
     asm = tmp_path / "k.s"
