@@ -175,7 +175,8 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
 // 2: every workgroup sums the table (nb x E ints) into the padded expert offsets and its own prefix, then scatters its pairs; the padding slots
 // (disjoint from every real slot, so no ordering between workgroups is needed) and tile tables of the experts go round the workgroups.
 // us, one workgroup -> many, in brackets with the lookup of table[token]: 8000 pairs, 16 experts 7.2 -> 5.0 (13.4 -> 5.4), 16384 pairs 11.9 -> 5.2
-// (24.4 -> 5.6), of 128 experts 13.8 -> 6.4 (25.4 -> 6.8); 4096 pairs 4.0 (5.5) on one.
+// (24.4 -> 5.6), of 128 experts 13.8 -> 6.1 (25.4 -> 6.5), 4097 pairs of 128 experts 5.9 -> 5.6 (with an expert's rest per workgroup, not per wave, 8.9); 4096
+// pairs 4.0 (5.5) on one.
 template <int PER>
 __global__ __launch_bounds__(1024) void moe_count_kernel(const int* __restrict__ ids, const int* __restrict__ table, const long* __restrict__ tokens,
                                                          int top, int top_shift, long table_rows, int npairs, int* __restrict__ pair_slot,
@@ -237,9 +238,9 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(int npairs, int E, int 
     }
   }
   const int total = off[128];
-  for (int x = b; x < E; x += nb) {   // the rest of the experts' last tiles, their tiles' labels
-    for (int s = off[x] + cnt[x] + tid; s < off[x + 1]; s += 1024) slots[s] = -1;
-    for (int t = (off[x] >> tile_shift) + tid; t < off[x + 1] >> tile_shift; t += 1024) tile_expert[t] = x;
+  for (int x = b * 16 + (tid >> 6); x < E; x += nb * 16) {   // the rest of the experts' last tiles, their tiles' labels: an expert per wave
+    for (int s = off[x] + cnt[x] + (tid & 63); s < off[x + 1]; s += 64) slots[s] = -1;
+    for (int t = (off[x] >> tile_shift) + (tid & 63); t < off[x + 1] >> tile_shift; t += 64) tile_expert[t] = x;
   }
   for (int s = total + b * 1024 + tid; s < slots_cap; s += nb * 1024) slots[s] = -1;
   for (int t = (total >> tile_shift) + b * 1024 + tid; t < tiles_cap; t += nb * 1024) tile_expert[t] = -1;
