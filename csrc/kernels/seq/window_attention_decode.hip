@@ -328,15 +328,22 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
     u = min(u, last);
     return u < nk ? u : u - nk + lo_all;
   };
+  // Global addresses by their type: of pointers that come from either of two places below the compiler forgets it, and flat loads wait for
+  // each other and for LDS (bf16, 64 rows of 32 heads over 8, 1000 keys 54 -> 58 us, before / with those).
+  using Row1 = const __attribute__((address_space(1))) T*;
+  const Row1 keys = reinterpret_cast<Row1>(reinterpret_cast<unsigned long>(cache));
   auto row_of = [&](int block, int key) {
-    return cache + (unsigned long)(unsigned)((block << block_shift) + (key & in_block)) * (unsigned)(2 * kv_heads * D);
+    return keys + (unsigned long)(unsigned)((block << block_shift) + (key & in_block)) * (unsigned)(2 * kv_heads * D);
   };
   using Keys = u32x4[SUB][QN];
   // as they lie in memory: 16-bit elements of their own are taken apart, and waited for, where they are loaded
   using Part = __attribute__((ext_vector_type(E * sizeof(T) / 4))) unsigned;
   using Values = Part[4 * SUB][NB];
   // A decode row's 16 keys side by side lie in at most two blocks, which are the same in every lane, unless blocks are smaller or keys are kept:
-  // ten rows per lane, each with a load and a 64-bit address of its own, were a quarter of a short step's time.
+  // ten rows per lane, each with a load and a 64-bit address of its own, were a quarter of a short step's time. us with those two / each lane's own: steps with
+  // their preparation in bf16, 1000 keys, 41 rows of 40 heads of 128 over 2 22.7 / 24.7, 64 of 32 of 64 over 4 19.5 / 21.2; decode rows beside prompts in 32
+  // bits, 64 of 32 of 128 over 8, 500 keys 53 / 65, of 64 over 4, 1000 keys 29.8 / 34.1; but in bf16, where nothing else is between them, 64 of 32 of 128
+  // over 8, 1000 keys 58 / 54, 16 of 256 over 4, 500 keys 31.5 / 29.6.
   const bool near = !MULTI && nk == 0 && block_shift >= 4;
   typedef int i32x2 __attribute__((ext_vector_type(2)));
   using Blocks = i32x2[SUB];
@@ -344,26 +351,30 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
 #pragma unroll
     for (int a = 0; a < SUB; ++a) block[a] = i32x2{bt[key_of(u0 + 16 * a) >> block_shift], bt[key_of(u0 + 16 * a + 15) >> block_shift]};
   };
-  using Rows = const T*[5 * SUB];
-  auto rows_of = [&](int u0, const Blocks& block, Rows& src) {
-    auto all = [&](auto&& row) {
-#pragma unroll
-      for (int a = 0; a < SUB; ++a) src[a] = row(a, key_of(u0 + 16 * a + c)) + kvh * D;
-#pragma unroll
-      for (int i = 0; i < 4 * SUB; ++i) src[SUB + i] = row(i >> 2, key_of(u0 + 16 * (i >> 2) + 4 * g + (i & 3))) + (kv_heads + kvh) * D + E * c;
+  using Rows = Row1[5 * SUB];
+  auto rows_of = [&](int u0, Rows& src, auto&& block) {   // block(a, key): of a key of the 16 from u0 + 16 a on
+    auto row = [&](int a, int u) {
+      const int key = key_of(u);
+      return row_of(block(a, key), key);
     };
-    if (near) all([&](int a, int key) { return row_of(key >> block_shift == key_of(u0 + 16 * a) >> block_shift ? block[a][0] : block[a][1], key); });
-    else all([&](int, int key) { return row_of(bt[key >> block_shift], key); });
+#pragma unroll
+    for (int a = 0; a < SUB; ++a) src[a] = row(a, u0 + 16 * a + c) + kvh * D;
+#pragma unroll
+    for (int i = 0; i < 4 * SUB; ++i) src[SUB + i] = row(i >> 2, u0 + 16 * (i >> 2) + 4 * g + (i & 3)) + (kv_heads + kvh) * D + E * c;
+  };
+  auto looked_up = [&](int, int key) { return bt[key >> block_shift]; };
+  auto rows_of_blocks = [&](int u0, Rows& src, const Blocks& block) {
+    rows_of(u0, src, [&](int a, int key) { return key >> block_shift == key_of(u0 + 16 * a) >> block_shift ? block[a][0] : block[a][1]; });
   };
   auto load = [&](const Rows& src, Keys& k, Values& v) {
 #pragma unroll
     for (int a = 0; a < SUB; ++a)
 #pragma unroll
-      for (int i = 0; i < QN; ++i) k[a][i] = reinterpret_cast<const u32x4*>(src[a])[4 * i + g];
+      for (int i = 0; i < QN; ++i) k[a][i] = reinterpret_cast<const __attribute__((address_space(1))) u32x4*>(src[a])[4 * i + g];
 #pragma unroll
     for (int i = 0; i < 4 * SUB; ++i)
 #pragma unroll
-      for (int b = 0; b < NB; ++b) v[i][b] = *reinterpret_cast<const Part*>(src[SUB + i] + 16 * E * b);
+      for (int b = 0; b < NB; ++b) v[i][b] = *reinterpret_cast<const __attribute__((address_space(1))) Part*>(src[SUB + i] + 16 * E * b);
   };
   const int first = lo + wave * KT;
   constexpr bool EARLY = PREP && D * sizeof(T) <= 256;      // the first tile fits the registers beside the preparation
@@ -383,7 +394,11 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
     }, [&] {
       if constexpr (EARLY) {
         Rows src;
-        rows_of(first, block0, src);
+        if (near) rows_of_blocks(first, src, block0);
+        else {
+          rows_of(first, src, looked_up);
+          __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the paths meet with none of these look-ups open, for which the other would wait
+        }
         load(src, k0, v0);
       }
     });
@@ -409,10 +424,14 @@ __global__ __launch_bounds__(512) void window_decode_kernel(
     Keys& k = EARLY ? k0 : kl;
     Values& v = EARLY ? v0 : vl;
     if (!EARLY || u0 != first) {
-      Blocks block;
       Rows src;
-      blocks_of(u0, block);
-      rows_of(u0, block, src);
+      if ((F32 || PREP) && near) {
+        Blocks block;
+        blocks_of(u0, block);
+        rows_of_blocks(u0, src, block);
+      } else {
+        rows_of(u0, src, looked_up);
+      }
       load(src, k, v);
     }
     if (PREP && fresh && hi - u0 < KT) {   // the cache row is being written: its key and value are in LDS

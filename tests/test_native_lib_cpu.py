@@ -66,6 +66,16 @@ def test_a_carried_state_is_asked_for_at_once(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+def test_decode_window_attention_knows_its_keys_are_global(tmp_path):
+    """No flat loads, which wait for each other and for LDS."""
+    asm = tmp_path / "k.s"
+    subprocess.run([_build.HIPCC, *_build.HIP_FLAGS, "-I", os.path.join(_build.CSRC, "include"), "-S", "--cuda-device-only",
+                    os.path.join(_build.CSRC, "kernels", "seq", "window_attention_decode.hip"), "-o", asm], check=True, capture_output=True)
+    text = asm.read_text()
+    assert "global_load_dwordx4" in text and "flat_load" not in text
+
+
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
 def test_short_prompts_of_mingru_leave_room_for_twice_the_waves(tmp_path):
     """Sequences of one block of rows: no registers for a next block's, and no loads of it."""
     asm = tmp_path / "k.s"
