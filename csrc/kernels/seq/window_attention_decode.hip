@@ -169,8 +169,11 @@ HS_DEVICE void prepare_row(const WindowPrep& pr, int waves, const T* __restrict_
 #pragma unroll
       for (int e = 0; e < 4; ++e) { const float p = x[e] * grow, q = y[e] * grow; v[e] = p * p + q * q; }
       ss = (v[0] + v[1]) + (v[2] + v[3]);
-#pragma unroll
-      for (int o = 1; o < PER; o <<= 1) ss += __shfl_xor(ss, o, 64);
+      static_assert(PER == 8 || PER == 16, "a head's lanes are a lane row or half of one");
+      ss = dpp_step<0xB1, 0xf, false>(ss);                              // quad_perm [1, 0, 3, 2]
+      ss = dpp_step<0x4E, 0xf, false>(ss);                              // quad_perm [2, 3, 0, 1]
+      ss = dpp_step<0x141, 0xf, false>(ss);                             // row_half_mirror
+      if constexpr (PER == 16) ss = dpp_step<0x140, 0xf, false>(ss);    // row_mirror
     }
   };
   if ((tid & ~63) < items) take(min(tid, items - 1));   // whole waves: a head's sum is over its lanes
