@@ -218,21 +218,27 @@ HS_DEVICE __amdgpu_buffer_rsrc_t rows_at(const float* p, int bytes) {   // `byte
   return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(hi << 32 | lo), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
 }
 
+constexpr unsigned kNone = 0x80000000u;   // outside every buffer: reads as zero, is not stored
+
 HS_DEVICE float ld_at(__amdgpu_buffer_rsrc_t from, unsigned at) { return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from, at, 0, 0)); }
 
 // grid (heads, ceil(vdim / kCols), sequences), four waves: the step's first sequences (its prompt portions, the
 // long ones) are dispatched first and spread over the CUs before the one-token sequences fill in. A state column (one value channel) is held by the 16
 // lanes of a DPP row, DS key channels each (dim <= 16 DS; the padding rows stay zero): a product with the
 // state is DS multiply-adds per lane and four DPP steps, so the chain from one token to the next is short. The instructions that a wave issues
-// in turn bound it, so a full batch of tokens tests nothing, a token's vectors are read while the one before is computed, and what does not exist
-// is outside the buffers instead of behind branches. The whole rule in 32 bits, 3 prompts of 300 rows, 8 heads of 128: 124 -> 90 us, one of 700 237 ->
-// 175 (the generalized one, 16 heads of 64: 102 -> 70, 209 -> 132).
+// in turn bound it, so a full batch of tokens tests nothing and what does not exist is outside the buffers instead of behind branches. The whole rule in
+// 32 bits, 3 prompts of 300 rows, 8 heads of 128: 124 -> 90 us, one of 700 237 -> 175 (the generalized one, 16 heads of 64: 102 -> 70, 209 -> 132).
+// AHEAD: a token's vectors are read while the one before is computed. Its second set of them is 2 - 5 DS registers, so wider rows go without it (and,
+// past 8 channels a lane, without the second copy of the tokens): the generalized rule with it 209 and 388 registers at 8 and 16 channels, without 122
+// and 168, two and three waves per SIMD more. 200 sequences of 10 rows with / without, us: 16 heads of 128 406 / 334, 8 of 200 995 / 593; this rule with a
+// decay per channel, 8 of 200, 793 / 489, 8 of 256 with one 617 / 515. One prompt of 300 of 8 heads of 128 gives 86 / 93 back.
 // CH: a decay per key channel, staged beside q and k.
 template <int DS, bool CH>
 __global__ __launch_bounds__(kScanThreads) void gated_delta_scan_kernel(
     float* __restrict__ o, float* __restrict__ S, const float* __restrict__ qk, const float* __restrict__ vv,
     const float* __restrict__ gg, const float* __restrict__ bb, const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx,
     const int* __restrict__ seq_state, int heads, int kv_heads, int dim, int vdim) {
+  constexpr bool AHEAD = DS <= 4;
   constexpr int DP = kSeg * DS;
   __shared__ __attribute__((aligned(16))) float sq[kTB][DP], sk[kTB][DP], sg[CH ? kTB : 1][CH ? DP : 1];
   __shared__ float sb[kTB][2];   // beta, and the head's decay without CH
@@ -244,14 +250,13 @@ __global__ __launch_bounds__(kScanThreads) void gated_delta_scan_kernel(
   const int kh = h / (heads / kv_heads), nqk = kv_heads * dim, nv = heads * vdim;
   float* Sp = S + (((long)seq_state[s] * heads + h) * dim) * vdim;
   const bool carried = seq_ctx[s] - n > 0;
+  const auto kept = rows_at(Sp, carried ? dim * vdim * 4 : 0);
   float st[DS];
 #pragma unroll
-  for (int i = 0; i < DS; ++i) st[i] = (carried && v0 < vdim && k0 + i < dim) ? Sp[(long)(k0 + i) * vdim + v0] : 0.f;
+  for (int i = 0; i < DS; ++i) st[i] = ld_at(kept, v0 < vdim ? ((k0 + i) * vdim + v0) * 4u : kNone);
   // the next batch of tokens is loaded into registers while this batch is computed
   constexpr int kLd = (kTB * DP + kScanThreads - 1) / kScanThreads;
   float rq[kLd], rk[kLd], rg[CH ? kLd : 1], rv[kTB], rb = 0.f;
-  // rows, channels and columns that do not exist are outside the buffers and read as zeros
-  constexpr unsigned kNone = 0x80000000u;
   const unsigned v_at = v0 < vdim ? (h * vdim + v0) * 4u : kNone, b_at = tid < 2 * kTB ? ((tid >> 1) * heads + h) * 4u : kNone;
   auto fetch = [&](int t0) {
     const int nt = min(kTB, n - t0);
@@ -297,10 +302,9 @@ __global__ __launch_bounds__(kScanThreads) void gated_delta_scan_kernel(
     __syncthreads();
     if (t0 + kTB < n) fetch(t0 + kTB);
     const auto to = rows_at(o + (long)(r0 + t0) * nv, nt * nv * 4);
-    // a token's vectors are read while the one before it is computed
     struct Token {
       float beta, g, kk[DS], qq[DS], gd[CH ? DS : 1];
-    } x[2];
+    } x[AHEAD ? 2 : 1];
     auto read = [&](Token& x, int tt) {
       x.beta = sb[tt][0];
       x.g = sb[tt][1];
@@ -312,9 +316,10 @@ __global__ __launch_bounds__(kScanThreads) void gated_delta_scan_kernel(
       }
     };
     auto token = [&](int tt) {
-      if (tt + 1 < kTB) read(x[(tt + 1) & 1], tt + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      const auto& [beta, g, kk, qq, gd] = x[tt & 1];
+      if (!AHEAD) read(x[0], tt);
+      else if (tt + 1 < kTB) read(x[(tt + 1) & 1], tt + 1);
+      if (AHEAD) __builtin_amdgcn_sched_barrier(0);   // those loads stay here
+      const auto& [beta, g, kk, qq, gd] = x[AHEAD ? tt & 1 : 0];
       float pred = 0.f, pred2 = 0.f;
 #pragma unroll
       for (int i = 0; i < DS; ++i) {
@@ -332,8 +337,8 @@ __global__ __launch_bounds__(kScanThreads) void gated_delta_scan_kernel(
       }
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, row_sum(out + out2)), to, out_at + tt * nv * 4, 0, 0);
     };
-    read(x[0], 0);
-    if (nt == kTB) {   // no tests between the tokens
+    if (AHEAD) read(x[0], 0);
+    if (DS <= 8 && nt == kTB) {   // no tests between the tokens
 #pragma unroll
       for (int tt = 0; tt < kTB; ++tt) token(tt);
     } else {
@@ -374,11 +379,14 @@ __global__ __launch_bounds__(256) void delta_rule_prepare_kernel(
   }
 }
 
+// As gated_delta_scan_kernel. Rows past a partial batch are not asked for where a row is wide: they hold up a step of one token each (200 sequences of 8
+// heads of 200: 302 us with them, 252 without), and are never read back from LDS.
 template <typename T, int DS>
 __global__ __launch_bounds__(kScanThreads) void delta_rule_scan_kernel(
     float* __restrict__ o, float* __restrict__ S, const float* __restrict__ pre, const T* __restrict__ proj, long ld,
     const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, int heads,
     int dim) {
+  constexpr bool AHEAD = DS <= 4;
   constexpr int DP = kSeg * DS, TB = kTB;
   __shared__ __attribute__((aligned(16))) float sv[TB][5][DP];  // w, a u, u, k, r (zero past dim), all from `pre`
   const int s = blockIdx.z, h = blockIdx.x, zb = blockIdx.y, tid = threadIdx.x;
@@ -389,31 +397,36 @@ __global__ __launch_bounds__(kScanThreads) void delta_rule_scan_kernel(
   const int N = heads * dim;
   float* Sp = S + (((long)seq_state[s] * heads + h) * dim) * dim;
   const bool carried = seq_ctx[s] - n > 0;
+  const auto kept = rows_at(Sp, carried ? dim * dim * 4 : 0);
   float st[DS];
 #pragma unroll
-  for (int i = 0; i < DS; ++i) st[i] = (carried && v0 < dim && k0 + i < dim) ? Sp[(long)(k0 + i) * dim + v0] : 0.f;
+  for (int i = 0; i < DS; ++i) st[i] = ld_at(kept, v0 < dim ? ((k0 + i) * dim + v0) * 4u : kNone);
   // the next batch of tokens is loaded into registers while this batch is computed
   constexpr int kLd = (TB * DP + kScanThreads - 1) / kScanThreads;
-  float rg[5][kLd], rv[TB];
-  constexpr unsigned kNone = 0x80000000u;   // outside the buffers
+  float rg[5][kLd] = {}, rv[TB] = {};
   const unsigned v_at = v0 < dim ? (h * dim + v0) * 4u : kNone;
+  const unsigned k_at = tid % DP < dim ? (tid / DP * 6 * N + h * dim + tid % DP) * 4u : kNone;
   auto fetch = [&](int t0) {
     const int nt = min(TB, n - t0);
     const float* p = pre + (long)(r0 + t0) * 6 * N;
+    unsigned at = k_at, v = v_at;
+    if (DS > 8) asm volatile("" : "+v"(at), "+v"(v));   // the rows' offsets are added up here, not kept over the batches
+    auto rows = [&](auto full) {
 #pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      const auto from = rows_at(p + j * N, (nt * 6 - j) * N * 4);
+      for (int j = 0; j < 5; ++j) {
+        const auto from = rows_at(p + j * N, (nt * 6 - j) * N * 4);
 #pragma unroll
-      for (int it = 0; it < kLd; ++it) {
-        const int i = it * kScanThreads + tid, k = i % DP;
-        rg[j][it] = ld_at(from, k < dim ? (i / DP * 6 * N + h * dim + k) * 4u : kNone);
+        for (int it = 0; it < kLd; ++it)
+          if (full || it * kScanThreads < nt * DP) rg[j][it] = ld_at(from, at + it * (kScanThreads / DP) * 6 * N * 4);
       }
-    }
-    const auto fv = rows_at(p + 5 * N, (nt * 6 - 5) * N * 4);
+      const auto fv = rows_at(p + 5 * N, (nt * 6 - 5) * N * 4);
 #pragma unroll
-    for (int tt = 0; tt < TB; ++tt) rv[tt] = ld_at(fv, v_at + tt * 6 * N * 4);
+      for (int tt = 0; tt < TB; ++tt)
+        if (full || tt < nt) rv[tt] = ld_at(fv, v + tt * 6 * N * 4);
+    };
+    if (AHEAD || nt == TB) rows(std::true_type{});
+    else rows(std::false_type{});
   };
-  const unsigned out_at = seg == 0 ? v_at : kNone;
   fetch(0);
   for (int t0 = 0; t0 < n; t0 += TB) {
     const int nt = min(TB, n - t0);
@@ -432,9 +445,11 @@ __global__ __launch_bounds__(kScanThreads) void delta_rule_scan_kernel(
     __syncthreads();
     if (t0 + TB < n) fetch(t0 + TB);
     const auto to = rows_at(o + (long)(r0 + t0) * N, nt * N * 4);
+    unsigned out_at = seg == 0 ? v_at : kNone;
+    if (DS > 8) asm volatile("" : "+v"(out_at));
     struct Token {
       float w[DS], au[DS], uu[DS], kk[DS], rr[DS];
-    } x[2];
+    } x[AHEAD ? 2 : 1];
     auto read = [&](Token& x, int tt) {
 #pragma unroll
       for (int i = 0; i < DS; ++i) {
@@ -443,9 +458,10 @@ __global__ __launch_bounds__(kScanThreads) void delta_rule_scan_kernel(
       }
     };
     auto token = [&](int tt) {
-      if (tt + 1 < TB) read(x[(tt + 1) & 1], tt + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      const auto& [w, au, uu, kk, rr] = x[tt & 1];
+      if (!AHEAD) read(x[0], tt);
+      else if (tt + 1 < TB) read(x[(tt + 1) & 1], tt + 1);
+      if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+      const auto& [w, au, uu, kk, rr] = x[AHEAD ? tt & 1 : 0];
       float us = 0.f, us2 = 0.f;
 #pragma unroll
       for (int i = 0; i < DS; ++i) {
@@ -462,8 +478,8 @@ __global__ __launch_bounds__(kScanThreads) void delta_rule_scan_kernel(
       }
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, row_sum(out + out2)), to, out_at + tt * N * 4, 0, 0);
     };
-    read(x[0], 0);
-    if (nt == TB) {
+    if (AHEAD) read(x[0], 0);
+    if (DS <= 8 && nt == TB) {
 #pragma unroll
       for (int tt = 0; tt < TB; ++tt) token(tt);
     } else {

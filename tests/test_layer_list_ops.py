@@ -1210,6 +1210,47 @@ def test_gated_delta_chunks_precision(lens, dim, vdim, a, carried):
     assert errs[1][0] <= 1.4 * errs[0][0] and errs[1][1] <= 1.5 * errs[0][1], errs
 
 
+@gpu
+@pytest.mark.parametrize("dim,vdim", [(70, 70), (128, 40), (129, 129), (200, 72), (256, 256)])
+def test_scans_of_wide_heads(dim, vdim):
+    """8 and 16 channels per lane, token by token: whole and partly filled batches of tokens, carried and fresh states, beside the reference; a slot that
+    no sequence has stays as it was."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(dim)
+    lens, H, G = [3, 1, 8, 17, 10], 4, 2
+    T, n, N, nq = sum(lens), len(lens), H * vdim, G * dim
+    cols = 2 * nq + N
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist()).int()
+    ctx, slots = torch.tensor([m + (7 if i % 2 else 0) for i, m in enumerate(lens)]).int(), torch.randperm(n + 1, generator=g)[:n].int()
+    S, ops = torch.randn(n + 1, H, dim, vdim, generator=g), get_ops("cuda")
+    meta = SimpleNamespace(seq_cu=cu.cuda(), seq_ctx=ctx.cuda(), seq_state=slots.cuda(), max_q=max(lens))
+
+    def same(got, want):   # sums of up to 256 products of either order, 2^-24 each
+        for a, b in zip(got, want):
+            assert ((a.cpu() - b).abs() <= 2.0 ** -15 * b.abs().max()).all()
+    proj = torch.randn(T, cols + 2 * H + N, generator=g)
+    conv, dt, nw = torch.randn(cols, 4, generator=g), torch.randn(H, dim, generator=g), torch.rand(vdim, generator=g) + 0.5
+    a_log, per, gate = torch.randn(H, generator=g) * 0.5, torch.randn(T, H * dim, generator=g), torch.randn(T, N, generator=g)
+    for wide in (False, True):   # a decay per head, from the row; per key channel, given as the gate is
+        sp = SimpleNamespace(heads=H, kv_heads=G, dim=dim, vdim=vdim, out_size=N, conv=4, conv_channels=cols, gate_act="silu", channel_decay=wide)
+        bias, offs, kept = (dt if wide else dt[:, 0]).flatten(), (cols + H, cols + 2 * H, cols), torch.randn(n + 1, 3, cols, generator=g)
+        own = (per, gate) if wide else (None, None)
+        y, want, wc = torch.empty(T, N), S.clone(), kept.clone()
+        ref.gated_delta(y, want, wc, proj, conv, a_log, bias, nw, *own, offs, sp, 1e-6, cu, ctx, slots)
+        out, state = torch.empty(T, N, device="cuda"), [S.cuda(), kept.cuda()]
+        ops.gated_delta(out, state, proj.cuda(), conv.cuda(), a_log.cuda(), bias.cuda(), nw.cuda(), *(x if x is None else x.cuda() for x in own), offs, sp,
+                        1e-6, meta)
+        same((out, *state), (y, want, wc))
+    if dim != vdim: return
+    proj, wl = torch.randn(T, 5 * N + 64, generator=g), torch.randn(T, N, generator=g) * 2
+    a_b, w0, nw = torch.randn(N, generator=g), torch.randn(N, generator=g), torch.rand(N, generator=g) + 0.5
+    sp = SimpleNamespace(heads=H, dim=dim, size=N)
+    y, want, out, state = torch.empty(T, N), S.clone(), torch.empty(T, N, device="cuda"), S.cuda()
+    ref.delta_rule(y, want, proj, wl, a_b, w0, nw, sp, 1e-5, cu, ctx, slots, 1.0)
+    ops.delta_rule(out, [state], proj.cuda(), wl.cuda(), a_b.cuda(), w0.cuda(), nw.cuda(), sp, 1e-5, meta)
+    same((out, state), (y, want))
+
+
 # ------------------------------------------------------------------ window attention of prompts
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

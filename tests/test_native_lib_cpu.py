@@ -89,6 +89,19 @@ def test_short_prompts_of_mingru_leave_room_for_twice_the_waves(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+def test_scans_of_wide_heads_leave_room_for_three_waves(tmp_path):
+    """Token by token: no second set of a token's vectors at 8 and 16 channels per lane."""
+    asm = tmp_path / "k.s"
+    subprocess.run([_build.HIPCC, *_build.HIP_FLAGS, "-I", os.path.join(_build.CSRC, "include"), "-S", "--cuda-device-only",
+                    os.path.join(_build.CSRC, "kernels", "seq", "delta_scan.hip"), "-o", asm], check=True, capture_output=True)
+    regs = {}
+    for entry in asm.read_text().split(".name: ")[1:]:
+        scan = re.match(r"\s+_ZN\S*?\d(gated_delta|delta_rule)_scan_kernelI([ft]?)Li(\d+)(\S*?)EEE?v", entry)
+        if scan: regs[scan.groups()] = int(re.search(r"\.vgpr_count:\s+(\d+)", entry)[1])
+    assert len(regs) == 20 and all(n <= (168 if int(ds) == 16 else 128) for (_, _, ds, _), n in regs.items()), regs
+
+
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
 def test_a_gate_is_asked_for_beside_the_weights_of_the_runs(tmp_path):
     """The merge of latent decode runs waits for the weights and the gate while the runs' rows are on their way."""
     asm = tmp_path / "k.s"
