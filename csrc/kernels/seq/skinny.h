@@ -18,7 +18,7 @@
 //   32000 x 2048  25.2 -> 25.0 (32.3) 33.7 -> 27.5 (32.7) 60 -> 33.3, two tiles per workgroup (37.4)
 // Deeper copies of whole tiles (3 or 5 pieces) changed nothing at one workgroup per CU and cost up to a fifth where they leave room for fewer; so do two
 // pieces but for up to 16 rows and more than a piece per wave. Half tiles, one workgroup per CU, run two for any rows, three for up to 8 rows of more
-// than 4096 k (skinny_linear.hip).
+// than 4096 k, in 32 bits what whole tiles do (skinny_linear.hip).
 // 32-bit operands (F32) are the same rows of twice as many 16-bit halves: a step is 64 bytes of a row, 16 numbers, and four
 // products of 4 k each; the four numbers of a lane are k 4 g + e on both sides, so nothing else differs.
 #pragma once

@@ -220,12 +220,13 @@ bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, long out_zs, 
   return true;
 }
 
-template <int XG, int NT, int DEPTH, bool GLU, bool HALF = false>
+// DEPTH32: of 32-bit operands.
+template <int XG, int NT, int DEPTH, bool GLU, bool HALF = false, int DEPTH32 = DEPTH>
 bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, int parts, const void* x, long x_ld, long x_bs,
                 const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
   const int cols = GLU ? N / 2 : N, per = GLU ? 16 : HALF ? 8 : 16 * NT;
   const dim3 grid((cols + per - 1) / per, batch, parts);
-#define HS_SK(TO, F32) launch_kernel<XG, NT, DEPTH, GLU, TO, F32, kPlain, HALF>(grid, out, out_ld, out_bs, out_zs, x, x_ld, x_bs, w, bias, M, N, K, act, act_from, c0, c1, s)
+#define HS_SK(TO, F32) launch_kernel<XG, NT, F32 ? DEPTH32 : DEPTH, GLU, TO, F32, kPlain, HALF>(grid, out, out_ld, out_bs, out_zs, x, x_ld, x_bs, w, bias, M, N, K, act, act_from, c0, c1, s)
   return f32 ? HS_SK(float, true) : out_f32 ? HS_SK(float, false) : HS_SK(unsigned short, false);
 #undef HS_SK
 }
@@ -287,9 +288,13 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
          : xg <= 6 ? HS_SK(6, 2, 1, true) : HS_SK(8, 2, 1, true);
   const long tiles = ((long)N * batch + 15) / 16 * parts;
   if (skinny_half(M, tiles, K / parts)) {
-    if (xg <= 1) return K / parts > 4096 ? HS_SK(1, 1, 3, false, true) : HS_SK(1, 1, 2, false, true);
-    return xg <= 2 ? HS_SK(2, 1, 2, false, true) : xg <= 3 ? HS_SK(3, 1, 2, false, true) : xg <= 4 ? HS_SK(4, 1, 2, false, true)
-         : xg <= 6 ? HS_SK(6, 1, 2, false, true) : HS_SK(8, 1, 2, false, true);
+    // 32 bits, whose products of a piece take longer than its copies, have what whole tiles have: two for up to 16 rows, up to 24 where the weights are
+    // 12 MB, else one. With two or three / so (whole tiles), us: 64 columns of k 4096, one row 8.2 / 7.7 (7.8), 64 rows 20.3 / 19.2 (19.4); 16 columns
+    // of k 8192, 20 rows 20.6 / 18.7 (19.0). 20 rows of 2048 columns of k 3072 10.4 with two, 11.0 with one.
+    if (xg <= 1) return K / parts > 4096 ? HS_SK(1, 1, 3, false, true, 2) : HS_SK(1, 1, 2, false, true);
+    if (xg == 3) return tiles * K / parts >= 393216 ? HS_SK(3, 1, 2, false, true) : HS_SK(3, 1, 2, false, true, 1);
+    return xg <= 2 ? HS_SK(2, 1, 2, false, true) : xg <= 4 ? HS_SK(4, 1, 2, false, true, 1) : xg <= 6 ? HS_SK(6, 1, 2, false, true, 1)
+         : HS_SK(8, 1, 2, false, true, 1);
   }
   const int nt = skinny_tiles(M, tiles, K / parts);
   // One piece ahead: two are faster (up to 40 %) where a wave waits for its few copies, up to 16 rows and more than a piece per wave (more than

@@ -114,6 +114,14 @@ def test_a_gate_is_asked_for_beside_the_weights_of_the_runs(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
+def test_half_tiles_of_32_bits_copy_no_further_ahead_than_whole_ones():
+    """The kernels that the library brings: groups of 8 rows, pieces ahead. 3 groups have one and two, by the weights' size."""
+    with open(_SEQ_LIBS["seq"], "rb") as f:
+        names = set(re.findall(rb"skinny_linear_kernelILi(\d)ELi1ELi(\d)ELb0EfLb1ELi0ELb1E", f.read()))
+    assert {(int(g), int(d)) for g, d in names} == {(1, 2), (2, 2), (3, 1), (3, 2), (4, 1), (6, 1), (8, 1)}
+
+
+@pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
 @pytest.mark.parametrize("cols,k,tiles_and_pairs", [   # measured: whether the kernel for few rows per tile is at least 10 % faster, or slower
     (2048, 1024, {(1, 1): True, (17, 32): True, (143, 4080): True}), (512, 512, {(1, 1): True, (64, 64): True, (36, 1020): True}),
     (2048, 704, {(4, 4): True, (66, 128): True, (572, 16320): True}), (1024, 640, {(16, 16): True, (132, 256): True}), (4096, 1024, {(64, 64): True, (1144, 32640): True}),
