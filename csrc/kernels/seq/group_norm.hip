@@ -397,9 +397,12 @@ void launch_group_norm(T* out, float* residual, const float* w, int T_, int H, i
                         (const void*)y, (const void*)ls2, (const void*)extra, (const void*)table})
     at |= reinterpret_cast<uintptr_t>(p);
   // 4, 8 and 16 waves, two expert rows or none: the widths and the choices per token of this package's own layer-list configurations, 1024, 2048 and 4096
-  // (both sides: at the kernel). Powers of two, so that a wave's group is a shift and 1 / columns exact; other sizes take the kernels below.
+  // (both sides: at the kernel). Powers of two, so that a wave's group is a shift and 1 / columns exact; other sizes take the kernels below. So do more than
+  // 2000 rows of 4096 16-bit elements from a table, whose 16 waves leave too few rows under way: 4096, 8192, 16384 rows 24.8 / 24.2, 58.3 / 55.0, 132 / 116 us
+  // (known / below; 2000 rows 14.9 / 14.9, 1000 9.1 - 9.3 / 9.4 - 9.6).
   const int waves = H / 256;
-  if (at % 16 == 0 && extra == nullptr && H % 256 == 0 && (waves == 4 || waves == 8 || waves == 16) && groups > 0 &&
+  const bool long_table = table != nullptr && waves == 16 && sizeof(T) == 2 && T_ > 2000;
+  if (!long_table && at % 16 == 0 && extra == nullptr && H % 256 == 0 && (waves == 4 || waves == 8 || waves == 16) && groups > 0 &&
       waves % groups == 0 && (y == nullptr || (top == 2 && ls2 != nullptr)) && (table != nullptr ? mix == nullptr && y == nullptr : mix != nullptr) &&
       mix_parts <= 4) {
     const KnownNormRest rest{out, mix_parts, T_, __builtin_ctz(waves / groups), (float)groups / (float)H, eps, table_rows};

@@ -110,6 +110,24 @@ def test_group_norm_of_known_sizes(H, groups, T, kind, dtype):
     assert ((got.cpu().double() - want).abs()[ok] <= tol * want.abs()[ok] + 3 * err).all()
 
 
+@gpu
+@pytest.mark.parametrize("T", [2000, 2001])
+@pytest.mark.parametrize("groups", [1, 16])
+def test_embedding_rows_of_long_prompts(T, groups):
+    """Wide rows from a table, at both sides of the change of kernels; ids outside the table give NaN."""
+    g = torch.Generator().manual_seed(T)
+    H, table, w, ids = 4096, torch.randn(50, 4096, generator=g).bfloat16(), 1 + 0.1 * torch.randn(4096, generator=g), torch.randint(0, 50, (T,), generator=g)
+    ids[[0, T - 1]] = torch.tensor([50, -1])
+    x = table[ids.clamp(0, 49)].double()
+    want = (x.view(T, groups, -1) * torch.rsqrt(x.view(T, groups, -1).square().mean(-1, keepdim=True) + 1e-6)).view(T, H) * w.double()
+    ops, res, out = get_ops("cuda"), torch.empty(T, H, device="cuda"), torch.empty(T, H, dtype=torch.bfloat16, device="cuda")
+    ops.norm_library = "delta"
+    ops.scaled_add_group_rmsnorm(out, res, w.cuda(), groups, 1e-6, table=table.cuda(), ids=ids.cuda())
+    res, out, known = res.cpu().double(), out.cpu().double(), slice(1, T - 1)
+    assert torch.equal(res[known], x[known]) and ((out - want).abs()[known] <= 2.0 ** -8 * want.abs()[known]).all()   # a neighbouring bf16 number
+    assert all(v[i].isnan().all() for v in (res, out) for i in (0, T - 1))
+
+
 # ------------------------------------------------------------------ soft cap
 @pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=gpu)])
 @pytest.mark.parametrize("shape", [(1, 5), (3, 2048), (2, 32001)])
