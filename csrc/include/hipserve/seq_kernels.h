@@ -25,6 +25,8 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
 
 // us that such a launch takes, cold weights; k in numbers of the operands' type
 double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts);
+// Tiles of 16 columns that a workgroup takes, where it doesn't take half a one
+int skinny_tiles(int M, long tiles, int K);
 // Whether its workgroups take 8 columns for 16; tiles of 16 columns, over all batches and parts, K in 16-bit halves
 bool skinny_half(int M, long tiles, int K);
 // A norm around such a product of up to 32 rows, in one part: with a residual [M, N] (fp32, updated in place), out = residual * weight
@@ -116,6 +118,26 @@ void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, cons
 
 // Whether so many launched tiles of 32 slots with so many pairs run the kernel for few rows per tile (cols of the result).
 bool expert_rows_pay(long ntiles, long pairs, long cols, long K);
+
+// The experts' product of tiles of 32 slots, as launch_expert_gemm (bf16, act 0 or 1), for a launch that holds a dense product besides.
+struct ExpertRows {
+  void* out;
+  const void *x, *w;
+  const int *slots, *tile_expert;
+  long x_ld, ntiles;
+  int gather_k, N, K, act, E, pairs;
+  long cap;   // slots
+};
+bool expert_rows_ok(const ExpertRows& ex);   // whether the kernel for few rows takes them
+// launch_skinny_linear (bf16, one batch, no bias or act) and the experts' product in one launch; false, and nothing done, where there is none for
+// these sizes.
+bool launch_skinny_linear_experts(void* out, bool out_f32, long out_ld, long out_zs, int parts, const void* x, long x_ld, const void* w, int M, int N,
+                                  int K, const ExpertRows& ex, hipStream_t s);
+
+// launch_mingru_product (bf16) alike.
+bool launch_mingru_product_experts(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x,
+                                   const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K,
+                                   const ExpertRows& ex, hipStream_t s);
 
 // Norms before and after a sublayer (sandwich.hip): residual[T, H] (fp32, in place; `table` [vocab, H] in the activation
 // type: it starts as table_scale * table[ids[t]]) += mult * y / rms(y) * w_post; out = residual / rms(residual) * w_next.

@@ -17,8 +17,7 @@
 // unrounded, and the states arrive beside its weights. Width 4096, K 2048, in a captured step: one row 11.6 + 4.4
 // -> 12.0 us, 48 rows 16.0 + 4.7 -> 15.4. The copies need no arguments that have to be loaded, and the rows' sequences come through the scalar unit:
 // 1, 16, 48, 64 rows 12.4 -> 11.5, 12.5 -> 11.8, 15.4 -> 14.6, 16.8 -> 15.7 (in a loop), width 2048, K 1024 5.0 -> 4.4, 5.2 -> 4.5, 7.4 -> 6.8, 8.3 -> 7.5.
-#include "skinny.h"
-#include "hipserve/seq_kernels.h"
+#include "expert_rows.h"
 
 #include <type_traits>
 
@@ -168,11 +167,13 @@ __global__ __launch_bounds__(256) void mingru_step_kernel(T* __restrict__ y, flo
   Row<float, kV>::st(st, S);
 }
 
+struct MinGruSeqs { const int *cu = nullptr, *ctx = nullptr, *state = nullptr; };
 struct MinGruRest {
   void* y;
   float* state;
   const float *b_z, *b_x;
   int nseq;
+  MinGruSeqs seqs;   // where the kernel has no parameters of them
 };
 struct MinGruArgs {
   const void *x, *w, *seq_cu, *seq_ctx, *seq_state;
@@ -181,16 +182,15 @@ struct MinGruArgs {
 };
 
 // y, state of the rows x [M, K], one per sequence, and w = [z rows; x rows; g rows]. F32: x, w, x_ld and K in 16-bit halves (skinny.h).
+// A MinGruRest lies at byte rest_at of the kernel's arguments.
 template <int XG, int DEPTH, bool F32>
-__global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
-    const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx,
-    const int* __restrict__ seq_state, int x_ld, int M, int width, int K, const MinGruRest) {
+HS_DEVICE void mingru_block(int wg, const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const MinGruSeqs& seqs, int x_ld, int M,
+                            int width, int K, int rest_at, unsigned char* smem) {
   using SK = Skinny<XG, 3, DEPTH, F32>;
   using T = std::conditional_t<F32, float, unsigned short>;
   constexpr int ST = SK::ST, IT = (ST + 1) / 2;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = blockIdx.x * 16, c = min(n0 + (tid & 15), width - 1);
+  const int n0 = wg * 16, c = min(n0 + (tid & 15), width - 1);
   const unsigned char* wt[3];
   unsigned w_row[6], x_row[XG];
 #pragma unroll
@@ -212,8 +212,10 @@ __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
   long at[IT];   // the channel's place in the row's state, -1: the row has no sequence
   bool fresh[IT];
   SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave, [&] {
-    const auto rest = late_args<MinGruRest>(offsetof(MinGruArgs, rest));
+    const auto rest = late_args<MinGruRest>(rest_at);
     const int nseq = rest->nseq;
+    const int *seq_cu = seqs.cu, *seq_ctx = seqs.ctx, *seq_state = seqs.state;
+    if (seq_cu == nullptr) { seq_cu = rest->seqs.cu; seq_ctx = rest->seqs.ctx; seq_state = rest->seqs.state; }
     y = static_cast<T*>(rest->y);
     state = rest->state;
     bz = rest->b_z[c];
@@ -247,10 +249,37 @@ __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
     const int m = (tid + kSkThreads * i) >> 4;
     if (m >= M || n0 + (tid & 15) >= width || at[i] < 0) continue;
     const Gru g(v[0][i], v[1][i], bz, bx);
-    const float o = g.keep * (fresh[i] ? 0.f : S[i]) + g.zc;
+    const float o = fmaf(g.keep, fresh[i] ? 0.f : S[i], g.zc);   // as the scan has it, in both kernels
     stf<T>(y, (long)m * width + c, o * (v[2][i] * sigmoid_f(v[2][i])));
     state[at[i]] = o;
   }
+}
+
+template <int XG, int DEPTH, bool F32>
+__global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
+    const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx,
+    const int* __restrict__ seq_state, int x_ld, int M, int width, int K, const MinGruRest) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  mingru_block<XG, DEPTH, F32>(blockIdx.x, x, w, MinGruSeqs{seq_cu, seq_ctx, seq_state}, x_ld, M, width, K, offsetof(MinGruArgs, rest), smem);
+}
+
+struct MinGruBesideArgs {
+  const void *x, *w, *slots, *tile_expert;
+  int x_ld, M, width, K, split;
+  MinGruRest rest;
+  ExpertBeside experts;
+};
+
+// The same with the experts' product of tiles with few rows besides (expert_beside.hip): workgroups from `split` on. One piece ahead, so that two workgroups
+// fit a compute unit.
+template <int XG, int DEPTH>
+__global__ __launch_bounds__(kSkThreads) void mingru_product_experts_kernel(
+    const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const int* __restrict__ slots, const int* __restrict__ tile_expert,
+    int x_ld, int M, int width, int K, int split, const MinGruRest, const ExpertBeside) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int b = blockIdx.x;
+  if (b >= split) expert_beside(b - split, slots, tile_expert, offsetof(MinGruBesideArgs, experts), smem);
+  else mingru_block<XG, DEPTH, false>(b, x, w, MinGruSeqs{}, x_ld, M, width, K, offsetof(MinGruBesideArgs, rest), smem);
 }
 
 template <int XG, int DEPTH>
@@ -259,12 +288,26 @@ bool launch_product(void* y, float* state, const void* x, long x_ld, const void*
   constexpr int lds = Skinny<XG, 3, DEPTH>::kLds;
   auto go = [&](auto* kernel) {
     kernel<<<(width + 15) / 16, kSkThreads, lds, s>>>((const unsigned short*)x, (const unsigned short*)w, seq_cu, seq_ctx, seq_state, (int)x_ld, M,
-                                                       width, K, MinGruRest{y, state, b_z, b_x, nseq});
+                                                       width, K, MinGruRest{y, state, b_z, b_x, nseq, {}});
   };
   static const bool ok = allow_lds(&mingru_product_kernel<XG, DEPTH, false>, lds) && allow_lds(&mingru_product_kernel<XG, DEPTH, true>, lds);
   if (!ok) return false;
   if (f32) go(&mingru_product_kernel<XG, DEPTH, true>);
   else go(&mingru_product_kernel<XG, DEPTH, false>);
+  return true;
+}
+
+template <int XG, int DEPTH>
+bool launch_beside(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x, const int* seq_cu,
+                   const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, const ExpertRows& ex, hipStream_t s) {
+  constexpr int own = Skinny<XG, 3, DEPTH>::kLds, lds = own > expert_lds<1>() ? own : expert_lds<1>();
+  static const bool ok = allow_lds(&mingru_product_experts_kernel<XG, DEPTH>, lds);
+  if (!ok) return false;
+  const int split = (width + 15) / 16;
+  const ExpertBeside experts = expert_beside_args(ex);
+  mingru_product_experts_kernel<XG, DEPTH><<<split + experts.per_tile * ex.ntiles, kSkThreads, lds, s>>>(
+      (const unsigned short*)x, (const unsigned short*)w, ex.slots, ex.tile_expert, (int)x_ld, M, width, K, split,
+      MinGruRest{y, state, b_z, b_x, nseq, {seq_cu, seq_ctx, seq_state}}, experts);
   return true;
 }
 
@@ -293,6 +336,15 @@ bool launch_mingru_product(void* y, float* state, const void* x, long x_ld, cons
   if (f32) { x_ld *= 2; K *= 2; }   // in halves
 #define HS_MG(XG, DEPTH) launch_product<XG, DEPTH>(y, state, x, x_ld, w, b_z, b_x, seq_cu, seq_ctx, seq_state, nseq, M, width, K, f32, s)
   return M <= 8 ? HS_MG(1, 2) : M <= 16 ? HS_MG(2, 2) : M <= 32 ? HS_MG(4, 1) : M <= 48 ? HS_MG(6, 1) : HS_MG(8, 1);
+#undef HS_MG
+}
+
+bool launch_mingru_product_experts(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x,
+                                   const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K,
+                                   const ExpertRows& ex, hipStream_t s) {
+  if (M <= 0 || nseq <= 0 || width <= 0 || M > 32 || !expert_rows_ok(ex)) return false;   // more rows: 96 KB, the experts would have a compute unit's LDS to themselves each
+#define HS_MG(XG, DEPTH) launch_beside<XG, DEPTH>(y, state, x, x_ld, w, b_z, b_x, seq_cu, seq_ctx, seq_state, nseq, M, width, K, ex, s)
+  return M <= 8 ? HS_MG(1, 1) : M <= 16 ? HS_MG(2, 1) : HS_MG(4, 1);
 #undef HS_MG
 }
 

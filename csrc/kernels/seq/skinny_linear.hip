@@ -10,187 +10,23 @@
 // read these rows (SkinnyNorm without one) sum the squares and scale their results, of which a norm's factor per row is part
 // as well. The rows are rounded once either way, and the update sees the unrounded product. Six norms less in a decode step of Fikizen: one
 // row, width 1024, 2450 -> 2328 us (17 steps), 16 rows, width 2048, 9271 -> 8957 (33 steps); both products take about 0.3 us longer.
-#include "skinny.h"
+#include "skinny_block.h"
 
 #include <algorithm>
 #include <cmath>
-#include <type_traits>
 
 #include "hipserve/seq_kernels.h"
 
 namespace hipserve {
 namespace {
 
-HS_DEVICE float skinny_act(float z, int act, float c0, float c1) {
-  if (act == 0) return tanhf(z);
-  if (act == 1) return z > 0.f ? c0 * z * z + 0.5f * z : c1 * (expm1f(z) - z) + 0.5f * z;
-  if (act == 2) { z = fmaxf(z, 0.f); return z * z; }
-  if (act == 5) return tanhf(z / c0) * c0;
-  return z;
-}
-
-// Sum over the lanes of a row's columns; every one of them gets it.
-template <int COLS> HS_DEVICE float cols_sum(float v) {
-  if constexpr (COLS == 16) return row_sum(v);
-  v = dpp_step<0xB1, 0xf, false>(v);      // quad_perm [1, 0, 3, 2]
-  v = dpp_step<0x4E, 0xf, false>(v);      // quad_perm [2, 3, 0, 1]
-  return dpp_step<0x141, 0xf, false>(v);  // row_half_mirror
-}
-
-enum { kPlain, kNormed, kUpdate };   // SkinnyNorm: none; rows without their norm's factor; a result that goes into the residual stream
-struct NoNorm {};
-// The kernel's arguments: the parameters are what its first loads need, the rest is loaded once the copies are on their way (seq_common.h), and
-// nothing is asked for after the product any more. us of four products in a captured loop (square, 3 x wider, back, 1.5 x wider), cold weights,
-// 1 and 16 rows: width 1024 15.1 -> 13.6, 17.4 -> 16.0, width 2048 24.4 -> 22.8, 29.4 -> 27.8.
-template <int NORM> struct SkinnyRest {
-  long x_bs, out_ld, out_bs, out_zs;
-  int act, act_from;
-  float c0, c1, cols, eps;
-  void* out;
-  float* squares;      // kUpdate
-  const void* bias;
-};
-template <int NORM> struct SkinnyArgs {
-  const void *x, *w, *p, *q;
-  int x_ld, M, N, K, i;
-  SkinnyRest<NORM> rest;
-};
-
-// XG: groups of 8 rows; NT: 16-column tiles (GLU: the gate's and the up projection's of the same 16 output columns).
-// F32: 32-bit operands, x, w, their strides and K in 16-bit halves (skinny.h). Workgroups z take `part` of K each (a multiple of 64) and write
-// their sums out_zs elements apart (the bias in the first).
-// p, q, i: kPlain - , bias, part; kNormed squares, bias, blocks; kUpdate residual, weight, blocks (K in one part for both).
 template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM, bool HALF>
 __global__ __launch_bounds__(kSkThreads) void skinny_linear_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, void* p, const void* q, int x_ld, int M, int N, int K, int ni,
     const SkinnyRest<NORM>) {
-  static_assert(!GLU || NT == 2, "a gate tile and an up tile");
-  using SK = Skinny<XG, NT, DEPTH, F32, HALF>;
-  constexpr int ST = SK::ST, kCols = SK::kCols;
-  using TB = std::conditional_t<F32, float, unsigned short>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int No = GLU ? N / 2 : N;
-  const int n0 = blockIdx.x * (GLU ? 16 : kCols * NT);
-  const int k0 = NORM == kPlain ? blockIdx.z * ni : 0, k1 = NORM == kPlain ? min(K, k0 + ni) : K;
-  const int rest_at = offsetof(SkinnyArgs<NORM>, rest);
-  if (NORM == kPlain && blockIdx.y != 0) {
-    x += (long)blockIdx.y * late_args<SkinnyRest<NORM>>(rest_at)->x_bs;
-    w += (long)blockIdx.y * N * K;
-  }
-  const unsigned char* wt[NT];
-  unsigned w_row[SK::WG];
-  unsigned x_row[XG];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    const int first = GLU ? n0 : min(n0 + 16 * nt, N - 1);   // of the tile's columns
-    wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)(GLU ? nt * No : 0) + first) * K + k0);
-#pragma unroll
-    for (int h = 0; h < (HALF ? 1 : 2); ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), No - 1 - first) * (unsigned)(2 * K);
-  }
-#pragma unroll
-  for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)(2 * x_ld);
-  f32x4 acc[NT][ST];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int IT = SK::kElems, SQ = HALF ? 8 : 4;   // kCols threads x SQ loads x 4 sums: 256 of them, rows of up to 4096 at 16 columns each
-  [[maybe_unused]] f32x4 sq[IT][SQ];
-  [[maybe_unused]] float res[IT][NT], wgt[NT];
-  [[maybe_unused]] TB bs[NT];
-  // for the epilogue, ahead of the copies: without branches, behind which the copies would be waited for, and first, since loads return in
-  // order and a wait for the copies would be one for these too
-  const int c = tid % kCols;
-  const bool biased = NORM != kUpdate && q != nullptr && blockIdx.z == 0;
-  const TB* bias = static_cast<const TB*>(biased ? q : x);
-#pragma unroll
-  for (int i = 0; i < IT; ++i) {
-    [[maybe_unused]] const long m = min((tid + kSkThreads * i) / kCols, M - 1);
-    if constexpr (NORM == kNormed) {
-#pragma unroll
-      for (int j = 0; j < SQ; ++j) sq[i][j] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(p) + m * ni + min(4 * kCols * j + 4 * c, ni - 4));
-    }
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const int n = (GLU ? nt * No : 0) + min(n0 + (GLU ? 0 : 16 * nt) + c, No - 1);
-      if constexpr (NORM == kUpdate) res[i][nt] = static_cast<const float*>(p)[m * N + n];
-      if (i == 0) {
-        if constexpr (NORM == kUpdate) wgt[nt] = static_cast<const float*>(q)[n];
-        else bs[nt] = bias[biased ? n : 0];
-      }
-    }
-  }
-  int act = 0, act_from = 0;
-  float c0 = 0.f, c1 = 0.f, cols = 1.f, eps = 0.f;
-  long out_ld = 0;
-  TO* out = nullptr;
-  [[maybe_unused]] float* squares = nullptr;
-  [[maybe_unused]] const TB* late_bias = nullptr;
-  SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x + k0), x_row, k1 - k0, smem, lane, wave, [&] {
-    const auto rest = late_args<SkinnyRest<NORM>>(rest_at);
-    out = static_cast<TO*>(rest->out);
-    out_ld = NORM == kPlain ? rest->out_ld : GLU ? No : N;
-    if constexpr (NORM == kPlain) out += (long)blockIdx.y * rest->out_bs + (long)blockIdx.z * rest->out_zs;
-    if constexpr (NORM == kUpdate) squares = rest->squares;
-    act = rest->act;
-    act_from = rest->act_from;
-    c0 = rest->c0;
-    c1 = rest->c1;
-    cols = rest->cols;
-    eps = rest->eps;
-    asm volatile("" ::"s"(act), "s"(act_from), "s"(c0), "s"(c1), "s"(cols), "s"(eps), "s"(out), "s"(out_ld), "s"(squares));
-    if constexpr (NORM == kUpdate) {
-      late_bias = static_cast<const TB*>(rest->bias);
-      if (late_bias != nullptr) {
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) bs[nt] = late_bias[n0 + 16 * nt + c];
-      }
-    }
-  });
-  float v[NT][IT];
-  SK::reduce(v, acc, smem);
-#pragma unroll
-  for (int i = 0; i < IT; ++i) {
-    const int e = tid + kSkThreads * i, m = e / kCols;
-    if (m >= M) continue;   // a row's lanes together
-    if constexpr (NORM == kUpdate) {   // N is a multiple of the workgroup's columns
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int n = n0 + 16 * nt + e % kCols;
-        const float r = res[i][nt] + (v[nt][i] + (late_bias != nullptr ? ldf<TB>(&bs[nt], 0) : 0.f));
-        static_cast<float*>(p)[(long)m * N + n] = r;
-        stf<TO>(out, m * out_ld + n, r * wgt[nt]);
-        const float s = cols_sum<kCols>(r * r);
-        if (e % kCols == 0) squares[(long)m * ni + n / kCols] = s;
-      }
-      continue;
-    }
-    if constexpr (NORM == kNormed) {
-      float s = 0.f;
-#pragma unroll
-      for (int j = 0; j < SQ; ++j)
-        if (4 * kCols * j + 4 * c < ni) s += (sq[i][j][0] + sq[i][j][1]) + (sq[i][j][2] + sq[i][j][3]);
-      const float inv = 1.f / sqrtf(cols_sum<kCols>(s) / cols + eps);
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) v[nt][i] *= inv;
-    }
-    if constexpr (GLU) {
-      const int n = n0 + (e & 15);
-      if (n >= No) continue;
-      const float gv = v[0][i] + (biased ? ldf<TB>(&bs[0], 0) : 0.f);
-      const float uv = v[1][i] + (biased ? ldf<TB>(&bs[1], 0) : 0.f);
-      stf<TO>(out, m * out_ld + n, act == 4 ? clamped_glu_f(gv, uv, c0) : gv * sigmoid_f(gv) * uv);
-    } else {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int n = n0 + 16 * nt + e % kCols;
-        if (n >= N) continue;
-        const float z = v[nt][i] + (biased ? ldf<TB>(&bs[nt], 0) : 0.f);
-        stf<TO>(out, m * out_ld + n, skinny_act(z, n >= act_from ? act : -1, c0, c1));
-      }
-    }
-  }
+  skinny_block<XG, NT, DEPTH, GLU, TO, F32, NORM, HALF>(blockIdx.x, blockIdx.y, blockIdx.z, x, w, p, q, x_ld, M, N, K, ni,
+                                                         offsetof(SkinnyArgs<NORM>, rest), smem);
 }
 
 template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM = kPlain, bool HALF = false>
@@ -231,18 +67,6 @@ bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, 
 #undef HS_SK
 }
 
-// How many tiles of 16 columns a workgroup takes. One, unless their workgroups are more than the compute units (or a few of them hold
-// many k each): then two or four share what they copy of the rows; up to 16 rows there is too little of that. Cold weights, us with 1 / 2 / 4
-// tiles: 6144 x 4096, 16 rows 14.5 / 15.1 / 21, 48 rows 20.9 / 18.7 / 26; 16384 x 2048, 16 rows 17.0 / 15.5 / 15.5, 24 rows 18.3 / 16.4 /
-// 16.2, 48 rows 22.6 / 19.4 / 18.8; 32000 x 512, 24 rows 10.4 / 10.0 / 11.9; 16384 x 4096, 64 rows 41.6 / 35.9 / 29.3.
-int skinny_tiles(int M, long tiles, int K) {
-  if (tiles <= 256) return 1;
-  if (M <= 16) return M > 8 && tiles <= 512 && K >= 8192 ? 2 : 1;
-  if (tiles <= 512) return K >= 1024 ? 2 : 1;
-  if (M > 48) return K >= 1024 ? 4 : 1;
-  return K >= 4096 ? 4 : 2;
-}
-
 // us of a launch (K in halves, over `parts`): a latency, the results, and the time the weights take at 5.2 TB/s, or, where that is more, at 9 TB/s and with it
 // what the busiest compute unit takes in (80 KB per us), its sums in LDS and its products of 32-bit operands. 9 % off on average over 5127 sizes (1 -
 // 64 rows, 64 - 65536 columns, k 128 - 12288, plain and gated, 32 bits).
@@ -254,6 +78,18 @@ double skinny_time_of(int M, long cols, double K, int nt, int parts, bool f32, d
 }
 
 }  // namespace
+
+// How many tiles of 16 columns a workgroup takes. One, unless their workgroups are more than the compute units (or a few of them hold
+// many k each): then two or four share what they copy of the rows; up to 16 rows there is too little of that. Cold weights, us with 1 / 2 / 4
+// tiles: 6144 x 4096, 16 rows 14.5 / 15.1 / 21, 48 rows 20.9 / 18.7 / 26; 16384 x 2048, 16 rows 17.0 / 15.5 / 15.5, 24 rows 18.3 / 16.4 /
+// 16.2, 48 rows 22.6 / 19.4 / 18.8; 32000 x 512, 24 rows 10.4 / 10.0 / 11.9; 16384 x 4096, 64 rows 41.6 / 35.9 / 29.3.
+int skinny_tiles(int M, long tiles, int K) {
+  if (tiles <= 256) return 1;
+  if (M <= 16) return M > 8 && tiles <= 512 && K >= 8192 ? 2 : 1;
+  if (tiles <= 512) return K >= 1024 ? 2 : 1;
+  if (M > 48) return K >= 1024 ? 4 : 1;
+  return K >= 4096 ? 4 : 2;
+}
 
 // Whether a workgroup takes half a tile, 8 columns: where whole ones leave half of the compute units idle, and K (in halves) is long enough for what
 // a workgroup takes in to matter. Two pieces ahead (three for up to 8 rows of more than 4096). The sums are the same. Cold weights, us, whole ->

@@ -73,22 +73,74 @@ void mingru_scan(at::Tensor& y, at::Tensor& state, const at::Tensor& proj, const
 }
 
 // mingru_scan of the rows x [M, K] of a step in which every sequence has one row at most, the product x . w^T included.
-void mingru_product(at::Tensor& y, at::Tensor& state, const at::Tensor& x, const at::Tensor& w, const at::Tensor& b_z,
-                    const at::Tensor& b_x, const at::Tensor& seq_cu, const at::Tensor& seq_ctx, const at::Tensor& seq_state) {
+void check_mingru_product(const at::Tensor& y, const at::Tensor& state, const at::Tensor& x, const at::Tensor& w, const at::Tensor& b_z,
+                          const at::Tensor& b_x, const at::Tensor& seq_cu, const at::Tensor& seq_ctx, const at::Tensor& seq_state) {
   CHECK_DEV(x); CHECK_CONTIG(w); CHECK_CONTIG(y); CHECK_F32(state); CHECK_F32(b_z); CHECK_F32(b_x);
   CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_state);
   for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&y, &state, &w, &b_z, &b_x, &seq_cu, &seq_ctx, &seq_state}) CHECK_SAME_DEV(*t, x);
-  const bool f32 = is_f32(x, "mingru_product");
-  const long per = f32 ? 4 : 8, M = x.size(0), K = x.size(-1), width = state.size(1), nseq = seq_ctx.numel();
+  const long per = is_f32(x, "mingru_product") ? 4 : 8, M = x.size(0), K = x.size(-1), width = state.size(1), nseq = seq_ctx.numel();
   TORCH_CHECK(y.scalar_type() == x.scalar_type() && w.scalar_type() == x.scalar_type());
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && state.dim() == 2 && w.size(0) == 3 * width && w.size(1) == K && y.numel() == M * width && M <= 64);
   TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % per == 0 && K % per == 0 && K < (1L << 24) && x.stride(0) < (1L << 24) && width < (1L << 26) &&
               (uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0, "mingru_product: rows at multiples of 16 bytes");
   TORCH_CHECK(b_z.numel() == width && b_x.numel() == width && seq_cu.numel() == nseq + 1 && seq_state.numel() >= nseq);
+}
+
+void mingru_product(at::Tensor& y, at::Tensor& state, const at::Tensor& x, const at::Tensor& w, const at::Tensor& b_z,
+                    const at::Tensor& b_x, const at::Tensor& seq_cu, const at::Tensor& seq_ctx, const at::Tensor& seq_state) {
+  check_mingru_product(y, state, x, w, b_z, b_x, seq_cu, seq_ctx, seq_state);
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   TORCH_CHECK(hipserve::launch_mingru_product(y.data_ptr(), state.data_ptr<float>(), x.data_ptr(), x.stride(0), w.data_ptr(),
                                               b_z.data_ptr<float>(), b_x.data_ptr<float>(), seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(),
-                                              seq_state.data_ptr<int>(), nseq, M, width, K, f32, cur_stream()), "mingru_product: LDS");
+                                              seq_state.data_ptr<int>(), seq_ctx.numel(), x.size(0), state.size(1), x.size(1),
+                                              x.scalar_type() == at::kFloat, cur_stream()), "mingru_product: LDS");
+}
+
+// The experts' product of expert_gemm (bf16, tiles of 32 slots) for a launch that holds a dense product of device `like`'s besides.
+hipserve::ExpertRows expert_rows(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, const at::Tensor& slots, const at::Tensor& tile_expert,
+                                 int64_t gather_k, int64_t act, int64_t pairs, int64_t tiles, const at::Tensor& like) {
+  CHECK_CONTIG(out); CHECK_CONTIG(w); CHECK_I32(slots); CHECK_I32(tile_expert);
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&out, &x, &w, &slots, &tile_expert}) CHECK_SAME_DEV(*t, like);
+  TORCH_CHECK(out.scalar_type() == at::kBFloat16 && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16, "experts beside: bf16");
+  TORCH_CHECK(w.dim() == 3 && x.dim() == 2 && x.stride(1) == 1 && out.dim() == 2 && (act == 0 || act == 1));
+  const long N = w.size(1), K = w.size(2), cap = slots.numel();
+  TORCH_CHECK(x.size(1) == K && out.size(1) == N && out.size(0) >= cap && cap % 32 == 0 && tile_expert.numel() * 32 >= cap);
+  TORCH_CHECK(gather_k > 0 || x.size(0) >= cap, "ungathered x needs one row per slot");
+  TORCH_CHECK(pairs > 0 && pairs <= cap && tiles > 0 && N < (1L << 31) && w.size(0) < (1L << 31));
+  return {out.data_ptr(), x.data_ptr(), w.data_ptr(), slots.data_ptr<int>(), tile_expert.data_ptr<int>(), x.stride(0),
+          std::min<long>(tiles, cap / 32), (int)gather_k, (int)N, (int)std::min<long>(K, 1L << 30), (int)act, (int)w.size(0), (int)pairs, cap};
+}
+
+// A plain product as skinny_linear (out [M, N]) or skinny_linear_parts (out [S, M, N] in 32 bits) and the experts' in one launch; false, and nothing
+// done, where there is none for these sizes.
+bool skinny_linear_experts(at::Tensor& out, const at::Tensor& x, const at::Tensor& w, at::Tensor& e_out, const at::Tensor& e_x, const at::Tensor& e_w,
+                           const at::Tensor& slots, const at::Tensor& tile_expert, int64_t gather_k, int64_t act, int64_t pairs, int64_t tiles) {
+  CHECK_DEV(x); CHECK_CONTIG(w); CHECK_CONTIG(out); CHECK_SAME_DEV(w, x); CHECK_SAME_DEV(out, x);
+  const bool f32 = out.scalar_type() == at::kFloat;
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 && (f32 || out.scalar_type() == at::kBFloat16));
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && (out.dim() == 2 || (out.dim() == 3 && f32)), "skinny_linear_experts: rows");
+  const long M = x.size(0), K = x.size(1), N = w.size(0), S = out.dim() == 3 ? out.size(0) : 1;
+  TORCH_CHECK(w.size(1) == K && out.size(-2) == M && out.size(-1) == N && M <= 64 && K % 8 == 0 && N < (1L << 31) && K < (1L << 24) &&
+              x.stride(0) < (1L << 24) && S >= 1 && S <= 64 && S <= (K + 63) / 64, "skinny_linear_experts: shapes");
+  auto aligned = [](const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
+  TORCH_CHECK(x.stride(1) == 1 && x.stride(0) % 8 == 0 && aligned(x) && aligned(w), "skinny_linear_experts: rows at multiples of 16 bytes");
+  const auto ex = expert_rows(e_out, e_x, e_w, slots, tile_expert, gather_k, act, pairs, tiles, x);
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  return hipserve::launch_skinny_linear_experts(out.data_ptr(), f32, N, M * N, S, x.data_ptr(), x.stride(0), w.data_ptr(), M, N, K, ex, cur_stream());
+}
+
+// mingru_product and the experts' product in one launch, alike.
+bool mingru_product_experts(at::Tensor& y, at::Tensor& state, const at::Tensor& x, const at::Tensor& w, const at::Tensor& b_z, const at::Tensor& b_x,
+                            const at::Tensor& seq_cu, const at::Tensor& seq_ctx, const at::Tensor& seq_state, at::Tensor& e_out, const at::Tensor& e_x,
+                            const at::Tensor& e_w, const at::Tensor& slots, const at::Tensor& tile_expert, int64_t gather_k, int64_t act,
+                            int64_t pairs, int64_t tiles) {
+  check_mingru_product(y, state, x, w, b_z, b_x, seq_cu, seq_ctx, seq_state);
+  TORCH_CHECK(x.scalar_type() == at::kBFloat16, "mingru_product_experts: bf16");
+  const auto ex = expert_rows(e_out, e_x, e_w, slots, tile_expert, gather_k, act, pairs, tiles, x);
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  return hipserve::launch_mingru_product_experts(y.data_ptr(), state.data_ptr<float>(), x.data_ptr(), x.stride(0), w.data_ptr(), b_z.data_ptr<float>(),
+                                                 b_x.data_ptr<float>(), seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_state.data_ptr<int>(),
+                                                 seq_ctx.numel(), x.size(0), state.size(1), x.size(1), ex, cur_stream());
 }
 
 }  // namespace
@@ -119,6 +171,11 @@ TORCH_LIBRARY(hipserve_seq, m) {
   });
   m.def("mingru_product(Tensor(a!) y, Tensor(b!) state, Tensor x, Tensor w, Tensor b_z, Tensor b_x, Tensor seq_cu, Tensor seq_ctx, "
         "Tensor seq_state) -> ()");
+  m.def("mingru_product_experts(Tensor(a!) y, Tensor(b!) state, Tensor x, Tensor w, Tensor b_z, Tensor b_x, Tensor seq_cu, Tensor seq_ctx, "
+        "Tensor seq_state, Tensor(c!) e_out, Tensor e_x, Tensor e_w, Tensor slots, Tensor tile_expert, int gather_k, int act, int pairs, "
+        "int tiles) -> bool");
+  m.def("skinny_linear_experts(Tensor(a!) out, Tensor x, Tensor w, Tensor(b!) e_out, Tensor e_x, Tensor e_w, Tensor slots, Tensor tile_expert, "
+        "int gather_k, int act, int pairs, int tiles) -> bool");
   m.def("mingru_scan(Tensor(a!) y, Tensor(b!) state, Tensor proj, Tensor b_z, Tensor b_x, Tensor seq_cu, "
         "Tensor seq_ctx, Tensor seq_state, int max_q) -> ()");
 }
@@ -133,4 +190,6 @@ TORCH_LIBRARY_IMPL(hipserve_seq, CUDA, m) {
   m.impl("latent_prompt_attention", &latent_prompt_attention);
   m.impl("mingru_scan", &mingru_scan);
   m.impl("mingru_product", &mingru_product);
+  m.impl("mingru_product_experts", &mingru_product_experts);
+  m.impl("skinny_linear_experts", &skinny_linear_experts);
 }

@@ -51,7 +51,8 @@ HIP_FLAGS = [
 LIBS = {
     "core": ("_C.so", ["kernels/*.hip"], "torch_bindings.cpp"),
     "seq": ("_C_seq.so", ["kernels/seq/group_norm.hip", "kernels/seq/latent_attention*.hip", "kernels/seq/mingru.hip",
-                          "kernels/seq/expert_ffn.hip", "kernels/seq/skinny_linear.hip", "kernels/moe.hip"], "seq_bindings.cpp"),
+                          "kernels/seq/expert_ffn.hip", "kernels/seq/expert_beside.hip", "kernels/seq/skinny_linear.hip", "kernels/moe.hip"],
+            "seq_bindings.cpp"),
     "delta": ("_C_delta.so", ["kernels/seq/group_norm.hip", "kernels/seq/window_attention*.hip",
                               "kernels/seq/delta_scan.hip", "kernels/seq/delta_chunk.hip", "kernels/seq/delta_rule_*.hip",
                               "kernels/seq/sandwich.hip", "kernels/seq/router.hip", "kernels/seq/expert_ffn.hip",

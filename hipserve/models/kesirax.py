@@ -183,14 +183,16 @@ class KesiraxModel:
         aligned = dict(zip(experts, aligned)) if aligned is not None else {}
         for r, (i, _, _) in enumerate(self.runs):
             lw = self.layers[i]
-            if isinstance(lw.mixer, LatentAttention):
-                mix = lw.mixer.forward(h, meta, kv_caches[r])
-            else:
-                mix = lw.mixer.forward(h, meta, state[r])
-            y = pair_slot = None
+            y = pair_slot = steps = None
+            if i in aligned and T <= ops.SKINNY_ROWS:   # the experts' products go into launches of the mixer's, which are independent of them
+                y, pair_slot, steps = lw.mlp.steps(h, aligned[i])
+            mix = lw.mixer.forward(h, meta, kv_caches[r] if isinstance(lw.mixer, LatentAttention) else state[r], beside=steps)
             top = 0
             if lw.mlp is not None:
-                y, pair_slot = lw.mlp.forward(h, ids, aligned.get(i))
+                if steps is not None:
+                    steps.finish()
+                else:
+                    y, pair_slot = lw.mlp.forward(h, ids, aligned.get(i))
                 top = lw.mlp.spec.top
             last = r + 1 == len(self.runs)
             nxt = self.final_norm if last else self.layers[self.runs[r + 1][0]].norm

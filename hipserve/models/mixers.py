@@ -78,6 +78,7 @@ import torch.nn.functional as F
 
 from ..config import (DeltaRuleSpec, DenseFFSpec, GatedDeltaSpec, LatentAttentionSpec, LightningSpec, MinGRUSpec, MLstmSpec,
                       ParallelMixerSpec, RoutedMoESpec, TableMoESpec, WindowAttentionSpec, WkvSpec)
+from ..ops import ExpertSteps
 
 MOE_TILE = 32        # slots per expert tile of the expert GEMMs ...
 MOE_TILE_LARGE = 64  # ... when every expert has several tiles' worth of rows on average
@@ -103,15 +104,16 @@ def _side(sub, proj: torch.Tensor):
     sub.side_out = proj[:, proj.shape[1] - n:] if n else None
 
 
-def _last(sub, x: torch.Tensor, w: torch.Tensor, b=None, update=None):
+def _last(sub, x: torch.Tensor, w: torch.Tensor, b=None, update=None, beside=None):
     """The last product of a sublayer: [T, hidden], or 32-bit parts of it [parts, T, hidden] for a model whose residual update adds
     them up (it sets ``takes_parts``); with ``update`` = (residual, the next norm's weights, eps) the product may do the update
-    itself and return the next sublayer's ``NormedRows``."""
+    itself and return the next sublayer's ``NormedRows``; ``beside``: an ``ops.ExpertSteps`` whose next product may go into the launch."""
     if update is not None:
         rows = sub.ops.linear_update(x, w, b, *update)
         if rows is not None:
             return rows
-    return sub.ops.linear_parts(x, w, b) if getattr(sub, "takes_parts", False) else sub.ops.linear(x, w, b)
+    linear = sub.ops.linear_parts if getattr(sub, "takes_parts", False) else sub.ops.linear
+    return linear(x, w, b, beside=beside)
 
 
 def _deinterleave(w: torch.Tensor, dims: int) -> torch.Tensor:
@@ -205,22 +207,23 @@ class LatentAttention:
     def cache_shape(self, num_blocks: int, block_size: int):
         return (num_blocks, block_size, self.spec.key_dim)
 
-    def forward(self, h: torch.Tensor, meta, cache: torch.Tensor, state=None) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta, cache: torch.Tensor, state=None, beside=None) -> torch.Tensor:
+        """``beside``: ``ops.ExpertSteps`` that read ``h`` and may go into the launches of the plain products."""
         s, ops = self.spec, self.ops
         T = h.shape[0]
-        proj = self.ops.linear(h, self.w_in)
+        proj = self.ops.linear(h, self.w_in, beside=beside)
         _side(self, proj)
         gate_off = s.q_rank + s.key_dim
         cq = torch.empty(T, s.q_rank, device=h.device, dtype=h.dtype)
         ops.latent_prepare(cq, cache, proj, meta.positions, meta.slot_mapping, self.q_norm, self.kv_norm,
                            self.inv_freq, s.q_rank, s.kv_rank, s.rot_dim, self.eps)
-        q = self.ops.linear(cq, self.w_uq)                             # [T, heads * (dim + rot_dim)]
+        q = self.ops.linear(cq, self.w_uq, beside=beside)              # [T, heads * (dim + rot_dim)]
         rows = ops.latent_prompt_rows(h.dtype, s, self.inv_freq.numel(), cache, meta, T)
         if rows:   # a prompt step: every head's keys and values are formed
             cat = torch.empty(T, s.heads * s.vdim, device=h.device, dtype=h.dtype)
             ops.latent_prompt_attention(cat, q, proj, cache, meta, self.inv_freq, s, self.w_kv, rows,
                                         -1 if s.gate == "none" else gate_off)
-            return _last(self, cat, self.w_o)
+            return _last(self, cat, self.w_o, beside=beside)
         qh = q.view(T, s.heads, s.dim + s.rot_dim)
         if ops.latent_query_in_place(h.dtype, s.kv_rank, s.rot_dim):
             # the absorption GEMM writes the attention kernel's query rows directly: bf16, the cached width,
@@ -238,15 +241,15 @@ class LatentAttention:
                              s.kv_rank, gate_off if s.gate == "head" else -1, s.scale, s.window)
         cat = torch.empty(T, s.heads * s.vdim, device=h.device, dtype=h.dtype)
         if s.gate != "channel" and ops.linear_heads(cat.view(T, s.heads, s.vdim).transpose(0, 1), o_lat, self.w_uv):
-            return _last(self, cat, self.w_o)                          # the heads were written side by side
+            return _last(self, cat, self.w_o, beside=beside)           # the heads were written side by side
         o = torch.empty(s.heads, T, s.vdim, device=h.device, dtype=h.dtype)
         if not ops.linear_heads(o, o_lat, self.w_uv):
             torch.bmm(o_lat, self.w_uv_t, out=o)                       # [heads, T, vdim]
         if s.gate == "channel":
             # heads side by side per token, each element times the sigmoid of its gate column: one pass
             ops.gate_mul(cat, o, proj[:, gate_off:gate_off + s.heads * s.vdim])
-            return _last(self, cat, self.w_o)
-        return _last(self, o.transpose(0, 1).reshape(T, s.heads * s.vdim), self.w_o)
+            return _last(self, cat, self.w_o, beside=beside)
+        return _last(self, o.transpose(0, 1).reshape(T, s.heads * s.vdim), self.w_o, beside=beside)
 
 
 class MinGRU:
@@ -276,11 +279,11 @@ class MinGRU:
     def state_shape(self, num_slots: int):
         return (num_slots, self.spec.width)
 
-    def forward(self, h: torch.Tensor, meta, state: torch.Tensor) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, meta, state: torch.Tensor, beside=None) -> torch.Tensor:
         y = torch.empty(h.shape[0], self.spec.width, device=h.device, dtype=h.dtype)
-        if not self.ops.mingru_product(y, state, h, self.w_in, self.b_z, self.b_x, meta):
-            self.ops.mingru_scan(y, state, self.ops.linear(h, self.w_in), self.b_z, self.b_x, meta)
-        return _last(self, y, self.w_o)
+        if not self.ops.mingru_product(y, state, h, self.w_in, self.b_z, self.b_x, meta, beside=beside):
+            self.ops.mingru_scan(y, state, self.ops.linear(h, self.w_in, beside=beside), self.b_z, self.b_x, meta)
+        return _last(self, y, self.w_o, beside=beside)
 
 
 class TableMoE:
@@ -341,22 +344,26 @@ class TableMoE:
         m.ops.moe_table_align(tables, ids, m.spec.experts, tile, *aligned)
         return [(tile, *a) for a in zip(*aligned)]
 
+    def steps(self, h: torch.Tensor, aligned):
+        """(y, pair_slot) as ``forward`` returns them, once the ``ExpertSteps`` that come with them have run."""
+        s, P = self.spec, h.shape[0] * self.spec.top
+        tile, slots, tile_expert, pair_slot = aligned
+        act = torch.empty(slots.shape[0], s.ff, device=h.device, dtype=h.dtype)
+        y = torch.empty(slots.shape[0], self.hidden, device=h.device, dtype=h.dtype)
+        return y, pair_slot, ExpertSteps(self.ops, [(act, h, self.w_up, slots, tile_expert, tile, s.top, True, P, P),
+                                                    (y, act, self.w_down, slots, tile_expert, tile, 0, False, P, P)])
+
     def forward(self, h: torch.Tensor, ids: torch.Tensor, aligned=None):
-        s, ops = self.spec, self.ops
-        T, dev = h.shape[0], h.device
-        P = T * s.top
+        s = self.spec
+        P = h.shape[0] * s.top
         if aligned is None and self._packed_ok(h, P):
             return self._forward_packed(h, ids, P)
         if aligned is None:
-            tile, (slots, tile_expert, pair_slot) = self._tables(P, dev)
-            ops.moe_table_align(self.table, ids, s.experts, tile, slots, tile_expert, pair_slot)
-        else:
-            tile, slots, tile_expert, pair_slot = aligned
-        cap = slots.shape[0]
-        act = torch.empty(cap, s.ff, device=dev, dtype=h.dtype)
-        ops.expert_gemm(act, h, self.w_up, slots, tile_expert, tile, s.top, True, pairs=P, tiles=P)
-        y = torch.empty(cap, self.hidden, device=dev, dtype=h.dtype)
-        ops.expert_gemm(y, act, self.w_down, slots, tile_expert, tile, 0, False, pairs=P, tiles=P)
+            tile, tables = self._tables(P, h.device)
+            self.ops.moe_table_align(self.table, ids, s.experts, tile, *tables)
+            aligned = (tile, *tables)
+        y, pair_slot, steps = self.steps(h, aligned)
+        steps.finish()
         return y, pair_slot
 
     def _packed_ok(self, h: torch.Tensor, P: int) -> bool:

@@ -112,6 +112,31 @@ class NormedRows:
         return (self.rows.float() * torch.rsqrt(self.squares.sum(1, keepdim=True) / self.shape[1] + self.eps)).to(self.dtype)
 
 
+class ExpertSteps:
+    """The products of a step's experts, to be launched in their order: each beside an independent product of the same step that takes it
+    into its launch (``take``), or on its own (``finish``). None of them reads or writes what such a product writes or reads."""
+
+    def __init__(self, ops, products):
+        self.ops, self.left = ops, list(products)
+
+    def take(self, launch) -> bool:
+        """Whether ``launch`` (out, x, w, slots, tile_expert, gather_k, act, pairs, tiles) has taken the next product along."""
+        if not self.left:
+            return False
+        out, x, w, slots, tile_expert, tile, gather_k, act, pairs, tiles = self.left[0]
+        if not (tile == 32 and x.dtype == torch.bfloat16 and int(act) <= 1 and pairs > 0 and tiles > 0):
+            return False
+        if not launch(out, x, w, slots, tile_expert, gather_k, int(act), pairs, tiles):
+            return False
+        del self.left[0]
+        return True
+
+    def finish(self):
+        for out, x, w, slots, tile_expert, tile, gather_k, act, pairs, tiles in self.left:
+            self.ops.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, act, pairs=pairs, tiles=tiles)
+        self.left = []
+
+
 class KernelOps:
     """gfx950 HIP kernels (all outputs written in place; graph-capturable)."""
 
@@ -345,11 +370,14 @@ class KernelOps:
         apart = min(self._skinny_time(rows, 3 * width, k, False, f32), 1.2 * self._vendor_time(rows, 3 * width, k, f32))
         return self._seq.mingru_product_time(rows, width, k, f32) < apart + (1.0 if f32 else 2.0)
 
-    def mingru_product(self, y, state, x, w, b_z, b_x, meta) -> bool:
-        """``mingru_scan`` of the product x . w^T for a step of one row per sequence; False, and nothing done, where they are two launches."""
+    def mingru_product(self, y, state, x, w, b_z, b_x, meta, beside=None) -> bool:
+        """``mingru_scan`` of the product x . w^T for a step of one row per sequence; False, and nothing done, where they are two launches.
+        ``beside``: an ``ExpertSteps`` whose next product may go into the launch."""
         if not (meta.max_q == 1 and x.dim() == 2 and self._skinny_ok(x, w) and self.mingru_pays(x.shape[0], y.shape[-1], w.shape[1], x.dtype == torch.float32)):
             return False
-        self._seq.mingru_product(y, state, x, w, b_z, b_x, meta.seq_cu, meta.seq_ctx, meta.seq_state)
+        seqs = (meta.seq_cu, meta.seq_ctx, meta.seq_state)
+        if beside is None or not beside.take(lambda *e: self._seq.mingru_product_experts(y, state, x, w, b_z, b_x, *seqs, *e)):
+            self._seq.mingru_product(y, state, x, w, b_z, b_x, *seqs)
         return True
 
     def mingru_scan(self, y, state, proj, b_z, b_x, meta):
@@ -587,12 +615,27 @@ class KernelOps:
             return float("inf")
         return self._skinny_time(rows, cols, k, False, f32, p) + (p > 1) * 0.7 + (p - 1) * (0.15 + 0.2e-5 * rows * cols)
 
-    def linear_parts(self, x, w, bias=None):
+    def _linear_beside(self, x, w, beside, parts=1):
+        """The product x . w^T in one launch with the next product of ``beside``, or None. What would be ``parts`` of k without it is one, still in 32
+        bits: the experts fill the compute units that parts are for. From 33 rows on such a product holds a compute unit for longer than the launch saves:
+        16 experts of 2048 x 1024 beside 2048 x 4096, us apart / in one launch: 32 rows 20.6 / 19.3, 48 rows 21.9 / 23.6, 64 rows 23.0 / 25.6; 8 of
+        1024 x 512 beside 1024 x 2048, 40, 64 rows 7.9 / 6.4, 8.5 / 7.6."""
+        if parts > 1 and x.shape[0] > 32 and w.numel() > 1 << 21:
+            return None
+        T, N = x.shape[0], w.shape[0]
+        out = torch.empty(*((1, T, N) if parts > 1 else (T, N)), device=x.device, dtype=torch.float32 if parts > 1 else x.dtype)
+        return out if beside.take(lambda *e: self._seq.skinny_linear_experts(out, x, w, *e)) else None
+
+    def linear_parts(self, x, w, bias=None, beside=None):
         """``linear`` for a result that ``scaled_add_group_rmsnorm`` takes as ``mix``: where that is faster, 32-bit sums over parts of k,
-        [parts, T, N]."""
+        [parts, T, N]. ``beside``: an ``ExpertSteps`` whose next product may go into the launch."""
         if x.dim() == 2 and x.shape[0] <= self.SKINNY_ROWS and self._skinny_ok(x, w, bias):
             T, N, K = x.shape[0], w.shape[0], w.shape[1]
             parts = self.skinny_parts(T, N, K, x.dtype == torch.float32)
+            if parts and bias is None and beside is not None:
+                out = self._linear_beside(x, w, beside, parts)
+                if out is not None:
+                    return out
             if parts > 1:
                 out = torch.empty(parts, T, N, device=x.device, dtype=torch.float32)
                 self._moe_lib.skinny_linear_parts(out, x, w, bias)
@@ -611,10 +654,10 @@ class KernelOps:
                 and x.data_ptr() % 16 == 0 and w.is_contiguous() and w.data_ptr() % 16 == 0
                 and (bias is None or (bias.dtype == x.dtype and bias.shape == w.shape[:1] and bias.is_contiguous())))
 
-    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0):
+    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0, beside=None):
         """act(x . w^T + bias) of rows x [T, K]; ``out_f32``: a 32-bit result of 16-bit operands; ``act_from``: the first column that
         the activation applies to. A few rows run the weight-streaming kernel with the activation in its epilogue, anything else the
-        vendor's GEMM and a second launch."""
+        vendor's GEMM and a second launch. ``beside``: an ``ExpertSteps`` whose next product may go into the launch of a plain one."""
         if isinstance(x, NormedRows):
             if self._skinny_ok(x.rows, w, bias):
                 N = w.shape[0] // 2 if act in self.GLU_ACTS else w.shape[0]
@@ -624,6 +667,10 @@ class KernelOps:
             x = x.normed()
         if (x.dim() == 2 and x.shape[0] <= self.SKINNY_ROWS and self._skinny_ok(x, w, bias)
                 and self.skinny_pays(x.shape[0], w.shape[0], w.shape[1], act in self.GLU_ACTS, x.dtype == torch.float32, act is not None)):
+            if beside is not None and bias is None and act is None and not out_f32:
+                out = self._linear_beside(x, w, beside)
+                if out is not None:
+                    return out
             return self._skinny_linear(x, w, bias, out_f32, act, c0, c1, act_from)
         if out_f32 and x.dtype != torch.float32:
             y = torch.mm(x, w.t(), out_dtype=torch.float32)
@@ -967,7 +1014,7 @@ class ReferenceOps:
     def latent_prompt_rows(self, dtype, sp, nfreq, cache, meta, T) -> int:
         return 0
 
-    def mingru_product(self, y, state, x, w, b_z, b_x, meta) -> bool:
+    def mingru_product(self, y, state, x, w, b_z, b_x, meta, beside=None) -> bool:
         return False
 
     def mingru_scan(self, y, state, proj, b_z, b_x, meta):
@@ -1065,7 +1112,7 @@ class ReferenceOps:
         ref.delta_rule(out, state[0], proj, wl, a_b, w0, norm_w, sp, eps, meta.seq_cu, meta.seq_ctx,
                        meta.seq_state, out_scale)
 
-    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0):
+    def linear(self, x, w, bias=None, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0, beside=None):
         if out_f32 and x.dtype != torch.float32:
             x, w, bias = x.float(), w.float(), None if bias is None else bias.float()
         y = F.linear(x, w, bias)
@@ -1077,7 +1124,7 @@ class ReferenceOps:
         out = y.new_empty(*y.shape[:-1], y.shape[-1] // 2) if act in KernelOps.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)
 
-    def linear_parts(self, x, w, bias=None):
+    def linear_parts(self, x, w, bias=None, beside=None):
         return self.linear(x, w, bias)
 
     def linear_update(self, x, w, bias, residual, norm_w, eps):

@@ -1632,3 +1632,70 @@ def test_expert_gemm_of_known_tiles_by_the_other_kernels(tile, dtype, E, top, N,
     # a result of its type, and the sums' rounding
     assert ((outs[0].double() - y).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * y.abs() + K * 2.0 ** -23 * size).all()
     assert torch.equal(outs[1], outs[0]) and torch.equal(outs[2], outs[0])
+
+
+# ------------------------------------------------------------------ experts beside another product
+@gpu
+@pytest.mark.parametrize("M,N,K,parts", [(1, 8, 64, 1), (1, 3232, 2048, 1), (3, 2048, 4160, 2), (7, 1000, 4800, 1), (9, 2048, 1048, 1), (16, 1032, 520, 4), (24, 4104, 1024, 1),
+                                         (33, 2000, 2048, 1), (41, 2048, 4096, 4), (48, 6152, 1096, 1), (64, 40, 8192, 2), (64, 4112, 2048, 1)])
+@pytest.mark.parametrize("E,top,eN,eK,gather", [(16, 2, 1024, 2048, True), (3, 3, 40, 648, False)])
+def test_experts_beside_a_product(M, N, K, parts, E, top, eN, eK, gather):
+    """Every form of the dense product, tiles of one row to 32: the bits of the two launches."""
+    g = torch.Generator().manual_seed(M + N + E)
+    P, tile, ops = M * top, 32, get_ops("cuda")
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()  # noqa: E731
+    ids = torch.stack([torch.randperm(E, generator=g)[:top] for _ in range(M)]).int().cuda()
+    cap = -(-(P + E * (tile - 1)) // tile) * tile
+    slots, te, ps = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (cap, cap // tile, P))
+    ops.moe_align(ids.view(-1), E, tile, slots, te, ps)
+    x, w, ex, ew = rnd(M, K + 8)[:, :K], rnd(N, K) / K ** 0.5, rnd(M if gather else cap, eK), rnd(E, eN, eK) / eK ** 0.5
+    nan = lambda *s, dt=torch.bfloat16: torch.full(s, float("nan"), dtype=dt, device="cuda")  # noqa: E731
+    k = top if gather else 0
+    want_e, got_e = nan(cap, eN), nan(cap, eN)
+    ops.expert_gemm(want_e, ex, ew, slots, te, tile, k, int(gather), pairs=P, tiles=P)
+    dt = torch.float32 if parts > 1 else torch.bfloat16
+    want, got = (nan(*((parts, M, N) if parts > 1 else (M, N)), dt=dt) for _ in range(2))
+    if parts > 1:
+        ops._seq.skinny_linear_parts(want, x, w, None)
+    else:
+        ops._seq.skinny_linear(want, x, w, None, -1, 0.0, 0.0)
+    assert ops._seq.skinny_linear_experts(got, x, w, got_e, ex, ew, slots, te, k, int(gather), P, P)
+    assert torch.equal(got, want) and torch.equal(got_e[ps.long()], want_e[ps.long()])
+    # minGRU's product
+    width, n = max(8, N // 4), M
+    wide, bz, bx, state = rnd(3 * width, K) / K ** 0.5, *(torch.randn(*s, generator=g).cuda() for s in ((width,), (width,), (n + 2, width)))
+    cu, ctx = torch.arange(n + 1, dtype=torch.int32, device="cuda"), torch.arange(n, dtype=torch.int32, device="cuda") % 3 + 1
+    seq = torch.randperm(n + 2, generator=g)[:n].int().cuda()
+    outs = []
+    for beside in (False, True):
+        y, s, e = nan(M, width), state.clone(), nan(cap, eN)
+        if beside and ops._seq.mingru_product_experts(y, s, x, wide, bz, bx, cu, ctx, seq, e, ex, ew, slots, te, k, int(gather), P, P):
+            assert M <= 32
+        else:
+            assert not beside or M > 32
+            ops._seq.mingru_product(y, s, x, wide, bz, bx, cu, ctx, seq)
+            e = want_e
+        outs.append((y, s, e[ps.long()]))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+class _Recorder:
+    """Expert products that are asked for and never launched."""
+
+
+def test_expert_steps_run_in_order_and_once():
+    from hipserve.ops import ExpertSteps
+
+    ran = []
+    ops = _Recorder()
+    ops.expert_gemm = lambda out, *a, **kw: ran.append(("alone", out))
+    h = torch.zeros(1, 8, dtype=torch.bfloat16)
+    steps = ExpertSteps(ops, [(i, h, h, h, h, 32, 1, True, 2, 2) for i in "ab"])
+    assert not steps.take(lambda *e: False) and steps.take(lambda *e: ran.append(("beside", e[0])) or True)
+    steps.finish()
+    steps.finish()
+    assert ran == [("beside", "a"), ("alone", "b")] and not steps.take(lambda *e: True)
+    for other in (dict(tile=64), dict(x=h.float()), dict(pairs=0), dict(tiles=0), dict(act=2)):
+        a = dict(out="a", x=h, w=h, slots=h, te=h, tile=32, k=1, act=0, pairs=2, tiles=2, **{})
+        a.update(other)
+        assert not ExpertSteps(ops, [tuple(a.values())]).take(lambda *e: True)
