@@ -495,7 +495,7 @@ class WindowAttention:
             t["sink"] = _rand(gen, s.heads)
         return t
 
-    takes_proj = property(lambda self: self.b_in is None and not self.side_rows)   # ``mix`` takes ``proj`` from outside
+    takes_proj = property(lambda self: not self.side_rows)   # ``mix`` takes ``proj`` from outside
 
     def mix(self, h, meta, cache, state, out, out_scale: float = 1.0, proj=None):
         """Head outputs (before the output projection), times ``out_scale``, into ``out`` [T, heads * vdim]
@@ -679,6 +679,8 @@ class GatedDelta:
 
 class DeltaRule:
     cache_dim = 0
+    takes_proj = True
+    in_act = property(lambda self: ("tanh", 5 * self.spec.size))   # of the input projection's columns from the second on
 
     def __init__(self, spec: DeltaRuleSpec, hidden: int, eps: float, device, dtype, ops):
         self.spec, self.hidden, self.eps, self.device, self.dtype, self.ops = spec, hidden, eps, device, dtype, ops
@@ -712,9 +714,10 @@ class DeltaRule:
                   "a.b": _rand(gen, N, std=0.5), "norm": 1.0 + 0.2 * _rand(gen, N), "o": _rand(gen, H, N, std=std)})
         return t
 
-    def mix(self, h, meta, cache, state, out, out_scale: float = 1.0):
+    def mix(self, h, meta, cache, state, out, out_scale: float = 1.0, proj=None):
         N, ops = self.spec.size, self.ops
-        proj = ops.linear(h, self.w_in, act="tanh", act_from=5 * N)
+        if proj is None:
+            proj = ops.linear(h, self.w_in, act=self.in_act[0], act_from=self.in_act[1])
         if ops.delta_rule_low(out, state, proj, self.w2, self.a_b, self.w0, self.norm, self.spec, self.eps, meta, out_scale):
             return out
         wl = ops.linear(proj[:, 5 * N:], self.w2, out_f32=True)
@@ -841,7 +844,9 @@ class ParallelMixer:
         self.w_o = None      # [hidden, left out | right out]
         self.left_norm = self.right_norm = None   # fp32 [hidden] with out_norms
         self.w_in = None     # [left inputs | zero rows up to a multiple of 8 | right inputs, hidden], when one GEMM serves both
+        self.b_in = None     # its biases, where a half has them
         self.split = 0       # rows of w_in before the right half's
+        self.in_act = {}     # its activation: the right half's, on the last columns
 
     @property
     def cache_dim(self) -> int:
@@ -862,10 +867,19 @@ class ParallelMixer:
         else:
             self.w_o = torch.cat([self.left.w_o, self.right.w_o], 1).contiguous()
             self.left.w_o = self.right.w_o = None
-        if getattr(self.left, "takes_proj", False) and getattr(self.right, "takes_proj", False):
+        if all(getattr(m, "takes_proj", False) for m in (self.left, self.right)) and not hasattr(self.left, "in_act"):
             wl, wr = self.left.w_in, self.right.w_in
+            bl, br = getattr(self.left, "b_in", None), getattr(self.right, "b_in", None)
             self.split = -(-wl.shape[0] // 8) * 8   # 16-byte aligned rows in bf16
             self.w_in = torch.cat([F.pad(wl, (0, 0, 0, self.split - wl.shape[0])), wr], 0).contiguous()
+            if bl is not None or br is not None:
+                self.b_in = wl.new_zeros(self.w_in.shape[0])
+                for at, b in ((0, bl), (self.split, br)):
+                    if b is not None:
+                        self.b_in[at:at + b.shape[0]] = b
+            if hasattr(self.right, "in_act"):
+                act, first = self.right.in_act
+                self.in_act = dict(act=act, act_from=self.split + first)
             self.left.w_in = self.right.w_in = None
 
     def init_random(self, gen, std: float):
@@ -878,7 +892,7 @@ class ParallelMixer:
     def _forward_normed(self, h, meta, cache, state):
         pl = pr = None
         if self.w_in is not None:
-            proj = self.ops.linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)
             pl, pr = proj[:, :self.split], proj[:, self.split:]
         ys = []
         for m, p in ((self.left, pl), (self.right, pr)):
@@ -893,7 +907,7 @@ class ParallelMixer:
         a, b = self.left.out_size, self.right.out_size
         buf = torch.empty(h.shape[0], a + b, device=h.device, dtype=h.dtype)
         if self.w_in is not None:
-            proj = self.ops.linear(h, self.w_in)
+            proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)
             self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale, proj[:, :self.split])
             self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale, proj[:, self.split:])
             return _last(self, buf, self.w_o, None, update)
