@@ -195,6 +195,8 @@ struct PwGroup {
   // PW_EPI_CGLU (gather form): products of slot row s times row_scale[gather_slots[s]] (null: 1), clamped at limit
   const float* row_scale = nullptr;
   float limit = 0.f;
+  // the order the m-tiles are taken in, as place << 16 | expert << 8 | rows - 1 (moe_table_align's order; null: as they lie, all rows)
+  const int* order = nullptr;
 };
 bool launch_prefill_gemm_packed(int epi, void* C, long ldc, const void* X, long ldx, const void* Wp, int M, int N,
                                 int K, const void* bias, int wm, int grid_req, hipStream_t s,
@@ -265,11 +267,17 @@ void launch_moe_topk_softmax(const void* logits, bool logits_f32, float* w, int*
                              bool renorm, hipStream_t s, int splits = 0);
 void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
                       int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist);
+// Orders of the tiles for GEMMs that take per_round[j] of them at once (one table): to [rows, tiles] int32, place << 16 | expert << 8 | pairs - 1
+struct MoeOrder {
+  int* to = nullptr;
+  int rows = 0;
+  int per_round[2] = {1, 1};
+};
 // the same for the pairs (t, j), expert table[i][tokens[t]][j] of `tables` tables [table_rows, top], outputs side by side (num_tiles
 // [tables]): a workgroup each, or many for a large step of one table (hist as below)
 void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
                             int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot,
-                            int* hist, hipStream_t s);
+                            int* hist, const MoeOrder& order, hipStream_t s);
 // Workgroups of moe_align for npairs. More than one need hist, int32 [moe_align_blocks(npairs) * 128] scratch (of one table; else it is not
 // looked at). The number does not grow with npairs (65536: 64, 65537: 17): it is asked for at every call.
 int moe_align_blocks(int npairs);

@@ -63,11 +63,30 @@ HS_DEVICE void pw_tile(int L, int tiles_m, int tiles_n, int& tm, int& tn) {
   tn = r / gsz;
 }
 
-// Tiles of `total` that are taken by a workgroup each when `ncu` of them run at once: all, or whole rounds where the quarters of the
-// tiles left over fit one round.
-HS_DEVICE int pw_whole(int total, int ncu) {
-  const int left = total % ncu;
-  return 4 * left <= ncu ? total - left : total;
+// The m-tile that is taken tm-th: its place, its expert, its rows. One load either way: it stands before every tile's first one.
+// readfirstlane: a load through a generic pointer counts as divergent, which put the weight descriptor in VGPRs and wrapped every weight load of
+// the main loop in a waterfall loop (197 VALU instructions per loop body vs 0)
+struct PwPlace { int place, expert, rows; };
+HS_DEVICE PwPlace pw_place(const PwGroup& grp, int tm, int tile_rows) {
+  const int* from = grp.order != nullptr ? grp.order : grp.tile_expert;
+  const int v = __builtin_amdgcn_readfirstlane(from[tm]);
+  if (grp.order == nullptr) return {tm, v, tile_rows};
+  return {v >> 16, v >> 8 & 255, (v & 255) + 1};
+}
+
+// What whole rounds of `ncu` tiles leave over, and how it is taken: as one more round (24 us per 1024 of K), by quarters (pw_tail, 9 + 12.5 us per 1024) or by
+// columns (pw_few: each round of theirs 3 us and, per 1024, 3 us for up to 32 rows, 5 for 64, 8 for 128, beside the latency of the first).
+enum PwRest { kRestRound, kRestQuarters, kRestColumns };
+HS_DEVICE PwRest pw_rest(int left, int tiles_m, int tiles_n, int ncu, int K, const PwGroup& grp) {
+  if (left == 0) return kRestRound;
+  const int rounds = (16 * left + ncu - 1) / ncu;
+  if (rounds <= 1) return kRestColumns;
+  if (rounds <= 3) {
+    // the most rows that one of them has: the first m-tile's of the group that the first of them lies in
+    const int rows = pw_place(grp, (tiles_m * tiles_n - left) / (PW_GM * tiles_n) * PW_GM, 128).rows;
+    if (rounds <= (rows <= 32 ? 3 : rows <= 64 || K < 1536 ? 2 : 1)) return kRestColumns;
+  }
+  return 4 * left <= ncu && K >= 1536 ? kRestQuarters : kRestRound;
 }
 
 HS_DEVICE void pw_barrier() {
@@ -98,13 +117,14 @@ HS_DEVICE PwTile pw_make(int L, int tiles_m, int tiles_n, int wn, const unsigned
   int tm, tn;
   pw_tile(L, tiles_m, tiles_n, tm, tn);
   PwTile T;
+  if constexpr (kGroup) {
+    const PwPlace p = pw_place(grp, tm, BM);
+    tm = p.place;
+    Wp += (long)p.expert * grp.estride;
+  }
   T.m0 = tm * BM;
   T.t = tn * WN + wn;
   const int tl = min(T.t, ntiles - 1);  // waves past the last weight tile compute a copy, store nothing
-  // this m-tile's expert. readfirstlane: a load through a generic pointer counts as
-  // divergent, which put the weight descriptor in VGPRs and wrapped every weight load of
-  // the main loop in a waterfall loop (197 VALU instructions per loop body vs 0)
-  if constexpr (kGroup) Wp += (long)__builtin_amdgcn_readfirstlane(grp.tile_expert[tm]) * grp.estride;
   T.w = __builtin_amdgcn_make_buffer_rsrc((void*)(Wp + (long)tl * KS * 32768), 0, KS * 65536, 0x00020000);
   if constexpr (kGather) {  // token rows through the slot table; padding slots read past the end = zero
     const int bytes = (int)((long)grp.x_rows * ldx * 2);
@@ -126,15 +146,15 @@ HS_DEVICE PwTile pw_make(int L, int tiles_m, int tiles_n, int wn, const unsigned
 
 // Stores a wave's 128 x 128 block, weight tile t: this lane's columns 16 rg + 4 fq .. + 3 of rows mb + 16 i. own >= 0: the row groups
 // own and own + 4 alone (a gate and its up projection lie four groups apart).
-template <int EPI>
-HS_DEVICE void pw_epilogue(f32x4 (&acc)[8][8], int own, int t, int mb, int fq, int ntiles, unsigned short* __restrict__ C, long ldc,
+template <int EPI, int NI = 8, int STEP = 16>   // rows mb + STEP * i, i < NI
+HS_DEVICE void pw_epilogue(f32x4 (&acc)[8][NI], int own, int t, int mb, int fq, int ntiles, unsigned short* __restrict__ C, long ldc,
                            int M, int N, const unsigned short* __restrict__ bias, const PwGroup& grp) {
   if (t >= ntiles) return;
   if constexpr (EPI == PW_EPI_GLU || EPI == PW_EPI_GEGLU || EPI == PW_EPI_CGLU) {
     const int I = N >> 1;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int m = mb + 16 * i;
+    for (int i = 0; i < NI; ++i) {
+      const int m = mb + STEP * i;
       if (m >= M) continue;
       float rs = 1.f;
       if constexpr (EPI == PW_EPI_CGLU) {
@@ -173,8 +193,8 @@ HS_DEVICE void pw_epilogue(f32x4 (&acc)[8][8], int own, int t, int mb, int fq, i
 #pragma unroll
         for (int j = 0; j < 4; ++j) bv[j] = n + j < N ? bf16_to_f32(bias[n + j]) : 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int m = mb + 16 * i;
+      for (int i = 0; i < NI; ++i) {
+        const int m = mb + STEP * i;
         if (m >= M) continue;
         uint2* dst = reinterpret_cast<uint2*>(C + (long)m * ldc + n);
         float o[4];
@@ -206,7 +226,7 @@ HS_DEVICE void pw_epilogue(f32x4 (&acc)[8][8], int own, int t, int mb, int fq, i
 // barriers; loads a 64-deep stage ahead), and the waves' sums meet in LDS, in the order of K. A stage is bound by what a compute unit
 // takes in (X and weights 1 : 1 instead of 1 : 4: 40 KB per us), so that a quarter costs about 9 + 12.5 us per 1024 of K where
 // the round that it replaces costs 24 us per 1024, as it has the memory to itself: nothing is gained below K = 1536 (1024: 24 -> 22 us),
-// and two rounds of quarters never pay. Whole rounds alone -> with quarters, 8 experts: 1024 x 2048, 260 tiles 102 -> 80 us; 2048 x 4096, 520
+// and two rounds of quarters never pay; few tiles go by columns instead (pw_rest). Whole rounds alone -> with quarters, 8 experts: 1024 x 2048, 260 tiles 102 -> 80 us; 2048 x 4096, 520
 // tiles 290 -> 247; 4096 x 2048, 560 tiles 160 -> 141. The quarters follow in the launch of the whole rounds: one of its own, which has to come
 // whatever the device's counts are, cost 2 - 3 us of products that leave nothing over (1024 x 2048, 400 tiles: 114, 117 with it, 114 now).
 constexpr int PW_TAIL_LDS = 4 * 2 * 128 * 128;   // [wave][2][128 rows of 128 bytes], then the sums [owner][other][8 KB]
@@ -229,9 +249,10 @@ HS_DEVICE void pw_tail(unsigned char* lds, int r, const unsigned short* __restri
   for (int u = r; u < units; u += gridDim.x) {
     int tm, tn;
     pw_tile(whole + (u >> 2), tiles_m, tiles_n, tm, tn);
-    const int m0 = tm * 128, t = 4 * tn + (u & 3);
+    const PwPlace p = pw_place(grp, tm, 128);
+    const int m0 = p.place * 128, t = 4 * tn + (u & 3);
     if (t >= ntiles) continue;
-    const unsigned short* wp = Wp + (long)__builtin_amdgcn_readfirstlane(grp.tile_expert[tm]) * grp.estride + (long)t * KS * 32768;
+    const unsigned short* wp = Wp + (long)p.expert * grp.estride + (long)t * KS * 32768;
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)wp, 0, KS * 65536, 0x00020000);
     // rows that do not exist lie past the buffer and read as zero (pw_make)
     const int bytes = kGather ? (int)((long)grp.x_rows * ldx * 2) : (int)((long)min(128, M - m0) * ldx * 2);
@@ -323,6 +344,129 @@ HS_DEVICE void pw_tail(unsigned char* lds, int r, const unsigned short* __restri
     }
     pw_epilogue<EPI>(acc, wave, t, m0 + fr, fq, ntiles, C, ldc, M, N, nullptr, grp);
     __syncthreads();   // the sums are read before the next unit's rows come
+  }
+}
+
+// The same by columns: a workgroup takes 32 columns (row groups own and own + 4 of a weight tile), its waves a quarter of K each with rows of their own in LDS,
+// and of the rows the 16 RI that there are. Four times as many workgroups as by quarters, each of which takes in 8 KB per 64-deep stage and 32 rows (40 of
+// 128) for 128; what bounds it is the latency of a unit's first loads (its place, its slots, its rows) and then the intake, some 40 KB per us. With
+// the order that leaves the tiles of few rows for last (order_tiles), one round of columns is 11 - 15 us, of quarters 25 - 35, a whole round 24 per 1024
+// of K. Up and down of 16384 pairs, whole rounds and quarters -> with these: 16 experts of 1024 x 2048 84.7 -> 76.0, 89.8 -> 77.2 us, 8 of 2048 x 4096 243 ->
+// 222, 256 -> 248; 12000 pairs, down, 190 -> 181; 2048 pairs of 512 x 1024 31 -> 22.
+template <int EPI, bool kGather, int RI>
+HS_DEVICE void pw_few_unit(unsigned char* lds, const unsigned short* __restrict__ X, long ldx, const unsigned short* __restrict__ wp,
+                           unsigned short* __restrict__ C, long ldc, int M, int N, int K, int t, int own, int m0, int rows, const PwGroup& grp) {
+  constexpr int BUF = 128 * 128, XP = 2 * RI, PD = RI == 2 ? 4 : 2;   // PD: stages in flight
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ntiles = (N + 127) >> 7, KS = K >> 8;
+  const int nst = K >> 8, q0 = wave * 2 * nst;
+  const int fr = lane & 15, fq = lane >> 4, sw = (fr >> 1) & 7;
+  const int foff = wave * 2 * BUF + fr * 128;
+  const int ch[2] = {(fq ^ sw) * 16, ((4 + fq) ^ sw) * 16};
+  const int xd = wave * 2 * BUF + (lane >> 3) * 128;
+  const int xdo[2] = {xd + (((lane & 7) ^ (lane >> 4)) * 16), xd + (((lane & 7) ^ (4 + (lane >> 4))) * 16)};
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)wp, 0, KS * 65536, 0x00020000);
+  // rows that do not exist lie past the buffer and read as zero (pw_make)
+  const int bytes = kGather ? (int)((long)grp.x_rows * ldx * 2) : (int)((long)min(rows, M - m0) * ldx * 2);
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)(kGather ? X : X + (long)m0 * ldx), 0, bytes, 0x00020000);
+  int xo[XP];
+#pragma unroll
+  for (int p = 0; p < XP; ++p) {
+    const int r = 8 * p + (lane >> 3);
+    if constexpr (kGather) {
+      const int s = m0 + r < M ? grp.gather_slots[m0 + r] : -1;
+      xo[p] = (s >= 0 ? (s / grp.gather_k) * (int)ldx * 2 : bytes) + (lane & 7) * 16;
+    } else {
+      xo[p] = r * (int)ldx * 2 + (lane & 7) * 16;
+    }
+  }
+  u32x4 xst[PD][XP], w[PD][2][2];   // [stage][half][row group]
+  f32x4 acc[2][RI];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int i = 0; i < RI; ++i) acc[g][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto wload = [&](int st, u32x4 (&to)[2][2]) {
+    const int q = q0 + 2 * st;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+        to[h][g] = __builtin_amdgcn_raw_buffer_load_b128(wr, lane * 16, ((q + h) >> 3) * 65536 + (own + 4 * g) * 8192 + ((q + h) & 7) * 1024, 0);
+  };
+  auto xload = [&](int st, u32x4 (&to)[XP]) {
+#pragma unroll
+    for (int p = 0; p < XP; ++p) to[p] = __builtin_amdgcn_raw_buffer_load_b128(xr, xo[p], q0 * 64 + st * 128, 0);
+  };
+#pragma unroll
+  for (int j = 0; j < PD; ++j) {
+    xload(min(j, nst - 1), xst[j]);
+    wload(min(j, nst - 1), w[j]);
+  }
+  for (int s0 = 0; s0 < nst; s0 += PD) {
+#pragma unroll
+    for (int j = 0; j < PD; ++j) {
+      if (s0 + j >= nst) break;
+      const int next = min(s0 + j + PD, nst - 1);
+#pragma unroll
+      for (int p = 0; p < XP; ++p) *reinterpret_cast<u32x4*>(lds + (j & 1) * BUF + p * 1024 + xdo[p & 1]) = xst[j][p];
+      xload(next, xst[j]);
+      u32x4 x[2][RI];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < RI; ++i) x[h][i] = *reinterpret_cast<const u32x4*>(lds + (j & 1) * BUF + foff + i * 2048 + ch[h]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+          for (int i = 0; i < RI; ++i)
+            acc[g][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[j][h][g]), __builtin_bit_cast(bf16x8, x[h][i]), acc[g][i], 0, 0, 0);
+      wload(next, w[j]);
+    }
+  }
+  // wave v ends with the row groups of X v, v + 4, ..: the others' parts through LDS, added in the order of K
+  f32x4* sums = reinterpret_cast<f32x4*>(lds);   // [wave][2][RI][64 lanes]
+  __syncthreads();
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int i = 0; i < RI; ++i) sums[((wave * 2 + g) * RI + i) * 64 + lane] = acc[g][i];
+  __syncthreads();
+  constexpr int NI = (RI + 3) / 4;
+  f32x4 all[8][NI];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int o = 0; o < 4; ++o) a += sums[((o * 2 + g) * RI + min(wave + 4 * i, RI - 1)) * 64 + lane];
+#pragma unroll
+      for (int rg = 0; rg < 4; ++rg) all[4 * g + rg][i] = a;
+    }
+  if (wave < RI) pw_epilogue<EPI, NI, 64>(all, own, t, m0 + 16 * wave + fr, fq, ntiles, C, ldc, M, N, nullptr, grp);
+  __syncthreads();   // the sums are read before the next unit's rows come
+}
+
+template <int EPI, bool kGather>
+HS_DEVICE void pw_few(unsigned char* lds, int r, const unsigned short* __restrict__ X, long ldx, const unsigned short* __restrict__ Wp,
+                      unsigned short* __restrict__ C, long ldc, int M, int N, int K, int tiles_m, int tiles_n, const PwGroup& grp, int whole) {
+  const int ntiles = (N + 127) >> 7, units = 16 * (tiles_m * tiles_n - whole);
+  for (int u = r; u < units; u += gridDim.x) {
+    int tm, tn;
+    pw_tile(whole + (u >> 4), tiles_m, tiles_n, tm, tn);
+    const PwPlace p = pw_place(grp, tm, 128);
+    const int t = 4 * tn + (u >> 2 & 3);
+    if (t >= ntiles) continue;
+    const unsigned short* wp = Wp + (long)p.expert * grp.estride + (long)t * (K >> 8) * 32768;
+#define PW_FEW(RI) pw_few_unit<EPI, kGather, RI>(lds, X, ldx, wp, C, ldc, M, N, K, t, u & 3, p.place * 128, p.rows, grp)
+    if (p.rows <= 32) PW_FEW(2);
+    else if (p.rows <= 64) PW_FEW(4);
+    else PW_FEW(8);
+#undef PW_FEW
   }
 }
 
@@ -475,7 +619,7 @@ HS_DEVICE void pw_tiles(unsigned char* lds, int r, int G, int total, const unsig
 // (moe_align with tile BM, moe_gather); m-tile tm multiplies expert grp.tile_expert[tm]'s
 // packed weight (Wp + e * estride) and only the first *grp.num_tiles m-tiles (the
 // device-side count: no host round trip, graph-capturable) are walked. TAIL: whole rounds of
-// `ncu` tiles, then what they leave over (pw_whole, pw_tail).
+// `ncu` tiles, then what they leave over (pw_rest).
 template <int WM, int EPI, bool kGroup, int RW, bool LDLY = false, bool kGather = false, bool TAIL = false>
 __global__ __launch_bounds__(PW_T) __attribute__((amdgpu_waves_per_eu(1, 1))) void pgw_kernel(
     const unsigned short* __restrict__ X, long ldx, const unsigned short* __restrict__ Wp,
@@ -486,12 +630,20 @@ __global__ __launch_bounds__(PW_T) __attribute__((amdgpu_waves_per_eu(1, 1))) vo
   // TAIL: of the grid, as many as there can be whole tiles for, which the XCDs share evenly that way
   const int G = TAIL ? min((int)gridDim.x, tiles_m * tiles_n) : gridDim.x;
   if constexpr (kGroup) tiles_m = min(tiles_m, __builtin_amdgcn_readfirstlane(*grp.num_tiles));
-  const int total = TAIL ? pw_whole(tiles_m * tiles_n, ncu) : tiles_m * tiles_n;
+  int total = tiles_m * tiles_n;
+  [[maybe_unused]] PwRest rest = kRestRound;
+  if constexpr (TAIL) {
+    const int left = total % ncu;
+    rest = pw_rest(left, tiles_m, tiles_n, ncu, K, grp);
+    if (rest != kRestRound) total -= left;
+  }
   const int r = (int)blockIdx.x < G ? xcd_remap(blockIdx.x, G) : total;
   pw_tiles<WM, EPI, kGroup, RW, LDLY, kGather>(lds, r, G, total, X, ldx, Wp, C, ldc, M, N, K, tiles_m, tiles_n, bias, grp);
   if constexpr (TAIL) {
     __syncthreads();   // the last tile's rows are read
-    pw_tail<EPI, kGather>(lds, xcd_remap(blockIdx.x, gridDim.x), X, ldx, Wp, C, ldc, M, N, K, tiles_m, tiles_n, grp, total);
+    const int u = xcd_remap(blockIdx.x, gridDim.x);
+    if (rest == kRestColumns) pw_few<EPI, kGather>(lds, u, X, ldx, Wp, C, ldc, M, N, K, tiles_m, tiles_n, grp, total);
+    else if (rest == kRestQuarters) pw_tail<EPI, kGather>(lds, u, X, ldx, Wp, C, ldc, M, N, K, tiles_m, tiles_n, grp, total);
   }
 }
 
@@ -546,8 +698,8 @@ bool launch_prefill_gemm_packed(int epi, void* C, long ldc, const void* X, long 
     else                                                                                                     \
       pgw_kernel<WM_, E_, false, 4, true><<<grid, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu); \
   } while (0)
-  if (grouped && wm == 1 && grid_req <= 0 && K >= 1536) {
-    const dim3 tg(std::min(4 * total, ncu));   // fewer tiles than compute units may come in quarters
+  if (grouped && wm == 1 && grid_req <= 0) {
+    const dim3 tg(std::min(16L * total, (long)ncu));   // fewer tiles than compute units may come in parts
 #define PW_TAIL(E_)                                                                                                                  \
   do {                                                                                                                               \
     if (gather) pgw_kernel<1, E_, true, 4, false, true, true><<<tg, PW_T, 0, s>>>(x, ldx, w, c, ldc, M, N, K, tiles_m, tiles_n, b, grp, ncu); \

@@ -835,7 +835,7 @@ void prefill_gemm_packed(at::Tensor& out, const at::Tensor& x, const at::Tensor&
 void prefill_gemm_packed_grouped(at::Tensor& out, const at::Tensor& x, const at::Tensor& wp, int64_t N, int64_t epi,
                                  const at::Tensor& tile_expert, const at::Tensor& num_tiles, int64_t wm, int64_t rw,
                                  const c10::optional<at::Tensor>& gather_slots, int64_t gather_k,
-                                 const c10::optional<at::Tensor>& row_scale, double limit) {
+                                 const c10::optional<at::Tensor>& row_scale, double limit, const c10::optional<at::Tensor>& order) {
   CHECK_DEV(x); CHECK_BF16(x); CHECK_BF16(wp); CHECK_BF16(out); CHECK_ROWMAJOR(x); CHECK_ROWMAJOR(out);
   TORCH_CHECK(wp.dim() == 2 && wp.is_contiguous(), "prefill_gemm_packed_grouped: wp [E, packed]");
   // gather: x holds the token rows and slot row s reads x[gather_slots[s] / gather_k] (moe_align's slots)
@@ -858,6 +858,11 @@ void prefill_gemm_packed_grouped(at::Tensor& out, const at::Tensor& x, const at:
   TORCH_CHECK(out.size(0) == M && out.size(1) == (glu ? N / 2 : N), "prefill_gemm_packed_grouped: out shape");
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   hipserve::PwGroup grp{tile_expert.data_ptr<int>(), num_tiles.data_ptr<int>(), (long)wp.size(1)};
+  if (order.has_value()) {
+    TORCH_CHECK(order->is_cuda() && order->device() == x.device() && order->scalar_type() == at::kInt && order->is_contiguous() &&
+                    order->numel() >= M / (128 * wm), "prefill_gemm_packed_grouped: an order of the tiles");
+    grp.order = order->data_ptr<int>();
+  }
   if (gather) {
     grp.gather_slots = gather_slots->data_ptr<int>();
     grp.gather_k = (int)gather_k;
@@ -1345,7 +1350,7 @@ TORCH_LIBRARY(hipserve, m) {
   m.def("decode_gemm_partial(Tensor(a!) ws, Tensor x, Tensor w, int N, int rt, int splits, bool packed) -> ()");
   m.def("decode_gemm_glu(Tensor(a!) act, Tensor x, Tensor wp, Tensor(b!) ws, int N, int rt, int splits) -> ()");
   m.def("prefill_gemm_packed(Tensor(a!) out, Tensor x, Tensor wp, int N, int epi, Tensor? bias=None, int wm=1, int grid=0, int rw=4) -> ()");
-  m.def("prefill_gemm_packed_grouped(Tensor(a!) out, Tensor x, Tensor wp, int N, int epi, Tensor tile_expert, Tensor num_tiles, int wm=1, int rw=4, Tensor? gather_slots=None, int gather_k=1, Tensor? row_scale=None, float limit=0.0) -> ()");
+  m.def("prefill_gemm_packed_grouped(Tensor(a!) out, Tensor x, Tensor wp, int N, int epi, Tensor tile_expert, Tensor num_tiles, int wm=1, int rw=4, Tensor? gather_slots=None, int gather_k=1, Tensor? row_scale=None, float limit=0.0, Tensor? order=None) -> ()");
   m.def("prefill_gemm_f8(Tensor(a!) out, Tensor xq, Tensor xs, Tensor[] q, Tensor[] rs, int epi) -> ()");
   m.def("fp8_decode_gemm(Tensor(a!) ws, Tensor xq, Tensor xs, Tensor[] q, Tensor[] rs, int splits) -> ()");
   m.def("glu_quant(Tensor(a!)? out, Tensor(b!) q8, Tensor(c!) xs, Tensor x, bool gelu) -> ()");

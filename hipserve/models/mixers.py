@@ -392,15 +392,19 @@ class TableMoE:
         tile_expert = torch.empty(cap // tile, dtype=torch.int32, device=dev)
         ntiles = torch.empty(1, dtype=torch.int32, device=dev)
         pair_slot = torch.empty(P, dtype=torch.int32, device=dev)
+        orders = (None, None)
         if self.ops.moe_tables_align_ok(self.table, ids, E):
-            self.ops.moe_table_align(self.table, ids, E, tile, slots, tile_expert, pair_slot, ntiles)
+            # a round of either product: 512 columns (tile 256: 256) of so many tiles as there are compute units for
+            cus, cols = torch.cuda.get_device_properties(dev).multi_processor_count, 512 // gemm.PW_WM
+            orders = torch.empty(2, cap // tile, dtype=torch.int32, device=dev)
+            self.ops.moe_table_align(self.table, ids, E, tile, slots, tile_expert, pair_slot, ntiles, orders, [max(1, cus // -(-n // cols)) for n in (ff, H)])
         else:
             op.moe_align(self.table.index_select(0, ids).reshape(-1), E, tile, slots, tile_expert, ntiles, pair_slot, None)
         pu, pd = self.packed
         act = torch.empty(cap, ff, dtype=h.dtype, device=dev)
-        op.prefill_gemm_packed_grouped(act, h, pu, ff, 4, tile_expert, ntiles, gemm.PW_WM, gemm.PW_RW, slots, s.top)
+        op.prefill_gemm_packed_grouped(act, h, pu, ff, 4, tile_expert, ntiles, gemm.PW_WM, gemm.PW_RW, slots, s.top, order=orders[0])
         y = torch.empty(cap, H, dtype=h.dtype, device=dev)
-        op.prefill_gemm_packed_grouped(y, act, pd, H, 0, tile_expert, ntiles, gemm.PW_WM, gemm.PW_RW)
+        op.prefill_gemm_packed_grouped(y, act, pd, H, 0, tile_expert, ntiles, gemm.PW_WM, gemm.PW_RW, order=orders[1])
         return y, pair_slot
 
 

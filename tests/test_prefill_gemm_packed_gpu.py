@@ -237,3 +237,53 @@ def test_packed_grouped_in_one_launch(tiles, counted, N, tmp_path):
     want = torch.cat([x[t * 128:(t + 1) * 128].double() @ w[int(tile_expert[t])].double().t() for t in range(counted)] + [x.new_zeros(0, N).double()])
     # sums of K products in 32 bits and the result's rounding
     assert ((got[:rows].double() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -9 * K ** 0.5 * 0.05).all()
+
+
+@pytest.mark.parametrize("counts,N,K,epi", [([5, 200, 64], 512, 256, 0), ([128, 33, 0, 17], 1024, 512, 4), ([129, 97, 1], 640, 768, 2),
+                                            ([30] * 16 + [1000, 4096], 2048, 1024, 0), ([128 * 16 + 40, 128 * 15 + 31, 128], 4096, 1536, 4)])
+@pytest.mark.parametrize("gather", [False, True])
+def test_packed_grouped_by_order(counts, N, K, epi, gather):
+    """Tiles in the order that the alignment leaves for rounds of them, what they leave over by columns: one to 128 rows, a weight tile cut off, fewer stages
+    than are in flight, as whole rounds and as the only ones; K too short for quarters."""
+    from hipserve.ops import get_ops
+
+    g, op, E, k = torch.Generator(device=DEV).manual_seed(len(counts) + N), torch.ops.hipserve, len(counts), 2
+    P = -(-sum(counts) // k) * k
+    ids = torch.repeat_interleave(torch.arange(E, device=DEV), torch.tensor(counts, device=DEV))
+    ids = torch.cat([ids, ids.new_full((P - len(ids),), E - 1)])[torch.randperm(P, device=DEV, generator=g)].int()
+    cnt = torch.bincount(ids, minlength=E)
+    cap = -(-(P + E * 127) // 128) * 128
+    table, tokens = ids.view(-1, 1).contiguous(), torch.arange(P, device=DEV)   # a token per pair
+    slots, te, nt, ps = (torch.empty(n, dtype=torch.int32, device=DEV) for n in (cap, cap // 128, 1, P))
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    per_round = [max(1, cus // -(-N // 512)), 3]
+    orders = torch.full((2, cap // 128), -1, dtype=torch.int32, device=DEV)
+    get_ops("cuda").moe_table_align(table, tokens, E, 128, slots, te, ps, nt, orders, per_round)
+    n, rows = int(nt), (slots.view(-1, 128) >= 0).sum(1).cpu()
+    for o, r in zip(orders[:, :n].cpu(), per_round):
+        place = o >> 16
+        assert torch.equal(place.sort().values, torch.arange(n)) and torch.equal(te.cpu()[place.long()], o >> 8 & 255)
+        assert torch.equal(rows[place.long()], (o & 255).long() + 1)
+        left = n % r if 16 * (n % r) <= 3 * r else 0
+        few = sorted(x for x in rows[:n].tolist() if x < 128)[:left]
+        assert rows[place.long()][n - len(few):].tolist() == few
+        assert torch.equal(place[:n - len(few)], place[:n - len(few)].sort().values)   # the others as they lie
+    assert torch.equal(cnt.cpu(), torch.bincount(torch.repeat_interleave(te[:n].cpu().long(), rows[:n]), minlength=E))
+    w, x = _rnd(g, E, N, K, scale=0.05), _rnd(g, P, K)
+    wp = torch.stack([_pack(w[e], epi == 2) for e in range(E)])
+    No = N // 2 if epi == 2 else N
+    xs = torch.full((cap, K), float("nan"), device=DEV, dtype=torch.bfloat16)   # rows of no pair may hold anything
+    xs[ps.long()] = x
+    out = torch.full((cap, No), 7.0, device=DEV, dtype=torch.bfloat16)
+    if gather:
+        op.prefill_gemm_packed_grouped(out, x, wp, N, epi, te, nt, 1, 4, slots, 1, order=orders[0])
+    else:
+        op.prefill_gemm_packed_grouped(out, xs, wp, N, epi, te, nt, 1, order=orders[0])
+    assert bool((out[n * 128:] == 7.0).all())
+    got = out[ps.long()]
+    for e in range(E):
+        mine = (ids == e).nonzero()[:, 0]
+        h = x[mine].double() @ w[e].double().t()
+        want = h.clamp(min=0).square() if epi == 4 else torch.nn.functional.silu(h[:, :No]) * h[:, No:] if epi == 2 else h
+        rel = 2.0 ** -6 if epi == 2 else 2.0 ** -7   # as above
+        assert len(mine) == 0 or ((got[mine].double() - want).abs() <= rel * want.abs() + 2.0 ** -9 * want.abs().mean()).all()
