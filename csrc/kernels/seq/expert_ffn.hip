@@ -191,6 +191,110 @@ __global__ __launch_bounds__(256) void expert_gemm_mfma_kernel(
   }
 }
 
+// bf16, tiles of 128 slots (prompts of some dozen to a few thousand rows): a workgroup of four waves computes a tile's live rows (32, 64, 96 or 128 of them)
+// x 64 columns, a wave 16 columns of all rows. Rows and weights are copied to LDS as in skinny.h, stages of 64 k, two ahead, one barrier each. What
+// bounds it is what a compute unit takes in, 40 - 50 KB per us: an expert's weights once per 128 rows instead of once per 32, its rows once per
+// 64 columns instead of once per 16. 72 KB of LDS, so that two workgroups fit a compute unit: with three or five stages ahead and one workgroup 54 and 55 us
+// where this takes 43 (16 experts, 4000 pairs, 1024 x 2048), nowhere less than 2 % faster. us of both products by tiles of 32 (expert_rows; packed weights) ->
+// this, 16 experts of 1024 x 2048: 200 pairs 32.8 -> 28.9, 600 47.6 -> 31.6, 1400 76 -> 39, 4000 167 (96) -> 82; 8 of 2048 x 4096: 600 pairs 128 -> 69, 2000 303
+// -> 145 (2000 pairs; packed 165); 8 of 512 x 1024: 1400 24.1 (24.4) -> 19.7, 4000 59 (55) -> 27.6.
+constexpr int kMidRows = 128, kMidCols = 64, kMidStages = 3, kMidLds = kMidStages * (kMidRows + kMidCols) * 128;
+template <int RT>
+HS_DEVICE void expert_mid(unsigned short* __restrict__ out, const unsigned short* __restrict__ x, unsigned x_ld, const unsigned char* __restrict__ we,
+                          const int (&mine)[2], int slot0, int n0, int gather_k, int gather_shift, int N, int K, int act, unsigned char* smem) {
+  constexpr int D = kMidStages, kX = RT * 2048, kStage = kX + kMidCols * 128, XC = RT / 2, kCopies = XC + 2;   // XC: copies of a wave's rows per stage
+  static_assert(RT % 2 == 0 && kCopies * (D - 2) < 64, "copies that a wait can count");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4, r8 = lane >> 3;
+  const unsigned lds0 = lds_at(smem);
+  unsigned x_at[XC], w_at[2];
+  auto part = [&](int row) { return 16u * ((lane & 7) ^ (row >> 1 & 7)); };
+  auto pair_of = [&](int r) {   // every lane asks
+    const int a = __shfl(mine[0], r & 63, 64), b = __shfl(mine[1], r & 63, 64);
+    return r < 64 ? a : b;
+  };
+#pragma unroll
+  for (int j = 0; j < XC; ++j) {
+    const int r = 8 * (wave * XC + j) + r8, p = pair_of(r);
+    const int from = gather_shift >= 0 ? p >> gather_shift : gather_k > 0 ? p / gather_k : slot0 + r;
+    x_at[j] = (unsigned)(p < 0 ? 0 : from) * x_ld * 2 + part(r);   // no pair: any row
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int r = 8 * (2 * wave + j) + r8;
+    w_at[j] = (unsigned)min(r, N - 1 - n0) * (unsigned)K * 2 + part(r);
+  }
+  const unsigned char* xb = reinterpret_cast<const unsigned char*>(x);
+  const int nst = K >> 6;
+  auto copy = [&](int st) {
+    const unsigned to = lds0 + st % D * kStage;
+    const long k = 128L * st;
+#pragma unroll
+    for (int j = 0; j < XC; ++j) copy_1k(xb + k, x_at[j], to + (wave * XC + j) * 1024);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) copy_1k(we + k, w_at[j], to + kX + (2 * wave + j) * 1024);
+  };
+  f32x4 acc[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < D - 1; ++i)
+    if (i < nst) copy(i);
+  int at[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) at[s] = c * 128 + (((4 * s + g) ^ (c >> 1)) << 4);
+  for (int st = 0; st < nst; ++st) {
+    // the stage's copies are there, every wave's; and every wave has read the stage before, whose place the next copies take
+    if (st + D - 1 <= nst) barrier_copies<kCopies * (D - 2)>();
+    else barrier_copies<0>();
+    if (st + D - 1 < nst) copy(st + D - 1);
+    const unsigned char* t = smem + st % D * kStage;
+    u16x8 a[2], b[2][RT];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      a[s] = *reinterpret_cast<const u16x8*>(t + kX + wave * 2048 + at[s]);
+#pragma unroll
+      for (int i = 0; i < RT; ++i) b[s][i] = *reinterpret_cast<const u16x8*>(t + i * 2048 + at[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[s]), __builtin_bit_cast(bf16x8, b[s][i]), acc[i], 0, 0, 0);
+  }
+  // lane (c, g): columns n0 + 16 wave + 4 g .. + 3 of slot 16 i + c
+  const int n = n0 + 16 * wave + 4 * g;
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int r = 16 * i + c, p = pair_of(r);
+    if (p < 0 || n >= N) continue;   // N % 8 == 0: the four columns are inside together
+    u16x4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float v = acc[i][j];
+      if (act == 1) { v = fmaxf(v, 0.f); v *= v; }
+      o[j] = f32_to_bf16(v);
+    }
+    *reinterpret_cast<u16x4*>(out + (long)(slot0 + r) * N + n) = o;
+  }
+}
+
+__global__ __launch_bounds__(256) void expert_gemm_mid_kernel(
+    const int* __restrict__ slots, const int* __restrict__ tile_expert, const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
+    int x_ld, int N, int K, int E, int gather_k, int gather_shift, unsigned short* __restrict__ out, int act) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  const int lane = threadIdx.x & 63, slot0 = blockIdx.y * kMidRows, n0 = blockIdx.x * kMidCols;
+  const int e = tile_expert[blockIdx.y], mine[2] = {slots[slot0 + lane], slots[slot0 + 64 + lane]};
+  const int rows = __popcll(__ballot(mine[0] >= 0)) + __popcll(__ballot(mine[1] >= 0));   // moe_align fills a tile from its first slot on
+  if (e < 0 || e >= E) return;
+  const unsigned char* we = reinterpret_cast<const unsigned char*>(w + ((long)e * N + n0) * K);
+#define HS_EM(RT) expert_mid<RT>(out, x, x_ld, we, mine, slot0, n0, gather_k, gather_shift, N, K, act, smem)
+  if (rows <= 32) HS_EM(2);
+  else if (rows <= 64) HS_EM(4);
+  else if (rows <= 96) HS_EM(6);
+  else HS_EM(8);
+#undef HS_EM
+}
+
 template <int NT, bool GLU>
 __global__ __launch_bounds__(kSkThreads) void expert_gemm_skinny_kernel(
     const int* __restrict__ slots, const int* __restrict__ tile_expert, const unsigned short* __restrict__ x, const unsigned short* __restrict__ w,
@@ -226,6 +330,16 @@ void launch_expert_gemm(void* out, const void* x, long x_ld, const void* w, cons
   // the capacity covers a partly filled tile per expert
   pairs = pairs > 0 ? pairs : std::max(1, ntiles_cap * tile - E * (tile - 1));
   const int No = act >= 2 ? N / 2 : N;
+  if (!f32 && tile == kMidRows && act <= 1 && row_scale == nullptr && K % 64 == 0 && N % 8 == 0 && x_ld % 8 == 0 && K < (1 << 24) &&
+      2L * ntiles_cap * tile * x_ld < (1L << 32) && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0) {
+    const dim3 mg((N + kMidCols - 1) / kMidCols, ntiles);
+    const int shift = gather_k > 0 && (gather_k & (gather_k - 1)) == 0 ? __builtin_ctz(gather_k) : -1;
+    if (allow_lds(&expert_gemm_mid_kernel, kMidLds)) {
+      expert_gemm_mid_kernel<<<mg, 256, kMidLds, s>>>(slots, tile_expert, (const unsigned short*)x, (const unsigned short*)w, (int)x_ld, N, K, E, gather_k,
+                                                      shift, (unsigned short*)out, act);
+      return;
+    }
+  }
   if (!f32 && K % 8 == 0 && No % 8 == 0 && x_ld % 8 == 0 && (tile == 32 || tile == 64)) {
     dim3 mg(act >= 2 ? (No + 63) / 64 : (N + 127) / 128, ntiles);
     auto o = (unsigned short*)out;

@@ -82,6 +82,7 @@ from ..ops import ExpertSteps
 
 MOE_TILE = 32        # slots per expert tile of the expert GEMMs ...
 MOE_TILE_LARGE = 64  # ... when every expert has several tiles' worth of rows on average
+MOE_TILE_PROMPT = 128  # ... in bf16 prompts, where ``ops.expert_plan`` says so
 # bf16 batches with at least this many (token, expert) pairs per expert run the packed-layout grouped
 # GEMM of the dense families' MoE prefill (prefill_gemm_packed.hip: 128-row tiles, X through LDS, the
 # weights pre-shuffled into MFMA operand order) with the squared ReLU in its epilogue
@@ -296,6 +297,9 @@ class TableMoE:
         self.w_up = None    # [E, ff, hidden]
         self.w_down = None  # [E, hidden, ff]
         self.packed = None  # (up, down) in the packed grouped-GEMM layout, made at the first large batch
+        # pairs above which ``ops.expert_plan`` chooses the kernel: of bf16 prompts, k of 512 and more (shorter ones were not looked at)
+        known = (getattr(ops, "name", "") == "hip" and dtype == torch.bfloat16 and min(spec.ff, hidden) >= 512 and spec.ff % 64 == 0 and hidden % 64 == 0)
+        self.planned = ops.SKINNY_ROWS * spec.top if known else float("inf")
 
     def load(self, get, prefix: str):
         dt, dev, E = self.dtype, self.device, self.spec.experts
@@ -316,6 +320,8 @@ class TableMoE:
         """The tile of an expert GEMM over P pairs and empty (slots, tile_expert, pair_slot), a row per layer where they are given."""
         E = self.spec.experts
         tile = MOE_TILE_LARGE if P >= 4 * MOE_TILE_LARGE * E else MOE_TILE
+        if P > self.planned:   # not packed (``forward``)
+            tile = MOE_TILE_PROMPT if self.ops.expert_plan(P, E, self.spec.ff, self.hidden, False) == "tiles" else MOE_TILE
         cap = -(-(P + E * (tile - 1)) // tile) * tile
         return tile, [torch.empty(*layers, n, dtype=torch.int32, device=dev) for n in (cap, cap // tile, P)]
 
@@ -368,9 +374,9 @@ class TableMoE:
 
     def _packed_ok(self, h: torch.Tensor, P: int) -> bool:
         s = self.spec
-        return (getattr(self.ops, "name", "") == "hip" and h.dtype == torch.bfloat16 and s.experts <= 128
-                and self.hidden % 256 == 0 and s.ff % 256 == 0
-                and P >= MOE_PACKED_MIN_PAIRS_PER_EXPERT * s.experts and not torch.cuda.is_current_stream_capturing())
+        return (P >= MOE_PACKED_MIN_PAIRS_PER_EXPERT * s.experts and getattr(self.ops, "name", "") == "hip" and h.dtype == torch.bfloat16 and s.experts <= 128
+                and self.hidden % 256 == 0 and s.ff % 256 == 0 and not torch.cuda.is_current_stream_capturing()
+                and (P <= self.planned or self.ops.expert_plan(P, s.experts, s.ff, self.hidden, True) == "packed"))
 
     def _forward_packed(self, h: torch.Tensor, ids: torch.Tensor, P: int):
         """Large bf16 batches: the experts as two launches of the packed-layout grouped GEMM (token rows

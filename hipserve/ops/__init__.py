@@ -150,9 +150,9 @@ class KernelOps:
         self.norm_library = "seq"
         # the rules of products of a few rows: arithmetic on sizes, a few us each, and a step asks for every product. What they said of
         # the last sizes is kept (a step that is not captured, of four layers and a few rows, took 20 - 40 us longer)
-        self.skinny_pays, self.skinny_parts, self.update_pays, self.update_cols, self.mingru_pays = (
+        self.skinny_pays, self.skinny_parts, self.update_pays, self.update_cols, self.mingru_pays, self.expert_plan = (
             functools.lru_cache(maxsize=4096)(rule)
-            for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._update_cols, self._mingru_pays))
+            for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._update_cols, self._mingru_pays, self._expert_plan))
 
     @property
     def _op(self):
@@ -852,6 +852,34 @@ class KernelOps:
         ``pairs``: how many (token, choice) pairs the tiles hold, where the caller knows (the choice of kernel); ``tiles``: the tiles in use are
         among the first so many, as the alignments leave them with a pair in each (the rest is not launched)."""
         self._moe_lib.expert_gemm(out, x, w, slots, tile_expert, tile, gather_k, int(act), row_scale, limit, pairs, tiles)
+
+    def _expert_plan(self, pairs: int, experts: int, ff: int, hidden: int, may_pack: bool) -> str:
+        """How a prompt's two expert products, [ff, hidden] and back, are expected to be fastest in bf16: "rows" (tiles of 32, the kernel for few rows),
+        "tiles" (of 128; some pairs per expert, else most of their rows are empty) or, with ``may_pack``, "packed" (the grouped GEMM over packed weights), in us of a
+        model of each: a latency and the larger of the weights at 4.4 or 5.2 TB/s and what a compute unit takes in, per workgroup rows and columns times k; rounds of
+        512 columns x 128 rows for packed ones. 91 sizes (4 - 64 experts, 512 x 1024 to 2048 x 4096, 66 - 5600 tokens): the choice takes 1.1 % longer than the
+        fastest on average, at most 1 % longer than tiles of 32 and packed weights alone did. us rows / tiles / packed of both: 16 experts of 1024 x 2048, 87, 250,
+        350 pairs each 76 / 39 / -, 167 / 82 / 96, 222 / 100 / 97; 8 of 512 x 1024, 75, 175, 1000 each 13.6 / 15.9 / -, 24 / 20 / 24, 103 / 39 / 59."""
+        each = pairs / experts
+
+        def rows(n, k):
+            tiles, r = experts * max(1.0, each / 32 + 0.5), min(32.0, 8 * math.ceil(each / 8))
+            return 2.2 + max(2e-6 * experts * n * k / 4.4, n / 16 * tiles * 2e-3 * k * (16 + r) / 256 / 70)
+
+        def tiles(n, k):
+            wgs = math.ceil(n / 64) * experts * max(1.0, each / 128 + (0.5 if each > 96 else 0.0))
+            r = min(128.0, 32 * math.ceil(each / 32))
+            return 2.5 + max(2e-6 * experts * n * k / 5.2, max(1.0, wgs / 256) * 2e-3 * k * (64 + r) / (42 if wgs <= 256 else 50))
+
+        def packed(n, k):
+            t = math.ceil(n / 512) * experts * (each / 128 + 0.5)
+            whole, left = divmod(t, 256)
+            return 9 + whole * 24e-3 * k + (0 if left == 0 else min(24e-3 * k, 10) if whole and left <= 48 else 24e-3 * k)
+
+        def both(f):
+            return f(ff, hidden) + f(hidden, ff)
+        options = [(both(rows), "rows")] + ([(both(tiles), "tiles")] if each >= 10 else []) + ([(both(packed), "packed")] if may_pack else [])
+        return min(options)[1]
 
     # ---- norms before and after every sublayer (csrc/kernels/seq/sandwich.hip)
     def sandwich_update(self, out, residual, w_next, eps, y=None, w_post=None, mult=1.0, table=None):

@@ -1699,3 +1699,54 @@ def test_expert_steps_run_in_order_and_once():
         a = dict(out="a", x=h, w=h, slots=h, te=h, tile=32, k=1, act=0, pairs=2, tiles=2, **{})
         a.update(other)
         assert not ExpertSteps(ops, [tuple(a.values())]).take(lambda *e: True)
+
+
+# ------------------------------------------------------------------ experts of prompts
+@gpu
+@pytest.mark.parametrize("counts", [[1, 128, 33, 0, 97], [64, 65, 300, 32], [31, 96, 16, 129, 2]])
+@pytest.mark.parametrize("N,K,top", [(64, 64, 2), (200, 192, 3), (1024, 128, 2), (72, 640, 1), (2048, 1024, 2)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_expert_gemm_of_prompt_tiles(counts, N, K, top, act):
+    """Tiles of 128 slots: every number of row groups, columns that fill no tile, fewer stages than are in flight, rows by token and by slot."""
+    from hipserve.models.mixers import MOE_TILE_PROMPT as tile
+
+    g, E, ops = torch.Generator().manual_seed(sum(counts) + N), len(counts), get_ops("cuda")
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    P = -(-len(ids) // top) * top
+    ids = torch.cat([ids, torch.full((P - len(ids),), E - 1)])[torch.randperm(P, generator=g)]
+    cap = -(-(P + E * (tile - 1)) // tile) * tile
+    slots, te, ps = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (cap, cap // tile, P))
+    ops.moe_align(ids.int().cuda(), E, tile, slots, te, ps)
+    x, w = torch.randn(P // top, K + 8, generator=g).bfloat16().cuda()[:, :K], (torch.randn(E, N, K, generator=g) / K ** 0.5).bfloat16().cuda()
+    rows, at = x.repeat_interleave(top, 0), ps.long()
+    by_slot = torch.full((cap, K), float("nan"), dtype=torch.bfloat16, device="cuda")   # what lies in slots of no pair is not used
+    by_slot[at] = rows
+    y, size = (torch.stack([a[p] @ b[e].T for p, e in enumerate(ids.tolist())]) for a, b in ((rows.double(), w.double()), (rows.double().abs(), w.double().abs())))
+    if act:
+        y, size = y.clamp(min=0) ** 2, 2 * y.abs() * size
+    for src, k in ((x, top), (by_slot, 0)):
+        out = torch.full((cap, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops.expert_gemm(out, src, w, slots, te, tile, k, act, pairs=P, tiles=P)
+        assert ((out[at].double() - y).abs() <= 2.0 ** -8 * y.abs() + K * 2.0 ** -23 * size + 1e-30).all()   # the result's type, the sums' rounding
+        assert bool((out[slots < 0] == 7.0).all())
+
+
+def test_expert_plan_of_a_prompt():
+    """What the three kernels were measured to take has the choice; sizes that were not looked at stay where they were."""
+    from types import SimpleNamespace
+
+    from hipserve.models.mixers import TableMoE
+    from hipserve.ops import KernelOps
+
+    rule = KernelOps()._expert_plan
+    assert rule(132, 8, 512, 1024, False) == "rows" and rule(600, 8, 512, 1024, False) == "rows" and rule(2000, 8, 512, 1024, False) == "tiles"
+    assert rule(400, 16, 1024, 2048, False) == "tiles" and rule(4096, 16, 1024, 2048, True) == "tiles" and rule(8000, 16, 1024, 2048, True) == "packed"
+    assert rule(2048, 8, 2048, 4096, True) == "tiles" and rule(4000, 8, 2048, 4096, True) == "packed" and rule(4000, 8, 2048, 4096, False) == "tiles"
+    assert rule(500, 64, 768, 1536, False) == "rows"
+    ops = SimpleNamespace(name="hip", SKINNY_ROWS=64, expert_plan=lambda *a: "tiles")
+    spec = lambda **kw: SimpleNamespace(**{**dict(experts=4, top=2, ff=512), **kw})  # noqa: E731
+    planned = lambda dtype=torch.bfloat16, hidden=1024, ops=ops, **kw: TableMoE(spec(**kw), hidden, 9, "cpu", dtype, ops).planned  # noqa: E731
+    none = float("inf")
+    assert planned() == 128 and planned(torch.float32) == planned(ff=256) == planned(ff=520) == planned(hidden=1000) == planned(ops=None) == none
+    tile = lambda P, **kw: TableMoE(spec(**kw), 1024, 9, "cpu", torch.bfloat16, ops)._tables(P, "cpu")[0]  # noqa: E731
+    assert tile(128) == 32 and tile(129) == 128 and tile(1024, ff=256) == 64
