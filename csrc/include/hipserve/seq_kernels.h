@@ -250,6 +250,27 @@ void launch_window_attention_decode(void* out, long out_ld, const void* proj, lo
                                     bool sink, float out_scale, int nparts, int part_keys, float* ws_acc, float* ws_ml, int keep,
                                     float softcap, const float* sink_w, bool channel_gate, int chunk, bool f32, const WindowPrep* prep,
                                     hipStream_t s);
+// The same with its preparation (every sequence one row), heads of 64 or 128, and the generalized delta rule's decode step, its bottleneck's product included, in one
+// launch: the halves of a parallel mixer. False, and nothing done: too many workgroups for it.
+struct DeltaStep {
+  void* out;
+  long out_ld;
+  float* S;
+  const void* proj;
+  long ld;
+  const void* w2;
+  int heads, rank;
+  const float *a_b, *w0, *norm_w;
+  const int* seq_state;
+  float eps, out_scale;
+};
+bool launch_window_delta_step(void* out, long out_ld, const void* proj, long proj_ld, const void* cache, int block_size, const int* seq_cu,
+                              const int* seq_ctx, const int* seq_bt, int bt_width, int rows, int heads, int kv_heads, int dim, int gate_off, float scale,
+                              int window, bool sink, float out_scale, int nparts, int part_keys, float* ws_acc, float* ws_ml, int keep, float softcap,
+                              const float* sink_w, bool channel_gate, int chunk, bool f32, const WindowPrep& prep, const DeltaStep& delta, hipStream_t s);
+// The merge of the runs of a launch of decode rows.
+void launch_window_decode_reduce(void* out, long out_ld, const float* ws_acc, const float* ws_ml, const void* proj, long proj_ld, int gate_off, int nparts,
+                                 int heads, int rows, int row_base, int vdim, float out_scale, bool channel_gate, bool f32, hipStream_t s);
 
 // fp32 prompt portions of the sequences seq0 .. seq1 - 1 (the sizes of window_attention_decode_ok).
 void launch_window_attention_prompts_f32(float* out, long out_ld, const float* proj, long proj_ld, const float* cache, int block_size,

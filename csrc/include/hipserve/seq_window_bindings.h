@@ -137,12 +137,14 @@ inline bool window_attention_decode_ok(const at::Tensor& proj, const at::Tensor&
          reinterpret_cast<uintptr_t>(proj.data_ptr()) % 16 == 0 && reinterpret_cast<uintptr_t>(cache.data_ptr()) % 16 == 0;
 }
 
-inline void window_decode(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
+// launch(f32, rows, ws_acc, ws_ml): of arguments that are right
+template <typename F>
+inline auto window_decode(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
                            const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t seq0, int64_t row_base, int64_t heads,
                            int64_t kv_heads, int64_t dim, int64_t gate_off, double scale, int64_t window, bool sink,
                            double out_scale, int64_t nparts, int64_t part_keys, const c10::optional<at::Tensor>& ws_acc,
                            const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap,
-                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk, const hipserve::WindowPrep* prep) {
+                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk, F&& launch) {
   TORCH_CHECK(chunk >= 0 && (chunk == 0 || (window == 0 && keep == 0)), "window attention: chunks or a window");
   CHECK_DEV(proj); CHECK_CONTIG(cache); CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_bt);
   const bool f32 = is_f32(proj, "window_attention_decode");
@@ -169,12 +171,15 @@ inline void window_decode(at::Tensor& out, const at::Tensor& proj, const at::Ten
     wm = ws_ml->data_ptr<float>();
   }
   c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
-  hipserve::launch_window_attention_decode(out.data_ptr(), out.stride(0), proj.data_ptr(), proj.stride(0), cache.data_ptr(),
-                                           cache.size(1), seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_bt.data_ptr<int>(),
-                                           seq_bt.size(1), seq0, rows, row_base, heads, kv_heads, dim, gate_off, (float)scale,
-                                           window, sink, (float)out_scale, nparts, part_keys, wa, wm, keep, (float)softcap,
-                                           (const float*)opt_ptr(sink_w), channel_gate, chunk, f32, prep, cur_stream());
+  return launch(f32, rows, wa, wm);
 }
+
+#define HS_WINDOW_DECODE(SEQ0, ROW_BASE, PREP)                                                                                                \
+  hipserve::launch_window_attention_decode(out.data_ptr(), out.stride(0), proj.data_ptr(), proj.stride(0), cache.data_ptr(), cache.size(1),   \
+                                           seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_bt.data_ptr<int>(), seq_bt.size(1), SEQ0, rows, \
+                                           ROW_BASE, heads, kv_heads, dim, gate_off, (float)scale, window, sink, (float)out_scale, nparts,    \
+                                           part_keys, wa, wm, keep, (float)softcap, (const float*)opt_ptr(sink_w), channel_gate, chunk, f32,  \
+                                           PREP, cur_stream())
 
 inline void window_attention_decode(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
                            const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t seq0, int64_t row_base, int64_t heads,
@@ -183,11 +188,14 @@ inline void window_attention_decode(at::Tensor& out, const at::Tensor& proj, con
                            const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap,
                            const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk) {
   window_decode(out, proj, cache, seq_cu, seq_ctx, seq_bt, seq0, row_base, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale,
-                nparts, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, nullptr);
+                nparts, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk,
+                [&](bool f32, long rows, float* wa, float* wm) { HS_WINDOW_DECODE(seq0, row_base, nullptr); });
 }
 
 // The two ops above for steps of at most one row per sequence; the queries in proj stay as they are.
-inline void window_attention_step(at::Tensor& out, const at::Tensor& proj, at::Tensor& cache, const at::Tensor& positions,
+// launch(prep, f32, rows, ws_acc, ws_ml): of arguments that are right.
+template <typename F>
+inline auto window_step(at::Tensor& out, const at::Tensor& proj, at::Tensor& cache, const at::Tensor& positions,
                            const at::Tensor& slots, const at::Tensor& inv_freq, bool own_kv, const c10::optional<at::Tensor>& q_norm,
                            const c10::optional<at::Tensor>& k_norm, int64_t norm_mode, bool v_norm, double eps, double amp,
                            double temp_coef, int64_t temp_every, const at::Tensor& seq_cu,
@@ -195,7 +203,7 @@ inline void window_attention_step(at::Tensor& out, const at::Tensor& proj, at::T
                            int64_t kv_heads, int64_t dim, int64_t gate_off, double scale, int64_t window, bool sink,
                            double out_scale, int64_t nparts, int64_t part_keys, const c10::optional<at::Tensor>& ws_acc,
                            const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap,
-                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk) {
+                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk, F&& launch) {
   CHECK_DEV(proj); CHECK_F32(inv_freq);
   TORCH_CHECK(heads >= 1 && kv_heads >= 1 && temp_every >= 0 && temp_every < (1LL << 31) && norm_mode >= 0 && norm_mode <= 3);
   const long T = proj.size(0), nq = heads * dim, nk = kv_heads * dim;
@@ -213,9 +221,27 @@ inline void window_attention_step(at::Tensor& out, const at::Tensor& proj, at::T
   const hipserve::WindowPrep prep{cache.data_ptr(), positions.data_ptr<long>(), slots.data_ptr<long>(), inv_freq.data_ptr<float>(),
                                   (const float*)opt_ptr(q_norm), own_kv ? (const float*)opt_ptr(k_norm) : nullptr, (int)inv_freq.numel(),
                                   (int)norm_mode, (int)temp_every, (float)eps, (float)amp, (float)temp_coef, own_kv, v_norm, (int)T};
-  window_decode(out, proj, cache, seq_cu, seq_ctx, seq_bt, 0, 0, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale,
-                nparts, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk, &prep);
+  return window_decode(out, proj, cache, seq_cu, seq_ctx, seq_bt, 0, 0, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale,
+                       nparts, part_keys, ws_acc, ws_ml, keep, softcap, sink_w, channel_gate, chunk,
+                       [&](bool f32, long rows, float* wa, float* wm) { return launch(prep, f32, rows, wa, wm); });
 }
+
+inline void window_attention_step(at::Tensor& out, const at::Tensor& proj, at::Tensor& cache, const at::Tensor& positions,
+                           const at::Tensor& slots, const at::Tensor& inv_freq, bool own_kv, const c10::optional<at::Tensor>& q_norm,
+                           const c10::optional<at::Tensor>& k_norm, int64_t norm_mode, bool v_norm, double eps, double amp,
+                           double temp_coef, int64_t temp_every, const at::Tensor& seq_cu,
+                           const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t heads,
+                           int64_t kv_heads, int64_t dim, int64_t gate_off, double scale, int64_t window, bool sink,
+                           double out_scale, int64_t nparts, int64_t part_keys, const c10::optional<at::Tensor>& ws_acc,
+                           const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap,
+                           const c10::optional<at::Tensor>& sink_w, bool channel_gate, int64_t chunk) {
+  window_step(out, proj, cache, positions, slots, inv_freq, own_kv, q_norm, k_norm, norm_mode, v_norm, eps, amp, temp_coef, temp_every, seq_cu,
+              seq_ctx, seq_bt, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale, nparts, part_keys, ws_acc, ws_ml, keep, softcap,
+              sink_w, channel_gate, chunk,
+              [&](const hipserve::WindowPrep& prep, bool f32, long rows, float* wa, float* wm) { HS_WINDOW_DECODE(0, 0, &prep); });
+}
+#undef HS_WINDOW_DECODE
+
 
 inline void window_attention_prompts_f32(at::Tensor& out, const at::Tensor& proj, const at::Tensor& cache, const at::Tensor& seq_cu,
                            const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t seq0, int64_t seq1, int64_t rows_bound,

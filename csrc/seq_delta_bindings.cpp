@@ -242,10 +242,9 @@ void delta_rule(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const at
 bool delta_rule_step_ok(int64_t dim) { return hipserve::delta_rule_step_ok(dim); }
 
 // delta_rule of a step in which every sequence has one row.
-void delta_rule_step(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const c10::optional<at::Tensor>& wl, const at::Tensor& a_b,
+bool check_delta_rule_step(const at::Tensor& out, const at::Tensor& S, const at::Tensor& proj, const c10::optional<at::Tensor>& wl, const at::Tensor& a_b,
                      const at::Tensor& w0, const at::Tensor& norm_w, const at::Tensor& seq_cu, const at::Tensor& seq_ctx,
-                     const at::Tensor& seq_state, int64_t heads, int64_t dim, double eps, double out_scale,
-                     const c10::optional<at::Tensor>& w2) {
+                     const at::Tensor& seq_state, int64_t heads, int64_t dim, const c10::optional<at::Tensor>& w2) {
   CHECK_DEV(proj); CHECK_F32(S); CHECK_F32(a_b); CHECK_F32(w0); CHECK_F32(norm_w);
   CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_state);
   const bool f32 = is_f32(proj, "delta_rule_step");
@@ -266,11 +265,46 @@ void delta_rule_step(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, con
                 reinterpret_cast<uintptr_t>(w2->data_ptr()) % 16 == 0, "delta_rule_step: bottleneck");
   }
   TORCH_CHECK(seq_cu.numel() == nseq + 1 && seq_state.numel() >= nseq && nseq <= 65535);
+  return f32;
+}
+
+void delta_rule_step(at::Tensor& out, at::Tensor& S, const at::Tensor& proj, const c10::optional<at::Tensor>& wl, const at::Tensor& a_b,
+                     const at::Tensor& w0, const at::Tensor& norm_w, const at::Tensor& seq_cu, const at::Tensor& seq_ctx,
+                     const at::Tensor& seq_state, int64_t heads, int64_t dim, double eps, double out_scale,
+                     const c10::optional<at::Tensor>& w2) {
+  const bool f32 = check_delta_rule_step(out, S, proj, wl, a_b, w0, norm_w, seq_cu, seq_ctx, seq_state, heads, dim, w2);
   c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
   hipserve::launch_delta_rule_step(out.data_ptr(), out.stride(0), S.data_ptr<float>(), proj.data_ptr(), proj.stride(0),
                                    (const float*)opt_ptr(wl), a_b.data_ptr<float>(), w0.data_ptr<float>(), norm_w.data_ptr<float>(),
-                                   seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_state.data_ptr<int>(), nseq, heads,
+                                   seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_state.data_ptr<int>(), seq_ctx.numel(), heads,
                                    (float)eps, (float)out_scale, opt_ptr(w2), w2.has_value() ? w2->size(1) : 0, f32, cur_stream());
+}
+
+// window_attention_step and delta_rule_step (with w2) of the same rows in one launch; false, and nothing done, where there are too many workgroups for it.
+bool window_delta_step(at::Tensor& out, const at::Tensor& proj, at::Tensor& cache, const at::Tensor& positions, const at::Tensor& slots,
+                       const at::Tensor& inv_freq, bool own_kv, const c10::optional<at::Tensor>& q_norm, const c10::optional<at::Tensor>& k_norm,
+                       int64_t norm_mode, bool v_norm, double eps, double amp, double temp_coef, int64_t temp_every, const at::Tensor& seq_cu,
+                       const at::Tensor& seq_ctx, const at::Tensor& seq_bt, int64_t heads, int64_t kv_heads, int64_t dim, int64_t gate_off, double scale,
+                       int64_t window, bool sink, double out_scale, int64_t nparts, int64_t part_keys, const c10::optional<at::Tensor>& ws_acc,
+                       const c10::optional<at::Tensor>& ws_ml, int64_t keep, double softcap, const c10::optional<at::Tensor>& sink_w, bool channel_gate,
+                       int64_t chunk, at::Tensor& d_out, at::Tensor& S, const at::Tensor& d_proj, const at::Tensor& a_b, const at::Tensor& w0,
+                       const at::Tensor& norm_w, const at::Tensor& seq_state, int64_t d_heads, int64_t d_dim, double d_eps, double d_scale,
+                       const at::Tensor& w2) {
+  const bool d32 = check_delta_rule_step(d_out, S, d_proj, c10::nullopt, a_b, w0, norm_w, seq_cu, seq_ctx, seq_state, d_heads, d_dim, w2);
+  for (const at::Tensor* t : std::initializer_list<const at::Tensor*>{&d_out, &S, &d_proj, &a_b, &w0, &norm_w, &seq_state, &seq_cu, &seq_ctx, &seq_bt, &out})
+    CHECK_SAME_DEV(*t, proj);
+  const hipserve::DeltaStep delta{d_out.data_ptr(), d_out.stride(0), S.data_ptr<float>(), d_proj.data_ptr(), d_proj.stride(0), w2.data_ptr(), (int)d_heads,
+                                  (int)w2.size(1), a_b.data_ptr<float>(), w0.data_ptr<float>(), norm_w.data_ptr<float>(), seq_state.data_ptr<int>(),
+                                  (float)d_eps, (float)d_scale};
+  return window_step(out, proj, cache, positions, slots, inv_freq, own_kv, q_norm, k_norm, norm_mode, v_norm, eps, amp, temp_coef, temp_every, seq_cu,
+                     seq_ctx, seq_bt, heads, kv_heads, dim, gate_off, scale, window, sink, out_scale, nparts, part_keys, ws_acc, ws_ml, keep, softcap,
+                     sink_w, channel_gate, chunk, [&](const hipserve::WindowPrep& prep, bool f32, long rows, float* wa, float* wm) {
+    TORCH_CHECK(f32 == d32 && (dim == 64 || dim == 128), "window_delta_step: one type, heads of 64 or 128");
+    return hipserve::launch_window_delta_step(out.data_ptr(), out.stride(0), proj.data_ptr(), proj.stride(0), cache.data_ptr(), cache.size(1),
+                                              seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_bt.data_ptr<int>(), seq_bt.size(1), rows, heads,
+                                              kv_heads, dim, gate_off, (float)scale, window, sink, (float)out_scale, nparts, part_keys, wa, wm, keep,
+                                              (float)softcap, (const float*)opt_ptr(sink_w), channel_gate, chunk, f32, prep, delta, cur_stream());
+  });
 }
 
 // floats of delta_rule's `chunks`; 0: not for these rows
@@ -397,6 +431,12 @@ TORCH_LIBRARY(hipserve_delta, m) {
   m.def("delta_rule_step_ok(int dim) -> bool", &delta_rule_step_ok);
   m.def("delta_rule_step(Tensor(a!) out, Tensor(b!) S, Tensor proj, Tensor? wl, Tensor a_b, Tensor w0, Tensor norm_w, "
         "Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, int heads, int dim, float eps, float out_scale, Tensor? w2=None) -> ()");
+  m.def("window_delta_step(Tensor(a!) out, Tensor proj, Tensor(b!) cache, Tensor positions, Tensor slots, Tensor inv_freq, "
+        "bool own_kv, Tensor? q_norm, Tensor? k_norm, int norm_mode, bool v_norm, float eps, float amp, float temp_coef, "
+        "int temp_every, Tensor seq_cu, Tensor seq_ctx, Tensor seq_bt, int heads, int kv_heads, int dim, int gate_off, float scale, "
+        "int window, bool sink, float out_scale, int nparts, int part_keys, Tensor(c!)? ws_acc, Tensor(d!)? ws_ml, int keep, "
+        "float softcap, Tensor? sink_w, bool channel_gate, int chunk, Tensor(e!) d_out, Tensor(f!) S, Tensor d_proj, Tensor a_b, Tensor w0, "
+        "Tensor norm_w, Tensor seq_state, int d_heads, int d_dim, float d_eps, float d_scale, Tensor w2) -> bool");
   m.def("delta_rule_chunk_floats(Tensor proj, int nseq, int heads, int dim) -> int");
   m.def("add_normed(Tensor(a!) out, Tensor(b!) residual, Tensor w, float eps, Tensor? y, Tensor? ye, Tensor? pair_slot, "
         "Tensor? ids, Tensor? wts, int E, Tensor? h, Tensor? shared) -> ()");
@@ -416,6 +456,7 @@ TORCH_LIBRARY_IMPL(hipserve_delta, CUDA, m) {
   m.impl("sandwich_update", &sandwich_update);
   m.impl("delta_rule", &delta_rule);
   m.impl("delta_rule_step", &delta_rule_step);
+  m.impl("window_delta_step", &window_delta_step);
   m.impl("delta_rule_chunk_floats", &delta_rule_chunk_floats);
   m.impl("add_normed", &add_normed);
   m.impl("token_shift", &token_shift);

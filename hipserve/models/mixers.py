@@ -507,15 +507,16 @@ class WindowAttention:
 
     takes_proj = property(lambda self: not self.side_rows)   # ``mix`` takes ``proj`` from outside
 
-    def mix(self, h, meta, cache, state, out, out_scale: float = 1.0, proj=None):
+    def mix(self, h, meta, cache, state, out, out_scale: float = 1.0, proj=None, beside=None):
         """Head outputs (before the output projection), times ``out_scale``, into ``out`` [T, heads * vdim]
         (a column slice of a wider buffer is fine). ``proj``: the input projection's rows, when it is part of
-        a wider one (a column slice, overwritten)."""
+        a wider one (a column slice, overwritten). ``beside``: a step that may go into the attention's launch (``ops.DeltaBeside``)."""
         s, ops = self.spec, self.ops
         if proj is None:
             proj = self.ops.linear(h, self.w_in, self.b_in)
             _side(self, proj)
-        if ops.window_step(out, proj, cache, meta, self.inv_freq, s, self.q_norm, self.k_norm, self.eps, self.gate_off, out_scale, self.sink_w):
+        if ops.window_step(out, proj, cache, meta, self.inv_freq, s, self.q_norm, self.k_norm, self.eps, self.gate_off, out_scale, self.sink_w,
+                           beside):
             return out
         ops.attn_prepare(proj, cache, meta, self.inv_freq, s, self.q_norm, self.k_norm, self.eps)
         ops.window_attention(out, proj, cache, meta, s, self.gate_off, out_scale, self.lam, self.eps, self.sink_w)
@@ -734,6 +735,10 @@ class DeltaRule:
         ops.delta_rule(out, state, proj, wl, self.a_b, self.w0, self.norm, self.spec, self.eps, meta, out_scale)
         return out
 
+    def beside(self, meta, state, out, out_scale, proj):
+        """This step for another kernel's launch (``mix`` with ``proj``), or None."""
+        return self.ops.delta_beside(out, state, proj, self.w2, self.a_b, self.w0, self.norm, self.spec, self.eps, meta, out_scale)
+
     def forward(self, h, meta, cache, state, update=None):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
         return _last(self, self.mix(h, meta, cache, state, out), self.w_o, None, update)
@@ -918,8 +923,11 @@ class ParallelMixer:
         buf = torch.empty(h.shape[0], a + b, device=h.device, dtype=h.dtype)
         if self.w_in is not None:
             proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)
-            self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale, proj[:, :self.split])
-            self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale, proj[:, self.split:])
+            right = (state, buf[:, a:], self.spec.right_scale, proj[:, self.split:])
+            beside = self.right.beside(meta, *right) if isinstance(self.left, WindowAttention) and isinstance(self.right, DeltaRule) else None
+            self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale, proj[:, :self.split], **({} if beside is None else {"beside": beside}))
+            if beside is None or not beside.taken:
+                self.right.mix(h, meta, cache, *right)
             return _last(self, buf, self.w_o, None, update)
         self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale)
         self.right.mix(h, meta, cache, state, buf[:, a:], self.spec.right_scale)

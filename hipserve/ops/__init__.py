@@ -112,6 +112,17 @@ class NormedRows:
         return (self.rows.float() * torch.rsqrt(self.squares.sum(1, keepdim=True) / self.shape[1] + self.eps)).to(self.dtype)
 
 
+class DeltaBeside:
+    """A delta rule's decode step that another kernel of the same step may take into its launch; ``taken`` says whether one has."""
+
+    def __init__(self, args):
+        self.args, self.taken = args, False
+
+    def take(self, launch) -> bool:
+        self.taken = bool(launch(*self.args))
+        return self.taken
+
+
 class ExpertSteps:
     """The products of a step's experts, to be launched in their order: each beside an independent product of the same step that takes it
     into its launch (``take``), or on its own (``finish``). None of them reads or writes what such a product writes or reads."""
@@ -150,9 +161,9 @@ class KernelOps:
         self.norm_library = "seq"
         # the rules of products of a few rows: arithmetic on sizes, a few us each, and a step asks for every product. What they said of
         # the last sizes is kept (a step that is not captured, of four layers and a few rows, took 20 - 40 us longer)
-        self.skinny_pays, self.skinny_parts, self.update_pays, self.update_cols, self.mingru_pays, self.expert_plan = (
+        self.skinny_pays, self.skinny_parts, self.update_pays, self.update_cols, self.mingru_pays, self.expert_plan, self.latent_run = (
             functools.lru_cache(maxsize=4096)(rule)
-            for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._update_cols, self._mingru_pays, self._expert_plan))
+            for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._update_cols, self._mingru_pays, self._expert_plan, self._latent_run))
 
     @property
     def _op(self):
@@ -341,11 +352,7 @@ class KernelOps:
                 span = min(window, meta.max_ctx or window) if window > 0 else meta.max_ctx
                 part = self.LATENT_DECODE_RUN
                 if self._latent_lib.latent_attention_dma_ok(kv_rank, rot_dim):
-                    # a workgroup multiplies 64 keys at a time: short runs, unless the batch fills the chip several times over
-                    # (a run's unnormalised output is written and read once more)
-                    part = 64
-                    while part < 256 and nd * -(-heads // 16) * -(-span // part) > 1024:
-                        part *= 2
+                    part = self.latent_run(nd, heads, span)
                 while -(-span // part) > 64:
                     part *= 2
                 nparts = max(1, -(-span // part))
@@ -362,6 +369,22 @@ class KernelOps:
                 self._latent_lib.latent_attention(o_lat, q_abs, q, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt,
                                            s0, s1, rows, tq, inv_freq, heads, dim, rot_dim, kv_rank, gate_off,
                                            scale, window)
+
+    @staticmethod
+    def _latent_run(rows, heads, span) -> int:
+        """Keys of a run of the decode kernel that multiplies 64 at a time: us of a latency, of its pieces, which take longer where a compute unit has more than one
+        workgroup, of rounds of two workgroups per unit, and of the merge of the runs, with the unnormalised outputs that are written and read once more.
+        192 sizes (1 - 64 rows, 8, 16, 32 heads, 40 - 1024 keys): the choice takes 1.0 % longer than the best of runs of 64 - 1024 keys, at most 16 %; runs of 64 that
+        get longer from 1024 workgroups on took 5.6, at most 57. us of 64 / 128 / 192 / 256 / 512 keys: 16 heads, one row of 700 keys 9.5 / 11.2 / 12.9 / 14.8 / 22.4,
+        48 rows of 150 10.8 / 12.5 / 12.0, of 100 10.5 / 9.8, of 700 24.6 / 18.1 / 18.3 / 19.3 / 25.6; 32 heads, 16 rows of 1024 16.8 / 14.0 / 15.2 / 16.8 / 24.6, 64 rows of
+        1024 61.9 / 41.2 / 39.4 / 31.0 / 34.3."""
+        def time(part):
+            runs, pieces = -(-span // part), -(-min(part, span) // 64)
+            wgs = rows * -(-heads // 16) * runs
+            return (4.7 + 2.1 * pieces * max(1.0, 1.1 * wgs / 256) + 1.1 * max(0.0, wgs / 512 - 1)
+                    + (1.75 + 1e-3 * rows * heads * runs if runs > 1 else 0.0))
+        # (runs of 64, which were taken up to 1024 workgroups, where the others are not clearly expected to be faster: nothing of the above got slower)
+        return min((time(part) * (0.93 if part == 64 else 1.0), part) for part in (64, 128, 192, 256, 512, 1024))[1]
 
     def _mingru_pays(self, rows, width, k, f32) -> bool:
         """Whether the step in its product's epilogue is expected to take less than the faster product of the two and its launch, 2 us (1 in 32 bits)
@@ -396,18 +419,18 @@ class KernelOps:
     WINDOW_MFMA = os.environ.get("HIPSERVE_WINDOW_MFMA", "1") != "0"
     WINDOW_DECODE_RUN = 128  # keys per run of a decode row (a multiple of 32)
 
-    def window_step(self, out, proj, cache, meta, inv_freq, sp, q_norm, k_norm, eps, gate_off, out_scale=1.0, sink_w=None) -> bool:
+    def window_step(self, out, proj, cache, meta, inv_freq, sp, q_norm, k_norm, eps, gate_off, out_scale=1.0, sink_w=None, beside=None) -> bool:
         """``attn_prepare`` and ``window_attention`` of a decode step (one row per sequence) in one launch; False, and nothing done, where they
-        are two."""
+        are two. ``beside``: a ``DeltaBeside`` that may go into the launch (it says so)."""
         if not (meta.max_q == 1 and meta.num_prefill_tokens == 0 and meta.num_decode == meta.seq_ctx.shape[0] > 0 and inv_freq.numel() % 8 == 0
                 and 2 * inv_freq.numel() <= sp.dim <= 128 and all(w is None or w.data_ptr() % 16 == 0 for w in (q_norm, k_norm))):
             return False
         mode, own_kv = 1 if sp.qk_norm else 2 if sp.head_norm else 3 if sp.unit_qk else 0, sp.kv_from is None
         prep = (meta.positions, meta.slot_mapping, inv_freq, own_kv, q_norm if mode in (1, 2) else None, k_norm if mode in (1, 2) and own_kv else None,
                 mode, sp.v_norm, eps, sp.scaling.amplitude if sp.scaling is not None else 1.0, sp.temp_coef, sp.temp_every)
-        return self._window_decode(out, proj, cache, meta, sp, gate_off, out_scale, sink_w, prep)
+        return self._window_decode(out, proj, cache, meta, sp, gate_off, out_scale, sink_w, prep, beside)
 
-    def _window_decode(self, out, proj, cache, meta, sp, gate_off, out_scale, sink_w, prep=None) -> bool:
+    def _window_decode(self, out, proj, cache, meta, sp, gate_off, out_scale, sink_w, prep=None, beside=None) -> bool:
         """The decode rows of ``window_attention`` by the kernel for them; False where it does not take the sizes. ``prep``: what is between
         the cache and the table in ``window_attention_step``."""
         if sp.maps != 1 or not self.WINDOW_MFMA or not self._window_lib.window_attention_decode_ok(proj, cache, sp.dim, sp.vdim):
@@ -441,7 +464,9 @@ class KernelOps:
         rest = (sp.heads, sp.kv_heads, sp.dim, gate_off, sp.scale, sp.window, sp.sink, out_scale, nparts, part, ws_acc, ws_ml,
                 sp.keep_first, sp.softcap, sink_w, sp.channel_gate, sp.chunk)
         if prep is not None:
-            self._window_lib.window_attention_step(out, proj, cache, *prep, meta.seq_cu, meta.seq_ctx, meta.seq_bt, *rest)
+            args = (out, proj, cache, *prep, meta.seq_cu, meta.seq_ctx, meta.seq_bt, *rest)
+            if beside is None or not beside.take(lambda *d: self._delta.window_delta_step(*args, *d)):
+                self._window_lib.window_attention_step(*args)
         else:
             self._window_lib.window_attention_decode(out, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt,
                                                      meta.seq_ctx.shape[0] - nd, meta.num_prefill_tokens, *rest)
@@ -525,21 +550,30 @@ class KernelOps:
 
     DELTA_LOW_RANK = 128   # widest bottleneck that every (sequence, head) multiplies for itself
 
-    def delta_rule_low(self, out, state, proj, w2, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0) -> bool:
-        """``delta_rule`` of a decode step with the bottleneck's product (the last columns of ``proj`` times ``w2``) in its launch; False, and
-        nothing done, where it is a product before it."""
+    def _delta_low_ok(self, state, proj, w2, sp, meta) -> bool:
         # Every workgroup (a head of a row) reads its 64 rows of w2 again, from its compute unit's 32 KB of cache where they fit: a launch saved
         # (1.9 us) against that. us, one launch / two: rank 64 in bf16 1024 workgroups 10.6 / 12.1, 4096 33.2 / 33.0, in fp32 2048 19.7 / 20.6, 3072
         # 28.9 / 27.8; rank 128 in bf16 2048 19.6 / 20.2, 3072 31.2 / 27.4, 16384 137 / 111, in fp32 512 7.9 / 8.7, 1024 13.1 / 12.3, 16384 176 / 117.
         per, row = 16 // proj.element_size(), w2.shape[1] * w2.element_size()
         if proj.shape[0] * sp.heads * row > (1 << 19 if row <= 256 else 1 << 18):
             return False
-        if not (meta.max_q == 1 and self._delta.delta_rule_step_ok(sp.dim) and w2.shape[1] % 32 == 0 and w2.shape[1] <= self.DELTA_LOW_RANK
-                and proj.dtype == w2.dtype and w2.is_contiguous() and proj.stride(0) % per == 0 and all(t.data_ptr() % 16 == 0 for t in (state[0], proj, w2))):
+        return (meta.max_q == 1 and self._delta.delta_rule_step_ok(sp.dim) and w2.shape[1] % 32 == 0 and w2.shape[1] <= self.DELTA_LOW_RANK
+                and proj.dtype == w2.dtype and w2.is_contiguous() and proj.stride(0) % per == 0 and all(t.data_ptr() % 16 == 0 for t in (state[0], proj, w2)))
+
+    def delta_rule_low(self, out, state, proj, w2, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0) -> bool:
+        """``delta_rule`` of a decode step with the bottleneck's product (the last columns of ``proj`` times ``w2``) in its launch; False, and
+        nothing done, where it is a product before it."""
+        if not self._delta_low_ok(state, proj, w2, sp, meta):
             return False
         self._delta.delta_rule_step(out, state[0], proj, None, a_b, w0, norm_w, meta.seq_cu, meta.seq_ctx, meta.seq_state,
                                     sp.heads, sp.dim, eps, out_scale, w2)
         return True
+
+    def delta_beside(self, out, state, proj, w2, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
+        """``delta_rule_low`` for ``window_step`` to take into its launch: a ``DeltaBeside``, or None where it has no such launch."""
+        if not (meta.num_prefill_tokens == 0 and self._delta_low_ok(state, proj, w2, sp, meta)):
+            return None
+        return DeltaBeside((out, state[0], proj, a_b, w0, norm_w, meta.seq_state, sp.heads, sp.dim, eps, out_scale, w2))
 
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
         def aligned(*tensors):   # the kernels below read and write 16 bytes at a time
@@ -1134,8 +1168,11 @@ class ReferenceOps:
     def delta_rule_low(self, out, state, proj, w2, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0) -> bool:
         return False
 
-    def window_step(self, out, proj, cache, meta, inv_freq, sp, q_norm, k_norm, eps, gate_off, out_scale=1.0, sink_w=None) -> bool:
+    def window_step(self, out, proj, cache, meta, inv_freq, sp, q_norm, k_norm, eps, gate_off, out_scale=1.0, sink_w=None, beside=None) -> bool:
         return False
+
+    def delta_beside(self, *args):
+        return None
 
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
         ref.delta_rule(out, state[0], proj, wl, a_b, w0, norm_w, sp, eps, meta.seq_cu, meta.seq_ctx,

@@ -1750,3 +1750,41 @@ def test_expert_plan_of_a_prompt():
     assert planned() == 128 and planned(torch.float32) == planned(ff=256) == planned(ff=520) == planned(hidden=1000) == planned(ops=None) == none
     tile = lambda P, **kw: TableMoE(spec(**kw), 1024, 9, "cpu", torch.bfloat16, ops)._tables(P, "cpu")[0]  # noqa: E731
     assert tile(128) == 32 and tile(129) == 128 and tile(1024, ff=256) == 64
+
+
+# ------------------------------------------------------------------ window attention and the generalized delta rule in one launch
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("heads,kv,dim,ctxs,mode,dheads,rank", [(1, 1, 64, [1], 0, 1, 32), (16, 4, 128, [1, 31, 33, 700], 1, 5, 64), (8, 2, 128, [16, 40, 290], 2, 32, 128),
+                                                               (40, 2, 64, [5, 129, 400, 1], 1, 3, 96), (32, 8, 128, [90] * 20, 0, 64, 64)])
+def test_window_and_delta_step_in_one_launch(heads, kv, dim, ctxs, mode, dheads, rank, dtype):
+    """Fewer and more waves than the rule's four, several runs, each norm, a sequence without a row: the bits of the two launches."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(heads * dim + rank)
+    n, bs, nq, nk, N, eps = len(ctxs), 8, heads * dim, kv * dim, 64 * dheads, 1e-5
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=heads, kv_heads=kv, window=0, reach=0, scale=dim ** -0.5, sink=True, keep_first=0, softcap=0.0,
+                         channel_gate=False, chunk=0, diff=0.0, q_size=nq, k_size=nk, v_size=nk, kv_from=None, qk_norm=mode == 1, head_norm=mode == 2,
+                         unit_qk=False, v_norm=True, temp_coef=0.0, temp_every=0, scaling=None)
+    width = -(-max(ctxs) // bs)
+    bt = torch.randperm((n + 1) * width, generator=g).int().view(n + 1, width)
+    cache = torch.randn((n + 1) * width, bs, 2 * nk, generator=g).to(dtype).cuda()
+    both = torch.randn(n + 1, nq + 2 * nk + 5 * N + rank + 8, generator=g).to(dtype).cuda()   # the two projections side by side, a padding row
+    left, right = both[:, :nq + 2 * nk], both[:, nq + 2 * nk:]
+    w = [torch.rand(m, generator=g).cuda() + 0.5 for m in {1: (nq, nk), 2: (dim, dim)}[mode]] if mode else [None, None]
+    meta = SimpleNamespace(seq_ctx=torch.tensor(ctxs + [3]).int().cuda(), seq_cu=torch.tensor([*range(n + 1), n]).int().cuda(), seq_bt=bt.cuda(),
+                           num_decode=n + 1, num_prefill_tokens=0, max_ctx=max(ctxs), max_q=1, positions=torch.tensor([c - 1 for c in ctxs] + [0]).cuda(),
+                           slot_mapping=torch.tensor([int(bt[s, (c - 1) // bs]) * bs + (c - 1) % bs for s, c in enumerate(ctxs)] + [-1]).cuda(),
+                           seq_state=torch.randperm(n + 2, generator=g)[:n + 1].int().cuda())
+    inv = (1e4 ** (-torch.arange(16).float() / 16)).cuda()
+    S = torch.randn(n + 2, dheads, 64, 64, generator=g).cuda()
+    w2 = (torch.randn(N, rank, generator=g) / rank ** 0.5).to(dtype).cuda()
+    a_b, w0, nw = (torch.randn(N, generator=g).cuda() for _ in range(3))
+    dsp, ops, outs = SimpleNamespace(heads=dheads, dim=64, size=N), get_ops("cuda"), []
+    for one in (False, True):
+        c, s, out = cache.clone(), S.clone(), torch.zeros(n + 1, nq + N, dtype=dtype, device="cuda")
+        rule = (out[:, nq:], [s], right, w2, a_b, w0, nw, dsp, eps, meta, 1.25)
+        beside = ops.delta_beside(*rule) if one else None
+        assert ops.window_step(out[:, :nq], left, c, meta, inv, sp, *w, eps, -1, 0.75, beside=beside)
+        assert beside.taken if one else ops.delta_rule_low(*rule)
+        outs.append((out[:n], c, s))
+    assert all(torch.equal(a, b) for a, b in zip(*outs)) and outs[0][0].isfinite().all()
