@@ -298,7 +298,20 @@ struct GatedDelta {
   const float* decay; const void* gate; // launch_gated_delta, channel
   float* chunks;                        // launch_gated_delta: delta_chunk_floats() floats: in chunks (dim <= delta_chunk_max_dim())
   const void *a2, *g2; int ra, rg;      // launch_gated_delta_step, channel: up-projections [heads * dim, ra], [heads * vdim, rg]
+  bool update_conv = true;              // launch_gated_delta_step, shared queries and keys: the kept inputs too (else launch_conv_update has to follow)
 };
+// The last taps - 1 of C channels' inputs (the first columns of proj) into every sequence's slot.
+struct ConvUpdate {
+  const int *seq_cu, *seq_ctx, *seq_state;
+  const void* proj;
+  long ld;
+  float* conv_state;
+  int C, taps;
+};
+void launch_conv_update(const ConvUpdate& c, int nseq, bool f32, hipStream_t s);
+// It and launch_skinny_linear_normed with a residual in one launch, four taps; false, and nothing done, where there is none for these sizes.
+bool launch_skinny_update_conv(void* out, const SkinnyNorm& norm, const void* x, long x_ld, const void* w, const void* bias, bool f32, int M, int N, int K,
+                               const ConvUpdate& conv, int nseq, hipStream_t s);
 void launch_gated_delta(const GatedDelta& p, float* scratch, bool f32, hipStream_t s);
 // The recurrence in chunks of 16 tokens on the fp32 matrix cores (delta_chunk.hip) from the prepared rows: qk [T, 2 *
 // kv_heads * dim], vv [T, heads * vdim], gg [T, heads * (dim or 1)], bb [T, heads]; o [T, heads * vdim] and 64 floats behind it (written, not read).

@@ -218,8 +218,8 @@ inline void skinny_linear_normed(at::Tensor& out, const at::Tensor& x, const at:
 
 // residual [M, N] += x . w^T + bias; out = residual * weight; squares [M, N / 16] or [M, N / 8] = the residual's squares summed over 16 or 8 columns,
 // which is what a workgroup then takes (skinny_half).
-inline void skinny_linear_update(at::Tensor& out, at::Tensor& squares, at::Tensor& residual, const at::Tensor& weight, const at::Tensor& x,
-                                 const at::Tensor& w, const c10::optional<at::Tensor>& bias) {
+inline hipserve::SkinnyNorm check_update(const at::Tensor& out, at::Tensor& squares, at::Tensor& residual, const at::Tensor& weight, const at::Tensor& x,
+                                         const at::Tensor& w, const c10::optional<at::Tensor>& bias) {
   check_normed_rows(out, squares, x, w, bias);
   CHECK_F32(residual); CHECK_F32(weight); CHECK_SAME_DEV(residual, x); CHECK_SAME_DEV(weight, x);
   const long M = x.size(0), N = w.size(0);
@@ -230,9 +230,15 @@ inline void skinny_linear_update(at::Tensor& out, at::Tensor& squares, at::Tenso
   norm.blocks = squares.size(1);
   norm.residual = residual.data_ptr<float>();
   norm.weight = weight.data_ptr<float>();
+  return norm;
+}
+
+inline void skinny_linear_update(at::Tensor& out, at::Tensor& squares, at::Tensor& residual, const at::Tensor& weight, const at::Tensor& x,
+                                 const at::Tensor& w, const c10::optional<at::Tensor>& bias) {
+  const auto norm = check_update(out, squares, residual, weight, x, w, bias);
   c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
   TORCH_CHECK(hipserve::launch_skinny_linear_normed(out.data_ptr(), false, norm, x.data_ptr(), x.stride(0), w.data_ptr(), opt_ptr(bias),
-                                                    x.scalar_type() == at::kFloat, M, N, x.size(1), -1, 0, 0.f, 0.f, cur_stream()),
+                                                    x.scalar_type() == at::kFloat, x.size(0), w.size(0), x.size(1), -1, 0, 0.f, 0.f, cur_stream()),
               "skinny_linear: LDS");
 }
 

@@ -23,6 +23,7 @@
 //
 // Steps in which every sequence brings one row run the whole gated rule of a (sequence, head) in one workgroup
 // (gated_delta_step).
+#include "conv_update.h"
 #include "seq_common.h"
 #include "hipserve/seq_kernels.h"
 
@@ -177,34 +178,11 @@ __global__ __launch_bounds__(256) void gated_delta_prepare_kernel(
   }
 }
 
-// The last taps - 1 conv inputs of every sequence into its slot (after the prepare kernel has read the old ones).
-constexpr int kMaxHist = 15;
-// HIST inputs are kept per channel (0: taps - 1, up to kMaxHist). All loads side by side, of rows that exist, and the sequence's numbers in one batch: one
-// row of four taps beside the step before it (below).
 template <typename T, int HIST>
 __global__ __launch_bounds__(256) void conv_state_update_kernel(
     const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx, const int* __restrict__ seq_state, const T* __restrict__ proj,
     float* __restrict__ conv_state, int C, int taps, long ld) {
-  constexpr int N = HIST > 0 ? HIST : kMaxHist;
-  const int s = blockIdx.x, c = blockIdx.y * 256 + threadIdx.x;
-  const int r0 = seq_cu[s], r1 = seq_cu[s + 1], ctx = seq_ctx[s], slot = seq_state[s], hist = HIST > 0 ? HIST : taps - 1;
-  asm volatile("" ::"s"(r0), "s"(r1), "s"(ctx), "s"(slot), "s"(ld));
-  const int n = r1 - r0;
-  if (c >= C || n <= 0 || hist <= 0) return;
-  const bool carried = ctx - n > 0;
-  float* cs = conv_state + (long)slot * hist * C + c;
-  const T* rows = proj + (long)r0 * ld + c;
-  float old[N], now[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {   // new input i is row n - hist + i of the step, or (negative) one of the old ones
-    if (i >= hist) continue;
-    const int j = n - hist + i;
-    now[i] = ldf<T>(rows, (long)max(j, 0) * ld);
-    old[i] = cs[(long)min(max(hist + j, 0), hist - 1) * C];
-  }
-#pragma unroll
-  for (int i = 0; i < N; ++i)
-    if (i < hist) cs[(long)i * C] = n - hist + i >= 0 ? now[i] : carried ? old[i] : 0.f;
+  conv_update_block<T, HIST>(blockIdx.x, blockIdx.y * 256 + threadIdx.x, seq_cu, seq_ctx, seq_state, proj, conv_state, C, taps, ld);
 }
 
 constexpr int kTB = 8;     // tokens staged at a time
@@ -1119,7 +1097,7 @@ void gated_delta_step(const GatedDelta& p, hipStream_t s) {
   } else {
     go(&gated_delta_step_kernel<T, CH, 1, false>);
   }
-  if (!own_conv) conv_state_update<T>(p, s);   // its readers are other workgroups too: after all of them
+  if (!own_conv && p.update_conv) conv_state_update<T>(p, s);   // its readers are other workgroups too: after all of them
 }
 
 }  // namespace
@@ -1136,6 +1114,14 @@ void launch_gated_delta_step(const GatedDelta& p, bool f32, hipStream_t s) {
   if (f32) { if (p.channel) gated_delta_step<float, true>(p, s); else gated_delta_step<float, false>(p, s); }
   else if (p.channel) gated_delta_step<unsigned short, true>(p, s);
   else gated_delta_step<unsigned short, false>(p, s);
+}
+
+void launch_conv_update(const ConvUpdate& c, int nseq, bool f32, hipStream_t s) {
+  if (nseq <= 0) return;
+  GatedDelta p{};
+  p.seq_cu = c.seq_cu; p.seq_ctx = c.seq_ctx; p.seq_state = c.seq_state; p.proj = c.proj; p.conv_state = c.conv_state; p.ld = c.ld; p.nseq = nseq;
+  p.taps = c.taps; p.heads = 1; p.vdim = c.C;   // so many channels
+  if (f32) conv_state_update<float>(p, s); else conv_state_update<unsigned short>(p, s);
 }
 
 void launch_delta_rule(void* out, long out_ld, float* S, const void* proj, long ld, const float* wl, const float* a_b,

@@ -130,9 +130,10 @@ void gated_delta_step(at::Tensor& y, at::Tensor& S, at::Tensor& conv_state, cons
                       const at::Tensor& norm_w, const c10::optional<at::Tensor>& a2, const c10::optional<at::Tensor>& g2,
                       const at::Tensor& seq_cu, const at::Tensor& seq_ctx, const at::Tensor& seq_state, int64_t heads,
                       int64_t kv_heads, int64_t dim, int64_t vdim, int64_t taps, double eps, int64_t off_a, int64_t off_g,
-                      int64_t off_b, bool channel, bool silu) {
+                      int64_t off_b, bool channel, bool silu, bool update_conv) {
   auto p = gated_args(y, S, conv_state, proj, conv_w, a_log, dt_bias, norm_w, seq_cu, seq_ctx, seq_state, heads, kv_heads,
                       dim, vdim, taps, eps, off_a, off_g, off_b, channel, silu);
+  p.update_conv = update_conv;
   TORCH_CHECK(vdim <= 256, "gated_delta_step: value size");
   TORCH_CHECK(channel == a2.has_value() && channel == g2.has_value(), "gated_delta_step: bottlenecks");
   if (channel) {
@@ -146,6 +147,39 @@ void gated_delta_step(at::Tensor& y, at::Tensor& S, at::Tensor& conv_state, cons
   }
   c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
   hipserve::launch_gated_delta_step(p, is_f32(proj, "gated_delta_step"), cur_stream());
+}
+
+// What the two ops that move a convolution's kept inputs on check and pass on.
+hipserve::ConvUpdate conv_args(at::Tensor& conv_state, const at::Tensor& proj, const at::Tensor& seq_cu, const at::Tensor& seq_ctx,
+                               const at::Tensor& seq_state, int64_t taps) {
+  CHECK_DEV(proj); CHECK_F32(conv_state); CHECK_I32(seq_cu); CHECK_I32(seq_ctx); CHECK_I32(seq_state);
+  CHECK_SAME_DEV(conv_state, proj); CHECK_SAME_DEV(seq_cu, proj); CHECK_SAME_DEV(seq_ctx, proj); CHECK_SAME_DEV(seq_state, proj);
+  const long nseq = seq_ctx.numel();
+  TORCH_CHECK(taps >= 1 && taps <= hipserve::delta_max_taps() && rows2d(proj) && conv_state.dim() == 3 &&
+              conv_state.size(1) == (taps > 1 ? taps - 1 : 1) && conv_state.size(2) <= proj.size(1), "conv_update: sizes");
+  TORCH_CHECK(seq_cu.numel() == nseq + 1 && seq_state.numel() >= nseq && nseq <= 65535, "conv_update: sequences");
+  return {seq_cu.data_ptr<int>(), seq_ctx.data_ptr<int>(), seq_state.data_ptr<int>(), proj.data_ptr(), proj.stride(0), conv_state.data_ptr<float>(),
+          (int)conv_state.size(2), (int)taps};
+}
+
+void conv_update(at::Tensor& conv_state, const at::Tensor& proj, const at::Tensor& seq_cu, const at::Tensor& seq_ctx, const at::Tensor& seq_state,
+                 int64_t taps) {
+  const auto c = conv_args(conv_state, proj, seq_cu, seq_ctx, seq_state, taps);
+  c10::hip::HIPGuardMasqueradingAsCUDA g(proj.device());
+  hipserve::launch_conv_update(c, seq_ctx.numel(), is_f32(proj, "conv_update"), cur_stream());
+}
+
+// skinny_linear_update and conv_update, of which neither writes what the other reads, in one launch; false, and nothing done, where it has none.
+bool skinny_update_conv(at::Tensor& out, at::Tensor& squares, at::Tensor& residual, const at::Tensor& weight, const at::Tensor& x, const at::Tensor& w,
+                        const c10::optional<at::Tensor>& bias, at::Tensor& conv_state, const at::Tensor& proj, const at::Tensor& seq_cu,
+                        const at::Tensor& seq_ctx, const at::Tensor& seq_state, int64_t taps) {
+  const auto norm = check_update(out, squares, residual, weight, x, w, bias);
+  const auto c = conv_args(conv_state, proj, seq_cu, seq_ctx, seq_state, taps);
+  CHECK_SAME_DEV(proj, x);
+  if (proj.scalar_type() != x.scalar_type()) return false;
+  c10::hip::HIPGuardMasqueradingAsCUDA g(x.device());
+  return hipserve::launch_skinny_update_conv(out.data_ptr(), norm, x.data_ptr(), x.stride(0), w.data_ptr(), opt_ptr(bias), is_f32(x, "conv_update"),
+                                             x.size(0), w.size(0), x.size(1), c, seq_ctx.numel(), cur_stream());
 }
 
 void sandwich_update(at::Tensor& out, at::Tensor& residual, const at::Tensor& w_next, double eps,
@@ -421,7 +455,10 @@ TORCH_LIBRARY(hipserve_delta, m) {
   m.def("delta_chunk_floats(int T, int nseq, int heads, int dim, int vdim) -> int", &delta_chunk_floats);
   m.def("gated_delta_step(Tensor(a!) y, Tensor(b!) S, Tensor(c!) conv_state, Tensor proj, Tensor conv_w, Tensor a_log, "
         "Tensor dt_bias, Tensor norm_w, Tensor? a2, Tensor? g2, Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, int heads, "
-        "int kv_heads, int dim, int vdim, int taps, float eps, int off_a, int off_g, int off_b, bool channel, bool silu) -> ()");
+        "int kv_heads, int dim, int vdim, int taps, float eps, int off_a, int off_g, int off_b, bool channel, bool silu, bool update_conv=True) -> ()");
+  m.def("conv_update(Tensor(a!) conv_state, Tensor proj, Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, int taps) -> ()");
+  m.def("skinny_update_conv(Tensor(a!) out, Tensor(b!) squares, Tensor(c!) residual, Tensor weight, Tensor x, Tensor w, Tensor? bias, "
+        "Tensor(d!) conv_state, Tensor proj, Tensor seq_cu, Tensor seq_ctx, Tensor seq_state, int taps) -> bool");
   m.def("sandwich_update(Tensor(a!) out, Tensor(b!) residual, Tensor w_next, float eps, Tensor? w_post, float mult, "
         "Tensor? table, Tensor? ids, float table_scale, Tensor? a, Tensor? a_w, Tensor? b, Tensor? b_w, float a_scale, "
         "float b_scale, Tensor? ye, Tensor? pair_slot, Tensor? wts, Tensor? shared, Tensor? gate) -> ()");
@@ -453,6 +490,8 @@ TORCH_LIBRARY_IMPL(hipserve_delta, CUDA, m) {
   m.impl("scaled_add_group_rmsnorm", &scaled_add_group_rmsnorm);
   m.impl("gated_delta", &gated_delta);
   m.impl("gated_delta_step", &gated_delta_step);
+  m.impl("conv_update", &conv_update);
+  m.impl("skinny_update_conv", &skinny_update_conv);
   m.impl("sandwich_update", &sandwich_update);
   m.impl("delta_rule", &delta_rule);
   m.impl("delta_rule_step", &delta_rule_step);

@@ -105,12 +105,15 @@ def _side(sub, proj: torch.Tensor):
     sub.side_out = proj[:, proj.shape[1] - n:] if n else None
 
 
-def _last(sub, x: torch.Tensor, w: torch.Tensor, b=None, update=None, beside=None):
+def _last(sub, x: torch.Tensor, w: torch.Tensor, b=None, update=None, beside=None, conv=None):
     """The last product of a sublayer: [T, hidden], or 32-bit parts of it [parts, T, hidden] for a model whose residual update adds
     them up (it sets ``takes_parts``); with ``update`` = (residual, the next norm's weights, eps) the product may do the update
-    itself and return the next sublayer's ``NormedRows``; ``beside``: an ``ops.ExpertSteps`` whose next product may go into the launch."""
+    itself and return the next sublayer's ``NormedRows``; ``beside``: an ``ops.ExpertSteps`` whose next product may go into the launch; ``conv``:
+    an ``ops.ConvBeside`` that an update's launch may take."""
     if update is not None:
-        rows = sub.ops.linear_update(x, w, b, *update)
+        rows = sub.ops.linear_update(x, w, b, *update, conv=conv)
+        if conv is not None:
+            conv.finish()
         if rows is not None:
             return rows
     linear = sub.ops.linear_parts if getattr(sub, "takes_parts", False) else sub.ops.linear
@@ -664,7 +667,7 @@ class GatedDelta:
             t[n + ".conv"] = _rand(gen, c, s.conv, std=0.5)
         return t
 
-    def mix(self, h, meta, cache, state, out, out_scale: float = 1.0, proj=None):
+    def mix(self, h, meta, cache, state, out, out_scale: float = 1.0, proj=None, conv=None):
         s, ops = self.spec, self.ops
         assert out_scale == 1.0
         if proj is None:
@@ -674,7 +677,7 @@ class GatedDelta:
         ra, rg = (self.w_a2.shape[1], self.w_g2.shape[1]) if s.channel_decay else (0, 0)
         if meta.max_q == 1 and max(s.dim, s.vdim) <= self.STEP_MAX_DIM and ra + rg <= self.STEP_MAX_RANK:
             # every sequence brings one row (decode steps): bottlenecks, convolution, recurrence, norm and gate
-            ops.gated_delta_step(out, state, proj, *weights, self.w_a2, self.w_g2, offs, s, self.eps, meta)
+            ops.gated_delta_step(out, state, proj, *weights, self.w_a2, self.w_g2, offs, s, self.eps, meta, conv)
             return out
         decay = gate = None
         if s.channel_decay:
@@ -685,7 +688,8 @@ class GatedDelta:
 
     def forward(self, h, meta, cache, state, update=None):
         out = torch.empty(h.shape[0], self.out_size, device=h.device, dtype=h.dtype)
-        return _last(self, self.mix(h, meta, cache, state, out), self.w_o, None, update)
+        conv = None if update is None else self.ops.conv_beside()
+        return _last(self, self.mix(h, meta, cache, state, out, conv=conv), self.w_o, None, update, conv=conv)
 
 
 class DeltaRule:

@@ -123,6 +123,25 @@ class DeltaBeside:
         return self.taken
 
 
+class ConvBeside:
+    """The update of the inputs that a gated delta rule's convolution keeps, left by a decode step (``KernelOps.gated_delta_step``) for the layer's
+    last product: ``take`` runs it in that product's launch, ``finish`` on its own unless it has run."""
+
+    def __init__(self, ops):
+        self.ops, self.left = ops, None   # (kept inputs, projection, sequences, taps)
+
+    def take(self, launch) -> bool:
+        if self.left is None or not launch(*self.left):
+            return False
+        self.left = None
+        return True
+
+    def finish(self):
+        if self.left is not None:
+            self.ops._delta.conv_update(*self.left)
+            self.left = None
+
+
 class ExpertSteps:
     """The products of a step's experts, to be launched in their order: each beside an independent product of the same step that takes it
     into its launch (``take``), or on its own (``finish``). None of them reads or writes what such a product writes or reads."""
@@ -541,12 +560,19 @@ class KernelOps:
                                 meta.seq_ctx, meta.seq_state, scratch, sp.heads, sp.kv_heads, sp.dim, sp.vdim, sp.conv, eps,
                                 *offs, sp.channel_decay, sp.gate_act == "silu", chunks)
 
-    def gated_delta_step(self, y, state, proj, conv_w, a_log, dt_bias, norm_w, w_a2, w_g2, offs, sp, eps, meta):
+    def conv_beside(self):
+        return ConvBeside(self)
+
+    def gated_delta_step(self, y, state, proj, conv_w, a_log, dt_bias, norm_w, w_a2, w_g2, offs, sp, eps, meta, conv=None):
         """``gated_delta`` for steps in which every sequence has one row (``meta.max_q`` == 1), the bottlenecks'
-        up-projections ``w_a2`` / ``w_g2`` included."""
+        up-projections ``w_a2`` / ``w_g2`` included; ``conv``: a ``ConvBeside`` that is given the update of the convolution's kept inputs where
+        that is a launch of its own (queries and keys shared by several heads)."""
+        later = conv is not None and sp.heads != sp.kv_heads
         self._delta.gated_delta_step(y, state[0], state[1], proj, conv_w, a_log, dt_bias, norm_w, w_a2, w_g2, meta.seq_cu,
                                      meta.seq_ctx, meta.seq_state, sp.heads, sp.kv_heads, sp.dim, sp.vdim, sp.conv, eps,
-                                     *offs, sp.channel_decay, sp.gate_act == "silu")
+                                     *offs, sp.channel_decay, sp.gate_act == "silu", not later)
+        if later:
+            conv.left = (state[1], proj, meta.seq_cu, meta.seq_ctx, meta.seq_state, sp.conv)
 
     DELTA_LOW_RANK = 128   # widest bottleneck that every (sequence, head) multiplies for itself
 
@@ -742,15 +768,17 @@ class KernelOps:
         up to 32 rows."""
         return 8 if cols <= 2048 and k * (2 if f32 else 1) > (4096 if rows <= 8 and cols <= 1024 else 1024) else 16
 
-    def linear_update(self, x, w, bias, residual, norm_w, eps):
+    def linear_update(self, x, w, bias, residual, norm_w, eps, conv=None):
         """residual += x . w^T + bias, and the rows for the next products as ``NormedRows`` of its norm; None, and nothing done, where the
-        update and norm are a launch of their own (``update_pays``)."""
+        update and norm are a launch of their own (``update_pays``). ``conv``: a ``ConvBeside`` that the launch may take."""
         T, N, K = x.shape[0], w.shape[0], w.shape[1]
         if not (0 < T <= self.NORM_ROWS and N % 64 == 0 and N <= 4096 and self.update_pays(T, N, K, x.dtype == torch.float32)
                 and self._skinny_ok(x, w, bias) and residual.is_contiguous() and residual.data_ptr() % 16 == 0):
             return None
         rows, squares = torch.empty(T, N, device=x.device, dtype=x.dtype), torch.empty(T, N // self.update_cols(T, N, K, x.dtype == torch.float32), device=x.device, dtype=torch.float32)
-        self._moe_lib.skinny_linear_update(rows, squares, residual, norm_w, x, w, bias)
+        product = (rows, squares, residual, norm_w, x, w, bias)
+        if conv is None or not conv.take(lambda *c: self._delta.skinny_update_conv(*product, *c)):
+            self._moe_lib.skinny_linear_update(*product)
         return NormedRows(rows, squares, eps)
 
     def linear_heads(self, out, x, w) -> bool:
@@ -1152,7 +1180,10 @@ class ReferenceOps:
         ref.gated_delta(y, state[0], state[1], proj, conv_w, a_log, dt_bias, norm_w, decay, gate, offs, sp, eps,
                         meta.seq_cu, meta.seq_ctx, meta.seq_state)
 
-    def gated_delta_step(self, y, state, proj, conv_w, a_log, dt_bias, norm_w, w_a2, w_g2, offs, sp, eps, meta):
+    def conv_beside(self):
+        return None
+
+    def gated_delta_step(self, y, state, proj, conv_w, a_log, dt_bias, norm_w, w_a2, w_g2, offs, sp, eps, meta, conv=None):
         decay = gate = None
         if sp.channel_decay:
             low_a, low_g = (proj[:, o:o + w.shape[1]].float() for o, w in ((offs[0], w_a2), (offs[1], w_g2)))
@@ -1193,7 +1224,7 @@ class ReferenceOps:
     def linear_parts(self, x, w, bias=None, beside=None):
         return self.linear(x, w, bias)
 
-    def linear_update(self, x, w, bias, residual, norm_w, eps):
+    def linear_update(self, x, w, bias, residual, norm_w, eps, conv=None):
         return None
 
     def linear_heads(self, out, x, w) -> bool:

@@ -1788,3 +1788,36 @@ def test_window_and_delta_step_in_one_launch(heads, kv, dim, ctxs, mode, dheads,
         assert beside.taken if one else ops.delta_rule_low(*rule)
         outs.append((out[:n], c, s))
     assert all(torch.equal(a, b) for a, b in zip(*outs)) and outs[0][0].isfinite().all()
+
+
+@gpu
+@pytest.mark.parametrize("T,N,K,C,dtype", [(1, 64, 512, 1, torch.bfloat16), (8, 1024, 6144, 513, torch.bfloat16), (9, 1024, 2048, 512, torch.float32),
+                                           (16, 4096, 512, 96, torch.bfloat16), (17, 4096, 512, 96, torch.float32), (32, 1024, 3072, 1025, torch.bfloat16),
+                                           (20, 2048, 256, 2048, torch.float32)])
+def test_update_and_conv_in_one_launch(T, N, K, C, dtype):
+    """A workgroup's channels and one more, a first step, sequences without a row, every size of a product's workgroups: the bits of the two launches."""
+    from hipserve.ops import ConvBeside
+    g = torch.Generator().manual_seed(T + N + C)
+    ops, nseq = get_ops("cuda"), T + 2
+    x, w, proj = (torch.randn(*s, generator=g).to(dtype).cuda() for s in ((T, K), (N, K), (T, C + 24)))
+    norm, kept = torch.rand(N, generator=g).cuda(), torch.randn(nseq + 1, 3, C, generator=g).cuda()
+    seqs = (torch.tensor([0, *range(T + 1), T]).int().cuda(), torch.randint(1, 3, (nseq,), generator=g).int().cuda(),
+            torch.randperm(nseq + 1, generator=g)[:nseq].int().cuda())   # the first and the last have no row
+    ops.update_pays = lambda *a: True
+    outs = []
+    for one in (False, True):
+        conv, c, r = ConvBeside(ops), kept.clone(), torch.ones(T, N).cuda()
+        conv.left = (c, proj, *seqs, 4)
+        got = ops.linear_update(x, w, None, r, norm, 1e-6, conv=conv if one else None)
+        assert (conv.left is None) == one
+        conv.finish()
+        outs.append((got.rows, got.squares, r, c))
+    assert all(torch.equal(a, b) for a, b in zip(*outs)) and outs[0][0].isfinite().all()
+    want = kept.clone()
+    for s in range(1, T + 1):
+        old = kept[seqs[2][s], 1:] * float(seqs[1][s] > 1)
+        want[seqs[2][s]] = torch.cat([old, proj[s - 1:s, :C].float()])
+    assert torch.equal(outs[0][3], want)
+    conv.left = (kept[:, :2].contiguous(), proj, *seqs, 3)   # other taps are a launch of their own
+    ops.linear_update(x, w, None, r, norm, 1e-6, conv=conv)
+    assert conv.left is not None
