@@ -27,6 +27,8 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
 double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts);
 // Tiles of 16 columns that a workgroup takes, where it doesn't take half a one
 int skinny_tiles(int M, long tiles, int K);
+// columns of a workgroup where it takes neither half a tile nor the tiles above (0: it does)
+int skinny_cols(int M, long cols, int K);
 // Whether its workgroups take 8 columns for 16; tiles of 16 columns, over all batches and parts, K in 16-bit halves
 bool skinny_half(int M, long tiles, int K);
 // A norm around such a product of up to 32 rows, in one part: with a residual [M, N] (fp32, updated in place), out = residual * weight

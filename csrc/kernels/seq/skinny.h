@@ -34,9 +34,9 @@ template <int N> HS_DEVICE void wait_copies() { asm volatile("s_waitcnt vmcnt(%0
 // One wave's part of W[NT tiles of 16 columns] . x[XG groups of 8 rows]. K in 16-bit halves, K % 8 == 0.
 // A piece (64 k) in LDS: [NT tiles][16 rows][128 bytes] of W, then [XG][8 rows][128 bytes] of x; the 16-byte part q of row r sits
 // at part q ^ (r / 2 % 8), so that the 16 rows of an operand use all banks evenly: a lane copies the part that belongs at its place.
+// HALF: the last tile is its first 8 columns.
 template <int XG, int NT, int DEPTH, bool F32 = false, bool HALF = false> struct Skinny {
-  static_assert(!HALF || NT == 1, "eight columns");
-  static constexpr int WG = HALF ? 1 : 2 * NT;   // groups of 8 rows of W
+  static constexpr int WG = 2 * NT - HALF;   // groups of 8 rows of W
   static constexpr int ST = (XG + 1) / 2, kCopies = WG + XG, kPiece = kCopies * 1024;
   // the last tile's missing 8 rows, where XG is odd, are read past the piece
   static constexpr int kRing = kSkWaves * DEPTH * kPiece + (XG & 1) * 1024, kSums = kSkWaves * 16 * ST * kSkLd * 4;
@@ -83,9 +83,9 @@ template <int XG, int NT, int DEPTH, bool F32 = false, bool HALF = false> struct
     int at[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) at[s] = c * 128 + (((4 * s + g) ^ (c >> 1)) << 4);
-    int w_of[2];   // HALF: both halves of the tile are the same eight rows
+    int half_of[2];   // HALF: both halves of the last tile are the same eight rows
 #pragma unroll
-    for (int s = 0; s < 2; ++s) w_of[s] = HALF ? (c & 7) * 128 + (((4 * s + g) ^ ((c & 7) >> 1)) << 4) : at[s];
+    for (int s = 0; s < 2; ++s) half_of[s] = (c & 7) * 128 + (((4 * s + g) ^ ((c & 7) >> 1)) << 4);
 #pragma unroll
     for (int i = 0; i < DEPTH; ++i)
       if (i < n) copy(i);
@@ -98,7 +98,7 @@ template <int XG, int NT, int DEPTH, bool F32 = false, bool HALF = false> struct
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) a[s][nt] = *reinterpret_cast<const u16x8*>(t + nt * 2048 + w_of[s]);
+        for (int nt = 0; nt < NT; ++nt) a[s][nt] = *reinterpret_cast<const u16x8*>(t + nt * 2048 + (HALF && nt == NT - 1 ? half_of[s] : at[s]));
 #pragma unroll
         for (int st = 0; st < ST; ++st) b[s][st] = *reinterpret_cast<const u16x8*>(t + WG * 1024 + st * 2048 + at[s]);
       }
@@ -141,7 +141,7 @@ template <int XG, int NT, int DEPTH, bool F32 = false, bool HALF = false> struct
 
   // Sums the waves' parts: v[nt][i] = element (row, column) = (e / kCols, e % kCols), e = threadIdx.x + kSkThreads * i, of
   // the [16 ST, kCols] result of column tile nt (threads past it get nothing).
-  static constexpr int kCols = HALF ? 8 : 16, kElems = (16 * ST * kCols + kSkThreads - 1) / kSkThreads;
+  static constexpr int kCols = HALF && NT == 1 ? 8 : 16, kElems = (16 * ST * kCols + kSkThreads - 1) / kSkThreads;
   static HS_DEVICE void reduce(float (&v)[NT][kElems], const f32x4 (&acc)[NT][ST], unsigned char* smem) {
     float* red = reinterpret_cast<float*>(smem);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c = lane & 15, g = lane >> 4;

@@ -47,16 +47,18 @@ template <int NORM> struct SkinnyArgs {
 // F32: 32-bit operands, x, w, their strides and K in 16-bit halves (skinny.h). Workgroups z take `part` of K each (a multiple of 64) and write
 // their sums out_zs elements apart (the bias in the first).
 // p, q, i: kPlain - , bias, part; kNormed squares, bias, blocks; kUpdate residual, weight, blocks (K in one part for both).
+// HALF: the last of the NT tiles is half of one; one of its own is 8 columns of squares, too.
 template <int XG, int NT, int DEPTH, bool GLU, typename TO, bool F32, int NORM, bool HALF>
 HS_DEVICE void skinny_block(int bx, int by, int bz, const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, void* p, const void* q,
                             int x_ld, int M, int N, int K, int ni, int rest_at, unsigned char* smem) {
   static_assert(!GLU || NT == 2, "a gate tile and an up tile");
+  static_assert(!HALF || NT == 1 || NORM != kUpdate, "squares of whole tiles");
   using SK = Skinny<XG, NT, DEPTH, F32, HALF>;
-  constexpr int ST = SK::ST, kCols = SK::kCols;
+  constexpr int ST = SK::ST, kCols = SK::kCols, kTileCols = GLU ? 16 : 8 * SK::WG;   // of a workgroup
   using TB = std::conditional_t<F32, float, unsigned short>;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int No = GLU ? N / 2 : N;
-  const int n0 = bx * (GLU ? 16 : kCols * NT);
+  const int n0 = bx * kTileCols;
   const int k0 = NORM == kPlain ? bz * ni : 0, k1 = NORM == kPlain ? min(K, k0 + ni) : K;
   if (NORM == kPlain && by != 0) {
     x += (long)by * late_args<SkinnyRest<NORM>>(rest_at)->x_bs;
@@ -70,7 +72,7 @@ HS_DEVICE void skinny_block(int bx, int by, int bz, const unsigned short* __rest
     const int first = GLU ? n0 : min(n0 + 16 * nt, N - 1);   // of the tile's columns
     wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)(GLU ? nt * No : 0) + first) * K + k0);
 #pragma unroll
-    for (int h = 0; h < (HALF ? 1 : 2); ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), No - 1 - first) * (unsigned)(2 * K);
+    for (int h = 0; h < (HALF && nt == NT - 1 ? 1 : 2); ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), No - 1 - first) * (unsigned)(2 * K);
   }
 #pragma unroll
   for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)(2 * x_ld);
@@ -79,7 +81,7 @@ HS_DEVICE void skinny_block(int bx, int by, int bz, const unsigned short* __rest
   for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr int IT = SK::kElems, SQ = HALF ? 8 : 4;   // kCols threads x SQ loads x 4 sums: 256 of them, rows of up to 4096 at 16 columns each
+  constexpr int IT = SK::kElems, SQ = kCols == 8 ? 8 : 4;   // kCols threads x SQ loads x 4 sums: 256 of them, rows of up to 4096 at 16 columns each
   [[maybe_unused]] f32x4 sq[IT][SQ];
   [[maybe_unused]] float res[IT][NT], wgt[NT];
   [[maybe_unused]] TB bs[NT];
@@ -169,7 +171,7 @@ HS_DEVICE void skinny_block(int bx, int by, int bz, const unsigned short* __rest
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const int n = n0 + 16 * nt + e % kCols;
-        if (n >= N) continue;
+        if (n >= N || (HALF && NT > 1 && nt == NT - 1 && e % kCols >= 8)) continue;
         const float z = v[nt][i] + (biased ? ldf<TB>(&bs[nt], 0) : 0.f);
         stf<TO>(out, m * out_ld + n, skinny_act(z, n >= act_from ? act : -1, c0, c1));
       }

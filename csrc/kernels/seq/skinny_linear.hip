@@ -60,20 +60,31 @@ bool launch_kernel(dim3 grid, void* out, long out_ld, long out_bs, long out_zs, 
 template <int XG, int NT, int DEPTH, bool GLU, bool HALF = false, int DEPTH32 = DEPTH>
 bool launch_one(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, int parts, const void* x, long x_ld, long x_bs,
                 const void* w, const void* bias, bool f32, int batch, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
-  const int cols = GLU ? N / 2 : N, per = GLU ? 16 : HALF ? 8 : 16 * NT;
+  const int cols = GLU ? N / 2 : N, per = GLU ? 16 : 16 * NT - 8 * HALF;
   const dim3 grid((cols + per - 1) / per, batch, parts);
 #define HS_SK(TO, F32) launch_kernel<XG, NT, F32 ? DEPTH32 : DEPTH, GLU, TO, F32, kPlain, HALF>(grid, out, out_ld, out_bs, out_zs, x, x_ld, x_bs, w, bias, M, N, K, act, act_from, c0, c1, s)
   return f32 ? HS_SK(float, true) : out_f32 ? HS_SK(float, false) : HS_SK(unsigned short, false);
 #undef HS_SK
 }
 
+// The same for 16-bit operands alone.
+template <int XG, int NT, int DEPTH, bool HALF>
+bool launch_16(void* out, bool out_f32, long out_ld, const void* x, long x_ld, const void* w, const void* bias, int M, int N, int K, int act, int act_from,
+               float c0, float c1, hipStream_t s) {
+  constexpr int per = 16 * NT - 8 * HALF;
+#define HS_SK(TO) launch_kernel<XG, NT, DEPTH, false, TO, false, kPlain, HALF>(dim3((N + per - 1) / per), out, out_ld, 0, 0, x, x_ld, 0, w, bias, M, N, K, act, act_from, c0, c1, s)
+  return out_f32 ? HS_SK(float) : HS_SK(unsigned short);
+#undef HS_SK
+}
+
 // us of a launch (K in halves, over `parts`): a latency, the results, and the time the weights take at 5.2 TB/s, or, where that is more, at 9 TB/s and with it
 // what the busiest compute unit takes in (80 KB per us), its sums in LDS and its products of 32-bit operands. 9 % off on average over 5127 sizes (1 -
 // 64 rows, 64 - 65536 columns, k 128 - 12288, plain and gated, 32 bits).
-double skinny_time_of(int M, long cols, double K, int nt, int parts, bool f32, double out_bytes, bool half = false) {
-  const long wgs = ((cols + 15) / 16 + nt - 1) / nt * parts, rounds = (wgs + 255) / 256;   // of whole tiles; halves are one round
-  const double bytes = 2.0 * cols * K, rows = (M + 7) / 8 * 8, k = K / parts, st = nt * ((M + 15) / 16);
-  const double each = 2.0 * k * ((half ? 8 : 16 * nt) + rows) / 80e3 + st * (0.09 + (f32 ? 8.5e-5 * k : 0));
+// per: columns of a workgroup.
+double skinny_time_of(int M, long cols, double K, int per, int parts, bool f32, double out_bytes) {
+  const long wgs = (cols + per - 1) / per * parts, rounds = (wgs + 255) / 256;
+  const double bytes = 2.0 * cols * K, rows = (M + 7) / 8 * 8, k = K / parts, st = (per + 15) / 16 * ((M + 15) / 16);
+  const double each = 2.0 * k * (per + rows) / 80e3 + st * (0.09 + (f32 ? 8.5e-5 * k : 0));
   return 2.16 + std::max(bytes / 5.2e6, bytes / 9e6 + rounds * each) + 0.7e-6 * out_bytes;
 }
 
@@ -101,15 +112,53 @@ bool skinny_half(int M, long tiles, int K) {
   return tiles <= 128 && (M <= 8 && tiles <= 64 ? K > 4096 : K > 1024) && (M <= 32 || tiles <= 104 || K > 2048);
 }
 
+// Columns of a workgroup where whole tiles by the rules above would be rounds of workgroups over the compute units of which the last is far from full: 24, 40, 48 or 56,
+// which are one round, or two. 0: by the rules above. 16-bit operands of 9 - 48 rows. What a compute unit takes in, its columns' weights and the rows once per
+// workgroup, is what bounds these sizes, and a started round costs as much as a full one. Cold weights, us, by the rules above -> here, 16, 24, 48
+// rows: 6144 x 2048 7.7 -> 7.0, 8.0 -> 7.5, 9.9 -> 9.2, 5120 x 4096 12.4 -> 10.2, 13.1 -> 11.2, 15.8 -> 14.4 (24 columns); 10240 x 3072 15.1 -> 13.0, 18.0 ->
+// 13.6, 22.7 -> 16.8 (40); 12288 x 4096, 24, 48 rows 22.5 -> 21.1, 25.5 -> 23.6 (48); 13376 x 3072 18.8 -> 16.6, 19.8 -> 17.4, 24.0 -> 20.7 (56); 20480 x 2048, 24
+// rows 19.6 -> 18.4 (40, two rounds). A short k is latency, and wider workgroups sum more tiles: 4104 x 1024, 16 rows 4.1 -> 4.6; 8200 x 2048, 16 rows 9.2 -> 9.2;
+// 13376 x 2048, 24 rows 14.1 -> 14.3; 20480 x 2048, 48 rows 23.3 -> 24.4: these stay. Of 320 sizes (16 - 48 rows, 4104 - 32000 columns, k 512 - 4096) 150 are
+// taken, none of which got slower by more than 1.1 %.
+int skinny_cols(int M, long cols, int K) {
+  const long tiles = (cols + 15) / 16;
+  if (M <= 8 || M > 48 || tiles <= 256 || tiles > 1792) return 0;
+  if (tiles <= 384) return K >= (M > 16 ? 1024 : 2048) ? 24 : 0;
+  if (tiles <= 512) return 0;
+  if (tiles <= 768) {
+    if (M <= 16 && (K < 3072 || tiles > 704)) return 0;
+    return K >= 1024 && !(tiles <= 544 && K < 2048) ? tiles <= 640 ? 40 : 48 : 0;
+  }
+  if (tiles <= 896) return K >= 3072 && K < (M <= 16 ? 4096 : 1 << 30) ? 56 : 0;
+  if (tiles <= 1024) return 0;
+  if (tiles <= 1280) return M > 16 && K >= (M > 32 ? 3072 : 1024) ? 40 : 0;
+  return tiles > 1536 && K >= 3072 && K < (M <= 16 ? 4096 : 1 << 30) ? 56 : 0;
+}
+
+// Of up to 8 rows and more workgroups than compute units: how many pieces a workgroup of one whole tile copies ahead where three are best (0: by the rules of
+// the launch), and whether half tiles are better still. Three are for k (in halves) of 2048 and more, once the units have two workgroups each; half tiles are for rows
+// of weights 4096 bytes apart, of which eight per load and workgroup go to the same channels and not sixteen, as long as the rows that they read twice as
+// often are few. Cold weights, us, one row, before -> three pieces -> half tiles: 8192 x 2048 8.4 -> 7.9 -> 7.3, 12288 x 2048 11.0 -> 10.5 -> 9.9, 32000 x 2048 23.9 ->
+// 22.7 -> 22.3, 8192 x 4096 13.9 -> 12.8 -> 13.6, 12288 x 4096 18.6 -> 17.9 -> 19.1, 32000 x 3072 32.8 -> 32.2 -> 32.5; 8 rows, 32000 x 2048 24.0 -> 23.4 -> 24.3; in 32
+// bits, 32000 x 1024 24.5 -> 23.5 -> 26.7. As they were: 5152 x 2048 6.1 (half tiles 6.2), 8192 x 3072 9.7 (10.0), 32000 x 1024 11.8 (15).
+struct SkinnyWide { int ahead; bool half; };
+static SkinnyWide skinny_wide(int M, long tiles, int K, bool f32) {
+  if (M > 8 || K < 2048) return {0, false};
+  if (M <= 4 && !f32 && K == 2048 && tiles > 352) return {2, true};
+  return {tiles > 512 || (tiles > 384 && K % 2048 == 0) ? 3 : 0, false};
+}
+
 double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts) {
   const int K = f32 ? 2 * k : k;
   const double out = (double)M * (glu ? cols / 2 : cols) * (f32 ? 4 : 2);
   const long tiles = (cols + 15) / 16 * parts;
-  return skinny_time_of(M, cols, K, glu ? 2 : skinny_tiles(M, tiles, K / parts), parts, f32, out, !glu && skinny_half(M, tiles, K / parts));
+  const int own = !glu && !f32 && parts == 1 ? skinny_cols(M, cols, K) : 0;
+  const int per = glu ? 32 : own > 0 ? own : skinny_half(M, tiles, K / parts) ? 8 : 16 * skinny_tiles(M, tiles, K / parts);
+  return skinny_time_of(M, cols, K, per, parts, f32, out);
 }
 
 double mingru_product_time(int M, int width, int k, bool f32) {   // a workgroup's three tiles (mingru.hip)
-  return skinny_time_of(M, 3L * width, f32 ? 2 * k : k, 3, 1, f32, (double)M * width * (f32 ? 4 : 2));
+  return skinny_time_of(M, 3L * width, f32 ? 2 * k : k, 48, 1, f32, (double)M * width * (f32 ? 4 : 2));
 }
 
 bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, long out_zs, int parts, const void* x, long x_ld, long x_bs,
@@ -132,6 +181,15 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
     return xg <= 2 ? HS_SK(2, 1, 2, false, true) : xg <= 4 ? HS_SK(4, 1, 2, false, true, 1) : xg <= 6 ? HS_SK(6, 1, 2, false, true, 1)
          : HS_SK(8, 1, 2, false, true, 1);
   }
+  if (const int cols = batch == 1 && parts == 1 && !f32 ? skinny_cols(M, N, K) : 0) {
+#define HS_S16(XG, NT, HALF) launch_16<XG, NT, 1, HALF>(out, out_f32, out_ld, x, x_ld, w, bias, M, N, K, act, act_from, c0, c1, s)
+#define HS_SG(NT, HALF) (xg <= 2 ? HS_S16(2, NT, HALF) : xg <= 4 ? HS_S16(4, NT, HALF) : HS_S16(6, NT, HALF))
+    return cols == 24 ? HS_SG(2, true) : cols == 40 ? HS_SG(3, true) : cols == 48 ? HS_SG(3, false) : HS_SG(4, true);
+#undef HS_SG
+#undef HS_S16
+  }
+  if (const auto wide = batch == 1 && parts == 1 ? skinny_wide(M, tiles, K, f32) : SkinnyWide{}; wide.ahead > 0)
+    return wide.half ? HS_SK(1, 1, 2, false, true) : HS_SK(1, 1, 3, false);
   const int nt = skinny_tiles(M, tiles, K / parts);
   // One piece ahead: two are faster (up to 40 %) where a wave waits for its few copies, up to 16 rows and more than a piece per wave (more than
   // two where a compute unit holds several workgroups: 12288 x 1024, 16 rows 9 % slower; 3072 x 1024, one row 4 % faster), and slower
@@ -152,7 +210,7 @@ static bool launch_normed(void* out, bool out_f32, const SkinnyNorm& norm, const
   const bool glu = act == 3 || act == 4;
   const long No = glu ? N / 2 : N;
 #define HS_SN(XG, NT, DEPTH, GLU, TO, F32, HALF)                                                                                              \
-  launch_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM, HALF>(dim3((No + (GLU ? 16 : HALF ? 8 : 16 * NT) - 1) / (GLU ? 16 : HALF ? 8 : 16 * NT)), out, No, \
+  launch_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM, HALF>(dim3((No + (GLU ? 16 : 16 * NT - 8 * HALF) - 1) / (GLU ? 16 : 16 * NT - 8 * HALF)), out, No, \
                                                          0, 0, x, x_ld, 0, w, bias, M, N, K, act, act_from, c0, c1, s, norm)
 #define HS_SX(NT, D, GLU, TO, F32) \
   (M <= 8 ? HS_SN(1, NT, D, GLU, TO, F32, false) : M <= 16 ? HS_SN(2, NT, D, GLU, TO, F32, false) : HS_SN(4, NT, F32 ? 1 : D, GLU, TO, F32, false))
@@ -170,6 +228,20 @@ static bool launch_normed(void* out, bool out_f32, const SkinnyNorm& norm, const
   // where squares are written, their number says what the workgroups are to take
   if (NORM == kUpdate ? norm.blocks == N / 8 : skinny_half(M, (N + 15) / 16, K))
     return f32 ? HS_SH(float, true) : out_f32 ? HS_SH(Wide, false) : HS_SH(unsigned short, false);
+  if constexpr (NORM == kNormed) {
+    if (const int cols = f32 ? 0 : skinny_cols(M, N, K)) {
+#define HS_SG(NT, HALF, TO) (M <= 16 ? HS_SN(2, NT, 1, false, TO, false, HALF) : HS_SN(4, NT, 1, false, TO, false, HALF))
+#define HS_SO(NT, HALF) (out_f32 ? HS_SG(NT, HALF, Wide) : HS_SG(NT, HALF, unsigned short))
+      return cols == 24 ? HS_SO(2, true) : cols == 40 ? HS_SO(3, true) : cols == 48 ? HS_SO(3, false) : HS_SO(4, true);
+#undef HS_SO
+#undef HS_SG
+    }
+    if (const auto wide = skinny_wide(M, (N + 15) / 16, K, f32); wide.ahead > 0) {
+      if (wide.half) return out_f32 ? HS_SN(1, 1, 2, false, Wide, false, true) : HS_SN(1, 1, 2, false, unsigned short, false, true);
+      return f32 ? HS_SN(1, 1, 3, false, float, true, false) : out_f32 ? HS_SN(1, 1, 3, false, Wide, false, false)
+           : HS_SN(1, 1, 3, false, unsigned short, false, false);
+    }
+  }
   const int nt = skinny_tiles(M, (N + 15) / 16, K);   // 4 above 16 rows alone; where squares are written, N is a multiple of 64
   return nt == 4 ? HS_S4() : nt == 2 ? HS_ST(2, 1, false) : HS_ST(1, 2, false);
 #undef HS_S4

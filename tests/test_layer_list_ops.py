@@ -327,6 +327,39 @@ def test_products_in_half_tiles(M, N, K, dtype):
 
 
 @gpu
+@pytest.mark.parametrize("M,N,K,dtype", [
+    (9, 4097, 2048, "bf16"), (16, 6144, 2056, "bf16"), (17, 6133, 1024, "bf16"), (48, 4104, 1032, "bf16"),    # 24 columns
+    (16, 8193, 3072, "bf16"), (25, 10239, 1096, "bf16"), (33, 8705, 2048, "bf16"),                           # 40
+    (24, 12288, 1024, "bf16"), (41, 10241, 2056, "bf16"), (15, 11264, 3080, "bf16"),                          # 48
+    (10, 12289, 3072, "bf16"), (32, 14329, 3080, "bf16"),                                                     # 56
+    (18, 20473, 1032, "bf16"), (48, 28665, 3072, "bf16"),                                                     # two rounds, of 40 and 56
+    (1, 5648, 2048, "bf16"), (4, 8191, 2048, "bf16"),                                                         # up to 4 rows: half tiles
+    (5, 6145, 2048, "bf16"), (8, 8193, 2568, "bf16"), (3, 8200, 4096, "bf16"), (1, 8193, 1032, "f32"), (7, 6160, 1024, "f32")])   # three pieces ahead
+def test_products_of_many_columns(M, N, K, dtype):
+    """Forms for more workgroups than compute units: the first and last columns have the bits that a product of them alone has, from rows as they are and from
+    rows without their norm's factor; a last workgroup that is partly filled, a bias, an activation from some column on."""
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    g = torch.Generator("cuda").manual_seed(M + N)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g).to(dt)  # noqa: E731
+    x, w, b, ops = rand(M, K), rand(N, K) / 32, rand(N), get_ops("cuda")
+    rows = [x] if K % 64 or M > 32 else [x, NormedRows(x, torch.rand(M, K // 16, device="cuda", generator=g) * 16, 1e-6)]
+    n = 200   # columns that are looked at, at either end
+    for h in rows:
+        if h is x:
+            got, first, last = (torch.empty(M, c, dtype=dt, device="cuda") for c in (N, n, n))
+            for out, a, z, start in ((got, w, b, 50), (first, w[:n], b[:n], 50), (last, w[-n:], b[-n:], 0)):
+                ops._moe_lib.skinny_linear(out, x, a, z, 0, 0.0, 0.0, start)
+        else:
+            got, first, last = (ops.linear(h, a, z, act="tanh", act_from=start) for a, z, start in ((w, b, 50), (w[:n], b[:n], 50), (w[-n:], b[-n:], 0)))
+        assert torch.equal(got[:, :n], first) and torch.equal(got[:, -n:], last)
+        whole = h.normed() if h is not x else x
+        want = torch.mm(whole.float(), w.t().float()) + b.float()
+        want = torch.cat([want[:, :50], torch.tanh(want[:, 50:])], 1)
+        err = (got.float() - want).abs() / (1 + want.abs())
+        assert err.max() < (0.02 if dt == torch.bfloat16 else 1e-4)   # what lies between them: no column left out (a result rounded to 2^-9, of rows rounded to 2^-9; 32-bit sums)
+
+
+@gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,H,K", [(1, 64, 2056), (8, 2048, 4104), (9, 192, 1032), (16, 1024, 3072), (17, 2048, 520), (32, 832, 2048)])
 def test_updates_in_half_tiles(M, H, K, dtype):
