@@ -152,7 +152,9 @@ double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts) {
   const int K = f32 ? 2 * k : k;
   const double out = (double)M * (glu ? cols / 2 : cols) * (f32 ? 4 : 2);
   const long tiles = (cols + 15) / 16 * parts;
-  const int own = !glu && !f32 && parts == 1 ? skinny_cols(M, cols, K) : 0;
+  // (not of two rounds of 56 columns: what this time is compared with for such sizes is an estimate of the vendor's that is up to a fifth too long: 40 rows,
+  // 25600 x 3072, vendor 32.5 us, ours 37.7, estimates 40.7 and, with 56 columns, 38.0; 24 rows 30.8 and 32.8; but 48 rows 47.1 and 39.1)
+  const int own = !glu && !f32 && parts == 1 && cols <= 1280 * 16 ? skinny_cols(M, cols, K) : 0;
   const int per = glu ? 32 : own > 0 ? own : skinny_half(M, tiles, K / parts) ? 8 : 16 * skinny_tiles(M, tiles, K / parts);
   return skinny_time_of(M, cols, K, per, parts, f32, out);
 }
