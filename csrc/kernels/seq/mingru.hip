@@ -183,27 +183,32 @@ struct MinGruArgs {
 
 // y, state of the rows x [M, K], one per sequence, and w = [z rows; x rows; g rows]. F32: x, w, x_ld and K in 16-bit halves (skinny.h).
 // A MinGruRest lies at byte rest_at of the kernel's arguments.
-template <int XG, int DEPTH, bool F32>
+// HALF: 8 channels per workgroup (mingru_half): the z and x rows are the halves of one tile, the g rows half of another, and a channel's x meets its z from 8
+// lanes further. Twice the workgroups, eight rows of weights per load and tile, and two pieces ahead beside the experts, too; the sums are the same. us, cold
+// weights, 16 channels -> 8: one row, 2048 x 2048 8.2 -> 7.5, 4096 x 2048 12.0 -> 10.9, with the experts of a row beside 13.2 -> 12.4, 6144 x 2048 18.3 ->
+// 15.8, 8192 x 4096 38.8 -> 37.3, with experts 44.5 -> 41.7; 16 rows, 2048 x 2048 9.5 -> 8.6.
+template <int XG, int DEPTH, bool F32, bool HALF>
 HS_DEVICE void mingru_block(int wg, const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const MinGruSeqs& seqs, int x_ld, int M,
                             int width, int K, int rest_at, unsigned char* smem) {
-  using SK = Skinny<XG, 3, DEPTH, F32>;
+  using SK = std::conditional_t<HALF, Skinny<XG, 2, DEPTH, F32, true>, Skinny<XG, 3, DEPTH, F32>>;
   using T = std::conditional_t<F32, float, unsigned short>;
-  constexpr int ST = SK::ST, IT = (ST + 1) / 2;
+  constexpr int ST = SK::ST, IT = (ST + 1) / 2, NT = HALF ? 2 : 3, kChannels = HALF ? 8 : 16;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = wg * 16, c = min(n0 + (tid & 15), width - 1);
-  const unsigned char* wt[3];
-  unsigned w_row[6], x_row[XG];
+  const int n0 = wg * kChannels, c = min(n0 + (tid & (kChannels - 1)), width - 1);
+  const unsigned char* wt[NT];
+  unsigned w_row[SK::WG], x_row[XG];
 #pragma unroll
-  for (int nt = 0; nt < 3; ++nt) {
-    wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)nt * width + n0) * K);
+  for (int nt = 0; nt < NT; ++nt) {
+    wt[nt] = reinterpret_cast<const unsigned char*>(w + ((long)(HALF ? 2 * nt : nt) * width + n0) * K);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) w_row[2 * nt + h] = (unsigned)min(8 * h + (lane >> 3), width - 1 - n0) * (unsigned)K * 2;
+    for (int h = 0; h < (HALF && nt == 1 ? 1 : 2); ++h)
+      w_row[2 * nt + h] = (unsigned)(HALF ? h * width + min(lane >> 3, width - 1 - n0) : min(8 * h + (lane >> 3), width - 1 - n0)) * (unsigned)K * 2;
   }
 #pragma unroll
   for (int j = 0; j < XG; ++j) x_row[j] = (unsigned)min(8 * j + (lane >> 3), M - 1) * (unsigned)x_ld * 2;
-  f32x4 acc[3][ST];
+  f32x4 acc[NT][ST];
 #pragma unroll
-  for (int nt = 0; nt < 3; ++nt)
+  for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
     for (int st = 0; st < ST; ++st) acc[nt][st] = f32x4{0.f, 0.f, 0.f, 0.f};
   T* y = nullptr;
@@ -242,25 +247,26 @@ HS_DEVICE void mingru_block(int wg, const unsigned short* __restrict__ x, const 
       S[i] = state[at[i] < 0 ? c : at[i]];
     }
   });
-  float v[3][IT];
+  float v[NT][IT];
   SK::reduce(v, acc, smem);
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
     const int m = (tid + kSkThreads * i) >> 4;
-    if (m >= M || n0 + (tid & 15) >= width || at[i] < 0) continue;
-    const Gru g(v[0][i], v[1][i], bz, bx);
+    const float xv = HALF ? __shfl_xor(v[0][i], 8, 64) : v[1][i], gv = v[NT - 1][i];
+    if (m >= M || n0 + (tid & 15) >= width || at[i] < 0 || (HALF && (tid & 8))) continue;
+    const Gru g(v[0][i], xv, bz, bx);
     const float o = fmaf(g.keep, fresh[i] ? 0.f : S[i], g.zc);   // as the scan has it, in both kernels
-    stf<T>(y, (long)m * width + c, o * (v[2][i] * sigmoid_f(v[2][i])));
+    stf<T>(y, (long)m * width + c, o * (gv * sigmoid_f(gv)));
     state[at[i]] = o;
   }
 }
 
-template <int XG, int DEPTH, bool F32>
+template <int XG, int DEPTH, bool F32, bool HALF>
 __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx,
     const int* __restrict__ seq_state, int x_ld, int M, int width, int K, const MinGruRest) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  mingru_block<XG, DEPTH, F32>(blockIdx.x, x, w, MinGruSeqs{seq_cu, seq_ctx, seq_state}, x_ld, M, width, K, offsetof(MinGruArgs, rest), smem);
+  mingru_block<XG, DEPTH, F32, HALF>(blockIdx.x, x, w, MinGruSeqs{seq_cu, seq_ctx, seq_state}, x_ld, M, width, K, offsetof(MinGruArgs, rest), smem);
 }
 
 struct MinGruBesideArgs {
@@ -270,42 +276,39 @@ struct MinGruBesideArgs {
   ExpertBeside experts;
 };
 
-// The same with the experts' product of tiles with few rows besides (expert_beside.hip): workgroups from `split` on. One piece ahead, so that two workgroups
-// fit a compute unit.
-template <int XG, int DEPTH>
+// The same with the experts' product of tiles with few rows besides (expert_beside.hip): workgroups from `split` on. With 16 channels one piece ahead, so that
+// two workgroups fit a compute unit.
+template <int XG, int DEPTH, bool HALF>
 __global__ __launch_bounds__(kSkThreads) void mingru_product_experts_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const int* __restrict__ slots, const int* __restrict__ tile_expert,
     int x_ld, int M, int width, int K, int split, const MinGruRest, const ExpertBeside) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int b = blockIdx.x;
   if (b >= split) expert_beside(b - split, slots, tile_expert, offsetof(MinGruBesideArgs, experts), smem);
-  else mingru_block<XG, DEPTH, false>(b, x, w, MinGruSeqs{}, x_ld, M, width, K, offsetof(MinGruBesideArgs, rest), smem);
+  else mingru_block<XG, DEPTH, false, HALF>(b, x, w, MinGruSeqs{}, x_ld, M, width, K, offsetof(MinGruBesideArgs, rest), smem);
 }
 
-template <int XG, int DEPTH>
+template <int XG, int DEPTH, bool HALF, bool F32>
 bool launch_product(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x, const int* seq_cu,
-                    const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, bool f32, hipStream_t s) {
-  constexpr int lds = Skinny<XG, 3, DEPTH>::kLds;
-  auto go = [&](auto* kernel) {
-    kernel<<<(width + 15) / 16, kSkThreads, lds, s>>>((const unsigned short*)x, (const unsigned short*)w, seq_cu, seq_ctx, seq_state, (int)x_ld, M,
-                                                       width, K, MinGruRest{y, state, b_z, b_x, nseq, {}});
-  };
-  static const bool ok = allow_lds(&mingru_product_kernel<XG, DEPTH, false>, lds) && allow_lds(&mingru_product_kernel<XG, DEPTH, true>, lds);
+                    const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, hipStream_t s) {
+  constexpr int lds = HALF ? Skinny<XG, 2, DEPTH, F32, true>::kLds : Skinny<XG, 3, DEPTH>::kLds, per = HALF ? 8 : 16;
+  static const bool ok = allow_lds(&mingru_product_kernel<XG, DEPTH, F32, HALF>, lds);
   if (!ok) return false;
-  if (f32) go(&mingru_product_kernel<XG, DEPTH, true>);
-  else go(&mingru_product_kernel<XG, DEPTH, false>);
+  mingru_product_kernel<XG, DEPTH, F32, HALF><<<(width + per - 1) / per, kSkThreads, lds, s>>>(
+      (const unsigned short*)x, (const unsigned short*)w, seq_cu, seq_ctx, seq_state, (int)x_ld, M, width, K, MinGruRest{y, state, b_z, b_x, nseq, {}});
   return true;
 }
 
-template <int XG, int DEPTH>
+template <int XG, int DEPTH, bool HALF>
 bool launch_beside(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x, const int* seq_cu,
                    const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, const ExpertRows& ex, hipStream_t s) {
-  constexpr int own = Skinny<XG, 3, DEPTH>::kLds, lds = own > expert_lds<1>() ? own : expert_lds<1>();
-  static const bool ok = allow_lds(&mingru_product_experts_kernel<XG, DEPTH>, lds);
+  constexpr int own = HALF ? Skinny<XG, 2, DEPTH, false, true>::kLds : Skinny<XG, 3, DEPTH>::kLds, lds = own > expert_lds<1>() ? own : expert_lds<1>();
+  constexpr int per = HALF ? 8 : 16;
+  static const bool ok = allow_lds(&mingru_product_experts_kernel<XG, DEPTH, HALF>, lds);
   if (!ok) return false;
-  const int split = (width + 15) / 16;
+  const int split = (width + per - 1) / per;
   const ExpertBeside experts = expert_beside_args(ex);
-  mingru_product_experts_kernel<XG, DEPTH><<<split + experts.per_tile * ex.ntiles, kSkThreads, lds, s>>>(
+  mingru_product_experts_kernel<XG, DEPTH, HALF><<<split + experts.per_tile * ex.ntiles, kSkThreads, lds, s>>>(
       (const unsigned short*)x, (const unsigned short*)w, ex.slots, ex.tile_expert, (int)x_ld, M, width, K, split,
       MinGruRest{y, state, b_z, b_x, nseq, {seq_cu, seq_ctx, seq_state}}, experts);
   return true;
@@ -329,22 +332,34 @@ void launch(T* y, float* state, const T* proj, const float* b_z, const float* b_
 
 }  // namespace
 
+// Whether workgroups take 8 channels (mingru_block): where 16 leave half of the compute units idle, and, for up to 4 rows, where either has the units full and k
+// is long; not between the two, where 16 are one round and 8 nearly two (3000 x 2048, one row 9.7 -> 9.9 us), nor for more rows, which are read twice as often
+// then (8192 x 4096, 16 rows 39.2 -> 42.2; with experts beside 4096 x 2048, 8 rows 20.3 -> 21.3). Offsets within a workgroup's rows have 32 bits.
+static bool mingru_half(int M, int width, int K) {
+  if (M > 16 || 4L * (width + 8) * K >= (1L << 32)) return false;
+  return width <= 2048 ? width > 1024 && K >= 1024 : M <= 4 && width >= 4096 && K >= 2048;
+}
+
 bool launch_mingru_product(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x,
                            const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K, bool f32,
                            hipStream_t s) {
   if (M <= 0 || nseq <= 0 || width <= 0) return true;
   if (f32) { x_ld *= 2; K *= 2; }   // in halves
-#define HS_MG(XG, DEPTH) launch_product<XG, DEPTH>(y, state, x, x_ld, w, b_z, b_x, seq_cu, seq_ctx, seq_state, nseq, M, width, K, f32, s)
+#define HS_MH(XG, DEPTH, HALF, F32) launch_product<XG, DEPTH, HALF, F32>(y, state, x, x_ld, w, b_z, b_x, seq_cu, seq_ctx, seq_state, nseq, M, width, K, s)
+#define HS_MG(XG, DEPTH) (f32 ? HS_MH(XG, DEPTH, false, true) : HS_MH(XG, DEPTH, false, false))
+  if (!f32 && mingru_half(M, width, K)) return M <= 8 ? HS_MH(1, 2, true, false) : HS_MH(2, 2, true, false);
   return M <= 8 ? HS_MG(1, 2) : M <= 16 ? HS_MG(2, 2) : M <= 32 ? HS_MG(4, 1) : M <= 48 ? HS_MG(6, 1) : HS_MG(8, 1);
 #undef HS_MG
+#undef HS_MH
 }
 
 bool launch_mingru_product_experts(void* y, float* state, const void* x, long x_ld, const void* w, const float* b_z, const float* b_x,
                                    const int* seq_cu, const int* seq_ctx, const int* seq_state, int nseq, int M, int width, int K,
                                    const ExpertRows& ex, hipStream_t s) {
   if (M <= 0 || nseq <= 0 || width <= 0 || M > 32 || !expert_rows_ok(ex)) return false;   // more rows: 96 KB, the experts would have a compute unit's LDS to themselves each
-#define HS_MG(XG, DEPTH) launch_beside<XG, DEPTH>(y, state, x, x_ld, w, b_z, b_x, seq_cu, seq_ctx, seq_state, nseq, M, width, K, ex, s)
-  return M <= 8 ? HS_MG(1, 1) : M <= 16 ? HS_MG(2, 1) : HS_MG(4, 1);
+#define HS_MG(XG, DEPTH, HALF) launch_beside<XG, DEPTH, HALF>(y, state, x, x_ld, w, b_z, b_x, seq_cu, seq_ctx, seq_state, nseq, M, width, K, ex, s)
+  if (mingru_half(M, width, K)) return M <= 8 ? HS_MG(1, 2, true) : HS_MG(2, 2, true);
+  return M <= 8 ? HS_MG(1, 1, false) : M <= 16 ? HS_MG(2, 1, false) : HS_MG(4, 1, false);
 #undef HS_MG
 }
 

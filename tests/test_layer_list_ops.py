@@ -763,6 +763,25 @@ def test_mingru_product(M, width, K, gaps, dtype):
 
 
 @gpu
+@pytest.mark.parametrize("M,width,K", [(1, 2048, 1024), (3, 4101, 2056), (4, 4096, 2048), (8, 1030, 1032), (9, 2041, 2048), (16, 1999, 1096)])
+def test_mingru_product_of_8_channels(M, width, K):
+    """Workgroups of 8 channels for up to 16 rows: the bits that the same rows have among more of them, which take 16; a last workgroup that is partly filled, k
+    past a whole piece, a sequence without a row."""
+    g = torch.Generator("cuda").manual_seed(M + width)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g)  # noqa: E731
+    x, w, state, bz, bx = rand(20, K).bfloat16(), (rand(3 * width, K) / K ** 0.5).bfloat16(), rand(24, width), rand(width), rand(width)
+    seq = torch.randperm(24, device="cuda", generator=g)[:21].int()
+    cu = torch.tensor([0, 0, *range(1, 21)], dtype=torch.int32, device="cuda")   # the first sequence has no row
+    ctx = torch.arange(21, dtype=torch.int32, device="cuda") % 3 + 1
+    outs = []
+    for n in (M, 20):
+        y, s = torch.full((n, width), float("nan"), dtype=torch.bfloat16, device="cuda"), state.clone()
+        get_ops("cuda")._seq.mingru_product(y, s, x[:n], w, bz, bx, cu[:n + 2], ctx[:n + 1], seq[:n + 1])
+        outs.append((y[:M], s[seq[1:M + 1].long()], s[seq[:1].long()]))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
+@gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("width", [4, 260, 1028, 6])
 @pytest.mark.parametrize("lens", [[1], [1, 1, 1], [17], [16, 1, 256], [1, 300, 63]])
