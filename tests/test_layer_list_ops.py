@@ -359,6 +359,31 @@ def test_products_of_many_columns(M, N, K, dtype):
         assert err.max() < (0.02 if dt == torch.bfloat16 else 1e-4)   # what lies between them: no column left out (a result rounded to 2^-9, of rows rounded to 2^-9; 32-bit sums)
 
 
+@pytest.mark.parametrize("rows,cols,cut", [
+    (8192, 6176, 6144), (8192, 26688, 26624), (7900, 4128, 4096), (2048, 8200, 8192), (1024, 16512, 16384), (1100, 13072, 13056),   # a round for few columns
+    (8192, 6144, 0), (8192, 13376, 0), (8192, 6148, 0), (8192, 6288, 0), (7900, 6176, 0), (1000, 16400, 0), (3133, 15120, 0), (6144, 13584, 0), (8192, 200, 0), (0, 6176, 0)])
+def test_columns_that_would_start_a_round(rows, cols, cut):
+    from hipserve.ops import KernelOps
+
+    assert KernelOps._round_columns(rows, cols) == cut
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("rows,cols,K,grad", [(1024, 16400, 72, False), (1100, 13072, 40, True)])
+def test_products_in_whole_rounds(rows, cols, K, grad, device):
+    """A long prompt's product in two: rows and weights at strides of their own, and one product where a gradient is asked for."""
+    from hipserve.ops import KernelOps
+
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, K + 8, generator=g).bfloat16().to(device)[:, 8:]
+    w = torch.randn(2 * cols, K, generator=g).bfloat16().to(device)[::2].requires_grad_(grad)
+    y = KernelOps()._vendor_linear(x, w, None)
+    assert y.requires_grad == grad and y.is_contiguous()
+    want = x.float() @ w.detach().float().t()
+    # rounded to 2^-9, and sums of K products in 32 bits
+    assert ((y.detach().float() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -23 * (x.float().abs() @ w.detach().float().abs().t())).all()
+
+
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,H,K", [(1, 64, 2056), (8, 2048, 4104), (9, 192, 1032), (16, 1024, 3072), (17, 2048, 520), (32, 832, 2048)])
