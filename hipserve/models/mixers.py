@@ -866,6 +866,7 @@ class ParallelMixer:
         self.b_in = None     # its biases, where a half has them
         self.split = 0       # rows of w_in before the right half's
         self.in_act = {}     # its activation: the right half's, on the last columns
+        self.left_biased = False   # whether the left half alone has biases
 
     @property
     def cache_dim(self) -> int:
@@ -892,6 +893,7 @@ class ParallelMixer:
             self.split = -(-wl.shape[0] // 8) * 8   # 16-byte aligned rows in bf16
             self.w_in = torch.cat([F.pad(wl, (0, 0, 0, self.split - wl.shape[0])), wr], 0).contiguous()
             if bl is not None or br is not None:
+                self.left_biased = br is None
                 self.b_in = wl.new_zeros(self.w_in.shape[0])
                 for at, b in ((0, bl), (self.split, br)):
                     if b is not None:
@@ -908,11 +910,19 @@ class ParallelMixer:
             t.update({n + ".out": 1.0 + 0.2 * _rand(gen, self.hidden) for n in ("left", "right")})
         return t
 
+    def _project(self, h):
+        """The halves' input projections of rows ``h``: parts of one product, or, in long prompts whose right half without biases goes
+        in whole rounds (``ops.in_rounds``), one each. (A product with biases cannot be cut where rounds end: the library adds them in a pass of its own then.)"""
+        if self.left_biased and self.ops.in_rounds(h, self.w_in.shape[0] - self.split):
+            act = dict(self.in_act, act_from=self.in_act["act_from"] - self.split) if self.in_act else {}
+            return self.ops.linear(h, self.w_in[:self.split], self.b_in[:self.split]), self.ops.linear(h, self.w_in[self.split:], **act)
+        proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)
+        return proj[:, :self.split], proj[:, self.split:]
+
     def _forward_normed(self, h, meta, cache, state):
         pl = pr = None
         if self.w_in is not None:
-            proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)
-            pl, pr = proj[:, :self.split], proj[:, self.split:]
+            pl, pr = self._project(h)
         ys = []
         for m, p in ((self.left, pl), (self.right, pr)):
             out = torch.empty(h.shape[0], m.out_size, device=h.device, dtype=h.dtype)
@@ -926,10 +936,10 @@ class ParallelMixer:
         a, b = self.left.out_size, self.right.out_size
         buf = torch.empty(h.shape[0], a + b, device=h.device, dtype=h.dtype)
         if self.w_in is not None:
-            proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)
-            right = (state, buf[:, a:], self.spec.right_scale, proj[:, self.split:])
+            pl, pr = self._project(h)
+            right = (state, buf[:, a:], self.spec.right_scale, pr)
             beside = self.right.beside(meta, *right) if isinstance(self.left, WindowAttention) and isinstance(self.right, DeltaRule) else None
-            self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale, proj[:, :self.split], **({} if beside is None else {"beside": beside}))
+            self.left.mix(h, meta, cache, state, buf[:, :a], self.spec.left_scale, pl, **({} if beside is None else {"beside": beside}))
             if beside is None or not beside.taken:
                 self.right.mix(h, meta, cache, *right)
             return _last(self, buf, self.w_o, None, update)

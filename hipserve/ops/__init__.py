@@ -760,8 +760,12 @@ class KernelOps:
         more = -(-tiles * (whole + 1) // 256) > -(-now // 256)
         return 256 * whole if more and (now % 256 == 0 or now <= 512) else 0
 
+    def in_rounds(self, x, cols) -> bool:
+        """Whether a product of rows x onto so many columns is cut where rounds end (``_round_columns``)."""
+        return isinstance(x, torch.Tensor) and x.dim() == 2 and x.dtype == torch.bfloat16 and self._round_columns(x.shape[0], cols) > 0
+
     def _vendor_linear(self, x, w, bias):
-        cut = self._round_columns(x.shape[0], w.shape[0]) if x.dim() == 2 and x.dtype == w.dtype == torch.bfloat16 and bias is None else 0
+        cut = self._round_columns(x.shape[0], w.shape[0]) if bias is None and w.dtype == torch.bfloat16 and self.in_rounds(x, w.shape[0]) else 0
         if cut == 0 or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
             return F.linear(x, w, bias)
         y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
@@ -1030,6 +1034,9 @@ class ReferenceOps:
     """PyTorch reference path (CPU plumbing engine / numerics oracle)."""
 
     name = "reference"
+
+    def in_rounds(self, x, cols) -> bool:
+        return False
 
     def fill_uniform(self, out, row0, col0, gcols, key, scale):
         return ref.fill_uniform(out, row0, col0, gcols, key, scale)

@@ -384,6 +384,27 @@ def test_products_in_whole_rounds(rows, cols, K, grad, device):
     assert ((y.detach().float() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -23 * (x.float().abs() @ w.detach().float().abs().t())).all()
 
 
+def test_halves_projected_apart():
+    """A parallel mixer whose left half has biases and whose right half ends with an activation: two products give what parts of one do."""
+    from hipserve.models.mixers import ParallelMixer
+
+    def linear(x, w, bias=None, act=None, act_from=0):
+        y = torch.nn.functional.linear(x, w, bias)
+        return y if act is None else torch.cat([y[:, :act_from], torch.tanh(y[:, act_from:])], 1)
+
+    g = torch.Generator().manual_seed(3)
+    x, outs = torch.randn(5, 16, generator=g, dtype=torch.float64), []
+    for apart in (False, True):
+        m = ParallelMixer.__new__(ParallelMixer)
+        m.w_in, m.b_in = (torch.randn(*s, generator=torch.Generator().manual_seed(4), dtype=torch.float64) for s in ((40, 16), (40,)))
+        m.split, m.left_biased, m.in_act = 24, True, dict(act="tanh", act_from=36)
+        m.b_in[24:] = 0
+        m.ops = SimpleNamespace(linear=linear, in_rounds=lambda x, cols: apart and cols == 16)
+        outs.append(m._project(x))
+    for a, b in zip(*outs):
+        assert a.shape == b.shape and torch.allclose(a, b, rtol=1e-12)
+
+
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,H,K", [(1, 64, 2056), (8, 2048, 4104), (9, 192, 1032), (16, 1024, 3072), (17, 2048, 520), (32, 832, 2048)])
