@@ -386,6 +386,8 @@ def test_products_in_whole_rounds(rows, cols, K, grad, device):
 
 def test_halves_projected_apart():
     """A parallel mixer whose left half has biases and whose right half ends with an activation: two products give what parts of one do."""
+    from types import SimpleNamespace
+
     from hipserve.models.mixers import ParallelMixer
 
     def linear(x, w, bias=None, act=None, act_from=0):
