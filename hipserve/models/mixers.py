@@ -111,13 +111,13 @@ def _last(sub, x: torch.Tensor, w: torch.Tensor, b=None, update=None, beside=Non
     itself and return the next sublayer's ``NormedRows``; ``beside``: an ``ops.ExpertSteps`` whose next product may go into the launch; ``conv``:
     an ``ops.ConvBeside`` that an update's launch may take."""
     if update is not None:
-        rows = sub.ops.linear_update(x, w, b, *update, conv=conv)
+        rows = sub.ops.linear_update(x, w, b, *update, *(() if conv is None else (conv,)))
         if conv is not None:
             conv.finish()
         if rows is not None:
             return rows
     linear = sub.ops.linear_parts if getattr(sub, "takes_parts", False) else sub.ops.linear
-    return linear(x, w, b, beside=beside)
+    return linear(x, w, b) if beside is None else linear(x, w, b, beside=beside)
 
 
 def _deinterleave(w: torch.Tensor, dims: int) -> torch.Tensor:
