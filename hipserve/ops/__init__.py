@@ -19,6 +19,7 @@ import threading
 import torch
 import torch.nn.functional as F
 
+from . import gemm
 from . import reference as ref
 
 _PKG = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -746,32 +747,13 @@ class KernelOps:
         out = torch.empty(*y.shape[:-1], y.shape[-1] // 2, device=y.device, dtype=y.dtype) if act in self.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)
 
-    @staticmethod
-    def _round_columns(rows, cols) -> int:
-        """The columns of a long prompt's product that the vendor's tiles of 256 x 256 take in whole rounds over the compute units, where the few columns behind
-        them (gates of a head each) would start a round of their own; else 0. The columns behind them then are a product of their own, which reads the rows
-        once more (10 - 20 us for 8192), where a round is 44 us of k 2048. Of 160 such sizes (1024 - 8192 rows, 1040 - 26752 columns, k 1024 - 4096, 16 - 128 columns
-        behind) every one got faster, 19 % on average; us, one product -> two, 8192 rows: 6160 x 2048 222 -> 156, 6208 x 4096 373 -> 277, 26688 x 2048 683 -> 611, 2048
-        rows: 8208 x 4096, 0.73 of the time. Where the whole tiles themselves are neither full rounds nor up to two of them, some lose: 3133 rows of 15120 x 1024 104 -> 120."""
-        tiles, whole, behind = -(-rows // 256), cols // 256, cols % 256
-        if not (rows >= 1024 and cols % 8 == 0 and 0 < behind <= 128 and whole):
-            return 0
-        now = tiles * whole
-        more = -(-tiles * (whole + 1) // 256) > -(-now // 256)
-        return 256 * whole if more and (now % 256 == 0 or now <= 512) else 0
-
     def in_rounds(self, x, cols) -> bool:
-        """Whether a product of rows x onto so many columns is cut where rounds end (``_round_columns``)."""
-        return isinstance(x, torch.Tensor) and x.dim() == 2 and x.dtype == torch.bfloat16 and self._round_columns(x.shape[0], cols) > 0
+        """Whether a product of rows x onto so many columns is cut before the last of them (``gemm.round_columns``)."""
+        return isinstance(x, torch.Tensor) and x.dim() == 2 and x.dtype == torch.bfloat16 and gemm.round_columns(x.shape[0], cols) > 0
 
     def _vendor_linear(self, x, w, bias):
-        cut = self._round_columns(x.shape[0], w.shape[0]) if bias is None and w.dtype == torch.bfloat16 and self.in_rounds(x, w.shape[0]) else 0
-        if cut == 0 or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
-            return F.linear(x, w, bias)
-        y = torch.empty(x.shape[0], w.shape[0], device=x.device, dtype=x.dtype)
-        torch.mm(x, w[:cut].t(), out=y[:, :cut])
-        torch.mm(x, w[cut:].t(), out=y[:, cut:])
-        return y
+        y = gemm.linear_in_rounds(x, w) if bias is None and x.dim() == 2 else None
+        return F.linear(x, w, bias) if y is None else y
 
     def _skinny_linear(self, x, w, bias, out_f32=False, act=None, c0=0.0, c1=0.0, act_from=0):
         out = torch.empty(x.shape[0], w.shape[0] // 2 if act in self.GLU_ACTS else w.shape[0], device=x.device,

@@ -12,6 +12,7 @@ real decode step streams from HBM once per layer.
 from __future__ import annotations
 
 import logging
+import math
 import weakref
 
 import torch
@@ -523,6 +524,54 @@ def packed_glu(x: torch.Tensor, w: PackedLinear, gelu: bool = False) -> torch.Te
     return packed_prefill(x, w, 3 if gelu else 2)
 
 
+# Long prompts' products in whole rounds. The vendor's kernels take tiles of 256 x 256, a round of them on the 256 compute units at a time, and a few tiles more than
+# whole rounds cost up to a round (about 21 us per 1000 k) or more: as a product of their own they run in smaller tiles, or over parts of k.
+def round_columns(rows: int, cols: int) -> int:
+    """Columns in whole tiles, where the few columns behind them (gates of a head each) would start a round of their own; else 0. The second product reads the rows
+    once more (10 - 20 us for 8192), where a round is 44 us of k 2048. Of 160 such sizes (1024 - 8192 rows, 1040 - 26752 columns, k 1024 - 4096, 16 - 128 columns
+    behind) every one got faster, 19 % on average; us, one product -> two, 8192 rows: 6160 x 2048 222 -> 156, 6208 x 4096 373 -> 277, 26688 x 2048 683 -> 611, 2048
+    rows: 8208 x 4096, 0.73 of the time. Where the whole tiles themselves are neither full rounds nor up to two of them, some lose: 3133 rows of 15120 x 1024 104 -> 120."""
+    tiles, whole, behind = -(-rows // 256), cols // 256, cols % 256
+    if not (rows >= 1024 and cols % 8 == 0 and 0 < behind <= 128 and whole):
+        return 0
+    now = tiles * whole
+    more = -(-tiles * (whole + 1) // 256) > -(-now // 256)
+    return 256 * whole if more and (now % 256 == 0 or now <= 512) else 0
+
+
+def round_rows(rows: int, cols: int, k: int) -> int:
+    """Rows whose tiles are whole rounds, where the others leave the last round up to three eighths full; else 0. Of 127 such sizes (2048 - 8192 rows, 4096 - 28672
+    columns, k 2048 - 14336) two products take 13 % less on average, at most 2.4 % more. us, one -> two: 5142 rows of 4096 x 14336 824 -> 417, 4200 of 4096 x
+    12288 621 -> 287, 4200 of 12288 x 4096 397 -> 287, 6500 of 28672 x 4096 1154 -> 1031, 5600 of 12288 x 4096 417 -> 401, 7500 of 24576 x 2048 the same. Not
+    for a fuller last round (5700 rows of 4096 x 12288 407 -> 542), shorter k (3510 of 24576 x 1024 152 -> 157), few rows (1040 of 16384 x 8192 241 -> 316), or
+    many behind (7000 of 12288 x 2048 253 -> 264)."""
+    tm, tn = -(-rows // 256), cols // 256
+    if not (2048 < rows <= 8192 and cols > 0 and cols % 256 == 0 and k >= 2048 and 0 < tm * tn % 256 <= 96):
+        return 0
+    whole = 256 // math.gcd(tn, 256)   # row tiles of a whole number of rounds
+    cut = (tm - 1) // whole * whole
+    return 256 * cut if 8 <= cut and tm - cut <= 10 else 0
+
+
+def linear_in_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
+    """x W^T of rows [M, K] in two products of whole rounds and of what lies behind them, or None where it is one (also where gradients are recorded: the
+    products write into parts of the result)."""
+    M, N = x.shape[0], w.shape[0]
+    if M < 1024 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or torch.is_grad_enabled():
+        return None
+    cols, rows = round_columns(M, N), round_rows(M, N, w.shape[1])
+    if not cols and not rows:
+        return None
+    y = torch.empty(M, N, device=x.device, dtype=x.dtype)
+    if cols:
+        torch.mm(x, w[:cols].t(), out=y[:, :cols])
+        torch.mm(x, w[cols:].t(), out=y[:, cols:])
+    else:
+        torch.mm(x[:rows], w.t(), out=y[:rows])
+        torch.mm(x[rows:], w.t(), out=y[rows:])
+    return y
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     if isinstance(w, PackedLinear):
         return packed_linear(x, w)
@@ -532,4 +581,5 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         if c != "blas" and x.stride(1) == 1 and x.stride(0) % 8 == 0:
             out = torch.empty(M, w.shape[0], device=x.device, dtype=x.dtype)
             return run_choice(c, out, x, w)
-    return F.linear(x, w)
+    y = linear_in_rounds(x, w) if x.is_cuda and x.dim() == 2 else None
+    return F.linear(x, w) if y is None else y

@@ -363,13 +363,23 @@ def test_products_of_many_columns(M, N, K, dtype):
     (8192, 6176, 6144), (8192, 26688, 26624), (7900, 4128, 4096), (2048, 8200, 8192), (1024, 16512, 16384), (1100, 13072, 13056),   # a round for few columns
     (8192, 6144, 0), (8192, 13376, 0), (8192, 6148, 0), (8192, 6288, 0), (7900, 6176, 0), (1000, 16400, 0), (3133, 15120, 0), (6144, 13584, 0), (8192, 200, 0), (0, 6176, 0)])
 def test_columns_that_would_start_a_round(rows, cols, cut):
-    from hipserve.ops import KernelOps
+    from hipserve.ops.gemm import round_columns
 
-    assert KernelOps._round_columns(rows, cols) == cut
+    assert round_columns(rows, cols) == cut
+
+
+@pytest.mark.parametrize("rows,cols,k,cut", [
+    (5142, 4096, 14336, 4096), (4097, 4096, 2048, 4096), (2713, 24576, 4096, 2048), (6500, 28672, 4096, 4096), (7310, 16384, 2048, 7168),
+    (4096, 4096, 14336, 0), (5700, 4096, 12288, 0), (7000, 12288, 2048, 0), (3510, 24576, 1024, 0), (1040, 16384, 8192, 0), (5142, 4104, 14336, 0), (9000, 4096, 4096, 0),
+    (5142, 6144, 4096, 0), (0, 4096, 4096, 0), (5142, 0, 4096, 0)])
+def test_rows_that_would_start_a_round(rows, cols, k, cut):
+    from hipserve.ops.gemm import round_rows
+
+    assert round_rows(rows, cols, k) == cut
 
 
 @pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
-@pytest.mark.parametrize("rows,cols,K,grad", [(1024, 16400, 72, False), (1100, 13072, 40, True)])
+@pytest.mark.parametrize("rows,cols,K,grad", [(1024, 16400, 72, False), (1100, 13072, 40, True), (2049, 8192, 2048, False), (4100, 4096, 2056, False)])
 def test_products_in_whole_rounds(rows, cols, K, grad, device):
     """A long prompt's product in two: rows and weights at strides of their own, and one product where a gradient is asked for."""
     from hipserve.ops import KernelOps
@@ -377,7 +387,8 @@ def test_products_in_whole_rounds(rows, cols, K, grad, device):
     g = torch.Generator().manual_seed(rows)
     x = torch.randn(rows, K + 8, generator=g).bfloat16().to(device)[:, 8:]
     w = torch.randn(2 * cols, K, generator=g).bfloat16().to(device)[::2].requires_grad_(grad)
-    y = KernelOps()._vendor_linear(x, w, None)
+    with torch.set_grad_enabled(grad):
+        y = KernelOps()._vendor_linear(x, w, None)
     assert y.requires_grad == grad and y.is_contiguous()
     want = x.float() @ w.detach().float().t()
     # rounded to 2^-9, and sums of K products in 32 bits
