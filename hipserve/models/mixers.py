@@ -911,9 +911,9 @@ class ParallelMixer:
         return t
 
     def _project(self, h):
-        """The halves' input projections of rows ``h``: parts of one product, or, in long prompts whose right half without biases goes
-        in whole rounds (``ops.in_rounds``), one each. (A product with biases cannot be cut where rounds end: the library adds them in a pass of its own then.)"""
-        if self.left_biased and self.ops.in_rounds(h, self.w_in.shape[0] - self.split):
+        """The halves' input projections of rows ``h``: parts of one product, or, in long prompts whose right half without biases can be cut
+        where rounds end (``ops.in_rounds``), one each. (A product with biases cannot be cut where rounds end: the library adds them in a pass of its own then.)"""
+        if self.left_biased and self.ops.in_rounds(h, self.split, self.w_in.shape[0] - self.split):
             act = dict(self.in_act, act_from=self.in_act["act_from"] - self.split) if self.in_act else {}
             return self.ops.linear(h, self.w_in[:self.split], self.b_in[:self.split]), self.ops.linear(h, self.w_in[self.split:], **act)
         proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)

@@ -747,9 +747,11 @@ class KernelOps:
         out = torch.empty(*y.shape[:-1], y.shape[-1] // 2, device=y.device, dtype=y.dtype) if act in self.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)
 
-    def in_rounds(self, x, cols) -> bool:
-        """Whether a product of rows x onto so many columns is cut before the last of them (``gemm.round_columns``)."""
-        return isinstance(x, torch.Tensor) and x.dim() == 2 and x.dtype == torch.bfloat16 and gemm.round_columns(x.shape[0], cols) > 0
+    def in_rounds(self, x, before, cols) -> bool:
+        """Whether rows x onto ``before`` columns are whole rounds of the vendor's tiles, and a product onto so many further ones is cut where rounds end
+        (``gemm.round_columns``)."""
+        return (isinstance(x, torch.Tensor) and x.dim() == 2 and x.dtype == torch.bfloat16 and before % 256 == 0 and -(-x.shape[0] // 256) * before // 256 % 256 == 0
+                and gemm.round_columns(x.shape[0], cols, x.shape[1]) > 0)
 
     def _vendor_linear(self, x, w, bias):
         y = gemm.linear_in_rounds(x, w) if bias is None and x.dim() == 2 else None
@@ -1017,7 +1019,7 @@ class ReferenceOps:
 
     name = "reference"
 
-    def in_rounds(self, x, cols) -> bool:
+    def in_rounds(self, x, before, cols) -> bool:
         return False
 
     def fill_uniform(self, out, row0, col0, gcols, key, scale):

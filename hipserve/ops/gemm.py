@@ -526,17 +526,29 @@ def packed_glu(x: torch.Tensor, w: PackedLinear, gelu: bool = False) -> torch.Te
 
 # Long prompts' products in whole rounds. The vendor's kernels take tiles of 256 x 256, a round of them on the 256 compute units at a time, and a few tiles more than
 # whole rounds cost up to a round (about 21 us per 1000 k) or more: as a product of their own they run in smaller tiles, or over parts of k.
-def round_columns(rows: int, cols: int) -> int:
-    """Columns in whole tiles, where the few columns behind them (gates of a head each) would start a round of their own; else 0. The second product reads the rows
-    once more (10 - 20 us for 8192), where a round is 44 us of k 2048. Of 160 such sizes (1024 - 8192 rows, 1040 - 26752 columns, k 1024 - 4096, 16 - 128 columns
-    behind) every one got faster, 19 % on average; us, one product -> two, 8192 rows: 6160 x 2048 222 -> 156, 6208 x 4096 373 -> 277, 26688 x 2048 683 -> 611, 2048
-    rows: 8208 x 4096, 0.73 of the time. Where the whole tiles themselves are neither full rounds nor up to two of them, some lose: 3133 rows of 15120 x 1024 104 -> 120."""
+def round_columns(rows: int, cols: int, k: int) -> int:
+    """Columns whose tiles are whole rounds, or up to two of them, where the columns behind them would start a round; else 0. Either up to 128 columns (gates of a head
+    each): of 160 such sizes (1024 - 8192 rows, 1040 - 26752 columns, k 1024 - 4096) every one got faster as two products, 19 % on average. Or, from k
+    2048 on, so many that the last round is up to three eighths full: of 93 such sizes (2048 - 8192 rows, k up to 8192) 20 % on average, at most 0.6 % slower.
+    The second product reads the rows once more (10 - 20 us for 8192). us, one -> two, 8192 rows: 6160 x 2048 222 -> 156, 6208 x 4096 373 -> 277, 2656 x 4096 283 ->
+    137, 8960 x 4096 404 -> 406, 2048 rows: 10304 x 4096 209 -> 134. Where the whole tiles themselves are neither full rounds nor up to two of them, some
+    lose: 3133 rows of 15120 x 1024 104 -> 120."""
     tiles, whole, behind = -(-rows // 256), cols // 256, cols % 256
-    if not (rows >= 1024 and cols % 8 == 0 and 0 < behind <= 128 and whole):
+    if rows < 1024 or cols % 8:
         return 0
-    now = tiles * whole
-    more = -(-tiles * (whole + 1) // 256) > -(-now // 256)
-    return 256 * whole if more and (now % 256 == 0 or now <= 512) else 0
+    now, more = tiles * whole, tiles * -(-cols // 256)
+    if whole and 0 < behind <= 128 and -(-more // 256) > -(-now // 256) and (now % 256 == 0 or now <= 512):
+        return 256 * whole
+    return 256 * _cut(-(-cols // 256), tiles) if k >= 2048 and 2048 <= rows <= 8192 else 0
+
+
+def _cut(tiles: int, across: int) -> int:
+    """Of ``tiles`` x ``across`` tiles whose last round is up to three eighths full: how many of the first are whole rounds, with up to ten behind them, or 0."""
+    if not 0 < tiles * across % 256 <= 96:
+        return 0
+    step = 256 // math.gcd(across, 256)
+    cut = (tiles - 1) // step * step
+    return cut if tiles - cut <= 10 else 0
 
 
 def round_rows(rows: int, cols: int, k: int) -> int:
@@ -545,12 +557,10 @@ def round_rows(rows: int, cols: int, k: int) -> int:
     12288 621 -> 287, 4200 of 12288 x 4096 397 -> 287, 6500 of 28672 x 4096 1154 -> 1031, 5600 of 12288 x 4096 417 -> 401, 7500 of 24576 x 2048 the same. Not
     for a fuller last round (5700 rows of 4096 x 12288 407 -> 542), shorter k (3510 of 24576 x 1024 152 -> 157), few rows (1040 of 16384 x 8192 241 -> 316), or
     many behind (7000 of 12288 x 2048 253 -> 264)."""
-    tm, tn = -(-rows // 256), cols // 256
-    if not (2048 < rows <= 8192 and cols > 0 and cols % 256 == 0 and k >= 2048 and 0 < tm * tn % 256 <= 96):
+    if not (2048 < rows <= 8192 and cols % 256 == 0 and k >= 2048):
         return 0
-    whole = 256 // math.gcd(tn, 256)   # row tiles of a whole number of rounds
-    cut = (tm - 1) // whole * whole
-    return 256 * cut if 8 <= cut and tm - cut <= 10 else 0
+    cut = _cut(-(-rows // 256), cols // 256)
+    return 256 * cut if cut >= 8 else 0
 
 
 def linear_in_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
@@ -559,7 +569,7 @@ def linear_in_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
     M, N = x.shape[0], w.shape[0]
     if M < 1024 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or torch.is_grad_enabled():
         return None
-    cols, rows = round_columns(M, N), round_rows(M, N, w.shape[1])
+    cols, rows = round_columns(M, N, w.shape[1]), round_rows(M, N, w.shape[1])
     if not cols and not rows:
         return None
     y = torch.empty(M, N, device=x.device, dtype=x.dtype)

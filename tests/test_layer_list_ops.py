@@ -359,13 +359,15 @@ def test_products_of_many_columns(M, N, K, dtype):
         assert err.max() < (0.02 if dt == torch.bfloat16 else 1e-4)   # what lies between them: no column left out (a result rounded to 2^-9, of rows rounded to 2^-9; 32-bit sums)
 
 
-@pytest.mark.parametrize("rows,cols,cut", [
-    (8192, 6176, 6144), (8192, 26688, 26624), (7900, 4128, 4096), (2048, 8200, 8192), (1024, 16512, 16384), (1100, 13072, 13056),   # a round for few columns
-    (8192, 6144, 0), (8192, 13376, 0), (8192, 6148, 0), (8192, 6288, 0), (7900, 6176, 0), (1000, 16400, 0), (3133, 15120, 0), (6144, 13584, 0), (8192, 200, 0), (0, 6176, 0)])
-def test_columns_that_would_start_a_round(rows, cols, cut):
+@pytest.mark.parametrize("rows,cols,k,cut", [
+    (8192, 6176, 1024, 6144), (8192, 26688, 4096, 26624), (7900, 4128, 2048, 4096), (2048, 8200, 1024, 8192), (1024, 16512, 64, 16384), (1100, 13072, 64, 13056),
+    (8192, 2656, 4096, 2048), (8192, 6288, 2048, 6144), (2048, 10304, 2048, 8192), (4073, 13376, 4096, 12288),   # some columns more
+    (8192, 6144, 2048, 0), (8192, 13376, 2048, 0), (8192, 6148, 2048, 0), (8192, 6288, 1024, 0), (1000, 16400, 2048, 0), (3133, 15120, 2048, 0), (6144, 13584, 2048, 0),
+    (8192, 200, 2048, 0), (0, 6176, 2048, 0), (5142, 0, 4096, 0), (8448, 2656, 4096, 0)])
+def test_columns_that_would_start_a_round(rows, cols, k, cut):
     from hipserve.ops.gemm import round_columns
 
-    assert round_columns(rows, cols) == cut
+    assert round_columns(rows, cols, k) == cut
 
 
 @pytest.mark.parametrize("rows,cols,k,cut", [
@@ -379,7 +381,7 @@ def test_rows_that_would_start_a_round(rows, cols, k, cut):
 
 
 @pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
-@pytest.mark.parametrize("rows,cols,K,grad", [(1024, 16400, 72, False), (1100, 13072, 40, True), (2049, 8192, 2048, False), (4100, 4096, 2056, False)])
+@pytest.mark.parametrize("rows,cols,K,grad", [(1024, 16400, 72, False), (1100, 13072, 40, True), (2049, 8192, 2048, False), (4100, 4096, 2056, False), (2050, 9736, 2048, False)])
 def test_products_in_whole_rounds(rows, cols, K, grad, device):
     """A long prompt's product in two: rows and weights at strides of their own, and one product where a gradient is asked for."""
     from hipserve.ops import KernelOps
@@ -412,7 +414,7 @@ def test_halves_projected_apart():
         m.w_in, m.b_in = (torch.randn(*s, generator=torch.Generator().manual_seed(4), dtype=torch.float64) for s in ((40, 16), (40,)))
         m.split, m.left_biased, m.in_act = 24, True, dict(act="tanh", act_from=36)
         m.b_in[24:] = 0
-        m.ops = SimpleNamespace(linear=linear, in_rounds=lambda x, cols: apart and cols == 16)
+        m.ops = SimpleNamespace(linear=linear, in_rounds=lambda x, before, cols: apart and (before, cols) == (24, 16))
         outs.append(m._project(x))
     for a, b in zip(*outs):
         assert a.shape == b.shape and torch.allclose(a, b, rtol=1e-12)
