@@ -372,7 +372,7 @@ class KernelOps:
                 span = min(window, meta.max_ctx or window) if window > 0 else meta.max_ctx
                 part = self.LATENT_DECODE_RUN
                 if self._latent_lib.latent_attention_dma_ok(kv_rank, rot_dim):
-                    part = self.latent_run(nd, heads, span)
+                    part = self.latent_run(nd, heads, -(-span // 128) * 128)   # (so that a growing context seldom asks anew)
                 while -(-span // part) > 64:
                     part *= 2
                 nparts = max(1, -(-span // part))
@@ -392,19 +392,31 @@ class KernelOps:
 
     @staticmethod
     def _latent_run(rows, heads, span) -> int:
-        """Keys of a run of the decode kernel that multiplies 64 at a time: us of a latency, of its pieces, which take longer where a compute unit has more than one
-        workgroup, of rounds of two workgroups per unit, and of the merge of the runs, with the unnormalised outputs that are written and read once more.
-        192 sizes (1 - 64 rows, 8, 16, 32 heads, 40 - 1024 keys): the choice takes 1.0 % longer than the best of runs of 64 - 1024 keys, at most 16 %; runs of 64 that
-        get longer from 1024 workgroups on took 5.6, at most 57. us of 64 / 128 / 192 / 256 / 512 keys: 16 heads, one row of 700 keys 9.5 / 11.2 / 12.9 / 14.8 / 22.4,
-        48 rows of 150 10.8 / 12.5 / 12.0, of 100 10.5 / 9.8, of 700 24.6 / 18.1 / 18.3 / 19.3 / 25.6; 32 heads, 16 rows of 1024 16.8 / 14.0 / 15.2 / 16.8 / 24.6, 64 rows of
-        1024 61.9 / 41.2 / 39.4 / 31.0 / 34.3."""
-        def time(part):
-            runs, pieces = -(-span // part), -(-min(part, span) // 64)
-            wgs = rows * -(-heads // 16) * runs
-            return (4.7 + 2.1 * pieces * max(1.0, 1.1 * wgs / 256) + 1.1 * max(0.0, wgs / 512 - 1)
-                    + (1.75 + 1e-3 * rows * heads * runs if runs > 1 else 0.0))
-        # (runs of 64, which were taken up to 1024 workgroups, where the others are not clearly expected to be faster: nothing of the above got slower)
-        return min((time(part) * (0.93 if part == 64 else 1.0), part) for part in (64, 128, 192, 256, 512, 1024))[1]
+        """Keys of a run of the decode kernel that multiplies 64 at a time. ``span`` is a bound on the contexts, and a captured step's is the model's length or its
+        window, whatever its contexts are: so the choice is made over contexts of the span, half of it, a quarter, .. 128 keys, by a model of each (us of a latency, of
+        a run's pieces one behind the other, which take longer where a compute unit has more than one workgroup, of workgroups that find no keys, and of the merge of
+        the runs). Runs of 64, longer ones up to 256 where their workgroups are more than 1024, are left only for a length that is expected to take less on
+        average over the contexts and nowhere more than 6 % more.
+        360 measured (rows, heads, span, contexts) of 1 - 64 rows, 16, 32, 64 heads, spans of 200 - 8192 and contexts of 60 keys up to the span, equal and mixed: 7 % less than
+        with those runs on average, at most 11 % more; chosen as if contexts were as long as the span, 6 % less and up to twice as long. us of runs of 64 / 128 / 256 / 512 / 1024
+        keys: 48 rows, 16 heads, span 1024, contexts of 150 13.2 / 13.8 / 15.4 / 15.4 / 13.1, of 700 28.5 / 21.1 / 22.8 / 32.6 / 38.4, of 1024 30.7 / 24.9 / 25.6 / 33.5 / 52.4; 16 rows,
+        32 heads, span 8192, of 700 - / 20.3 / 20.3 / 26.5 / 32.1, of 2000 - / 30.2 / 27.0 / 34.2 / 54.1, of 8192 - / 77 / 59 / 48 / 60."""
+        groups = rows * -(-heads // 16)
+
+        def time(part, ctx):
+            runs, live, pieces = -(-span // part), -(-ctx // part), -(-min(part, ctx) // 64)
+            return (5.6 + 2.3 * pieces * max(1.0, groups * live / 256) + 2.7e-3 * groups * runs
+                    + (1.3 + 0.07 * runs + 0.83e-3 * rows * heads * live if runs > 1 else 0.0))
+        plain = 64
+        while plain < 256 and groups * -(-span // plain) > 1024:
+            plain *= 2
+        ctxs = [span >> i for i in range(max(1, span.bit_length())) if i == 0 or span >> i >= 128]
+        known, best = [time(plain, c) for c in ctxs], (float("inf"), plain)
+        for part in (64, 128, 256, 512):
+            times = [time(part, c) for c in ctxs]
+            if all(t <= 1.06 * k for t, k in zip(times, known)):
+                best = min(best, (math.prod(t / k for t, k in zip(times, known)), part))
+        return best[1]
 
     def _mingru_pays(self, rows, width, k, f32) -> bool:
         """Whether the step in its product's epilogue is expected to take less than the faster product of the two and its launch, 2 us (1 in 32 bits)

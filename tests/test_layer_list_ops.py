@@ -636,6 +636,62 @@ def test_latent_attention_dma(kv, heads, window, lens, ctxs, nd):
     assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
 
 
+# us of latent attention's decode rows by keys per run: (rows, heads, span), then by context. The first length is what the rule took before it knew the contexts
+RUN_TIMES = {
+    (48, 16, 1024): {150: {64: 13.2, 128: 13.8, 256: 15.4, 512: 15.4, 1024: 13.1}, 300: {64: 16.0, 128: 14.6, 256: 17.8, 512: 19.7, 1024: 17.4},
+                     700: {64: 28.5, 128: 21.1, 256: 22.8, 512: 32.6, 1024: 38.4}, 1024: {64: 30.7, 128: 24.9, 256: 25.6, 512: 33.5, 1024: 52.4}},
+    (16, 32, 8192): {700: {256: 20.3, 128: 20.3, 512: 26.5, 1024: 32.1}, 2000: {256: 27.0, 128: 30.2, 512: 34.2, 1024: 54.1},
+                     4096: {256: 34.0, 128: 45.3, 512: 35.6, 1024: 53.0}, 8192: {256: 59.0, 128: 77.3, 512: 47.9, 1024: 59.9}},
+    (16, 64, 4096): {700: {256: 22.2, 128: 24.5, 512: 26.5, 1024: 32.1}, 2000: {256: 32.3, 128: 41.4, 512: 34.9, 1024: 54.1}, 4096: {256: 51.5, 128: 71.9, 512: 42.1, 1024: 53.9}},
+    (64, 64, 1024): {60: {256: 16.9, 128: 23.2, 512: 13.8, 1024: 9.1}, 300: {256: 28.7, 128: 39.8, 512: 26.6, 1024: 20.5}, 1024: {256: 54.0, 128: 76.0, 512: 43.6, 1024: 50.7}},
+    (1, 16, 1024): {60: {64: 9.9, 128: 9.7, 256: 9.6, 512: 9.6, 1024: 7.6}, 300: {64: 10.1, 128: 11.6, 256: 15.7, 512: 18.7, 1024: 16.2},
+                    1024: {64: 10.1, 128: 11.8, 256: 16.4, 512: 25.0, 1024: 39.1}}}
+
+
+@pytest.mark.parametrize("size", sorted(RUN_TIMES))
+def test_latent_runs_of_contexts_below_the_span(size):
+    """A captured step's span is a bound: the run length is not one that contexts far below it pay for."""
+    from hipserve.ops import KernelOps
+
+    part, gain = KernelOps._latent_run(*size), 1.0
+    for us in RUN_TIMES[size].values():
+        before = next(iter(us.values()))
+        assert us[part] <= 1.1 * before, (part, us)
+        gain *= us[part] / before
+    assert gain <= 1.0
+
+
+@pytest.mark.parametrize("rows,heads,span", [(0, 16, 0), (1, 1, 1), (1, 16, 128), (64, 128, 1 << 17)])
+def test_latent_runs_of_any_size(rows, heads, span):
+    from hipserve.ops import KernelOps
+
+    assert KernelOps._latent_run(rows, heads, span) in (64, 128, 256, 512)
+
+
+@gpu
+@pytest.mark.parametrize("part", [64, 128, 192, 256, 512])
+def test_latent_decode_runs(part):
+    """Contexts that end one key before, at and behind the runs' ends, and a span that leaves runs empty, in 64 bits; a length that is no power of two."""
+    kv, heads, rot, dim, block, scale, span = 512, 20, 64, 24, 16, 0.11, 2048
+    ctxs = [1, part - 1, part, part + 1, 2 * part, 2 * part + 1, 3 * part + 33]
+    lens = [1] * len(ctxs)
+    cache, cu, pos, bt, q_abs, q, proj, meta = latent_case(lens, ctxs, heads, dim, kv, rot, block, torch.bfloat16, "cuda", part)
+    meta.max_ctx = span
+    inv = torch.zeros(rot // 2)   # no rotation
+    want = torch.empty(heads, len(ctxs), kv, dtype=torch.float64)
+    for i, ctx in enumerate(ctxs):
+        j = torch.arange(ctx)
+        keys = cache[bt[i, j // block].long(), j % block].double()
+        sc = (q_abs[:, i, :kv].double() @ keys[:, :kv].T + q[i].double().view(heads, dim + rot)[:, dim:] @ keys[:, kv:].T) * scale
+        want[:, i] = torch.softmax(sc, -1) @ keys[:, :kv]
+    ops = type(get_ops("cuda"))()
+    ops.latent_run = lambda rows, heads, span: part
+    out = torch.full((heads, len(ctxs), kv), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.latent_attention(out, q_abs.cuda(), q.cuda(), proj.cuda(), cache.cuda(), meta, inv.cuda(), heads, dim, rot, kv, -1, scale, 0)
+    # as in test_latent_attention_dma
+    assert ((out.double().cpu() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -8 * cache.double().abs().max() * 0.5).all()
+
+
 @gpu
 @pytest.mark.parametrize("heads,gate,window,lens,ctxs", [
     (3, "head", 0, [130], [130]), (4, "head", 50, [70, 1, 33, 200], [70, 9, 64, 331]), (2, "channel", 33, [31, 128, 129], [31, 128, 400]),
