@@ -16,6 +16,7 @@ import math
 import weakref
 
 import torch
+import torch.autograd.forward_ad as forward_ad
 import torch.nn.functional as F
 
 log = logging.getLogger("hipserve.gemm")
@@ -563,11 +564,17 @@ def round_rows(rows: int, cols: int, k: int) -> int:
     return 256 * cut if cut >= 8 else 0
 
 
+def _writes_into_parts(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether products may write into parts of a result: not where gradients are recorded or a tangent comes along, under vmap and its like, where the calls are
+    traced (the cut is one for these rows) or intercepted, nor for tensors of a class of their own."""
+    return not (torch.is_grad_enabled() or forward_ad._current_level >= 0 or torch._C._are_functorch_transforms_active() or torch.jit.is_tracing()
+                or torch._C._len_torch_dispatch_stack() > 0 or type(x) is not torch.Tensor or type(w) not in (torch.Tensor, torch.nn.Parameter))
+
+
 def linear_in_rounds(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | None:
-    """x W^T of rows [M, K] in two products of whole rounds and of what lies behind them, or None where it is one (also where gradients are recorded: the
-    products write into parts of the result)."""
+    """x W^T of rows [M, K] in two products of whole rounds and of what lies behind them, or None where it is one."""
     M, N = x.shape[0], w.shape[0]
-    if M < 1024 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or torch.is_grad_enabled():
+    if M < 1024 or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not _writes_into_parts(x, w):
         return None
     cols, rows = round_columns(M, N, w.shape[1]), round_rows(M, N, w.shape[1])
     if not cols and not rows:

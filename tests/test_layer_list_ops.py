@@ -397,6 +397,44 @@ def test_products_in_whole_rounds(rows, cols, K, grad, device):
     assert ((y.detach().float() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -23 * (x.float().abs() @ w.detach().float().abs().t())).all()
 
 
+@pytest.mark.parametrize("rows,cols,K", [(1024, 16400, 16), (2049, 8192, 2048)])   # cut by columns, by rows
+@pytest.mark.parametrize("way", ["dual", "jvp", "vmap", "vmap of weights", "trace", "fx", "subclass"])
+def test_products_in_whole_rounds_are_one_where_calls_are_transformed(way, rows, cols, K):
+    """Forward mode, vmap, traces and tensor classes without gradients recorded: what one product does."""
+    import torch.autograd.forward_ad as fw
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    from hipserve.ops import KernelOps
+
+    class Rows(torch.Tensor):
+        pass
+
+    g = torch.Generator().manual_seed(rows)
+    x, t, w = (torch.randn(*s, generator=g).bfloat16() for s in ((rows, K), (rows, K), (cols, K)))
+    few, linear = x[:3], KernelOps()._vendor_linear
+
+    def run(f):
+        if way == "dual":
+            with fw.dual_level():
+                return fw.unpack_dual(f(fw.make_dual(x, t), w, None)).tangent
+        if way == "jvp":
+            return torch.func.jvp(lambda a: f(a, w, None), (x,), (t,))[1]
+        if way == "vmap":
+            return torch.vmap(lambda a: f(a, w, None))(x[None])
+        if way == "vmap of weights":
+            return torch.vmap(lambda a: f(x, a, None))(w[None])
+        if way == "trace":   # of many rows, used for few
+            return torch.jit.trace(lambda a: f(a, w, None), x, check_trace=False)(few)
+        if way == "fx":
+            return make_fx(lambda a: f(a, w, None))(x)(few)
+        y = f(x.as_subclass(Rows), w, None)
+        assert type(y) is Rows
+        return y.as_subclass(torch.Tensor)
+
+    with torch.no_grad():
+        assert torch.equal(run(linear), run(torch.nn.functional.linear))
+
+
 def test_halves_projected_apart():
     """A parallel mixer whose left half has biases and whose right half ends with an activation: two products give what parts of one do."""
     from types import SimpleNamespace
