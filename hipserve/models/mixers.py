@@ -855,6 +855,7 @@ class ParallelMixer:
     """left_scale * left(h) + right_scale * right(h): both halves write their scaled head outputs
     into one [T, left | right] buffer; one GEMM with the concatenated output weights sums them.
     With ``spec.out_norms`` each half has an output GEMM of its own and ``forward`` returns a ``NormedPair``."""
+    end = None   # row of ``w_in`` behind the right half's (None: the last)
 
     def __init__(self, spec: ParallelMixerSpec, hidden: int, eps: float, device, dtype, ops):
         self.spec, self.hidden, self.device, self.dtype, self.ops = spec, hidden, device, dtype, ops
@@ -862,7 +863,7 @@ class ParallelMixer:
         self.right = make_mixer(spec.right, hidden, eps, device, dtype, ops)
         self.w_o = None      # [hidden, left out | right out]
         self.left_norm = self.right_norm = None   # fp32 [hidden] with out_norms
-        self.w_in = None     # [left inputs | zero rows up to a multiple of 8 | right inputs, hidden], when one GEMM serves both
+        self.w_in = None     # [left inputs | zero rows up to a multiple of 8 | right inputs | such zero rows, hidden], when one GEMM serves both
         self.b_in = None     # its biases, where a half has them
         self.split = 0       # rows of w_in before the right half's
         self.in_act = {}     # its activation: the right half's, on the last columns
@@ -890,8 +891,10 @@ class ParallelMixer:
         if all(getattr(m, "takes_proj", False) for m in (self.left, self.right)) and not hasattr(self.left, "in_act"):
             wl, wr = self.left.w_in, self.right.w_in
             bl, br = getattr(self.left, "b_in", None), getattr(self.right, "b_in", None)
-            self.split = -(-wl.shape[0] // 8) * 8   # 16-byte aligned rows in bf16
-            self.w_in = torch.cat([F.pad(wl, (0, 0, 0, self.split - wl.shape[0])), wr], 0).contiguous()
+            # both halves' rows at multiples of 16 bytes, whatever the size of the other one (a rank from the checkpoint, say): the kernels that read wide need them
+            self.split = -(-wl.shape[0] // 8) * 8
+            self.end = self.split + wr.shape[0]
+            self.w_in = torch.cat([F.pad(wl, (0, 0, 0, self.split - wl.shape[0])), F.pad(wr, (0, 0, 0, -wr.shape[0] % 8))], 0).contiguous()
             if bl is not None or br is not None:
                 self.left_biased = br is None
                 self.b_in = wl.new_zeros(self.w_in.shape[0])
@@ -915,9 +918,10 @@ class ParallelMixer:
         where rounds end (``ops.in_rounds``), one each. (A product with biases cannot be cut where rounds end: the library adds them in a pass of its own then.)"""
         if self.left_biased and self.ops.in_rounds(h, self.split, self.w_in.shape[0] - self.split):
             act = dict(self.in_act, act_from=self.in_act["act_from"] - self.split) if self.in_act else {}
-            return self.ops.linear(h, self.w_in[:self.split], self.b_in[:self.split]), self.ops.linear(h, self.w_in[self.split:], **act)
+            left, right = self.ops.linear(h, self.w_in[:self.split], self.b_in[:self.split]), self.ops.linear(h, self.w_in[self.split:], **act)
+            return left, right if self.end is None else right[:, :self.end - self.split]
         proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)
-        return proj[:, :self.split], proj[:, self.split:]
+        return proj[:, :self.split], proj[:, self.split:self.end]
 
     def _forward_normed(self, h, meta, cache, state):
         pl = pr = None

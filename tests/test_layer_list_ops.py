@@ -458,6 +458,45 @@ def test_halves_projected_apart():
         assert a.shape == b.shape and torch.allclose(a, b, rtol=1e-12)
 
 
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rank", [3, 20, 24])
+@pytest.mark.parametrize("biased", [False, True])
+@pytest.mark.parametrize("rows", [1, 70])
+def test_one_projection_of_both_halves_keeps_rows_aligned(rows, biased, rank, dtype, device):
+    """A parallel mixer's projection whose right half ends with a bottleneck of any rank: the left half's rows stay where the wide kernels take them, and each half has the
+    columns of its own product."""
+    from hipserve.config import DeltaRuleSpec, ParallelMixerSpec, WindowAttentionSpec
+    from hipserve.models.mixers import DeltaRule, ParallelMixer, WindowAttention
+    from hipserve.ops import ReferenceOps
+
+    ops = get_ops("cuda") if device == "cuda" else ReferenceOps()
+    spec = ParallelMixerSpec(WindowAttentionSpec(heads=2, kv_heads=1, dim=64, vdim=64, scale=0.125, window=8, rot_dims=32, bias=biased), DeltaRuleSpec(2, 64, rank), 0.5, 2.0)
+    dev = torch.device(device)
+    m = ParallelMixer(spec, 128, 1e-5, dev, dtype, ops)
+    t = m.init_random(torch.Generator().manual_seed(rank), 0.1)
+    m.load(lambda n: t[n], "")
+    assert m.w_in is not None
+    h = torch.randn(rows, 128, generator=torch.Generator().manual_seed(rows)).to(dev, dtype)
+    left, right = m._project(h)
+    assert left.stride(0) * left.element_size() % 16 == 0 and left.data_ptr() % 16 == 0 and right.data_ptr() % 16 == 0
+    halves = [(left, WindowAttention(spec.left, 128, 1e-5, dev, dtype, ops), "left."), (right, DeltaRule(spec.right, 128, 1e-5, dev, dtype, ops), "right.")]
+    for got, half, name in halves:
+        half.load(lambda n: t[n], name)
+        want = h.double() @ half.w_in.double().t()
+        if getattr(half, "b_in", None) is not None:
+            want += half.b_in.double()
+        if name == "right.":
+            assert got.shape == want.shape
+            want[:, 5 * 128:] = torch.tanh(want[:, 5 * 128:])
+        # rounded once, and before the activation; sums of 128 products in 32 bits
+        tol = 2.0 ** -7 if dtype == torch.bfloat16 else 1e-4
+        assert ((got[:, :want.shape[1]].double() - want).abs() <= tol * (want.abs() + 0.1 * want.abs().max())).all()
+    if device == "cuda" and rows == 1:
+        cache = torch.zeros(2, 16, spec.left.cache_dim, dtype=dtype, device=dev)
+        assert ops._window_lib.window_attention_decode_ok(left, cache, 64, 64)
+
+
 @gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,H,K", [(1, 64, 2056), (8, 2048, 4104), (9, 192, 1032), (16, 1024, 3072), (17, 2048, 520), (32, 832, 2048)])
