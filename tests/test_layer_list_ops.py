@@ -458,6 +458,30 @@ def test_halves_projected_apart():
         assert a.shape == b.shape and torch.allclose(a, b, rtol=1e-12)
 
 
+@gpu
+@pytest.mark.parametrize("rows,rank,apart", [(1024, 96, True), (1000, 96, False), (1024, 90, True)])
+def test_halves_projected_apart_in_rounds(rows, rank, apart):
+    """Sizes at which the right half's product goes in whole rounds: what its rule says, and the columns of either product against 64 bits."""
+    from hipserve.config import DeltaRuleSpec, ParallelMixerSpec, WindowAttentionSpec
+    from hipserve.models.mixers import ParallelMixer
+
+    ops, dev, H, N = get_ops("cuda"), torch.device("cuda"), 64, 51 * 64
+    spec = ParallelMixerSpec(WindowAttentionSpec(heads=64, kv_heads=32, dim=128, vdim=128, scale=0.1, window=8, rot_dims=32, bias=True), DeltaRuleSpec(51, 64, rank))
+    m = ParallelMixer(spec, H, 1e-5, dev, torch.bfloat16, ops)
+    t = m.init_random(torch.Generator().manual_seed(5), 0.05)
+    m.load(lambda n: t[n], "")
+    h = torch.randn(rows, H, generator=torch.Generator().manual_seed(6)).to(dev, torch.bfloat16)
+    assert ops.in_rounds(h, m.split, m.w_in.shape[0] - m.split) == apart
+    left, right = m._project(h)
+    assert (left.untyped_storage().data_ptr() != right.untyped_storage().data_ptr()) == apart
+    assert left.shape == (rows, 16384) and right.shape == (rows, 5 * N + rank)
+    w, b = m.w_in.double(), m.b_in.double()
+    for got, at, act in ((left, 0, right.shape[1]), (right, m.split, 5 * N)):
+        want = h.double() @ w[at:at + got.shape[1]].t() + b[at:at + got.shape[1]]
+        want[:, act:] = torch.tanh(want[:, act:])
+        assert ((got.double() - want).abs() <= 2.0 ** -7 * (want.abs() + 0.1 * want.abs().max())).all()   # as above
+
+
 @pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("rank", [3, 20, 24])
