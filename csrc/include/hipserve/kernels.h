@@ -267,11 +267,14 @@ void launch_moe_topk_softmax(const void* logits, bool logits_f32, float* w, int*
                              bool renorm, hipStream_t s, int splits = 0);
 void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
                       int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist);
-// Orders of the tiles for GEMMs that take per_round[j] of them at once (one table): to [rows, tiles] int32, place << 16 | expert << 8 | pairs - 1
+// m-tiles of a group of the packed GEMM's tiles, which it walks column by column (prefill_gemm_packed.hip)
+constexpr int kTileGroup = 8;
+// Orders of the tiles for GEMMs of across[j] tiles beside each other that take per_round[j] tiles at once (one table): to [rows, tiles] int32,
+// place << 16 | expert << 8 | pairs - 1
 struct MoeOrder {
   int* to = nullptr;
   int rows = 0;
-  int per_round[2] = {1, 1};
+  int per_round[2] = {1, 1}, across[2] = {1, 1};
 };
 // the same for the pairs (t, j), expert table[i][tokens[t]][j] of `tables` tables [table_rows, top], outputs side by side (num_tiles
 // [tables]): a workgroup each, or many for a large step of one table (hist as below)

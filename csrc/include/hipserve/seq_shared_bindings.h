@@ -49,10 +49,10 @@ inline void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor
 
 // moe_align of the pairs (t, j) whose expert is table[tokens[t]][j], table [rows, top]; or of every table of [L, rows, top], with outputs
 // [L, slots], [L, tiles], [L, pairs]; num_tiles [L]: the tiles in use; order [n, tiles], one table: those
-// as a GEMM takes them that has per_round[j] in a round (order_tiles), place << 16 | expert << 8 | pairs - 1.
+// as a GEMM takes them that has per_round[j] in a round, across[j] of them (none given: one) for each of these (order_tiles), place << 16 | expert << 8 | pairs - 1.
 inline void moe_table_align(const at::Tensor& table, const at::Tensor& tokens, int64_t E, int64_t tile, at::Tensor& slots,
                             at::Tensor& tile_expert, at::Tensor& pair_slot, const c10::optional<at::Tensor>& num_tiles,
-                            const c10::optional<at::Tensor>& order, at::IntArrayRef per_round) {
+                            const c10::optional<at::Tensor>& order, at::IntArrayRef per_round, at::IntArrayRef across) {
   CHECK_DEV(table); CHECK_I32(table); CHECK_I32(slots); CHECK_I32(tile_expert); CHECK_I32(pair_slot);
   CHECK_SAME_DEV(tokens, table); CHECK_SAME_DEV(slots, table); CHECK_SAME_DEV(tile_expert, table); CHECK_SAME_DEV(pair_slot, table);
   const long d = table.dim(), L = d == 3 ? table.size(0) : 1;
@@ -74,12 +74,15 @@ inline void moe_table_align(const at::Tensor& table, const at::Tensor& tokens, i
   if (order.has_value()) {
     CHECK_I32(*order); CHECK_SAME_DEV(*order, table);
     TORCH_CHECK(L == 1 && order->dim() == 2 && order->size(1) == tiles && order->size(0) == (long)per_round.size() && per_round.size() <= 2 &&
-                tiles < (1L << 15) && tile <= 256, "moe_table_align: orders of the tiles");
+                (across.empty() || across.size() == per_round.size()) && tiles < (1L << 15) && tile <= 256, "moe_table_align: orders of the tiles");
     orders.to = order->data_ptr<int>();
     orders.rows = per_round.size();
     for (size_t i = 0; i < per_round.size(); ++i) {
       TORCH_CHECK(per_round[i] >= 1 && per_round[i] < (1L << 20), "moe_table_align: tiles in a round");
       orders.per_round[i] = per_round[i];
+      if (across.empty()) continue;
+      TORCH_CHECK(across[i] >= 1 && across[i] < (1L << 15), "moe_table_align: tiles beside each other");
+      orders.across[i] = across[i];
     }
   }
   const int nb = L == 1 ? hipserve::moe_align_blocks(npairs) : 1;
@@ -257,7 +260,7 @@ inline void def_moe_ops(torch::Library& m) {
   m.def("skinny_linear_update(Tensor(a!) out, Tensor(b!) squares, Tensor(c!) residual, Tensor weight, Tensor x, Tensor w, Tensor? bias) -> ()");
   m.def("moe_align(Tensor ids, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, Tensor(c!) pair_slot) -> ()");
   m.def("moe_table_align(Tensor table, Tensor tokens, int E, int tile, Tensor(a!) slots, Tensor(b!) tile_expert, "
-        "Tensor(c!) pair_slot, Tensor(d!)? num_tiles=None, Tensor(e!)? order=None, int[] per_round=[]) -> ()");
+        "Tensor(c!) pair_slot, Tensor(d!)? num_tiles=None, Tensor(e!)? order=None, int[] per_round=[], int[] across=[]) -> ()");
   m.def("moe_align_small(int npairs) -> bool", &moe_align_small);
   m.def("expert_gemm(Tensor(a!) out, Tensor x, Tensor w, Tensor slots, Tensor tile_expert, int tile, int gather_k, "
         "int act, Tensor? row_scale=None, float limit=0.0, int pairs=0, int tiles=0) -> ()");

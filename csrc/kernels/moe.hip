@@ -119,12 +119,15 @@ HS_DEVICE void padded_offsets(const int* cnt, int* off, int E, int tile_shift, i
   }
 }
 
-// The order for a GEMM that takes the tiles in rounds of `per_round`, as place << 16 | expert << 8 | pairs - 1: as they lie, but for what the last round would
-// be short of if it is few (three sixteenths of one): so many of the tiles that hold the fewest pairs come last. (All partial tiles last, by their pairs: a
-// full round of them has another expert's weights in every workgroup, 16 experts of 1024 x 2048 in two rounds 65 -> 74 us.) One wave, two experts per lane.
-HS_DEVICE void order_tiles(const int* cnt, const int* off, int E, int tile_shift, int per_round, int* __restrict__ order) {
-  const int lane = threadIdx.x & 63, total = off[128] >> tile_shift, left = total % per_round;
-  const bool moves = 16 * left <= 3 * per_round;
+// The order for a GEMM of `across` tiles for each of these that takes them in rounds of `per_round`, as place << 16 | expert << 8 | pairs - 1: as they lie, but
+// if what whole rounds leave over is few (three sixteenths of one), as many of those that hold the fewest pairs as it is tiles of come last. (All partial tiles
+// last, by their pairs: a full round of them has another expert's weights in every workgroup, 16 experts of 1024 x 2048 in two rounds 65 -> 74 us.) One
+// wave, two experts per lane.
+HS_DEVICE void order_tiles(const int* cnt, const int* off, int E, int tile_shift, int per_round, int across, int* __restrict__ order) {
+  const int lane = threadIdx.x & 63, total = off[128] >> tile_shift, over = total * across % per_round, whole = total * across - over;
+  // those that the left ones are of: the first group of them may start before them (the GEMM's walk: its tiles column by column)
+  const int first = whole / (kTileGroup * across) * kTileGroup, taken = whole - first * across - (across - 1) * min(kTileGroup, total - first);
+  const int left = over > 0 ? total - first - max(taken, 0) : 0;
   int rest[2], rank[2] = {0, 0};   // pairs of the experts' last tiles, where they are partial, and how many of those have fewer
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -137,6 +140,7 @@ HS_DEVICE void order_tiles(const int* cnt, const int* off, int E, int tile_shift
 #pragma unroll
     for (int i = 0; i < 2; ++i) rank[i] += r > 0 && (r < rest[i] || (r == rest[i] && x < 2 * lane + i)) ? 1 : 0;
   }
+  const bool moves = 16 * over <= 3 * per_round;
   unsigned long moved[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) moved[i] = __ballot(moves && rest[i] > 0 && rank[i] < left);
@@ -205,7 +209,7 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
   if (tid < E)
     for (int t = off[tid] >> tile_shift; t < off[tid + 1] >> tile_shift; ++t) tile_expert[t] = tid;
   for (int t = (total >> tile_shift) + tid; t < tiles_cap; t += 1024) tile_expert[t] = -1;
-  if (tid >> 6 < order.rows) order_tiles(cnt, off, E, tile_shift, order.per_round[tid >> 6], order.to + (long)(tid >> 6) * tiles_cap);
+  if (tid >> 6 < order.rows) order_tiles(cnt, off, E, tile_shift, order.per_round[tid >> 6], order.across[tid >> 6], order.to + (long)(tid >> 6) * tiles_cap);
 }
 
 // moe_align over many workgroups, for prefill-sized pair counts (one workgroup is bound by its compute unit's lookups and stores). Pass 1: a
@@ -282,7 +286,7 @@ __global__ __launch_bounds__(1024) void moe_place_kernel(int npairs, int E, int 
   }
   for (int s = total + b * 1024 + tid; s < slots_cap; s += nb * 1024) slots[s] = -1;
   for (int t = (total >> tile_shift) + b * 1024 + tid; t < tiles_cap; t += nb * 1024) tile_expert[t] = -1;
-  if (b == nb - 1 && tid >> 6 < order.rows) order_tiles(cnt, off, E, tile_shift, order.per_round[tid >> 6], order.to + (long)(tid >> 6) * tiles_cap);
+  if (b == nb - 1 && tid >> 6 < order.rows) order_tiles(cnt, off, E, tile_shift, order.per_round[tid >> 6], order.across[tid >> 6], order.to + (long)(tid >> 6) * tiles_cap);
 }
 
 static int align_chunk(int npairs) { return npairs > 65536 ? 4096 : 1024; }

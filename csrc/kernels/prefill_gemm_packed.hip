@@ -54,7 +54,7 @@ constexpr int PW_T = 256;
 // L = it * G + r (r = b remapped so an XCD's workgroups hold consecutive r), and a
 // logical tile L -> (tm, tn) walks groups of PW_GM m-tiles n-major: the ~32 workgroups an
 // XCD runs at once cover 8 m-tiles x 4 n-tiles and share both operands in its L2.
-constexpr int PW_GM = 8;
+constexpr int PW_GM = kTileGroup;
 HS_DEVICE void pw_tile(int L, int tiles_m, int tiles_n, int& tm, int& tn) {
   const int grp = L / (PW_GM * tiles_n), first = grp * PW_GM;
   const int gsz = min(PW_GM, tiles_m - first);

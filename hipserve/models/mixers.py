@@ -403,10 +403,10 @@ class TableMoE:
         pair_slot = torch.empty(P, dtype=torch.int32, device=dev)
         orders = (None, None)
         if self.ops.moe_tables_align_ok(self.table, ids, E):
-            # a round of either product: 512 columns (tile 256: 256) of so many tiles as there are compute units for
+            # either product has a tile per 512 columns (tile 256: 256), and a round is one per compute unit
             cus, cols = torch.cuda.get_device_properties(dev).multi_processor_count, 512 // gemm.PW_WM
             orders = torch.empty(2, cap // tile, dtype=torch.int32, device=dev)
-            self.ops.moe_table_align(self.table, ids, E, tile, slots, tile_expert, pair_slot, ntiles, orders, [max(1, cus // -(-n // cols)) for n in (ff, H)])
+            self.ops.moe_table_align(self.table, ids, E, tile, slots, tile_expert, pair_slot, ntiles, orders, [cus, cus], [-(-n // cols) for n in (ff, H)])
         else:
             op.moe_align(self.table.index_select(0, ids).reshape(-1), E, tile, slots, tile_expert, ntiles, pair_slot, None)
         pu, pd = self.packed

@@ -921,12 +921,12 @@ class KernelOps:
         """Whether ``moe_table_align`` takes ``tables`` [(layers,) rows, top] in one launch, with a row of outputs per table."""
         return E <= 128 and tokens.dtype == torch.long and tokens.is_contiguous() and self._moe_lib.moe_align_small(tokens.numel() * tables.shape[-1])
 
-    def moe_table_align(self, table, tokens, E, tile, slots, tile_expert, pair_slot, num_tiles=None, order=None, per_round=()):
+    def moe_table_align(self, table, tokens, E, tile, slots, tile_expert, pair_slot, num_tiles=None, order=None, per_round=(), across=()):
         """``moe_align`` of the experts table[tokens] [T, top]: one launch for small batches. ``table`` may hold the tables of several
-        layers, and ``num_tiles`` (the tiles in use) and ``order`` (for GEMMs that
-        take ``per_round`` of them at once, a row each; one table) be asked for, where ``moe_tables_align_ok`` says so."""
+        layers, and ``num_tiles`` (the tiles in use) and ``order`` (for GEMMs of ``across`` tiles for each of these, or of one, that
+        take ``per_round`` tiles at once, a row each; one table) be asked for, where ``moe_tables_align_ok`` says so."""
         if self.moe_tables_align_ok(table, tokens, E):
-            self._moe_lib.moe_table_align(table, tokens, E, tile, slots, tile_expert, pair_slot, num_tiles, order, list(per_round))
+            self._moe_lib.moe_table_align(table, tokens, E, tile, slots, tile_expert, pair_slot, num_tiles, order, list(per_round), list(across))
         else:
             assert table.dim() == 2 and num_tiles is None and order is None, "the tables of several layers: small batches"
             self.moe_align(table.index_select(0, tokens).view(-1), E, tile, slots, tile_expert, pair_slot)

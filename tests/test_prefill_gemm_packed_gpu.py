@@ -287,3 +287,35 @@ def test_packed_grouped_by_order(counts, N, K, epi, gather):
         want = h.clamp(min=0).square() if epi == 4 else torch.nn.functional.silu(h[:, :No]) * h[:, No:] if epi == 2 else h
         rel = 2.0 ** -6 if epi == 2 else 2.0 ** -7   # as above
         assert len(mine) == 0 or ((got[mine].double() - want).abs() <= rel * want.abs() + 2.0 ** -9 * want.abs().mean()).all()
+
+
+def _left_over(n, across, per_round):
+    """The m-tiles that the tiles behind whole rounds are of, as the kernel walks them: groups of 8 m-tiles, column by column."""
+    walk = [tm for g in range(0, n, 8) for _ in range(across) for tm in range(g, min(g + 8, n))]
+    return sorted(set(walk[len(walk) // per_round * per_round:])), len(walk) % per_round
+
+
+@pytest.mark.parametrize("across,per_round", [(1, 16), (2, 16), (3, 16), (3, 32), (6, 64), (5, 48), (8, 256), (3, 256)])
+@pytest.mark.parametrize("counts", [[5, 200, 64], [1000, 129, 40, 300, 0, 257, 33, 1], [128] * 9, [20, 130] * 12, [700, 65, 193, 90, 321, 511, 66, 1200], [10] * 60])
+def test_order_of_tiles_for_whole_rounds(counts, across, per_round):
+    """Tiles of few pairs last where whole rounds of the GEMM's tiles leave little over; numbers of tiles beside each other that divide a round, and that do not."""
+    from hipserve.ops import get_ops
+
+    E, P = len(counts), sum(counts)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(P, generator=torch.Generator().manual_seed(P))].int().to(DEV)
+    cap = -(-(P + E * 127) // 128) * 128
+    slots, te, nt, ps = (torch.empty(n, dtype=torch.int32, device=DEV) for n in (cap, cap // 128, 1, P))
+    orders = torch.full((2, cap // 128), -1, dtype=torch.int32, device=DEV)
+    get_ops("cuda").moe_table_align(ids.view(-1, 1), torch.arange(P, device=DEV), E, 128, slots, te, ps, nt, orders, [7, per_round], [1, across])
+    n, rows = int(nt), (slots.view(-1, 128) >= 0).sum(1).cpu()
+    o = orders[1, :n].cpu().long()
+    place = o >> 16
+    assert torch.equal(te.cpu()[place].long(), o >> 8 & 255) and torch.equal(rows[place], (o & 255) + 1)
+    left, over = _left_over(n, across, per_round)
+    partial = sorted((int(rows[t]), t) for t in range(n) if rows[t] < 128)
+    moved = partial[:len(left)]
+    if 16 * over > 3 * per_round:
+        moved = []
+    gone = {t for _, t in moved}
+    assert place.tolist() == [t for t in range(n) if t not in gone] + [t for _, t in moved]
+    assert not moved or left == list(range(left[0], n))   # they are the last places
