@@ -120,9 +120,10 @@ HS_DEVICE void padded_offsets(const int* cnt, int* off, int E, int tile_shift, i
 }
 
 // The order for a GEMM of `across` tiles for each of these that takes them in rounds of `per_round`, as place << 16 | expert << 8 | pairs - 1: as they lie, but
-// if what whole rounds leave over is few (three sixteenths of one), as many of those that hold the fewest pairs as it is tiles of come last. (All partial tiles
-// last, by their pairs: a full round of them has another expert's weights in every workgroup, 16 experts of 1024 x 2048 in two rounds 65 -> 74 us.) One
-// wave, two experts per lane.
+// where it takes what whole rounds leave over by columns (pw_rest: up to two sixteenths of a round, up to three if none of it has more than 64 rows), as many of
+// those that hold the fewest pairs as it is tiles of come last. Taken in another way they are better left (8 experts of 2048 x 4096, 36 of 73 tiles by
+// quarters 145 -> 153 us: each workgroup has another expert's weights), and so are all partial tiles (16 experts of 1024 x 2048 in two rounds 65 -> 74). One wave,
+// two experts per lane.
 HS_DEVICE void order_tiles(const int* cnt, const int* off, int E, int tile_shift, int per_round, int across, int* __restrict__ order) {
   const int lane = threadIdx.x & 63, total = off[128] >> tile_shift, over = total * across % per_round, whole = total * across - over;
   // those that the left ones are of: the first group of them may start before them (the GEMM's walk: its tiles column by column)
@@ -140,7 +141,8 @@ HS_DEVICE void order_tiles(const int* cnt, const int* off, int E, int tile_shift
 #pragma unroll
     for (int i = 0; i < 2; ++i) rank[i] += r > 0 && (r < rest[i] || (r == rest[i] && x < 2 * lane + i)) ? 1 : 0;
   }
-  const bool moves = 16 * over <= 3 * per_round;
+  const int few = __popcll(__ballot(rest[0] > 0 && rest[0] <= 64)) + __popcll(__ballot(rest[1] > 0 && rest[1] <= 64));
+  const bool moves = 16 * over <= (left <= few ? 3 : 2) * per_round;
   unsigned long moved[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) moved[i] = __ballot(moves && rest[i] > 0 && rank[i] < left);

@@ -74,18 +74,31 @@ HS_DEVICE PwPlace pw_place(const PwGroup& grp, int tm, int tile_rows) {
   return {v >> 16, v >> 8 & 255, (v & 255) + 1};
 }
 
+// Whether none of the last `left` tiles has more than 64 rows. Their m-tiles are those of the group that the first of them lies in, without the ones whose last
+// column of tiles is taken before, and all behind it; a lane asks for each.
+HS_DEVICE bool pw_rest_short(int left, int tiles_m, int tiles_n, const PwGroup& grp) {
+  const int whole = tiles_m * tiles_n - left, first = whole / (PW_GM * tiles_n) * PW_GM;
+  const int from = first + max(whole - first * tiles_n - (tiles_n - 1) * min(PW_GM, tiles_m - first), 0);
+  for (int tm = from; tm < tiles_m; tm += 64) {
+    const int at = tm + (int)(threadIdx.x & 63);
+    if (__ballot(at < tiles_m && (grp.order[min(at, tiles_m - 1)] & 255) >= 64) != 0) return false;
+  }
+  return true;
+}
+
 // What whole rounds of `ncu` tiles leave over, and how it is taken: as one more round (24 us per 1024 of K), by quarters (pw_tail, 9 + 12.5 us per 1024) or by
-// columns (pw_few: each round of theirs 3 us and, per 1024, 3 us for up to 32 rows, 5 for 64, 8 for 128, beside the latency of the first).
+// columns (pw_few: each round of theirs 3 us and, per 1024, 3 us for up to 32 rows, 5 for 64, 8 for 128, beside the latency of the first). In an order that has
+// the tiles of the fewest rows last: one round of columns or two always, three if all are short or K is too short for quarters. us of a round / quarters /
+// columns, two rounds: 16 experts of 2048 x 1024, 24 tiles of up to 59 rows 69 / 58 / 49, 8 of 4096 x 2048, 32 of up to 66 123 / 93 / 88, 16 of 1536 x 3072, 32 of
+// up to 126 176 / 127 / 125; three: 32 of 1536 x 1536, 38 of up to 63 100 / 77 / 69, 8 of 2048 x 4096, 36 of up to 126 (as they lie) 184 / 145 / 154. 131 such
+// sizes: this takes 1.2 % longer than the best of these and both orders, a choice by the rows of the first of the tiles 2.9 %.
 enum PwRest { kRestRound, kRestQuarters, kRestColumns };
 HS_DEVICE PwRest pw_rest(int left, int tiles_m, int tiles_n, int ncu, int K, const PwGroup& grp) {
   if (left == 0) return kRestRound;
   const int rounds = (16 * left + ncu - 1) / ncu;
-  if (rounds <= 1) return kRestColumns;
-  if (rounds <= 3) {
-    // the most rows that one of them has: the first m-tile's of the group that the first of them lies in
-    const int rows = pw_place(grp, (tiles_m * tiles_n - left) / (PW_GM * tiles_n) * PW_GM, 128).rows;
-    if (rounds <= (rows <= 32 ? 3 : rows <= 64 || K < 1536 ? 2 : 1)) return kRestColumns;
-  }
+  const bool ordered = grp.order != nullptr;
+  if (rounds <= 1 || (rounds == 2 && (ordered || K < 1536))) return kRestColumns;
+  if (rounds == 3 && ordered && (K < 1536 || pw_rest_short(left, tiles_m, tiles_n, grp))) return kRestColumns;
   return 4 * left <= ncu && K >= 1536 ? kRestQuarters : kRestRound;
 }
 

@@ -298,7 +298,8 @@ def _left_over(n, across, per_round):
 @pytest.mark.parametrize("across,per_round", [(1, 16), (2, 16), (3, 16), (3, 32), (6, 64), (5, 48), (8, 256), (3, 256)])
 @pytest.mark.parametrize("counts", [[5, 200, 64], [1000, 129, 40, 300, 0, 257, 33, 1], [128] * 9, [20, 130] * 12, [700, 65, 193, 90, 321, 511, 66, 1200], [10] * 60])
 def test_order_of_tiles_for_whole_rounds(counts, across, per_round):
-    """Tiles of few pairs last where whole rounds of the GEMM's tiles leave little over; numbers of tiles beside each other that divide a round, and that do not."""
+    """Tiles of few pairs last where what whole rounds of the GEMM's tiles leave over goes by columns, which it does not for three sixteenths of a round with
+    longer ones; numbers of tiles beside each other that divide a round, and that do not."""
     from hipserve.ops import get_ops
 
     E, P = len(counts), sum(counts)
@@ -314,7 +315,8 @@ def test_order_of_tiles_for_whole_rounds(counts, across, per_round):
     left, over = _left_over(n, across, per_round)
     partial = sorted((int(rows[t]), t) for t in range(n) if rows[t] < 128)
     moved = partial[:len(left)]
-    if 16 * over > 3 * per_round:
+    short = len(moved) == len(left) and all(r <= 64 for r, _ in moved)
+    if 16 * over > (3 if short else 2) * per_round:
         moved = []
     gone = {t for _, t in moved}
     assert place.tolist() == [t for t in range(n) if t not in gone] + [t for _, t in moved]
