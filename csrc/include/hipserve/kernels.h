@@ -265,8 +265,9 @@ namespace hipserve {
 // moe.hip — tile in {16, 32, 64}
 void launch_moe_topk_softmax(const void* logits, bool logits_f32, float* w, int* ids, int T, int E, int k,
                              bool renorm, hipStream_t s, int splits = 0);
+// same: pairs take the same places in every run, for GEMMs that sum some tiles in another order (the packed one)
 void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
-                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist);
+                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, bool same, hipStream_t s, int* hist);
 // m-tiles of a group of the packed GEMM's tiles, which it walks column by column (prefill_gemm_packed.hip)
 constexpr int kTileGroup = 8;
 // Orders of the tiles for GEMMs of across[j] tiles beside each other that take per_round[j] tiles at once (one table): to [rows, tiles] int32,
@@ -280,7 +281,7 @@ struct MoeOrder {
 // [tables]): a workgroup each, or many for a large step of one table (hist as below)
 void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
                             int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot,
-                            int* hist, const MoeOrder& order, hipStream_t s);
+                            int* hist, bool same, const MoeOrder& order, hipStream_t s);
 // Workgroups of moe_align for npairs. More than one need hist, int32 [moe_align_blocks(npairs) * 128] scratch (of one table; else it is not
 // looked at). The number does not grow with npairs (65536: 64, 65537: 17): it is asked for at every call.
 int moe_align_blocks(int npairs);

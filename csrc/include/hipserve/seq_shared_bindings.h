@@ -43,7 +43,7 @@ inline void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor
   at::Tensor scratch = at::empty({(long)(nb > 1 ? nb : 0) * 128 + 1}, ids.options());  // [hist | tile count]
   hipserve::launch_moe_align(ids.data_ptr<int>(), npairs, E, tile, slots.data_ptr<int>(), slots.numel(),
                              tile_expert.data_ptr<int>(), tile_expert.numel(),
-                             scratch.data_ptr<int>() + (scratch.numel() - 1), pair_slot.data_ptr<int>(), nullptr,
+                             scratch.data_ptr<int>() + (scratch.numel() - 1), pair_slot.data_ptr<int>(), nullptr, false,
                              stream, nb > 1 ? scratch.data_ptr<int>() : nullptr);
 }
 
@@ -90,7 +90,7 @@ inline void moe_table_align(const at::Tensor& table, const at::Tensor& tokens, i
   at::Tensor count = num_tiles.has_value() ? *num_tiles : at::empty({L}, slots.options());
   hipserve::launch_moe_table_align(table.data_ptr<int>(), L, tokens.data_ptr<long>(), top, table.size(d - 2), npairs, E, tile,
                                    slots.data_ptr<int>(), cap, tile_expert.data_ptr<int>(), tiles, count.data_ptr<int>(),
-                                   pair_slot.data_ptr<int>(), hist.data_ptr<int>(), orders, cur_stream());
+                                   pair_slot.data_ptr<int>(), hist.data_ptr<int>(), num_tiles.has_value() && tile >= 128, orders, cur_stream());
 }
 
 inline bool moe_align_small(int64_t npairs) { return hipserve::moe_align_small(npairs); }

@@ -162,12 +162,52 @@ HS_DEVICE void order_tiles(const int* cnt, const int* off, int E, int tile_shift
   }
 }
 
+// The places of the workgroup's pairs (experts e, pairs first + 1024 i) among their experts' pairs of this wave, which are counted in mine [128]: the same in every
+// run, as those by atomics on counts of the workgroup are not, since these depend on the order between the waves. A place decides about the tile, and the packed
+// GEMM sums k in another order for the tiles that whole rounds leave over: its results were repeated but for the last bits. Bits of the expert are compared over
+// the wave, those that E has; experts past it, which no caller has, are at least not mixed up with others. us, by atomics -> this: 16384 pairs of 8 experts 5.7 -> 5.9, of
+// 128 5.9 -> 6.4, 4096 of 8 4.2 -> 4.9, 2048 3.4 -> 4.2. (Decode steps, whose tiles of 32 are all summed alike, keep the atomics: 96 pairs of four tables 3.0 us, 3.4 this way.)
+template <int PER> HS_DEVICE void wave_places(const int (&e)[PER], int first, int npairs, int E, int* mine, int (&place)[PER]) {
+  const int lane = threadIdx.x & 63;
+  mine[lane] = mine[lane + 64] = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    asm volatile("" ::: "memory");   // other lanes' counts are read: the LDS takes a wave's accesses in order
+    const bool live = first + 1024 * i < npairs;
+    unsigned long same = __ballot(live && e[i] < E);   // the lanes with this expert
+    if (e[i] >= E) same = __ballot(live) & ~same;
+    for (int b = 0; 1 << b < E; ++b) {
+      const unsigned long set = __ballot(e[i] >> b & 1);
+      same &= e[i] >> b & 1 ? set : ~set;
+    }
+    const int before = __popcll(same & ((1UL << lane) - 1)), known = mine[e[i]];
+    place[i] = known + before;
+    asm volatile("" ::: "memory");
+    if (live && before == 0) mine[e[i]] = known + __popcll(same);
+  }
+}
+
+// The counts of 16 waves summed to cnt, and in their place those of the waves before, of the experts 2 lane and 2 lane + 1. One wave.
+HS_DEVICE void wave_totals(int (&part)[16][128], int* cnt) {
+  const int lane = threadIdx.x & 63;
+  int2 n[16], c = {0, 0};
+#pragma unroll
+  for (int w = 0; w < 16; ++w) n[w] = *reinterpret_cast<const int2*>(&part[w][2 * lane]);
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    *reinterpret_cast<int2*>(&part[w][2 * lane]) = c;
+    c.x += n[w].x;
+    c.y += n[w].y;
+  }
+  *reinterpret_cast<int2*>(&cnt[2 * lane]) = c;
+}
+
 // table (may be null): the experts come from table[tokens[t]][j] (top of them per token) instead of ids, without a
 // launch of its own for the lookup (4.5 - 6.3 us); a token outside the table counts as its first entry. Workgroup b serves table b of as many
 // (decode steps: the tables of all layers in one launch, 2.6 - 3.8 us instead of that for each).
 // PER: pairs per thread at most, all looked up at once; a pair's place among its expert's is what the count gives it, and only slots that hold
-// no pair are cleared (96 pairs 3.2 -> 2.6 us beside a second pass that counts again).
-template <int PER>
+// no pair are cleared (96 pairs 3.2 -> 2.6 us beside a second pass that counts again). SAME: places as wave_places has them.
+template <int PER, bool SAME>
 __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__ ids, const int* __restrict__ table,
                                                          const long* __restrict__ tokens, int top, int top_shift, long table_rows,
                                                          int npairs, int E, int tile_shift,
@@ -175,8 +215,9 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
                                                          int* __restrict__ tile_expert, int tiles_cap,
                                                          int* __restrict__ num_tiles, int* __restrict__ pair_slot,
                                                          int* __restrict__ group_end, const MoeOrder order) {
-  __shared__ int cnt[128], off[129];
-  const int tid = threadIdx.x;
+  __shared__ __attribute__((aligned(16))) int part[SAME ? 16 : 1][128], cnt[128];
+  __shared__ int off[129];
+  const int tid = threadIdx.x, wave = tid >> 6;
   const long b = blockIdx.x;
   if (table != nullptr) table += b * table_rows * top;
   slots += b * slots_cap;
@@ -186,19 +227,26 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
   int e[PER], rank[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) e[i] = npairs > 0 ? pair_expert(min(tid + 1024 * i, npairs - 1), ids, table, tokens, top, top_shift, table_rows) : 0;
-  if (tid < 128) cnt[tid] = 0;
-  __syncthreads();
+  if constexpr (SAME) {
+    wave_places<PER>(e, tid, npairs, E, part[wave], rank);
+  } else {
+    if (tid < 128) cnt[tid] = 0;
+    __syncthreads();
 #pragma unroll
-  for (int i = 0; i < PER; ++i)
-    if (tid + 1024 * i < npairs) rank[i] = atomicAdd(&cnt[e[i]], 1);
+    for (int i = 0; i < PER; ++i)
+      if (tid + 1024 * i < npairs) rank[i] = atomicAdd(&cnt[e[i]], 1);
+  }
   __syncthreads();
-  if (tid < 64) padded_offsets(cnt, off, E, tile_shift, num_tiles, group_end, true);
+  if (tid < 64) {
+    if constexpr (SAME) wave_totals(part, cnt);
+    padded_offsets(cnt, off, E, tile_shift, num_tiles, group_end, true);
+  }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int p = tid + 1024 * i;
     if (p < npairs) {
-      const int pos = off[e[i]] + rank[i];
+      const int pos = off[e[i]] + rank[i] + (SAME ? part[wave][e[i]] : 0);
       slots[pos] = p;
       pair_slot[p] = pos;
     }
@@ -221,21 +269,33 @@ __global__ __launch_bounds__(1024) void moe_align_kernel(const int* __restrict__
 // us, one workgroup -> many, in brackets with the lookup of table[token]: 8000 pairs, 16 experts 7.2 -> 5.0 (13.4 -> 5.4), 16384 pairs 11.9 -> 5.2
 // (24.4 -> 5.6), of 128 experts 13.8 -> 6.1 (25.4 -> 6.5), 4097 pairs of 128 experts 5.9 -> 5.6 (with an expert's rest per workgroup, not per wave, 8.9); 4096
 // pairs 4.0 (5.5) on one.
-template <int PER>
+template <int PER, bool SAME>
 __global__ __launch_bounds__(1024) void moe_count_kernel(const int* __restrict__ ids, const int* __restrict__ table, const long* __restrict__ tokens,
-                                                         int top, int top_shift, long table_rows, int npairs, int* __restrict__ pair_slot,
-                                                         int* __restrict__ hist) {
-  __shared__ int cnt[128];
+                                                         int top, int top_shift, long table_rows, int npairs, int E,
+                                                         int* __restrict__ pair_slot, int* __restrict__ hist) {
+  __shared__ __attribute__((aligned(16))) int part[SAME ? 16 : 1][128], cnt[128];
   const int tid = threadIdx.x, b = blockIdx.x, p0 = b * PER * 1024 + tid;
+  [[maybe_unused]] const int wave = tid >> 6;
   int e[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) e[i] = pair_expert(min(p0 + 1024 * i, npairs - 1), ids, table, tokens, top, top_shift, table_rows);
-  if (tid < 128) cnt[tid] = 0;
-  __syncthreads();
+  if constexpr (SAME) {
+    int place[PER];
+    wave_places<PER>(e, p0, npairs, E, part[wave], place);
+    __syncthreads();
+    if (tid < 64) wave_totals(part, cnt);
+    __syncthreads();
 #pragma unroll
-  for (int i = 0; i < PER; ++i)
-    if (p0 + 1024 * i < npairs) pair_slot[p0 + 1024 * i] = e[i] << 16 | atomicAdd(&cnt[e[i]], 1);
-  __syncthreads();
+    for (int i = 0; i < PER; ++i)
+      if (p0 + 1024 * i < npairs) pair_slot[p0 + 1024 * i] = e[i] << 16 | (part[wave][e[i]] + place[i]);
+  } else {
+    if (tid < 128) cnt[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (p0 + 1024 * i < npairs) pair_slot[p0 + 1024 * i] = e[i] << 16 | atomicAdd(&cnt[e[i]], 1);
+    __syncthreads();
+  }
   if (tid < 128) hist[b * 128 + tid] = cnt[tid];
 }
 
@@ -524,30 +584,33 @@ void launch_moe_topk_softmax(const void* logits, bool logits_f32, float* w, int*
                                                                    T, E, k, renorm ? 1 : 0);
 }
 
-// tiles of a power of two; hist: [moe_align_blocks, 128] where that is more than one and there is one table
+// tiles of a power of two; hist: [moe_align_blocks, 128] where that is more than one and there is one table; same: see wave_places
+template <bool SAME>
 static void align(int tables, const int* ids, const int* table, const long* tokens, int top, long table_rows, int npairs, int E, int tile, int* slots,
                   int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, int* hist, const MoeOrder& order, hipStream_t s) {
   const int top_shift = (top & (top - 1)) == 0 ? __builtin_ctz(top) : -1, shift = __builtin_ctz(tile), nb = moe_align_blocks(npairs);
   if (nb > 1 && tables == 1) {
     const bool wide = align_chunk(npairs) > 1024;
-    (wide ? moe_count_kernel<4> : moe_count_kernel<1>)<<<nb, 1024, 0, s>>>(ids, table, tokens, top, top_shift, table_rows, npairs, pair_slot, hist);
+    (wide ? moe_count_kernel<4, SAME> : moe_count_kernel<1, SAME>)<<<nb, 1024, 0, s>>>(ids, table, tokens, top, top_shift, table_rows, npairs, E, pair_slot, hist);
     (wide ? moe_place_kernel<4> : moe_place_kernel<1>)<<<nb, 1024, 0, s>>>(npairs, E, shift, hist, nb, slots, slots_cap, tile_expert, tiles_cap,
                                                                            num_tiles, pair_slot, group_end, order);
     return;
   }
-  (npairs <= 1024 ? moe_align_kernel<1> : npairs <= 4096 ? moe_align_kernel<4> : moe_align_kernel<16>)<<<tables, 1024, 0, s>>>(
+  (npairs <= 1024 ? moe_align_kernel<1, SAME> : npairs <= 4096 ? moe_align_kernel<4, SAME> : moe_align_kernel<16, SAME>)<<<tables, 1024, 0, s>>>(
       ids, table, tokens, top, top_shift, table_rows, npairs, E, shift, slots, slots_cap, tile_expert, tiles_cap, num_tiles, pair_slot, group_end,
       order);
 }
 
 void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
-                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist) {
-  align(1, ids, nullptr, nullptr, 1, 0, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap, num_tiles, pair_slot, group_end, hist, MoeOrder{}, s);
+                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, bool same, hipStream_t s, int* hist) {
+  (same ? align<true> : align<false>)(1, ids, nullptr, nullptr, 1, 0, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap, num_tiles, pair_slot, group_end,
+                                      hist, MoeOrder{}, s);
 }
 
-void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile,
-                            int* slots, int slots_cap, int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot, int* hist, const MoeOrder& order, hipStream_t s) {
-  align(tables, nullptr, table, tokens, top, table_rows, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap, num_tiles, pair_slot, nullptr, hist, order, s);
+void launch_moe_table_align(const int* table, int tables, const long* tokens, int top, long table_rows, int npairs, int E, int tile, int* slots, int slots_cap,
+                            int* tile_expert, int tiles_cap, int* num_tiles, int* pair_slot, int* hist, bool same, const MoeOrder& order, hipStream_t s) {
+  (same ? align<true> : align<false>)(tables, nullptr, table, tokens, top, table_rows, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap, num_tiles,
+                                      pair_slot, nullptr, hist, order, s);
 }
 
 // Prefill MoE input: xs[slot] = x[slots[slot] / k] (the token of the pair in that

@@ -321,3 +321,32 @@ def test_order_of_tiles_for_whole_rounds(counts, across, per_round):
     gone = {t for _, t in moved}
     assert place.tolist() == [t for t in range(n) if t not in gone] + [t for _, t in moved]
     assert not moved or left == list(range(left[0], n))   # they are the last places
+
+
+@pytest.mark.parametrize("P", [1, 65, 1024, 1025, 4096, 4097, 16384, 65537])
+@pytest.mark.parametrize("E", [1, 2, 16, 100, 128])
+def test_alignments_for_the_packed_gemm_repeat(P, E):
+    """A pair has the same place in every run, whatever the order of the waves, and every pair one of its expert's: with a table and without one."""
+    from hipserve.ops import get_ops
+
+    op, g = torch.ops.hipserve, torch.Generator(device=DEV).manual_seed(P + E)
+    ids = (torch.randint(0, E, (P,), device=DEV, generator=g) if E < 100 else (torch.rand(P, device=DEV, generator=g) ** 3 * E).long()).int()
+    cap = -(-(P + E * 127) // 128) * 128
+    first = None
+    for _ in range(6):
+        runs = []
+        for table in (False, True) if P <= 16384 else (False,):
+            slots, te, nt, ps = (torch.full((n,), -7, dtype=torch.int32, device=DEV) for n in (cap, cap // 128, 1, P))
+            if table:
+                get_ops("cuda").moe_table_align(ids.view(-1, 1), torch.arange(P, device=DEV), E, 128, slots, te, ps, nt)
+            else:
+                op.moe_align(ids, E, 128, slots, te, nt, ps)
+            runs.append((slots, te, nt, ps))
+        first = first or runs
+        assert all(torch.equal(a, b) for x, y in zip(first, runs) for a, b in zip(x, y))
+    for slots, te, nt, ps in first:
+        assert torch.equal(slots[ps.long()], torch.arange(P, device=DEV).int()) and int((slots >= 0).sum()) == P
+        assert torch.equal(te[ps.long() // 128], ids)
+        live = slots.view(-1, 128) >= 0   # a tile is filled from its first slot on
+        assert bool((live[:, 1:] <= live[:, :-1]).all())
+        assert int(nt) == int((-(-torch.bincount(ids, minlength=E) // 128)).sum())
