@@ -1,7 +1,8 @@
 // A dense product of a few rows and the experts' product of the same step in one launch, where neither reads what the other writes (a parallel block:
 // the mixer's products and the experts' both start from the block's norm). A launch of its own costs each at least 1.6 us, which is what empty ones
 // in a captured graph take, and about 1 us more until its first loads are back, while the other product would keep the memory busy. The dense
-// product's workgroups come first, since they are fewer and longer; every workgroup runs what its own launch would, the sums are the same bits.
+// product's workgroups come first, since they are fewer and longer. The sums are the bits of the two launches; a dense workgroup may take other columns and
+// copy fewer pieces ahead than in a launch of its own (skinny_cols and skinny_wide are not asked here).
 //
 // What bounds it is the memory once the two overlap, and the LDS of the larger workgroup, which all get: with one workgroup per compute unit (more than 80
 // KB) the experts lose more than the launch costs, so dense workgroups of more than 16 rows copy one piece ahead. us apart -> in one launch, in a captured
@@ -41,6 +42,15 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_experts_kernel(
   skinny_block<XG, NT, DEPTH, false, TO, false, kPlain, HALF>(b, 0, part, x, w, nullptr, nullptr, x_ld, M, N, K, ni, offsetof(BesideArgs, rest), smem);
 }
 
+// Whether the two are faster together where a compute unit has room for two of these workgroups and not for three, which is what the experts have on their
+// own: not where thousands of theirs are of a short k, whose start is what they take, nor where the dense ones are many. us apart -> in one launch, 40 rows: 16 experts
+// of 4096 x 1024 beside 8192 x 2048 35.8 -> 41.0, 64 of 1024 x 512 22.8 -> 25.7; 16 of 2048 x 1024 beside 4096 x 2048 22.0 -> 22.8, of 1024 x 1024 16.0 -> 15.6. Of 1306
+// sizes (1 - 64 rows, 2 M - 32 M dense weights, experts of k 512 - 4096) 488 are left apart for these bounds; of the others one takes more than 1 % longer than apart
+// (33 rows, 2.8 %), and all take 17 % less on average; without the bounds 307 do, up to 15 %. With room for three, all were faster together.
+bool two_per_unit_pay(const ExpertRows& ex, long wgs, int K, int split) {
+  return ex.K >= 2048 || wgs <= 512 || (wgs <= 1536 && K <= 2048 && split <= 384) || (wgs <= 2560 && split <= 160);
+}
+
 template <int XG, int NT, int DEPTH, typename TO, bool HALF = false>
 bool launch_beside(void* out, long out_ld, long out_zs, int parts, const void* x, long x_ld, const void* w, int M, int N, int K,
                    const ExpertRows& ex, hipStream_t s) {
@@ -49,6 +59,7 @@ bool launch_beside(void* out, long out_ld, long out_zs, int parts, const void* x
   if (!ok) return false;
   const int split = (N + per - 1) / per * parts;
   const ExpertBeside experts = expert_beside_args(ex);
+  if (3 * lds > 160 * 1024 && !two_per_unit_pay(ex, experts.per_tile * ex.ntiles, K, split)) return false;
   skinny_linear_experts_kernel<XG, NT, DEPTH, TO, HALF><<<split + experts.per_tile * ex.ntiles, kSkThreads, lds, s>>>(
       (const unsigned short*)x, (const unsigned short*)w, ex.slots, ex.tile_expert, (int)x_ld, M, N, K, ((K + 63) / 64 + parts - 1) / parts * 64, split,
       SkinnyRest<kPlain>{0, out_ld, 0, out_zs, -1, 0, 0.f, 0.f, 1.f, 0.f, out, nullptr, nullptr}, experts);

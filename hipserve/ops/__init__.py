@@ -689,8 +689,8 @@ class KernelOps:
         return self._skinny_time(rows, cols, k, False, f32, p) + (p > 1) * 0.7 + (p - 1) * (0.15 + 0.2e-5 * rows * cols)
 
     def _linear_beside(self, x, w, beside, parts=1):
-        """The product x . w^T in one launch with the next product of ``beside``, or None. What would be ``parts`` of k without it is one, still in 32
-        bits: the experts fill the compute units that parts are for. From 33 rows on such a product holds a compute unit for longer than the launch saves:
+        """The product x . w^T in one launch with the next product of ``beside``, or None (also where they are faster apart for the numbers of their
+        workgroups: expert_beside.hip). What would be ``parts`` of k without it is one, still in 32 bits: the experts fill the compute units that parts are for. From 33 rows on such a product holds a compute unit for longer than the launch saves:
         16 experts of 2048 x 1024 beside 2048 x 4096, us apart / in one launch: 32 rows 20.6 / 19.3, 48 rows 21.9 / 23.6, 64 rows 23.0 / 25.6; 8 of
         1024 x 512 beside 1024 x 2048, 40, 64 rows 7.9 / 6.4, 8.5 / 7.6."""
         if parts > 1 and x.shape[0] > 32 and w.numel() > 1 << 21:
