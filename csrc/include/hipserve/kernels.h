@@ -267,7 +267,7 @@ void launch_moe_topk_softmax(const void* logits, bool logits_f32, float* w, int*
                              bool renorm, hipStream_t s, int splits = 0);
 // same: pairs take the same places in every run, for GEMMs that sum some tiles in another order (the packed one)
 void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
-                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, bool same, hipStream_t s, int* hist);
+                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist, bool same = false);
 // m-tiles of a group of the packed GEMM's tiles, which it walks column by column (prefill_gemm_packed.hip)
 constexpr int kTileGroup = 8;
 // Orders of the tiles for GEMMs of across[j] tiles beside each other that take per_round[j] tiles at once (one table): to [rows, tiles] int32,

@@ -43,7 +43,7 @@ inline void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor
   at::Tensor scratch = at::empty({(long)(nb > 1 ? nb : 0) * 128 + 1}, ids.options());  // [hist | tile count]
   hipserve::launch_moe_align(ids.data_ptr<int>(), npairs, E, tile, slots.data_ptr<int>(), slots.numel(),
                              tile_expert.data_ptr<int>(), tile_expert.numel(),
-                             scratch.data_ptr<int>() + (scratch.numel() - 1), pair_slot.data_ptr<int>(), nullptr, false,
+                             scratch.data_ptr<int>() + (scratch.numel() - 1), pair_slot.data_ptr<int>(), nullptr,
                              stream, nb > 1 ? scratch.data_ptr<int>() : nullptr);
 }
 

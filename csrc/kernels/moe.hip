@@ -602,7 +602,7 @@ static void align(int tables, const int* ids, const int* table, const long* toke
 }
 
 void launch_moe_align(const int* ids, int npairs, int E, int tile, int* slots, int slots_cap, int* tile_expert,
-                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, bool same, hipStream_t s, int* hist) {
+                      int tiles_cap, int* num_tiles, int* pair_slot, int* group_end, hipStream_t s, int* hist, bool same) {
   (same ? align<true> : align<false>)(1, ids, nullptr, nullptr, 1, 0, npairs, E, tile, slots, slots_cap, tile_expert, tiles_cap, num_tiles, pair_slot, group_end,
                                       hist, MoeOrder{}, s);
 }

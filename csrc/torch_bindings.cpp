@@ -1139,7 +1139,7 @@ void moe_align(const at::Tensor& ids, int64_t E, int64_t tile, at::Tensor& slots
   if (nb > 1) hist = at::empty({(long)nb * 128}, ids.options().dtype(at::kInt));
   hipserve::launch_moe_align(ids.data_ptr<int>(), npairs, E, tile, slots.data_ptr<int>(), slots.numel(),
                              tile_expert.data_ptr<int>(), tile_expert.numel(), num_tiles.data_ptr<int>(),
-                             pair_slot.data_ptr<int>(), ge, tile >= 128, cur_stream(), nb > 1 ? hist.data_ptr<int>() : nullptr);
+                             pair_slot.data_ptr<int>(), ge, cur_stream(), nb > 1 ? hist.data_ptr<int>() : nullptr, tile >= 128);
 }
 
 void moe_gather(at::Tensor& out, const at::Tensor& x, const at::Tensor& slots, int64_t k) {
