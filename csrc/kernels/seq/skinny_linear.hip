@@ -118,21 +118,23 @@ bool skinny_half(int M, long tiles, int K) {
 // rows: 6144 x 2048 7.7 -> 7.0, 8.0 -> 7.5, 9.9 -> 9.2, 5120 x 4096 12.4 -> 10.2, 13.1 -> 11.2, 15.8 -> 14.4 (24 columns); 10240 x 3072 15.1 -> 13.0, 18.0 ->
 // 13.6, 22.7 -> 16.8 (40); 12288 x 4096, 24, 48 rows 22.5 -> 21.1, 25.5 -> 23.6 (48); 13376 x 3072 18.8 -> 16.6, 19.8 -> 17.4, 24.0 -> 20.7 (56); 20480 x 2048, 24
 // rows 19.6 -> 18.4 (40, two rounds). A short k is latency, and wider workgroups sum more tiles: 4104 x 1024, 16 rows 4.1 -> 4.6; 8200 x 2048, 16 rows 9.2 -> 9.2;
-// 13376 x 2048, 24 rows 14.1 -> 14.3; 20480 x 2048, 48 rows 23.3 -> 24.4: these stay. Of 320 sizes (16 - 48 rows, 4104 - 32000 columns, k 512 - 4096) 150 are
-// taken, none of which got slower by more than 1.1 %.
+// 13376 x 2048, 24 rows 14.1 -> 14.3; 20480 x 2048, 48 rows 23.3 -> 24.4: these stay. Nor for 9 - 12 rows where the others are taken for 16: fewer rows are less
+// to share, above all where those of the weights lie 4096 bytes apart (9, 12, 16 rows: 11264 x 3328 15.6 -> 16.3, 16.1 -> 16.1, 17.3 -> 16.3; 11264 x 6144 26.8 -> 30.6, 28.2 -> 30.7, 30.4 ->
+// 30.7; 28672 x 3072 30.5 -> 32.1, 31.9 -> 32.1, 34.5 -> 32.0). Of 2770 sizes (9 - 48 rows, 4104 - 32000 columns, k 512 - 10240) 1480 are taken, which take 10 % less
+// on average and at most 2 % more.
 int skinny_cols(int M, long cols, int K) {
   const long tiles = (cols + 15) / 16;
   if (M <= 8 || M > 48 || tiles <= 256 || tiles > 1792) return 0;
   if (tiles <= 384) return K >= (M > 16 ? 1024 : 2048) ? 24 : 0;
   if (tiles <= 512) return 0;
   if (tiles <= 768) {
-    if (M <= 16 && (K < 3072 || tiles > 704)) return 0;
+    if (M <= 16 && (K < 3072 || tiles > (M <= 12 ? 672 : 704) || ((M <= 12 || tiles > 640) && K % 2048 == 0))) return 0;
     return K >= 1024 && !(tiles <= 544 && K < 2048) ? tiles <= 640 ? 40 : 48 : 0;
   }
   if (tiles <= 896) return K >= 3072 && K < (M <= 16 ? 4096 : 1 << 30) ? 56 : 0;
   if (tiles <= 1024) return 0;
   if (tiles <= 1280) return M > 16 && K >= (M > 32 ? 3072 : 1024) ? 40 : 0;
-  return tiles > 1536 && K >= 3072 && K < (M <= 16 ? 4096 : 1 << 30) ? 56 : 0;
+  return tiles > 1536 && M > 12 && K >= 3072 && K < (M <= 16 ? 4096 : 1 << 30) ? 56 : 0;
 }
 
 // Of up to 8 rows and more workgroups than compute units: how many pieces a workgroup of one whole tile copies ahead where three are best (0: by the rules of

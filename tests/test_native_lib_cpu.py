@@ -156,6 +156,17 @@ def test_an_update_takes_the_columns_that_its_product_would():
 
 
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
+@pytest.mark.parametrize("rows,cols,k,faster", [
+    (9, 11264, 6144, False), (12, 10752, 6144, False), (10, 11264, 4096, False), (13, 11264, 6144, False), (9, 28672, 3072, False), (11, 27648, 3328, False), (9, 10240, 6144, False),
+    (16, 6144, 2048, True), (9, 6144, 2048, True), (9, 8704, 3072, True), (12, 10304, 3584, True), (13, 11264, 3072, True), (16, 28672, 3072, True), (16, 8704, 6144, True),
+    (33, 8704, 3328, True), (24, 12288, 4096, True), (48, 13376, 3072, True), (24, 20480, 2048, True), (48, 20480, 2048, False), (16, 8200, 2048, False), (16, 4104, 1024, False)])
+def test_columns_of_a_workgroup_by_whole_rounds(rows, cols, k, faster):
+    """Sizes at which 24 - 56 columns per workgroup were measured to take at least 3 % less than whole tiles (``faster``), or no less."""
+    load_kernel_library("seq")
+    assert (torch.ops.hipserve_seq.skinny_cols(rows, cols, k) > 0) == faster
+
+
+@pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
 @pytest.mark.parametrize("rows,cols,k,f32,glu,pays", [
     (1, 2048, 2048, False, False, True), (48, 2048, 2048, False, False, True), (64, 6144, 1024, False, False, True), (16, 32000, 1024, True, False, True),
     (48, 512, 8192, False, False, False), (40, 576, 12288, False, False, False), (64, 32768, 128, False, False, False), (64, 65536, 512, False, False, False),
