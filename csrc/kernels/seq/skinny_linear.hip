@@ -138,15 +138,17 @@ int skinny_cols(int M, long cols, int K) {
 }
 
 // Of up to 8 rows and more workgroups than compute units: how many pieces a workgroup of one whole tile copies ahead where three are best (0: by the rules of
-// the launch), and whether half tiles are better still. Three are for k (in halves) of 2048 and more, once the units have two workgroups each; half tiles are for rows
-// of weights 4096 bytes apart, of which eight per load and workgroup go to the same channels and not sixteen, as long as the rows that they read twice as
-// often are few. Cold weights, us, one row, before -> three pieces -> half tiles: 8192 x 2048 8.4 -> 7.9 -> 7.3, 12288 x 2048 11.0 -> 10.5 -> 9.9, 32000 x 2048 23.9 ->
-// 22.7 -> 22.3, 8192 x 4096 13.9 -> 12.8 -> 13.6, 12288 x 4096 18.6 -> 17.9 -> 19.1, 32000 x 3072 32.8 -> 32.2 -> 32.5; 8 rows, 32000 x 2048 24.0 -> 23.4 -> 24.3; in 32
-// bits, 32000 x 1024 24.5 -> 23.5 -> 26.7. As they were: 5152 x 2048 6.1 (half tiles 6.2), 8192 x 3072 9.7 (10.0), 32000 x 1024 11.8 (15).
-struct SkinnyWide { int ahead; bool half; };
-static SkinnyWide skinny_wide(int M, long tiles, int K, bool f32) {
+// the launch), and whether half tiles are better still. Three are for k (in halves) of 2048 and more, once the units have two workgroups each; half tiles are for up to 4
+// rows and weights whose rows lie a power of two of bytes apart, 4096 or 16384 and more, where whole tiles' loads of 16 rows meet on fewer channels. (8192 apart
+// they take 2 - 10 % longer, for which there is no reason but the measurement; at other multiples of 4096 they gain 2 % on average and lose up to 7; rows a little off
+// such places are as fast in whole tiles.) 105 sizes of 5632 - 32000 columns, k 2048, 8192 and 16384, 1 - 4 rows: 10 % less than whole tiles on average, one 3.6 %
+// more. Cold weights, us, one row, one or two pieces / three / half tiles: 8192 x 2048 9.2 / 8.2 / 7.5, 12288 x 2048 12.3 / 11.2 / 10.1, 32000 x 2048 25.8 / 23.9 / 22.1, 32000 x
+// 1984 21.7 / 22.1 / 21.4, 32000 x 2112 22.8 / 23.0 / 22.7, 8192 x 4096 14.2 / 13.2 / 13.9, 12288 x 4096 19.3 / 18.5 / 19.4, 8192 x 8192 28.8 / 27.1 / 24.0, 12288 x 8192 39.4 / 38.5 /
+// 34.1; 8 rows, 32000 x 2048 26.3 / 25.0 / 24.7; in 32 bits, 32000 x 1024 26.2 / 24.5 / 26.5. As they were: 5152 x 2048 6.5 (half tiles 6.4), 8192 x 3072 10.0 (10.3).
+SkinnyWide skinny_wide(int M, long tiles, int K, bool f32) {
   if (M > 8 || K < 2048) return {0, false};
-  if (M <= 4 && !f32 && K == 2048 && tiles > 352) return {2, true};
+  const bool apart = (K & (K - 1)) == 0 && K % 8192 != 4096;
+  if (M <= 4 && !f32 && apart && tiles > 352) return {K > 4096 ? 3 : 2, true};
   return {tiles > 512 || (tiles > 384 && K % 2048 == 0) ? 3 : 0, false};
 }
 
@@ -193,7 +195,7 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
 #undef HS_S16
   }
   if (const auto wide = batch == 1 && parts == 1 ? skinny_wide(M, tiles, K, f32) : SkinnyWide{}; wide.ahead > 0)
-    return wide.half ? HS_SK(1, 1, 2, false, true) : HS_SK(1, 1, 3, false);
+    return !wide.half ? HS_SK(1, 1, 3, false) : wide.ahead > 2 ? HS_SK(1, 1, 3, false, true, 2) : HS_SK(1, 1, 2, false, true);
   const int nt = skinny_tiles(M, tiles, K / parts);
   // One piece ahead: two are faster (up to 40 %) where a wave waits for its few copies, up to 16 rows and more than a piece per wave (more than
   // two where a compute unit holds several workgroups: 12288 x 1024, 16 rows 9 % slower; 3072 x 1024, one row 4 % faster), and slower
@@ -241,6 +243,7 @@ static bool launch_normed(void* out, bool out_f32, const SkinnyNorm& norm, const
 #undef HS_SG
     }
     if (const auto wide = skinny_wide(M, (N + 15) / 16, K, f32); wide.ahead > 0) {
+      if (wide.half && wide.ahead > 2) return out_f32 ? HS_SN(1, 1, 3, false, Wide, false, true) : HS_SN(1, 1, 3, false, unsigned short, false, true);
       if (wide.half) return out_f32 ? HS_SN(1, 1, 2, false, Wide, false, true) : HS_SN(1, 1, 2, false, unsigned short, false, true);
       return f32 ? HS_SN(1, 1, 3, false, float, true, false) : out_f32 ? HS_SN(1, 1, 3, false, Wide, false, false)
            : HS_SN(1, 1, 3, false, unsigned short, false, false);

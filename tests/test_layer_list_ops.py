@@ -359,6 +359,26 @@ def test_products_of_many_columns(M, N, K, dtype):
         assert err.max() < (0.02 if dt == torch.bfloat16 else 1e-4)   # what lies between them: no column left out (a result rounded to 2^-9, of rows rounded to 2^-9; 32-bit sums)
 
 
+@gpu
+@pytest.mark.parametrize("normed", [False, True])
+@pytest.mark.parametrize("M,N,K", [(1, 5648, 8192), (4, 6137, 8192), (3, 5640, 16384)])
+def test_half_tiles_of_wide_products_are_exact(M, N, K, normed):
+    """Three pieces ahead: the bits of the columns' products alone at either end, and in between what 64 bits give."""
+    g = torch.Generator("cuda").manual_seed(M + N)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()  # noqa: E731
+    x, w, b, ops, n = rand(M, K), rand(N, K) / 64, rand(N), get_ops("cuda"), 200
+    assert ops._moe_lib.skinny_wide(M, N, K, False) == [3, True]
+    out, first, last = (torch.empty(M, c, dtype=x.dtype, device="cuda") for c in (N, n, n))
+    for o, a, z in ((out, w, b), (first, w[:n], b[:n]), (last, w[-n:], b[-n:])):
+        if normed:
+            ops._moe_lib.skinny_linear_normed(o, x, torch.full((M, 256), K / 256, device="cuda"), 1e-6, a, z, -1, 0.0, 0.0, 0)
+        else:
+            ops._moe_lib.skinny_linear(o, x, a, z, -1, 0.0, 0.0)
+    assert torch.equal(out[:, :n], first) and torch.equal(out[:, -n:], last)
+    want = x.double() @ w.double().t() * (1 / (1 + 1e-6) ** 0.5 if normed else 1) + b.double()
+    assert ((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + K * 2.0 ** -23 * (x.double().abs() @ w.double().abs().t())).all()
+
+
 @pytest.mark.parametrize("rows,cols,k,cut", [
     (8192, 6176, 1024, 6144), (8192, 26688, 4096, 26624), (7900, 4128, 2048, 4096), (2048, 8200, 1024, 8192), (1024, 16512, 64, 16384), (1100, 13072, 64, 13056),
     (8192, 2656, 4096, 2048), (8192, 6288, 2048, 6144), (2048, 10304, 2048, 8192), (4073, 13376, 4096, 12288),   # some columns more

@@ -156,6 +156,20 @@ def test_an_update_takes_the_columns_that_its_product_would():
 
 
 @pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
+@pytest.mark.parametrize("k,half", [(1024, False), (1792, False), (1984, False), (2048, True), (2112, False), (2304, False), (2560, False), (4096, False), (6144, False),
+                                    (8192, True), (12288, False), (16384, True)])
+def test_half_tiles_of_wide_products(k, half):
+    """By the distance of the weights' rows, as measured: a class of them, not one, and neither their neighbours nor more rows, 32 bits or fewer workgroups."""
+    load_kernel_library("seq")
+    wide = torch.ops.hipserve_seq.skinny_wide
+    for cols in (5648, 8192, 32000):
+        for rows in (1, 4):
+            assert wide(rows, cols, k, False) == [(2 if k <= 4096 else 3) if half else 0 if k < 2048 or cols == 5648 or (cols <= 8192 and k % 2048) else 3, half], (rows, cols)
+        assert not wide(5, cols, k, False)[1] and not wide(1, cols, k // 2, True)[1] and wide(9, cols, k, False) == [0, False]
+    assert wide(1, 5632, k, False) == [0, False]
+
+
+@pytest.mark.skipif(not os.path.exists(_SEQ_LIBS["seq"]), reason="hipserve/_C_seq.so not built")
 @pytest.mark.parametrize("rows,cols,k,faster", [
     (9, 11264, 6144, False), (12, 10752, 6144, False), (10, 11264, 4096, False), (13, 11264, 6144, False), (9, 28672, 3072, False), (11, 27648, 3328, False), (9, 10240, 6144, False),
     (16, 6144, 2048, True), (9, 6144, 2048, True), (9, 8704, 3072, True), (12, 10304, 3584, True), (13, 11264, 3072, True), (16, 28672, 3072, True), (16, 8704, 6144, True),
