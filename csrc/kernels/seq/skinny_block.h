@@ -3,6 +3,7 @@
 #pragma once
 #include <type_traits>
 
+#include "hipserve/seq_kernels.h"
 #include "skinny.h"
 
 namespace hipserve {
@@ -177,6 +178,22 @@ HS_DEVICE void skinny_block(int bx, int by, int bz, const unsigned short* __rest
       }
     }
   }
+}
+
+// launch.run<XG, NT, DEPTH, F32, HALF>() for a kUpdate product of up to 32 rows, K in halves: one rule for its launches. The number of its squares' blocks says
+// whether its workgroups are to take 8 columns. Two pieces ahead for one tile, but for more than 16 rows of 32 bits: a decode step of 20 rows (width
+// 1024) 122.4 us with two, 124.2 with one, in 32 bits 167.1 and 166.0, of 32 rows 128.4 and 130.0, 173.7 and 170.0.
+template <bool F32, typename L> bool run_update(const L& launch, int M, int N, int K, int blocks) {
+  if (blocks == N / 8) {
+    if (M <= 8) return K > 4096 ? launch.template run<1, 1, 3, F32, true>() : launch.template run<1, 1, 2, F32, true>();
+    return M <= 16 ? launch.template run<2, 1, 2, F32, true>() : launch.template run<4, 1, 2, F32, true>();
+  }
+  const int nt = skinny_tiles(M, (N + 15) / 16, K);   // 4 above 16 rows alone; N is a multiple of 64
+  if (nt == 4) return launch.template run<4, 4, 1, F32, false>();
+  if (nt == 2)
+    return M <= 8 ? launch.template run<1, 2, 1, F32, false>() : M <= 16 ? launch.template run<2, 2, 1, F32, false>() : launch.template run<4, 2, 1, F32, false>();
+  return M <= 8 ? launch.template run<1, 1, 2, F32, false>() : M <= 16 ? launch.template run<2, 1, 2, F32, false>()
+       : launch.template run<4, 1, F32 ? 1 : 2, F32, false>();
 }
 
 }  // namespace

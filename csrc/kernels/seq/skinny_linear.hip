@@ -209,47 +209,39 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
 #undef HS_SK
 }
 
-template <int NORM>
+// The products of rows without their norm's factor (kNormed), K in halves.
 static bool launch_normed(void* out, bool out_f32, const SkinnyNorm& norm, const void* x, long x_ld, const void* w, const void* bias,
                           bool f32, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
-  if (f32) { x_ld *= 2; K *= 2; }   // in halves
   const bool glu = act == 3 || act == 4;
   const long No = glu ? N / 2 : N;
 #define HS_SN(XG, NT, DEPTH, GLU, TO, F32, HALF)                                                                                              \
-  launch_kernel<XG, NT, DEPTH, GLU, TO, F32, NORM, HALF>(dim3((No + (GLU ? 16 : 16 * NT - 8 * HALF) - 1) / (GLU ? 16 : 16 * NT - 8 * HALF)), out, No, \
-                                                         0, 0, x, x_ld, 0, w, bias, M, N, K, act, act_from, c0, c1, s, norm)
+  launch_kernel<XG, NT, DEPTH, GLU, TO, F32, kNormed, HALF>(dim3((No + (GLU ? 16 : 16 * NT - 8 * HALF) - 1) / (GLU ? 16 : 16 * NT - 8 * HALF)), out, No, \
+                                                            0, 0, x, x_ld, 0, w, bias, M, N, K, act, act_from, c0, c1, s, norm)
 #define HS_SX(NT, D, GLU, TO, F32) \
   (M <= 8 ? HS_SN(1, NT, D, GLU, TO, F32, false) : M <= 16 ? HS_SN(2, NT, D, GLU, TO, F32, false) : HS_SN(4, NT, F32 ? 1 : D, GLU, TO, F32, false))
 #define HS_SH(TO, F32)                                                                                                              \
   (M <= 8 ? K > 4096 ? HS_SN(1, 1, 3, false, TO, F32, true) : HS_SN(1, 1, 2, false, TO, F32, true)                                  \
           : M <= 16 ? HS_SN(2, 1, 2, false, TO, F32, true) : HS_SN(4, 1, 2, false, TO, F32, true))
-  using Wide = std::conditional_t<NORM == kNormed, float, unsigned short>;   // an update writes rows of the operands' type
-#define HS_ST(NT, D, GLU) (f32 ? HS_SX(NT, D, GLU, float, true) : out_f32 ? HS_SX(NT, D, GLU, Wide, false) : HS_SX(NT, D, GLU, unsigned short, false))
+#define HS_ST(NT, D, GLU) (f32 ? HS_SX(NT, D, GLU, float, true) : out_f32 ? HS_SX(NT, D, GLU, float, false) : HS_SX(NT, D, GLU, unsigned short, false))
 #define HS_S4() \
-  (f32 ? HS_SN(4, 4, 1, false, float, true, false) : out_f32 ? HS_SN(4, 4, 1, false, Wide, false, false) : HS_SN(4, 4, 1, false, unsigned short, false, false))
-  // Two pieces ahead for one tile, but for more than 16 rows of 32 bits: a decode step of 20 rows (width 1024) 122.4 us with two, 124.2 with
-  // one, in 32 bits 167.1 and 166.0, of 32 rows 128.4 and 130.0, 173.7 and 170.0.
-  if constexpr (NORM == kNormed)
-    if (glu) return HS_ST(2, 1, true);
-  // where squares are written, their number says what the workgroups are to take
-  if (NORM == kUpdate ? norm.blocks == N / 8 : skinny_half(M, (N + 15) / 16, K))
-    return f32 ? HS_SH(float, true) : out_f32 ? HS_SH(Wide, false) : HS_SH(unsigned short, false);
-  if constexpr (NORM == kNormed) {
-    if (const int cols = f32 ? 0 : skinny_cols(M, N, K)) {
+  (f32 ? HS_SN(4, 4, 1, false, float, true, false) : out_f32 ? HS_SN(4, 4, 1, false, float, false, false) : HS_SN(4, 4, 1, false, unsigned short, false, false))
+  if (glu) return HS_ST(2, 1, true);
+  if (skinny_half(M, (N + 15) / 16, K)) return f32 ? HS_SH(float, true) : out_f32 ? HS_SH(float, false) : HS_SH(unsigned short, false);
+  if (const int cols = f32 ? 0 : skinny_cols(M, N, K)) {
 #define HS_SG(NT, HALF, TO) (M <= 16 ? HS_SN(2, NT, 1, false, TO, false, HALF) : HS_SN(4, NT, 1, false, TO, false, HALF))
-#define HS_SO(NT, HALF) (out_f32 ? HS_SG(NT, HALF, Wide) : HS_SG(NT, HALF, unsigned short))
-      return cols == 24 ? HS_SO(2, true) : cols == 40 ? HS_SO(3, true) : cols == 48 ? HS_SO(3, false) : HS_SO(4, true);
+#define HS_SO(NT, HALF) (out_f32 ? HS_SG(NT, HALF, float) : HS_SG(NT, HALF, unsigned short))
+    return cols == 24 ? HS_SO(2, true) : cols == 40 ? HS_SO(3, true) : cols == 48 ? HS_SO(3, false) : HS_SO(4, true);
 #undef HS_SO
 #undef HS_SG
-    }
-    if (const auto wide = skinny_wide(M, (N + 15) / 16, K, f32); wide.ahead > 0) {
-      if (wide.half && wide.ahead > 2) return out_f32 ? HS_SN(1, 1, 3, false, Wide, false, true) : HS_SN(1, 1, 3, false, unsigned short, false, true);
-      if (wide.half) return out_f32 ? HS_SN(1, 1, 2, false, Wide, false, true) : HS_SN(1, 1, 2, false, unsigned short, false, true);
-      return f32 ? HS_SN(1, 1, 3, false, float, true, false) : out_f32 ? HS_SN(1, 1, 3, false, Wide, false, false)
-           : HS_SN(1, 1, 3, false, unsigned short, false, false);
-    }
   }
-  const int nt = skinny_tiles(M, (N + 15) / 16, K);   // 4 above 16 rows alone; where squares are written, N is a multiple of 64
+  if (const auto wide = skinny_wide(M, (N + 15) / 16, K, f32); wide.ahead > 0) {
+    if (wide.half && wide.ahead > 2) return out_f32 ? HS_SN(1, 1, 3, false, float, false, true) : HS_SN(1, 1, 3, false, unsigned short, false, true);
+    if (wide.half) return out_f32 ? HS_SN(1, 1, 2, false, float, false, true) : HS_SN(1, 1, 2, false, unsigned short, false, true);
+    return f32 ? HS_SN(1, 1, 3, false, float, true, false) : out_f32 ? HS_SN(1, 1, 3, false, float, false, false)
+         : HS_SN(1, 1, 3, false, unsigned short, false, false);
+  }
+  // Pieces ahead for one tile: as run_update has them.
+  const int nt = skinny_tiles(M, (N + 15) / 16, K);   // 4 above 16 rows alone
   return nt == 4 ? HS_S4() : nt == 2 ? HS_ST(2, 1, false) : HS_ST(1, 2, false);
 #undef HS_S4
 #undef HS_SH
@@ -258,11 +250,32 @@ static bool launch_normed(void* out, bool out_f32, const SkinnyNorm& norm, const
 #undef HS_SN
 }
 
+namespace {
+
+// A residual update's launch: rows of the operands' type.
+struct UpdateLaunch {
+  void* out;
+  const SkinnyNorm& norm;
+  const void *x, *w, *bias;
+  long x_ld;
+  int M, N, K;
+  hipStream_t s;
+  template <int XG, int NT, int DEPTH, bool F32, bool HALF> bool run() const {
+    constexpr int per = 16 * NT - 8 * HALF;
+    return launch_kernel<XG, NT, DEPTH, false, std::conditional_t<F32, float, unsigned short>, F32, kUpdate, HALF>(
+        dim3((N + per - 1) / per), out, N, 0, 0, x, x_ld, 0, w, bias, M, N, K, -1, 0, 0.f, 0.f, s, norm);
+  }
+};
+
+}  // namespace
+
 bool launch_skinny_linear_normed(void* out, bool out_f32, const SkinnyNorm& norm, const void* x, long x_ld, const void* w, const void* bias,
                                  bool f32, int M, int N, int K, int act, int act_from, float c0, float c1, hipStream_t s) {
   if (M <= 0 || N <= 0) return true;
-  auto go = norm.residual != nullptr ? launch_normed<kUpdate> : launch_normed<kNormed>;
-  return go(out, out_f32, norm, x, x_ld, w, bias, f32, M, N, K, act, act_from, c0, c1, s);
+  if (f32) { x_ld *= 2; K *= 2; }   // in halves
+  if (norm.residual == nullptr) return launch_normed(out, out_f32, norm, x, x_ld, w, bias, f32, M, N, K, act, act_from, c0, c1, s);
+  const UpdateLaunch l{out, norm, x, w, bias, x_ld, M, N, K, s};
+  return f32 ? run_update<true>(l, M, N, K, norm.blocks) : run_update<false>(l, M, N, K, norm.blocks);
 }
 
 }  // namespace hipserve

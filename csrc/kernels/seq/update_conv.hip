@@ -39,18 +39,25 @@ __global__ __launch_bounds__(kSkThreads) void skinny_update_conv_kernel(
   skinny_block<XG, NT, DEPTH, false, T, F32, kUpdate, HALF>(b, 0, 0, x, w, p, q, x_ld, M, N, K, ni, offsetof(UpdateConvArgs, rest), smem);
 }
 
-template <int XG, int NT, int DEPTH, bool F32, bool HALF>
-bool launch(void* out, const SkinnyNorm& norm, const void* x, long x_ld, const void* w, const void* bias, int M, int N, int K, const ConvUpdate& conv,
-            int nseq, hipStream_t s) {
-  constexpr int lds = Skinny<XG, NT, DEPTH, F32, HALF>::kLds, per = HALF ? 8 : 16 * NT;
-  static const bool ok = allow_lds(&skinny_update_conv_kernel<XG, NT, DEPTH, F32, HALF>, lds);
-  if (!ok) return false;
-  const int split = (N + per - 1) / per, per_seq = (conv.C + kSkThreads - 1) / kSkThreads;
-  skinny_update_conv_kernel<XG, NT, DEPTH, F32, HALF><<<split + nseq * per_seq, kSkThreads, lds, s>>>(
-      (const unsigned short*)x, (const unsigned short*)w, norm.residual, norm.weight, (int)x_ld, M, N, K, norm.blocks, split,
-      SkinnyRest<kUpdate>{0, N, 0, 0, -1, 0, 0.f, 0.f, norm.cols, norm.eps, out, norm.squares, bias}, UpdateConvRest{conv, per_seq});
-  return true;
-}
+struct UpdateConvLaunch {
+  void* out;
+  const SkinnyNorm& norm;
+  const void *x, *w, *bias;
+  long x_ld;
+  int M, N, K, nseq;
+  const ConvUpdate& conv;
+  hipStream_t s;
+  template <int XG, int NT, int DEPTH, bool F32, bool HALF> bool run() const {
+    constexpr int lds = Skinny<XG, NT, DEPTH, F32, HALF>::kLds, per = HALF ? 8 : 16 * NT;
+    static const bool ok = allow_lds(&skinny_update_conv_kernel<XG, NT, DEPTH, F32, HALF>, lds);
+    if (!ok) return false;
+    const int split = (N + per - 1) / per, per_seq = (conv.C + kSkThreads - 1) / kSkThreads;
+    skinny_update_conv_kernel<XG, NT, DEPTH, F32, HALF><<<split + nseq * per_seq, kSkThreads, lds, s>>>(
+        (const unsigned short*)x, (const unsigned short*)w, norm.residual, norm.weight, (int)x_ld, M, N, K, norm.blocks, split,
+        SkinnyRest<kUpdate>{0, N, 0, 0, -1, 0, 0.f, 0.f, norm.cols, norm.eps, out, norm.squares, bias}, UpdateConvRest{conv, per_seq});
+    return true;
+  }
+};
 
 }  // namespace
 
@@ -58,23 +65,8 @@ bool launch_skinny_update_conv(void* out, const SkinnyNorm& norm, const void* x,
                                const ConvUpdate& conv, int nseq, hipStream_t s) {
   if (M <= 0 || N <= 0 || M > 32 || nseq <= 0 || conv.taps != 4) return false;
   if (f32) { x_ld *= 2; K *= 2; }   // in halves
-  // the forms that launch_skinny_linear_normed has for an update
-#define HS_UC(XG, NT, D, HALF) \
-  return f32 ? launch<XG, NT, D, true, HALF>(out, norm, x, x_ld, w, bias, M, N, K, conv, nseq, s) \
-             : launch<XG, NT, D, false, HALF>(out, norm, x, x_ld, w, bias, M, N, K, conv, nseq, s)
-  if (norm.blocks == N / 8) {
-    if (M <= 8) { if (K > 4096) HS_UC(1, 1, 3, true); HS_UC(1, 1, 2, true); }
-    if (M <= 16) HS_UC(2, 1, 2, true);
-    HS_UC(4, 1, 2, true);
-  }
-  const int nt = skinny_tiles(M, (N + 15) / 16, K);
-  if (nt == 4) HS_UC(4, 4, 1, false);   // above 16 rows alone
-  if (nt == 2) { if (M <= 8) HS_UC(1, 2, 1, false); if (M <= 16) HS_UC(2, 2, 1, false); HS_UC(4, 2, 1, false); }
-  if (M <= 8) HS_UC(1, 1, 2, false);
-  if (M <= 16) HS_UC(2, 1, 2, false);
-  if (f32) return launch<4, 1, 1, true, false>(out, norm, x, x_ld, w, bias, M, N, K, conv, nseq, s);
-  return launch<4, 1, 2, false, false>(out, norm, x, x_ld, w, bias, M, N, K, conv, nseq, s);
-#undef HS_UC
+  const UpdateConvLaunch l{out, norm, x, w, bias, x_ld, M, N, K, nseq, conv, s};
+  return f32 ? run_update<true>(l, M, N, K, norm.blocks) : run_update<false>(l, M, N, K, norm.blocks);
 }
 
 }  // namespace hipserve
