@@ -284,7 +284,8 @@ __global__ __launch_bounds__(256) void expert_gemm_mid_kernel(
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int lane = threadIdx.x & 63, slot0 = blockIdx.y * kMidRows, n0 = blockIdx.x * kMidCols;
   const int e = tile_expert[blockIdx.y], mine[2] = {slots[slot0 + lane], slots[slot0 + 64 + lane]};
-  const int rows = __popcll(__ballot(mine[0] >= 0)) + __popcll(__ballot(mine[1] >= 0));   // moe_align fills a tile from its first slot on
+  const unsigned long low = __ballot(mine[0] >= 0), high = __ballot(mine[1] >= 0);
+  const int rows = high != 0 ? 128 - __clzll(high) : 64 - (low != 0 ? __clzll(low) : 64);   // up to the last one: a table may have slots without a pair before it
   if (e < 0 || e >= E) return;
   const unsigned char* we = reinterpret_cast<const unsigned char*>(w + ((long)e * N + n0) * K);
 #define HS_EM(RT) expert_mid<RT>(out, x, x_ld, we, mine, slot0, n0, gather_k, gather_shift, N, K, act, smem)

@@ -2042,6 +2042,25 @@ def test_expert_gemm_of_prompt_tiles(counts, N, K, top, act):
         assert bool((out[slots < 0] == 7.0).all())
 
 
+@gpu
+@pytest.mark.parametrize("live", [[0], [33], [127], [1, 40, 63], [64, 96], [0, 31, 95], [5, 70, 126]])
+@pytest.mark.parametrize("tile", [32, 64, 128])
+def test_expert_gemm_of_tables_with_gaps(live, tile):
+    """Slots without a pair ahead of ones with a pair, as a table of one's own may have them: all of these are computed, by the kernels of every tile."""
+    g = torch.Generator().manual_seed(len(live) + tile)
+    E, N, K, cap = 3, 72, 128, 256
+    x, w = torch.randn(cap, K, generator=g).bfloat16().cuda(), torch.randn(E, N, K, generator=g).bfloat16().cuda() / K ** 0.5
+    slots = torch.full((cap,), -1, dtype=torch.int32)
+    at = torch.tensor([s + t for t in (0, 128) for s in live])
+    slots[at] = torch.randperm(len(at), generator=g).int()
+    te = (torch.arange(cap // tile) * tile // 128).int() + 1   # the first 128 slots are expert 1's, the rest expert 2's
+    out = torch.full((cap, N), 7.0, dtype=torch.bfloat16, device="cuda")
+    get_ops("cuda").expert_gemm(out, x, w, slots.cuda(), te.cuda(), tile, 1, 0)
+    want = (x.double()[slots[at].long().cuda()][:, None] * w.double()[1 + at.cuda() // 128]).sum(-1)
+    got = out[at.cuda()].double()
+    assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -16 * K ** 0.5).all()   # rounded to bf16; sums of 128 products in 32 bits
+
+
 def test_expert_plan_of_a_prompt():
     """What the three kernels were measured to take has the choice; sizes that were not looked at stay where they were."""
     from types import SimpleNamespace
