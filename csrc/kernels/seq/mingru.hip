@@ -187,7 +187,7 @@ struct MinGruArgs {
 // lanes further. Twice the workgroups, eight rows of weights per load and tile, and two pieces ahead beside the experts, too; the sums are the same. us, cold
 // weights, 16 channels -> 8: one row, 2048 x 2048 8.2 -> 7.5, 4096 x 2048 12.0 -> 10.9, with the experts of a row beside 13.2 -> 12.4, 6144 x 2048 18.3 ->
 // 15.8, 8192 x 4096 38.8 -> 37.3, with experts 44.5 -> 41.7; 16 rows, 2048 x 2048 9.5 -> 8.6.
-template <int XG, int DEPTH, bool F32, bool HALF>
+template <int XG, int DEPTH, bool F32, bool HALF, bool LATE>
 HS_DEVICE void mingru_block(int wg, const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const MinGruSeqs& seqs, int x_ld, int M,
                             int width, int K, int rest_at, unsigned char* smem) {
   using SK = std::conditional_t<HALF, Skinny<XG, 2, DEPTH, F32, true>, Skinny<XG, 3, DEPTH, F32>>;
@@ -219,13 +219,17 @@ HS_DEVICE void mingru_block(int wg, const unsigned short* __restrict__ x, const 
   SK::accumulate(acc, wt, w_row, reinterpret_cast<const unsigned char*>(x), x_row, K, smem, lane, wave, [&] {
     const auto rest = late_args<MinGruRest>(rest_at);
     const int nseq = rest->nseq;
-    const int *seq_cu = seqs.cu, *seq_ctx = seqs.ctx, *seq_state = seqs.state;
-    if (seq_cu == nullptr) { seq_cu = rest->seqs.cu; seq_ctx = rest->seqs.ctx; seq_state = rest->seqs.state; }
+    // Nothing writes these while the kernel runs, and as constants they are read by the scalar unit, whichever way the pointers come; as loads behind the copies'
+    // inline assembly they would be the vector unit's, which wait for the copies.
+    using Numbers = const __attribute__((address_space(4))) int*;
+    auto numbers = [](const int* p) { return (Numbers)(unsigned long)p; };
+    const Numbers seq_cu = numbers(LATE ? rest->seqs.cu : seqs.cu), seq_ctx = numbers(LATE ? rest->seqs.ctx : seqs.ctx),
+                  seq_state = numbers(LATE ? rest->seqs.state : seqs.state);
     y = static_cast<T*>(rest->y);
     state = rest->state;
     bz = rest->b_z[c];
     bx = rest->b_x[c];
-    // A wave's four rows' sequences through the scalar unit, whose loads the copies in flight are not waited for with.
+    // A wave's four rows' sequences
 #pragma unroll
     for (int i = 0; i < IT; ++i) {
       int slot = -1, ctx = 0;
@@ -266,7 +270,7 @@ __global__ __launch_bounds__(kSkThreads) void mingru_product_kernel(
     const unsigned short* __restrict__ x, const unsigned short* __restrict__ w, const int* __restrict__ seq_cu, const int* __restrict__ seq_ctx,
     const int* __restrict__ seq_state, int x_ld, int M, int width, int K, const MinGruRest) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  mingru_block<XG, DEPTH, F32, HALF>(blockIdx.x, x, w, MinGruSeqs{seq_cu, seq_ctx, seq_state}, x_ld, M, width, K, offsetof(MinGruArgs, rest), smem);
+  mingru_block<XG, DEPTH, F32, HALF, false>(blockIdx.x, x, w, MinGruSeqs{seq_cu, seq_ctx, seq_state}, x_ld, M, width, K, offsetof(MinGruArgs, rest), smem);
 }
 
 struct MinGruBesideArgs {
@@ -285,7 +289,7 @@ __global__ __launch_bounds__(kSkThreads) void mingru_product_experts_kernel(
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int b = blockIdx.x;
   if (b >= split) expert_beside(b - split, slots, tile_expert, offsetof(MinGruBesideArgs, experts), smem);
-  else mingru_block<XG, DEPTH, false, HALF>(b, x, w, MinGruSeqs{}, x_ld, M, width, K, offsetof(MinGruBesideArgs, rest), smem);
+  else mingru_block<XG, DEPTH, false, HALF, true>(b, x, w, MinGruSeqs{}, x_ld, M, width, K, offsetof(MinGruBesideArgs, rest), smem);
 }
 
 template <int XG, int DEPTH, bool HALF, bool F32>

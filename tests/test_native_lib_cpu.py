@@ -55,6 +55,19 @@ def test_copies_into_lds_keep_their_wait_states(name, tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
+def test_sequences_of_a_product_come_through_the_scalar_unit(tmp_path):
+    """minGRU's product asks for its rows' sequences behind its copies into LDS: the vector unit's loads would be waited for with these. Its own are the biases, the
+    states and what the experts beside it need."""
+    asm = tmp_path / "k.s"
+    subprocess.run([_build.HIPCC, *_build.HIP_FLAGS, "-I", os.path.join(_build.CSRC, "include"), "-S", "--cuda-device-only",
+                    os.path.join(_build.CSRC, "kernels", "seq", "mingru.hip"), "-o", asm], check=True, capture_output=True)
+    kernels = re.findall(r"\n(_ZN8hipserve\S*mingru_product\S*):\s.*?\n(.*?)s_endpgm", asm.read_text(), re.S)
+    assert len(kernels) >= 12
+    for name, code in kernels:
+        assert len(re.findall(r"global_load_(?!lds)", code)) <= 8 and len(re.findall(r"s_load", code)) >= 24, name
+
+
+@pytest.mark.skipif(not os.path.exists(_build.HIPCC), reason="no hipcc")
 def test_a_carried_state_is_asked_for_at_once(tmp_path):
     """The chunked gated rule's scan loads its 16 numbers per lane with no wait between them."""
     asm = tmp_path / "k.s"
