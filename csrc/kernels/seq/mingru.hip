@@ -312,10 +312,10 @@ bool launch_beside(void* y, float* state, const void* x, long x_ld, const void* 
   if (!ok) return false;
   const int split = (width + per - 1) / per;
   const ExpertBeside experts = expert_beside_args(ex);
-  // Two workgroups fit a compute unit and not three: thousands of experts' workgroups of a short k lose more than the launch (two_per_unit_pay, expert_beside.hip). us
-  // apart -> in one, 16 experts of 4096 x 1024: 16 rows, width 2048, k 1024 27.7 -> 29.9, 32 rows, 4096, k 2048 39.2 -> 41.0. 832 sizes of 1 - 32 rows: of those that go
-  // together seven take 1 - 3 % longer than apart and all 12 % less on average, without this 27 up to 8 % longer.
-  if (M > 8 && ex.K < 2048 && (long)experts.per_tile * ex.ntiles >= 4096) return false;
+  // Two workgroups fit a compute unit and not three: thousands of experts' workgroups of a short k lose more than the launch (two_per_unit_pay, expert_beside.hip), the
+  // sooner the shorter minGRU's own are. us apart -> in one, experts of 4096 x 1024: 16 of them, 16 rows, width 2048, k 1024 27.7 -> 29.9, 32 rows, 4096, k 2048 39.2 ->
+  // 41.0; 8 of them, 9 rows, 2048, k 1024 19.0 -> 19.8. Of 832 sizes of 1 - 32 rows three that go together take 1.1 - 1.4 % longer than apart, and all 12 % less on average.
+  if (ex.K < 2048 && (long)experts.per_tile * ex.ntiles > (HALF ? 2200 : 4000)) return false;
   mingru_product_experts_kernel<XG, DEPTH, HALF><<<split + experts.per_tile * ex.ntiles, kSkThreads, lds, s>>>(
       (const unsigned short*)x, (const unsigned short*)w, ex.slots, ex.tile_expert, (int)x_ld, M, width, K, split,
       MinGruRest{y, state, b_z, b_x, nseq, {seq_cu, seq_ctx, seq_state}}, experts);

@@ -1972,7 +1972,7 @@ def test_experts_beside_a_product(M, N, K, parts, E, top, eN, eK, gather):
 @gpu
 @pytest.mark.parametrize("M,N,K,E,eN,eK,together", [
     (33, 4096, 1024, 16, 4096, 1024, False), (40, 8192, 2048, 64, 1024, 512, False), (24, 6144, 2048, 32, 2048, 768, False), (48, 4096, 2048, 16, 2048, 1024, False),
-    (33, 4096, 1024, 16, 1024, 2048, True), (40, 4096, 2048, 16, 1024, 1024, True), (24, 4096, 1024, 16, 4096, 1024, True), (64, 1024, 1024, 8, 1024, 512, True)])
+    (33, 4096, 1024, 16, 1024, 2048, True), (40, 4096, 2048, 16, 1024, 1024, True), (24, 4096, 1024, 16, 4096, 1024, True), (8, 2048, 1024, 16, 4096, 1024, True), (9, 2048, 1024, 8, 4096, 1024, True), (64, 1024, 1024, 8, 1024, 512, True)])
 def test_experts_beside_where_they_are_faster(M, N, K, E, eN, eK, together):
     """Thousands of experts' workgroups of a short k stay in a launch of their own where the dense product's leave room for two per compute unit; minGRU's product alike."""
     P, tile, ops = 2 * M, 32, get_ops("cuda")
@@ -1987,7 +1987,7 @@ def test_experts_beside_where_they_are_faster(M, N, K, E, eN, eK, together):
         seqs = [torch.arange(c, dtype=torch.int32, device="cuda") for c in (n + 1, n, n)]
         f32 = lambda *s: zeros(*s, dt=torch.float32)  # noqa: E731
         got = ops._seq.mingru_product_experts(zeros(M, width), f32(n, width), zeros(M, K), zeros(3 * width, K), f32(width), f32(width), *seqs, *experts)
-        assert got == (eN // 16 * (cap // tile) < 4096 or eK >= 2048)
+        assert got == (eN // 16 * (cap // tile) <= (2200 if M <= 16 else 4000) or eK >= 2048)
 
 
 class _Recorder:
