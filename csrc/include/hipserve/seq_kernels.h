@@ -31,7 +31,7 @@ int skinny_tiles(int M, long tiles, int K);
 int skinny_cols(int M, long cols, int K);
 // Of up to 8 rows: pieces that a workgroup copies ahead, where they are three, or it takes 8 columns (half); 0: neither
 struct SkinnyWide { int ahead; bool half; };
-SkinnyWide skinny_wide(int M, long tiles, int K, bool f32);
+SkinnyWide skinny_wide(int M, long tiles, int K, bool f32, bool normed);
 // Whether its workgroups take 8 columns for 16; tiles of 16 columns, over all batches and parts, K in 16-bit halves
 bool skinny_half(int M, long tiles, int K);
 // A norm around such a product of up to 32 rows, in one part: with a residual [M, N] (fp32, updated in place), out = residual * weight

@@ -250,9 +250,9 @@ inline bool skinny_half(int64_t rows, int64_t cols, int64_t k, bool f32) {
   return hipserve::skinny_half(rows, (cols + 15) / 16, f32 ? 2 * k : k);
 }
 
-inline std::vector<int64_t> skinny_wide(int64_t rows, int64_t cols, int64_t k, bool f32) {   // pieces ahead, whether half tiles
+inline std::vector<int64_t> skinny_wide(int64_t rows, int64_t cols, int64_t k, bool f32, bool normed) {   // pieces ahead, whether half tiles
   TORCH_CHECK(rows >= 0 && rows <= 64 && cols >= 0 && cols < (1L << 40) && k >= 0 && k < (1L << 30), "skinny_wide: sizes");
-  const auto w = hipserve::skinny_wide(rows, (cols + 15) / 16, f32 ? 2 * k : k, f32);
+  const auto w = hipserve::skinny_wide(rows, (cols + 15) / 16, f32 ? 2 * k : k, f32, normed);
   return {w.ahead, w.half};
 }
 
@@ -266,7 +266,7 @@ inline void def_moe_ops(torch::Library& m) {
   m.def("skinny_time(int rows, int cols, int k, bool glu, bool f32, int parts) -> float", &skinny_time);
   m.def("skinny_half(int rows, int cols, int k, bool f32) -> bool", &skinny_half);
   m.def("skinny_cols(int rows, int cols, int k) -> int", &skinny_cols);
-  m.def("skinny_wide(int rows, int cols, int k, bool f32) -> int[]", &skinny_wide);
+  m.def("skinny_wide(int rows, int cols, int k, bool f32, bool normed=False) -> int[]", &skinny_wide);
   m.def("skinny_linear_parts(Tensor(a!) out, Tensor x, Tensor w, Tensor? bias) -> ()");
   m.def("skinny_linear_normed(Tensor(a!) out, Tensor x, Tensor squares, float eps, Tensor w, Tensor? bias, int act, float c0, float c1, "
         "int act_from) -> ()");

@@ -138,18 +138,22 @@ int skinny_cols(int M, long cols, int K) {
 }
 
 // Of up to 8 rows and more workgroups than compute units: how many pieces a workgroup of one whole tile copies ahead where three are best (0: by the rules of
-// the launch), and whether half tiles are better still. Three are for k (in halves) of 2048 and more, once the units have two workgroups each; half tiles are for up to 4
-// rows and weights whose rows lie a power of two of bytes apart, 4096 or 16384 and more, where whole tiles' loads of 16 rows meet on fewer channels. (8192 apart
-// they take 2 - 10 % longer, for which there is no reason but the measurement; at other multiples of 4096 they gain 2 % on average and lose up to 7; rows a little off
-// such places are as fast in whole tiles.) 105 sizes of 5632 - 32000 columns, k 2048, 8192 and 16384, 1 - 4 rows: 10 % less than whole tiles on average, one 3.6 %
-// more. Cold weights, us, one row, one or two pieces / three / half tiles: 8192 x 2048 9.2 / 8.2 / 7.5, 12288 x 2048 12.3 / 11.2 / 10.1, 32000 x 2048 25.8 / 23.9 / 22.1, 32000 x
-// 1984 21.7 / 22.1 / 21.4, 32000 x 2112 22.8 / 23.0 / 22.7, 8192 x 4096 14.2 / 13.2 / 13.9, 12288 x 4096 19.3 / 18.5 / 19.4, 8192 x 8192 28.8 / 27.1 / 24.0, 12288 x 8192 39.4 / 38.5 /
-// 34.1; 8 rows, 32000 x 2048 26.3 / 25.0 / 24.7; in 32 bits, 32000 x 1024 26.2 / 24.5 / 26.5. As they were: 5152 x 2048 6.5 (half tiles 6.4), 8192 x 3072 10.0 (10.3).
-SkinnyWide skinny_wide(int M, long tiles, int K, bool f32) {
+// the launch), and whether half tiles are better still.
+// Three are for weights whose rows lie a multiple of 4096 bytes apart, once the units have a workgroup and a half each, and in 16 bits for k of 2560 and more and two each.
+// Half tiles are for up to 4 rows and weights whose rows lie a power of two of bytes apart, 4096 or 16384 and more, where whole tiles' loads of 16 rows meet on
+// fewer channels. (8192 apart they take 2 - 10 % longer, for which there is no reason but the measurement; at other multiples of 4096 they gain 2 % on average and lose
+// up to 7; rows a little off such places are as fast in whole tiles.) 105 sizes of 5632 - 32000 columns, k 2048, 8192 and 16384, 1 - 4 rows: 10 % less than whole tiles on
+// average, one 3.6 % more. Not for rows without their norm's factor (normed): a workgroup sums all of their squares, for half the columns (k 1024 - 4096: 5 - 50 %
+// longer than whole tiles, 32000 x 2048 15 %).
+// Cold weights, us, one row, one or two pieces / three / half tiles: 8192 x 2048 9.2 / 8.2 / 7.5, 12288 x 2048 12.3 / 11.2 / 10.1, 32000 x 2048 25.8 / 23.9 / 22.1, 32000 x
+// 1984 21.7 / 22.1 / 21.4, 32000 x 2112 22.8 / 23.0 / 22.7, 12288 x 2112 10.4 / 10.9 / 10.8, 12288 x 2560 12.1 / 12.2 / 12.0, 8192 x 4096 14.2 / 13.2 / 13.9, 12288 x 4096 19.3 / 18.5 /
+// 19.4, 8192 x 8192 28.8 / 27.1 / 24.0, 12288 x 8192 39.4 / 38.5 / 34.1; 8 rows, 32000 x 2048 26.3 / 25.0 / 24.7; in 32 bits, 32000 x 1024 26.2 / 24.5 / 26.5, 12288 x 1152 11.3 / 12.1 /
+// 13.8. As they were: 5152 x 2048 6.5 (half tiles 6.4), 8192 x 3072 10.0 (10.3).
+SkinnyWide skinny_wide(int M, long tiles, int K, bool f32, bool normed) {
   if (M > 8 || K < 2048) return {0, false};
   const bool apart = (K & (K - 1)) == 0 && K % 8192 != 4096;
-  if (M <= 4 && !f32 && apart && tiles > 352) return {K > 4096 ? 3 : 2, true};
-  return {tiles > 512 || (tiles > 384 && K % 2048 == 0) ? 3 : 0, false};
+  if (M <= 4 && !f32 && !normed && apart && tiles > 352) return {K > 4096 ? 3 : 2, true};
+  return {K % 2048 == 0 ? (tiles > 384 ? 3 : 0) : !f32 && K >= 2560 && tiles > 512 ? 3 : 0, false};
 }
 
 double skinny_time(int M, long cols, int k, bool glu, bool f32, int parts) {
@@ -194,7 +198,7 @@ bool launch_skinny_linear(void* out, bool out_f32, long out_ld, long out_bs, lon
 #undef HS_SG
 #undef HS_S16
   }
-  if (const auto wide = batch == 1 && parts == 1 ? skinny_wide(M, tiles, K, f32) : SkinnyWide{}; wide.ahead > 0)
+  if (const auto wide = batch == 1 && parts == 1 ? skinny_wide(M, tiles, K, f32, false) : SkinnyWide{}; wide.ahead > 0)
     return !wide.half ? HS_SK(1, 1, 3, false) : wide.ahead > 2 ? HS_SK(1, 1, 3, false, true, 2) : HS_SK(1, 1, 2, false, true);
   const int nt = skinny_tiles(M, tiles, K / parts);
   // One piece ahead: two are faster (up to 40 %) where a wave waits for its few copies, up to 16 rows and more than a piece per wave (more than
@@ -234,12 +238,9 @@ static bool launch_normed(void* out, bool out_f32, const SkinnyNorm& norm, const
 #undef HS_SO
 #undef HS_SG
   }
-  if (const auto wide = skinny_wide(M, (N + 15) / 16, K, f32); wide.ahead > 0) {
-    if (wide.half && wide.ahead > 2) return out_f32 ? HS_SN(1, 1, 3, false, float, false, true) : HS_SN(1, 1, 3, false, unsigned short, false, true);
-    if (wide.half) return out_f32 ? HS_SN(1, 1, 2, false, float, false, true) : HS_SN(1, 1, 2, false, unsigned short, false, true);
+  if (skinny_wide(M, (N + 15) / 16, K, f32, true).ahead == 3)
     return f32 ? HS_SN(1, 1, 3, false, float, true, false) : out_f32 ? HS_SN(1, 1, 3, false, float, false, false)
          : HS_SN(1, 1, 3, false, unsigned short, false, false);
-  }
   // Pieces ahead for one tile: as run_update has them.
   const int nt = skinny_tiles(M, (N + 15) / 16, K);   // 4 above 16 rows alone
   return nt == 4 ? HS_S4() : nt == 2 ? HS_ST(2, 1, false) : HS_ST(1, 2, false);

@@ -175,10 +175,13 @@ def test_half_tiles_of_wide_products(k, half):
     """By the distance of the weights' rows, as measured: a class of them, not one, and neither their neighbours nor more rows, 32 bits or fewer workgroups."""
     load_kernel_library("seq")
     wide = torch.ops.hipserve_seq.skinny_wide
-    for cols in (5648, 8192, 32000):
+    for cols in (5648, 6160, 8192, 32000):
+        whole = [3 if k >= 2048 and (cols > 6144 if k % 2048 == 0 else k >= 2560 and cols > 8192) else 0, False]
         for rows in (1, 4):
-            assert wide(rows, cols, k, False) == [(2 if k <= 4096 else 3) if half else 0 if k < 2048 or cols == 5648 or (cols <= 8192 and k % 2048) else 3, half], (rows, cols)
-        assert not wide(5, cols, k, False)[1] and not wide(1, cols, k // 2, True)[1] and wide(9, cols, k, False) == [0, False]
+            assert wide(rows, cols, k, False) == ([2 if k <= 4096 else 3, True] if half else whole), (rows, cols)
+            assert wide(rows, cols, k, False, True) == whole   # rows without their norm's factor: squares would be summed for half the columns
+        assert wide(5, cols, k, False) == whole and wide(9, cols, k, False) == [0, False]
+        assert wide(1, cols, k // 2, True) == [3 if whole[0] and k % 2048 == 0 else 0, False]
     assert wide(1, 5632, k, False) == [0, False]
 
 
