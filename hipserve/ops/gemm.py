@@ -529,16 +529,19 @@ def packed_glu(x: torch.Tensor, w: PackedLinear, gelu: bool = False) -> torch.Te
 # whole rounds cost up to a round (about 21 us per 1000 k) or more: as a product of their own they run in smaller tiles, or over parts of k.
 def round_columns(rows: int, cols: int, k: int) -> int:
     """Columns whose tiles are whole rounds, or up to two of them, where the columns behind them would start a round; else 0. Either up to 128 columns (gates of a head
-    each): of 160 such sizes (1024 - 8192 rows, 1040 - 26752 columns, k 1024 - 4096) every one got faster as two products, 19 % on average. Or, from k
-    2048 on, so many that the last round is up to three eighths full: of 93 such sizes (2048 - 8192 rows, k up to 8192) 20 % on average, at most 0.6 % slower.
+    each): of 242 such sizes (1024 - 8192 rows, 1040 - 33000 columns, k 64 - 14336) 20 % faster as two products on average; slower only where one takes less than
+    about 50 us, the host's time for two launches (1100 rows of 13072 x 64 20 -> 45). Or, from k 2048 on, so many that the last round is up to three eighths
+    full: of 272 such sizes (2048 - 8192 rows) 20 % on average, at most 0.6 % slower.
     The second product reads the rows once more (10 - 20 us for 8192). us, one -> two, 8192 rows: 6160 x 2048 222 -> 156, 6208 x 4096 373 -> 277, 2656 x 4096 283 ->
     137, 8960 x 4096 404 -> 406, 2048 rows: 10304 x 4096 209 -> 134. Where the whole tiles themselves are neither full rounds nor up to two of them, some
-    lose: 3133 rows of 15120 x 1024 104 -> 120."""
+    lose: 3133 rows of 15120 x 1024 104 -> 120. So do most in the second round that are an odd number both ways: 7195 rows of 4456 x 8192 410 -> 664, 3312 of
+    10072 x 4096 240 -> 381, 1628 of 18768 x 4096 228 -> 257; 510, 10 x 51 or 17 x 30, gain: 2505 of 13160 x 2048 143 -> 119, 4290 of 7808 x 14336 1047 -> 684."""
     tiles, whole, behind = -(-rows // 256), cols // 256, cols % 256
     if rows < 1024 or cols % 8:
         return 0
     now, more = tiles * whole, tiles * -(-cols // 256)
-    if whole and 0 < behind <= 128 and -(-more // 256) > -(-now // 256) and (now % 256 == 0 or now <= 512):
+    rounds = now % 256 == 0 or now < 256 or now < 512 and now % 2 == 0
+    if whole and 0 < behind <= 128 and -(-more // 256) > -(-now // 256) and rounds:
         return 256 * whole
     return 256 * _cut(-(-cols // 256), tiles) if k >= 2048 and 2048 <= rows <= 8192 else 0
 
@@ -553,8 +556,8 @@ def _cut(tiles: int, across: int) -> int:
 
 
 def round_rows(rows: int, cols: int, k: int) -> int:
-    """Rows whose tiles are whole rounds, where the others leave the last round up to three eighths full; else 0. Of 127 such sizes (2048 - 8192 rows, 4096 - 28672
-    columns, k 2048 - 14336) two products take 13 % less on average, at most 2.4 % more. us, one -> two: 5142 rows of 4096 x 14336 824 -> 417, 4200 of 4096 x
+    """Rows whose tiles are whole rounds, where the others leave the last round up to three eighths full; else 0. Of 161 such sizes (2048 - 8192 rows, 4096 - 28672
+    columns, k 2048 - 14336) two products take 10 % less on average, at most 4.4 % more (7 or 8 rounds of 20480 columns, k up to 4096). us, one -> two: 5142 rows of 4096 x 14336 824 -> 417, 4200 of 4096 x
     12288 621 -> 287, 4200 of 12288 x 4096 397 -> 287, 6500 of 28672 x 4096 1154 -> 1031, 5600 of 12288 x 4096 417 -> 401, 7500 of 24576 x 2048 the same. Not
     for a fuller last round (5700 rows of 4096 x 12288 407 -> 542), shorter k (3510 of 24576 x 1024 152 -> 157), few rows (1040 of 16384 x 8192 241 -> 316), or
     many behind (7000 of 12288 x 2048 253 -> 264)."""

@@ -391,6 +391,16 @@ def test_columns_that_would_start_a_round(rows, cols, k, cut):
 
 
 @pytest.mark.parametrize("rows,cols,k,cut", [
+    (7195, 4456, 8192, 0), (3312, 10072, 4096, 0), (1628, 18768, 4096, 0),              # 29 x 17, 13 x 39, 7 x 73 tiles
+    (4298, 7768, 4096, 7680), (1100, 13072, 4096, 13056), (7900, 4128, 4096, 4096)])    # 17 x 30, 5 x 51, 31 x 16
+def test_columns_of_tiles_odd_both_ways(rows, cols, k, cut):
+    """Tiles in the second round, in an odd number both ways, are slower apart by up to two thirds."""
+    from hipserve.ops.gemm import round_columns
+
+    assert round_columns(rows, cols, k) == cut
+
+
+@pytest.mark.parametrize("rows,cols,k,cut", [
     (5142, 4096, 14336, 4096), (4097, 4096, 2048, 4096), (2713, 24576, 4096, 2048), (6500, 28672, 4096, 4096), (7310, 16384, 2048, 7168),
     (4096, 4096, 14336, 0), (5700, 4096, 12288, 0), (7000, 12288, 2048, 0), (3510, 24576, 1024, 0), (1040, 16384, 8192, 0), (5142, 4104, 14336, 0), (9000, 4096, 4096, 0),
     (5142, 6144, 4096, 0), (0, 4096, 4096, 0), (5142, 0, 4096, 0)])
