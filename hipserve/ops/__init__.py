@@ -940,11 +940,14 @@ class KernelOps:
 
     def _expert_plan(self, pairs: int, experts: int, ff: int, hidden: int, may_pack: bool) -> str:
         """How a prompt's two expert products, [ff, hidden] and back, are expected to be fastest in bf16: "rows" (tiles of 32, the kernel for few rows),
-        "tiles" (of 128; some pairs per expert, else most of their rows are empty) or, with ``may_pack``, "packed" (the grouped GEMM over packed weights), in us of a
-        model of each: a latency and the larger of the weights at 4.4 or 5.2 TB/s and what a compute unit takes in, per workgroup rows and columns times k; rounds of
-        512 columns x 128 rows for packed ones. 91 sizes (4 - 64 experts, 512 x 1024 to 2048 x 4096, 66 - 5600 tokens): the choice takes 1.1 % longer than the
-        fastest on average, at most 1 % longer than tiles of 32 and packed weights alone did. us rows / tiles / packed of both: 16 experts of 1024 x 2048, 87, 250,
-        350 pairs each 76 / 39 / -, 167 / 82 / 96, 222 / 100 / 97; 8 of 512 x 1024, 75, 175, 1000 each 13.6 / 15.9 / -, 24 / 20 / 24, 103 / 39 / 59."""
+        "tiles" (of 128; from 16 pairs per expert on, and below 128 of them if 7 % faster by the model than 32) or, with ``may_pack``, "packed" (the grouped GEMM
+        over packed weights), in us of a model of each: a latency and the larger of the weights at 4.4 or 5.2 TB/s and what a compute unit takes in, per workgroup
+        rows and columns times k; rounds of 512 columns x 128 rows for packed ones, half a round up to 64 of them, whose columns go to workgroups of their own. Of
+        1000 sizes where the choice is tiles (4 - 128 experts, 512 x 512 to 4096 x 4096, 65 - 8200 tokens, even and uneven) they take 0.64 of the time of tiles of
+        32 and 0.74 of packed weights' on average, and 3 - 12 % more in one of a hundred. What the bounds leave out, us: 10 - 15 pairs each gain 5 %
+        on average, but 24 experts of 2048 x 4096, 13 pairs each, 162 -> 182; 6 of 896 x 4096, 74 each, 44 -> 51; 12 of 4096 x 768, 257 each, packed 89, tiles 111.
+        us rows / tiles / packed of both: 16 experts of 1024 x 2048, 87, 250, 350 pairs each 76 / 39 / -, 167 / 82 / 96, 222 / 100 / 97; 8 of 512 x 1024, 75, 175,
+        1000 each 13.6 / 15.9 / -, 24 / 20 / 24, 103 / 39 / 59."""
         each = pairs / experts
 
         def rows(n, k):
@@ -959,11 +962,12 @@ class KernelOps:
         def packed(n, k):
             t = math.ceil(n / 512) * experts * (each / 128 + 0.5)
             whole, left = divmod(t, 256)
-            return 9 + whole * 24e-3 * k + (0 if left == 0 else min(24e-3 * k, 10) if whole and left <= 48 else 24e-3 * k)
+            return 9 + whole * 24e-3 * k + (0 if left == 0 else min(24e-3 * k, 10) if whole and left <= 48 else (24e-3 if t > 64 else 12e-3) * k)
 
         def both(f):
             return f(ff, hidden) + f(hidden, ff)
-        options = [(both(rows), "rows")] + ([(both(tiles), "tiles")] if each >= 10 else []) + ([(both(packed), "packed")] if may_pack else [])
+        options = [(both(rows), "rows")] + ([(both(tiles), "tiles")] if each >= 16 and both(tiles) < (0.93 if each < 128 else 1.0) * both(rows) else [])
+        options += [(both(packed), "packed")] if may_pack else []
         return min(options)[1]
 
     # ---- norms before and after every sublayer (csrc/kernels/seq/sandwich.hip)
