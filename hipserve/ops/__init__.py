@@ -114,10 +114,10 @@ class NormedRows:
 
 
 class DeltaBeside:
-    """A delta rule's decode step that another kernel of the same step may take into its launch; ``taken`` says whether one has."""
+    """A delta rule's decode step, of so many workgroups, that another kernel of the same step may take into its launch; ``taken`` says whether one has."""
 
-    def __init__(self, args):
-        self.args, self.taken = args, False
+    def __init__(self, args, workgroups=0):
+        self.args, self.workgroups, self.taken = args, workgroups, False
 
     def take(self, launch) -> bool:
         self.taken = bool(launch(*self.args))
@@ -497,7 +497,7 @@ class KernelOps:
                 sp.keep_first, sp.softcap, sink_w, sp.channel_gate, sp.chunk)
         if prep is not None:
             args = (out, proj, cache, *prep, meta.seq_cu, meta.seq_ctx, meta.seq_bt, *rest)
-            if beside is None or not beside.take(lambda *d: self._delta.window_delta_step(*args, *d)):
+            if beside is None or not self._window_delta_pays(sp.dim, min(part, span), beside.workgroups) or not beside.take(lambda *d: self._delta.window_delta_step(*args, *d)):
                 self._window_lib.window_attention_step(*args)
         else:
             self._window_lib.window_attention_decode(out, proj, cache, meta.seq_cu, meta.seq_ctx, meta.seq_bt,
@@ -612,7 +612,15 @@ class KernelOps:
         """``delta_rule_low`` for ``window_step`` to take into its launch: a ``DeltaBeside``, or None where it has no such launch."""
         if not (meta.num_prefill_tokens == 0 and self._delta_low_ok(state, proj, w2, sp, meta)):
             return None
-        return DeltaBeside((out, state[0], proj, a_b, w0, norm_w, meta.seq_state, sp.heads, sp.dim, eps, out_scale, w2))
+        return DeltaBeside((out, state[0], proj, a_b, w0, norm_w, meta.seq_state, sp.heads, sp.dim, eps, out_scale, w2), meta.num_decode * sp.heads)
+
+    @staticmethod
+    def _window_delta_pays(dim: int, keys: int, workgroups: int) -> bool:
+        """Whether window attention over runs of so many keys takes a delta rule's workgroups into its launch. They have its LDS and waves then, up to eight of
+        128 dims from 128 keys on, and many of them wait for room. Beside such runs in bf16, 24 sizes with 1000 - 2000 of
+        them are 7 % faster in one launch on average, of 55 with 2000 - 8000 29 are slower, by up to 15 %: us, apart / one, 128 rows of 2 heads, 300 keys and
+        32 of the rule's 43.4 / 49.7, 96 of 16 over 4, 230 and 48 50.0 / 56.1; but 128 rows of 16 over 2 of 64 dims and 48 48.9 / 45.4."""
+        return not (dim == 128 and keys > 128 and workgroups >= 2048)
 
     def delta_rule(self, out, state, proj, wl, a_b, w0, norm_w, sp, eps, meta, out_scale=1.0):
         def aligned(*tensors):   # the kernels below read and write 16 bytes at a time

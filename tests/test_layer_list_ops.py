@@ -2140,6 +2140,25 @@ def test_window_and_delta_step_in_one_launch(heads, kv, dim, ctxs, mode, dheads,
     assert all(torch.equal(a, b) for a, b in zip(*outs)) and outs[0][0].isfinite().all()
 
 
+@pytest.mark.parametrize("dim,ctx,rows,dheads,want", [
+    (128, 300, 128, 32, False), (128, 230, 64, 64, False), (128, 230, 64, 32, False),              # up to 15 % slower in one launch
+    (128, 230, 63, 32, True), (128, 100, 96, 48, True), (64, 300, 128, 32, True), (128, 230, 16, 32, True)])
+def test_delta_step_apart_where_many_workgroups_wait(monkeypatch, dim, ctx, rows, dheads, want):
+    """What window attention is offered and takes, by its runs and the rule's workgroups."""
+    from types import SimpleNamespace
+
+    from hipserve.ops import DeltaBeside, KernelOps
+    ops, apart = KernelOps(), []
+    monkeypatch.setattr(KernelOps, "_window_lib", SimpleNamespace(window_attention_decode_ok=lambda *a: True, window_attention_step=lambda *a: apart.append(a)))
+    monkeypatch.setattr(KernelOps, "_delta", SimpleNamespace(window_delta_step=lambda *a: True))
+    sp = SimpleNamespace(maps=1, dim=dim, vdim=dim, heads=16, kv_heads=4, reach=0, scale=1.0, window=0, sink=True, keep_first=0, softcap=0.0,
+                         channel_gate=False, chunk=0)
+    meta = SimpleNamespace(num_decode=rows, max_ctx=ctx, seq_cu=None, seq_ctx=None, seq_bt=None)
+    beside = DeltaBeside((), rows * dheads)
+    assert ops._window_decode(None, torch.empty(1, dtype=torch.bfloat16), None, meta, sp, -1, 1.0, None, (), beside)
+    assert beside.taken == want and len(apart) == (not want)
+
+
 @gpu
 @pytest.mark.parametrize("T,N,K,C,dtype", [(1, 64, 512, 1, torch.bfloat16), (8, 1024, 6144, 513, torch.bfloat16), (9, 1024, 2048, 512, torch.float32),
                                            (16, 4096, 512, 96, torch.bfloat16), (17, 4096, 512, 96, torch.float32), (32, 1024, 3072, 1025, torch.bfloat16),
