@@ -801,14 +801,17 @@ class KernelOps:
 
     def linear_update(self, x, w, bias, residual, norm_w, eps, conv=None):
         """residual += x . w^T + bias, and the rows for the next products as ``NormedRows`` of its norm; None, and nothing done, where the
-        update and norm are a launch of their own (``update_pays``). ``conv``: a ``ConvBeside`` that the launch may take."""
+        update and norm are a launch of their own (``update_pays``). ``conv``: a ``ConvBeside`` that the launch may take, but for 17 rows and
+        more of 32 bits from k 2048 on whose workgroups take 8 columns: of 1025 such sizes 633 took 1 - 11 % longer in one launch (22 rows of
+        2048 x 4096, 8192 channels, 16.9 -> 18.6 us). Of 31991 others 55 took more than 1 % longer, three of them 5, 7 and 15, and all 23 % less on average."""
         T, N, K = x.shape[0], w.shape[0], w.shape[1]
         if not (0 < T <= self.NORM_ROWS and N % 64 == 0 and N <= 4096 and self.update_pays(T, N, K, x.dtype == torch.float32)
                 and self._skinny_ok(x, w, bias) and residual.is_contiguous() and residual.data_ptr() % 16 == 0):
             return None
-        rows, squares = torch.empty(T, N, device=x.device, dtype=x.dtype), torch.empty(T, N // self.update_cols(T, N, K, x.dtype == torch.float32), device=x.device, dtype=torch.float32)
+        cols = self.update_cols(T, N, K, x.dtype == torch.float32)
+        rows, squares = torch.empty(T, N, device=x.device, dtype=x.dtype), torch.empty(T, N // cols, device=x.device, dtype=torch.float32)
         product = (rows, squares, residual, norm_w, x, w, bias)
-        if conv is None or not conv.take(lambda *c: self._delta.skinny_update_conv(*product, *c)):
+        if conv is None or (x.dtype == torch.float32 and T > 16 and cols == 8 and K >= 2048) or not conv.take(lambda *c: self._delta.skinny_update_conv(*product, *c)):
             self._moe_lib.skinny_linear_update(*product)
         return NormedRows(rows, squares, eps)
 

@@ -2159,6 +2159,23 @@ def test_delta_step_apart_where_many_workgroups_wait(monkeypatch, dim, ctx, rows
     assert beside.taken == want and len(apart) == (not want)
 
 
+@pytest.mark.parametrize("T,N,K,dtype,want", [(16, 2048, 4096, torch.float32, True), (17, 2048, 2048, torch.float32, False), (17, 2048, 2044, torch.float32, True),
+                                              (32, 2112, 4096, torch.float32, True), (17, 2048, 4096, torch.bfloat16, True)])
+def test_update_and_conv_apart_where_faster(monkeypatch, T, N, K, dtype, want):
+    """The launch of a residual update takes the convolution's at the measured side of its bounds alone, and the update runs either way."""
+    from types import SimpleNamespace
+    from hipserve.ops import ConvBeside, KernelOps
+    ops, ran = KernelOps(), []
+    monkeypatch.setattr(KernelOps, "_delta", SimpleNamespace(skinny_update_conv=lambda *a: ran.append("both") or True))
+    monkeypatch.setattr(KernelOps, "_moe_lib", SimpleNamespace(skinny_linear_update=lambda *a: ran.append("update")))
+    ops.update_pays = lambda *a: True
+    conv = ConvBeside(ops)
+    conv.left = ()
+    x, w, r = torch.empty(T, K, dtype=dtype), torch.empty(N, K, dtype=dtype), torch.empty(T, N)
+    assert ops.linear_update(x, w, None, r, torch.empty(N), 1e-6, conv=conv) is not None
+    assert ran == ["both" if want else "update"] and (conv.left is None) == want
+
+
 @gpu
 @pytest.mark.parametrize("T,N,K,C,dtype", [(1, 64, 512, 1, torch.bfloat16), (8, 1024, 6144, 513, torch.bfloat16), (9, 1024, 2048, 512, torch.float32),
                                            (16, 4096, 512, 96, torch.bfloat16), (17, 4096, 512, 96, torch.float32), (32, 1024, 3072, 1025, torch.bfloat16),
