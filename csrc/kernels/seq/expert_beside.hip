@@ -47,7 +47,11 @@ __global__ __launch_bounds__(kSkThreads) void skinny_linear_experts_kernel(
 // of 4096 x 1024 beside 8192 x 2048 35.8 -> 41.0, 64 of 1024 x 512 22.8 -> 25.7; 16 of 2048 x 1024 beside 4096 x 2048 22.0 -> 22.8, of 1024 x 1024 16.0 -> 15.6. Of 1306
 // sizes (1 - 64 rows, 2 M - 32 M dense weights, experts of k 512 - 4096) 488 are left apart for these bounds; of the others one takes more than 1 % longer than apart
 // (33 rows, 2.8 %), and all take 17 % less on average; without the bounds 307 do, up to 15 %. With room for three, all were faster together.
-bool two_per_unit_pay(const ExpertRows& ex, long wgs, int K, int split) {
+// Nor where more than 1.6 rounds of 33 rows and more go onto dense workgroups of one tile, as all here are, which two tiles are for otherwise (skinny_tiles): of 17774
+// sizes these are 214, which took 2.9 % less together on average and up to 9.5 % more (56 rows, 16 experts of 2560 x 512 beside 8000 x 2560 24.0 -> 26.3); of the
+// others 23 take more than 1 % more, up to 5 %.
+bool two_per_unit_pay(const ExpertRows& ex, long wgs, int M, int K, int parts, int split) {
+  if (M > 32 && parts == 1 && split >= 416 && K > 2048) return false;
   return ex.K >= 2048 || wgs <= 512 || (wgs <= 1536 && K <= 2048 && split <= 384) || (wgs <= 2560 && split <= 160);
 }
 
@@ -59,7 +63,7 @@ bool launch_beside(void* out, long out_ld, long out_zs, int parts, const void* x
   if (!ok) return false;
   const int split = (N + per - 1) / per * parts;
   const ExpertBeside experts = expert_beside_args(ex);
-  if (3 * lds > 160 * 1024 && !two_per_unit_pay(ex, experts.per_tile * ex.ntiles, K, split)) return false;
+  if (3 * lds > 160 * 1024 && !two_per_unit_pay(ex, experts.per_tile * ex.ntiles, M, K, parts, split)) return false;
   skinny_linear_experts_kernel<XG, NT, DEPTH, TO, HALF><<<split + experts.per_tile * ex.ntiles, kSkThreads, lds, s>>>(
       (const unsigned short*)x, (const unsigned short*)w, ex.slots, ex.tile_expert, (int)x_ld, M, N, K, ((K + 63) / 64 + parts - 1) / parts * 64, split,
       SkinnyRest<kPlain>{0, out_ld, 0, out_zs, -1, 0, 0.f, 0.f, 1.f, 0.f, out, nullptr, nullptr}, experts);

@@ -1982,9 +1982,11 @@ def test_experts_beside_a_product(M, N, K, parts, E, top, eN, eK, gather):
 @gpu
 @pytest.mark.parametrize("M,N,K,E,eN,eK,together", [
     (33, 4096, 1024, 16, 4096, 1024, False), (40, 8192, 2048, 64, 1024, 512, False), (24, 6144, 2048, 32, 2048, 768, False), (48, 4096, 2048, 16, 2048, 1024, False),
-    (33, 4096, 1024, 16, 1024, 2048, True), (40, 4096, 2048, 16, 1024, 1024, True), (24, 4096, 1024, 16, 4096, 1024, True), (8, 2048, 1024, 16, 4096, 1024, True), (9, 2048, 1024, 8, 4096, 1024, True), (64, 1024, 1024, 8, 1024, 512, True)])
+    (33, 4096, 1024, 16, 1024, 2048, True), (40, 4096, 2048, 16, 1024, 1024, True), (24, 4096, 1024, 16, 4096, 1024, True), (8, 2048, 1024, 16, 4096, 1024, True), (9, 2048, 1024, 8, 4096, 1024, True), (64, 1024, 1024, 8, 1024, 512, True),
+    (33, 6656, 2056, 16, 512, 2560, False), (40, 6640, 2560, 16, 512, 2560, True), (64, 6656, 2048, 8, 1024, 2048, True)])
 def test_experts_beside_where_they_are_faster(M, N, K, E, eN, eK, together):
-    """Thousands of experts' workgroups of a short k stay in a launch of their own where the dense product's leave room for two per compute unit; minGRU's product alike."""
+    """Thousands of experts' workgroups of a short k stay in a launch of their own where the dense product's leave room for two per compute unit, and any beside
+    many dense ones of 33 rows and a long k; minGRU's product alike."""
     P, tile, ops = 2 * M, 32, get_ops("cuda")
     cap = -(-(P + E * (tile - 1)) // tile) * tile
     slots, te, ps = (torch.empty(n, dtype=torch.int32, device="cuda") for n in (cap, cap // tile, P))
