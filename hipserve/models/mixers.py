@@ -914,12 +914,13 @@ class ParallelMixer:
         return t
 
     def _project(self, h):
-        """The halves' input projections of rows ``h``: parts of one product, or, in long prompts whose right half without biases can be cut
-        where rounds end (``ops.in_rounds``), one each. (A product with biases cannot be cut where rounds end: the library adds them in a pass of its own then.)"""
-        if self.left_biased and self.ops.in_rounds(h, self.split, self.w_in.shape[0] - self.split):
+        """The halves' input projections of rows ``h``: parts of one product, or one each where those are faster (``ops.in_rounds``)."""
+        cols = self.w_in.shape[0] - self.split
+        if self.ops.in_rounds(h, self.split, cols, **({} if self.left_biased else {"biased": self.b_in is not None})):
             act = dict(self.in_act, act_from=self.in_act["act_from"] - self.split) if self.in_act else {}
-            left, right = self.ops.linear(h, self.w_in[:self.split], self.b_in[:self.split]), self.ops.linear(h, self.w_in[self.split:], **act)
-            return left, right if self.end is None else right[:, :self.end - self.split]
+            left, right = (None if self.b_in is None else self.b_in[at] for at in (slice(self.split), slice(self.split, None)))
+            right = self.ops.linear(h, self.w_in[self.split:], None if self.left_biased else right, **act)
+            return self.ops.linear(h, self.w_in[:self.split], left), right if self.end is None else right[:, :self.end - self.split]
         proj = self.ops.linear(h, self.w_in, self.b_in, **self.in_act)
         return proj[:, :self.split], proj[:, self.split:self.end]
 

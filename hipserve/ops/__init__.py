@@ -181,9 +181,11 @@ class KernelOps:
         self.norm_library = "seq"
         # the rules of products of a few rows: arithmetic on sizes, a few us each, and a step asks for every product. What they said of
         # the last sizes is kept (a step that is not captured, of four layers and a few rows, took 20 - 40 us longer)
-        self.skinny_pays, self.skinny_parts, self.update_pays, self.update_cols, self.mingru_pays, self.expert_plan, self.latent_run = (
+        (self.skinny_pays, self.skinny_parts, self.update_pays, self.update_cols, self.mingru_pays, self.expert_plan, self.latent_run,
+         self.two_pay) = (
             functools.lru_cache(maxsize=4096)(rule)
-            for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._update_cols, self._mingru_pays, self._expert_plan, self._latent_run))
+            for rule in (self._skinny_pays, self._skinny_parts, self._update_pays, self._update_cols, self._mingru_pays, self._expert_plan, self._latent_run,
+                         self._two_pay))
 
     @property
     def _op(self):
@@ -767,11 +769,37 @@ class KernelOps:
         out = torch.empty(*y.shape[:-1], y.shape[-1] // 2, device=y.device, dtype=y.dtype) if act in self.GLU_ACTS else y
         return self.activation(out, y, act, c0, c1)
 
-    def in_rounds(self, x, before, cols) -> bool:
-        """Whether rows x onto ``before`` columns are whole rounds of the vendor's tiles, and a product onto so many further ones is cut where rounds end
-        (``gemm.round_columns``)."""
-        return (isinstance(x, torch.Tensor) and x.dim() == 2 and x.dtype == torch.bfloat16 and before % 256 == 0 and -(-x.shape[0] // 256) * before // 256 % 256 == 0
-                and gemm.round_columns(x.shape[0], cols, x.shape[1]) > 0)
+    def in_rounds(self, x, before, cols, biased=True) -> bool:
+        """Whether rows x onto ``before`` columns and so many further ones, which have no biases or some of which have (``biased``), are faster as a product each than as
+        one, in rounds of tiles that they fill better."""
+        if len(x.shape) != 2 or not x.shape[0] or x.dtype not in (torch.bfloat16, torch.float32):
+            return False
+        rows, k = x.shape
+        if (isinstance(x, torch.Tensor) and x.dtype == torch.bfloat16 and before % 256 == 0 and -(-rows // 256) * before // 256 % 256 == 0
+                and gemm.round_columns(rows, cols, k) > 0):
+            return True   # whole rounds, and a product that is cut where rounds end
+        return k >= 512 and self.two_pay(rows, before, cols, k, biased, x.dtype == torch.float32)   # (shorter ones were not measured)
+
+    def _two_pay(self, rows, before, cols, k, biased, f32) -> bool:
+        """``in_rounds`` by estimates. Up to 64 rows, by the time of the own kernel, whose workgroups over the sum of the columns may be a round that neither half starts (or the
+        vendor's product is to run). Else by rounds of tiles of 256 x 256, 256 at a time: one product where it saves a round and is up to two of them, not of halves that
+        fill one by themselves, or three to four; above 5000 rows two, as rounds are many. In 32 bits the vendor's tiles are smaller, and one is taken where it saves
+        a round of 64 x 64. Time against two products always, of parallel mixers' widths (k 512 - 4096, 384 - 37000 columns), one product always / as chosen here: 9973
+        sizes of up to 64 rows -23 / -23 %, 53 / 4 of them more than 3 % longer, up to 16 / 4; 2898 of 65 - 8192 rows -14 / -16 %, 451 / 11, up to 56 / 19 (35 us); in 32 bits 2533
+        of up to 64 rows -17 / -18 %, 229 / 24, up to 38 / 11, 1001 of 65 - 2048 rows -7 / -7 %, 224 / 54, up to 50 / 50 (65 rows of k 4096). us, two / one: 4073 rows of 3840 +
+        7808 x 3072 231 / 334, 3000 of 1280 + 10304 x 2048 137 / 169, 33 of 10240 + 10304 x 4096 40.8 / 46.9, 4096 of 4608 + 10256 x 2048 264 / 205."""
+        both = before + cols
+        if rows <= self.SKINNY_ROWS and (f32 or self.skinny_pays(rows, before, k) and self.skinny_pays(rows, cols, k)):
+            apart = self._skinny_time(rows, before, k, False, f32) + self._skinny_time(rows, cols, k, False, f32)
+            return self._skinny_time(rows, both, k, False, f32) > (0.975 if self.skinny_pays(rows, both, k, False, f32) else 0.925) * apart
+        tile = 64 if f32 else 256
+        left, right, one = (-(-rows // tile) * -(-n // tile) / 256 for n in (before, cols, both))
+        saves = math.ceil(one) < math.ceil(left) + math.ceil(right)
+        if f32:
+            return not saves
+        if not biased and gemm.round_columns(rows, both, k) > 0:
+            return rows > 5000
+        return rows > 5000 or not (saves and (one <= 1 or one <= 2 and max(left, right) > 1.1 or 3 < one <= 4))
 
     def _vendor_linear(self, x, w, bias):
         y = gemm.linear_in_rounds(x, w) if bias is None and x.dim() == 2 else None
@@ -1046,7 +1074,7 @@ class ReferenceOps:
 
     name = "reference"
 
-    def in_rounds(self, x, before, cols) -> bool:
+    def in_rounds(self, x, before, cols, biased=True) -> bool:
         return False
 
     def fill_uniform(self, out, row0, col0, gcols, key, scale):

@@ -488,6 +488,24 @@ def test_halves_projected_apart():
         assert a.shape == b.shape and torch.allclose(a, b, rtol=1e-12)
 
 
+@pytest.mark.parametrize("rows,left,right,k,biased,dtype,apart", [
+    (4073, 3840, 7712, 3072, True, torch.bfloat16, True), (4096, 4608, 10272, 2048, True, torch.bfloat16, False), (128, 16384, 20512, 4096, True, torch.bfloat16, False),
+    (3200, 2560, 5184, 1024, True, torch.bfloat16, True), (6000, 1280, 10272, 2048, False, torch.bfloat16, True), (1500, 3072, 5152, 1024, True, torch.bfloat16, False),
+    (2048, 2048, 8256, 4096, True, torch.bfloat16, True), (2048, 2048, 8256, 4096, False, torch.bfloat16, False),   # the one without biases is cut
+    (33, 10240, 10336, 4096, True, torch.bfloat16, True), (8, 10240, 10336, 4096, True, torch.bfloat16, False), (16, 2048, 5184, 1024, True, torch.bfloat16, False),
+    (40, 3328, 15392, 3072, True, torch.float32, True), (16, 2048, 5184, 1024, True, torch.float32, False), (789, 640, 1296, 512, False, torch.float32, False),
+    (900, 1536, 5184, 1024, True, torch.float32, True), (0, 2048, 5184, 1024, True, torch.bfloat16, False), (4073, 3840, 7712, 504, True, torch.bfloat16, False),
+    (4073, 3840, 7712, 3072, True, torch.float16, False)])
+def test_halves_projected_apart_where_faster(rows, left, right, k, biased, dtype, apart):
+    """Either side of the rules on one projection or two, at sizes that were measured, and what they leave alone."""
+    from hipserve.ops import KernelOps, NormedRows
+
+    x, ops = torch.empty(rows, k, dtype=dtype, device="meta"), KernelOps()
+    assert ops.in_rounds(x, left, right, biased=biased) == apart
+    if rows <= 32:
+        assert ops.in_rounds(NormedRows(x, None, 1e-5), left, right, biased=biased) == apart
+
+
 @gpu
 @pytest.mark.parametrize("rows,rank,apart", [(1024, 96, True), (1000, 96, False), (1024, 90, True)])
 def test_halves_projected_apart_in_rounds(rows, rank, apart):
