@@ -985,6 +985,7 @@ class KernelOps:
         1000 sizes where the choice is tiles (4 - 128 experts, 512 x 512 to 4096 x 4096, 65 - 8200 tokens, even and uneven) they take 0.64 of the time of tiles of
         32 and 0.74 of packed weights' on average, and 3 - 12 % more in one of a hundred. What the bounds leave out, us: 10 - 15 pairs each gain 5 %
         on average, but 24 experts of 2048 x 4096, 13 pairs each, 162 -> 182; 6 of 896 x 4096, 74 each, 44 -> 51; 12 of 4096 x 768, 257 each, packed 89, tiles 111.
+        Up to two rounds of workgroups of a long k count as 1.6 at least: 4 of 2816 x 512, 1201 each, packed 69, tiles 84.
         us rows / tiles / packed of both: 16 experts of 1024 x 2048, 87, 250, 350 pairs each 76 / 39 / -, 167 / 82 / 96, 222 / 100 / 97; 8 of 512 x 1024, 75, 175,
         1000 each 13.6 / 15.9 / -, 24 / 20 / 24, 103 / 39 / 59."""
         each = pairs / experts
@@ -996,7 +997,8 @@ class KernelOps:
         def tiles(n, k):
             wgs = math.ceil(n / 64) * experts * max(1.0, each / 128 + (0.5 if each > 96 else 0.0))
             r = min(128.0, 32 * math.ceil(each / 32))
-            return 2.5 + max(2e-6 * experts * n * k / 5.2, max(1.0, wgs / 256) * 2e-3 * k * (64 + r) / (42 if wgs <= 256 else 50))
+            rounds = max(1.0, wgs / 256, 1.6 if wgs > 256 and k >= 2048 else 0.0)   # a second one is not hidden where there are no more
+            return 2.5 + max(2e-6 * experts * n * k / 5.2, rounds * 2e-3 * k * (64 + r) / (42 if wgs <= 256 else 50))
 
         def packed(n, k):
             t = math.ceil(n / 512) * experts * (each / 128 + 0.5)

@@ -2114,7 +2114,8 @@ def test_expert_plan_of_a_prompt():
 
 @pytest.mark.parametrize("pairs,experts,ff,hidden,may_pack,want", [
     (320, 24, 2048, 4096, False, "rows"), (240, 24, 4096, 2560, False, "rows"), (441, 6, 896, 4096, False, "rows"), (525, 6, 1024, 1536, False, "rows"),
-    (3088, 12, 4096, 768, True, "packed"), (426, 24, 576, 2048, False, "tiles"), (1524, 4, 640, 640, False, "tiles"), (2496, 8, 1024, 1024, True, "tiles")])
+    (3088, 12, 4096, 768, True, "packed"), (426, 24, 576, 2048, False, "tiles"), (1524, 4, 640, 640, False, "tiles"), (2496, 8, 1024, 1024, True, "tiles"),
+    (4806, 4, 2816, 512, True, "packed"), (3130, 4, 3840, 768, True, "packed"), (4806, 4, 2816, 512, False, "tiles")])
 def test_expert_plan_where_a_choice_was_slower(pairs, experts, ff, hidden, may_pack, want):
     """Few pairs each, or little between the two by the model: tiles of 32; few groups of columns with many k: packed weights."""
     from hipserve.ops import KernelOps
