@@ -401,12 +401,17 @@ class TableMoE:
         tile_expert = torch.empty(cap // tile, dtype=torch.int32, device=dev)
         ntiles = torch.empty(1, dtype=torch.int32, device=dev)
         pair_slot = torch.empty(P, dtype=torch.int32, device=dev)
-        orders = (None, None)
+        orders = [None, None]
         if self.ops.moe_tables_align_ok(self.table, ids, E):
-            # either product has a tile per 512 columns (tile 256: 256), and a round is one per compute unit
+            # either product has a tile per 512 columns (tile 256: 256), and a round is one per compute unit; no order (about 2.5 us) for tiles of less than a round that are
+            # too many to go by columns: all of them are taken alike
             cus, cols = torch.cuda.get_device_properties(dev).multi_processor_count, 512 // gemm.PW_WM
-            orders = torch.empty(2, cap // tile, dtype=torch.int32, device=dev)
-            self.ops.moe_table_align(self.table, ids, E, tile, slots, tile_expert, pair_slot, ntiles, orders, [cus, cus], [-(-n // cols) for n in (ff, H)])
+            across = [-(-n // cols) for n in (ff, H)]
+            ordered = [i for i, a in enumerate(across) if 16 * a * -(-P // tile) <= 3 * cus or a * (cap // tile) > cus]
+            made = torch.empty(len(ordered), cap // tile, dtype=torch.int32, device=dev) if ordered else None
+            for row, i in enumerate(ordered):
+                orders[i] = made[row]
+            self.ops.moe_table_align(self.table, ids, E, tile, slots, tile_expert, pair_slot, ntiles, made, [cus] * len(ordered), [across[i] for i in ordered])
         else:
             op.moe_align(self.table.index_select(0, ids).reshape(-1), E, tile, slots, tile_expert, ntiles, pair_slot, None)
         pu, pd = self.packed

@@ -350,3 +350,29 @@ def test_alignments_for_the_packed_gemm_repeat(P, E):
         live = slots.view(-1, 128) >= 0   # a tile is filled from its first slot on
         assert bool((live[:, 1:] <= live[:, :-1]).all())
         assert int(nt) == int((-(-torch.bincount(ids, minlength=E) // 128)).sum())
+
+
+@pytest.mark.parametrize("T,E,H,ff,ordered", [(3000, 4, 512, 512, 2), (8192, 8, 512, 512, 0), (8192, 8, 2048, 512, 1), (8192, 8, 512, 2048, 1), (16384, 8, 1024, 512, 1),
+                                              (6145, 1, 512, 512, 0), (6144, 1, 512, 512, 2)])
+def test_packed_experts_ordered_where_it_matters(T, E, H, ff, ordered, monkeypatch):
+    """Products whose tiles are all taken alike get no order of them, with the bits that they have in one."""
+    from hipserve.config import TableMoESpec
+    from hipserve.models.mixers import TableMoE
+    from hipserve.ops import get_ops, gemm
+
+    ops, op, g = get_ops("cuda"), torch.ops.hipserve, torch.Generator(device=DEV).manual_seed(T + E)
+    m = TableMoE(TableMoESpec(experts=E, top=1, ff=ff), H, 97, torch.device("cuda"), torch.bfloat16, ops)
+    m.w_up, m.w_down, m.table = _rnd(g, E, ff, H, scale=0.05), _rnd(g, E, H, ff, scale=0.05), torch.randint(0, E, (97, 1), device=DEV, generator=g).int()
+    h, ids, asked, align = _rnd(g, T, H), torch.randint(0, 97, (T,), device=DEV, generator=g), [], ops.moe_table_align
+    monkeypatch.setattr(ops, "moe_table_align", lambda *a: (asked.append(len(a[9])), align(*a)))
+    y, ps = m._forward_packed(h, ids, T)
+    assert asked == [ordered]
+    tile, cus = 128 * gemm.PW_WM, torch.cuda.get_device_properties(0).multi_processor_count
+    cap = -(-(T + E * (tile - 1)) // tile) * tile
+    slots, te, nt, pair = (torch.empty(n, dtype=torch.int32, device=DEV) for n in (cap, cap // tile, 1, T))
+    orders = torch.empty(2, cap // tile, dtype=torch.int32, device=DEV)
+    align(m.table, ids, E, tile, slots, te, pair, nt, orders, [cus, cus], [-(-n * gemm.PW_WM // 512) for n in (ff, H)])
+    act, want = (torch.empty(cap, n, dtype=torch.bfloat16, device=DEV) for n in (ff, H))
+    op.prefill_gemm_packed_grouped(act, h, m.packed[0], ff, 4, te, nt, gemm.PW_WM, gemm.PW_RW, slots, 1, order=orders[0])
+    op.prefill_gemm_packed_grouped(want, act, m.packed[1], H, 0, te, nt, gemm.PW_WM, gemm.PW_RW, order=orders[1])
+    assert torch.equal(y[ps.long()], want[pair.long()]) and y[ps.long()].isfinite().all()
